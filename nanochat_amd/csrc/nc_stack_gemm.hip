@@ -6,7 +6,7 @@
 //
 //   linear_few_kernel    up to 64 rows (decode): the weight is streamed once, K is dealt to the four waves of a workgroup (and, where a
 //                        consumer adds partial sums, to several workgroups); no LDS in the loop.
-//   linear_tiled_kernel  more rows: 64 x 128 or 128 x 256 tiles, operands straight into a ring of three LDS stages.
+//   linear_tiled_kernel  more rows: 64 x 128, 128 x 128 or 128 x 256 tiles, operands straight into a ring of three LDS stages.
 //
 // A stacked weight is several matrices that read the same input; the epilogue sends each run of output columns its own way (store,
 // gelu, silu, GLUs, softplus, router logits, residual add, soft-capped logits).  Rows can be grouped by weight (experts).
@@ -90,6 +90,49 @@ __device__ __forceinline__ void store_cols(const NcLinear& g, int64_t out_off, i
             for (int r = 0; r < 4; r++)
                 if (n + r < g.N) {
                     const float z = v[r] * sg.p0;
+                    o[r] = sg.p1 > 0.f ? sg.p1 * tanhf(z / sg.p1) : z;
+                }
+        }
+    }
+}
+
+// eight consecutive columns n .. n+7 (column c of segment sg, a multiple of 8) of output row `row`
+typedef uint32_t v4u_a8 __attribute__((ext_vector_type(4), aligned(8)));       // (rows of an output are 8-byte aligned, no more)
+template <typename T>
+__device__ __forceinline__ void st8_f32(T* p, v4f a, v4f b) {
+    if constexpr (sizeof(T) == 2) *(v4u_a8*)p = v4u_a8{pack_bf16(a[0], a[1]), pack_bf16(a[2], a[3]), pack_bf16(b[0], b[1]), pack_bf16(b[2], b[3])};
+    else *(v4f*)p = a, *(v4f*)(p + 4) = b;
+}
+template <typename T>
+__device__ __forceinline__ void store_cols8(const NcSeg& sg, int N, int64_t out_off, int row, int n, int c, v4f a, v4f b) {
+    const int64_t at = out_off + (int64_t)row * sg.ld;
+    auto each = [](v4f v, auto f) { return v4f{f(v[0]), f(v[1]), f(v[2]), f(v[3])}; };
+    switch (sg.kind) {
+        case NC_SEG_PLAIN: st8_f32((T*)sg.out + at + c, a, b); break;
+        case NC_SEG_GELU: st8_f32((T*)sg.out + at + c, each(a, gelu_tanh_f32), each(b, gelu_tanh_f32)); break;
+        case NC_SEG_SILU: st8_f32((T*)sg.out + at + c, each(a, silu_f32), each(b, silu_f32)); break;
+        case NC_SEG_GLU:
+            st4_f32((T*)sg.out + at + (c >> 1), v4f{clamped_glu_f32(a[0], a[1], sg.p0), clamped_glu_f32(a[2], a[3], sg.p0), clamped_glu_f32(b[0], b[1], sg.p0),
+                                                    clamped_glu_f32(b[2], b[3], sg.p0)});
+            break;
+        case NC_SEG_SWIGLU:
+            st4_f32((T*)sg.out + at + (c >> 1), v4f{silu_f32(a[0]) * a[1], silu_f32(a[2]) * a[3], silu_f32(b[0]) * b[1], silu_f32(b[2]) * b[3]});
+            break;
+        case NC_SEG_SOFTPLUS:
+            st8_f32((float*)sg.out + at + c, each(a + *(const v4f*)(sg.bias + c), softplus_f32), each(b + *(const v4f*)(sg.bias + c + 4), softplus_f32));
+            break;
+        case NC_SEG_F32: st8_f32((float*)sg.out + at + c, a, b); break;
+        case NC_SEG_RESIDUAL: {
+            float* o = (float*)sg.out + at + c;
+            st8_f32(o, *(const v4f*)o + a, *(const v4f*)(o + 4) + b);
+            break;
+        }
+        default: {
+            float* o = (float*)sg.out + at + c;
+#pragma unroll
+            for (int r = 0; r < 8; r++)
+                if (n + r < N) {
+                    const float z = (r < 4 ? a[r & 3] : b[r & 3]) * sg.p0;
                     o[r] = sg.p1 > 0.f ? sg.p1 * tanhf(z / sg.p1) : z;
                 }
         }
@@ -186,6 +229,11 @@ __global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g) {
 // on the global side, so that the fragment reads of 16 rows are free of bank conflicts.  A ring of STAGES: the loads of STAGES - 1 steps
 // are in flight while one is multiplied.  Past the end of K the loads are issued all the same (into stages nobody reads any more), so
 // that the barrier counts the same number of loads in every step.
+//
+// What bounds it: the loads.  A compute unit takes some 35 bytes per clock straight into LDS (4096^3, 128 x 256: 88 us of loads alone, 62 of
+// products, 105 of both), which is why the widest tile that fills the chip is the one to take.  4096^3 140 -> 117 us, 1792 x 12352 x 2048
+// 120 -> 95 (954 TFLOP/s; the library's own product 90-95), 1792 x 2048 x 4096 41 -> 33: most of it by the epilogue, which cost 15 us per
+// round of tiles where its stores take 3.
 #define TILE_SWZ(row) (((row) & 7) ^ (((row) >> 3) & 1))
 #define TILE_OOB 0x80000000u       // a buffer offset past every descriptor: the load returns zeros
 #define TILE_GROUP_M 8
@@ -211,23 +259,16 @@ __device__ __forceinline__ bool group_tile_order(const NcLinear& g, int id, int 
     return true;
 }
 
-template <int A_P, int W_P, int STRIDE>
-__device__ __forceinline__ void tile_fetch(const void* A, uint32_t a_bytes, const void* W, uint32_t w_bytes, uint8_t* st, int w_part,
-                                           const uint32_t* vo_a, const uint32_t* vo_w, int k_off) {
-    const __amdgpu_buffer_rsrc_t da = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, a_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t dw = __builtin_amdgcn_make_buffer_rsrc((void*)W, 0, w_bytes, 0x00020000);
-#pragma unroll
-    for (int i = 0; i < A_P; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(da, (lds_ptr_t)(st + i * STRIDE), 16, vo_a[i], k_off, 0, 0);
-#pragma unroll
-    for (int i = 0; i < W_P; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(dw, (lds_ptr_t)(st + w_part + i * STRIDE), 16, vo_w[i], k_off, 0, 0);
+__device__ __forceinline__ void tile_load(const void* base, uint32_t bytes, uint8_t* st, uint32_t lane_off, int k_off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000), (lds_ptr_t)st, 16, lane_off, k_off, 0, 0);
 }
 
 template <typename T, int BM, int BN, int WM, int WN, int STAGES>
 __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, int tiles_m, int tiles_n, uint32_t a_bytes) {
     constexpr int NW = WM * WN, WTM = BM / WM / 16, WTN = BN / WN / 16, STAGE = (BM + BN) * 128, A_P = BM / 8 / NW, W_P = BN / 8 / NW;
-    // s_waitcnt vmcnt(loads of the STAGES - 2 youngest steps), other counters untouched
-    constexpr int FLIGHT = (STAGES - 2) * (A_P + W_P), WAIT = 0x0F70 | (FLIGHT & 15) | ((FLIGHT >> 4) << 14);
-    static_assert(A_P >= 1 && W_P >= 1 && NW % 2 == 0, "waves");
+    // s_waitcnt vmcnt(loads of the STAGES - 2 youngest steps) lgkmcnt(0)
+    constexpr int FLIGHT = (STAGES - 2) * (A_P + W_P), FIRST = FLIGHT + (A_P + W_P) / 2, WAIT = 0x0070 | (FLIGHT & 15) | ((FLIGHT >> 4) << 14);
+    static_assert(A_P >= 1 && W_P >= 1 && NW % 2 == 0 && STAGES >= 3, "waves");
     extern __shared__ __align__(16) uint8_t lds[];
     int tm, tn;
     if (g.tiles) {
@@ -264,49 +305,70 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
     for (int i = 0; i < WTM; i++)
 #pragma unroll
         for (int j = 0; j < WTN; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    auto fetch = [&](int t, int stage) {
-        tile_fetch<A_P, W_P, NW * 1024>(A, a_bytes, W, (uint32_t)(g.N - 1) * row_w + k_bytes, lds + stage * STAGE + wave * 1024, BM * 128, vo_a, vo_w,
-                                        t < ksteps ? t * 128 : 0);
-    };
+    // A step has two halves (the low and the high 64 bytes of K of a lane's 128-byte row).  While the low half multiplies, the fragments of the
+    // high half are read; then every wave has read all of its stage, the waves meet, and while the high half multiplies, the low fragments of
+    // the next step are read: neither the barrier nor an LDS read is ever waited for with the matrix cores idle.  The stage that was read is
+    // free from the meeting on: the loads of step kt + STAGES go there, spread over the products.
     auto meet = [&]() {
         asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(WAIT);    // the operands of the next step have landed (this wave's share; the barrier says everybody's)
+        __builtin_amdgcn_s_waitcnt(WAIT);    // the operands of the next step have landed, this step's fragments are read (this wave's share; the barrier says everybody's)
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
+    constexpr int LOADS = A_P + W_P, EARLY = LOADS / 2, PRODUCTS = WTM * WTN, READS = WTM + WTN;
+    const uint32_t w_bytes = (uint32_t)(g.N - 1) * row_w + k_bytes;
+    auto load = [&](int i, int k_off, uint8_t* st) {
+        if (i < A_P) tile_load(A, a_bytes, st + i * NW * 1024, vo_a[i], k_off);
+        else tile_load(W, w_bytes, st + BM * 128 + (i - A_P) * NW * 1024, vo_w[i - A_P], k_off);
+    };
+    v4i al[WTM], ah[WTM], wl[WTN], wh[WTN];
+    // half a step: products of (w, a), between them the reads of the other half's fragments and the loads [L0, L1) of a later step
+    auto half = [&](const v4i (&a)[WTM], const v4i (&w)[WTN], v4i (&na)[WTM], v4i (&nw)[WTN], const uint8_t* pa, const uint8_t* pw, int rd, auto l0, auto l1, int k_off, uint8_t* st) {
+        constexpr int L0 = decltype(l0)::value, NL = decltype(l1)::value - L0;
 #pragma unroll
-    for (int i = 0; i < STAGES - 1; i++) fetch(i, i);
-    meet();
-    int cur = 0, nxt = STAGES - 1;
+        for (int j = 0; j < WTN; j++)
+#pragma unroll
+            for (int p = 0; p < MMA_PARTS<T>; p++)
+#pragma unroll
+                for (int i = 0; i < WTM; i++) {
+                    const int n = j * WTM + i;
+                    if (p == 0) {
+#pragma unroll
+                        for (int r = 0; r < READS; r++)
+                            if (r * PRODUCTS / READS / 2 == n) {
+                                if (r == 0) nw[0] = *(const v4i*)(pw + rd);
+                                else if (r <= WTM) na[r - 1] = *(const v4i*)(pa + (r - 1) * 2048 + rd);
+                                else nw[r - WTM] = *(const v4i*)(pw + (r - WTM) * 2048 + rd);
+                            }
+#pragma unroll
+                        for (int r = 0; r < NL; r++)
+                            if ((2 * r + 1) * PRODUCTS / (2 * NL) == n) load(L0 + r, k_off, st);
+                    }
+                    mma_in_place<T>(acc[i][j], w[j], a[i], p);
+                }
+    };
+    const int wa = wm * (BM / WM) * 128, ww = BM * 128 + wn * (BN / WN) * 128;
+#pragma unroll
+    for (int i = 0; i < STAGES; i++)
+#pragma unroll
+        for (int r = 0; r < (i < STAGES - 1 ? LOADS : EARLY); r++) load(r, i < ksteps ? i * 128 : 0, lds + i * STAGE + wave * 1024);
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (FIRST & 15) | ((FIRST >> 4) << 14));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    wl[0] = *(const v4i*)(lds + ww + rd_lo);
+#pragma unroll
+    for (int i = 0; i < WTM; i++) al[i] = *(const v4i*)(lds + wa + i * 2048 + rd_lo);
+#pragma unroll
+    for (int j = 1; j < WTN; j++) wl[j] = *(const v4i*)(lds + ww + j * 2048 + rd_lo);
+    int cur = 0, prev = (STAGES - 1) * STAGE;     // byte offsets of the stage being read and of the one before it
     for (int kt = 0; kt < ksteps; kt++) {
-        const uint8_t* a = lds + cur * STAGE + wm * (BM / WM) * 128;
-        const uint8_t* w = lds + cur * STAGE + BM * 128 + wn * (BN / WN) * 128;
-        v4i al[WTM], ah[WTM], wl[2], wh[2];
-        wl[0] = *(const v4i*)(w + rd_lo);
-#pragma unroll
-        for (int i = 0; i < WTM; i++) al[i] = *(const v4i*)(a + i * 2048 + rd_lo);
-        wh[0] = *(const v4i*)(w + rd_hi);
-#pragma unroll
-        for (int i = 0; i < WTM; i++) ah[i] = *(const v4i*)(a + i * 2048 + rd_hi);
-        fetch(kt + STAGES - 1, nxt);         // into the stage read in step kt - 1: everyone is past the barrier that ended it
-#pragma unroll
-        for (int j = 0; j < WTN; j++) {
-            if (j + 1 < WTN) {               // one group ahead of its use
-                wl[(j + 1) & 1] = *(const v4i*)(w + (j + 1) * 2048 + rd_lo);
-                wh[(j + 1) & 1] = *(const v4i*)(w + (j + 1) * 2048 + rd_hi);
-            }
-#pragma unroll
-            for (int p = 0; p < MMA_PARTS<T>; p++)
-#pragma unroll
-                for (int i = 0; i < WTM; i++) mma_in_place<T>(acc[i][j], wl[j & 1], al[i], p);
-#pragma unroll
-            for (int p = 0; p < MMA_PARTS<T>; p++)
-#pragma unroll
-                for (int i = 0; i < WTM; i++) mma_in_place<T>(acc[i][j], wh[j & 1], ah[i], p);
-        }
+        const uint8_t* st = lds + cur;
+        const int next = cur + STAGE == STAGES * STAGE ? 0 : cur + STAGE;
+        const int k1 = kt + STAGES - 1 < ksteps ? (kt + STAGES - 1) * 128 : 0, k2 = kt + STAGES < ksteps ? (kt + STAGES) * 128 : 0;
+        half(al, wl, ah, wh, st + wa, st + ww, rd_hi, std::integral_constant<int, EARLY>{}, std::integral_constant<int, LOADS>{}, k1, lds + prev + wave * 1024);
         meet();
-        cur = cur + 1 == STAGES ? 0 : cur + 1;
-        nxt = nxt + 1 == STAGES ? 0 : nxt + 1;
+        half(ah, wh, al, wl, lds + next + wa, lds + next + ww, rd_lo, std::integral_constant<int, 0>{}, std::integral_constant<int, EARLY>{}, k2, lds + cur + wave * 1024);
+        prev = cur, cur = next;
     }
     // the loads past the end of K are still landing: they must be done before the workgroup gives its LDS back
     asm volatile("" ::: "memory");
@@ -318,14 +380,31 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
     for (int i = 0; i < WTM; i++)
 #pragma unroll
         for (int j = 0; j < WTN; j++) asm volatile("" : "+a"(acc[i][j]));
+    // out through LDS, each wave its own part: a lane then has eight neighbouring columns of a row, so a store is whole lines, and the code of
+    // the epilogues is there once (inlined per accumulator it was 16 times as long, and took longer than its stores)
+    constexpr int ROW = BN / WN + 4;                          // floats: rows shifted by four banks
+    constexpr int FIT = STAGES * STAGE / (NW * 64 * ROW), SUBS = FIT >= WTM ? WTM : FIT >= 4 ? 4 : FIT >= 2 ? 2 : 1;      // 16-row tiles at a time
+    static_assert(FIT >= 1 && WTM % SUBS == 0, "output staging");
+    float* const own = (float*)lds + wave * 16 * SUBS * ROW;
+    constexpr int CHUNKS = BN / WN / 8, ROWS_AT_ONCE = 64 / CHUNKS;
+    const int c = 8 * (lane % CHUNKS), n = n0 + wn * (BN / WN) + c;
+    NcSeg sg = g.seg[0];
+    int base = 0;
 #pragma unroll
-    for (int i = 0; i < WTM; i++) {
-        const int m = wm * (BM / WM) + 16 * i + frow;
-        if (m >= sp.rows) continue;
+    for (int i = 1; i < 4; i++)
+        if (i < g.nseg && n >= g.seg[i - 1].end) sg = g.seg[i], base = g.seg[i - 1].end;
 #pragma unroll
-        for (int j = 0; j < WTN; j++) {
-            const int n = n0 + wn * (BN / WN) + 16 * j + 4 * piece;
-            if (n < g.N) store_cols<T>(g, sp.out_off, sp.row0 + m, n, acc[i][j]);
+    for (int i0 = 0; i0 < WTM; i0 += SUBS) {
+#pragma unroll
+        for (int i = 0; i < SUBS; i++)
+#pragma unroll
+            for (int j = 0; j < WTN; j++) *(v4f*)(own + (16 * i + frow) * ROW + 16 * j + 4 * piece) = acc[i0 + i][j];
+#pragma unroll 1
+        for (int r = lane / CHUNKS; r < 16 * SUBS; r += ROWS_AT_ONCE) {
+            const int m = wm * (BM / WM) + 16 * i0 + r;
+            if (m >= sp.rows || n >= g.N) break;
+            const float* v = own + r * ROW + c;
+            store_cols8<T>(sg, g.N, sp.out_off, sp.row0 + m, n, n - base, *(const v4f*)v, *(const v4f*)(v + 4));
         }
     }
 }
@@ -378,11 +457,10 @@ int launch_tiled(const NcLinear& l, hipStream_t s) {
     NC_CHECK_LAUNCH("linear_tiled");
     return 0;
 }
-// tile shapes: 1 = 64 x 128 (two workgroups per compute unit), 2 = 128 x 256.  Measured and not kept: 128 x 128 in two stages (711 to 848
-// TFLOP/s where 128 x 256 has 833 to 870), 256 x 256 in two stages (598 to 690).
+// tile shapes: 1 = 64 x 128 (two workgroups per compute unit), 2 = 128 x 256, 3 = 128 x 128
 template <typename T>
 int launch_tiled_shape(const NcLinear& l, int shape, hipStream_t s) {
-    return shape == 1 ? launch_tiled<T, 64, 128, 2, 2, 3>(l, s) : launch_tiled<T, 128, 256, 2, 4, 3>(l, s);
+    return shape == 1 ? launch_tiled<T, 64, 128, 2, 2, 3>(l, s) : shape == 2 ? launch_tiled<T, 128, 256, 2, 4, 3>(l, s) : launch_tiled<T, 128, 128, 2, 4, 3>(l, s);
 }
 
 double linear_units(const NcLinear& l, int dtype, bool few) {
@@ -413,12 +491,16 @@ int nc_launch_linear_tiled(int dtype, const NcLinear& l, hipStream_t s, int cls,
     NC_CHECK_ARG(!l.partials && l.K % 64 == 0, "linear: the tiled kernel takes whole K-steps and finishes its sums");
     NcProfScope prof(cls, linear_units(l, dtype, false), s, linear_tag(l));
     if (!shape) {
-        // the widest tile unless it leaves compute units without one (measured at 1792 rows: 858 against 679 TFLOP/s at N = 12352, 551
-        // against 717 at N = 2048, where the launch has 112 or 448 tiles)
-        const int64_t wide = (int64_t)((l.M + 127) / 128) * ((l.N + 255) / 256) * l.batch;
-        // (a sum of a few K-steps is mostly its epilogue: two workgroups per compute unit, one of which works while the other stores)
-        const bool brief = l.K * (dtype ? 4 : 2) <= 512;
-        shape = l.tiles ? (l.tile_rows == 64 ? 1 : 2) : wide < 200 || brief ? 1 : 2;
+        // rounds of tiles over the compute units, times what a tile takes of one.  bf16, us at K = 2048: 11 / 30 / 18 (64 x 128, 128 x 256,
+        // 128 x 128): a tile's loads, not its products.  1792 rows: N = 2048 21 / 25 / 17.6, N = 4096 38 / 29 / 34, N = 12352 118 / 94 / 116;
+        // 500 rows, N = 4096: 15 / 25 / 16.  fp32 is bound by its products, where narrow tiles lose nothing (1792 x 4096 x 2048: 238 / 236 / 241).
+        const int cus = nc_cu_count(), unit[3] = {dtype ? 10 : 11, dtype ? 38 : 30, dtype ? 19 : 18}, bm[3] = {64, 128, 128}, bn[3] = {128, 256, 128};
+        int64_t best = 0;
+        for (int i = 0; i < 3; i++) {
+            const int64_t tiles = (int64_t)((l.M + bm[i] - 1) / bm[i]) * ((l.N + bn[i] - 1) / bn[i]) * l.batch, cost = (tiles + cus - 1) / cus * unit[i];
+            if (!shape || cost < best) best = cost, shape = i + 1;
+        }
+        if (l.tiles) shape = l.tile_rows == 64 ? 1 : 2;
     }
     if (l.tiles) NC_CHECK_ARG(l.tile_rows == (shape == 1 ? 64 : 128), "linear: group tiles of %d rows", l.tile_rows);
     return dtype ? launch_tiled_shape<float>(l, shape, s) : launch_tiled_shape<bf16_t>(l, shape, s);

@@ -61,6 +61,21 @@ def test_linear_kernels(dtype, kind):
             assert torch.allclose(got.double(), want, rtol=tol, atol=tol), (M, N, K, kernel, (got.double() - want).abs().max().item())
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("kernel", (3, 4, 5))
+def test_tiles_at_their_edges(kernel, dtype):
+    """One row and column group less than a tile, a tile, one more; sums of one, two and three K-steps and more than the ring of stages holds."""
+    say(f"tile edges, kernel {kernel}, {dtype}")
+    g = torch.Generator().manual_seed(5)
+    steps = 64 if dtype == torch.bfloat16 else 32
+    for M, N, K in [(63, 112, 1), (64, 128, 2), (65, 144, 3), (127, 240, 4), (128, 256, 5), (129, 272, 7), (257, 528, 4)]:
+        K = -(-K * steps // 64) * 64
+        a, w = torch.randn(M, K, generator=g).to(dtype), (torch.randn(N, K, generator=g) / K ** 0.5).to(dtype)
+        got = ops.stack_linear(a.to(DEV), w.to(DEV), kernel=kernel).cpu()
+        tol = 1e-2 if dtype == torch.bfloat16 else 2e-5       # one rounding to bf16 is 2^-9 of values up to about 4; fp32 sums of up to 448 terms
+        assert torch.allclose(got.double(), a.double() @ w.double().T, rtol=tol, atol=tol), (M, N, K)
+
+
 # ------------------------------------------------------------------------------------------------ whole prompts
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", list(CASES))
