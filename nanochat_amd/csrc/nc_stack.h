@@ -87,25 +87,27 @@ struct NcLinear {
     int max_tiles, tile_rows;
     const int32_t* a_rows;
     int a_div;
-    // the few-rows kernel may leave fp32 partial sums [splits][M][N] for its consumer instead of finishing
+    // the tiled kernel may leave fp32 partial sums [splits][M][N] for its consumer instead of finishing
     float* partials;
     int splits;
+    bool few;              // the sum in four chains, as the few-rows kernel has it
 };
+#define NC_FEW_ROWS 64                     // up to here a linear is a stream of its weight
 inline NcLinear nc_linear(const void* a, int64_t lda, const void* w, int M, int N, int K) {
     NcLinear l{};
-    l.a = a, l.lda = lda, l.w = w, l.ldw = K, l.M = M, l.N = N, l.K = K, l.batch = 1, l.a_div = 1, l.splits = 1;
+    l.a = a, l.lda = lda, l.w = w, l.ldw = K, l.M = M, l.N = N, l.K = K, l.batch = 1, l.a_div = 1, l.splits = 1, l.few = M <= NC_FEW_ROWS;
     return l;
 }
 inline void nc_linear_seg(NcLinear& l, int end, int kind, void* out, int ld, float p0 = 0.f, float p1 = 0.f, const float* bias = nullptr) {
     l.seg[l.nseg++] = NcSeg{end, kind, out, ld, p0, p1, bias};
 }
-#define NC_FEW_ROWS 64                     // up to here the few-rows kernel
 #define NC_TILE_WORDS 5
-#define NC_GROUP_TILE_FEW 16               // rows per group tile of the few-rows kernel (the tiled one takes 64 or 128)
-int nc_launch_linear_few(int dtype, const NcLinear& l, hipStream_t s, int cls = NC_CLS_LINEAR);
+#define NC_GROUP_TILE_FEW 32               // rows per group tile where groups have few rows (others: 64 or 128)
+int nc_launch_linear_few(int dtype, const NcLinear& l, hipStream_t s);
 int nc_launch_linear_tiled(int dtype, const NcLinear& l, hipStream_t s, int cls = NC_CLS_LINEAR, int shape = 0);     // shape 0: choose
-// splits of the summed index over workgroups that fill the chip for a few-rows linear whose consumer adds partial sums
-int nc_linear_few_splits(int M, int N, int K);
+int nc_launch_linear(int dtype, const NcLinear& l, hipStream_t s);                                                   // whichever is the faster
+// shares of the summed index that fill the chip for a linear whose consumer adds partial sums
+int nc_linear_splits(int dtype, int M, int N, int K);
 
 // ---------------------------------------------------------------- row kernels (nc_stack_rows.hip)
 // What the rows that leave for the next linear are: layer norm or RMS norm of x times a weight, or x itself in the storage type.

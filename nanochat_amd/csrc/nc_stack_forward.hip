@@ -5,13 +5,12 @@
 //   linear   [projections | router logits | first feed-forward matrix] . h    the activation of the feed-forward in the epilogue
 //   mixer    -> its part of `cat`; the feed-forward's part is there already
 //   experts  route (softmax, choice, expert order), gate and up with their activation, down: one row per (token, choice)
-//   linear   w_out . cat, added to the residual stream: in its epilogue, or (few rows) as partial sums by the row kernel
+//   linear   w_out . cat, added to the residual stream: in its epilogue, or (few tiles) as partial sums by the row kernel
 //   row add  x += partial sums + weighted expert rows (+ embedding output + step vector at the start of a pass), norm -> h
 // Per run of a post-norm layer, h = x in the storage type:
 //   linear   projections . h;  mixers, side by side if there are two  -> `cat`
-//   linear   w_out . cat -> sums in fp32 (few rows: partial ones);  row add  x += norm1(sums) -> h
+//   linear   w_out . cat -> sums in fp32 (few tiles: partial ones);  row add  x += norm1(sums) -> h
 //   linear   gate and up . h, activation in the epilogue;  linear  down -> sums;  row add  x += norm2(sums) -> h
-// Few rows (decode): weights are streamed by linear_few_kernel; more rows: the tiled kernel.
 #include "../../include/nanochat_amd_stack.h"
 #include "nc_stack.h"
 
@@ -53,8 +52,8 @@ NcWindowGeom window_geom(const nc_stack_mixer& l, int B, int T, int Tmax, int po
 }
 // shares of the sum over channels that the few columns of w_x are cut into, to fill the chip
 int scan_x_cols(const nc_stack_mixer& l) { return l.dt_rank_p + 2 * nc_scan_bc_cols(l.state_p); }
-int scan_x_splits(const nc_stack_mixer& l, int M) {
-    if (M <= NC_FEW_ROWS) return nc_linear_few_splits(M, scan_x_cols(l), l.inner_p);
+int scan_x_splits(int dtype, const nc_stack_mixer& l, int M) {
+    if (M <= NC_FEW_ROWS) return nc_linear_splits(dtype, M, scan_x_cols(l), l.inner_p);
     const int64_t tiles = (int64_t)((M + 63) / 64) * ((scan_x_cols(l) + 127) / 128);
     int splits = 1;
     while (splits < 16 && tiles * splits < 512 && l.inner_p % (2 * splits * NC_STACK_PAD) == 0 && l.inner_p / (2 * splits) >= 256) splits *= 2;
@@ -71,7 +70,7 @@ bool expand(int dtype, const nc_stack_mixer& l, const NcLatentGeom& g) {
 }
 int expert_tile_rows(const nc_stack_layer& l, int M) {
     const int per = M * l.top / l.experts;
-    return M <= NC_FEW_ROWS || per < 16 ? NC_GROUP_TILE_FEW : per < 128 ? 64 : 128;
+    return per < 32 ? NC_GROUP_TILE_FEW : per < 128 ? 64 : 128;
 }
 int expert_max_tiles(const nc_stack_layer& l, int M, int tile_rows) {
     const int pairs = M * l.top;
@@ -89,10 +88,11 @@ Workspace carve(const nc_stack_model* m, int B, int T, int n_logits, int max_key
         const nc_stack_layer& l = m->layers[i];
         proj = max_of(proj, M * l.mix_cols * es);
         router = max_of(router, M * l.router_cols * 4);
-        if (M <= NC_FEW_ROWS) parts = max_of(parts, (size_t)nc_linear_few_splits((int)M, (int)Wp, l.k_out) * M * Wp * 4);
-        else if (l.block == NC_BLOCK_POST_NORM) parts = max_of(parts, M * Wp * 4);
-        if (l.block == NC_BLOCK_POST_NORM && l.ff) {
-            if (M <= NC_FEW_ROWS) parts = max_of(parts, (size_t)nc_linear_few_splits((int)M, (int)Wp, l.ff_p) * M * Wp * 4);
+        const bool post = l.block == NC_BLOCK_POST_NORM;
+        const int splits = nc_linear_splits(m->dtype, (int)M, (int)Wp, l.k_out);
+        if (post || splits > 1) parts = max_of(parts, splits * M * Wp * 4);
+        if (post && l.ff) {
+            parts = max_of(parts, nc_linear_splits(m->dtype, (int)M, (int)Wp, l.ff_p) * M * Wp * 4);
             act = max_of(act, M * l.ff_p * es);
         }
         for (int j = 0; j < l.n_mixers; j++) {
@@ -119,7 +119,7 @@ Workspace carve(const nc_stack_model* m, int B, int T, int n_logits, int max_key
                 default:
                     ret = max_of(ret, nc_scan_workspace_bytes(scan_geom(x, B, T)));
                     u = max_of(u, M * x.inner_p * es);
-                    x_parts = max_of(x_parts, (size_t)scan_x_splits(x, (int)M) * M * scan_x_cols(x) * 4);
+                    x_parts = max_of(x_parts, (size_t)scan_x_splits(m->dtype, x, (int)M) * M * scan_x_cols(x) * 4);
                     if (T == 1) break;
                     dt = max_of(dt, M * x.inner_p * 4);
                     dtr = max_of(dtr, M * x.dt_rank_p * es), bc = max_of(bc, M * 2 * nc_scan_bc_cols(x.state_p) * 4);
@@ -171,10 +171,6 @@ Workspace carve(const nc_stack_model* m, int B, int T, int n_logits, int max_key
 const void* at(const void* p, int64_t elems, int dtype) { return (const uint8_t*)p + elems * (dtype ? 4 : 2); }
 void* at(void* p, int64_t elems, int dtype) { return (uint8_t*)p + elems * (dtype ? 4 : 2); }
 
-int run_linear(int dtype, const NcLinear& l, hipStream_t s) {
-    return l.M <= NC_FEW_ROWS || l.K % 64 != 0 ? nc_launch_linear_few(dtype, l, s) : nc_launch_linear_tiled(dtype, l, s);
-}
-
 // A mixer reads its columns of the projected rows (`proj`, leading dimension ldp) and writes its columns of what the output matrix multiplies
 // (`cat`, leading dimension ld_cat).
 int run_latent_attention(int dt, const nc_stack_mixer& l, const NcLatentGeom& g, const Workspace& w, void* proj, int ldp, float eps, int rope_len,
@@ -194,13 +190,13 @@ int run_latent_attention(int dt, const nc_stack_mixer& l, const NcLatentGeom& g,
     NcLinear q = nc_linear(proj, ldp, l.w_uk_t, M, l.rank_p, l.dim_p);
     q.batch = l.heads, q.a_stride = qd, q.w_stride = (int64_t)l.rank_p * l.dim_p, q.out_stride = rw;
     nc_linear_seg(q, q.N, NC_SEG_PLAIN, w.q_lat, l.heads * rw);
-    TRY(run_linear(dt, q, s));
+    TRY(nc_launch_linear(dt, q, s));
     TRY(nc_launch_latent_attention(dt, g, w.q_lat, cache, seqlens, w.o_lat, w.att_parts, w.att_part_bytes, s));
     // ... and the weighted latents out of it: the value rows of w_ukv sit behind the head's dim_p key rows
     NcLinear v = nc_linear(w.o_lat, l.heads * l.rank_p, at(l.w_ukv, (int64_t)l.dim_p * l.rank_p, dt), M, l.vdim_p, l.rank_p);
     v.batch = l.heads, v.a_stride = l.rank_p, v.w_stride = (int64_t)head_w * l.rank_p, v.out_stride = l.vdim_p;
     nc_linear_seg(v, v.N, NC_SEG_PLAIN, cat, ld_cat);
-    return run_linear(dt, v, s);
+    return nc_launch_linear(dt, v, s);
 }
 
 int run_window_attention(int dt, const nc_stack_mixer& l, const NcWindowGeom& g, const Workspace& w, void* proj, int ldp, float eps, int rope_len,
@@ -219,17 +215,11 @@ int run_retention(int dt, const nc_stack_mixer& l, const NcRetentionGeom& g, con
 
 int run_selective_scan(int dt, const nc_stack_mixer& l, const NcScanGeom& g, const Workspace& w, const void* proj, int ldp, const int32_t* seqlens,
                        const float* state_in, float* state_out, void* cat, int ld_cat, hipStream_t s) {
-    const int M = g.B * g.T, N = scan_x_cols(l), splits = scan_x_splits(l, M);
+    const int M = g.B * g.T, N = scan_x_cols(l), splits = scan_x_splits(dt, l, M);
     TRY(nc_launch_scan_conv(dt, g, proj, ldp, l.conv_w, l.conv_b, seqlens, state_in, state_out, w.u, s));
     NcLinear x = nc_linear(w.u, l.inner_p, l.w_x, M, N, l.inner_p);
-    if (M <= NC_FEW_ROWS) {
-        if (splits > 1) x.partials = w.x_parts, x.splits = splits;
-        else nc_linear_seg(x, N, NC_SEG_F32, w.x_parts, N);
-    } else {                                       // every share is a product of its own
-        x.K = l.inner_p / splits, x.batch = splits, x.a_stride = x.w_stride = x.K, x.out_stride = (int64_t)M * N;
-        nc_linear_seg(x, N, NC_SEG_F32, w.x_parts, N);
-    }
-    TRY(run_linear(dt, x, s));
+    x.partials = w.x_parts, x.splits = splits;
+    TRY(nc_launch_linear(dt, x, s));
     const void* z = at(proj, l.inner_p, dt);
     if (g.T == 1) {
         const NcScanStep p{w.x_parts, splits, l.w_dt_t, l.dt_b, l.a_log2, l.skip, w.u, z, ldp, seqlens, state_in, state_out, cat, ld_cat};
@@ -238,7 +228,7 @@ int run_selective_scan(int dt, const nc_stack_mixer& l, const NcScanGeom& g, con
     TRY(nc_launch_scan_join(dt, g, w.x_parts, splits, w.dtr, w.bc, s));
     NcLinear d = nc_linear(w.dtr, l.dt_rank_p, l.w_dt, M, l.inner_p, l.dt_rank_p);
     nc_linear_seg(d, d.N, NC_SEG_SOFTPLUS, w.dt, l.inner_p, 0.f, 0.f, l.dt_b);
-    TRY(run_linear(dt, d, s));
+    TRY(nc_launch_linear(dt, d, s));
     return nc_launch_scan(dt, g, w.u, w.dt, w.bc, l.a_log2, l.skip, z, ldp, seqlens, state_in, state_out, cat, ld_cat, w.ret, s);
 }
 
@@ -295,8 +285,8 @@ int run_experts(int dt, const nc_stack_layer& l, int M, int width_p, const Works
     TRY(nc_launch_stack_route(r, M, s));
     const int pairs = M * l.top;
     auto grouped = [&](NcLinear& g) {
-        g.tiles = w.tiles, g.n_tiles = w.n_tiles, g.max_tiles = r.max_tiles, g.tile_rows = r.tile_rows, g.w_stride = (int64_t)g.N * g.K;
-        return r.tile_rows == NC_GROUP_TILE_FEW ? nc_launch_linear_few(dt, g, s, NC_CLS_EXPERTS) : nc_launch_linear_tiled(dt, g, s, NC_CLS_EXPERTS);
+        g.tiles = w.tiles, g.n_tiles = w.n_tiles, g.max_tiles = r.max_tiles, g.tile_rows = r.tile_rows, g.few = M <= NC_FEW_ROWS || pairs / l.experts < 16, g.w_stride = (int64_t)g.N * g.K;
+        return nc_launch_linear_tiled(dt, g, s, NC_CLS_EXPERTS);
     };
     NcLinear up = nc_linear(w.h, width_p, l.w_e1, pairs, 2 * l.expert_ff_p, width_p);
     up.a_rows = w.perm, up.a_div = l.top;
@@ -368,14 +358,11 @@ void entry_norm(const nc_stack_model* m, const nc_stack_run& run, int& norm, con
     norm = l.block == NC_BLOCK_POST_NORM ? NC_ROW_COPY : m->norm == NC_NORM_RMS ? NC_ROW_RMS_NORM : NC_ROW_LAYER_NORM;
     w = l.norm_w;
 }
-// sums = W rows, in fp32 for the row kernel: whole, or (few rows) in as many shares as fill the chip
+// sums = W rows, in fp32 for the row kernel, in as many shares as fill the chip
 int run_sums(int dt, const void* a, const void* w, int M, int N, int K, float* parts, NcRowAdd& add, hipStream_t s) {
     NcLinear l = nc_linear(a, K, w, M, N, K);
-    const int splits = M <= NC_FEW_ROWS ? nc_linear_few_splits(M, N, K) : 1;
-    if (splits > 1) l.partials = parts, l.splits = splits;
-    else nc_linear_seg(l, N, NC_SEG_F32, parts, N);
-    add.partials = parts, add.splits = splits;
-    return run_linear(dt, l, s);
+    add.partials = l.partials = parts, add.splits = l.splits = nc_linear_splits(dt, M, N, K);
+    return nc_launch_linear(dt, l, s);
 }
 }  // namespace
 
@@ -423,7 +410,7 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
         mixer_segs(l, in, w, dt);
         if (l.router_cols) nc_linear_seg(in, l.mix_cols + l.router_cols, NC_SEG_F32, w.router, l.router_cols);
         if (!post && l.ff_cols) nc_linear_seg(in, l.n_in, ff_seg_kind(l.ff), at(w.cat, l.mix_out, dt), l.k_out, l.ff_limit);
-        TRY(run_linear(dt, in, s));
+        TRY(nc_launch_linear(dt, in, s));
         TRY(run_mixers(m, kv, run, w, B, T, s));
 
         NcRowAdd add{};
@@ -436,17 +423,19 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
                 TRY(nc_launch_stack_row_add(dt, add, m->eps, M, M, m->width, Wp, s));
                 NcLinear up = nc_linear(w.h, Wp, l.w_ff_in, M, l.ff_cols, Wp);
                 nc_linear_seg(up, l.ff_cols, ff_seg_kind(l.ff), w.act, l.ff_p);
-                TRY(run_linear(dt, up, s));
+                TRY(nc_launch_linear(dt, up, s));
                 TRY(run_sums(dt, w.act, l.w_ff_out, M, Wp, l.ff_p, w.parts, add, s));
                 add.post_norm_w = l.norm2_w, add.h = nullptr;
             }
         } else {
             if (l.ff == NC_FF_EXPERTS) TRY(run_experts(dt, l, M, Wp, w, s));
-            NcLinear out = nc_linear(w.cat, l.k_out, l.w_out, M, Wp, l.k_out);
-            const int splits = M <= NC_FEW_ROWS ? nc_linear_few_splits(M, Wp, l.k_out) : 1;
-            if (splits > 1) out.partials = w.parts, out.splits = splits, add.partials = w.parts, add.splits = splits;
-            else nc_linear_seg(out, Wp, NC_SEG_RESIDUAL, w.x, Wp);
-            TRY(run_linear(dt, out, s));
+            if (nc_linear_splits(dt, M, Wp, l.k_out) > 1) {
+                TRY(run_sums(dt, w.cat, l.w_out, M, Wp, l.k_out, w.parts, add, s));
+            } else {
+                NcLinear out = nc_linear(w.cat, l.k_out, l.w_out, M, Wp, l.k_out);
+                nc_linear_seg(out, Wp, NC_SEG_RESIDUAL, w.x, Wp);
+                TRY(nc_launch_linear(dt, out, s));
+            }
             if (l.ff == NC_FF_EXPERTS) add.expert_out = w.e_out, add.slot_of = w.slot_of, add.slot_w = w.slot_w, add.top = l.top;
         }
         if (taps) add.tap = taps + (int64_t)i * M * Wp;
@@ -470,17 +459,17 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
         TRY(nc_launch_stack_row_add(dt, add, m->eps, M, n_logits, m->width, Wp, s));
         NcLinear head = nc_linear(w.h_last, Wp, m->head, n_logits, m->vocab, Wp);
         nc_linear_seg(head, m->vocab, NC_SEG_LOGITS, logits_out, m->vocab, m->logit_scale, m->logit_softcap);
-        TRY(run_linear(dt, head, s));
+        TRY(nc_launch_linear(dt, head, s));
     }
     return 0;
 }
 
 extern "C" int nc_stack_linear(int dtype, const void* a, int64_t lda, const void* w, void* out, int ldc, int M, int N, int K, int kind, float limit,
                                int kernel, nc_stream_t stream) {
-    NC_CHECK_ARG(out && ((kind >= NC_SEG_PLAIN && kind <= NC_SEG_F32) || kind == NC_SEG_SILU || kind == NC_SEG_SWIGLU) && N % 16 == 0 && kernel >= 0 && kernel <= 5, "stack_linear: kind %d, N %d", kind, N);
+    NC_CHECK_ARG(out && ((kind >= NC_SEG_PLAIN && kind <= NC_SEG_F32) || kind == NC_SEG_SILU || kind == NC_SEG_SWIGLU) && N % 16 == 0 && kernel >= 0 && kernel <= 8, "stack_linear: kind %d, N %d", kind, N);
     NcLinear l = nc_linear(a, lda, w, M, N, K);
     nc_linear_seg(l, N, kind, out, ldc, limit);
-    if (kernel == 0) return run_linear(dtype, l, (hipStream_t)stream);
+    if (kernel == 0) return nc_launch_linear(dtype, l, (hipStream_t)stream);
     if (kernel == 1) return nc_launch_linear_few(dtype, l, (hipStream_t)stream);
     return nc_launch_linear_tiled(dtype, l, (hipStream_t)stream, NC_CLS_LINEAR, kernel - 2);
 }

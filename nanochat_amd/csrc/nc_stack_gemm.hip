@@ -4,9 +4,10 @@
 // matter as long as both operands agree.  Operands are issued as (W, A), so a lane ends up with four consecutive output columns of
 // one output row.
 //
-//   linear_few_kernel    up to 64 rows (decode): the weight is streamed once, K is dealt to the four waves of a workgroup (and, where a
-//                        consumer adds partial sums, to several workgroups); no LDS in the loop.
-//   linear_tiled_kernel  more rows: 64 x 128, 128 x 128 or 128 x 256 tiles, operands straight into a ring of three LDS stages.
+//   linear_tiled_kernel  tiles of 32 x 64 to 128 x 256 outputs, operands straight into a ring of LDS stages; the summed index may be dealt to
+//                        several workgroups, whose consumer adds their sums.
+//   linear_few_kernel    few rows of a small weight, or a summed index that is no multiple of 64: operands straight into registers, no LDS in
+//                        the loop.
 //
 // A stacked weight is several matrices that read the same input; the epilogue sends each run of output columns its own way (store,
 // gelu, silu, GLUs, softplus, router logits, residual add, soft-capped logits).  Rows can be grouped by weight (experts).
@@ -159,12 +160,12 @@ __device__ __forceinline__ int64_t a_row(const NcLinear& g, int row) { return g.
 // ------------------------------------------------------------------------------------------------
 // MT tiles of 16 rows x NB tiles of 16 weight rows per workgroup; wave w takes K-steps [its share] of 64 bytes.
 template <typename T, int MT, int NB>
-__global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g) {
+__global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g, int split_bits) {
     __shared__ v4f red[4][MT * NB][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int split = (int)blockIdx.z % g.splits, batch = (int)blockIdx.z / g.splits;
+    const int split = (int)blockIdx.z & (g.splits - 1);
     Span sp;
-    if (!find_span(g, blockIdx.y, batch, 16 * MT, sp)) return;
+    if (!find_span(g, blockIdx.y, (int)blockIdx.z >> split_bits, 16 * MT, sp)) return;
     const int n0 = blockIdx.x * 16 * NB, frow = lane & 15, piece = lane >> 4;
     const uint8_t* wp[NB];
     const uint8_t* ap[MT];
@@ -176,7 +177,7 @@ __global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g) {
 #pragma unroll
     for (int i = 0; i < MT; i++) {
         const int m = sp.row0 + min(16 * i + frow, sp.rows - 1);
-        ap[i] = (const uint8_t*)((const T*)g.a + sp.a_off + a_row(g, m) * g.lda) + piece * 16;
+        ap[i] = (const uint8_t*)((const T*)g.a + sp.a_off + (int64_t)m * g.lda) + piece * 16;
     }
     v4f acc[MT][NB];
 #pragma unroll
@@ -184,16 +185,15 @@ __global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g) {
 #pragma unroll
         for (int j = 0; j < NB; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-    const int steps = g.K * (int)sizeof(T) / 64, shares = 4 * g.splits, share = 4 * split + wave;
-    const int s0 = (int)((int64_t)steps * share / shares), s1 = (int)((int64_t)steps * (share + 1) / shares);
-    constexpr int U = MT * NB >= 16 ? 2 : 4;
+    const int steps = g.K * (int)sizeof(T) / 64, share = 4 * split + wave, s0 = steps * share >> (split_bits + 2), s1 = steps * (share + 1) >> (split_bits + 2);
+    constexpr int U = 4;
     auto step = [&](int s, auto unroll) {
         constexpr int N_ = decltype(unroll)::value;
         v4i wf[N_][NB], af[N_][MT];
 #pragma unroll
         for (int u = 0; u < N_; u++) {
 #pragma unroll
-            for (int j = 0; j < NB; j++) wf[u][j] = __builtin_nontemporal_load((const v4i*)(wp[j] + (int64_t)(s + u) * 64));
+            for (int j = 0; j < NB; j++) wf[u][j] = *(const v4i*)(wp[j] + (int64_t)(s + u) * 64);
 #pragma unroll
             for (int i = 0; i < MT; i++) af[u][i] = *(const v4i*)(ap[i] + (int64_t)(s + u) * 64);
         }
@@ -230,7 +230,10 @@ __global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g) {
 // are in flight while one is multiplied.  Past the end of K the loads are issued all the same (into stages nobody reads any more), so
 // that the barrier counts the same number of loads in every step.
 //
-// What bounds it: the loads.  A compute unit takes some 35 bytes per clock straight into LDS (4096^3, 128 x 256: 88 us of loads alone, 62 of
+// Up to 64 rows it is a stream of the weight; the few-rows kernel, with both operands in registers, read every activation from the L2 once per 32
+// columns and waited for each batch of its loads (64 x 12352 x 2048: 32.5 us, 17 of them without the activations).
+//
+// What bounds it on many rows: the loads.  A compute unit takes some 35 bytes per clock straight into LDS (4096^3, 128 x 256: 88 us of loads alone, 62 of
 // products, 105 of both), which is why the widest tile that fills the chip is the one to take.  4096^3 140 -> 117 us, 1792 x 12352 x 2048
 // 120 -> 95 (954 TFLOP/s; the library's own product 90-95), 1792 x 2048 x 4096 41 -> 33: most of it by the epilogue, which cost 15 us per
 // round of tiles where its stores take 3.
@@ -263,8 +266,8 @@ __device__ __forceinline__ void tile_load(const void* base, uint32_t bytes, uint
     __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000), (lds_ptr_t)st, 16, lane_off, k_off, 0, 0);
 }
 
-template <typename T, int BM, int BN, int WM, int WN, int STAGES>
-__global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, int tiles_m, int tiles_n, uint32_t a_bytes) {
+template <typename T, int BM, int BN, int WM, int WN, int STAGES, bool FEW>
+__global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, int tiles_m, int tiles_n, int split_bits, uint32_t a_bytes) {
     constexpr int NW = WM * WN, WTM = BM / WM / 16, WTN = BN / WN / 16, STAGE = (BM + BN) * 128, A_P = BM / 8 / NW, W_P = BN / 8 / NW;
     // s_waitcnt vmcnt(loads of the STAGES - 2 youngest steps) lgkmcnt(0)
     constexpr int FLIGHT = (STAGES - 2) * (A_P + W_P), FIRST = FLIGHT + (A_P + W_P) / 2, WAIT = 0x0070 | (FLIGHT & 15) | ((FLIGHT >> 4) << 14);
@@ -277,17 +280,24 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
         tile_order(blockIdx.x, tiles_m, tiles_n, tm, tn);
     }
     Span sp;
-    if (!find_span(g, tm, blockIdx.y, BM, sp)) return;
+    const int split = (int)blockIdx.y & (g.splits - 1);
+    if (!find_span(g, tm, (int)blockIdx.y >> split_bits, BM, sp)) return;
     const int n0 = tn * BN;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / WN, wn = wave % WN, frow = lane & 15, piece = lane >> 4;
     // staging: piece i of this wave is the 1 KB block (wave + NW i) of its operand's part of the stage; this lane's row inside an 8-row
     // block, and the global chunk that belongs in its LDS slot
     const int sub = lane >> 3, gch = (lane & 7) ^ sub ^ (wave & 1);
-    const int rd_lo = frow * 128 + (((2 * piece) ^ TILE_SWZ(frow)) << 4), rd_hi = frow * 128 + (((2 * piece + 1) ^ TILE_SWZ(frow)) << 4);
-    const uint32_t row_a = (uint32_t)(g.lda * sizeof(T)), row_w = (uint32_t)(g.ldw * sizeof(T)), k_bytes = (uint32_t)(g.K * sizeof(T));
-    const T* const A = (const T*)g.a + sp.a_off;
-    const T* const W = (const T*)g.w + sp.w_off;
+    // (the chunks of a lane's row that the halves of a step take; the same for both operands)
+    const int rd_lo = frow * 128 + (((FEW ? piece : 2 * piece) ^ TILE_SWZ(frow)) << 4), rd_hi = frow * 128 + (((FEW ? 4 + piece : 2 * piece + 1) ^ TILE_SWZ(frow)) << 4);
+    const uint32_t row_a = (uint32_t)(g.lda * sizeof(T)), row_w = (uint32_t)(g.ldw * sizeof(T));
+    // this workgroup's share of the summed index, in half steps of 64 bytes, and the steps that hold it
+    const int halves = g.K * (int)sizeof(T) / 64, h0 = halves * split >> split_bits, h1 = halves * (split + 1) >> split_bits;
+    const int steps = halves / 2, k0 = h0 / 2, ksteps = (h1 + 1) / 2 - k0;
+    const uint8_t* const A = (const uint8_t*)((const T*)g.a + sp.a_off) + k0 * 128;
+    const uint8_t* const W = (const uint8_t*)((const T*)g.w + sp.w_off + (int64_t)n0 * g.ldw) + k0 * 128;
+    a_bytes -= k0 * 128;
+    const uint32_t w_bytes = (uint32_t)(min(g.N - n0, BN) - 1) * row_w + (uint32_t)(steps - k0) * 128;
     uint32_t vo_a[A_P], vo_w[W_P];
 #pragma unroll
     for (int i = 0; i < A_P; i++) {
@@ -296,15 +306,19 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
     }
 #pragma unroll
     for (int i = 0; i < W_P; i++) {
-        const int r = n0 + 8 * (wave + NW * i) + sub;
-        vo_w[i] = r < g.N ? (uint32_t)r * row_w + gch * 16 : TILE_OOB;
+        const int r = 8 * (wave + NW * i) + sub;
+        vo_w[i] = n0 + r < g.N ? (uint32_t)r * row_w + gch * 16 : TILE_OOB;
     }
-    const int ksteps = k_bytes / 128;
-    v4f acc[WTM][WTN];
+    // FEW: the sum in four chains, a quarter of the share each: the same additions in the same order as in linear_few_kernel, so that a row's
+    // result does not depend on which of the kernels a batch of up to 64 rows took.
+    constexpr int CHAINS = FEW ? 4 : 1;
+    v4f acc[CHAINS][WTM][WTN];
 #pragma unroll
-    for (int i = 0; i < WTM; i++)
+    for (int c = 0; c < CHAINS; c++)
 #pragma unroll
-        for (int j = 0; j < WTN; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < WTM; i++)
+#pragma unroll
+            for (int j = 0; j < WTN; j++) acc[c][i][j] = v4f{0.f, 0.f, 0.f, 0.f};
     // A step has two halves (the low and the high 64 bytes of K of a lane's 128-byte row).  While the low half multiplies, the fragments of the
     // high half are read; then every wave has read all of its stage, the waves meet, and while the high half multiplies, the low fragments of
     // the next step are read: neither the barrier nor an LDS read is ever waited for with the matrix cores idle.  The stage that was read is
@@ -316,15 +330,18 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
         asm volatile("" ::: "memory");
     };
     constexpr int LOADS = A_P + W_P, EARLY = LOADS / 2, PRODUCTS = WTM * WTN, READS = WTM + WTN;
-    const uint32_t w_bytes = (uint32_t)(g.N - 1) * row_w + k_bytes;
     auto load = [&](int i, int k_off, uint8_t* st) {
         if (i < A_P) tile_load(A, a_bytes, st + i * NW * 1024, vo_a[i], k_off);
         else tile_load(W, w_bytes, st + BM * 128 + (i - A_P) * NW * 1024, vo_w[i - A_P], k_off);
     };
+    // 16-row tiles of this wave that hold rows at all: the last tile of a group of rows is seldom full
+    const int valid = __builtin_amdgcn_readfirstlane((sp.rows - wm * (BM / WM) + 15) >> 4);
+    enum { ALL, NONE, SOME, READ };           // which products a half step has; READ: none, but the fragments of the next half are read
     v4i al[WTM], ah[WTM], wl[WTN], wh[WTN];
     // half a step: products of (w, a), between them the reads of the other half's fragments and the loads [L0, L1) of a later step
-    auto half = [&](const v4i (&a)[WTM], const v4i (&w)[WTN], v4i (&na)[WTM], v4i (&nw)[WTN], const uint8_t* pa, const uint8_t* pw, int rd, auto l0, auto l1, int k_off, uint8_t* st) {
-        constexpr int L0 = decltype(l0)::value, NL = decltype(l1)::value - L0;
+    auto half = [&](const v4i (&a)[WTM], const v4i (&w)[WTN], v4i (&na)[WTM], v4i (&nw)[WTN], const uint8_t* pa, const uint8_t* pw, int rd, auto l0, auto l1, int k_off,
+                    uint8_t* st, auto rows, auto chain) __attribute__((always_inline)) {
+        constexpr int ROWS = decltype(rows)::value, CHAIN = decltype(chain)::value, L0 = decltype(l0)::value, NL = decltype(l1)::value - L0;
 #pragma unroll
         for (int j = 0; j < WTN; j++)
 #pragma unroll
@@ -335,7 +352,7 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
                     if (p == 0) {
 #pragma unroll
                         for (int r = 0; r < READS; r++)
-                            if (r * PRODUCTS / READS / 2 == n) {
+                            if (ROWS != NONE && r * PRODUCTS / READS / 2 == n) {
                                 if (r == 0) nw[0] = *(const v4i*)(pw + rd);
                                 else if (r <= WTM) na[r - 1] = *(const v4i*)(pa + (r - 1) * 2048 + rd);
                                 else nw[r - WTM] = *(const v4i*)(pw + (r - WTM) * 2048 + rd);
@@ -344,7 +361,7 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
                         for (int r = 0; r < NL; r++)
                             if ((2 * r + 1) * PRODUCTS / (2 * NL) == n) load(L0 + r, k_off, st);
                     }
-                    mma_in_place<T>(acc[i][j], w[j], a[i], p);
+                    if (ROWS == ALL || (ROWS == SOME && i < valid)) mma_in_place<T>(acc[CHAIN][i][j], w[j], a[i], p);
                 }
     };
     const int wa = wm * (BM / WM) * 128, ww = BM * 128 + wn * (BN / WN) * 128;
@@ -360,26 +377,52 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
     for (int i = 0; i < WTM; i++) al[i] = *(const v4i*)(lds + wa + i * 2048 + rd_lo);
 #pragma unroll
     for (int j = 1; j < WTN; j++) wl[j] = *(const v4i*)(lds + ww + j * 2048 + rd_lo);
-    int cur = 0, prev = (STAGES - 1) * STAGE;     // byte offsets of the stage being read and of the one before it
-    for (int kt = 0; kt < ksteps; kt++) {
-        const uint8_t* st = lds + cur;
-        const int next = cur + STAGE == STAGES * STAGE ? 0 : cur + STAGE;
-        const int k1 = kt + STAGES - 1 < ksteps ? (kt + STAGES - 1) * 128 : 0, k2 = kt + STAGES < ksteps ? (kt + STAGES) * 128 : 0;
-        half(al, wl, ah, wh, st + wa, st + ww, rd_hi, std::integral_constant<int, EARLY>{}, std::integral_constant<int, LOADS>{}, k1, lds + prev + wave * 1024);
+    int kt = 0, cur = 0, prev = (STAGES - 1) * STAGE;     // the step; byte offsets of the stage being read and of the one before it
+    auto low = [&](auto rows, auto chain) __attribute__((always_inline)) {
+        const int k1 = kt + STAGES - 1 < ksteps ? (kt + STAGES - 1) * 128 : 0;
+        half(al, wl, ah, wh, lds + cur + wa, lds + cur + ww, rd_hi, std::integral_constant<int, EARLY>{}, std::integral_constant<int, LOADS>{}, k1,
+             lds + prev + wave * 1024, rows, chain);
         meet();
-        half(ah, wh, al, wl, lds + next + wa, lds + next + ww, rd_lo, std::integral_constant<int, 0>{}, std::integral_constant<int, EARLY>{}, k2, lds + cur + wave * 1024);
-        prev = cur, cur = next;
+    };
+    auto high = [&](auto rows, auto chain) __attribute__((always_inline)) {
+        const int next = cur + STAGE == STAGES * STAGE ? 0 : cur + STAGE, k2 = kt + STAGES < ksteps ? (kt + STAGES) * 128 : 0;
+        half(ah, wh, al, wl, lds + next + wa, lds + next + ww, rd_lo, std::integral_constant<int, 0>{}, std::integral_constant<int, EARLY>{}, k2,
+             lds + cur + wave * 1024, rows, chain);
+        prev = cur, cur = next, kt++;
+    };
+    // half steps [from, to) into one chain; a half outside the share is read and not multiplied
+    auto run = [&](int from, int to, auto rows, auto chain) __attribute__((always_inline)) {
+        if (from >= to) return;
+        if (from & 1) high(rows, chain);
+        while (2 * (k0 + kt) + 1 < to) low(rows, chain), high(rows, chain);
+        if (to & 1) low(rows, chain);
+        // the last products: the compiler does not see that an asm statement wrote the accumulators late, and may copy them from here on
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    using std::integral_constant;
+    if constexpr (FEW) {
+        const integral_constant<int, SOME> rows;
+        const int e1 = halves * (4 * split + 1) >> (split_bits + 2), e2 = halves * (4 * split + 2) >> (split_bits + 2), e3 = halves * (4 * split + 3) >> (split_bits + 2);
+        if (h0 & 1) low(integral_constant<int, READ>{}, integral_constant<int, 0>{});
+        run(h0, e1, rows, integral_constant<int, 0>{});
+        run(e1, e2, rows, integral_constant<int, 1>{});
+        run(e2, e3, rows, integral_constant<int, 2>{});
+        run(e3, h1, rows, integral_constant<int, 3>{});
+#pragma unroll
+        for (int i = 0; i < WTM; i++)
+#pragma unroll
+            for (int j = 0; j < WTN; j++) acc[0][i][j] = (acc[0][i][j] + acc[1][i][j]) + (acc[2][i][j] + acc[3][i][j]);
+    } else {
+        if (h0 & 1) low(integral_constant<int, READ>{}, integral_constant<int, 0>{});
+        if (valid >= WTM) run(h0, h1, integral_constant<int, ALL>{}, integral_constant<int, 0>{});
+        else if (valid <= 0) run(h0, h1, integral_constant<int, NONE>{}, integral_constant<int, 0>{});
+        else run(h0, h1, integral_constant<int, SOME>{}, integral_constant<int, 0>{});
     }
     // the loads past the end of K are still landing: they must be done before the workgroup gives its LDS back
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0x0F70);
     __builtin_amdgcn_s_barrier();
-    // (the last products: the compiler does not see that an asm statement wrote the accumulators late)
-    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < WTM; i++)
-#pragma unroll
-        for (int j = 0; j < WTN; j++) asm volatile("" : "+a"(acc[i][j]));
     // out through LDS, each wave its own part: a lane then has eight neighbouring columns of a row, so a store is whole lines, and the code of
     // the epilogues is there once (inlined per accumulator it was 16 times as long, and took longer than its stores)
     constexpr int ROW = BN / WN + 4;                          // floats: rows shifted by four banks
@@ -393,12 +436,13 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
 #pragma unroll
     for (int i = 1; i < 4; i++)
         if (i < g.nseg && n >= g.seg[i - 1].end) sg = g.seg[i], base = g.seg[i - 1].end;
+    if (g.partials) sg = NcSeg{g.N, NC_SEG_F32, g.partials + (int64_t)split * g.M * g.N, g.N, 0.f, 0.f, nullptr}, base = 0;
 #pragma unroll
     for (int i0 = 0; i0 < WTM; i0 += SUBS) {
 #pragma unroll
         for (int i = 0; i < SUBS; i++)
 #pragma unroll
-            for (int j = 0; j < WTN; j++) *(v4f*)(own + (16 * i + frow) * ROW + 16 * j + 4 * piece) = acc[i0 + i][j];
+            for (int j = 0; j < WTN; j++) *(v4f*)(own + (16 * i + frow) * ROW + 16 * j + 4 * piece) = acc[0][i0 + i][j];
 #pragma unroll 1
         for (int r = lane / CHUNKS; r < 16 * SUBS; r += ROWS_AT_ONCE) {
             const int m = wm * (BM / WM) + 16 * i0 + r;
@@ -423,6 +467,8 @@ int check_linear(const NcLinear& l, int dtype) {
     NC_CHECK_ARG(l.M > 0 && l.N > 0 && l.K > 0 && l.K % 32 == 0 && l.batch >= 1, "linear: bad shape M=%d N=%d K=%d batch=%d", l.M, l.N, l.K, l.batch);
     NC_CHECK_ARG(dtype == 0 || dtype == 1, "linear: dtype must be 0 (bfloat16) or 1 (float)");
     NC_CHECK_ARG(l.lda % (dtype ? 4 : 8) == 0 && l.ldw % (dtype ? 4 : 8) == 0 && l.ldw >= l.K && ((uintptr_t)l.a & 15) == 0 && ((uintptr_t)l.w & 15) == 0, "linear: operands must be 16-byte aligned");
+    NC_CHECK_ARG(l.splits >= 1 && (l.splits & (l.splits - 1)) == 0 && l.splits <= 64 && l.K <= 1 << 20 && (l.splits == 1 || l.partials), "linear: %d shares of %d", l.splits, l.K);
+    NC_CHECK_ARG(!l.partials || (l.batch == 1 && !l.tiles && l.N % 16 == 0), "linear: partial sums of %d columns", l.N);
     for (int i = 0; i < l.nseg; i++)
         NC_CHECK_ARG(l.seg[i].kind == NC_SEG_LOGITS || (l.seg[i].end % 16 == 0 && l.seg[i].ld % 4 == 0), "linear: segments must end at multiples of 16 columns");
     return 0;
@@ -430,37 +476,71 @@ int check_linear(const NcLinear& l, int dtype) {
 
 template <typename T, int MT, int NB>
 int launch_few(const NcLinear& l, int ytiles, hipStream_t s) {
-    hipLaunchKernelGGL((linear_few_kernel<T, MT, NB>), dim3((l.N + 16 * NB - 1) / (16 * NB), ytiles, l.batch * l.splits), dim3(256), 0, s, l);
+    hipLaunchKernelGGL((linear_few_kernel<T, MT, NB>), dim3((l.N + 16 * NB - 1) / (16 * NB), ytiles, l.batch * l.splits), dim3(256), 0, s, l, __builtin_ctz(l.splits));
     NC_CHECK_LAUNCH("linear_few");
     return 0;
 }
 template <typename T>
 int launch_few_t(const NcLinear& l, hipStream_t s) {
-    if (l.tiles) return l.N >= 2048 ? launch_few<T, 1, 2>(l, l.max_tiles, s) : launch_few<T, 1, 1>(l, l.max_tiles, s);
-    if (l.M <= 16) return (int64_t)l.N * l.splits * l.batch >= 16384 ? launch_few<T, 1, 2>(l, 1, s) : launch_few<T, 1, 1>(l, 1, s);
-    if (l.M <= 32) return launch_few<T, 2, 2>(l, 1, s);
-    // (64 rows, K = 2048: N = 32768 54 us with four column tiles per workgroup against 66 with two, N = 7808 32 against 19)
-    return l.N >= 16384 ? launch_few<T, 4, 4>(l, (l.M + 63) / 64, s) : launch_few<T, 4, 2>(l, (l.M + 63) / 64, s);
+    return l.M <= 16 ? launch_few<T, 1, 1>(l, 1, s) : l.M <= 32 ? launch_few<T, 2, 2>(l, 1, s) : launch_few<T, 4, 2>(l, (l.M + 63) / 64, s);
 }
-template <typename T, int BM, int BN, int WM, int WN, int STAGES>
+template <typename T, int BM, int BN, int WM, int WN, int STAGES, bool FEW>
 int launch_tiled(const NcLinear& l, hipStream_t s) {
     static std::atomic<uint64_t> done{0};
     constexpr int LDS = (BM + BN) * 128 * STAGES;
-    const void* fn = (const void*)linear_tiled_kernel<T, BM, BN, WM, WN, STAGES>;
+    const void* fn = (const void*)linear_tiled_kernel<T, BM, BN, WM, WN, STAGES, FEW>;
     if (int rc = reserve_dynamic_lds(fn, LDS, done)) return rc;
     const int tm = l.tiles ? l.max_tiles : (l.M + BM - 1) / BM, tn = (l.N + BN - 1) / BN;
     // rows of A this launch may reach: all of them (a gathered row index is below M / a_div)
     const int64_t a_rows = l.a_rows ? (l.M + l.a_div - 1) / l.a_div : l.M;
     const int64_t a_bytes = ((a_rows - 1) * l.lda + l.K) * (int64_t)sizeof(T);
-    NC_CHECK_ARG(a_bytes < (1ll << 31) && (int64_t)l.N * l.ldw * (int64_t)sizeof(T) < (1ll << 31), "linear: operand past 2 GiB");
-    hipLaunchKernelGGL((linear_tiled_kernel<T, BM, BN, WM, WN, STAGES>), dim3(tm * tn, l.batch), dim3(64 * WM * WN), LDS, s, l, tm, tn, (uint32_t)a_bytes);
+    NC_CHECK_ARG(a_bytes < (1ll << 31) && BN * l.ldw * (int64_t)sizeof(T) < (1ll << 31), "linear: operand past 2 GiB");
+    hipLaunchKernelGGL((linear_tiled_kernel<T, BM, BN, WM, WN, STAGES, FEW>), dim3(tm * tn, l.batch * l.splits), dim3(64 * WM * WN), LDS, s, l, tm, tn,
+                       __builtin_ctz(l.splits), (uint32_t)a_bytes);
     NC_CHECK_LAUNCH("linear_tiled");
     return 0;
 }
-// tile shapes: 1 = 64 x 128 (two workgroups per compute unit), 2 = 128 x 256, 3 = 128 x 128
+// tile shapes: 1 = 64 x 128 (two workgroups per compute unit), 2 = 128 x 256, 3 = 128 x 128, 4 = 64 x 64 (two), 5 = 32 x 64 (two),
+// 6 = 32 x 32 (two)
+constexpr int SHAPES = 6, SHAPE_ROWS[SHAPES + 1] = {0, 64, 128, 128, 64, 32, 32}, SHAPE_COLS[SHAPES + 1] = {0, 128, 256, 128, 64, 64, 32};
 template <typename T>
 int launch_tiled_shape(const NcLinear& l, int shape, hipStream_t s) {
-    return shape == 1 ? launch_tiled<T, 64, 128, 2, 2, 3>(l, s) : shape == 2 ? launch_tiled<T, 128, 256, 2, 4, 3>(l, s) : launch_tiled<T, 128, 128, 2, 4, 3>(l, s);
+    if (l.few) {
+        if (shape == 4) return launch_tiled<T, 64, 64, 2, 2, 4, true>(l, s);
+        if (shape == 5) return launch_tiled<T, 32, 64, 1, 4, 6, true>(l, s);
+        if (shape == 6) return launch_tiled<T, 32, 32, 2, 2, 8, true>(l, s);
+    }
+    switch (shape) {
+        case 1: return launch_tiled<T, 64, 128, 2, 2, 3, false>(l, s);
+        case 2: return launch_tiled<T, 128, 256, 2, 4, 3, false>(l, s);
+        case 3: return launch_tiled<T, 128, 128, 2, 4, 3, false>(l, s);
+        case 4: return launch_tiled<T, 64, 64, 2, 2, 4, false>(l, s);
+        case 5: return launch_tiled<T, 32, 64, 1, 4, 6, false>(l, s);
+        default: return launch_tiled<T, 32, 32, 2, 2, 8, false>(l, s);
+    }
+}
+
+// us at K = 2048 (bf16) or 1024 (fp32), tenths: what a launch takes per round of tiles over the compute units, and beside the rounds.  A tile of
+// bf16 costs its loads, one of fp32 its products, where narrow tiles lose less.
+constexpr int ROUND_COST[2][SHAPES + 1] = {{0, 125, 270, 185, 90, 60, 50}, {0, 320, 1200, 620, 175, 100, 70}}, BASE_COST[2][SHAPES + 1] = {{0, 10, 0, 0, 10, 25, 25}, {0, 30, 0, 0, 30, 40, 40}};
+int64_t shape_tiles(const NcLinear& l, int shape) {
+    return (int64_t)((l.M + SHAPE_ROWS[shape] - 1) / SHAPE_ROWS[shape]) * ((l.N + SHAPE_COLS[shape] - 1) / SHAPE_COLS[shape]) * l.batch * l.splits;
+}
+// The shape with the least rounds times cost.  Few rows are a stream of the weight, which the narrow tiles with the most loads in flight read
+// best.  Measured, us, 64x128 / 128x256 / 128x128 / 64x64 / 32x64 / 32x32: bf16, K = 2048: 1792 x 2048 21 / 25 / 17.6, 1792 x 12352
+// 118 / 94 / 116, 700 x 4096 22 / 27 / 17.5 / 23 / 30, 333 x 2048 13 / 25 / 16 / 9.9 / 12, 80 x 2048 13 / 24 / 16 / 8.9 / 7.8 / 7.3; up to 64
+// rows, the last three and linear_few_kernel: 64 x 4096 12.1 / 9.9 / 8.7, 15.6, 64 x 12288 17.2 / 19.6 / 22, 28, 16 x 12288 16.0 / 13.6 / 14.7,
+// 16.7, 16 x 32768 34 / 31 / 36, 41.  fp32, K = 1024: 1792 x 4096 127 / 124 / 128 / 122 / 136, 333 x 4096 37 / 120 / 64 / 38 / 35, 80 x 4096
+// 35 / 92 / 50 / 22 / 15, 64 x 4096 23 / 15.3 / 11.6, 17.6.
+int choose_shape(const NcLinear& l, int dtype) {
+    const int cus = nc_cu_count();
+    int shape = 0;
+    int64_t best = 0;
+    for (int i = SHAPES; i >= (l.M <= NC_FEW_ROWS ? 4 : 1); i--) {
+        const int64_t cost = (shape_tiles(l, i) + cus - 1) / cus * ROUND_COST[dtype][i] + BASE_COST[dtype][i];
+        if (!shape || cost < best) best = cost, shape = i;
+    }
+    return shape;
 }
 
 double linear_units(const NcLinear& l, int dtype, bool few) {
@@ -470,38 +550,41 @@ double linear_units(const NcLinear& l, int dtype, bool few) {
 int64_t linear_tag(const NcLinear& l) { return ((int64_t)l.N << 32) | (uint32_t)l.K; }
 }  // namespace
 
-int nc_linear_few_splits(int M, int N, int K) {
-    const int nb = M <= 16 ? 16 : 32;
-    const int wgs = (N + nb - 1) / nb;
+int nc_linear_splits(int dtype, int M, int N, int K) {
     int splits = 1;
-    while (splits < 8 && wgs * splits < 384 && K / (splits * 2) >= 256) splits *= 2;
+    if (M <= NC_FEW_ROWS) {
+        const int nb = M <= 16 ? 16 : 32, wgs = (N + nb - 1) / nb;
+        while (splits < 8 && wgs * splits < 384 && K / (splits * 2) >= 256) splits *= 2;
+    } else if (dtype && K % 64 == 0) {
+        // fp32 tiles that leave compute units without one: a workgroup for each, unless a share becomes so short that its sums are more bytes
+        // than its weight (333 x 1024 x 5120: 152 us in one piece, 45 in four).  bf16 sums of many rows stay one chain, whatever the tile and
+        // the number of rows.
+        const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
+        while (splits < 8 && tiles * splits * 2 <= nc_cu_count() && K / (splits * 2) >= 512) splits *= 2;
+    }
     return splits;
 }
 
-int nc_launch_linear_few(int dtype, const NcLinear& l, hipStream_t s, int cls) {
+int nc_launch_linear_few(int dtype, const NcLinear& l, hipStream_t s) {
     if (int rc = check_linear(l, dtype)) return rc;
-    NC_CHECK_ARG(!l.tiles || l.tile_rows == NC_GROUP_TILE_FEW, "linear: group tiles of %d rows", l.tile_rows);
-    NC_CHECK_ARG(l.splits >= 1 && (l.splits == 1 || l.partials), "linear: split sums need a buffer");
-    NcProfScope prof(cls, linear_units(l, dtype, true), s, linear_tag(l));
+    NC_CHECK_ARG(!l.tiles, "linear: groups of rows are the tiled kernel's");
+    NcProfScope prof(NC_CLS_LINEAR, linear_units(l, dtype, true), s, linear_tag(l));
     return dtype ? launch_few_t<float>(l, s) : launch_few_t<bf16_t>(l, s);
 }
 
 int nc_launch_linear_tiled(int dtype, const NcLinear& l, hipStream_t s, int cls, int shape) {
     if (int rc = check_linear(l, dtype)) return rc;
-    NC_CHECK_ARG(!l.partials && l.K % 64 == 0, "linear: the tiled kernel takes whole K-steps and finishes its sums");
-    NcProfScope prof(cls, linear_units(l, dtype, false), s, linear_tag(l));
-    if (!shape) {
-        // rounds of tiles over the compute units, times what a tile takes of one.  bf16, us at K = 2048: 11 / 30 / 18 (64 x 128, 128 x 256,
-        // 128 x 128): a tile's loads, not its products.  1792 rows: N = 2048 21 / 25 / 17.6, N = 4096 38 / 29 / 34, N = 12352 118 / 94 / 116;
-        // 500 rows, N = 4096: 15 / 25 / 16.  fp32 is bound by its products, where narrow tiles lose nothing (1792 x 4096 x 2048: 238 / 236 / 241).
-        const int cus = nc_cu_count(), unit[3] = {dtype ? 10 : 11, dtype ? 38 : 30, dtype ? 19 : 18}, bm[3] = {64, 128, 128}, bn[3] = {128, 256, 128};
-        int64_t best = 0;
-        for (int i = 0; i < 3; i++) {
-            const int64_t tiles = (int64_t)((l.M + bm[i] - 1) / bm[i]) * ((l.N + bn[i] - 1) / bn[i]) * l.batch, cost = (tiles + cus - 1) / cus * unit[i];
-            if (!shape || cost < best) best = cost, shape = i + 1;
-        }
-        if (l.tiles) shape = l.tile_rows == 64 ? 1 : 2;
-    }
-    if (l.tiles) NC_CHECK_ARG(l.tile_rows == (shape == 1 ? 64 : 128), "linear: group tiles of %d rows", l.tile_rows);
+    NC_CHECK_ARG(l.K % 64 == 0 && l.splits <= l.K / 64 && shape >= 0 && shape <= SHAPES, "linear: the tiled kernel takes whole K-steps");
+    NcProfScope prof(cls, linear_units(l, dtype, !l.tiles ? l.M <= NC_FEW_ROWS : l.tile_rows == NC_GROUP_TILE_FEW), s, linear_tag(l));
+    if (!shape) shape = !l.tiles ? choose_shape(l, dtype) : l.tile_rows == 32 ? 5 : l.tile_rows == 64 ? 1 : 2;
+    if (l.tiles) NC_CHECK_ARG(l.tile_rows == SHAPE_ROWS[shape], "linear: group tiles of %d rows", l.tile_rows);
     return dtype ? launch_tiled_shape<float>(l, shape, s) : launch_tiled_shape<bf16_t>(l, shape, s);
+}
+
+// Up to 16 rows of few columns (times shares) the few-rows kernel: its workgroups of 16 columns are one or two per compute unit, and their four
+// waves share the summed index, which there is the launch (us, against the best tile: bf16, K = 2048: N = 2048 7.2 / 8.2, 4096 7.6 / 8.3, 6144
+// 10.2 / 8.5; fp32, K = 1024: 2048 6.9 / 10.7, 6144 10.4 / 10.9, 16384 21 / 17.4).  Same sums.
+int nc_launch_linear(int dtype, const NcLinear& l, hipStream_t s) {
+    const bool few = l.M <= 16 && (int64_t)l.N * l.batch * l.splits <= (dtype ? 8192 : 4096) && !l.tiles;
+    return few || l.K % 64 ? nc_launch_linear_few(dtype, l, s) : nc_launch_linear_tiled(dtype, l, s);
 }

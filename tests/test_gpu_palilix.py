@@ -62,18 +62,31 @@ def test_linear_kernels(dtype, kind):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("kernel", (3, 4, 5))
+@pytest.mark.parametrize("kernel", (3, 4, 5, 6, 7, 8))
 def test_tiles_at_their_edges(kernel, dtype):
     """One row and column group less than a tile, a tile, one more; sums of one, two and three K-steps and more than the ring of stages holds."""
     say(f"tile edges, kernel {kernel}, {dtype}")
     g = torch.Generator().manual_seed(5)
     steps = 64 if dtype == torch.bfloat16 else 32
-    for M, N, K in [(63, 112, 1), (64, 128, 2), (65, 144, 3), (127, 240, 4), (128, 256, 5), (129, 272, 7), (257, 528, 4)]:
+    for M, N, K in [(1, 16, 1), (31, 48, 2), (33, 80, 9), (63, 112, 1), (64, 128, 2), (65, 144, 3), (127, 240, 4), (128, 256, 5), (129, 272, 7), (257, 528, 4)]:
         K = -(-K * steps // 64) * 64
         a, w = torch.randn(M, K, generator=g).to(dtype), (torch.randn(N, K, generator=g) / K ** 0.5).to(dtype)
         got = ops.stack_linear(a.to(DEV), w.to(DEV), kernel=kernel).cpu()
         tol = 1e-2 if dtype == torch.bfloat16 else 2e-5       # one rounding to bf16 is 2^-9 of values up to about 4; fp32 sums of up to 448 terms
         assert torch.allclose(got.double(), a.double() @ w.double().T, rtol=tol, atol=tol), (M, N, K)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_few_rows_have_the_same_sums_in_every_kernel(dtype):
+    """Up to 64 rows a result does not depend on the kernel or the tile: the same additions in the same order, to the bit (sums of one K-step, of
+    steps that do not divide by four, and of chains that begin in the middle of one)."""
+    say(f"same sums, {dtype}")
+    g = torch.Generator().manual_seed(6)
+    for M, N, K in [(1, 16, 64), (5, 80, 192), (16, 144, 320), (17, 64, 704), (33, 208, 1088), (64, 320, 1792)]:
+        a, w = torch.randn(M, K, generator=g).to(DEV, dtype), torch.randn(N, K, generator=g).to(DEV, dtype)
+        want = ops.stack_linear(a, w, kind=3, kernel=1)
+        for kernel in (6, 7, 8):
+            assert torch.equal(ops.stack_linear(a, w, kind=3, kernel=kernel), want), (M, N, K, kernel)
 
 
 # ------------------------------------------------------------------------------------------------ whole prompts
