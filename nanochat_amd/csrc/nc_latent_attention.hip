@@ -149,6 +149,94 @@ __global__ __launch_bounds__(256) void latent_simple_kernel(NcLatentGeom g, cons
     }
 }
 
+// ------------------------------------------------------------------------------------------------ latent space, 32-bit, many query rows
+// 16 query rows (row = token * heads + head of one batch row) per workgroup, keys 64 at a time, on v_mfma_f32_16x16x4_f32: a lane supplies 16
+// bytes of row lane % 16 from piece lane / 16, which is four instructions (which dimension or key a lane's values stand for does not matter as
+// long as both operands agree).
+//   scores   wave w: keys 16 (w % 4) .. + 15, half w / 4 of the row; the halves meet in LDS
+//   softmax  wave w: rows 2 w and 2 w + 1, lane = key
+//   sums     wave w: columns 16 (w + 8 c) .. + 15 of the latent
+// What bounds latent_simple_kernel is the L2: every row reads all its keys twice (8 heads, rank 512, 333 tokens: 4 GB, 188 us).  Here 16 rows share
+// them: 69 us.
+constexpr int KEYS32 = 64, WAVES32 = 8, S32_PITCH = KEYS32 + 4;
+__device__ __forceinline__ v4f mma32(v4f a, v4f b, v4f c) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);
+    return c;
+}
+template <int NT>
+__global__ __launch_bounds__(64 * WAVES32) void latent32_kernel(NcLatentGeom g, const float* __restrict__ q_lat, const float* __restrict__ cache,
+                                                                const int32_t* __restrict__ seqlens, float* __restrict__ out, int groups) {
+    extern __shared__ __align__(16) float qs[];               // 16 rows of the query, then scores (two halves), weights
+    __shared__ float corr_of[16], sum_of[16];
+    const int rw = g.rank_p + g.rot_p, pitch = rw + 4, rows = g.T * g.heads, lane = threadIdx.x & 63, col = lane & 15, piece = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x / groups, r0 = 16 * (blockIdx.x % groups);
+    float *const sc = qs + 16 * pitch, *const ps = sc + 2 * 16 * S32_PITCH;
+    const int pos = seqlens[b], last = min(pos + (min(r0 + 15, rows - 1)) / g.heads, g.Tmax - 1);
+    for (int u = threadIdx.x; u < 16 * rw / 4; u += 64 * WAVES32) {
+        const int r = u / (rw / 4), d = 4 * (u % (rw / 4));
+        *(v4f*)(qs + r * pitch + d) = *(const v4f*)(q_lat + ((int64_t)b * rows + min(r0 + r, rows - 1)) * rw + d);
+    }
+    const float* keys = cache + (int64_t)b * g.Tmax * rw;
+    v4f acc[NT];
+#pragma unroll
+    for (int c = 0; c < NT; c++) acc[c] = v4f{0.f, 0.f, 0.f, 0.f};
+    float m_run[2] = {LA_M_FLOOR, LA_M_FLOOR}, l_run[2] = {0.f, 0.f};
+    __syncthreads();
+    for (int k0 = 0; k0 <= last; k0 += KEYS32) {
+        {                                                      // (a key past the last one is read as the last: masked below, finite)
+            const int kt = wave & 3, steps = rw / 16, s0 = (wave >> 2) * (steps / 2), s1 = wave >> 2 ? steps : steps / 2;
+            const float *kr = keys + (int64_t)min(k0 + 16 * kt + col, last) * rw + 4 * piece, *qr = qs + col * pitch + 4 * piece;
+            v4f s = v4f{0.f, 0.f, 0.f, 0.f};
+            for (int i = s0; i < s1; i++) s = mma32(*(const v4f*)(qr + 16 * i), *(const v4f*)(kr + 16 * i), s);
+#pragma unroll
+            for (int r = 0; r < 4; r++) sc[((wave >> 2) * 16 + 4 * piece + r) * S32_PITCH + 16 * kt + col] = s[r];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const int r = 2 * wave + i, see = min(pos + min(r0 + r, rows - 1) / g.heads, g.Tmax - 1);
+            const float s = k0 + lane <= see ? (sc[r * S32_PITCH + lane] + sc[(16 + r) * S32_PITCH + lane]) * g.scale : LA_MASKED;
+            const float m_new = fmaxf(m_run[i], wave_max(s)), corr = expf(m_run[i] - m_new), p = k0 + lane <= see ? expf(s - m_new) : 0.f;
+            ps[r * S32_PITCH + lane] = p;
+            l_run[i] = l_run[i] * corr + wave_sum(p);
+            m_run[i] = m_new;
+            if (lane == 0) corr_of[r] = corr;
+        }
+        __syncthreads();
+        v4f corr;
+#pragma unroll
+        for (int r = 0; r < 4; r++) corr[r] = corr_of[4 * piece + r];
+#pragma unroll
+        for (int c = 0; c < NT; c++) acc[c] *= corr;
+#pragma unroll
+        for (int k = 0; k < KEYS32; k += 16) {
+            const v4f p = *(const v4f*)(ps + col * S32_PITCH + k + 4 * piece);
+            const float* vr[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) vr[j] = keys + (int64_t)min(k0 + k + 4 * piece + j, last) * rw + 16 * wave + col;
+#pragma unroll
+            for (int c = 0; c < NT; c++)
+                if (16 * (wave + WAVES32 * c) < g.rank_p) acc[c] = mma32(p, v4f{vr[0][128 * c], vr[1][128 * c], vr[2][128 * c], vr[3][128 * c]}, acc[c]);
+        }
+        // (the scores of the next block are written before the barrier that follows them, by waves that are past their softmax; the weights after it)
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+        if (lane == 0) sum_of[2 * wave + i] = l_run[i];
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < NT; c++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int row = 4 * piece + r, at = 16 * (wave + WAVES32 * c) + col;
+            if (at < g.rank_p && r0 + row < rows) out[((int64_t)b * rows + r0 + row) * g.rank_p + at] = acc[c][r] / sum_of[row];
+        }
+}
+// From 64 query rows of a sequence on: fewer leave compute units to latent_simple_kernel's one workgroup per row.
+int latent32_lds(const NcLatentGeom& g) { return (16 * (g.rank_p + g.rot_p + 4) + 3 * 16 * S32_PITCH) * 4; }
+bool latent32_ok(const NcLatentGeom& g) { return g.T * g.heads >= 64 && g.T >= 8 && g.rank_p <= 128 * 4 && g.rank_p % 16 == 0 && g.rot_p % 16 == 0 && latent32_lds(g) <= 60 * 1024; }
+
 // ------------------------------------------------------------------------------------------------ latent space, matrix cores
 // A workgroup of eight waves takes 16 query rows (row = token * heads + head of one batch row) and a share of the keys, 32 keys at a time
 // through LDS:
@@ -605,7 +693,14 @@ int nc_launch_latent_attention(int dtype, const NcLatentGeom& g, const void* q_l
     }
     NC_CHECK_ARG(g.rank_p <= 256 * SIMPLE_COLS, "latent_attention: a latent of %d values is not supported", g.rank_p);
     const int bytes = (g.rank_p + g.rot_p + 256) * 4;
-    if (dtype)
+    if (dtype && latent32_ok(g)) {
+        const int groups = (g.T * g.heads + 15) / 16, lds = latent32_lds(g);
+#define GO32(NT) hipLaunchKernelGGL((latent32_kernel<NT>), dim3(groups * g.B), dim3(64 * WAVES32), lds, s, g, (const float*)q_lat, (const float*)cache, seqlens, (float*)out_lat, groups)
+        if (g.rank_p <= 128) GO32(1);
+        else if (g.rank_p <= 256) GO32(2);
+        else GO32(4);
+#undef GO32
+    } else if (dtype)
         hipLaunchKernelGGL((latent_simple_kernel<float>), dim3(rows), dim3(256), bytes, s, g, (const float*)q_lat, (const float*)cache, seqlens, (float*)out_lat);
     else
         hipLaunchKernelGGL((latent_simple_kernel<bf16_t>), dim3(rows), dim3(256), bytes, s, g, (const bf16_t*)q_lat, (const bf16_t*)cache, seqlens,

@@ -5,8 +5,8 @@
 // or o_t itself, in fp32, where a design norms all heads together.
 //
 // Two forms:
-//   step     token by token, the state in registers (decode, short portions, 32-bit);
-//   chunked  (bf16, long portions) the sequence in chunks of C tokens: the chunks' own sums  KV_c = sum_j decay^(n-1-j) k_j v_j^T  side by
+//   step     token by token, the state in registers (decode, short portions);
+//   chunked  (long portions) the sequence in chunks of C tokens: the chunks' own sums  KV_c = sum_j decay^(n-1-j) k_j v_j^T  side by
 //            side, a scan over the chunks  S <- decay^n S + KV_c, and per chunk  o_i = decay^(i+1) S^T q_i + sum_(j<=i) decay^(i-j) (q_i . k_j) v_j.
 // Everything that enters the recurrence is fp32.  On the matrix cores an fp32 operand goes in as two bf16 terms (hi + lo, 16 bits together):
 // turned q and k, decayed k, the state, and the decayed scores; products of two lo terms are left out.
@@ -409,9 +409,170 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void r
         }
 }
 
+// ------------------------------------------------------------------------------------------------ chunked, 32-bit
+// The same three kernels in fp32 throughout (v_mfma_f32_16x16x4_f32: a lane supplies row or column lane % 16 of the summed index lane / 16 and
+// holds rows 4 (lane / 16) .. + 3 of column lane % 16), chunks of 32 tokens, heads of up to 128 dimensions.  What bounds the step kernel is its
+// chain, 1.5 us a token in one workgroup per head; here a prompt is three launches whose workgroups are (chunk, head).  8 heads of 128 x 128, 333
+// tokens: 502 -> 41 us.
+constexpr int C32 = 32, THREADS32 = 512, PAD32 = 16;
+__device__ __forceinline__ v4f mma32(float a, float b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// rows [0, n) of `src` (leading dimension ld), turned and scaled, into LDS rows of width + PAD32 floats; zero rows behind
+template <typename F>
+__device__ __forceinline__ void stage32(float* dst, int width, int n, F value) {
+    for (int u = threadIdx.x; u < C32 * width; u += THREADS32) {
+        const int j = u / width, d = u % width;
+        dst[j * (width + PAD32) + d] = j < n ? value(j, d) : 0.f;
+    }
+}
+
+// KV [dim][vdim] of one chunk and head; waves take 16 x 16 tiles in turn
+__global__ __launch_bounds__(THREADS32) void retention32_kv_kernel(NcRetentionGeom g, const float* __restrict__ proj, int ldp, const float* __restrict__ decay,
+                                                                   const float* __restrict__ rope, int rope_len, const int32_t* __restrict__ seqlens,
+                                                                   float* __restrict__ kv, int chunks) {
+    extern __shared__ __align__(16) float sh32[];
+    const int DK = g.dim_p, DV = g.vdim_p, KP = DK + PAD32, VP = DV + PAD32;
+    float *const ks = sh32, *const vs = sh32 + C32 * KP;
+    const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z, lane = threadIdx.x & 63, half = g.rot_dims / 2, pos0 = seqlens[b];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t0 = chunk * C32, n = min(C32, g.T - t0), col = lane & 15, row = lane >> 4;
+    const float l2 = decay[2 * h + 1];
+    const float* base = proj + ((int64_t)b * g.T + t0) * ldp;
+    stage32(ks, DK, n, [&](int j, int d) {
+        const float2* turn = (const float2*)rope + (int64_t)min(pos0 + t0 + j, rope_len - 1) * half;
+        return turned(base + (int64_t)j * ldp + (g.heads + h) * DK, d, half, turn) * g.k_scale * exp2f((float)(n - 1 - j) * l2);
+    });
+    stage32(vs, DV, n, [&](int j, int d) { return base[(int64_t)j * ldp + 2 * g.heads * DK + h * DV + d]; });
+    __syncthreads();
+    float* dst = kv + (((int64_t)b * chunks + chunk) * g.heads + h) * DK * DV;
+    const int tiles_v = DV / 16;
+    for (int tile = wave; tile < DK / 16 * tiles_v; tile += THREADS32 / 64) {
+        const int d0 = 16 * (tile / tiles_v), v0 = 16 * (tile % tiles_v);
+        v4f acc = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < C32; j += 4) acc = mma32(ks[(j + row) * KP + d0 + col], vs[(j + row) * VP + v0 + col], acc);
+#pragma unroll
+        for (int r = 0; r < 4; r++) dst[(d0 + 4 * row + r) * DV + v0 + col] = acc[r];
+    }
+}
+
+// The state in front of every chunk, and the one behind the last
+__global__ __launch_bounds__(256) void retention32_scan_kernel(NcRetentionGeom g, const float* __restrict__ decay, const int32_t* __restrict__ seqlens,
+                                                               const float* __restrict__ kv, float* __restrict__ prefix, const float* __restrict__ state_in,
+                                                               float* __restrict__ state_out, int chunks) {
+    const int h = blockIdx.y, b = blockIdx.z, plane = g.dim_p * g.vdim_p, e = 4 * ((int)blockIdx.x * 256 + (int)threadIdx.x);
+    if (e >= plane) return;
+    const int64_t so = ((int64_t)b * g.heads + h) * plane + e, step = (int64_t)g.heads * plane, at = ((int64_t)b * chunks * g.heads + h) * plane + e;
+    v4f S = v4f{0.f, 0.f, 0.f, 0.f};
+    if (seqlens[b] > 0) S = *(const v4f*)(state_in + so);
+    const float l2 = decay[2 * h + 1], full = exp2f((float)C32 * l2), tail = exp2f((float)(g.T - (chunks - 1) * C32) * l2);
+#pragma unroll 4
+    for (int c = 0; c < chunks; c++) {
+        const v4f add = *(const v4f*)(kv + at + c * step);
+        *(v4f*)(prefix + at + c * step) = S;
+        S = S * (c + 1 < chunks ? full : tail) + add;
+    }
+    *(v4f*)(state_out + so) = S;
+}
+
+// The outputs of one chunk and head: a wave takes 16 columns of all rows
+__global__ __launch_bounds__(THREADS32) void retention32_out_kernel(NcRetentionGeom g, const float* __restrict__ proj, int ldp, const float* __restrict__ decay,
+                                                                    const float* __restrict__ rope, int rope_len, const int32_t* __restrict__ seqlens,
+                                                                    const float* __restrict__ prefix, int chunks, float eps, float* __restrict__ out, int ldo) {
+    extern __shared__ __align__(16) float sh32[];
+    __shared__ float red[THREADS32 / 64][C32];
+    constexpr int PP = C32 + 4;
+    const int DK = g.dim_p, DV = g.vdim_p, KP = DK + PAD32, VP = DV + PAD32;
+    float *const qs = sh32, *const ks = qs + C32 * KP, *const vs = ks + C32 * KP, *const ps = vs + C32 * VP;
+    const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z, lane = threadIdx.x & 63, half = g.rot_dims / 2, pos0 = seqlens[b];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), t0 = chunk * C32, n = min(C32, g.T - t0), col = lane & 15, row = lane >> 4;
+    const float l2 = decay[2 * h + 1];
+    const float* base = proj + ((int64_t)b * g.T + t0) * ldp;
+    const float2* turns = (const float2*)rope;
+    stage32(qs, DK, n, [&](int j, int d) { return turned(base + (int64_t)j * ldp + h * DK, d, half, turns + (int64_t)min(pos0 + t0 + j, rope_len - 1) * half); });
+    stage32(ks, DK, n, [&](int j, int d) {
+        return turned(base + (int64_t)j * ldp + (g.heads + h) * DK, d, half, turns + (int64_t)min(pos0 + t0 + j, rope_len - 1) * half) * g.k_scale;
+    });
+    stage32(vs, DV, n, [&](int j, int d) { return base[(int64_t)j * ldp + 2 * g.heads * DK + h * DV + d]; });
+    __syncthreads();
+    if (wave < 4) {                              // decayed scores, one 16 x 16 tile per wave
+        const int i0 = 16 * (wave >> 1), j0 = 16 * (wave & 1);
+        v4f s = v4f{0.f, 0.f, 0.f, 0.f};
+        for (int d = 0; d < DK; d += 4) s = mma32(qs[(i0 + col) * KP + d + row], ks[(j0 + col) * KP + d + row], s);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int i = i0 + 4 * row + r, j = j0 + col;
+            ps[i * PP + j] = j <= i ? s[r] * exp2f((float)(i - j) * l2) : 0.f;
+        }
+    }
+    // what came before the chunk
+    const int v0 = 16 * wave;                    // this wave's columns
+    const bool mine = v0 < DV;
+    v4f o[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
+    if (mine && (chunk > 0 || pos0 > 0)) {
+        const float* S = prefix + (((int64_t)b * chunks + chunk) * g.heads + h) * DK * DV + v0 + col;
+        for (int d0 = 0; d0 < DK; d0 += 16) {
+            float s[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) s[k] = S[(d0 + 4 * k + row) * DV];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                o[0] = mma32(qs[col * KP + d0 + 4 * k + row], s[k], o[0]);
+                o[1] = mma32(qs[(16 + col) * KP + d0 + 4 * k + row], s[k], o[1]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[i][r] *= exp2f((float)(16 * i + 4 * row + r + 1) * l2);
+    }
+    __syncthreads();
+    float ss[2][4] = {};
+    if (mine) {
+#pragma unroll
+        for (int j = 0; j < C32; j += 4) {
+            const float v = vs[(j + row) * VP + v0 + col];
+            o[0] = mma32(ps[col * PP + j + row], v, o[0]);
+            o[1] = mma32(ps[(16 + col) * PP + j + row], v, o[1]);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int t = 16 * i + 4 * row + r;
+                ss[i][r] = o[i][r] * o[i][r];
+                if (g.raw && t < n) g.raw[(((int64_t)b * g.T + t0 + t) * g.heads + h) * DV + v0 + col] = o[i][r];
+            }
+    }
+    if (g.raw) return;                           // (uniform)
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            float v = ss[i][r];
+#pragma unroll
+            for (int m = 8; m; m >>= 1) v += __shfl_xor(v, m);
+            if (col == 0) red[wave][16 * i + 4 * row + r] = v;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int t = 16 * i + 4 * row + r;
+            if (t >= n || !mine) continue;
+            float sum = 0.f;
+#pragma unroll
+            for (int w = 0; w < THREADS32 / 64; w++) sum += red[w][t];
+            const float inv = 1.0f / sqrtf(sum / (float)g.vdim + eps), z = base[(int64_t)t * ldp + 2 * g.heads * DK + (g.heads + h) * DV + v0 + col];
+            out[((int64_t)b * g.T + t0 + t) * ldo + h * DV + v0 + col] = o[i][r] * inv * (z * sigmoid_f32(z));
+        }
+}
+
 constexpr int CHUNK_MIN_TOKENS = 32;
+// Tokens per chunk, 0: the step kernel.  (fp32 takes the chunks as far as both operands of a chunk fit the 64 KB of LDS that need no asking for.)
 int chunk_size(int dtype, const NcRetentionGeom& g) {
-    if (dtype != 0 || g.T < CHUNK_MIN_TOKENS) return 0;
+    if (g.T < CHUNK_MIN_TOKENS) return 0;
+    if (dtype) return g.dim_p <= 128 && g.vdim_p <= 128 && g.dim_p % 16 == 0 && g.vdim_p % 16 == 0 ? C32 : 0;
     if ((g.dim_p == 64 || g.dim_p == 128) && (g.vdim_p == 64 || g.vdim_p == 128 || g.vdim_p == 256)) return 64;
     if (g.dim_p == 256 && (g.vdim_p == 128 || g.vdim_p == 256)) return 32;
     return 0;
@@ -473,6 +634,17 @@ int nc_launch_retention(int dtype, const NcRetentionGeom& g, const void* proj, i
     // bytes: the projections in, the outputs, and four passes over the chunks' states (written, scanned in and out, read)
     NcProfScope prof(NC_CLS_RETENTION, (double)g.B * g.heads * (g.T * (2.0 * g.dim_p + 3.0 * g.vdim_p) * 2 + 16.0 * ((g.T + C - 1) / C) * g.dim_p * g.vdim_p), s,
                      g.T);
+    if (dtype) {
+        const int chunks = (g.T + C - 1) / C, plane = g.dim_p * g.vdim_p;
+        const int kv_lds = C32 * (g.dim_p + g.vdim_p + 2 * PAD32) * 4, out_lds = C32 * (2 * g.dim_p + g.vdim_p + 3 * PAD32 + C32 + 4) * 4;
+        float *kv = (float*)workspace, *prefix = kv + (int64_t)g.B * chunks * g.heads * plane;
+        hipLaunchKernelGGL(retention32_kv_kernel, dim3(chunks, g.heads, g.B), dim3(THREADS32), kv_lds, s, g, (const float*)proj, ldp, decay, rope, rope_len, seqlens, kv, chunks);
+        hipLaunchKernelGGL(retention32_scan_kernel, dim3((plane + 1023) / 1024, g.heads, g.B), dim3(256), 0, s, g, decay, seqlens, kv, prefix, state_in, state_out, chunks);
+        hipLaunchKernelGGL(retention32_out_kernel, dim3(chunks, g.heads, g.B), dim3(THREADS32), out_lds, s, g, (const float*)proj, ldp, decay, rope, rope_len, seqlens, prefix,
+                           chunks, eps, (float*)out, ldo);
+        NC_CHECK_LAUNCH("retention_chunked");
+        return 0;
+    }
     const bf16_t* p = (const bf16_t*)proj;
     bf16_t* o = (bf16_t*)out;
 #define CHUNKED(K, V, CC) \

@@ -99,6 +99,16 @@ def test_whole_prompt(name, dtype):
         check(run(case_model(name, dtype), toks, [n]), oracle_logits(name, n), dtype, f"{name}, {n} tokens")
 
 
+@pytest.mark.parametrize("name", ["odd", "wide"])
+def test_32_bit_portions_at_the_edges_of_their_kernels(name):
+    """32 tokens to a chunk of the recurrence, 16 query rows and 64 keys to a block of the latent attention: one less, as many, one more, alone and
+    behind other portions."""
+    say(f"32-bit portions, {name}")
+    for cuts in ([31], [32], [33], [64], [65], [7, 32, 33], [64, 8, 63]):
+        n = sum(cuts)
+        check(run(case_model(name, torch.float32), tokens(CASES[name], n), cuts), oracle_logits(name, n), torch.float32, f"{name}, portions {cuts}")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_residual_stream_after_every_run(dtype):
     say(f"layer by layer, {dtype}")
