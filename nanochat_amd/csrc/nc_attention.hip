@@ -37,20 +37,53 @@
 // MODE 0: q is given, the new tokens are already in the cache.  MODE 1: FUSED as described above.  MODE 2: q and the new key and value
 // are given finished (flash_attn_with_kvcache(q, k_cache, v_cache, k=, v=), nanochat/flash_attention.py:139-185): the workgroup
 // copies its heads of them into LDS, appends key and value to the cache and attends like MODE 1.
+#define NC_DEAL_MAX_ROWS 512          // lengths that fit the smallest kernel's merge area (4 waves x PART_STRIDE words)
+static_assert(4 * PART_STRIDE >= NC_DEAL_MAX_ROWS, "row lengths");
 template <int G, int MODE, int HP>
 __global__ __launch_bounds__(256) void attn_partial_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ k_cache,
                                                            bf16_t* __restrict__ v_cache, const int32_t* __restrict__ cache_seqlens,
                                                            int window_left, int seqlens_include_new, bf16_t* __restrict__ out,
                                                            float* __restrict__ partials, uint32_t* __restrict__ counters,
                                                            uint32_t* __restrict__ amax_ws, int T, int H, int Hkv, int Tmax, int nsplit,
-                                                           NcRopeSrc rope, int k_min, const float* __restrict__ extra, int n_extra) {
+                                                           NcRopeSrc rope, int k_min, const float* __restrict__ extra, int n_extra, int deal) {
     constexpr bool FUSED = MODE != 0;                    // the row's own token comes from LDS, not from the cache
     constexpr int KPI = 4 / HP;                          // keys per load instruction
     constexpr int TASKS = (G + 2) * HP;                  // FUSED: per head the G query heads, then the new key and value
     __shared__ float merge[4][HP * G][PART_STRIDE];
     __shared__ float fresh[FUSED ? TASKS : 1][128];
     __shared__ int last_flag;
-    const int split = blockIdx.x, hp = blockIdx.y, row = blockIdx.z;
+    const int split = blockIdx.x, hp = blockIdx.y;
+    int row = blockIdx.z, dealt_pos = 0;
+    if (MODE == 2 && deal > 0) {
+        // Rows of unequal length, dealt by length: the longest to the first round of workgroups over the compute units (`deal` rows), the next
+        // ones to the second round in the opposite order, and so on, so that every unit gets about the same number of keys.  128 rows of 64 to
+        // 2040 keys, 16 query heads on 4: 79 -> 63 us; rows of about one length see one barrier of it.
+        int* const lens = (int*)&merge[0][0][0];
+        const int rows = gridDim.z, most = window_left < 0 ? 0x7ffffffe : min(window_left, 0x7ffffffd) + 1, first = min(cache_seqlens[0], most);
+        bool close = true;                               // no length is an eighth off the first one: not worth the count
+        for (int i = threadIdx.x; i < (rows + 3 & ~3); i += 256) {
+            const int n = i < rows ? cache_seqlens[i] : INT_MIN;         // (the padding is longer than no row, whatever lengths are passed)
+            lens[i] = n;
+            close &= i >= rows || abs(min(n, most) - first) <= first / 8;
+        }
+        if (!__syncthreads_and(close)) {
+            const int round = row / deal, rank_wanted = round & 1 ? min((round + 1) * deal, rows) - 1 - row % deal : row;
+            for (int i = threadIdx.x; i < rows; i += 256) {
+                const int mine = min(lens[i], most);
+                int rank = 0;
+#pragma unroll 4
+                for (int j = 0; j < rows; j += 4) {
+                    const int4 o = *(const int4*)(lens + j);
+                    rank += (min(o.x, most) + (j < i) > mine) + (min(o.y, most) + (j + 1 < i) > mine) + (min(o.z, most) + (j + 2 < i) > mine) +
+                            (min(o.w, most) + (j + 3 < i) > mine);          // (longer, or as long and earlier)
+                }
+                if (rank == rank_wanted) last_flag = i;
+            }
+            __syncthreads();
+            row = __builtin_amdgcn_readfirstlane(last_flag);
+        }
+        dealt_pos = __builtin_amdgcn_readfirstlane(lens[row]);
+    }
     const int b = row / T, t = row % T;
     // the wave index as a scalar: everything derived from it (the head tasks of this wave) then branches instead of predicating
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -61,7 +94,7 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(const bf16_t* __restr
     const int n_heads_here = (hp * HP + HP <= Hkv) ? HP : Hkv - hp * HP;
 
     // visible keys [lo, hi]
-    int pos = cache_seqlens[b];
+    int pos = MODE == 2 && deal > 0 ? dealt_pos : cache_seqlens[b];
     if (seqlens_include_new) pos -= T;
     int hi = pos + t;
     if (hi > Tmax - 1) hi = Tmax - 1;
@@ -451,6 +484,9 @@ static int launch_attention_impl(const bf16_t* q, const NcRopeSrc* rope, int mod
     float* parts = (float*)partials;
     const int hp = (force_splits > 0 || nsplit > 1) ? 1 : pick_heads_per_wg(B, T, Hkv);
     dim3 grid(nsplit, hp == 2 ? (Hkv + 1) / 2 : Hkv, B * T), block(256);
+    // rows per round of workgroups where the kernel deals them by length (it keeps the lengths where the merge of its waves goes later)
+    int deal = nc_cu_count() / (int)(grid.x * grid.y);
+    if (mode != 2 || nsplit > 1 || deal < 1 || B <= deal || B > NC_DEAL_MAX_ROWS || max_keys < 1024) deal = 0;      // (512 keys: 34 -> 38 us)
     const NcRopeSrc none{};
     const NcRopeSrc& rs = rope ? *rope : none;
 #define LAUNCH_GMH(GG, MM, HH)                                                                                                     \
@@ -458,11 +494,11 @@ static int launch_attention_impl(const bf16_t* q, const NcRopeSrc* rope, int mod
         if (timed)                                                                                                                 \
             hipExtLaunchKernelGGL((attn_partial_kernel<GG, MM, HH>), grid, block, 0, s, ev0, ev1, 0, q, k_cache, v_cache,         \
                                   cache_seqlens, window_left, seqlens_include_new, out, parts, counters, amax_ws, T, H, Hkv, Tmax, \
-                                  nsplit, rs, k_min, extra, n_extra);                                                              \
+                                  nsplit, rs, k_min, extra, n_extra, deal);                                                        \
         else                                                                                                                       \
             hipLaunchKernelGGL((attn_partial_kernel<GG, MM, HH>), grid, block, 0, s, q, k_cache, v_cache, cache_seqlens,           \
                                window_left, seqlens_include_new, out, parts, counters, amax_ws, T, H, Hkv, Tmax, nsplit, rs,       \
-                               k_min, extra, n_extra);                                                                             \
+                               k_min, extra, n_extra, deal);                                                                       \
     } while (0)
 #define LAUNCH_GH(GG, HH)                          \
     do {                                           \

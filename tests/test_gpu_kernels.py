@@ -1117,3 +1117,37 @@ def test_measurement_probes_run_and_report_their_work(ops):
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     assert flops.value == cus * 8 * 32 * 100 * 65536.0
     assert (clocks[::2] > 0).all()
+
+
+@pytest.mark.parametrize("lengths", ["spread", "equal but one", "empty and full", "ties"])
+@pytest.mark.parametrize("B,H,Hkv", [(65, 8, 4), (141, 4, 2), (300, 1, 1)])
+def test_attention_append_of_rows_dealt_by_length(ops, B, H, Hkv, lengths):
+    """More rows than one round of workgroups over the compute units: the kernel deals them by length, and every row is still its own."""
+    say(f"dealt rows B={B} H={H} Hkv={Hkv} {lengths}")
+    g = torch.Generator(device=DEV).manual_seed(B)
+    Tmax = 1030
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g, device=DEV).bfloat16()
+    q, k, v, kc, vc = normal(B, 1, H, 128), normal(B, 1, Hkv, 128), normal(B, 1, Hkv, 128), normal(B, Tmax, Hkv, 128), normal(B, Tmax, Hkv, 128)
+    n = torch.randint(0, Tmax, (B,), generator=g, device=DEV, dtype=torch.int32)
+    if lengths == "equal but one":
+        n.fill_(900)[B // 2] = 3
+    elif lengths == "empty and full":
+        n[::2], n[1::2] = 0, Tmax - 1
+    elif lengths == "ties":
+        n = n // 300 * 300
+    for window in (-1, 1027):
+        kd, vd = kc.clone(), vc.clone()
+        got = ops.decode_attention_append(q, k, v, kd, vd, n, window_left=window)
+        keys, values = kc.clone(), vc.clone()
+        at = torch.arange(B, device=DEV), n.long()
+        keys[at], values[at] = k[:, 0], v[:, 0]
+        assert torch.equal(kd, keys) and torch.equal(vd, values)
+        j = torch.arange(Tmax, device=DEV)[None, :]
+        seen = (j <= n[:, None]) & ((window < 0) | (n[:, None] - j <= window))
+        keys, values = (t.float().repeat_interleave(H // Hkv, dim=2).transpose(1, 2).contiguous() for t in (keys, values))
+        p = ((keys @ q.float().transpose(1, 2).transpose(2, 3).contiguous())[..., 0] * 128 ** -0.5).masked_fill(~seen[:, None], -math.inf).softmax(-1)
+        want = (p[:, :, None] @ values).transpose(1, 2)
+        # the result is one rounding to bf16 (2^-9) of sums of up to 1030 products of fp32 weights and bf16 values
+        assert torch.allclose(got.float(), want, rtol=1e-2, atol=1e-2), (window, (got.float() - want).abs().max().item())
