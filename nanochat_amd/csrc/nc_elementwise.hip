@@ -326,6 +326,96 @@ __global__ __launch_bounds__(256) void mix_norm_vec_kernel(bf16_t* __restrict__ 
     if (bump && threadIdx.x == 0) bump[blockIdx.x] += bump_by;
 }
 
+// The same rows for the many of a prompt, a wave to a row.  What bounds a thousand workgroups that each end with a maximum for the amax site is
+// that site: a look and an atomic per workgroup.  With four rows to a workgroup there are a quarter of them, and no barrier stands in front of
+// the rescale (1792 rows of 1664 columns with an amax site: 10.0 -> 8.5 us, and 12.2 -> 9.8 between a prompt's other kernels; 8 or 16 rows to a
+// workgroup: 9.3 and 10.9).  The lane holds the elements that threads lane, lane + 64, lane + 128 and lane + 192 of the kernel above hold and
+// sums them in that order: the same bits.
+__global__ __launch_bounds__(256) void mix_norm_rows_kernel(bf16_t* __restrict__ x, const bf16_t* __restrict__ add, const bf16_t* __restrict__ x0,
+                                                            const float* __restrict__ resid_lambda, const float* __restrict__ x0_lambda,
+                                                            const float* __restrict__ backout_lambda, const bf16_t* __restrict__ backout_src,
+                                                            bf16_t* __restrict__ backout_save, bf16_t* __restrict__ xn_out, int rows, int cols,
+                                                            uint32_t* __restrict__ amax_ws, int32_t* __restrict__ bump, int bump_by) {
+    __shared__ float red[4];
+    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    float am = 0.f;
+    if (row < rows) {
+        const size_t base = (size_t)row * cols;
+        const bool writes_x = add || resid_lambda || backout_lambda;
+        const bf16_t* zsrc = resid_lambda ? x0 : (backout_lambda ? backout_src : nullptr);
+        const float rl = rbf(resid_lambda ? *resid_lambda : 0.f), xl = rbf(x0_lambda ? *x0_lambda : 0.f), bl = rbf(backout_lambda ? *backout_lambda : 0.f);
+        uint4 xv[4], av[4], zv[4];
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const int c = (w * 64 + lane) * 8;
+            if (c < cols) {
+                xv[w] = *(const uint4*)(x + base + c);
+                if (add) av[w] = *(const uint4*)(add + base + c);
+                if (zsrc) zv[w] = *(const uint4*)(zsrc + base + c);
+            }
+        }
+        float v[4][8], ss[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const int c = (w * 64 + lane) * 8;
+            if (c < cols) {
+                const uint32_t xw[4] = {xv[w].x, xv[w].y, xv[w].z, xv[w].w};
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[w][2 * j] = bf16_lo(xw[j]), v[w][2 * j + 1] = bf16_hi(xw[j]);
+                if (add) {
+                    const uint32_t aw[4] = {av[w].x, av[w].y, av[w].z, av[w].w};
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        v[w][2 * j] = rbf(v[w][2 * j] + bf16_lo(aw[j]));
+                        v[w][2 * j + 1] = rbf(v[w][2 * j + 1] + bf16_hi(aw[j]));
+                    }
+                }
+                if (backout_save)
+                    *(uint4*)(backout_save + base + c) = make_uint4(pack_bf16(v[w][0], v[w][1]), pack_bf16(v[w][2], v[w][3]),
+                                                                    pack_bf16(v[w][4], v[w][5]), pack_bf16(v[w][6], v[w][7]));
+                const uint32_t zw[4] = {zv[w].x, zv[w].y, zv[w].z, zv[w].w};
+                if (resid_lambda) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        v[w][2 * j] = rbf(rbf(rl * v[w][2 * j]) + rbf(xl * bf16_lo(zw[j])));
+                        v[w][2 * j + 1] = rbf(rbf(rl * v[w][2 * j + 1]) + rbf(xl * bf16_hi(zw[j])));
+                    }
+                } else if (backout_lambda) {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        v[w][2 * j] = rbf(v[w][2 * j] - rbf(bl * bf16_lo(zw[j])));
+                        v[w][2 * j + 1] = rbf(v[w][2 * j + 1] - rbf(bl * bf16_hi(zw[j])));
+                    }
+                }
+                if (writes_x)
+                    *(uint4*)(x + base + c) = make_uint4(pack_bf16(v[w][0], v[w][1]), pack_bf16(v[w][2], v[w][3]),
+                                                         pack_bf16(v[w][4], v[w][5]), pack_bf16(v[w][6], v[w][7]));
+#pragma unroll
+                for (int j = 0; j < 8; j++) ss[w] += v[w][j] * v[w][j];
+            }
+        }
+        float total = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) total += wave_sum(ss[w]);
+        const float rstd = 1.0f / sqrtf(total / (float)cols + RMS_EPS);
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const int c = (w * 64 + lane) * 8;
+            if (c < cols) {
+                uint32_t o[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    o[j] = pack_bf16(v[w][2 * j] * rstd, v[w][2 * j + 1] * rstd);
+                    am = amax_fold(amax_fold(am, bf16_lo(o[j])), bf16_hi(o[j]));
+                }
+                *(uint4*)(xn_out + base + c) = make_uint4(o[0], o[1], o[2], o[3]);
+            }
+        }
+        if (bump && lane == 0) bump[row] += bump_by;
+    }
+    block_amax_commit(am, amax_ws, red);
+}
+
 // out = relu(h)^2, elementwise bf16, plus amax (gpt.py:139)
 __global__ __launch_bounds__(256) void relu2_kernel(const bf16_t* __restrict__ h, bf16_t* __restrict__ out, int64_t n,
                                                     uint32_t* __restrict__ amax_ws) {
@@ -558,7 +648,13 @@ static int launch_mix_norm_impl(bf16_t* x, const bf16_t* add, NcPartialSrc padd,
         if (padd.parts) hipLaunchKernelGGL((mix_norm_vec_kernel<NVV, true>), dim3(rows), dim3(256), 0, s, MIX_ARGS);      \
         else hipLaunchKernelGGL((mix_norm_vec_kernel<NVV, false>), dim3(rows), dim3(256), 0, s, MIX_ARGS);                \
     } while (0)
-    if (aligned && cols <= 2048) MIX_LAUNCH(1);
+    // a wave to a row once that many workgroups would queue at the amax site; a wave takes a row's 512-column pieces one after the other, so the
+    // line lies higher for wider rows (256 columns: 512 rows 4.5 -> 3.7 us; 1664: 1024 rows 6.7 against 7.2, 1792 rows 10.0 -> 8.5), and without a
+    // site a workgroup per row is the faster one at any count (1664 columns, 8192 rows: 22.5 against 25.5)
+    if (aligned && cols <= 2048 && !padd.parts && amax_ws && rows >= 512 + 256 * ((cols + 511) / 512))
+        hipLaunchKernelGGL(mix_norm_rows_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, x, add, x0, resid_lambda, x0_lambda, backout_lambda,
+                           backout_src, backout_save, xn_out, rows, cols, amax_ws, bump, bump_by);
+    else if (aligned && cols <= 2048) MIX_LAUNCH(1);
     else if (aligned && cols <= 4096) MIX_LAUNCH(2);
     else if (aligned && cols <= 8192) MIX_LAUNCH(4);
     else {

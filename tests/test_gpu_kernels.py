@@ -1151,3 +1151,31 @@ def test_attention_append_of_rows_dealt_by_length(ops, B, H, Hkv, lengths):
         want = (p[:, :, None] @ values).transpose(1, 2)
         # the result is one rounding to bf16 (2^-9) of sums of up to 1030 products of fp32 weights and bf16 values
         assert torch.allclose(got.float(), want, rtol=1e-2, atol=1e-2), (window, (got.float() - want).abs().max().item())
+
+
+@pytest.mark.parametrize("cols", [8, 512, 520, 1664, 2048])
+@pytest.mark.parametrize("over", [0, 1, 7])
+def test_mix_norm_of_many_rows_has_the_bits_of_a_row_alone(ops, cols, over):
+    """Rows with an amax site go a wave to a row from 512 + 256 * ceil(cols / 512) of them on: same bits as row by row, and their maximum."""
+    rows = 512 + 256 * ((cols + 511) // 512) + over
+    say(f"mix_norm rows={rows} cols={cols}")
+    g = torch.Generator(device=DEV).manual_seed(cols + over)
+    x, add, other = (torch.randn(rows, cols, generator=g, device=DEV).bfloat16() for _ in range(3))
+    lam = [torch.tensor([v], device=DEV) for v in (0.9, 0.3)]
+    null = ops.C.c_void_p(0)
+
+    def ptr(t):
+        return null if t is None else ops.C.c_void_p(t.data_ptr())
+    for kind in ("add", "mix", "backout", "plain"):
+        added, mixed, out = add if kind != "plain" else None, other if kind == "mix" else None, other if kind == "backout" else None
+        res = []
+        for amax in (torch.zeros(1, dtype=torch.int32, device=DEV), None):
+            y, xn, saved = x.clone(), torch.empty_like(x), torch.empty_like(x)
+            ops._lib.check(ops._lib.lib().nc_mix_norm(
+                ptr(y), ptr(added), ptr(mixed), ptr(lam[0] if kind == "mix" else None), ptr(lam[1] if kind == "mix" else None),
+                ptr(lam[0] if kind == "backout" else None), ptr(out), ptr(saved), ptr(xn), rows, cols, ptr(amax), ops._stream()))
+            res.append((y, xn, saved))
+            if amax is not None:
+                assert torch.equal(amax.view(torch.float32), xn.abs().max().float().reshape(1))
+        for name, many, alone in zip(("x", "xn", "saved"), *res):
+            assert torch.equal(many, alone), (kind, name)
