@@ -32,6 +32,21 @@ typedef __attribute__((address_space(3))) uint8_t* lds_u8_t;
 #define PF_M_FLOOR (-1.0e20f)  // running maximum (scaled units) before any visible key: far above PF_MASKED * scale, far below any score
 
 __device__ __forceinline__ v8bf as_v8bf(uint4 v) { return __builtin_bit_cast(v8bf, v); }
+// maximum of what this lane and lane ^ 32 hold, without a trip through LDS
+__device__ __forceinline__ float max_of_halves(float v) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+// The K fragments of a sub-block (lane: key `col`, d half hl), all asked for before the first product: left to itself the compiler reads two,
+// waits for them and multiplies, four times over, in a wave that has one other wave beside it at most (with max_of_halves and the first
+// values asked for ahead of the softmax: 1792 queries of 13 heads 32.8 -> 30.6 us, of 16 heads on 4 46.2 -> 43.5, four rows of 13 heads
+// 83.7 -> 79.9, a window of 512 keys 21.1 -> 20.6).  Working out the next sub-block's scores beside this one's weights, with two buffers of
+// keys and values and one barrier per 64 keys, was no faster than the one by one above (32.7 us).
+__device__ __forceinline__ void pf_read_keys(v8bf (&kf)[8], const uint8_t* kt, int col, int hl) {
+#pragma unroll
+    for (int c = 0; c < 8; c++) kf[c] = as_v8bf(*(const uint4*)(kt + col * PF_KPITCH + (16 * c + 8 * hl) * 2));
+    __builtin_amdgcn_sched_barrier(0);
+}
 
 // GS = query heads of one kv head that share a workgroup (1, 2 or 4), KS = waves that share one block of 32 queries and split
 // its keys between them (1 or 2), GS * KS <= 4.  Wave w serves head (w % GS) of the group, key share (w / GS) % KS and the
@@ -166,11 +181,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int r = 0; r < 16; r++) s[r] = 0.f;
         const uint8_t* kt = lds_k + sb * PF_KBYTES;
+        v8bf kf[8];
+        pf_read_keys(kf, kt, col, hl);
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const v8bf kf = as_v8bf(*(const uint4*)(kt + col * PF_KPITCH + (16 * c + 8 * hl) * 2));
-            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[c], s, 0, 0, 0);
-        }
+        for (int c = 0; c < 8; c++) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[c], qf[c], s, 0, 0, 0);
         // ---- mask, online softmax (per lane = per query; the other half of the keys sits in lane ^ 32)
         if (masked) {                      // wave-uniform
 #pragma unroll
@@ -180,10 +194,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 s[r] = vis ? s[r] : PF_MASKED;
             }
         }
+        // the values of the first 16 keys, asked for ahead of the softmax
+        v4s vlo[4], vhi[4];
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) {
+            const lds_u8_t vblk = lds_v3 + sb * PF_VBYTES + vtr_off + 32 * dt * 2;
+            vlo[dt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t)vblk);
+            vhi[dt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t)(vblk + 8 * PF_VPITCH));
+        }
+        __builtin_amdgcn_sched_barrier(0);
         float mx = s[0];
 #pragma unroll
         for (int r = 1; r < 16; r++) mx = fmaxf(mx, s[r]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        mx = max_of_halves(mx);
         // (a sub-block with nothing visible for this lane leaves the maximum where it was: PF_MASKED * sc lies below the floor,
         // and its weights come out as exp2(-huge) = 0)
         // The reference point of the exponentials only follows the maximum when it has moved by more than PF_LAZY (in log2 units)
@@ -215,8 +238,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
             for (int dt = 0; dt < 4; dt++) {
                 const lds_u8_t vblk = lds_v3 + sb * PF_VBYTES + vtr_off + 16 * c2 * PF_VPITCH + 32 * dt * 2;
-                const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t)vblk);
-                const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t)(vblk + 8 * PF_VPITCH));
+                const v4s lo = c2 == 0 ? vlo[dt] : __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t)vblk);
+                const v4s hi = c2 == 0 ? vhi[dt] : __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s_t)(vblk + 8 * PF_VPITCH));
                 const v8bf vf = __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
                 o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[c2], o[dt], 0, 0, 0);
             }
