@@ -393,6 +393,14 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
     // half steps [from, to) into one chain; a half outside the share is read and not multiplied
     auto run = [&](int from, int to, auto rows, auto chain) __attribute__((always_inline)) {
         if (from >= to) return;
+        // The accumulators hold their zeros from here on: left to itself the compiler writes one just in front of its first product, and does not
+        // see that the asm statement is an MFMA, which must not follow the write of its operand by less than a few cycles.
+#pragma unroll
+        for (int i = 0; i < WTM; i++)
+#pragma unroll
+            for (int j = 0; j < WTN; j++) asm volatile("" : "+a"(acc[decltype(chain)::value][i][j]));
+        asm volatile("s_nop 7" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
         if (from & 1) high(rows, chain);
         while (2 * (k0 + kt) + 1 < to) low(rows, chain), high(rows, chain);
         if (to & 1) low(rows, chain);

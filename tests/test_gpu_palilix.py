@@ -109,6 +109,21 @@ def test_32_bit_portions_at_the_edges_of_their_kernels(name):
         check(run(case_model(name, torch.float32), tokens(CASES[name], n), cuts), oracle_logits(name, n), torch.float32, f"{name}, portions {cuts}")
 
 
+@pytest.mark.parametrize("width", [64, 512, 1024])
+@pytest.mark.parametrize("ff", [2048, 2112, 1984])
+def test_32_bit_shares_that_begin_in_the_middle_of_a_step(width, ff):
+    """The output matrix of many rows in four shares of 33 half steps (ff = 2048), of 34, and in two of 64: a share may begin with the second half
+    of a step.  Whole prompts against portions of few rows, which take other kernels."""
+    say(f"shares, width {width}, ff {ff}")
+    cfg = config([(retention(heads=1, dim=64, vdim=64, rot_dims=32), dense(ff=ff))] * 2, width=width, vocab=50)
+    model = build(cfg, weights(cfg, seed=3), torch.float32)
+    for n in (65, 80, 130, 400):
+        toks = tokens(cfg, n)
+        few = run(model, toks, [50] * (n // 50) + ([n % 50] if n % 50 else [])).cpu()
+        for again in range(3):
+            check(run(model, toks, [n]), few, torch.float32, f"{n} rows")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_residual_stream_after_every_run(dtype):
     say(f"layer by layer, {dtype}")
