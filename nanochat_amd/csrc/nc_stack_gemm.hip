@@ -176,8 +176,8 @@ __global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g, int split_b
     }
 #pragma unroll
     for (int i = 0; i < MT; i++) {
-        const int m = sp.row0 + min(16 * i + frow, sp.rows - 1);
-        ap[i] = (const uint8_t*)((const T*)g.a + sp.a_off + (int64_t)m * g.lda) + piece * 16;
+        const int64_t m = a_row(g, sp.row0 + min(16 * i + frow, sp.rows - 1));
+        ap[i] = (const uint8_t*)((const T*)g.a + sp.a_off + m * g.lda) + piece * 16;
     }
     v4f acc[MT][NB];
 #pragma unroll
@@ -490,6 +490,7 @@ int launch_few(const NcLinear& l, int ytiles, hipStream_t s) {
 }
 template <typename T>
 int launch_few_t(const NcLinear& l, hipStream_t s) {
+    if (l.tiles) return l.N >= 2048 ? launch_few<T, 1, 2>(l, l.max_tiles, s) : launch_few<T, 1, 1>(l, l.max_tiles, s);
     return l.M <= 16 ? launch_few<T, 1, 1>(l, 1, s) : l.M <= 32 ? launch_few<T, 2, 2>(l, 1, s) : launch_few<T, 4, 2>(l, (l.M + 63) / 64, s);
 }
 template <typename T, int BM, int BN, int WM, int WN, int STAGES, bool FEW>
@@ -573,10 +574,9 @@ int nc_linear_splits(int dtype, int M, int N, int K) {
     return splits;
 }
 
-int nc_launch_linear_few(int dtype, const NcLinear& l, hipStream_t s) {
+int nc_launch_linear_few(int dtype, const NcLinear& l, hipStream_t s, int cls) {
     if (int rc = check_linear(l, dtype)) return rc;
-    NC_CHECK_ARG(!l.tiles, "linear: groups of rows are the tiled kernel's");
-    NcProfScope prof(NC_CLS_LINEAR, linear_units(l, dtype, true), s, linear_tag(l));
+    NcProfScope prof(cls, linear_units(l, dtype, true), s, linear_tag(l));
     return dtype ? launch_few_t<float>(l, s) : launch_few_t<bf16_t>(l, s);
 }
 
