@@ -102,7 +102,7 @@ inline void nc_linear_seg(NcLinear& l, int end, int kind, void* out, int ld, flo
     l.seg[l.nseg++] = NcSeg{end, kind, out, ld, p0, p1, bias};
 }
 #define NC_TILE_WORDS 5
-#define NC_GROUP_TILE_FEW 32               // rows per group tile where groups have few rows (others: 64 or 128)
+#define NC_GROUP_TILE_FEW 16               // rows per group tile of the few-rows kernel (the tiled one takes up to 32, 64 or 128)
 int nc_launch_linear_few(int dtype, const NcLinear& l, hipStream_t s, int cls = NC_CLS_LINEAR);
 int nc_launch_linear_tiled(int dtype, const NcLinear& l, hipStream_t s, int cls = NC_CLS_LINEAR, int shape = 0);     // shape 0: choose
 int nc_launch_linear(int dtype, const NcLinear& l, hipStream_t s);                                                   // whichever is the faster

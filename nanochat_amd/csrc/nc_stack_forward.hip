@@ -68,9 +68,10 @@ bool expand(int dtype, const nc_stack_mixer& l, const NcLatentGeom& g) {
     if (!nc_latent_expanded_ok(dtype, g) || g.T < 32) return false;
     return (double)g.T * (2.0 * l.rank_p + l.rot_p - 0.5 * (l.dim_p + l.rot_p + l.vdim_p)) > (double)l.rank_p * (l.dim_p + l.vdim_p);
 }
+// Rows of a tile of one expert's pairs.  Calls that may take the few-rows kernel get tiles that it holds, however many pairs an expert has.
 int expert_tile_rows(const nc_stack_layer& l, int M) {
     const int per = M * l.top / l.experts;
-    return per < 32 ? NC_GROUP_TILE_FEW : per < 128 ? 64 : 128;
+    return M <= NC_GROUP_TILE_FEW ? NC_GROUP_TILE_FEW : per < 32 ? 32 : per < 128 ? 64 : 128;
 }
 int expert_max_tiles(const nc_stack_layer& l, int M, int tile_rows) {
     const int pairs = M * l.top;
@@ -286,10 +287,9 @@ int run_experts(int dt, const nc_stack_layer& l, int M, int width_p, const Works
     const int pairs = M * l.top;
     auto grouped = [&](NcLinear& g) {
         g.tiles = w.tiles, g.n_tiles = w.n_tiles, g.max_tiles = r.max_tiles, g.tile_rows = r.tile_rows, g.few = M <= NC_FEW_ROWS || pairs / l.experts < 16, g.w_stride = (int64_t)g.N * g.K;
-        // A row chooses an expert once, so up to 16 rows no group has more than the 16 of the few-rows kernel, which a small launch suits better:
-        // same sums (2 rows, 16 experts, K = 512, N = 2048: 324 us a step against 345 in tiles of 32 rows; 4 rows of 64 experts, K = 1280, 590
-        // against 575)
-        if (M <= 16 && (int64_t)g.max_tiles * g.N <= 32768) return nc_launch_linear_few(dt, g, s, NC_CLS_EXPERTS);
+        // Up to 16 rows a small launch suits the few-rows kernel better: same sums (2 rows, 16 experts, K = 512, N = 2048: 324 us a step against 345
+        // in tiles of 32 rows; 4 rows of 64 experts, K = 1280, 590 against 575)
+        if (r.tile_rows <= NC_GROUP_TILE_FEW && (int64_t)g.max_tiles * g.N <= 32768) return nc_launch_linear_few(dt, g, s, NC_CLS_EXPERTS);
         return nc_launch_linear_tiled(dt, g, s, NC_CLS_EXPERTS);
     };
     NcLinear up = nc_linear(w.h, width_p, l.w_e1, pairs, 2 * l.expert_ff_p, width_p);

@@ -2,6 +2,7 @@
 unequal sequences, slots that are used again, generation through the Engine; both storage types."""
 import functools
 import json
+import math
 
 import pytest
 import torch
@@ -340,6 +341,31 @@ def test_prompts_of_several_rows_at_once(dtype):
         got = torch.cat(outs, dim=1)
         for r, s in enumerate(seqs):
             check(got[r], ref.forward(cfg, w64, s), dtype, f"row {r} of 3, cuts {cuts[:3]}")
+
+
+def spoiled_rows_leave_the_others_alone(cfg, rows, spoiled, dtype):
+    """One token to each of `rows` sequences; those of `spoiled` bring a token whose embedding is NaN: the others' logits are what they are where
+    every sequence is a healthy one, to the bit."""
+    w = weights(cfg, seed=8)
+    w["embed"][0] = math.nan
+    model = build(cfg, w, dtype)
+    healthy = torch.tensor([[1 + r % (cfg["vocab"] - 1)] for r in range(rows)], device=DEV)
+    some = healthy.clone()
+    some[spoiled] = 0
+    want = model.forward_last(healthy, kv_cache=model.new_cache(rows, 4)).clone()
+    got = model.forward_last(some, kv_cache=model.new_cache(rows, 4))
+    rest = [r for r in range(rows) if r not in spoiled]
+    assert torch.isfinite(want).all() and torch.isnan(got[spoiled]).all()
+    assert torch.equal(got[rest], want[rest]), (got[rest] - want[rest]).abs().amax(1).tolist()
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows,spoiled", [(16, [0, 9]), (7, [6]), (2, [0]), (40, [3, 38])])
+def test_rows_of_nan_scores_beside_others_that_share_their_expert(rows, spoiled, dtype):
+    """Whichever experts a row of NaN scores chooses, the pairs of an expert past the first tile of 16 are computed as well."""
+    say(f"NaN rows, 64 experts, {rows} rows, {dtype}")
+    cfg = config([(latent(), moe(experts=64, top=48, ff=40)), (retention(), moe(experts=64, top=6, ff=64))], vocab=50)
+    spoiled_rows_leave_the_others_alone(cfg, rows, spoiled, dtype)
 
 
 def test_a_slot_is_used_again_without_a_trace():
