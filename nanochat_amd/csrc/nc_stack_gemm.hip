@@ -159,7 +159,8 @@ __device__ __forceinline__ int64_t a_row(const NcLinear& g, int row) { return g.
 
 // ------------------------------------------------------------------------------------------------
 // MT tiles of 16 rows x NB tiles of 16 weight rows per workgroup; wave w takes K-steps [its share] of 64 bytes.
-template <typename T, int MT, int NB>
+// U K-steps are asked for at a time.
+template <typename T, int MT, int NB, int U>
 __global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g, int split_bits) {
     __shared__ v4f red[4][MT * NB][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -186,7 +187,6 @@ __global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g, int split_b
         for (int j = 0; j < NB; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
     const int steps = g.K * (int)sizeof(T) / 64, share = 4 * split + wave, s0 = steps * share >> (split_bits + 2), s1 = steps * (share + 1) >> (split_bits + 2);
-    constexpr int U = 4;
     auto step = [&](int s, auto unroll) {
         constexpr int N_ = decltype(unroll)::value;
         v4i wf[N_][NB], af[N_][MT];
@@ -206,6 +206,8 @@ __global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g, int split_b
     };
     int s = s0;
     for (; s + U <= s1; s += U) step(s, std::integral_constant<int, U>{});
+    if constexpr (U == 8)
+        if (s + 4 <= s1) step(s, std::integral_constant<int, 4>{}), s += 4;
     for (; s < s1; s++) step(s, std::integral_constant<int, 1>{});
 
 #pragma unroll
@@ -482,16 +484,22 @@ int check_linear(const NcLinear& l, int dtype) {
     return 0;
 }
 
-template <typename T, int MT, int NB>
+template <typename T, int MT, int NB, int U = 4>
 int launch_few(const NcLinear& l, int ytiles, hipStream_t s) {
-    hipLaunchKernelGGL((linear_few_kernel<T, MT, NB>), dim3((l.N + 16 * NB - 1) / (16 * NB), ytiles, l.batch * l.splits), dim3(256), 0, s, l, __builtin_ctz(l.splits));
+    hipLaunchKernelGGL((linear_few_kernel<T, MT, NB, U>), dim3((l.N + 16 * NB - 1) / (16 * NB), ytiles, l.batch * l.splits), dim3(256), 0, s, l, __builtin_ctz(l.splits));
     NC_CHECK_LAUNCH("linear_few");
     return 0;
 }
 template <typename T>
 int launch_few_t(const NcLinear& l, hipStream_t s) {
-    if (l.tiles) return l.N >= 2048 ? launch_few<T, 1, 2>(l, l.max_tiles, s) : launch_few<T, 1, 1>(l, l.max_tiles, s);
-    return l.M <= 16 ? launch_few<T, 1, 1>(l, 1, s) : l.M <= 32 ? launch_few<T, 2, 2>(l, 1, s) : launch_few<T, 4, 2>(l, (l.M + 63) / 64, s);
+    // One workgroup per compute unit or two wait for their loads, which eight steps at a time halve (bf16, 4 rows, K = 2048, N = 2048 6.6 -> 6.0 us,
+    // K = 4096 10.3 -> 9.2, six experts of 2048 x 2048 and back a step of 255 -> 244; from 16384 columns on 9.5 -> 10.3, and no fp32 launch gains).
+    const int64_t cols = (int64_t)l.N * (l.tiles ? l.max_tiles : l.batch * l.splits);
+    if (l.M <= 16 || l.tiles) {
+        const int y = l.tiles ? l.max_tiles : 1;
+        return sizeof(T) == 2 && cols <= 12288 ? launch_few<T, 1, 1, 8>(l, y, s) : launch_few<T, 1, 1>(l, y, s);
+    }
+    return l.M <= 32 ? launch_few<T, 2, 2>(l, 1, s) : launch_few<T, 4, 2>(l, (l.M + 63) / 64, s);
 }
 template <typename T, int BM, int BN, int WM, int WN, int STAGES, bool FEW>
 int launch_tiled(const NcLinear& l, hipStream_t s) {
@@ -590,10 +598,19 @@ int nc_launch_linear_tiled(int dtype, const NcLinear& l, hipStream_t s, int cls,
     return dtype ? launch_tiled_shape<float>(l, shape, s) : launch_tiled_shape<bf16_t>(l, shape, s);
 }
 
-// Up to 16 rows of few columns (times shares) the few-rows kernel: its workgroups of 16 columns are one or two per compute unit, and their four
-// waves share the summed index, which there is the launch (us, against the best tile: bf16, K = 2048: N = 2048 7.2 / 8.2, 4096 7.6 / 8.3, 6144
-// 10.2 / 8.5; fp32, K = 1024: 2048 6.9 / 10.7, 6144 10.4 / 10.9, 16384 21 / 17.4).  Same sums.
+// The few-rows kernel or a tile: same sums, so only time decides.  In the few-rows kernel four waves share the summed index, which pays where its
+// workgroups of 16 columns are few per compute unit or the whole weight is short; its price is that every workgroup reads every row from the L2.
+// us, few-rows kernel / best tile, by columns (times batch and shares):
+//   bf16, 1 to 4 rows    K = 512: 8192 4.5 / 5.3, 32768 9 / 10      1024: 8192 6.0 / 6.5, 32768 14.2 / 16.5      2048: 4096 6.2 / 8.1, 8192 10.5 / 9.7
+//   bf16, 16 rows        K = 512: 8192 5.0 / 5.4, 32768 11.2 / 10   1024: 8192 6.7 / 6.6, 16384 11.5 / 8.9       4096: 2048 10.9 / 12, 8192 19 / 14.7
+//   bf16, 32 rows        K = 128: 8192 3.4 / 4.0                    512: 8192 5.5 / 5.7, 16384 7.9 / 7.0         1024: 1024 6.8 / 5.7
+//   fp32, 16 rows        K = 512: 8192 7.4 / 7.7, 16384 12.5 / 10.2 2048: 4096 15 / 17.4, 8192 22 / 18           32 rows, 256: 8192 5.6 / 6.2
+bool few_is_faster(const NcLinear& l, int dtype) {
+    const int64_t cols = (int64_t)l.N * l.batch * l.splits, k = l.K / l.splits, weight = cols * k;
+    if (l.M <= 16 && (cols <= 4096 || weight <= (dtype ? 4 << 20 : 8 << 20))) return true;
+    if (l.M <= 4 && !dtype && k <= 1024) return true;
+    return l.M <= 32 && k <= 512 && weight <= 4 << 20;
+}
 int nc_launch_linear(int dtype, const NcLinear& l, hipStream_t s) {
-    const bool few = l.M <= 16 && (int64_t)l.N * l.batch * l.splits <= (dtype ? 8192 : 4096) && !l.tiles;
-    return few || l.K % 64 ? nc_launch_linear_few(dtype, l, s) : nc_launch_linear_tiled(dtype, l, s);
+    return l.K % 64 || few_is_faster(l, dtype) ? nc_launch_linear_few(dtype, l, s) : nc_launch_linear_tiled(dtype, l, s);
 }

@@ -90,6 +90,19 @@ def test_few_rows_have_the_same_sums_in_every_kernel(dtype):
             assert torch.equal(ops.stack_linear(a, w, kind=3, kernel=kernel), want), (M, N, K, kernel)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_whatever_kernel_is_chosen_for_few_rows_has_the_same_sums(dtype):
+    """The choice, on both sides of its borders (rows, columns, length of the sum), against a tile; sums whose quarters are 8, 12, 14 and 23 steps
+    of 64 bytes, that is whole and broken batches of the few-rows kernel."""
+    say(f"chosen kernel, {dtype}")
+    g = torch.Generator().manual_seed(7)
+    for M, N, K in [(1, 48, 1024), (16, 80, 1536), (4, 4112, 1792), (5, 4112, 1024), (4, 8208, 1024), (16, 8208, 512), (17, 8192, 512), (32, 8208, 512), (33, 64, 512), (2, 12304, 2944)]:
+        a, w = torch.randn(M, K, generator=g).to(DEV, dtype), torch.randn(N, K, generator=g).to(DEV, dtype)
+        want = ops.stack_linear(a, w, kind=3, kernel=6)
+        for kernel in (0, 1):
+            assert torch.equal(ops.stack_linear(a, w, kind=3, kernel=kernel), want), (M, N, K, kernel)
+
+
 # ------------------------------------------------------------------------------------------------ whole prompts
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", list(CASES))
