@@ -181,14 +181,18 @@ __device__ __forceinline__ void choose_experts_of(const NcRoute& r, int m, int l
         sum += e < r.experts ? s[i] : 0.f;
     }
     sum = wave_sum(sum);
+    // A score that is not a number comes after every other one, but before what must not be chosen: lanes past the experts and earlier choices.
+    // The choices of a row are thus distinct experts whatever its scores; its weights are NaN by the sum.
+#pragma unroll
+    for (int i = 0; i < PER; i++)
+        if (!(s[i] >= 0.f)) s[i] = lane + 64 * i < r.experts ? -1.f : -2.f;
     float chosen_sum = 0.f, mine = 0.f;       // lane k keeps the score of choice k (top <= 64)
     for (int k = 0; k < r.top; k++) {
-        float best = -2.f;
-        int at = 0;
+        float best = s[0];
+        int at = lane;
 #pragma unroll
-        for (int i = 0; i < PER; i++)
+        for (int i = 1; i < PER; i++)
             if (s[i] > best) best = s[i], at = lane + 64 * i;
-        // (a row of NaN scores chooses experts 0, 1, ..: `best` keeps its start value)
         const float top = row_wave_max(best);
         at = __builtin_amdgcn_readlane(at, __ffsll((unsigned long long)__builtin_amdgcn_ballot_w64(best == top)) - 1);
         best = top;
@@ -198,7 +202,7 @@ __device__ __forceinline__ void choose_experts_of(const NcRoute& r, int m, int l
         if (lane == 0) r.chosen[m * r.top + k] = at;
 #pragma unroll
         for (int i = 0; i < PER; i++)
-            if (at == lane + 64 * i) s[i] = -1.5f;
+            if (at == lane + 64 * i) s[i] = -2.f;
     }
     if (lane < r.top) r.slot_w[m * r.top + lane] = mine / (chosen_sum + 1e-20f);
 }

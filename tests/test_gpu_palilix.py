@@ -381,6 +381,32 @@ def test_rows_of_nan_scores_beside_others_that_share_their_expert(rows, spoiled,
     spoiled_rows_leave_the_others_alone(cfg, rows, spoiled, dtype)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("experts,top,rows", [(7, 7, 3), (20, 16, 16), (63, 5, 40), (70, 64, 9), (300, 20, 80)])
+def test_rows_of_nan_scores_choose_experts_that_are_there(experts, top, rows, dtype):
+    """Fewer experts than lanes (of one, four and sixteen experts each): a row of NaN scores chooses distinct ones of them, in small calls and in
+    the larger ones that choose in a launch of their own."""
+    say(f"NaN rows, {top} of {experts} experts, {rows} rows, {dtype}")
+    cfg = config([(latent(), moe(experts=experts, top=top, ff=16)), (retention(), None)], vocab=50)
+    spoiled_rows_leave_the_others_alone(cfg, rows, [1, rows - 1], dtype)
+
+
+@pytest.mark.parametrize("bad", [math.nan, math.inf])
+def test_experts_of_bad_scores(bad):
+    """More experts whose scores are no numbers than choices that may avoid them: every logit is NaN, and the next call is as if it had not been."""
+    say(f"router rows of {bad}")
+    cfg = config([(latent(), moe(experts=20, top=16, ff=16)), (retention(), None)], vocab=50)
+    w = weights(cfg, seed=8)
+    model = build(cfg, w, torch.bfloat16)
+    toks = ids(tokens(cfg, 9))
+    want = model.forward(toks, kv_cache=model.new_cache(1, 9)).clone()
+    spoiled = dict(w)
+    spoiled["l0.mlp.router"] = w["l0.mlp.router"].clone()
+    spoiled["l0.mlp.router"][3:15] = bad
+    assert torch.isnan(build(cfg, spoiled, torch.bfloat16).forward(toks)).any()
+    assert torch.equal(model.forward(toks, kv_cache=model.new_cache(1, 9)), want)
+
+
 def test_a_slot_is_used_again_without_a_trace():
     say("slots used again")
     model, cfg = case_model("odd", torch.bfloat16), CASES["odd"]
