@@ -593,8 +593,9 @@ int nc_launch_linear_tiled(int dtype, const NcLinear& l, hipStream_t s, int cls,
     if (int rc = check_linear(l, dtype)) return rc;
     NC_CHECK_ARG(l.K % 64 == 0 && l.splits <= l.K / 64 && shape >= 0 && shape <= SHAPES, "linear: the tiled kernel takes whole K-steps");
     NcProfScope prof(cls, linear_units(l, dtype, !l.tiles ? l.M <= NC_FEW_ROWS : l.tile_rows <= 32), s, linear_tag(l));
-    if (!shape) shape = !l.tiles ? choose_shape(l, dtype) : l.tile_rows <= 32 ? 5 : l.tile_rows <= 64 ? 1 : 2;
-    if (l.tiles) NC_CHECK_ARG(l.tile_rows <= SHAPE_ROWS[shape], "linear: group tiles of %d rows", l.tile_rows);
+    if (!shape) shape = !l.tiles ? choose_shape(l, dtype) : l.tile_rows <= 32 ? 5 : l.tile_rows <= 64 ? (l.few ? 4 : 1) : 2;
+    // (the wider shapes have one chain: they are no place for a group whose sums are those of few rows)
+    if (l.tiles) NC_CHECK_ARG(l.tile_rows <= SHAPE_ROWS[shape] && (!l.few || shape >= 4), "linear: group tiles of %d rows", l.tile_rows);
     return dtype ? launch_tiled_shape<float>(l, shape, s) : launch_tiled_shape<bf16_t>(l, shape, s);
 }
 

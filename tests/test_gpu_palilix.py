@@ -356,6 +356,20 @@ def test_prompts_of_several_rows_at_once(dtype):
             check(got[r], ref.forward(cfg, w64, s), dtype, f"row {r} of 3, cuts {cuts[:3]}")
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("experts,top", [(4, 4), (4, 2), (16, 8), (1, 1)])
+def test_experts_of_few_rows_have_the_same_sums_in_every_batch(experts, top, dtype):
+    """64 sequences, 16 to 64 of them to an expert, against the same ones 20 and 33 at a time: tiles of 64 or of 32 rows, the same additions."""
+    say(f"experts in batches, {top} of {experts}, {dtype}")
+    cfg = config([(latent(), moe(experts=experts, top=top, ff=320))], width=320, vocab=70)
+    model = build(cfg, weights(cfg, seed=9), dtype)
+    toks = torch.arange(64, device=DEV)[:, None]
+    want = model.forward_last(toks, kv_cache=model.new_cache(64, 2)).clone()
+    for part in (20, 33):
+        got = torch.cat([model.forward_last(p, kv_cache=model.new_cache(len(p), 2)).clone() for p in (toks[:part], toks[64 - part:])])
+        assert torch.equal(got, torch.cat([want[:part], want[64 - part:]])), part
+
+
 def spoiled_rows_leave_the_others_alone(cfg, rows, spoiled, dtype):
     """One token to each of `rows` sequences; those of `spoiled` bring a token whose embedding is NaN: the others' logits are what they are where
     every sequence is a healthy one, to the bit."""
