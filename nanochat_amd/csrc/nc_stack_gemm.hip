@@ -572,12 +572,11 @@ int nc_linear_splits(int dtype, int M, int N, int K) {
     if (M <= NC_FEW_ROWS) {
         const int nb = M <= 16 ? 16 : 32, wgs = (N + nb - 1) / nb;
         while (splits < 8 && wgs * splits < 384 && K / (splits * 2) >= 256) splits *= 2;
-    } else if (dtype && K % 64 == 0) {
-        // fp32 tiles that leave compute units without one: a workgroup for each, unless a share becomes so short that its sums are more bytes
-        // than its weight (333 x 1024 x 5120: 152 us in one piece, 45 in four).  bf16 sums of many rows stay one chain, whatever the tile and
-        // the number of rows.
-        const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
-        while (splits < 8 && tiles * splits * 2 <= nc_cu_count() && K / (splits * 2) >= 512) splits *= 2;
+    } else if (dtype && K % 64 == 0 && K >= 512) {
+        // fp32: four shares, whatever the number of rows, so that a row's sums do not depend on how many came with it.  Few tiles fill the chip with
+        // them (333 x 1024 x 5120: 152 us in one piece, 45 in four), many lose nothing (a prompt of 1792 tokens, in one piece / two / four: width
+        // 2048 6675 / 6637 / 6414 us, 1024 3307 / 3319 / 3349, 640 1425 / 1376 / 1363).  bf16 sums of many rows stay one chain.
+        splits = 4;
     }
     return splits;
 }

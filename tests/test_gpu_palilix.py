@@ -126,8 +126,7 @@ def test_32_bit_portions_at_the_edges_of_their_kernels(name):
 @pytest.mark.parametrize("width", [64, 512, 1024])
 @pytest.mark.parametrize("ff", [2048, 2112, 1984])
 def test_32_bit_shares_that_begin_in_the_middle_of_a_step(width, ff):
-    """The output matrix of many rows in four shares of 33 half steps (ff = 2048), of 34, and in two of 64: a share may begin with the second half
-    of a step.  Whole prompts against portions of few rows, which take other kernels."""
+    """The output matrix of many rows in four shares of 33 half steps (ff = 2048), of 34 and of 32: a share may begin with the second half of a step.  Whole prompts against portions of few rows, which take other kernels."""
     say(f"shares, width {width}, ff {ff}")
     cfg = config([(retention(heads=1, dim=64, vdim=64, rot_dims=32), dense(ff=ff))] * 2, width=width, vocab=50)
     model = build(cfg, weights(cfg, seed=3), torch.float32)
@@ -136,6 +135,19 @@ def test_32_bit_shares_that_begin_in_the_middle_of_a_step(width, ff):
         few = run(model, toks, [50] * (n // 50) + ([n % 50] if n % 50 else [])).cpu()
         for again in range(3):
             check(run(model, toks, [n]), few, torch.float32, f"{n} rows")
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_rows_of_a_longer_prompt_have_the_same_bits(dtype):
+    """From 65 tokens on a token's result is what it is in a shorter prompt that begins alike: one order of the sums for any number of rows."""
+    say(f"prompts of other lengths, {dtype}")
+    cfg = config([(latent(heads=8, dim=64), dense(ff=1100)), (retention(heads=2, dim=64, vdim=64, rot_dims=32), dense(ff=4096))], width=1024, vocab=50)
+    model = build(cfg, weights(cfg, seed=3), dtype)
+    toks = tokens(cfg, 700)
+    want = run(model, toks, [700])
+    for n in (65, 97, 333, 576):
+        if dtype == torch.float32 or n >= 333:                # (bf16 latent attention changes its form between)
+            assert torch.equal(run(model, toks[:n], [n]), want[:n]), n
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
