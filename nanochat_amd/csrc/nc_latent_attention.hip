@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void latent_simple_kernel(NcLatentGeom g, cons
 // 16 query rows (row = token * heads + head of one batch row) per workgroup, keys 64 at a time, on v_mfma_f32_16x16x4_f32: a lane supplies 16
 // bytes of row lane % 16 from piece lane / 16, which is four instructions (which dimension or key a lane's values stand for does not matter as
 // long as both operands agree).
-//   scores   wave w: keys 16 (w % 4) .. + 15, half w / 4 of the row; the halves meet in LDS
+//   scores   wave w: keys 16 (w % 4) .. + 15, half w / 4 of the row in two chains (four in all, as in latent_simple_kernel); the halves meet in LDS
 //   softmax  wave w: rows 2 w and 2 w + 1, lane = key
 //   sums     wave w: columns 16 (w + 8 c) .. + 15 of the latent
 // What bounds latent_simple_kernel is the L2: every row reads all its keys twice (8 heads, rank 512, 333 tokens: 4 GB, 188 us).  Here 16 rows share
@@ -187,10 +187,15 @@ __global__ __launch_bounds__(64 * WAVES32) void latent32_kernel(NcLatentGeom g, 
         {                                                      // (a key past the last one is read as the last: masked below, finite)
             const int kt = wave & 3, steps = rw / 16, s0 = (wave >> 2) * (steps / 2), s1 = wave >> 2 ? steps : steps / 2;
             const float *kr = keys + (int64_t)min(k0 + 16 * kt + col, last) * rw + 4 * piece, *qr = qs + col * pitch + 4 * piece;
-            v4f s = v4f{0.f, 0.f, 0.f, 0.f};
-            for (int i = s0; i < s1; i++) s = mma32(*(const v4f*)(qr + 16 * i), *(const v4f*)(kr + 16 * i), s);
+            v4f s[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
+            int i = s0;
+            for (; i + 1 < s1; i += 2) {
+                s[0] = mma32(*(const v4f*)(qr + 16 * i), *(const v4f*)(kr + 16 * i), s[0]);
+                s[1] = mma32(*(const v4f*)(qr + 16 * i + 16), *(const v4f*)(kr + 16 * i + 16), s[1]);
+            }
+            if (i < s1) s[0] = mma32(*(const v4f*)(qr + 16 * i), *(const v4f*)(kr + 16 * i), s[0]);
 #pragma unroll
-            for (int r = 0; r < 4; r++) sc[((wave >> 2) * 16 + 4 * piece + r) * S32_PITCH + 16 * kt + col] = s[r];
+            for (int r = 0; r < 4; r++) sc[((wave >> 2) * 16 + 4 * piece + r) * S32_PITCH + 16 * kt + col] = s[0][r] + s[1][r];
         }
         __syncthreads();
 #pragma unroll
