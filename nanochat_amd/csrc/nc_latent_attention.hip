@@ -238,9 +238,14 @@ __global__ __launch_bounds__(64 * WAVES32) void latent32_kernel(NcLatentGeom g, 
             if (at < g.rank_p && r0 + row < rows) out[((int64_t)b * rows + r0 + row) * g.rank_p + at] = acc[c][r] / sum_of[row];
         }
 }
-// From 64 query rows of a sequence on: fewer leave compute units to latent_simple_kernel's one workgroup per row.
+// From more query rows than compute units on: up to there latent_simple_kernel has a workgroup to itself for each row, and one workgroup of it walks
+// its keys faster than one of latent32_kernel (us of a forward pass, two such layers, latent32 / simple: 1000 cached tokens and 192 rows 626 / 594, 248
+// rows 667 / 631, 320 rows 642 / 712, 496 rows 832 / 863; 300 tokens and 248 rows 444 / 429, 320 rows 420 / 434, 512 rows 443 / 462; none and 192 rows
+// 294 / 304, 384 rows 311 / 314).  A step of one token has few rows of a sequence that could share its keys, whatever their number.
 int latent32_lds(const NcLatentGeom& g) { return (16 * (g.rank_p + g.rot_p + 4) + 3 * 16 * S32_PITCH) * 4; }
-bool latent32_ok(const NcLatentGeom& g) { return g.T * g.heads >= 64 && g.T >= 8 && g.rank_p <= 128 * 4 && g.rank_p % 16 == 0 && g.rot_p % 16 == 0 && latent32_lds(g) <= 60 * 1024; }
+bool latent32_ok(const NcLatentGeom& g) {
+    return (int64_t)g.B * g.T * g.heads > nc_cu_count() && g.T * g.heads >= 64 && g.T >= 8 && g.rank_p <= 128 * 4 && g.rank_p % 16 == 0 && g.rot_p % 16 == 0 && latent32_lds(g) <= 60 * 1024;
+}
 
 // ------------------------------------------------------------------------------------------------ latent space, matrix cores
 // A workgroup of eight waves takes 16 query rows (row = token * heads + head of one batch row) and a share of the keys, 32 keys at a time

@@ -123,6 +123,33 @@ def test_32_bit_portions_at_the_edges_of_their_kernels(name):
         check(run(case_model(name, torch.float32), tokens(CASES[name], n), cuts), oracle_logits(name, n), torch.float32, f"{name}, portions {cuts}")
 
 
+@pytest.mark.parametrize("name", ["odd", "wide"])
+def test_32_bit_portions_of_more_query_rows_than_compute_units(name):
+    """3 or 4 heads: from 86 or 65 tokens on 16 query rows share a block of keys; a last block of rows and of keys that is full, short by one or
+    has one, alone and behind other portions."""
+    say(f"32-bit portions of many rows, {name}")
+    for cuts in ([85], [86], [96], [97], [64, 128], [7, 121], [100, 91], [257]):
+        n = sum(cuts)
+        check(run(case_model(name, torch.float32), tokens(CASES[name], n), cuts), oracle_logits(name, n), torch.float32, f"{name}, portions {cuts}")
+
+
+@pytest.mark.parametrize("name", ["odd", "wide"])
+def test_32_bit_portions_of_unequal_sequences(name):
+    """24 tokens to each of five sequences of different lengths: their query rows together are more than the compute units, none shares another's keys."""
+    say(f"32-bit portions of unequal sequences, {name}")
+    cfg, model = CASES[name], case_model(name, torch.float32)
+    w64, lengths, new = {k: v.double() for k, v in case_weights(name).items()}, [3, 70, 33, 1, 104], 24
+    seqs = [tokens(cfg, n + new, seed=40 + n) for n in lengths]
+    cache = model.new_cache(len(seqs), 128)
+    for r, (s, n) in enumerate(zip(seqs, lengths)):
+        alone = model.new_cache(1, 128)
+        model.forward_last(ids(s[:n]), kv_cache=alone)
+        cache.load_row(r, alone)
+    got = model.forward(torch.tensor([s[n:] for s, n in zip(seqs, lengths)], device=DEV), kv_cache=cache)
+    for r, (s, n) in enumerate(zip(seqs, lengths)):
+        check(got[r], ref.forward(cfg, w64, s)[n:], torch.float32, f"{name}, row {r}")
+
+
 def test_32_bit_scores_of_many_rows_are_as_exact_as_of_few():
     """A whole prompt (16 query rows share their keys) against portions of 7 (one row each; a score in four chains of 144 terms), both against 64
     bits.  Rounding of a chain grows with its length: with a prompt's scores in two chains of 288 its error was 1.71 to 1.80 times that of the
