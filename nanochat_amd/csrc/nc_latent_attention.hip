@@ -172,7 +172,7 @@ __global__ __launch_bounds__(64 * WAVES32) void latent32_kernel(NcLatentGeom g, 
     const int rw = g.rank_p + g.rot_p, pitch = rw + 4, rows = g.T * g.heads, lane = threadIdx.x & 63, col = lane & 15, piece = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x / groups, r0 = 16 * (blockIdx.x % groups);
     float *const sc = qs + 16 * pitch, *const ps = sc + 2 * 16 * S32_PITCH;
-    const int pos = seqlens[b], last = min(pos + (min(r0 + 15, rows - 1)) / g.heads, g.Tmax - 1);
+    const int pos = seqlens[b], first = min(pos + r0 / g.heads, g.Tmax - 1), last = min(pos + (min(r0 + 15, rows - 1)) / g.heads, g.Tmax - 1);
     for (int u = threadIdx.x; u < 16 * rw / 4; u += 64 * WAVES32) {
         const int r = u / (rw / 4), d = 4 * (u % (rw / 4));
         *(v4f*)(qs + r * pitch + d) = *(const v4f*)(q_lat + ((int64_t)b * rows + min(r0 + r, rows - 1)) * rw + d);
@@ -182,7 +182,11 @@ __global__ __launch_bounds__(64 * WAVES32) void latent32_kernel(NcLatentGeom g, 
 #pragma unroll
     for (int c = 0; c < NT; c++) acc[c] = v4f{0.f, 0.f, 0.f, 0.f};
     float m_run[2] = {LA_M_FLOOR, LA_M_FLOOR}, l_run[2] = {0.f, 0.f};
-    __syncthreads();
+    // A key that some of the rows do not see has weight 0 there, which does not make an infinity or a NaN vanish: where there is one among the
+    // keys of these rows' own tokens, the block that holds them is summed key by key.
+    bool odd = false;
+    for (int u = threadIdx.x; u < (last - first + 1) * g.rank_p; u += 64 * WAVES32) odd |= !(fabsf(keys[(int64_t)(first + u / g.rank_p) * rw + u % g.rank_p]) < INFINITY);
+    odd = __syncthreads_or(odd);
     for (int k0 = 0; k0 <= last; k0 += KEYS32) {
         {                                                      // (a key past the last one is read as the last: masked below, finite)
             const int kt = wave & 3, steps = rw / 16, s0 = (wave >> 2) * (steps / 2), s1 = wave >> 2 ? steps : steps / 2;
@@ -214,6 +218,18 @@ __global__ __launch_bounds__(64 * WAVES32) void latent32_kernel(NcLatentGeom g, 
         for (int r = 0; r < 4; r++) corr[r] = corr_of[4 * piece + r];
 #pragma unroll
         for (int c = 0; c < NT; c++) acc[c] *= corr;
+        if (odd && k0 + KEYS32 > first) {                      // (uniform)
+            for (int k = 0; k < KEYS32 && k0 + k <= last; k++)
+#pragma unroll
+                for (int c = 0; c < NT; c++)
+                    if (16 * (wave + WAVES32 * c) < g.rank_p) {
+                        const float v = keys[(int64_t)(k0 + k) * rw + 16 * wave + col + 128 * c];
+#pragma unroll
+                        for (int r = 0; r < 4; r++)
+                            if (k0 + k <= min(pos + min(r0 + 4 * piece + r, rows - 1) / g.heads, g.Tmax - 1)) acc[c][r] = fmaf(ps[(4 * piece + r) * S32_PITCH + k], v, acc[c][r]);
+                    }
+            continue;
+        }
 #pragma unroll
         for (int k = 0; k < KEYS32; k += 16) {
             const v4f p = *(const v4f*)(ps + col * S32_PITCH + k + 4 * piece);

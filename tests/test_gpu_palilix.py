@@ -410,6 +410,23 @@ def test_prompts_of_several_rows_at_once(dtype):
             check(got[r], ref.forward(cfg, w64, s), dtype, f"row {r} of 3, cuts {cuts[:3]}")
 
 
+@pytest.mark.parametrize("mixer", [latent(heads=8, dim=32, kv_rank=200), latent(heads=3, kv_rank=56)])
+@pytest.mark.parametrize("at", [0, 70, 95, 99])
+def test_a_later_nan_does_not_reach_earlier_tokens(mixer, at):
+    """A token whose embedding is NaN in the middle of the tokens that share its block of keys, in 32-bit (in bfloat16 the matrix-core
+    kernels have always multiplied masked weights): what comes before it is what it is without it, what comes after it is NaN."""
+    say(f"a NaN at token {at}, {mixer['type']}")
+    cfg = config([(mixer, None)], vocab=50)
+    w, toks = weights(cfg, seed=12), [t or 1 for t in tokens(cfg, 100)]
+    want = ref.forward(cfg, {k: v.double() for k, v in w.items()}, toks)
+    w["embed"][0] = math.nan
+    toks[at] = 0
+    got = run(build(cfg, w, torch.float32), toks, [100])
+    assert torch.isnan(got[at:]).all()
+    if at:
+        check(got[:at], want[:at], torch.float32, f"{at} tokens before a NaN")
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("experts,top", [(4, 4), (4, 2), (16, 8), (1, 1)])
 def test_experts_of_few_rows_have_the_same_sums_in_every_batch(experts, top, dtype):
