@@ -492,8 +492,14 @@ __global__ __launch_bounds__(THREADS32) void retention32_out_kernel(NcRetentionG
     stage32(ks, DK, n, [&](int j, int d) {
         return turned(base + (int64_t)j * ldp + (g.heads + h) * DK, d, half, turns + (int64_t)min(pos0 + t0 + j, rope_len - 1) * half) * g.k_scale;
     });
-    stage32(vs, DV, n, [&](int j, int d) { return base[(int64_t)j * ldp + 2 * g.heads * DK + h * DV + d]; });
-    __syncthreads();
+    // (a later token's score is 0, which does not make an infinity or a NaN among its values vanish: such a chunk sums token by token below)
+    bool odd = false;
+    stage32(vs, DV, n, [&](int j, int d) {
+        const float v = base[(int64_t)j * ldp + 2 * g.heads * DK + h * DV + d];
+        odd |= !(fabsf(v) < INFINITY);
+        return v;
+    });
+    odd = __syncthreads_or(odd);
     if (wave < 4) {                              // decayed scores, one 16 x 16 tile per wave
         const int i0 = 16 * (wave >> 1), j0 = 16 * (wave & 1);
         v4f s = v4f{0.f, 0.f, 0.f, 0.f};
@@ -528,11 +534,20 @@ __global__ __launch_bounds__(THREADS32) void retention32_out_kernel(NcRetentionG
     __syncthreads();
     float ss[2][4] = {};
     if (mine) {
+        if (odd) {                               // (uniform)
+            for (int j = 0; j < n; j++)
 #pragma unroll
-        for (int j = 0; j < C32; j += 4) {
-            const float v = vs[(j + row) * VP + v0 + col];
-            o[0] = mma32(ps[col * PP + j + row], v, o[0]);
-            o[1] = mma32(ps[(16 + col) * PP + j + row], v, o[1]);
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++)
+                        if (16 * i + 4 * row + r >= j) o[i][r] = fmaf(ps[(16 * i + 4 * row + r) * PP + j], vs[j * VP + v0 + col], o[i][r]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < C32; j += 4) {
+                const float v = vs[(j + row) * VP + v0 + col];
+                o[0] = mma32(ps[col * PP + j + row], v, o[0]);
+                o[1] = mma32(ps[(16 + col) * PP + j + row], v, o[1]);
+            }
         }
 #pragma unroll
         for (int i = 0; i < 2; i++)

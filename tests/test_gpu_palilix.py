@@ -410,10 +410,10 @@ def test_prompts_of_several_rows_at_once(dtype):
             check(got[r], ref.forward(cfg, w64, s), dtype, f"row {r} of 3, cuts {cuts[:3]}")
 
 
-@pytest.mark.parametrize("mixer", [latent(heads=8, dim=32, kv_rank=200), latent(heads=3, kv_rank=56)])
+@pytest.mark.parametrize("mixer", [latent(heads=8, dim=32, kv_rank=200), latent(heads=3, kv_rank=56), retention(heads=2, dim=40, vdim=72), retention(heads=1, dim=128, vdim=128)])
 @pytest.mark.parametrize("at", [0, 70, 95, 99])
 def test_a_later_nan_does_not_reach_earlier_tokens(mixer, at):
-    """A token whose embedding is NaN in the middle of the tokens that share its block of keys, in 32-bit (in bfloat16 the matrix-core
+    """A token whose embedding is NaN in the middle of the tokens that share its block of keys or its chunk, in 32-bit (in bfloat16 the matrix-core
     kernels have always multiplied masked weights): what comes before it is what it is without it, what comes after it is NaN."""
     say(f"a NaN at token {at}, {mixer['type']}")
     cfg = config([(mixer, None)], vocab=50)
