@@ -34,14 +34,15 @@ template <> struct Mma<float> {
     }
 };
 
-// One instruction of the same, accumulated in place and kept in program order against every memory operation: the builtin lets the register
-// allocator pick another result tuple, which it repairs with copies in every K-step, and nothing would keep the LDS reads of a step in
-// front of the barrier that ends it.  PARTS instructions make up 16 bytes; the caller puts other accumulators between them.
+// One instruction of the same.  PARTS instructions make up 16 bytes; the caller puts other accumulators between them.  The memory operations on
+// both sides stay on their sides, so that the loads and LDS reads of a step lie between its products as they are written.  (The builtin, not an asm
+// statement: the compiler has to see a matrix instruction to keep its distance from the copies and zeros that it puts around it.)
 template <typename T> constexpr int MMA_PARTS = sizeof(T) == 2 ? 1 : 4;
 template <typename T>
-__device__ __forceinline__ void mma_in_place(v4f& acc, const v4i& w, const v4i& a, int part) {
-    if constexpr (sizeof(T) == 2) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(a) : "memory");
-    else asm volatile("v_mfma_f32_16x16x4_f32 %0, %1, %2, %0" : "+a"(acc) : "v"(w[part]), "v"(a[part]) : "memory");
+__device__ __forceinline__ void mma_part(v4f& acc, const v4i& w, const v4i& a, int part) {
+    if constexpr (sizeof(T) == 2) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, w), __builtin_bit_cast(v8bf, a), acc, 0, 0, 0);
+    else acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(v4f, w)[part], __builtin_bit_cast(v4f, a)[part], acc, 0, 0, 0);
+    asm volatile("" ::: "memory");
 }
 
 // four consecutive columns n .. n+3 (n a multiple of 4, all in one segment) of output row `row`
@@ -363,7 +364,7 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
                         for (int r = 0; r < NL; r++)
                             if ((2 * r + 1) * PRODUCTS / (2 * NL) == n) load(L0 + r, k_off, st);
                     }
-                    if (ROWS == ALL || (ROWS == SOME && i < valid)) mma_in_place<T>(acc[CHAIN][i][j], w[j], a[i], p);
+                    if (ROWS == ALL || (ROWS == SOME && i < valid)) mma_part<T>(acc[CHAIN][i][j], w[j], a[i], p);
                 }
     };
     const int wa = wm * (BM / WM) * 128, ww = BM * 128 + wn * (BN / WN) * 128;
@@ -395,20 +396,9 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
     // half steps [from, to) into one chain; a half outside the share is read and not multiplied
     auto run = [&](int from, int to, auto rows, auto chain) __attribute__((always_inline)) {
         if (from >= to) return;
-        // The accumulators hold their zeros from here on: left to itself the compiler writes one just in front of its first product, and does not
-        // see that the asm statement is an MFMA, which must not follow the write of its operand by less than a few cycles.
-#pragma unroll
-        for (int i = 0; i < WTM; i++)
-#pragma unroll
-            for (int j = 0; j < WTN; j++) asm volatile("" : "+a"(acc[decltype(chain)::value][i][j]));
-        asm volatile("s_nop 7" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
         if (from & 1) high(rows, chain);
         while (2 * (k0 + kt) + 1 < to) low(rows, chain), high(rows, chain);
         if (to & 1) low(rows, chain);
-        // the last products: the compiler does not see that an asm statement wrote the accumulators late, and may copy them from here on
-        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
     };
     using std::integral_constant;
     if constexpr (FEW) {
