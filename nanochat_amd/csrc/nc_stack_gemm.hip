@@ -592,13 +592,13 @@ int nc_launch_linear_tiled(int dtype, const NcLinear& l, hipStream_t s, int cls,
 // workgroups of 16 columns are few per compute unit or the whole weight is short; its price is that every workgroup reads every row from the L2.
 // us, few-rows kernel / best tile, by columns (times batch and shares):
 //   bf16, 1 to 4 rows    K = 512: 8192 4.5 / 5.3, 32768 9 / 10      1024: 8192 6.0 / 6.5, 32768 14.2 / 16.5      2048: 4096 6.2 / 8.1, 8192 10.5 / 9.7
-//   bf16, 16 rows        K = 512: 8192 5.0 / 5.4, 32768 11.2 / 10   1024: 8192 6.7 / 6.6, 16384 11.5 / 8.9       4096: 2048 10.9 / 12, 8192 19 / 14.7
+//   bf16, 16 rows        K = 512: 8192 5.0 / 5.4, 32768 11.2 / 10   1024: 6144 6.6 / 6.3, 16384 11.5 / 8.9       4096: 2048 10.9 / 12, 8192 19 / 14.7
 //   bf16, 32 rows        K = 128: 8192 3.4 / 4.0                    512: 8192 5.5 / 5.7, 16384 7.9 / 7.0         1024: 1024 6.8 / 5.7
 //   fp32, 4 rows         K = 512: 12288 8.9 / 9.4, 16384 11 / 10.1  1024: 6144 10.4 / 10.9, 8128 11.2 / 12.5 between a step's other launches
 //   fp32, 16 rows        K = 512: 8192 7.4 / 7.7, 16384 12.5 / 10.2 2048: 4096 15 / 17.4, 8192 22 / 18           32 rows, 256: 8192 5.6 / 6.2
 bool few_is_faster(const NcLinear& l, int dtype) {
     const int64_t cols = (int64_t)l.N * l.batch * l.splits, k = l.K / l.splits, weight = cols * k;
-    if (l.M <= 16 && (cols <= 4096 || weight <= (dtype && l.M > 8 && cols > 8192 ? 4 << 20 : 8 << 20))) return true;
+    if (l.M <= 16 && (cols <= 4096 || weight <= (l.M > 8 && (dtype ? cols > 8192 : k > 512) ? 4 << 20 : 8 << 20))) return true;
     if (l.M <= 4 && !dtype && k <= 1024) return true;
     return l.M <= 32 && k <= 512 && weight <= 4 << 20;
 }
