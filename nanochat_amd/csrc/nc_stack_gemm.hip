@@ -467,12 +467,16 @@ int check_linear(const NcLinear& l, int dtype) {
     NC_CHECK_ARG(l.M > 0 && l.N > 0 && l.K > 0 && l.K % 32 == 0 && l.batch >= 1, "linear: bad shape M=%d N=%d K=%d batch=%d", l.M, l.N, l.K, l.batch);
     NC_CHECK_ARG(dtype == 0 || dtype == 1, "linear: dtype must be 0 (bfloat16) or 1 (float)");
     NC_CHECK_ARG(l.lda % (dtype ? 4 : 8) == 0 && l.ldw % (dtype ? 4 : 8) == 0 && l.ldw >= l.K && ((uintptr_t)l.a & 15) == 0 && ((uintptr_t)l.w & 15) == 0, "linear: operands must be 16-byte aligned");
-    NC_CHECK_ARG(l.splits >= 1 && (l.splits & (l.splits - 1)) == 0 && l.splits <= 64 && l.K <= 1 << 20 && (l.splits == 1 || l.partials), "linear: %d shares of %d", l.splits, l.K);
+    NC_CHECK_ARG(l.splits >= 1 && (l.splits & (l.splits - 1)) == 0 && l.splits <= 64 && (int64_t)l.K * l.splits < 1 << 29 && (l.splits == 1 || l.partials), "linear: %d shares of %d", l.splits, l.K);
     NC_CHECK_ARG(!l.partials || (l.batch == 1 && !l.tiles && l.N % 16 == 0), "linear: partial sums of %d columns", l.N);
     for (int i = 0; i < l.nseg; i++)
         NC_CHECK_ARG(l.seg[i].kind == NC_SEG_LOGITS || (l.seg[i].end % 16 == 0 && l.seg[i].ld % 4 == 0), "linear: segments must end at multiples of 16 columns");
     return 0;
 }
+
+// what the tiles' 32-bit offsets reach: the rows of A of a launch (a gathered row index is below M / a_div), the weight rows of a tile
+constexpr int64_t TILE_BYTES = 1ll << 31;
+int64_t linear_a_bytes(const NcLinear& l, int es) { return (((l.a_rows ? (l.M + l.a_div - 1) / l.a_div : l.M) - 1) * l.lda + l.K) * es; }
 
 template <typename T, int MT, int NB, int U = 4>
 int launch_few(const NcLinear& l, int ytiles, hipStream_t s) {
@@ -498,10 +502,8 @@ int launch_tiled(const NcLinear& l, hipStream_t s) {
     const void* fn = (const void*)linear_tiled_kernel<T, BM, BN, WM, WN, STAGES, FEW>;
     if (int rc = reserve_dynamic_lds(fn, LDS, done)) return rc;
     const int tm = l.tiles ? l.max_tiles : (l.M + BM - 1) / BM, tn = (l.N + BN - 1) / BN;
-    // rows of A this launch may reach: all of them (a gathered row index is below M / a_div)
-    const int64_t a_rows = l.a_rows ? (l.M + l.a_div - 1) / l.a_div : l.M;
-    const int64_t a_bytes = ((a_rows - 1) * l.lda + l.K) * (int64_t)sizeof(T);
-    NC_CHECK_ARG(a_bytes < (1ll << 31) && BN * l.ldw * (int64_t)sizeof(T) < (1ll << 31), "linear: operand past 2 GiB");
+    const int64_t a_bytes = linear_a_bytes(l, sizeof(T));
+    NC_CHECK_ARG(a_bytes < TILE_BYTES && BN * l.ldw * (int64_t)sizeof(T) < TILE_BYTES, "linear: operand past 2 GiB");
     hipLaunchKernelGGL((linear_tiled_kernel<T, BM, BN, WM, WN, STAGES, FEW>), dim3(tm * tn, l.batch * l.splits), dim3(64 * WM * WN), LDS, s, l, tm, tn,
                        __builtin_ctz(l.splits), (uint32_t)a_bytes);
     NC_CHECK_LAUNCH("linear_tiled");
@@ -603,5 +605,8 @@ bool few_is_faster(const NcLinear& l, int dtype) {
     return l.M <= 32 && k <= 512 && weight <= 4 << 20;
 }
 int nc_launch_linear(int dtype, const NcLinear& l, hipStream_t s) {
+    // (the few-rows kernel has no limit on the size of its operands)
+    const int es = dtype ? 4 : 2;
+    if (l.M <= NC_FEW_ROWS && (linear_a_bytes(l, es) >= TILE_BYTES || 64 * l.ldw * es >= TILE_BYTES)) return nc_launch_linear_few(dtype, l, s);
     return l.K % 64 || few_is_faster(l, dtype) ? nc_launch_linear_few(dtype, l, s) : nc_launch_linear_tiled(dtype, l, s);
 }

@@ -73,7 +73,7 @@ def test_tiles_at_their_edges(kernel, dtype):
         K = -(-K * steps // 64) * 64
         a, w = torch.randn(M, K, generator=g).to(dtype), (torch.randn(N, K, generator=g) / K ** 0.5).to(dtype)
         got = ops.stack_linear(a.to(DEV), w.to(DEV), kernel=kernel).cpu()
-        tol = 1e-2 if dtype == torch.bfloat16 else 2e-5       # one rounding to bf16 is 2^-9 of values up to about 4; fp32 sums of up to 448 terms
+        tol = 1e-2 if dtype == torch.bfloat16 else 2e-5       # one rounding to bf16 is 2^-9 of values up to about 4; fp32 sums of up to 320 terms
         assert torch.allclose(got.double(), a.double() @ w.double().T, rtol=tol, atol=tol), (M, N, K)
 
 
@@ -101,6 +101,20 @@ def test_whatever_kernel_is_chosen_for_few_rows_has_the_same_sums(dtype):
         want = ops.stack_linear(a, w, kind=3, kernel=6)
         for kernel in (0, 1):
             assert torch.equal(ops.stack_linear(a, w, kind=3, kernel=kernel), want), (M, N, K, kernel)
+
+
+@pytest.mark.parametrize("M,K", [(1, (1 << 20) + 64), (20, (1 << 20) + 64), (64, (1 << 23) + 64)])
+def test_long_sums_of_few_rows(M, K):
+    """Sums of more than 2^20 terms, and 64 rows of them that make an operand of more than 2 GiB."""
+    say(f"long sums, {M} rows of {K}")
+    g = torch.Generator(device=DEV).manual_seed(8)
+    a, w = torch.randn(M, K, generator=g, device=DEV), torch.randn(48, K, generator=g, device=DEV) / K ** 0.5
+    want = sum(p.double() @ q.double().T for p, q in zip(a.split(1 << 20, 1), w.split(1 << 20, 1)))
+    got = ops.stack_linear(a, w)
+    # Four chains of K / 4 terms of size K^-1/2: after t terms a chain is t^1/2 K^-1/2, and adding a term rounds that by 2^-24 of it at most.  The squares
+    # add up to (K / 4)^2 / (2 K) 2^-48 a chain, K / 8 2^-48 for the four; five standard deviations of that for the largest of 3072 results.
+    bound = 5 * 2.0 ** -24 * (K / 8) ** 0.5
+    assert (got.double() - want).abs().max().item() < bound
 
 
 # ------------------------------------------------------------------------------------------------ whole prompts
