@@ -647,8 +647,8 @@ int nc_launch_retention(int dtype, const NcRetentionGeom& g, const void* proj, i
                      : launch_step<bf16_t>(g, (const bf16_t*)proj, ldp, decay, rope, rope_len, seqlens, state_in, state_out, eps, (bf16_t*)out, ldo, s);
     }
     // bytes: the projections in, the outputs, and four passes over the chunks' states (written, scanned in and out, read)
-    NcProfScope prof(NC_CLS_RETENTION, (double)g.B * g.heads * (g.T * (2.0 * g.dim_p + 3.0 * g.vdim_p) * 2 + 16.0 * ((g.T + C - 1) / C) * g.dim_p * g.vdim_p), s,
-                     g.T);
+    NcProfScope prof(NC_CLS_RETENTION, (double)g.B * g.heads * (g.T * (2.0 * g.dim_p + 3.0 * g.vdim_p) * (dtype ? 4 : 2) + 16.0 * ((g.T + C - 1) / C) * g.dim_p * g.vdim_p),
+                     s, g.T);
     if (dtype) {
         const int chunks = (g.T + C - 1) / C, plane = g.dim_p * g.vdim_p;
         const int kv_lds = C32 * (g.dim_p + g.vdim_p + 2 * PAD32) * 4, out_lds = C32 * (2 * g.dim_p + g.vdim_p + 3 * PAD32 + C32 + 4) * 4;

@@ -117,6 +117,27 @@ def test_long_sums_of_few_rows(M, K):
     assert (got.double() - want).abs().max().item() < bound
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [31, 100])
+def test_bytes_that_the_profile_states_for_the_recurrence(n, dtype):
+    """Projections in and outputs out in the storage type; the states (fp32) once in and out token by token, four times per chunk in chunks."""
+    say(f"profile of the recurrence, {n} tokens, {dtype}")
+    heads, dim = 2, 64
+    cfg = config([(retention(heads=heads, dim=dim, vdim=dim, rot_dims=32), None)], vocab=50)
+    model, lib = build(cfg, weights(cfg, seed=2), dtype), ops._lib.stack_lib()
+    lib.nc_profile_enable(1)
+    try:
+        run(model, tokens(cfg, n), [n])
+        torch.cuda.synchronize()
+        ms, units, launches = ops.C.c_double(), ops.C.c_double(), ops.C.c_int64()
+        assert lib.nc_profile_read(2, ops.C.byref(ms), ops.C.byref(units), ops.C.byref(launches)) == 0
+    finally:
+        lib.nc_profile_enable(0)
+    size, chunk = (4, 32) if dtype == torch.float32 else (2, 64)
+    states = 2 if n < 32 else 4 * -(-n // chunk)
+    assert launches.value == 1 and units.value == heads * (n * 5 * dim * size + states * 4 * dim * dim)
+
+
 # ------------------------------------------------------------------------------------------------ whole prompts
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", list(CASES))
