@@ -1120,10 +1120,11 @@ def test_measurement_probes_run_and_report_their_work(ops):
 
 
 @pytest.mark.parametrize("lengths", ["spread", "equal but one", "empty and full", "ties"])
-@pytest.mark.parametrize("B,H,Hkv", [(65, 8, 4), (141, 4, 2), (300, 1, 1)])
-def test_attention_append_of_rows_dealt_by_length(ops, B, H, Hkv, lengths):
-    """More rows than one round of workgroups over the compute units: the kernel deals them by length, and every row is still its own."""
-    say(f"dealt rows B={B} H={H} Hkv={Hkv} {lengths}")
+@pytest.mark.parametrize("B,H,Hkv,splits,heads", [(65, 8, 4, 1, 1), (141, 4, 2, 1, 1), (300, 1, 1, 1, 1), (512, 2, 2, 1, 1), (129, 4, 4, 0, 1), (97, 16, 8, 0, 2)])
+def test_attention_append_of_rows_dealt_by_length(ops, B, H, Hkv, splits, heads, lengths):
+    """More rows than one round of workgroups over the compute units, keys in one piece: the kernel deals them by length, and every row is still its
+    own.  One and two kv heads per workgroup; a last round of one row, of a part of a round, and a whole one."""
+    say(f"dealt rows B={B} H={H} Hkv={Hkv} splits={splits} {lengths}")
     g = torch.Generator(device=DEV).manual_seed(B)
     Tmax = 1030
 
@@ -1137,9 +1138,12 @@ def test_attention_append_of_rows_dealt_by_length(ops, B, H, Hkv, lengths):
         n[::2], n[1::2] = 0, Tmax - 1
     elif lengths == "ties":
         n = n // 300 * 300
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
     for window in (-1, 1027):
+        # what the launch deals: one piece of the keys, and rows for more than one round of workgroups
+        assert ops.decode_attention_plan(B, 1, Hkv, window, Tmax, splits) == (1, heads) and B > cus // (Hkv // heads)
         kd, vd = kc.clone(), vc.clone()
-        got = ops.decode_attention_append(q, k, v, kd, vd, n, window_left=window)
+        got = ops.decode_attention_append(q, k, v, kd, vd, n, window_left=window, splits=splits)
         keys, values = kc.clone(), vc.clone()
         at = torch.arange(B, device=DEV), n.long()
         keys[at], values[at] = k[:, 0], v[:, 0]
