@@ -157,7 +157,7 @@ __global__ __launch_bounds__(256) void latent_simple_kernel(NcLatentGeom g, cons
 //   softmax  wave w: rows 2 w and 2 w + 1, lane = key
 //   sums     wave w: columns 16 (w + 8 c) .. + 15 of the latent
 // What bounds latent_simple_kernel is the L2: every row reads all its keys twice (8 heads, rank 512, 333 tokens: 4 GB, 188 us).  Here 16 rows share
-// them: 69 us.
+// them: 64 us.
 constexpr int KEYS32 = 64, WAVES32 = 8, S32_PITCH = KEYS32 + 4;
 __device__ __forceinline__ v4f mma32(v4f a, v4f b, v4f c) {
 #pragma unroll

@@ -5,11 +5,11 @@
 //   linear   [projections | router logits | first feed-forward matrix] . h    the activation of the feed-forward in the epilogue
 //   mixer    -> its part of `cat`; the feed-forward's part is there already
 //   experts  route (softmax, choice, expert order), gate and up with their activation, down: one row per (token, choice)
-//   linear   w_out . cat, added to the residual stream: in its epilogue, or (few tiles) as partial sums by the row kernel
+//   linear   w_out . cat, added to the residual stream: in its epilogue, or (few rows; 32-bit) as partial sums by the row kernel
 //   row add  x += partial sums + weighted expert rows (+ embedding output + step vector at the start of a pass), norm -> h
 // Per run of a post-norm layer, h = x in the storage type:
 //   linear   projections . h;  mixers, side by side if there are two  -> `cat`
-//   linear   w_out . cat -> sums in fp32 (few tiles: partial ones);  row add  x += norm1(sums) -> h
+//   linear   w_out . cat -> sums in fp32 (few rows; 32-bit: partial ones);  row add  x += norm1(sums) -> h
 //   linear   gate and up . h, activation in the epilogue;  linear  down -> sums;  row add  x += norm2(sums) -> h
 #include "../../include/nanochat_amd_stack.h"
 #include "nc_stack.h"

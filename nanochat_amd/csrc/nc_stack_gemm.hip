@@ -313,7 +313,7 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
         vo_w[i] = n0 + r < g.N ? (uint32_t)r * row_w + gch * 16 : TILE_OOB;
     }
     // FEW: the sum in four chains, a quarter of the share each: the same additions in the same order as in linear_few_kernel, so that a row's
-    // result does not depend on which of the kernels a batch of up to 64 rows took.
+    // result does not depend on which of the kernels a batch of up to 64 rows took.  (The number of shares is the caller's.)
     constexpr int CHAINS = FEW ? 4 : 1;
     v4f acc[CHAINS][WTM][WTN];
 #pragma unroll
@@ -540,7 +540,8 @@ int64_t shape_tiles(const NcLinear& l, int shape) {
 // 118 / 94 / 116, 700 x 4096 22 / 27 / 17.5 / 23 / 30, 333 x 2048 13 / 25 / 16 / 9.9 / 12, 80 x 2048 13 / 24 / 16 / 8.9 / 7.8 / 7.3; up to 64
 // rows, the last three and linear_few_kernel: 64 x 4096 12.1 / 9.9 / 8.7, 15.6, 64 x 12288 17.2 / 19.6 / 22, 28, 16 x 12288 16.0 / 13.6 / 14.7,
 // 16.7, 16 x 32768 34 / 31 / 36, 41.  fp32, K = 1024: 1792 x 4096 127 / 124 / 128 / 122 / 136, 333 x 4096 37 / 120 / 64 / 38 / 35, 80 x 4096
-// 35 / 92 / 50 / 22 / 15, 64 x 4096 23 / 15.3 / 11.6, 17.6.
+// 35 / 92 / 50 / 22 / 15, 64 x 4096 23 / 15.3 / 11.6, 17.6.  Over sums of 128 to 8192 and 80 to 1792 rows the choice is 0.6 % (bf16) and 1.1 % (fp32)
+// above the best tile on average, with costs that leave the length of the sum out.
 int choose_shape(const NcLinear& l, int dtype) {
     const int cus = nc_cu_count();
     int shape = 0;
