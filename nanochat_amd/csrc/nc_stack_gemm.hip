@@ -234,7 +234,11 @@ __global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g, int split_b
 // that the barrier counts the same number of loads in every step.
 //
 // Up to 64 rows it is a stream of the weight; the few-rows kernel, with both operands in registers, read every activation from the L2 once per 32
-// columns and waited for each batch of its loads (64 x 12352 x 2048: 32.5 us, 17 of them without the activations).
+// columns and waited for each batch of its loads (64 x 12352 x 2048: 32.5 us, 17 of them without the activations).  Its weights (FEW) are loaded with
+// the hint that nobody reads them again, so that they do not push out of the L2 what a step's other launches find there (us a step, without / with: Palilix,
+// width 2048, 8 layers, 64 rows 1622 / 1498, Zodirax 16 rows 638 / 610, 1 row 558 / 504, its window append 7.8 / 6.1 and head 29.2 / 26.7; fp32, width 896,
+// 8 rows 262 / 258; width 512, whose weights would stay in the 256 MB behind the L2, 8 rows 193 / 196).  The small weights of the few-rows kernel
+// are loaded without it (fp32, width 896, 8 rows 258 / 293; bf16, width 1024, 2 rows 170 / 177, 64 experts, 8 rows 292 / 294).
 //
 // What bounds it on many rows: the loads.  A compute unit takes some 35 bytes per clock straight into LDS (4096^3, 128 x 256: 88 us of loads alone, 62 of
 // products, 105 of both), which is why the widest tile that fills the chip is the one to take.  4096^3 140 -> 117 us, 1792 x 12352 x 2048
@@ -265,8 +269,10 @@ __device__ __forceinline__ bool group_tile_order(const NcLinear& g, int id, int 
     return true;
 }
 
+template <bool STREAM>
 __device__ __forceinline__ void tile_load(const void* base, uint32_t bytes, uint8_t* st, uint32_t lane_off, int k_off) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000), (lds_ptr_t)st, 16, lane_off, k_off, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00020000), (lds_ptr_t)st, 16, lane_off, k_off, 0,
+                                             STREAM ? 2 : 0);      // (bit 1: non-temporal)
 }
 
 template <typename T, int BM, int BN, int WM, int WN, int STAGES, bool FEW>
@@ -334,8 +340,8 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
     };
     constexpr int LOADS = A_P + W_P, EARLY = LOADS / 2, PRODUCTS = WTM * WTN, READS = WTM + WTN;
     auto load = [&](int i, int k_off, uint8_t* st) {
-        if (i < A_P) tile_load(A, a_bytes, st + i * NW * 1024, vo_a[i], k_off);
-        else tile_load(W, w_bytes, st + BM * 128 + (i - A_P) * NW * 1024, vo_w[i - A_P], k_off);
+        if (i < A_P) tile_load<false>(A, a_bytes, st + i * NW * 1024, vo_a[i], k_off);
+        else tile_load<FEW>(W, w_bytes, st + BM * 128 + (i - A_P) * NW * 1024, vo_w[i - A_P], k_off);
     };
     // 16-row tiles of this wave that hold rows at all: the last tile of a group of rows is seldom full
     const int valid = __builtin_amdgcn_readfirstlane((sp.rows - wm * (BM / WM) + 15) >> 4);
@@ -594,11 +600,13 @@ int nc_launch_linear_tiled(int dtype, const NcLinear& l, hipStream_t s, int cls,
 // The few-rows kernel or a tile: same sums, so only time decides.  In the few-rows kernel four waves share the summed index, which pays where its
 // workgroups of 16 columns are few per compute unit or the whole weight is short; its price is that every workgroup reads every row from the L2.
 // us, few-rows kernel / best tile, by columns (times batch and shares):
-//   bf16, 1 to 4 rows    K = 512: 8192 4.5 / 5.3, 32768 9 / 10      1024: 8192 6.0 / 6.5, 32768 14.2 / 16.5      2048: 4096 6.2 / 8.1, 8192 10.5 / 9.7
-//   bf16, 16 rows        K = 512: 8192 5.0 / 5.4, 32768 11.2 / 10   1024: 6144 6.6 / 6.3, 16384 11.5 / 8.9       4096: 2048 10.9 / 12, 8192 19 / 14.7
-//   bf16, 32 rows        K = 128: 8192 3.4 / 4.0                    512: 8192 5.5 / 5.7, 16384 7.9 / 7.0         1024: 1024 6.8 / 5.7
-//   fp32, 4 rows         K = 512: 12288 8.9 / 9.4, 16384 11 / 10.1  1024: 6144 10.4 / 10.9, 8128 11.2 / 12.5 between a step's other launches
-//   fp32, 16 rows        K = 512: 8192 7.4 / 7.7, 16384 12.5 / 10.2 2048: 4096 15 / 17.4, 8192 22 / 18           32 rows, 256: 8192 5.6 / 6.2
+//   bf16, 4 rows     K = 512: 8192 4.8 / 5.2, 32768 8.9 / 9.2      1024: 6144 6.2 / 6.1, 32768 14.3 / 14.6     2048: 4096 6.8 / 8.1, 8192 10.0 / 9.5
+//   bf16, 16 rows    K = 512: 4096 4.3 / 5.1, 16384 7.6 / 6.1      1024: 4096 5.3 / 5.9, 6144 7.4 / 6.1       4096: 2048 11.8 / 11.9, 8192 19.3 / 13.6
+//   bf16, 32 rows    K = 128: 8192 3.4 / 4.0                       512: 8192 6.0 / 5.2, 16384 8.3 / 6.3       1024: 2048 7.7 / 6.1
+//   fp32, 4 rows     K = 512: 8192 7.6 / 7.3, 16384 10.7 / 9.3     1024: 4096 8.3 / 10.3, 8128 11.2 / 12.5 between a step's other launches
+//   fp32, 16 rows    K = 512: 4096 6.2 / 7.0, 16384 12.2 / 9.4     2048: 4096 14.7 / 16.5, 8192 22 / 17       32 rows, 256: 8192 6.6 / 6.0
+// A step's small launches gain more from the kernel that leaves its weight in the caches than these times of weights from memory say: without the second
+// line below, 1 row of width 1024 takes 179 us instead of 174, 132 instead of 127 (Zodirax, Palilix without experts).
 bool few_is_faster(const NcLinear& l, int dtype) {
     const int64_t cols = (int64_t)l.N * l.batch * l.splits, k = l.K / l.splits, weight = cols * k;
     if (l.M <= 16 && (cols <= 4096 || weight <= (l.M > 8 && (dtype ? cols > 8192 : k > 512) ? 4 << 20 : 8 << 20))) return true;
