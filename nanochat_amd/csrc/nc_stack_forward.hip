@@ -287,9 +287,10 @@ int run_experts(int dt, const nc_stack_layer& l, int M, int width_p, const Works
     const int pairs = M * l.top;
     auto grouped = [&](NcLinear& g) {
         g.tiles = w.tiles, g.n_tiles = w.n_tiles, g.max_tiles = r.max_tiles, g.tile_rows = r.tile_rows, g.few = M <= NC_FEW_ROWS || pairs / l.experts < 16, g.w_stride = (int64_t)g.N * g.K;
-        // Up to 16 rows the few-rows kernel, in 32-bit while the weights are few; same sums (us a step, against tiles of 32 rows: bf16, width 1024, 48
-        // experts, 1 row 154 / 171, 16 rows 226 / 248; width 2048, 64 experts, 4 rows 340 / 365, 16 rows 510 / 532; fp32, width 384, 16 experts, 1 row
-        // 154 / 176; width 768, 64 experts, 8 rows 415 / 390)
+        // Up to 16 rows the few-rows kernel, in 32-bit while the weights are few; same sums (us a step, against tiles of 32 rows: bf16, experts of 1024,
+        // width 512, 64 experts, 1 row 154 / 168, 16 rows 254 / 254; width 1024, 16 experts, 4 rows 225 / 214, 64 experts 247 / 247; width 2048, 64
+        // experts, 1 row 263 / 265, 4 rows 373 / 372, 16 rows 558 / 554; fp32, width 384, 16 experts, 1 row 154 / 176; width 768, 64 experts, 8 rows
+        // 415 / 390)
         if (r.tile_rows <= NC_GROUP_TILE_FEW && (!dt || (int64_t)g.max_tiles * g.N <= 32768)) return nc_launch_linear_few(dt, g, s, NC_CLS_EXPERTS);
         return nc_launch_linear_tiled(dt, g, s, NC_CLS_EXPERTS);
     };

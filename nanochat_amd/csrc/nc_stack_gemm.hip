@@ -544,9 +544,9 @@ int64_t shape_tiles(const NcLinear& l, int shape) {
 // The shape with the least rounds times cost.  Few rows are a stream of the weight, which the narrow tiles with the most loads in flight read
 // best.  Measured, us, 64x128 / 128x256 / 128x128 / 64x64 / 32x64 / 32x32: bf16, K = 2048: 1792 x 2048 21 / 25 / 17.6, 1792 x 12352
 // 118 / 94 / 116, 700 x 4096 22 / 27 / 17.5 / 23 / 30, 333 x 2048 13 / 25 / 16 / 9.9 / 12, 80 x 2048 13 / 24 / 16 / 8.9 / 7.8 / 7.3; up to 64
-// rows, the last three and linear_few_kernel: 64 x 4096 12.1 / 9.9 / 8.7, 15.6, 64 x 12288 17.2 / 19.6 / 22, 28, 16 x 12288 16.0 / 13.6 / 14.7,
-// 16.7, 16 x 32768 34 / 31 / 36, 41.  fp32, K = 1024: 1792 x 4096 127 / 124 / 128 / 122 / 136, 333 x 4096 37 / 120 / 64 / 38 / 35, 80 x 4096
-// 35 / 92 / 50 / 22 / 15, 64 x 4096 23 / 15.3 / 11.6, 17.6.  Over sums of 128 to 8192 and 80 to 1792 rows the choice is 0.6 % (bf16) and 1.1 % (fp32)
+// rows, the last three and linear_few_kernel: 64 x 4096 13.8 / 10.9 / 8.8, 16.4, 64 x 12288 15.5 / 19.0 / 20.2, 29, 16 x 12288 14.5 / 12.3 / 13.3,
+// 15.7, 16 x 32768 29 / 26 / 30, 38.  fp32, K = 1024: 1792 x 4096 127 / 124 / 128 / 122 / 136, 333 x 4096 37 / 120 / 64 / 38 / 35, 80 x 4096
+// 35 / 92 / 50 / 22 / 15, 64 x 4096 22.5 / 15.1 / 11.0, 19.2.  Over sums of 128 to 8192 and 80 to 1792 rows the choice is 0.6 % (bf16) and 1.1 % (fp32)
 // above the best tile on average, with costs that leave the length of the sum out.
 int choose_shape(const NcLinear& l, int dtype) {
     const int cus = nc_cu_count();
