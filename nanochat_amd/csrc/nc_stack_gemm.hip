@@ -160,8 +160,8 @@ __device__ __forceinline__ int64_t a_row(const NcLinear& g, int row) { return g.
 
 // ------------------------------------------------------------------------------------------------
 // MT tiles of 16 rows x NB tiles of 16 weight rows per workgroup; wave w takes K-steps [its share] of 64 bytes.
-// U K-steps are asked for at a time.
-template <typename T, int MT, int NB, int U>
+// U K-steps are asked for at a time.  STREAM: the weight is loaded with the hint that nobody reads it again (see the tiled kernel).
+template <typename T, int MT, int NB, int U, bool STREAM>
 __global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g, int split_bits) {
     __shared__ v4f red[4][MT * NB][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -194,7 +194,10 @@ __global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g, int split_b
 #pragma unroll
         for (int u = 0; u < N_; u++) {
 #pragma unroll
-            for (int j = 0; j < NB; j++) wf[u][j] = *(const v4i*)(wp[j] + (int64_t)(s + u) * 64);
+            for (int j = 0; j < NB; j++) {
+                const v4i* const p = (const v4i*)(wp[j] + (int64_t)(s + u) * 64);
+                wf[u][j] = STREAM ? __builtin_nontemporal_load(p) : *p;
+            }
 #pragma unroll
             for (int i = 0; i < MT; i++) af[u][i] = *(const v4i*)(ap[i] + (int64_t)(s + u) * 64);
         }
@@ -234,11 +237,11 @@ __global__ __launch_bounds__(256) void linear_few_kernel(NcLinear g, int split_b
 // that the barrier counts the same number of loads in every step.
 //
 // Up to 64 rows it is a stream of the weight; the few-rows kernel, with both operands in registers, read every activation from the L2 once per 32
-// columns and waited for each batch of its loads (64 x 12352 x 2048: 32.5 us, 17 of them without the activations).  Its weights (FEW) are loaded with
-// the hint that nobody reads them again, so that they do not push out of the L2 what a step's other launches find there (us a step, without / with: Palilix,
-// width 2048, 8 layers, 64 rows 1622 / 1498, Zodirax 16 rows 638 / 610, 1 row 558 / 504, its window append 7.8 / 6.1 and head 29.2 / 26.7; fp32, width 896,
-// 8 rows 262 / 258; width 512, whose weights would stay in the 256 MB behind the L2, 8 rows 193 / 196).  The small weights of the few-rows kernel
-// are loaded without it (fp32, width 896, 8 rows 258 / 293; bf16, width 1024, 2 rows 170 / 177, 64 experts, 8 rows 292 / 294).
+// columns and waited for each batch of its loads (64 x 12352 x 2048: 32.5 us, 17 of them without the activations).  Its weights (FEW), as the
+// few-rows kernel's, are loaded with the hint that nobody reads them again, so that they do not push out of the L2 what a step's other launches find
+// there (us a step, without / with: Palilix, width 2048, 8 layers, 64 rows 1622 / 1498, Zodirax 16 rows 638 / 613, 1 row 560 / 499, its window append 7.8 /
+// 6.1 and head 29.2 / 26.7; fp32, width 384, 2 rows 267 / 262, width 896, 8 rows 367 / 332, and 262 / 293 where one small model runs alone and its
+// weights would stay in the 256 MB behind the L2).
 //
 // What bounds it on many rows: the loads.  A compute unit takes some 35 bytes per clock straight into LDS (4096^3, 128 x 256: 88 us of loads alone, 62 of
 // products, 105 of both), which is why the widest tile that fills the chip is the one to take.  4096^3 140 -> 117 us, 1792 x 12352 x 2048
@@ -484,9 +487,9 @@ int check_linear(const NcLinear& l, int dtype) {
 constexpr int64_t TILE_BYTES = 1ll << 31;
 int64_t linear_a_bytes(const NcLinear& l, int es) { return (((l.a_rows ? (l.M + l.a_div - 1) / l.a_div : l.M) - 1) * l.lda + l.K) * es; }
 
-template <typename T, int MT, int NB, int U = 4>
+template <typename T, int MT, int NB, int U = 4, bool STREAM = true>
 int launch_few(const NcLinear& l, int ytiles, hipStream_t s) {
-    hipLaunchKernelGGL((linear_few_kernel<T, MT, NB, U>), dim3((l.N + 16 * NB - 1) / (16 * NB), ytiles, l.batch * l.splits), dim3(256), 0, s, l, __builtin_ctz(l.splits));
+    hipLaunchKernelGGL((linear_few_kernel<T, MT, NB, U, STREAM>), dim3((l.N + 16 * NB - 1) / (16 * NB), ytiles, l.batch * l.splits), dim3(256), 0, s, l, __builtin_ctz(l.splits));
     NC_CHECK_LAUNCH("linear_few");
     return 0;
 }
@@ -495,10 +498,10 @@ int launch_few_t(const NcLinear& l, hipStream_t s) {
     // One workgroup per compute unit or two wait for their loads, which eight steps at a time halve (bf16, 4 rows, K = 2048, N = 2048 6.6 -> 6.0 us,
     // K = 4096 10.3 -> 9.2, six experts of 2048 x 2048 and back a step of 255 -> 244; from 16384 columns on 9.5 -> 10.3, and no fp32 launch gains).
     const int64_t cols = (int64_t)l.N * (l.tiles ? l.max_tiles : l.batch * l.splits);
-    if (l.M <= 16 || l.tiles) {
-        const int y = l.tiles ? l.max_tiles : 1;
-        return sizeof(T) == 2 && cols <= 12288 ? launch_few<T, 1, 1, 8>(l, y, s) : launch_few<T, 1, 1>(l, y, s);
-    }
+    const bool ahead = sizeof(T) == 2 && cols <= 12288;
+    // (experts' weights without the hint: bf16, experts of 1024, width 2048, 16 rows a step of 609 us with it, 581 without; width 1024, 8 rows 303 / 294)
+    if (l.tiles) return ahead ? launch_few<T, 1, 1, 8, false>(l, l.max_tiles, s) : launch_few<T, 1, 1, 4, false>(l, l.max_tiles, s);
+    if (l.M <= 16) return ahead ? launch_few<T, 1, 1, 8>(l, 1, s) : launch_few<T, 1, 1>(l, 1, s);
     return l.M <= 32 ? launch_few<T, 2, 2>(l, 1, s) : launch_few<T, 4, 2>(l, (l.M + 63) / 64, s);
 }
 template <typename T, int BM, int BN, int WM, int WN, int STAGES, bool FEW>
@@ -544,9 +547,9 @@ int64_t shape_tiles(const NcLinear& l, int shape) {
 // The shape with the least rounds times cost.  Few rows are a stream of the weight, which the narrow tiles with the most loads in flight read
 // best.  Measured, us, 64x128 / 128x256 / 128x128 / 64x64 / 32x64 / 32x32: bf16, K = 2048: 1792 x 2048 21 / 25 / 17.6, 1792 x 12352
 // 118 / 94 / 116, 700 x 4096 22 / 27 / 17.5 / 23 / 30, 333 x 2048 13 / 25 / 16 / 9.9 / 12, 80 x 2048 13 / 24 / 16 / 8.9 / 7.8 / 7.3; up to 64
-// rows, the last three and linear_few_kernel: 64 x 4096 13.8 / 10.9 / 8.8, 16.4, 64 x 12288 15.5 / 19.0 / 20.2, 29, 16 x 12288 14.5 / 12.3 / 13.3,
-// 15.7, 16 x 32768 29 / 26 / 30, 38.  fp32, K = 1024: 1792 x 4096 127 / 124 / 128 / 122 / 136, 333 x 4096 37 / 120 / 64 / 38 / 35, 80 x 4096
-// 35 / 92 / 50 / 22 / 15, 64 x 4096 22.5 / 15.1 / 11.0, 19.2.  Over sums of 128 to 8192 and 80 to 1792 rows the choice is 0.6 % (bf16) and 1.1 % (fp32)
+// rows, the last three and linear_few_kernel: 64 x 4096 13.7 / 10.9 / 8.7, 17.4, 64 x 12288 15.7 / 18.9 / 20.2, 32, 16 x 12288 14.5 / 12.3 / 13.3,
+// 16.5, 16 x 32768 29 / 26 / 30, 41.  fp32, K = 1024: 1792 x 4096 127 / 124 / 128 / 122 / 136, 333 x 4096 37 / 120 / 64 / 38 / 35, 80 x 4096
+// 35 / 92 / 50 / 22 / 15, 64 x 4096 22.4 / 15.0 / 11.1, 21.5.  Over sums of 128 to 8192 and 80 to 1792 rows the choice is 0.6 % (bf16) and 1.1 % (fp32)
 // above the best tile on average, with costs that leave the length of the sum out.
 int choose_shape(const NcLinear& l, int dtype) {
     const int cus = nc_cu_count();
@@ -600,17 +603,14 @@ int nc_launch_linear_tiled(int dtype, const NcLinear& l, hipStream_t s, int cls,
 // The few-rows kernel or a tile: same sums, so only time decides.  In the few-rows kernel four waves share the summed index, which pays where its
 // workgroups of 16 columns are few per compute unit or the whole weight is short; its price is that every workgroup reads every row from the L2.
 // us, few-rows kernel / best tile, by columns (times batch and shares):
-//   bf16, 4 rows     K = 512: 8192 4.8 / 5.2, 32768 8.9 / 9.2      1024: 6144 6.2 / 6.1, 32768 14.3 / 14.6     2048: 4096 6.8 / 8.1, 8192 10.0 / 9.5
-//   bf16, 16 rows    K = 512: 4096 4.3 / 5.1, 16384 7.6 / 6.1      1024: 4096 5.3 / 5.9, 6144 7.4 / 6.1       4096: 2048 11.8 / 11.9, 8192 19.3 / 13.6
-//   bf16, 32 rows    K = 128: 8192 3.4 / 4.0                       512: 8192 6.0 / 5.2, 16384 8.3 / 6.3       1024: 2048 7.7 / 6.1
-//   fp32, 4 rows     K = 512: 8192 7.6 / 7.3, 16384 10.7 / 9.3     1024: 4096 8.3 / 10.3, 8128 11.2 / 12.5 between a step's other launches
-//   fp32, 16 rows    K = 512: 4096 6.2 / 7.0, 16384 12.2 / 9.4     2048: 4096 14.7 / 16.5, 8192 22 / 17       32 rows, 256: 8192 6.6 / 6.0
-// A step's small launches gain more from the kernel that leaves its weight in the caches than these times of weights from memory say: without the second
-// line below, 1 row of width 1024 takes 179 us instead of 174, 132 instead of 127 (Zodirax, Palilix without experts).
+//   bf16, 4 rows     K = 512: 8192 4.7 / 5.2, 32768 9.6 / 9.2      1024: 6144 6.1 / 6.0, 32768 16.0 / 14.8     2048: 4096 7.0 / 8.1, 8192 9.6 / 9.1
+//   bf16, 16 rows    K = 512: 4096 4.1 / 5.0, 16384 7.8 / 6.1      1024: 4096 5.2 / 5.9, 6144 7.2 / 6.1       4096: 2048 12.1 / 11.8, 8192 21 / 13.5
+//   bf16, 32 rows    K = 128: 8192 3.4 / 4.0                       512: 8192 5.9 / 5.2, 16384 8.7 / 6.2       1024: 2048 8.0 / 6.1
+//   fp32, 4 rows     K = 512: 8192 7.9 / 7.3, 16384 12.1 / 9.4     1024: 4096 10.0 / 10.1, 8128 11.2 / 12.5 between a step's other launches
+//   fp32, 16 rows    K = 512: 4096 7.0 / 7.1, 16384 14 / 9.6       2048: 4096 17.9 / 16.5, 8192 24 / 17       32 rows, 256: 8192 6.5 / 6.8
 bool few_is_faster(const NcLinear& l, int dtype) {
     const int64_t cols = (int64_t)l.N * l.batch * l.splits, k = l.K / l.splits, weight = cols * k;
     if (l.M <= 16 && (cols <= 4096 || weight <= (l.M > 8 && (dtype ? cols > 8192 : k > 512) ? 4 << 20 : 8 << 20))) return true;
-    if (l.M <= 4 && !dtype && k <= 1024) return true;
     return l.M <= 32 && k <= 512 && weight <= 4 << 20;
 }
 int nc_launch_linear(int dtype, const NcLinear& l, hipStream_t s) {
