@@ -280,9 +280,9 @@ __device__ __forceinline__ void amax_publish(uint32_t* h, float am) {
     if (bits == 0u || (bits >> 31)) return;
     uint32_t* p = (uint32_t*)((uintptr_t)h & ~(uintptr_t)3);
     if ((uintptr_t)h & 1u) p += ((blockIdx.x + 3u * blockIdx.y + 5u * blockIdx.z) % NC_AMAX_SLOTS) * NC_AMAX_STRIDE;
-    // with hundreds of workgroups per slot the atomics queue up behind each other and a look first pays; with a few, the look is
-    // a round trip to memory in front of an atomic that nobody waits for
-    if (gridDim.x * gridDim.y * gridDim.z > 16 * NC_AMAX_SLOTS && __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= bits) return;
+    // with hundreds of workgroups per slot the atomics queue up behind each other and a look first pays; with up to one workgroup per
+    // compute unit (32 per slot), the look is a round trip to memory in front of an atomic that nobody waits for
+    if (gridDim.x * gridDim.y * gridDim.z > 32 * NC_AMAX_SLOTS && __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= bits) return;
     atomicMax(p, bits);
 }
 

@@ -22,9 +22,10 @@
 //                               launch, 1.5 us the partial sums leaving the chip); 65 .. 128 rows take eight
 //                               waves, two halves of 64 rows against the same weight columns (d26 at 128 rows
 //                               with the prompt read once: 39.7 k -> 43.1 k tokens/s);
-//   gemm_decode_full_kernel     17 .. 64 rows, K <= 2048, relu^2 epilogue: unsplit, 32 columns per workgroup,
+//   gemm_decode_full_kernel     up to 64 rows, K <= 2048, relu^2 epilogue: unsplit, 32 columns per workgroup (few columns: 16),
 //                               the result leaves finished and the MLP activation needs no pass of its own
-//                               (10.6 us against 8.3 + 4.4 us for the split linear and its finishing pass);
+//                               (64 rows 10.6 us against 8.3 + 4.4 us for the split linear and its finishing pass; 8 rows,
+//                               5120 x 1280, 6.6 against 3.8 + 3.9);
 //   gemm_decode_kernel          everything else (longer K ranges walked in 512-wide chunks).
 //
 // Epilogues: 0 bf16;  1 fp32 softcap*tanh(bf16(v)/softcap) (lm_head, nanochat/gpt.py:512-515);
@@ -637,20 +638,23 @@ __global__ __launch_bounds__(256 * WR) __attribute__((amdgpu_waves_per_eu(WR, 2)
 }
 
 // ------------------------------------------------------------------------------------------------
-// Unsplit form for 17 .. 64 rows and K <= 2048 (the q|k|v and c_fc linears of a decode step): a workgroup of 8 waves owns 32 output
+// Unsplit form for up to 64 rows and K <= 2048 (the c_fc linear of a decode step): 4 CB waves own 16 CB output
 // columns over the whole of K, so the result leaves the kernel finished (bf16, relu^2 and its amax included) instead of as fp32
 // partial sums that cost more to write and to read back than the weights did, and the MLP activation needs no pass of its own.
-// The whole activation panel is converted into LDS once per workgroup ([K-step][64 rows][128 bytes] tiles); wave (cb, rh, kh) then
-// multiplies rows 32*rh .. +31 with columns 16*cb .. +15 over half of the K-steps, and the two K halves meet through LDS.
+// The whole activation panel is converted into LDS once per workgroup ([K-step][16 MB rows][128 bytes] tiles) by 2 MB waves that do nothing
+// else; wave (cb, kq) then multiplies all rows with columns 16*cb .. +15 over a quarter of the K-steps, and the quarters meet through LDS.
+// MB = 4: 17 .. 64 rows, CB = 2.  MB = 1: up to 16 rows, 32 columns per workgroup (160 workgroups for 5120 columns: 7.2 us, 320 of 16 columns 7.7)
+// or, where that leaves half of the chip without one, 16.  (A step of 3 .. 16 GPT rows: 812 -> 798 us at depth 20, 8 rows, 267 -> 254 at depth 8, 16 rows.)
 // Still one trip to memory: activation rows first, then the weight rows, everything asked for before the first wait.
 #define NC_DGF_MAX_K 2048
-template <bool A_BF16, int NKS>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) void gemm_decode_full_kernel(DecodeGemmArgs g) {
+template <bool A_BF16, int NKS, int MB, int CB>
+__global__ __launch_bounds__(256 * CB + 128 * MB) __attribute__((amdgpu_waves_per_eu((4 * CB + 2 * MB + 3) / 4, 4))) void gemm_decode_full_kernel(DecodeGemmArgs g) {
     constexpr int A_LD = A_BF16 ? 2 : 1;
     constexpr int NKQ = (NKS + 3) / 4;              // K-steps per quarter
-    extern __shared__ __align__(16) uint8_t dgf_lds[];            // NKS tiles of 8 KB, then 6 x 4 KB for the meeting of the quarters
-    float* const meet = (float*)(dgf_lds + NKS * 8192);
-    __shared__ float red[2];
+    constexpr int TILE = MB * 2048;                 // a K-step of the panel: 16 MB rows of 128 bytes
+    extern __shared__ __align__(16) uint8_t dgf_lds[];            // NKS such tiles, then 3 CB x MB KB for the meeting of the quarters
+    float* const meet = (float*)(dgf_lds + NKS * TILE);
+    __shared__ float red[CB];
 
     NC_ARG_NOW(g.A); NC_ARG_NOW(g.a_amax); NC_ARG_NOW(g.inv_a); NC_ARG_NOW(g.B); NC_ARG_NOW(g.inv_b); NC_ARG_NOW(g.out); NC_ARG_NOW(g.out_kind);
     NC_ARG_NOW(g.out_amax); NC_ARG_NOW(g.ldc); NC_ARG_NOW(g.M); NC_ARG_NOW(g.N); NC_ARG_NOW(g.K);
@@ -663,17 +667,17 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
     if (A_BF16) aw = amax_load_scalar(g.a_amax);
     else inv_a = *g.inv_a;
 
-    if (wave >= 8) {
+    if (wave >= 4 * CB) {
         // ---- the converting waves: thread t converts chunk (row t >> 3, 16-byte piece t & 7) of every K-step tile.  Their loads
-        // come from the L2; they are asked for after the scale is known, which lets the weight requests of the other waves, the
-        // long trip, through the address units first.
+        // come from the L2; with 64 rows they are asked for after the scale is known, which lets the weight requests of the other waves,
+        // the long trip, through the address units first.  (16 rows are two waves' loads, in nobody's way: they go out with the scale's.)
         float scale = 1.f;
-        if (A_BF16) {
+        if (A_BF16 && MB > 1) {
             scale = scale_from_amax(amax_from_words(aw));
             asm volatile("" : "+v"(scale));
         }
         const __amdgpu_buffer_rsrc_t desc_a = __builtin_amdgcn_make_buffer_rsrc((void*)g.A, 0, M * K * (A_BF16 ? 2 : 1), 0x00020000);
-        const int ct = tid - 512;
+        const int ct = tid - 256 * CB;
         const int arow = ct >> 3, ach = ct & 7;
         dg_v4i ra[NKS][A_LD];
 #pragma unroll
@@ -683,6 +687,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
 #pragma unroll
             for (int h = 0; h < A_LD; h++) ra[j][h] = __builtin_amdgcn_raw_buffer_load_b128(desc_a, vo, h * 16, 0);
         }
+        if (A_BF16 && MB == 1) scale = scale_from_amax(amax_from_words(aw));
 #pragma unroll
         for (int j = 0; j < NKS; j++) {
             dg_v4i v;
@@ -698,7 +703,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
             } else {
                 v = ra[j][0];
             }
-            *(dg_v4i*)(&dgf_lds[j * 8192 + arow * 128 + ((ach ^ (arow & 7)) << 4)]) = v;      // (tiles past K hold zeros)
+            *(dg_v4i*)(&dgf_lds[j * TILE + arow * 128 + ((ach ^ (arow & 7)) << 4)]) = v;      // (tiles past K hold zeros)
         }
         __syncthreads();                  // the panel is complete
         __syncthreads();                  // (the meeting of the K quarters)
@@ -708,8 +713,8 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
 
     // ---- the multiplying waves: wave (cb, kq) asks for its weight rows at once and waits for the panel
     const int frow = lane & 15, kb = lane >> 4;
-    const int cb = wave & 1, kq = wave >> 1;
-    const int n0 = blockIdx.x * 32 + cb * 16;
+    const int cb = wave % CB, kq = wave / CB;
+    const int n0 = blockIdx.x * (16 * CB) + cb * 16;
     const int brow = n0 + frow;
     const int nq = (nksteps + 3) >> 2;                             // K-steps [kq * nq, (kq + 1) * nq) belong to quarter kq
     const int ks0 = kq * nq;
@@ -726,21 +731,23 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
             rb[j][h] = __builtin_amdgcn_raw_buffer_load_b128(desc_b, vo, h * 64, 0);
         }
     }
+    // (the weight scale of this lane's columns: asked for here, not when the sums are there)
+    const float inv_b = n0 < N ? dg_seg_scale(g, n0 + 4 * kb < N ? n0 + 4 * kb : N - 1) : 0.f;
     if (A_BF16) inv_a = 1.0f / scale_from_amax(amax_from_words(aw));
     __syncthreads();
 
-    v4f acc[4];
+    v4f acc[MB];
 #pragma unroll
-    for (int i = 0; i < 4; i++) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < MB; i++) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
     // no branch per K-step (the waits then count loads): a step past this quarter multiplies zero weight rows with some tile of the panel
 #pragma unroll
     for (int j = 0; j < NKQ; j++) {
-        const uint8_t* tile = dgf_lds + (j < nk ? ks0 + j : 0) * 8192;
+        const uint8_t* tile = dgf_lds + (j < nk ? ks0 + j : 0) * TILE;
         v8i bf;
         bf[0] = rb[j][0][0], bf[1] = rb[j][0][1], bf[2] = rb[j][0][2], bf[3] = rb[j][0][3];
         bf[4] = rb[j][1][0], bf[5] = rb[j][1][1], bf[6] = rb[j][1][2], bf[7] = rb[j][1][3];
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < MB; i++) {
             const int row = i * 16 + frow;
             const dg_v4i alo = *(const dg_v4i*)(tile + row * 128 + ((kb ^ (row & 7)) << 4));
             const dg_v4i ahi = *(const dg_v4i*)(tile + row * 128 + (((4 + kb) ^ (row & 7)) << 4));
@@ -752,18 +759,18 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
 
     // the later K quarters hand their sums to the first one (always added in the order 1, 2, 3)
     if (kq) {
-        float* mp = meet + (((kq - 1) * 2 + cb) * 64 + lane) * 16;
+        float* mp = meet + (((kq - 1) * CB + cb) * 64 + lane) * (4 * MB);
 #pragma unroll
-        for (int i = 0; i < 4; i++) *(float4*)(mp + 4 * i) = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
+        for (int i = 0; i < MB; i++) *(float4*)(mp + 4 * i) = make_float4(acc[i][0], acc[i][1], acc[i][2], acc[i][3]);
     }
     __syncthreads();
     float am = 0.f;
     if (!kq) {
 #pragma unroll
         for (int q = 0; q < 3; q++) {
-            const float* mp = meet + ((q * 2 + cb) * 64 + lane) * 16;
+            const float* mp = meet + ((q * CB + cb) * 64 + lane) * (4 * MB);
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
+            for (int i = 0; i < MB; i++) {
                 const float4 u = *(const float4*)(mp + 4 * i);
                 acc[i][0] += u.x, acc[i][1] += u.y, acc[i][2] += u.z, acc[i][3] += u.w;
             }
@@ -771,10 +778,9 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
         // lane holds rows 16*i + frow, columns n0 + 4*kb .. +3
         const int n = n0 + 4 * kb;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < MB; i++) {
             const int m = i * 16 + frow;
             if (m < M && n < N) {
-                const float inv_b = dg_seg_scale(g, n);
                 float v[4];
 #pragma unroll
                 for (int r = 0; r < 4; r++) v[r] = (acc[i][r] * inv_a) * inv_b;
@@ -802,7 +808,7 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
         am = wave_amax(am);
         if (!kq && lane == 0) red[cb] = am;
         __syncthreads();
-        if (tid == 0) amax_publish(g.out_amax, amax_join(red[0], red[1]));
+        if (tid == 0) amax_publish(g.out_amax, amax_join(red[0], red[CB - 1]));
     }
 }
 
@@ -957,20 +963,26 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 }
 
 namespace {
-template <bool A_BF16, int NKS>
-int launch_full(const DecodeGemmArgs& g, int nblk32, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
+template <bool A_BF16, int NKS, int MB, int CB>
+int launch_full_as(const DecodeGemmArgs& g, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
     static bool reserved[64];
-    constexpr int lds_bytes = NKS * 8192 + 6 * 4096;
+    constexpr int lds_bytes = NKS * MB * 2048 + 3 * CB * MB * 1024, threads = 256 * CB + 128 * MB;
+    const int blocks = (g.N + 16 * CB - 1) / (16 * CB);
     int dev = 0;
     (void)hipGetDevice(&dev);
     if (dev < 0 || dev >= 64 || !reserved[dev]) {
-        const hipError_t e = hipFuncSetAttribute((const void*)gemm_decode_full_kernel<A_BF16, NKS>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+        const hipError_t e = hipFuncSetAttribute((const void*)gemm_decode_full_kernel<A_BF16, NKS, MB, CB>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
         if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm(decode): cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
         if (dev >= 0 && dev < 64) reserved[dev] = true;
     }
-    if (ev0) hipExtLaunchKernelGGL((gemm_decode_full_kernel<A_BF16, NKS>), dim3(nblk32), dim3(1024), lds_bytes, s, ev0, ev1, 0, g);
-    else hipLaunchKernelGGL((gemm_decode_full_kernel<A_BF16, NKS>), dim3(nblk32), dim3(1024), lds_bytes, s, g);
+    if (ev0) hipExtLaunchKernelGGL((gemm_decode_full_kernel<A_BF16, NKS, MB, CB>), dim3(blocks), dim3(threads), lds_bytes, s, ev0, ev1, 0, g);
+    else hipLaunchKernelGGL((gemm_decode_full_kernel<A_BF16, NKS, MB, CB>), dim3(blocks), dim3(threads), lds_bytes, s, g);
     return 0;
+}
+template <bool A_BF16, int NKS>
+int launch_full(const DecodeGemmArgs& g, int cb, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
+    if (g.M > 16) return launch_full_as<A_BF16, NKS, 4, 2>(g, s, ev0, ev1);
+    return cb == 2 ? launch_full_as<A_BF16, NKS, 1, 2>(g, s, ev0, ev1) : launch_full_as<A_BF16, NKS, 1, 1>(g, s, ev0, ev1);
 }
 }  // namespace
 
@@ -997,11 +1009,11 @@ static bool dg_wide_form(int M, int N, int K, bool made) {
     return !made && M > 16 && M <= 64 && K <= NC_DGF_MAX_K && (N + 127) / 128 >= 256 && (int64_t)N * K < ((int64_t)1 << 31);
 }
 
-// Whether nc_launch_gemm_decode, left to choose (ksplits 0), runs the unsplit form: enough 32-column blocks to occupy half the chip
-// and few enough to run in one round.
+// Whether nc_launch_gemm_decode, left to choose (ksplits 0), runs the unsplit form: enough 32-column blocks to occupy half the chip (up to 16 rows,
+// whose second launch costs more than idle units do: any number) and few enough to run in one round.
 static bool dg_full_form(int M, int N, int K, bool made, int out_kind) {
     const int nblk32 = (N + 31) / 32;
-    return out_kind == 2 && !made && M > 16 && M <= 64 && K <= NC_DGF_MAX_K && nblk32 >= 128 && nblk32 <= 256 && (int64_t)N * K < ((int64_t)1 << 31);
+    return out_kind == 2 && !made && M <= 64 && K <= NC_DGF_MAX_K && (M <= 16 || nblk32 >= 128) && nblk32 <= 256 && (int64_t)N * K < ((int64_t)1 << 31);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1191,11 +1203,11 @@ int nc_launch_gemm_decode(const void* a, int a_is_bf16, const uint32_t* a_amax, 
         return 0;
     }
     if (full) {
-        const int nblk32 = (N + 31) / 32;
+        const int cb = M <= 16 && (N + 31) / 32 < 128 ? 1 : 2;
         int rc;
-        if (nksteps <= 10) rc = a_is_bf16 ? launch_full<true, 10>(g, nblk32, s, ev0, ev1) : launch_full<false, 10>(g, nblk32, s, ev0, ev1);
-        else if (nksteps <= 13) rc = a_is_bf16 ? launch_full<true, 13>(g, nblk32, s, ev0, ev1) : launch_full<false, 13>(g, nblk32, s, ev0, ev1);
-        else rc = a_is_bf16 ? launch_full<true, 16>(g, nblk32, s, ev0, ev1) : launch_full<false, 16>(g, nblk32, s, ev0, ev1);
+        if (nksteps <= 10) rc = a_is_bf16 ? launch_full<true, 10>(g, cb, s, ev0, ev1) : launch_full<false, 10>(g, cb, s, ev0, ev1);
+        else if (nksteps <= 13) rc = a_is_bf16 ? launch_full<true, 13>(g, cb, s, ev0, ev1) : launch_full<false, 13>(g, cb, s, ev0, ev1);
+        else rc = a_is_bf16 ? launch_full<true, 16>(g, cb, s, ev0, ev1) : launch_full<false, 16>(g, cb, s, ev0, ev1);
         if (rc) return rc;
         NC_CHECK_LAUNCH("fp8_gemm(decode)");
         return 0;

@@ -450,6 +450,26 @@ def test_decode_linear_forms_agree_bit_for_bit(ops, M, N, K, forms):
         assert torch.equal(h2, acts[0][0]) and torch.equal(am, acts[0][1]), f"relu^2 form, ksplits={ks}"
 
 
+@pytest.mark.parametrize("M,N,K,forms", [(3, 5120, 1280, (0, 1, 3)), (16, 8192, 2048, (0, 2)), (9, 1024, 256, (0, 1, 2)), (1, 16, 16, (0, 1)), (16, 4100, 400, (0, 3)),
+                                         (5, 36, 1664, (0, 1, 4)), (16, 4096, 1664, (0, 1)), (12, 8196, 1280, (0, 1, 3))])
+def test_unsplit_relu2_linear_of_up_to_16_rows(ops, M, N, K, forms):
+    """Up to 16 rows leave the unsplit form finished (16 or 32 columns per workgroup): the bytes of the split form and its finishing pass, at the edges of
+    its range, blocks and K-steps (the last shape is one column block past it), and the amax of what was written."""
+    say(f"unsplit relu^2 linear M={M} N={N} K={K}")
+    a, w = make_operands(M, N, K, seed=5 * M + N + K)
+    a8, ia, _ = fp8_ref.to_fp8(a)
+    w8, iw, _ = fp8_ref.to_fp8(w)
+    ad, w8d, iwd = a.to(DEV), w8.to(DEV), iw.reshape(1).to(DEV)
+    bits = ops.amax_bits(ad)
+    got, am = ops.fp8_linear_small_m(ad, bits, w8d, iwd, relu2=True, ksplits=0)
+    # two bf16 roundings (of the product and of its square), twice the first one's error: 3 * 2^-9 at most
+    assert rel_l2(got.cpu(), torch.relu(fp8_ref.scaled_mm_emulated(a8, w8, ia, iw)).square()) <= 3 * 2.0 ** -9
+    assert am.view(torch.float32).item() == got.float().max().item()
+    for ks in forms[1:]:
+        h2, am2 = ops.fp8_linear_small_m(ad, bits, w8d, iwd, relu2=True, ksplits=ks)
+        assert torch.equal(h2, got) and torch.equal(am2, am), f"ksplits={ks}"
+
+
 def test_fused_small_m_linear_seeded_shape_sweep(ops):
     """Forty seeded shapes around the borders between the decode linear's forms (rows 1 .. 128 across the 16-row blocks, widths that
     are no multiple of the 32 / 64 / 128-column blocks, K that ends inside a 128-wide step, every split count the caller may ask
