@@ -15,7 +15,8 @@
 //   linear c_fc         quantize xn inside                                             -> partials
 //   finish_partials     sum, scale, relu^2, amax                                       -> h2
 //   linear mlp c_proj   quantize h2 inside                                             -> partials (added by the next mix_norm)
-// Prefill (M > 128) uses the explicit convert kernel and the tiled GEMM instead of the fused small-M linear.
+// Prefill (M > 128) uses the explicit convert kernel and the tiled GEMM instead of the fused small-M linear; the two narrow projections of a
+// few hundred rows leave partial sums to mix_norm as well.
 //
 // Workspace (carved from the caller's buffer, 256-byte aligned pieces), M = B*T rows:
 //   x, x0, xn, xb, o      bf16 [M,E]        residual stream, its initial value, normed rows, backout, GEMM out
@@ -132,6 +133,13 @@ Workspace carve(const nc_model_desc* m, int B, int T, void* base) {
             const size_t n = nc_gemm_decode_partial_bytes_auto((int)M, sh[0], sh[1]);
             gneed = n > gneed ? n : gneed;
         }
+    } else {
+        const int shapes[2][2] = {{(int)E, m->n_head * 128}, {(int)E, (int)(4 * E)}};
+        for (auto& sh : shapes) {
+            const int ks = nc_gemm_prompt_splits((int)M, sh[0], sh[1]);
+            const size_t n = ks > 1 ? ks * M * sh[0] * sizeof(float) : 0;
+            gneed = n > gneed ? n : gneed;
+        }
     }
     w.gemm_part_bytes = gneed;
     w.gemm_parts = c.take<uint8_t>(gneed);
@@ -199,6 +207,12 @@ struct LinearRunner {
         }
         // large M: explicit convert pass, tiled GEMM; relu^2 (out_kind 2) is a separate kernel there
         TRY(nc_launch_convert_only(in, (int64_t)rows * K, w.a8, w.inv + site, w.site(site), s));
+        const int splits = src && out_kind == 0 && segs.nseg == 1 ? nc_gemm_prompt_splits(rows, N, K) : 1;
+        if (splits > 1) {
+            TRY(nc_launch_gemm_partials(w.a8, w8, (float*)pbuf, w.gemm_part_bytes, splits, rows, N, K, s));
+            *src = NcPartialSrc{(const float*)pbuf, splits, N, (size_t)rows * N, w.site(site), inv_w, 0x7fffffff, 0x7fffffff};
+            return 0;
+        }
         if (out_kind == 2) {
             // relu^2 and its amax in the GEMM's epilogue; past the 32-bit buffer offsets, the plain-load kernel and a separate pass
             if ((long)rows * K < (1L << 31) && (long)N * K < (1L << 31))

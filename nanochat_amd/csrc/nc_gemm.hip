@@ -856,6 +856,9 @@ __device__ __forceinline__ void dr_fetch(const uint8_t* A, int a_bytes, const ui
 // of three steps ahead are on their way into LDS while one is multiplied, and a step costs its MFMAs or the L2's bandwidth, whichever
 // is longer.  Past the end of K the loads are issued all the same (the first step's operands again, into stages nobody reads), so that
 // the count the barrier waits for is the same in every step.
+//
+// OUT_KIND 3: the K-steps are dealt to gridDim.y workgroups per tile, which leave raw fp32 sums ([share][M][N] at ep.out) for the row pass
+// that adds the linear's output to the residual stream anyway (nc_gemm_prompt_splits).
 template <int BM, int OUT_KIND>
 __global__ __launch_bounds__(256) void gemm_dr_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, EpilogueArgs ep, int M,
                                                       int N, int K, int tiles_m, int tiles_n) {
@@ -881,7 +884,9 @@ __global__ __launch_bounds__(256) void gemm_dr_kernel(const uint8_t* __restrict_
         const int rb = n0 + 8 * g.wave + 32 * i + g.sub;
         vo_b[i] = rb < N ? (uint32_t)rb * (uint32_t)K + g.gch * 16 : NC_BUF_OOB;
     }
-    const int ksteps = K / 128;
+    const int k_first = OUT_KIND == 3 ? (int)((long)(K / 128) * blockIdx.y / gridDim.y) : 0;
+    const int ksteps = OUT_KIND == 3 ? (int)((long)(K / 128) * (blockIdx.y + 1) / gridDim.y) - k_first : K / 128;
+    A += k_first * 128, B += k_first * 128;
 
     v4f acc[WTM][4];
 #pragma unroll
@@ -890,7 +895,7 @@ __global__ __launch_bounds__(256) void gemm_dr_kernel(const uint8_t* __restrict_
         for (int j = 0; j < 4; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
     auto fetch = [&](int t) {
-        dr_fetch<A_P>(A, M * K, B, N * K, lds + (t & 3) * STAGE + wave_s * 1024, BM * 128, vo_a, vo_b, t < ksteps ? t * 128 : 0);
+        dr_fetch<A_P>(A, M * K - k_first * 128, B, N * K - k_first * 128, lds + (t & 3) * STAGE + wave_s * 1024, BM * 128, vo_a, vo_b, t < ksteps ? t * 128 : 0);
     };
     auto compute = [&](int t) {
         const uint8_t* st = lds + (t & 3) * STAGE;
@@ -930,11 +935,23 @@ __global__ __launch_bounds__(256) void gemm_dr_kernel(const uint8_t* __restrict_
     for (int i = 0; i < WTM; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++) asm volatile("" : "+a"(acc[i][j]));
-    const float inv_a = *ep.inv_a;
-    float sc[4];
+    if constexpr (OUT_KIND == 3) {
+        float* const out = (float*)ep.out + (size_t)blockIdx.y * M * N;
 #pragma unroll
-    for (int i = 0; i < 4; i++) sc[i] = ep.inv_b[i < ep.segs.nseg ? i : 0];
-    bl_epilogue<BM, 128, 2, 2, OUT_KIND>(acc, lds, ep, inv_a, sc, m0, n0, M, N);
+        for (int i = 0; i < WTM; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int m = m0 + g.wm * (BM / 2) + 16 * i + g.frow, n = n0 + g.wn * 64 + 16 * j + 4 * g.kb;
+                if (m < M && n < N) *(v4f*)(out + (size_t)m * N + n) = acc[i][j];
+            }
+        return;
+    } else {
+        const float inv_a = *ep.inv_a;
+        float sc[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) sc[i] = ep.inv_b[i < ep.segs.nseg ? i : 0];
+        bl_epilogue<BM, 128, 2, 2, OUT_KIND>(acc, lds, ep, inv_a, sc, m0, n0, M, N);
+    }
 }
 
 // Epilogue of the persistent kernel: the wave's 64 x (128 | 64) block leaves 16 rows at a time through a 4 KB LDS region of
@@ -1232,13 +1249,13 @@ static int launch_dln(int nj, int a_fmt, const uint8_t* a, const uint8_t* b, con
 }
 
 template <int BM, int OUT_KIND>
-static int launch_dr_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s) {
+static int launch_dr_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s, int splits = 1) {
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + 127) / 128;
     const size_t lds_bytes = 4 * (size_t)(BM + 128) * 128;
     const void* fn = (const void*)gemm_dr_kernel<BM, OUT_KIND>;
     hipError_t e = reserve_lds(fn, (int)lds_bytes);
     if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
-    hipLaunchKernelGGL((gemm_dr_kernel<BM, OUT_KIND>), dim3(tiles_m * tiles_n), dim3(256), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
+    hipLaunchKernelGGL((gemm_dr_kernel<BM, OUT_KIND>), dim3(tiles_m * tiles_n, splits), dim3(256), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
     return 0;
 }
 // e4m3 operands, bf16 or relu^2 output, K a multiple of 128
@@ -1350,15 +1367,16 @@ int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const
                 // a prompt of a few hundred to two thousand rows against a narrow weight leaves CUs without a 128x128 tile, and each
                 // tile's K loop is one dependent step after the other: lower tiles put a workgroup on more CUs with less MFMA work per
                 // step, as long as they still fit one round of one workgroup per CU (512..1024 rows x 1664 columns with 64-row tiles:
-                // 8 us against 10.7 at K = 1664, 21 against 31 at K = 6656; 1792 rows with 96-row tiles: 10.0 / 11.5 and 27.9 / 30.5)
-                if (which == 5 && out_kind != 2) {
+                // 8 us against 10.7 at K = 1664, 21 against 31 at K = 6656; 1792 rows with 96-row tiles: 10.0 / 11.5 and 27.9 / 30.5; the same for
+                // the relu^2 linear where it has that few: 170 x 4096 x 1024 12 us against 9, depth 26, 200 tokens 2356 -> 2257 us a prompt)
+                if (which == 5) {
                     const long tn = (N + 127) / 128;
                     if ((long)((M + 63) / 64) * tn <= cus) which = 10;
                     else if ((long)((M + 95) / 96) * tn <= cus) which = 11;
                     // the same tiles fed straight into a ring of four LDS stages where K allows it: three K-steps of operands on their
                     // way instead of two and no ds_write phase (1792 x 1664 x 6656: 27.5 -> 25.6 us, 1024 rows: 21.9 -> 20.8 us; what is
                     // left is the L2's bandwidth: 28 KB per K-step and CU for tiles this small)
-                    if (which >= 10 && K % 128 == 0 && out_kind == 0) which += 6;
+                    if (which >= 10 && K % 128 == 0 && out_kind != 1) which += 6;
                 }
             }
         }
@@ -1393,6 +1411,33 @@ int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const
     else if (which >= 12) rc = launch_dln(which - 8, 0, a, b, ep, M, N, K, s);
     else NC_FAIL(-1, "fp8_gemm: unknown kernel selector %d", force_kernel);
     if (rc) return rc;
+    NC_CHECK_LAUNCH("fp8_gemm");
+    return 0;
+}
+
+// Shares of K that a linear of more than 128 rows is cut into when its consumer adds partial sums: as many as give every CU a workgroup of 64 x 128
+// outputs, of four steps at least (what the ring of stages holds; of eight 0 to 2 % slower or faster, of two the same).  A prompt of a few hundred
+// tokens leaves most CUs without a tile of a narrow weight otherwise, and K = 4 E is one chain of 32 to 52 steps of half a microsecond (170 rows,
+// 1024 x 4096: 24 tiles, 17 us).  us a prompt, in one piece / in shares: depth 16, 170 tokens 1208 / 1045, depth 20, 250 1776 / 1492, 500 1965 / 1756,
+// depth 26, 200 2257 / 1968, 400 2624 / 2418, depth 12, 1000 1096 / 1054.  From more than cus / 2 tiles on there is nothing to fill.  (The q|k|v linear
+// has three times the tiles and a consumer that reads fp32 sums more slowly than bf16: 1045 / 1087.)
+int nc_gemm_prompt_splits(int M, int N, int K) {
+    if (M <= 128 || K % 128 != 0 || N % 8 != 0 || N > 8192 || (long)M * K >= (1L << 31) || (long)N * K >= (1L << 31)) return 1;
+    const long tiles = (long)((M + 63) / 64) * ((N + 127) / 128);
+    long s = cu_count() / tiles;
+    if (s > 8) s = 8;
+    if (s > K / 512) s = K / 512;
+    return s < 1 ? 1 : (int)s;
+}
+
+int nc_launch_gemm_partials(const uint8_t* a, const uint8_t* b, float* parts, size_t part_bytes, int splits, int M, int N, int K, hipStream_t s) {
+    NC_CHECK_ARG(a && b && parts && splits > 1 && splits <= K / 128 && splits <= nc_gemm_prompt_splits(M, N, K), "fp8_gemm: %d shares of K=%d", splits, K);
+    NC_CHECK_ARG((((uintptr_t)a | (uintptr_t)b | (uintptr_t)parts) & 15) == 0 && part_bytes >= (size_t)splits * M * N * sizeof(float),
+                 "fp8_gemm: %d shares need %zu bytes of 16-byte aligned room", splits, (size_t)splits * M * N * sizeof(float));
+    EpilogueArgs ep{};
+    ep.out = parts;
+    NcProfScope prof(1, 2.0 * M * N * K, s, ((int64_t)N << 32) | (uint32_t)K);
+    if (const int rc = launch_dr_as<64, 3>(a, b, ep, M, N, K, s, splits)) return rc;
     NC_CHECK_LAUNCH("fp8_gemm");
     return 0;
 }

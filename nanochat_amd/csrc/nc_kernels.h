@@ -32,6 +32,10 @@ int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const
                    size_t workspace_bytes, hipStream_t s, int a_fmt = 0,    // a_fmt: 0 e4m3fn, 1 e5m2 (kernels 5, 8, 9)
                    uint32_t* out_amax = nullptr);                            // out_kind 2: bf16 relu(v)^2, amax of it published here
 
+// raw fp32 sums [splits][M][N] of a linear of more than 128 rows for a consumer of NcPartialSrc; nc_gemm_prompt_splits: how many shares pay (1: none)
+int nc_gemm_prompt_splits(int M, int N, int K);
+int nc_launch_gemm_partials(const uint8_t* a, const uint8_t* b, float* parts, size_t part_bytes, int splits, int M, int N, int K, hipStream_t s);
+
 // small-M path (nc_gemm_decode.hip): A is e4m3 (+inv_a) or bf16 (+amax, quantized inside the kernel)
 // out_kind: 0 bf16, 1 softcapped fp32, 2 bf16 relu^2 with amax of the result into out_amax.
 // With K split over workgroups the raw fp32 sums land in `partials` [ksplits][M][N] and a consumer finishes them.

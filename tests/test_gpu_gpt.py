@@ -404,6 +404,12 @@ def test_long_prefill_matches_oracle(cfg_kwargs, B, P, trained_like):
     assert cache.get_pos() == P + 2
 
 
+@pytest.mark.parametrize("heads,B,P", [(3, 1, 129), (5, 1, 193), (8, 1, 131), (5, 2, 320), (2, 3, 70)])
+def test_prompt_whose_narrow_projections_are_shared_out(heads, B, P):
+    """129 to some hundred rows: the projections leave partial sums that the row pass adds (2 to 5 shares of uneven length, ragged last tiles)."""
+    test_long_prefill_matches_oracle(dict(sequence_len=512, vocab_size=512, n_layer=2, n_head=heads, n_kv_head=heads, n_embd=128 * heads, window_pattern="SL"), B, P, False)
+
+
 def test_ragged_rows():
     """Per-row cache lengths (outside the reference's GPT.forward, inside FA3's signature): every row
     must equal the same row run alone."""
