@@ -149,6 +149,102 @@ __global__ __launch_bounds__(256) void latent_simple_kernel(NcLatentGeom g, cons
     }
 }
 
+// ------------------------------------------------------------------------------------------------ latent space, 32-bit, few query rows
+// One workgroup per query row and share of its keys, so that a step of a few rows fills the chip; a wave takes a run of keys.  16 lanes hold one key, four
+// values of each piece of 64 a lane: a load is whole lines, and what was read for the score is in registers for the sum.  Every 16 lanes keep a softmax of
+// their own (four chains a score, summed over the lanes); the lane groups, then the waves, then the shares are merged by their maxima.
+// latent_simple_kernel, a thread to a key and then a thread to a column, waits for each of its loads: 4 rows of 5 heads, rank 512, 300 keys 57.5 us, here
+// 7.7 and 3.0 for the merge (a step of a 3-layer model 360 -> 255).
+constexpr int STEP32_KEYS = 4;                                // keys per lane group and batch
+template <int J>
+__global__ __launch_bounds__(256) void latent_step32_kernel(NcLatentGeom g, const float* __restrict__ q_lat, const float* __restrict__ cache,
+                                                            const int32_t* __restrict__ seqlens, float* __restrict__ out, float* __restrict__ partials,
+                                                            int splits) {
+    __shared__ __align__(16) float sums[4][64 * J];
+    __shared__ float ms[4], ls[4];
+    const int rw = g.rank_p + g.rot_p, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), grp = lane >> 4, sub = lane & 15;
+    const int64_t row = blockIdx.x;
+    const int b = (int)(row / ((int64_t)g.T * g.heads)), t = (int)(row / g.heads % g.T);
+    const int n = min(seqlens[b] + t, g.Tmax - 1) + 1, share = ((n + 4 * splits - 1) / (4 * splits) + 3) & ~3;
+    const int k_begin = ((int)blockIdx.y * 4 + wave) * share, k_end = min(k_begin + share, n);
+    const float* const keys = cache + (int64_t)b * g.Tmax * rw;
+    const v4f zero{0.f, 0.f, 0.f, 0.f};
+    v4f q[J], acc[J];
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        const int d = 64 * j + 4 * sub;
+        q[j] = d < rw ? *(const v4f*)(q_lat + row * rw + d) : zero;
+        acc[j] = zero;
+    }
+    float m_run = LA_M_FLOOR, l_run = 0.f;
+    for (int k0 = k_begin; k0 < k_end; k0 += 4 * STEP32_KEYS) {
+        v4f kr[STEP32_KEYS][J];
+        float s[STEP32_KEYS], m_new = m_run;
+        // (a place past the end of the run takes the run's last key, which this row sees, with weight 0)
+#pragma unroll
+        for (int u = 0; u < STEP32_KEYS; u++) {
+            const float* const src = keys + (int64_t)min(k0 + 4 * u + grp, k_end - 1) * rw;
+#pragma unroll
+            for (int j = 0; j < J; j++) {
+                const int d = 64 * j + 4 * sub;
+                kr[u][j] = d < rw ? *(const v4f*)(src + d) : zero;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < STEP32_KEYS; u++) {
+            v4f d = zero;
+#pragma unroll
+            for (int j = 0; j < J; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) d[r] = fmaf(kr[u][j][r], q[j][r], d[r]);
+            s[u] = row16_sum((d[0] + d[1]) + (d[2] + d[3])) * g.scale;
+            if (k0 + 4 * u + grp < k_end) m_new = fmaxf(m_new, s[u]);
+        }
+        const float corr = expf(m_run - m_new);
+        m_run = m_new, l_run *= corr;
+#pragma unroll
+        for (int j = 0; j < J; j++) acc[j] *= corr;
+#pragma unroll
+        for (int u = 0; u < STEP32_KEYS; u++) {
+            const float p = k0 + 4 * u + grp < k_end ? expf(s[u] - m_run) : 0.f;
+            l_run += p;
+#pragma unroll
+            for (int j = 0; j < J; j++) acc[j] += kr[u][j] * p;
+        }
+    }
+    float mt = fmaxf(m_run, __shfl_xor(m_run, 16));
+    mt = fmaxf(mt, __shfl_xor(mt, 32));
+    const float w = expf(m_run - mt);
+    l_run *= w;
+    l_run += __shfl_xor(l_run, 16);
+    l_run += __shfl_xor(l_run, 32);
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+        v4f a = acc[j] * w;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            a[r] += __shfl_xor(a[r], 16);
+            a[r] += __shfl_xor(a[r], 32);
+        }
+        if (grp == 0) *(v4f*)(&sums[wave][64 * j + 4 * sub]) = a;
+    }
+    if (lane == 0) ms[wave] = mt, ls[wave] = l_run;
+    __syncthreads();
+    mt = fmaxf(fmaxf(ms[0], ms[1]), fmaxf(ms[2], ms[3]));
+    float f[4], lt = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) f[i] = expf(ms[i] - mt), lt += f[i] * ls[i];
+    float* const part = partials + (row * splits + blockIdx.y) * (g.rank_p + 4);
+    if (splits > 1 && threadIdx.x == 0) part[0] = mt, part[1] = lt;
+    const int c = 4 * threadIdx.x;
+    if (c >= g.rank_p) return;
+    v4f y = zero;
+#pragma unroll
+    for (int i = 0; i < 4; i++) y += *(const v4f*)(&sums[i][c]) * f[i];
+    if (splits > 1) *(v4f*)(part + 4 + c) = y;
+    else *(v4f*)(out + row * g.rank_p + c) = y / lt;
+}
+
 // ------------------------------------------------------------------------------------------------ latent space, 32-bit, many query rows
 // 16 query rows (row = token * heads + head of one batch row) per workgroup, keys 64 at a time, on v_mfma_f32_16x16x4_f32: a lane supplies 16
 // bytes of row lane % 16 from piece lane / 16, which is four instructions (which dimension or key a lane's values stand for does not matter as
@@ -413,7 +509,9 @@ __global__ __launch_bounds__(MFMA_THREADS) void latent_mfma_kernel(NcLatentGeom 
 }
 
 constexpr int MAX_SPLITS = 32;
-__global__ __launch_bounds__(128) void latent_combine_kernel(const float* __restrict__ partials, int splits, int rank_p, bf16_t* __restrict__ out) {
+// (the maxima are in log2 units under bf16, in natural ones under 32-bit)
+template <typename T>
+__global__ __launch_bounds__(128) void latent_combine_kernel(const float* __restrict__ partials, int splits, int rank_p, T* __restrict__ out) {
     __shared__ float weight[64];
     const int64_t row = blockIdx.x;
     const int stride = rank_p + 4;
@@ -421,7 +519,7 @@ __global__ __launch_bounds__(128) void latent_combine_kernel(const float* __rest
     if (threadIdx.x < 64) {                     // lane = split (MAX_SPLITS <= 64)
         const bool in = (int)threadIdx.x < splits;
         const float m = in ? part[(int64_t)threadIdx.x * stride] : LA_M_FLOOR, l = in ? part[(int64_t)threadIdx.x * stride + 1] : 0.f;
-        const float w = __builtin_amdgcn_exp2f(m - wave_max(m));
+        const float top = wave_max(m), w = sizeof(T) == 4 ? expf(m - top) : __builtin_amdgcn_exp2f(m - top);
         const float total = wave_sum(l * w);
         weight[threadIdx.x] = total > 0.f ? w / total : 0.f;
     }
@@ -688,10 +786,22 @@ int nc_launch_latent_append(int dtype, const NcLatentGeom& g, void* proj, int ld
     return 0;
 }
 
+namespace {
+// 32-bit rows for latent_step32_kernel, and the workgroups that share a row's keys: two per compute unit, 64 keys each at least.  (One token per
+// sequence: portions of several would gain as well, 30 tokens behind 400 599 -> 497 us, but a prompt's rows are to be about as exact in portions as
+// in one piece, and the scores here, in 64 chains, are twice as exact as those of the kernels that take a whole prompt.)
+bool step32_ok(const NcLatentGeom& g) { return g.T == 1 && g.rank_p % 4 == 0 && g.rank_p + g.rot_p <= 576; }
+int step32_splits(const NcLatentGeom& g) {
+    const int rows = g.B * g.T * g.heads, blocks = (g.pos_max + g.T + 63) / 64;
+    int splits = 2 * nc_cu_count() / rows;
+    if (splits > blocks) splits = blocks;
+    return splits < 1 ? 1 : splits > MAX_SPLITS ? MAX_SPLITS : splits;
+}
+}  // namespace
+
 size_t nc_latent_partial_bytes(int dtype, const NcLatentGeom& g) {
-    if (!mfma_variant(dtype, g)) return 0;
     // sized for any cache length the step may see: the split count only falls with it
-    const int splits = mfma_splits(g);
+    const int splits = mfma_variant(dtype, g) ? mfma_splits(g) : dtype && step32_ok(g) ? step32_splits(g) : 1;
     return splits > 1 ? (size_t)g.B * g.T * g.heads * splits * (g.rank_p + 4) * sizeof(float) : 0;
 }
 
@@ -712,7 +822,7 @@ int nc_launch_latent_attention(int dtype, const NcLatentGeom& g, const void* q_l
                                       : launch_mfma<4, 5>(g, q, c, seqlens, o, p, splits, s);
         if (rc) return rc;
         if (splits > 1) {
-            hipLaunchKernelGGL(latent_combine_kernel, dim3(rows), dim3(128), 0, s, p, splits, g.rank_p, o);
+            hipLaunchKernelGGL((latent_combine_kernel<bf16_t>), dim3(rows), dim3(128), 0, s, p, splits, g.rank_p, o);
             NC_CHECK_LAUNCH("latent_combine");
         }
         return 0;
@@ -726,6 +836,14 @@ int nc_launch_latent_attention(int dtype, const NcLatentGeom& g, const void* q_l
         else if (g.rank_p <= 256) GO32(2);
         else GO32(4);
 #undef GO32
+    } else if (dtype && step32_ok(g)) {
+        const int splits = step32_splits(g);
+        NC_CHECK_ARG(splits == 1 || (partials && partial_bytes >= nc_latent_partial_bytes(dtype, g)), "latent_attention: partial buffer too small");
+#define STEP32(J) hipLaunchKernelGGL((latent_step32_kernel<J>), dim3(rows, splits), dim3(256), 0, s, g, (const float*)q_lat, (const float*)cache, seqlens, (float*)out_lat, (float*)partials, splits)
+        if (g.rank_p + g.rot_p <= 320) STEP32(5);
+        else STEP32(9);
+#undef STEP32
+        if (splits > 1) hipLaunchKernelGGL((latent_combine_kernel<float>), dim3(rows), dim3(128), 0, s, (const float*)partials, splits, g.rank_p, (float*)out_lat);
     } else if (dtype)
         hipLaunchKernelGGL((latent_simple_kernel<float>), dim3(rows), dim3(256), bytes, s, g, (const float*)q_lat, (const float*)cache, seqlens, (float*)out_lat);
     else

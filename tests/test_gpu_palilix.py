@@ -200,6 +200,30 @@ def test_32_bit_scores_of_many_rows_are_as_exact_as_of_few():
     assert whole < 1.66 * portions, whole / portions
 
 
+@pytest.mark.parametrize("heads,rank,rot_dim", [(5, 512, 64), (1, 256, 32), (3, 200, 64), (2, 320, 0), (7, 512, 32)])
+def test_32_bit_steps_whose_keys_are_shared_out(heads, rank, rot_dim):
+    """Single tokens and portions of a few behind 0, 1, 63, 64, 65 and 300 cached ones: runs of keys that are empty, ragged or a single key, one and several
+    shares of a row's keys, alone and for three sequences of different lengths."""
+    say(f"32-bit steps, {heads} heads, rank {rank}, {rot_dim} rotated")
+    cfg = config([(latent(heads=heads, dim=32, rot_dim=rot_dim, vdim=32, kv_rank=rank, scale=0.2), None)], width=128, vocab=90)
+    w = weights(cfg, seed=5)
+    model, w64 = build(cfg, w, torch.float32), {k: v.double() for k, v in w.items()}
+    for cuts in ([1] * 5, [62, 1, 1, 1, 1], [300, 1, 2, 5], [63, 7]):
+        n = sum(cuts)
+        check(run(model, tokens(cfg, n), cuts), ref.forward(cfg, w64, tokens(cfg, n)), torch.float32, f"portions {cuts}")
+    lengths = [3, 130, 65]
+    seqs = [tokens(cfg, n + 2, seed=60 + n) for n in lengths]
+    cache = model.new_cache(len(seqs), 160)
+    for r, (s, n) in enumerate(zip(seqs, lengths)):
+        alone = model.new_cache(1, 160)
+        model.forward_last(ids(s[:n]), kv_cache=alone)
+        cache.load_row(r, alone)
+    for i in range(2):
+        got = model.forward(torch.tensor([s[n + i:n + i + 1] for s, n in zip(seqs, lengths)], device=DEV), kv_cache=cache)
+        for r, (s, n) in enumerate(zip(seqs, lengths)):
+            check(got[r], ref.forward(cfg, w64, s[:n + i + 1])[-1:], torch.float32, f"step {i}, row {r}")
+
+
 @pytest.mark.parametrize("width", [64, 512, 1024])
 @pytest.mark.parametrize("ff", [2048, 2112, 1984])
 def test_32_bit_shares_that_begin_in_the_middle_of_a_step(width, ff):
