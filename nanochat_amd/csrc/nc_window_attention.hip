@@ -13,6 +13,7 @@
 //
 //   window_few_kernel      decode and short portions: 16 query rows of one kv head, keys dealt to waves and workgroups
 //   window_prefill_kernel  long portions: waves of 32 queries of one head, keys through LDS; two waves may share the keys of their queries
+//   window_step32_kernel   32-bit, one token: 16 lanes to a key, keys dealt to waves and workgroups
 //   window_simple_kernel   any sizes, either storage type
 #include "nc_stack.h"
 
@@ -156,6 +157,108 @@ __global__ __launch_bounds__(256) void window_simple_kernel(NcWindowGeom g, cons
         if (c >= g.vdim_p) break;
         st_f32(out + m * ldo + h * g.vdim_p + c, acc[i] / l_run * g.out_scale);
     }
+}
+
+// ------------------------------------------------------------------------------------------------ one token, 32-bit
+// One workgroup per query row and share of its keys, a wave takes a run of them.  16 lanes hold one key and its value, four numbers of each piece of 64 a
+// lane, in whole lines; every 16 lanes keep a softmax of their own, and lane groups, waves and shares are merged by their maxima.  window_simple_kernel,
+// a thread to a key and then a thread to a column, waits for each of its loads and leaves the chip to as many workgroups as there are rows: 3 rows of 5
+// heads, 480 keys 38.5 us; with its merge a step of four layers 298 -> 211.
+constexpr int STEP32_KEYS = 4;                                // keys per lane group and batch
+template <int QJ, int VJ>
+__global__ __launch_bounds__(256) void window_step32_kernel(NcWindowGeom g, const float* __restrict__ q, int ldq, const float* __restrict__ cache,
+                                                            const float* __restrict__ sink, const int32_t* __restrict__ seqlens, float* __restrict__ out, int ldo,
+                                                            float* __restrict__ partials, int splits) {
+    __shared__ __align__(16) float sums[4][64 * VJ];
+    __shared__ float ms[4], ls[4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), grp = lane >> 4, sub = lane & 15;
+    const int b = (int)blockIdx.x / g.heads, h = (int)blockIdx.x % g.heads, head_w = g.dim_p + g.vdim_p, rw = g.kv_heads * head_w;
+    const int pos = min(seqlens[b], g.Tmax - 1);
+    const KeyList list = key_list(g, pos, pos);
+    const int share = ((list.count + 4 * splits - 1) / (4 * splits) + 3) & ~3, v_begin = ((int)blockIdx.y * 4 + wave) * share, v_end = min(v_begin + share, list.count);
+    const float* const keys = cache + (int64_t)b * g.Tmax * rw + h / (g.heads / g.kv_heads) * head_w;
+    const v4f zero{0.f, 0.f, 0.f, 0.f};
+    v4f qf[QJ], acc[VJ];
+#pragma unroll
+    for (int j = 0; j < QJ; j++) {
+        const int d = 64 * j + 4 * sub;
+        qf[j] = d < g.dim_p ? *(const v4f*)(q + (int64_t)b * ldq + h * g.dim_p + d) : zero;
+    }
+#pragma unroll
+    for (int j = 0; j < VJ; j++) acc[j] = zero;
+    const bool has_sink = blockIdx.y == 0 && wave == 0 && grp == 0;
+    float m_run = has_sink ? sink[h] : WA_M_FLOOR, l_run = has_sink ? 1.f : 0.f;
+    for (int v0 = v_begin; v0 < v_end; v0 += 4 * STEP32_KEYS) {
+        v4f kf[STEP32_KEYS][QJ], vf[STEP32_KEYS][VJ];
+        float s[STEP32_KEYS], m_new = m_run;
+        // (a place past the end of the run takes the run's last key, which this row sees, with weight 0)
+#pragma unroll
+        for (int u = 0; u < STEP32_KEYS; u++) {
+            const float* const src = keys + (int64_t)list.key(min(v0 + 4 * u + grp, v_end - 1)) * rw;
+#pragma unroll
+            for (int j = 0; j < QJ; j++) {
+                const int d = 64 * j + 4 * sub;
+                kf[u][j] = d < g.dim_p ? *(const v4f*)(src + d) : zero;
+            }
+#pragma unroll
+            for (int j = 0; j < VJ; j++) {
+                const int d = 64 * j + 4 * sub;
+                vf[u][j] = d < g.vdim_p ? *(const v4f*)(src + g.dim_p + d) : zero;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < STEP32_KEYS; u++) {
+            v4f d = zero;
+#pragma unroll
+            for (int j = 0; j < QJ; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) d[r] = fmaf(kf[u][j][r], qf[j][r], d[r]);
+            s[u] = row16_sum((d[0] + d[1]) + (d[2] + d[3])) * g.scale;
+            if (v0 + 4 * u + grp < v_end) m_new = fmaxf(m_new, s[u]);
+        }
+        const float corr = expf(m_run - m_new);
+        m_run = m_new, l_run *= corr;
+#pragma unroll
+        for (int j = 0; j < VJ; j++) acc[j] *= corr;
+#pragma unroll
+        for (int u = 0; u < STEP32_KEYS; u++) {
+            const float p = v0 + 4 * u + grp < v_end ? expf(s[u] - m_run) : 0.f;
+            l_run += p;
+#pragma unroll
+            for (int j = 0; j < VJ; j++) acc[j] += vf[u][j] * p;
+        }
+    }
+    float mt = fmaxf(m_run, __shfl_xor(m_run, 16));
+    mt = fmaxf(mt, __shfl_xor(mt, 32));
+    const float w = expf(m_run - mt);
+    l_run *= w;
+    l_run += __shfl_xor(l_run, 16);
+    l_run += __shfl_xor(l_run, 32);
+#pragma unroll
+    for (int j = 0; j < VJ; j++) {
+        v4f a = acc[j] * w;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            a[r] += __shfl_xor(a[r], 16);
+            a[r] += __shfl_xor(a[r], 32);
+        }
+        if (grp == 0) *(v4f*)(&sums[wave][64 * j + 4 * sub]) = a;
+    }
+    if (lane == 0) ms[wave] = mt, ls[wave] = l_run;
+    __syncthreads();
+    mt = fmaxf(fmaxf(ms[0], ms[1]), fmaxf(ms[2], ms[3]));
+    float f[4], lt = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; i++) f[i] = expf(ms[i] - mt), lt += f[i] * ls[i];
+    float* const part = partials + ((int64_t)blockIdx.x * splits + blockIdx.y) * (g.vdim_p + 4);
+    if (splits > 1 && threadIdx.x == 0) part[0] = mt, part[1] = lt;
+    const int c = 4 * threadIdx.x;
+    if (c >= g.vdim_p) return;
+    v4f y = zero;
+#pragma unroll
+    for (int i = 0; i < 4; i++) y += *(const v4f*)(&sums[i][c]) * f[i];
+    if (splits > 1) *(v4f*)(part + 4 + c) = y;
+    else *(v4f*)(out + (int64_t)b * ldo + h * g.vdim_p + c) = y / lt * g.out_scale;
 }
 
 // ------------------------------------------------------------------------------------------------ few query rows
@@ -304,16 +407,18 @@ __global__ __launch_bounds__(256) void window_few_kernel(NcWindowGeom g, const b
     }
 }
 
-// One wave per (token, head): lane = split for the weights, then four columns per lane and step.
+// One wave per (token, head): lane = split for the weights, then four columns per lane and step.  (The maxima are in log2 units under bf16, in natural
+// ones under 32-bit.)
+template <typename T>
 __global__ __launch_bounds__(64) void window_combine_kernel(const float* __restrict__ partials, int splits, int heads, int vdim_p, float scale,
-                                                            bf16_t* __restrict__ out, int ldo) {
+                                                            T* __restrict__ out, int ldo) {
     __shared__ float weight[64];
     const int64_t row = blockIdx.x;
     const int stride = vdim_p + 4;
     const float* part = partials + row * splits * stride;
     const bool in = (int)threadIdx.x < splits;
     const float m = in ? part[(int64_t)threadIdx.x * stride] : WA_M_FLOOR, l = in ? part[(int64_t)threadIdx.x * stride + 1] : 0.f;
-    const float w = __builtin_amdgcn_exp2f(m - wave_max(m));
+    const float top = wave_max(m), w = sizeof(T) == 4 ? expf(m - top) : __builtin_amdgcn_exp2f(m - top);
     const float total = wave_sum(l * w);
     weight[threadIdx.x] = total > 0.f ? w * scale / total : 0.f;
     __syncthreads();
@@ -520,6 +625,15 @@ int few_splits(const NcWindowGeom& g) {
     if (splits > by_keys) splits = by_keys;
     return splits < 1 ? 1 : splits > MAX_SPLITS ? MAX_SPLITS : splits;
 }
+// 32-bit rows for window_step32_kernel, and the workgroups that share a row's keys: two per compute unit, 64 keys each at least
+bool step32_ok(int dtype, const NcWindowGeom& g) { return dtype == 1 && g.T == 1 && g.dim_p <= 256 && g.vdim_p <= 256; }
+int step32_splits(const NcWindowGeom& g) {
+    const int64_t most = (int64_t)g.window + g.keep_first;
+    const int keys = most < g.pos_max + 1 ? (int)most : g.pos_max + 1, blocks = (keys + 63) / 64;
+    int splits = 2 * nc_cu_count() / (g.B * g.heads);
+    if (splits > blocks) splits = blocks;
+    return splits < 1 ? 1 : splits > MAX_SPLITS ? MAX_SPLITS : splits;
+}
 bool use_few(const NcWindowGeom& g) { return g.T < PREFILL_MIN_TOKENS; }
 
 template <int DQ, int DV>
@@ -530,7 +644,7 @@ int launch_few(const NcWindowGeom& g, const bf16_t* q, int ldq, const bf16_t* ca
                        splits, groups);
     NC_CHECK_LAUNCH("window_few");
     if (splits > 1) {
-        hipLaunchKernelGGL(window_combine_kernel, dim3(g.B * g.T * g.heads), dim3(64), 0, s, partials, splits, g.heads, g.vdim_p, g.out_scale, out, ldo);
+        hipLaunchKernelGGL((window_combine_kernel<bf16_t>), dim3(g.B * g.T * g.heads), dim3(64), 0, s, partials, splits, g.heads, g.vdim_p, g.out_scale, out, ldo);
         NC_CHECK_LAUNCH("window_combine");
     }
     return 0;
@@ -565,8 +679,7 @@ int nc_launch_window_append(int dtype, const NcWindowGeom& g, void* proj, int ld
 }
 
 size_t nc_window_partial_bytes(int dtype, const NcWindowGeom& g) {
-    if (!mfma_ok(dtype, g) || !use_few(g)) return 0;
-    const int splits = few_splits(g);
+    const int splits = step32_ok(dtype, g) ? step32_splits(g) : mfma_ok(dtype, g) && use_few(g) ? few_splits(g) : 1;
     return splits > 1 ? (size_t)g.B * g.T * g.heads * splits * (g.vdim_p + 4) * sizeof(float) : 0;
 }
 
@@ -597,6 +710,20 @@ int nc_launch_window_attention(int dtype, const NcWindowGeom& g, const void* q, 
     }
     NC_CHECK_ARG(g.vdim_p <= 256 * SIMPLE_COLS && (g.dim_p + 256) * 4 <= 64 * 1024 - 64, "window_attention: dim=%d vdim=%d not supported", g.dim_p, g.vdim_p);
     const int bytes = (g.dim_p + 256) * 4;
+    if (step32_ok(dtype, g)) {
+        const int splits = step32_splits(g), rows = g.B * g.heads;
+        NC_CHECK_ARG(splits == 1 || (partials && partial_bytes >= nc_window_partial_bytes(dtype, g)), "window_attention: partial buffer too small");
+#define STEP32(Q, V) \
+    hipLaunchKernelGGL((window_step32_kernel<Q, V>), dim3(rows, splits), dim3(256), 0, s, g, (const float*)q, ldq, (const float*)cache, sink, seqlens, (float*)out, ldo, (float*)partials, splits)
+        if (g.dim_p <= 128 && g.vdim_p <= 128) STEP32(2, 2);
+        else STEP32(4, 4);
+#undef STEP32
+        NC_CHECK_LAUNCH("window_step32");
+        if (splits > 1)
+            hipLaunchKernelGGL((window_combine_kernel<float>), dim3(rows), dim3(64), 0, s, (const float*)partials, splits, g.heads, g.vdim_p, g.out_scale, (float*)out, ldo);
+        NC_CHECK_LAUNCH("window_combine");
+        return 0;
+    }
     if (dtype)
         hipLaunchKernelGGL((window_simple_kernel<float>), dim3(g.B * g.T * g.heads), dim3(256), bytes, s, g, (const float*)q, ldq, (const float*)cache, sink, seqlens,
                            (float*)out, ldo);

@@ -231,6 +231,17 @@ def test_portions_and_decoding(name, dtype):
         check(run(model, toks, cuts), want, dtype, f"{name}, cuts {cuts[:6]}")
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim,window,keep_first", [(5, 5, 128, 128, 512, 0), (4, 2, 160, 48, 100, 5), (6, 1, 96, 250, 64, 64), (2, 1, 256, 16, 1, 0)])
+def test_32_bit_steps_whose_keys_are_shared_out(heads, kv_heads, dim, vdim, window, keep_first):
+    """Heads of one to four pieces of 64 dimensions, whole and ragged, behind 0 to 300 tokens: runs of keys that are empty, ragged or a single key."""
+    say(f"32-bit steps, {heads} heads on {kv_heads}, {dim} and {vdim} dimensions")
+    cfg = mechanism(pair(heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, rot_dims=16, window=window, keep_first=keep_first, left_scale=1.0, **OFF))
+    model, w = build_model(Zodirax, cfg, weights(cfg, seed=3), torch.float32), weights(cfg, seed=3)
+    for cuts in ([1] * 5, [62, 1, 1, 1, 1], [300, 1, 1]):
+        toks = tokens(cfg, sum(cuts))
+        check(run(model, toks, cuts), oracle(cfg, w, toks), torch.float32, f"portions {cuts}")
+
+
 def test_long_decoding():
     say("long decoding")
     for name, n in (("odd", 420), ("wide", 300)):
