@@ -94,15 +94,17 @@ class Float8Linear(nn.Linear):
         input = input.to(torch.bfloat16 if COMPUTE_DTYPE == torch.float32 else COMPUTE_DTYPE)
         if input.dtype != torch.bfloat16:
             raise ValueError("Float8Linear: the GPU path computes in bf16")
-        orig_shape = input.shape
-        x2 = input.reshape(-1, orig_shape[-1])
+        # (a matrix passes as it is: a reshape is a view, and a node of its own for the backward to visit)
+        matrix, orig_shape = input.dim() == 2, input.shape
+        x2 = input if matrix else input.reshape(-1, orig_shape[-1])
         if torch.is_grad_enabled() and (x2.requires_grad or self.weight.requires_grad):
             out = _Float8Matmul.apply(x2, self.weight, self)
         else:
             a8, inv_a, _ = ops.fp8_quantize(x2)
             w8, inv_w = self._weight_fp8()
             out = ops.fp8_gemm(a8, w8, inv_a, inv_w)
-        out = out.reshape(*orig_shape[:-1], out.shape[-1])
+        if not matrix:
+            out = out.reshape(*orig_shape[:-1], out.shape[-1])
         if self.bias is not None:
             out = out + self.bias.to(out.dtype)
         return out
