@@ -368,13 +368,13 @@ class GPT(nn.Module):
         ws_ptr, ws_bytes = self._workspace(md, B, T, idx.device)
         if taps is None:
             rc = _lib.lib().nc_gpt_forward(C.byref(md), C.byref(cd), idx.data_ptr(), B, T, logits.data_ptr(), 1 if last_only else 0,
-                                           ws_ptr, ws_bytes, ops.stream_handle())
+                                           ws_ptr, ws_bytes, ops._stream())
         else:
             taps["x"] = torch.empty(cfg.n_layer + 1, B, T, cfg.n_embd, dtype=torch.bfloat16, device=idx.device)
             taps["y"] = torch.empty(cfg.n_layer, B, T, cfg.n_head, cfg.n_embd // cfg.n_head, dtype=torch.bfloat16, device=idx.device)
             rc = _lib.lib().nc_gpt_forward_tapped(C.byref(md), C.byref(cd), idx.data_ptr(), B, T, logits.data_ptr(), 1 if last_only else 0,
                                                   ws_ptr, ws_bytes, taps["x"].data_ptr(), taps["y"].data_ptr(),
-                                                  ops.stream_handle())
+                                                  ops._stream())
         _lib.check(rc)
         kv_cache.prev_embedding = prev_out
         if advance_inside:

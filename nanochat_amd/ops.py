@@ -15,10 +15,10 @@ _SCRATCH = {}
 # The current stream of the current device as an integer.  (torch.cuda.current_stream() makes two objects for it, 3 us of the 17 to 22 that a wrapper
 # here took on the host, and most wrappers ask twice; like pointers, ctypes takes it as it is.)
 if hasattr(torch._C, "_cuda_getCurrentRawStream"):
-    def stream_handle():
+    def _stream():
         return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 else:                                      # a torch without GPU support: the wrappers refuse its tensors
-    def stream_handle():
+    def _stream():
         return torch.cuda.current_stream().cuda_stream
 
 
@@ -34,7 +34,7 @@ def _need_cuda(*tensors):
 
 def _quantize_state(device):
     """The quantizer's state block (zero before first use, left zero by every call), one per device and stream."""
-    key = (device.index, stream_handle())
+    key = (device.index, _stream())
     t = _SCRATCH.get(key)
     if t is None:
         nbytes = _lib.lib().nc_fp8_quantize_state_bytes()
@@ -77,9 +77,9 @@ def fp8_quantize(x, encoder=0, fp8_dtype=torch.float8_e4m3fn, spin_limit=None):
     args = (_ptr(x), 0 if x.dtype == torch.bfloat16 else 1, x.numel(), _FP8_FORMATS[fp8_dtype], _ptr(out), scales.data_ptr(),
             scales.data_ptr() + 4, _ptr(state), encoder)
     if spin_limit is None:
-        rc = _lib.lib().nc_fp8_quantize_tensorwise_fused(*args, stream_handle())
+        rc = _lib.lib().nc_fp8_quantize_tensorwise_fused(*args, _stream())
     else:
-        rc = _lib.lib().nc_fp8_quantize_tensorwise_fused_bounded(*args, int(spin_limit), stream_handle())
+        rc = _lib.lib().nc_fp8_quantize_tensorwise_fused_bounded(*args, int(spin_limit), _stream())
     _lib.check(rc)
     scale, inv = scales.unbind()
     return out, inv, scale
@@ -103,7 +103,7 @@ def fp8_quantize_transposed(x, fp8_dtype=torch.float8_e4m3fn):
     state = _quantize_state(x.device)
     scratch = state.data_ptr() + 4 * 320          # the state block's scratch word
     _lib.check(_lib.lib().nc_fp8_quantize_tensorwise_transposed(_ptr(x), R, Cc, _FP8_FORMATS[fp8_dtype], _ptr(out), _ptr(out_t),
-                                                                scales.data_ptr(), scales.data_ptr() + 4, scratch, stream_handle()))
+                                                                scales.data_ptr(), scales.data_ptr() + 4, scratch, _stream()))
     scale, inv = scales.unbind()
     return out, out_t, inv, scale
 
@@ -114,7 +114,7 @@ def fp8_encode_with_scale(x_bf16, scale, fp8_dtype, encoder=0):
     assert x_bf16.dtype == torch.bfloat16
     x = x_bf16.contiguous()
     out = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-    _lib.check(_lib.lib().nc_fp8_encode_with_scale(_ptr(x), x.numel(), float(scale), _FP8_FORMATS[fp8_dtype], _ptr(out), encoder, stream_handle()))
+    _lib.check(_lib.lib().nc_fp8_encode_with_scale(_ptr(x), x.numel(), float(scale), _FP8_FORMATS[fp8_dtype], _ptr(out), encoder, _stream()))
     return out
 
 
@@ -126,7 +126,7 @@ def fp8_transpose(x8):
     x8 = x8.contiguous()
     R, Cc = x8.shape
     out = torch.empty(Cc, R, dtype=x8.dtype, device=x8.device)
-    _lib.check(_lib.lib().nc_fp8_transpose(_ptr(x8), R, Cc, _ptr(out), stream_handle()))
+    _lib.check(_lib.lib().nc_fp8_transpose(_ptr(x8), R, Cc, _ptr(out), _stream()))
     return out
 
 
@@ -150,7 +150,7 @@ def fp8_gemm_grad(a_e5m2, w8, inv_a, inv_w, kernel=0, out=None):
     if out is None:
         out = torch.empty(M, N, dtype=torch.bfloat16, device=a_e5m2.device)
     _lib.check(_lib.lib().nc_fp8_gemm_tn_grad(_ptr(a_e5m2), _ptr(w8), _ptr(inv_a), _ptr(inv_w), _ptr(out), M, N, K, out.stride(0), kernel,
-                                              stream_handle()))
+                                              _stream()))
     return out
 
 
@@ -159,7 +159,7 @@ def e4m3_encode_with_scale(x_bf16, scale, encoder=0):
     assert x_bf16.dtype == torch.bfloat16
     x = x_bf16.contiguous()
     out = torch.empty(x.shape, dtype=torch.uint8, device=x.device)
-    _lib.check(_lib.lib().nc_e4m3_encode_with_scale(_ptr(x), x.numel(), float(scale), _ptr(out), encoder, stream_handle()))
+    _lib.check(_lib.lib().nc_e4m3_encode_with_scale(_ptr(x), x.numel(), float(scale), _ptr(out), encoder, _stream()))
     return out
 
 
@@ -170,7 +170,7 @@ _GEMM_WS = {}
 def _small_m_workspace(device, M, N, K):
     """Zero-initialised split-K scratch, kept per device and stream (its counter block stays zero between calls)."""
     need = _lib.lib().nc_fp8_small_m_workspace_bytes(M, N, K)
-    key = (device.index, stream_handle())
+    key = (device.index, _stream())
     ws = _GEMM_WS.get(key)
     if ws is None or ws.numel() < need:
         ws = torch.zeros(max(need, 1 << 20), dtype=torch.uint8, device=device)
@@ -202,7 +202,7 @@ def fp8_gemm(a8, w8, inv_a, inv_w, seg_ends=None, softcap=None, kernel=0, out=No
     ws = _small_m_workspace(a8.device, M, N, K) if 1 <= M <= 128 else None
     rc = _lib.lib().nc_fp8_gemm_tn(_ptr(a8), _ptr(w8), _ptr(inv_a), _ptr(inv_w), segs, len(seg_ends), _ptr(out),
                                    1 if softcap is not None else 0, float(softcap or 0.0), M, N, K, out.stride(0), kernel,
-                                   _ptr(ws), ws.numel() if ws is not None else 0, stream_handle())
+                                   _ptr(ws), ws.numel() if ws is not None else 0, _stream())
     _lib.check(rc)
     return out
 
@@ -217,7 +217,7 @@ def fp8_gemm_relu2(a8, w8, inv_a, inv_w, kernel=0):
     out = torch.empty(M, N, dtype=torch.bfloat16, device=a8.device)
     amax = torch.zeros(1, dtype=torch.int32, device=a8.device)
     _lib.check(_lib.lib().nc_fp8_gemm_tn_relu2(_ptr(a8), _ptr(w8), _ptr(inv_a.reshape(-1).float()), _ptr(inv_w.reshape(-1).float()),
-                                               _ptr(out), _ptr(amax), M, N, K, out.stride(0), kernel, stream_handle()))
+                                               _ptr(out), _ptr(amax), M, N, K, out.stride(0), kernel, _stream()))
     return out, amax
 
 
@@ -241,7 +241,7 @@ def fp8_linear_small_m(a_bf16, amax_bits, w8, inv_w, seg_ends=None, softcap=None
     ws = _small_m_workspace(a.device, M, N, K)
     rc = _lib.lib().nc_fp8_linear_small_m(_ptr(a), _ptr(amax_bits), _ptr(w8), _ptr(inv_w), segs, len(seg_ends), _ptr(out), kind,
                                           float(softcap or 0.0), _ptr(out_amax), M, N, K, out.stride(0), _ptr(ws), ws.numel(),
-                                          ksplits, stream_handle())
+                                          ksplits, _stream())
     _lib.check(rc)
     return (out, out_amax) if relu2 else out
 
@@ -260,7 +260,7 @@ def rms_norm(x):
     x = x.contiguous()
     out = torch.empty_like(x)
     cols = x.shape[-1]
-    _lib.check(_lib.lib().nc_rmsnorm(_ptr(x), _ptr(out), x.numel() // cols, cols, None, stream_handle()))
+    _lib.check(_lib.lib().nc_rmsnorm(_ptr(x), _ptr(out), x.numel() // cols, cols, None, _stream()))
     return out
 
 
@@ -268,7 +268,7 @@ def relu2(h):
     _need_cuda(h)
     h = h.contiguous()
     out = torch.empty_like(h)
-    _lib.check(_lib.lib().nc_relu2(_ptr(h), _ptr(out), h.numel(), None, stream_handle()))
+    _lib.check(_lib.lib().nc_relu2(_ptr(h), _ptr(out), h.numel(), None, _stream()))
     return out
 
 
@@ -281,7 +281,7 @@ def embed_norm_smear(idx, wte, smear_w, smear_lambda, prev):
     prev_out = torch.empty(B, 1, E, dtype=torch.bfloat16, device=idx.device)
     rc = _lib.lib().nc_embed_norm_smear(_ptr(idx.contiguous()), _ptr(wte), _ptr(smear_w.float().contiguous()),
                                         _ptr(smear_lambda.float().contiguous()), _ptr(prev), _ptr(prev_out), _ptr(x), B, T, E,
-                                        wte.shape[0], stream_handle())
+                                        wte.shape[0], _stream())
     _lib.check(rc)
     return x, prev_out
 
@@ -296,7 +296,7 @@ def mix_norm(x, add=None, x0=None, resid_lambda=None, x0_lambda=None, backout_la
     xn = torch.empty_like(x)
     saved = torch.empty_like(x) if want_backout else None
     rc = _lib.lib().nc_mix_norm(_ptr(x), _ptr(add), _ptr(x0), _ptr(resid_lambda), _ptr(x0_lambda), _ptr(backout_lambda),
-                                _ptr(backout_src), _ptr(saved), _ptr(xn), rows, cols, None, stream_handle())
+                                _ptr(backout_src), _ptr(saved), _ptr(xn), rows, cols, None, _stream())
     _lib.check(rc)
     return xn, saved
 
@@ -316,7 +316,7 @@ def qkv_rope_append(qkv, xn, idx, ve_table, ve_gate_w, cos, sin, cache_seqlens, 
                                        _ptr(idx.contiguous() if idx is not None else None), _ptr(ve_table),
                                        _ptr(ve_gate_w.float().contiguous() if ve_gate_w is not None else None),
                                        _ptr(cos), _ptr(sin), cos.shape[0], _ptr(cache_seqlens), _ptr(k_cache), _ptr(v_cache),
-                                       _ptr(q), B, T, n_head, n_kv_head, Tmax, vocab_rows, stream_handle())
+                                       _ptr(q), B, T, n_head, n_kv_head, Tmax, vocab_rows, _stream())
     _lib.check(rc)
     return q
 
@@ -341,7 +341,7 @@ def decode_attention(q, k_cache, v_cache, cache_seqlens, window_left=-1, seqlens
     ws, ws_bytes = _attention_workspace(B, T, H, Tmax, q.device)
     rc = lib.nc_decode_attention(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(cache_seqlens), int(window_left), _ptr(out), B, T, H,
                                  Hkv, Tmax, 1 if seqlens_include_new else 0, _ptr(ws), ws_bytes, None, splits,
-                                 stream_handle())
+                                 _stream())
     _lib.check(rc)
     return out
 
@@ -364,13 +364,13 @@ def decode_attention_shared(q, k_cache, v_cache, cache_seqlens, shared_len, wind
     out = torch.empty_like(q)
     lib = _lib.lib()
     ws_bytes = lib.nc_decode_attention_shared_workspace_bytes(B, H, Hkv, int(shared_len))
-    key = (q.device.index, stream_handle(), "shared")
+    key = (q.device.index, _stream(), "shared")
     ws = _ATTN_WS.get(key)
     if ws is None or ws.numel() < ws_bytes:
         ws = torch.empty(max(ws_bytes, 1 << 20), dtype=torch.uint8, device=q.device)
         _ATTN_WS[key] = ws
     rc = lib.nc_decode_attention_shared(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(cache_seqlens), int(shared_len), int(window_left), _ptr(out),
-                                        B, H, Hkv, Tmax, 1 if seqlens_include_new else 0, _ptr(ws), ws.numel(), None, stream_handle())
+                                        B, H, Hkv, Tmax, 1 if seqlens_include_new else 0, _ptr(ws), ws.numel(), None, _stream())
     _lib.check(rc)
     return out
 
@@ -382,7 +382,7 @@ def _attention_workspace(B, T, H, Tmax, device):
     """Split counters and partial results of the stand-alone attention entries, kept per device and stream and grown on demand
     (calls on one stream run one after the other, and every call clears its own counters)."""
     ws_bytes = _lib.lib().nc_attention_workspace_bytes(B, T, H, Tmax)
-    key = (device.index, stream_handle())
+    key = (device.index, _stream())
     ws = _ATTN_WS.get(key)
     if ws is None or ws.numel() < ws_bytes:
         ws = torch.empty(max(ws_bytes, 1 << 20), dtype=torch.uint8, device=device)
@@ -410,7 +410,7 @@ def decode_attention_append(q, k_new, v_new, k_cache, v_cache, cache_seqlens, wi
     ws, ws_bytes = _attention_workspace(B, T, H, Tmax, q.device)
     rc = _lib.lib().nc_decode_attention_append(_ptr(q), _ptr(k_new), _ptr(v_new), _ptr(k_cache), _ptr(v_cache), _ptr(cache_seqlens),
                                                int(window_left), _ptr(out), B, T, H, Hkv, Tmax, _ptr(ws), ws_bytes, None,
-                                               splits, stream_handle())
+                                               splits, _stream())
     _lib.check(rc)
     return out
 
@@ -434,7 +434,7 @@ def qkv_rope_append_attention(qkv, xn, idx, ve_table, ve_gate_w, cos, sin, cache
         _ptr(qkv), qkv.shape[-1], _ptr(xn_c), xn_c.shape[-1] if xn_c is not None else 0, _ptr(idx.contiguous() if idx is not None else None),
         _ptr(ve_table), _ptr(ve_gate_w.float().contiguous() if ve_gate_w is not None else None), _ptr(cos), _ptr(sin), cos.shape[0],
         _ptr(cache_seqlens), _ptr(k_cache), _ptr(v_cache), int(window_left), _ptr(out), B, n_head, n_kv_head, Tmax, vocab_rows,
-        _ptr(ws), ws_bytes, None, splits, stream_handle())
+        _ptr(ws), ws_bytes, None, splits, _stream())
     _lib.check(rc)
     return out
 
@@ -455,7 +455,7 @@ def kv_cache_prefill(dst, src, n_tokens):
     Ls, Bs, Ts, Hs, Ds = src.shape
     if (Ls, Hs, Ds) != (L, Hkv, D):
         raise ValueError("kv_cache_prefill: layer / head geometry differs")
-    _lib.check(_lib.lib().nc_kv_cache_prefill(_ptr(src), _ptr(dst), L, Bs, Bd, Ts, Td, int(n_tokens), Hkv * D * 2, stream_handle()))
+    _lib.check(_lib.lib().nc_kv_cache_prefill(_ptr(src), _ptr(dst), L, Bs, Bd, Ts, Td, int(n_tokens), Hkv * D * 2, _stream()))
 
 
 # ----------------------------------------------------------------------------- (5) softcap / sample
@@ -463,7 +463,7 @@ def softcap(raw_bf16, cap=15.0):
     _need_cuda(raw_bf16)
     raw = raw_bf16.contiguous()
     out = torch.empty(raw.shape, dtype=torch.float32, device=raw.device)
-    _lib.check(_lib.lib().nc_softcap(_ptr(raw), _ptr(out), raw.numel(), float(cap), stream_handle()))
+    _lib.check(_lib.lib().nc_softcap(_ptr(raw), _ptr(out), raw.numel(), float(cap), _stream()))
     return out
 
 
@@ -482,7 +482,7 @@ def sample(logits, temperature, top_k, noise=None):
         want = k if (0 < k < V) else V
         if tuple(noise.shape) != (B, want):
             raise ValueError(f"sample: noise must have shape {(B, want)}, got {tuple(noise.shape)}")
-    rc = _lib.lib().nc_sample(_ptr(logits), B, V, logits.stride(0), float(temperature), k, _ptr(noise), _ptr(out), stream_handle())
+    rc = _lib.lib().nc_sample(_ptr(logits), B, V, logits.stride(0), float(temperature), k, _ptr(noise), _ptr(out), _stream())
     _lib.check(rc)
     return out
 
@@ -498,7 +498,7 @@ def stack_cache_copy(src, dst, n):
     assert src.shape[2:] == dst.shape[2:] and src.dtype == dst.dtype and src[0].is_contiguous() and dst[0].is_contiguous()
     es = src.element_size()
     n_bytes = n * (src[0].numel() // src.shape[1]) * es
-    rc = _lib.stack_lib().nc_stack_cache_copy(_ptr(src), _ptr(dst), src.shape[0], dst.shape[0], src.stride(0) * es, dst.stride(0) * es, n_bytes, stream_handle())
+    rc = _lib.stack_lib().nc_stack_cache_copy(_ptr(src), _ptr(dst), src.shape[0], dst.shape[0], src.stride(0) * es, dst.stride(0) * es, n_bytes, _stream())
     _lib.check(rc, _lib.stack_lib())
 
 
@@ -509,6 +509,6 @@ def stack_linear(a, w, kind=0, limit=0.0, kernel=0):
     (M, K), N = a.shape, w.shape[0]
     assert w.shape[1] == K and a.dtype == w.dtype and a.is_contiguous() and w.is_contiguous()
     out = torch.empty(M, N // 2 if kind in (2, 7) else N, dtype=torch.float32 if kind == 3 else a.dtype, device=a.device)
-    rc = _lib.stack_lib().nc_stack_linear(STACK_DTYPES[a.dtype], _ptr(a), K, _ptr(w), _ptr(out), out.shape[1], M, N, K, kind, limit, kernel, stream_handle())
+    rc = _lib.stack_lib().nc_stack_linear(STACK_DTYPES[a.dtype], _ptr(a), K, _ptr(w), _ptr(out), out.shape[1], M, N, K, kind, limit, kernel, _stream())
     _lib.check(rc, _lib.stack_lib())
     return out

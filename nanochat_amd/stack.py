@@ -792,7 +792,7 @@ class LayerStack(nn.Module):
         keys = kv_cache.max_seq_len if T == 1 else min(kv_cache.max_seq_len, round_up(pos_max + T, 256))
         ws_ptr, ws_bytes = self._workspace(md, B, T, n_logits, keys)
         rc = lib.nc_stack_forward(C.byref(md), C.byref(cd), idx.data_ptr(), B, T, rows.data_ptr() if rows is not None else None, n_logits,
-                                  logits.data_ptr(), ws_ptr, ws_bytes, tap.data_ptr() if taps else None, ops.stream_handle())
+                                  logits.data_ptr(), ws_ptr, ws_bytes, tap.data_ptr() if taps else None, ops._stream())
         _lib.check(rc, lib)
         if cd.advance:
             kv_cache.note_advanced(T)
