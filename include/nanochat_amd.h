@@ -78,6 +78,10 @@ int nc_fp8_quantize_tensorwise_fused_bounded(const void* x, int x_dtype, int64_t
  * nc_fp8_quantize_tensorwise_as.  rows and cols multiples of 16, pointers 16-byte aligned; amax_ws: one uint32, cleared by the call. */
 int nc_fp8_quantize_tensorwise_transposed(const uint16_t* x, int rows, int cols, int fp8_format, uint8_t* out, uint8_t* out_t,
                                           float* scale_out, float* inv_scale_out, uint32_t* amax_ws, nc_stream_t stream);
+/* The same in one launch where the matrix fits the chip (some 16 M elements), in the three above where it does not.  state and the wait of the
+ * launch's workgroups for each other: as for nc_fp8_quantize_tensorwise_fused; spin_limit: that wait's bound in polls, below 0 the usual one. */
+int nc_fp8_quantize_tensorwise_transposed_fused(const uint16_t* x, int rows, int cols, int fp8_format, uint8_t* out, uint8_t* out_t,
+                                                float* scale_out, float* inv_scale_out, void* state, int64_t spin_limit, nc_stream_t stream);
 
 /* dst[cols][rows] = transpose of the fp8 payload src[rows][cols]: the memory rearrangement of _to_col_major and
  * .t().contiguous() at nanochat/fp8.py:110-118,169,181-182 (the backward GEMMs want the summed index contiguous in

@@ -46,6 +46,13 @@ int nc_fp8_quantize_tensorwise_transposed(const uint16_t* x, int rows, int cols,
     return nc_launch_quantize_transposed(x, rows, cols, fp8_format, out, out_t, scale_out, inv_scale_out, amax_ws, (hipStream_t)stream);
 }
 
+int nc_fp8_quantize_tensorwise_transposed_fused(const uint16_t* x, int rows, int cols, int fp8_format, uint8_t* out, uint8_t* out_t, float* scale_out,
+                                                float* inv_scale_out, void* state, int64_t spin_limit, nc_stream_t stream) {
+    return nc_launch_quantize_transposed_fused(x, rows, cols, fp8_format, out, out_t, scale_out, inv_scale_out, (uint32_t*)state,
+                                               spin_limit < 0 ? NC_QUANTIZE_DEFAULT_SPINS : spin_limit > 0xffffffffll ? 0xffffffffu : (uint32_t)spin_limit,
+                                               (hipStream_t)stream);
+}
+
 int nc_fp8_transpose(const uint8_t* src, int rows, int cols, uint8_t* dst, nc_stream_t stream) {
     return nc_launch_transpose_u8(src, rows, cols, dst, (hipStream_t)stream);
 }

@@ -85,11 +85,11 @@ def fp8_quantize(x, encoder=0, fp8_dtype=torch.float8_e4m3fn, spin_limit=None):
     return out, inv, scale
 
 
-def fp8_quantize_transposed(x, fp8_dtype=torch.float8_e4m3fn):
+def fp8_quantize_transposed(x, fp8_dtype=torch.float8_e4m3fn, spin_limit=None):
     """Tensorwise fp8 quantization of a bf16 matrix [R,C] that also writes the transposed payload [C,R] from the same read (what the
     backward GEMMs of nanochat/fp8.py:156-192 take: grad_output both ways, the saved input transposed).
 
-    Returns (payload [R,C], payload_t [C,R], inv_scale fp32 0-dim, scale fp32 0-dim); the bits are those of fp8_quantize."""
+    Returns (payload [R,C], payload_t [C,R], inv_scale fp32 0-dim, scale fp32 0-dim); the bits are those of fp8_quantize, and spin_limit is its."""
     _need_cuda(x)
     if x.dtype != torch.bfloat16 or x.dim() != 2:
         raise ValueError("fp8_quantize_transposed: a 2-D bf16 tensor is required")
@@ -101,9 +101,9 @@ def fp8_quantize_transposed(x, fp8_dtype=torch.float8_e4m3fn):
     out_t = torch.empty(Cc, R, dtype=fp8_dtype, device=x.device)
     scales = torch.empty(2, dtype=torch.float32, device=x.device)
     state = _quantize_state(x.device)
-    scratch = state.data_ptr() + 4 * 320          # the state block's scratch word
-    _lib.check(_lib.lib().nc_fp8_quantize_tensorwise_transposed(_ptr(x), R, Cc, _FP8_FORMATS[fp8_dtype], _ptr(out), _ptr(out_t),
-                                                                scales.data_ptr(), scales.data_ptr() + 4, scratch, _stream()))
+    _lib.check(_lib.lib().nc_fp8_quantize_tensorwise_transposed_fused(_ptr(x), R, Cc, _FP8_FORMATS[fp8_dtype], _ptr(out), _ptr(out_t), scales.data_ptr(),
+                                                                      scales.data_ptr() + 4, _ptr(state), -1 if spin_limit is None else int(spin_limit),
+                                                                      _stream()))
     scale, inv = scales.unbind()
     return out, out_t, inv, scale
 

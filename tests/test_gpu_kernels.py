@@ -649,6 +649,28 @@ def test_quantize_with_transposed_copy_is_the_quantizer_plus_an_exact_transpose(
         ops.fp8_quantize_transposed(torch.zeros(24, 40, dtype=torch.bfloat16, device=DEV))        # not multiples of 16
 
 
+@pytest.mark.parametrize("R,C", [(16, 16), (48, 400), (4096, 2048), (3456, 2432), (4096, 4096), (5248, 3200), (144, 16384)])
+@pytest.mark.parametrize("fmt", [torch.float8_e4m3fn, torch.float8_e5m2])
+def test_transposing_quantizer_in_one_launch(ops, R, C, fmt):
+    """One tile, a ragged handful, 512 and 513 tiles (one and two to a workgroup), 1024 and 1025 (the last that fit, the first that do not): the bytes and scales of
+    the plain quantizer and their exact transpose, with the usual wait and with one that is given up at once; the state stays zero."""
+    say(f"transposing quantizer in one launch {R}x{C} {fmt}")
+    g = torch.Generator(device=DEV).manual_seed(R + C)
+    x = torch.randn(R, C, device=DEV, generator=g)
+    x = torch.where(torch.rand(R, C, device=DEV, generator=g) < 0.001, x * 20, x).bfloat16()
+    want, want_inv, want_scale = ops.fp8_quantize(x, fp8_dtype=fmt)
+    state, before = ops._quantize_state(x.device).view(torch.int32), ops.quantize_slow_count()
+    for limit in (None, 0, None) if R * C < 1 << 22 else (None,):
+        got, got_t, inv, scale = ops.fp8_quantize_transposed(x, fp8_dtype=fmt, spin_limit=limit)
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)) and torch.equal(got_t.view(torch.uint8), want.view(torch.uint8).t())
+        assert torch.equal(inv.view(torch.int32), want_inv.view(torch.int32)) and torch.equal(scale.view(torch.int32), want_scale.view(torch.int32))
+        words = state.clone()
+        words[ops.QUANTIZE_SLOW_WORD] = 0
+        assert not words[:320].any(), limit
+        if limit is None and R * C >= 1 << 22:
+            assert ops.quantize_slow_count() == before
+
+
 @pytest.mark.parametrize("M,N,K,kernel", [
     (300, 320, 256, 5), (64, 128, 400, 5), (513, 272, 1664, 5), (2100, 1300, 48, 5),
     (300, 320, 256, 8), (513, 272, 1664, 8), (4100, 2100, 384, 8),
