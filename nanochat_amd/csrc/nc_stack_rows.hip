@@ -161,74 +161,112 @@ __device__ __forceinline__ float row_wave_max(float v) {
     v = fmaxf(v, __shfl_xor(v, 16));
     return fmaxf(v, __shfl_xor(v, 32));
 }
-template <int PER>
-__device__ __forceinline__ void choose_experts_of(const NcRoute& r, int m, int lane) {
-    float s[PER];
-    const float* z = r.logits + (int64_t)m * r.ld;
-    float mx = -3.0e38f;
+// ROWS rows m0, m0 + step, ... below M, side by side: their loads are out together and their chains of choices fill each other's gaps.  `picks`: what
+// goes to r.chosen as well, or nullptr.
+template <int PER, int ROWS>
+__device__ __forceinline__ void choose_experts_of(const NcRoute& r, int m0, int step, int M, int lane, int* picks) {
+    float s[ROWS][PER], mx[ROWS], sum[ROWS], chosen_sum[ROWS], mine[ROWS];       // lane k keeps the score of choice k (top <= 64)
+    int mine_at[ROWS];
 #pragma unroll
-    for (int i = 0; i < PER; i++) {
-        const int e = lane + 64 * i;
-        s[i] = e < r.experts ? z[e] : -3.0e38f;
-        mx = fmaxf(mx, s[i]);
+    for (int q = 0; q < ROWS; q++) {
+        const float* z = r.logits + (int64_t)min(m0 + q * step, M - 1) * r.ld;
+        mx[q] = -3.0e38f;
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const int e = lane + 64 * i;
+            s[q][i] = e < r.experts ? z[e] : -3.0e38f;
+        }
     }
-    mx = row_wave_max(mx);
-    float sum = 0.f;
 #pragma unroll
-    for (int i = 0; i < PER; i++) {
-        const int e = lane + 64 * i;
-        s[i] = e < r.experts ? expf(s[i] - mx) : -1.f;
-        sum += e < r.experts ? s[i] : 0.f;
+    for (int q = 0; q < ROWS; q++) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) mx[q] = fmaxf(mx[q], s[q][i]);
+        mx[q] = row_wave_max(mx[q]);
     }
-    sum = wave_sum(sum);
-    // A score that is not a number comes after every other one, but before what must not be chosen: lanes past the experts and earlier choices.
-    // The choices of a row are thus distinct experts whatever its scores; its weights are NaN by the sum.
 #pragma unroll
-    for (int i = 0; i < PER; i++)
-        if (!(s[i] >= 0.f)) s[i] = lane + 64 * i < r.experts ? -1.f : -2.f;
-    float chosen_sum = 0.f, mine = 0.f;       // lane k keeps the score of choice k (top <= 64)
-    for (int k = 0; k < r.top; k++) {
-        float best = s[0];
-        int at = lane;
+    for (int q = 0; q < ROWS; q++) {
+        sum[q] = 0.f;
 #pragma unroll
-        for (int i = 1; i < PER; i++)
-            if (s[i] > best) best = s[i], at = lane + 64 * i;
-        const float top = row_wave_max(best);
-        at = __builtin_amdgcn_readlane(at, __ffsll((unsigned long long)__builtin_amdgcn_ballot_w64(best == top)) - 1);
-        best = top;
-        const float score = best / sum;
-        chosen_sum += score;
-        if (lane == k) mine = score;
-        if (lane == 0) r.chosen[m * r.top + k] = at;
+        for (int i = 0; i < PER; i++) {
+            const int e = lane + 64 * i;
+            s[q][i] = e < r.experts ? expf(s[q][i] - mx[q]) : -1.f;
+            sum[q] += e < r.experts ? s[q][i] : 0.f;
+        }
+        sum[q] = wave_sum(sum[q]);
+        // A score that is not a number comes after every other one, but before what must not be chosen: lanes past the experts and earlier choices.
+        // The choices of a row are thus distinct experts whatever its scores; its weights are NaN by the sum.
 #pragma unroll
         for (int i = 0; i < PER; i++)
-            if (at == lane + 64 * i) s[i] = -2.f;
+            if (!(s[q][i] >= 0.f)) s[q][i] = lane + 64 * i < r.experts ? -1.f : -2.f;
+        chosen_sum[q] = 0.f, mine[q] = 0.f, mine_at[q] = 0;
     }
-    if (lane < r.top) r.slot_w[m * r.top + lane] = mine / (chosen_sum + 1e-20f);
+    for (int k = 0; k < r.top; k++) {
+        float best[ROWS], top[ROWS];
+        int at[ROWS];
+#pragma unroll
+        for (int q = 0; q < ROWS; q++) {
+            best[q] = s[q][0], at[q] = lane;
+#pragma unroll
+            for (int i = 1; i < PER; i++)
+                if (s[q][i] > best[q]) best[q] = s[q][i], at[q] = lane + 64 * i;
+        }
+#pragma unroll
+        for (int q = 0; q < ROWS; q++) top[q] = row_wave_max(best[q]);
+#pragma unroll
+        for (int q = 0; q < ROWS; q++) {
+            at[q] = __builtin_amdgcn_readlane(at[q], __ffsll((unsigned long long)__builtin_amdgcn_ballot_w64(best[q] == top[q])) - 1);
+            const float score = top[q] / sum[q];
+            chosen_sum[q] += score;
+            if (lane == k) mine[q] = score, mine_at[q] = at[q];
+#pragma unroll
+            for (int i = 0; i < PER; i++)
+                if (at[q] == lane + 64 * i) s[q][i] = -2.f;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < ROWS; q++) {
+        const int m = m0 + q * step;
+        if (m < M && lane < r.top) {
+            r.slot_w[m * r.top + lane] = mine[q] / (chosen_sum[q] + 1e-20f);
+            r.chosen[m * r.top + lane] = mine_at[q];
+            if (picks) picks[m * r.top + lane] = mine_at[q];
+        }
+    }
 }
 
-__device__ __forceinline__ void choose_experts(const NcRoute& r, int m, int lane) {
-    if (r.experts <= 64) choose_experts_of<1>(r, m, lane);
-    else if (r.experts <= 256) choose_experts_of<4>(r, m, lane);
-    else choose_experts_of<ROUTE_MAX_EXPERTS / 64>(r, m, lane);
+template <int ROWS>
+__device__ __forceinline__ void choose_experts(const NcRoute& r, int m0, int step, int M, int lane, int* picks) {
+    if (r.experts <= 64) return choose_experts_of<1, ROWS>(r, m0, step, M, lane, picks);
+#pragma unroll 1
+    for (int q = 0; q < ROWS && m0 + q * step < M; q++) {
+        if (r.experts <= 256) choose_experts_of<4, 1>(r, m0 + q * step, step, M, lane, picks);
+        else choose_experts_of<ROUTE_MAX_EXPERTS / 64, 1>(r, m0 + q * step, step, M, lane, picks);
+    }
 }
 
 __global__ __launch_bounds__(256) void route_choose_kernel(NcRoute r, int M) {
     const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (m < M) choose_experts(r, m, threadIdx.x & 63);
+    if (m < M) choose_experts<1>(r, m, 1, M, threadIdx.x & 63, nullptr);
 }
 
-// The (row, choice) pairs in expert order: one workgroup counts, scans and deals out.  CHOOSE: it makes the choices first (few rows).
+// The (row, choice) pairs in expert order: one workgroup counts, scans and deals out.  CHOOSE: it makes the choices first (up to 64 rows, four to a
+// wave side by side) and passes them on in LDS: 64 rows, 6 of 64 experts 12.4 us with a row after the other and the choices through memory, now 10.5;
+// what is left is the instructions of 16 waves on one compute unit.
 // (The order of the pairs inside an expert is whatever the atomics give: every pair is a row of its own, so no result depends on it.)
 template <bool CHOOSE>
 __global__ __launch_bounds__(1024) void route_sort_kernel(NcRoute r, int M) {
-    __shared__ int count[ROUTE_MAX_EXPERTS], start[ROUTE_MAX_EXPERTS];
+    __shared__ int count[ROUTE_MAX_EXPERTS], start[ROUTE_MAX_EXPERTS], picks[CHOOSE ? 64 * 64 : 1];
     const int pairs = M * r.top;
+    auto chosen = [&](int p) { return CHOOSE ? picks[p] : r.chosen[p]; };
     for (int e = threadIdx.x; e < r.experts; e += 1024) count[e] = 0;
-    if (CHOOSE)
-        for (int m = threadIdx.x >> 6; m < M; m += 16) choose_experts(r, m, threadIdx.x & 63);
-    __syncthreads();          // (also makes the choices of all waves, global stores of this workgroup, visible to it)
-    for (int p = threadIdx.x; p < pairs; p += 1024) atomicAdd(&count[r.chosen[p]], 1);
+    if (CHOOSE) {
+        const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+        if (M > 32) choose_experts<4>(r, wave, 16, M, lane, picks);
+        else if (M > 16) choose_experts<2>(r, wave, 16, M, lane, picks);
+        else if (wave < M) choose_experts<1>(r, wave, 16, M, lane, picks);
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p < pairs; p += 1024) atomicAdd(&count[chosen(p)], 1);
     __syncthreads();
     // exclusive sums over the experts of rows and of tiles, by one wave, 64 experts at a time
     if (threadIdx.x < 64) {
@@ -256,7 +294,7 @@ __global__ __launch_bounds__(1024) void route_sort_kernel(NcRoute r, int M) {
     }
     __syncthreads();
     for (int p = threadIdx.x; p < pairs; p += 1024) {
-        const int slot = atomicAdd(&start[r.chosen[p]], 1);
+        const int slot = atomicAdd(&start[chosen(p)], 1);
         r.perm[slot] = p;
         r.slot_of[p] = slot;
     }

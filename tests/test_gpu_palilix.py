@@ -200,6 +200,17 @@ def test_32_bit_scores_of_many_rows_are_as_exact_as_of_few():
     assert whole < 1.66 * portions, whole / portions
 
 
+@pytest.mark.parametrize("experts", [7, 64, 65])
+def test_choices_of_several_rows_side_by_side(experts):
+    """Up to 64 rows choose in one workgroup, one, two or four rows to a wave: row counts at those borders, and experts of one and several to a lane."""
+    say(f"choices of several rows, {experts} experts")
+    cfg = config([(latent(), moe(experts=experts, top=6, ff=16))], vocab=50)
+    w, toks = weights(cfg, seed=11), tokens(cfg, 65)
+    model, want = build(cfg, w, torch.float32), ref.forward(cfg, {k: v.double() for k, v in w.items()}, toks)
+    for n in (1, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65):
+        check(run(model, toks[:n], [n]), want[:n], torch.float32, f"{n} rows")
+
+
 @pytest.mark.parametrize("heads,rank,rot_dim", [(5, 512, 64), (1, 256, 32), (3, 200, 64), (2, 320, 0), (7, 512, 32)])
 def test_32_bit_steps_whose_keys_are_shared_out(heads, rank, rot_dim):
     """Single tokens and portions of a few behind 0, 1, 63, 64, 65 and 300 cached ones: runs of keys that are empty, ragged or a single key, one and several
