@@ -97,70 +97,6 @@ __global__ __launch_bounds__(256) void window_append_kernel(NcWindowGeom g, T* _
     for (int j = threadIdx.x; j < nv; j += 256) st_f32(crow + j / g.vdim_p * head_w + g.dim_p + j % g.vdim_p, ld_f32(row + nq + nk + j) + bias[nq + nk + j]);
 }
 
-// The same with everything a token needs asked for at once and in fours: a thread keeps up to UNITS pairs of four dimensions that turn together (or four
-// that pass) from the sums to the stores.  What bounds the kernel above is its trips to memory, one for the norms and one to turn, and its two-byte
-// loads: 16 tokens of 16 heads on 4 7.0 -> 4.7 us, 1792 of 32 on 8 24.8 -> 20.3.
-template <typename T, int UNITS>
-__global__ __launch_bounds__(256) void window_append_vec_kernel(NcWindowGeom g, T* __restrict__ proj, int ldp, const float* __restrict__ bias,
-                                                                const float* __restrict__ q_norm_w, const float* __restrict__ k_norm_w, float eps,
-                                                                const float* __restrict__ rope, int rope_len, const int32_t* __restrict__ seqlens,
-                                                                T* __restrict__ cache) {
-    __shared__ float red[2][4];
-    const int64_t m = blockIdx.x;
-    const int b = (int)(m / g.T), t = (int)(m % g.T), pos = seqlens[b] + t, half = g.rot_dims / 2, turning = half / 4, per_head = turning + (g.dim_p - 2 * half) / 4;
-    const int nq = g.heads * g.dim_p, nk = g.kv_heads * g.dim_p, nv = g.kv_heads * g.vdim_p, head_w = g.dim_p + g.vdim_p, units = (g.heads + g.kv_heads) * per_head;
-    T* const row = proj + m * ldp;
-    const v4f zero{0.f, 0.f, 0.f, 0.f};
-    v4f a[UNITS], c[UNITS], wa[UNITS], wc[UNITS], turn[UNITS][2];
-    float sq = 0.f, sk = 0.f;
-#pragma unroll
-    for (int i = 0; i < UNITS; i++) {
-        const int u = threadIdx.x + 256 * i, h = u / per_head, p = u % per_head, d = p < turning ? 4 * p : 4 * p + half, at = h * g.dim_p + d;
-        a[i] = c[i] = wa[i] = wc[i] = turn[i][0] = turn[i][1] = zero;
-        if (u >= units) continue;
-        const float* const w = h < g.heads ? q_norm_w + at : k_norm_w + at - nq;
-        a[i] = ld4_f32(row + at) + *(const v4f*)(bias + at), wa[i] = *(const v4f*)w;
-        if (p < turning) {
-            const float* const table = rope + ((int64_t)min(pos, rope_len - 1) * half + d) * 2;
-            c[i] = ld4_f32(row + at + half) + *(const v4f*)(bias + at + half), wc[i] = *(const v4f*)(w + half);
-            turn[i][0] = *(const v4f*)table, turn[i][1] = *(const v4f*)(table + 4);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < UNITS; i++) {
-        const v4f s2 = a[i] * a[i] + c[i] * c[i];
-        const float s = (s2[0] + s2[1]) + (s2[2] + s2[3]);
-        if ((int)threadIdx.x + 256 * i < g.heads * per_head) sq += s;
-        else sk += s;
-    }
-    sq = wave_sum(sq), sk = wave_sum(sk);
-    if ((threadIdx.x & 63) == 0) red[0][threadIdx.x >> 6] = sq, red[1][threadIdx.x >> 6] = sk;
-    __syncthreads();
-    sq = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]), sk = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
-    const float iq = 1.0f / sqrtf(sq / (float)(g.heads * g.dim) + eps), ik = 1.0f / sqrtf(sk / (float)(g.kv_heads * g.dim) + eps);
-    const bool in = pos < g.Tmax;
-    T* const crow = cache + ((int64_t)b * g.Tmax + (in ? pos : 0)) * g.kv_heads * head_w;
-#pragma unroll
-    for (int i = 0; i < UNITS; i++) {
-        const int u = threadIdx.x + 256 * i, h = u / per_head, p = u % per_head, d = p < turning ? 4 * p : 4 * p + half;
-        const bool is_q = h < g.heads;
-        if (u >= units || (!is_q && !in)) continue;
-        const float inv = is_q ? iq : ik;
-        T* const o = (is_q ? row + h * g.dim_p : crow + (h - g.heads) * head_w) + d;
-        const v4f x = a[i] * inv * wa[i];
-        if (p < turning) {
-            const v4f y = c[i] * inv * wc[i], cs{turn[i][0][0], turn[i][0][2], turn[i][1][0], turn[i][1][2]}, sn{turn[i][0][1], turn[i][0][3], turn[i][1][1], turn[i][1][3]};
-            st4_f32(o, x * cs - y * sn);
-            st4_f32(o + half, y * cs + x * sn);
-        } else {
-            st4_f32(o, x);
-        }
-    }
-    if (!in) return;
-    for (int j = 4 * threadIdx.x; j < nv; j += 1024)
-        st4_f32(crow + j / g.vdim_p * head_w + g.dim_p + j % g.vdim_p, ld4_f32(row + nq + nk + j) + *(const v4f*)(bias + nq + nk + j));
-}
-
 // ------------------------------------------------------------------------------------------------ any sizes
 // One workgroup per (token, head).
 constexpr int SIMPLE_COLS = 4;       // value columns per thread: vdim_p <= 256 * 4
@@ -732,15 +668,12 @@ int nc_launch_window_append(int dtype, const NcWindowGeom& g, void* proj, int ld
     NC_CHECK_ARG(bias && q_norm_w && k_norm_w && (rope || g.rot_dims == 0) && ldp % 4 == 0, "window_append: null operand");
     NC_CHECK_ARG(g.pos_max + g.T <= rope_len && g.pos_max + g.T <= g.Tmax, "window_append: position %d past the rotary table of %d", g.pos_max + g.T, rope_len);
     NcProfScope prof(NC_CLS_ROWS, (double)g.B * g.T * (g.dim_p * (g.heads + g.kv_heads) + g.vdim_p * g.kv_heads) * (dtype ? 8 : 4), s);
-    // the fours of a head's dimensions that one token's threads keep (a table of angles and rows of all operands begin at multiples of four values)
-    const int fours = (g.heads + g.kv_heads) * (g.rot_dims / 8 + (g.dim_p - g.rot_dims) / 4);
-    const bool vec = g.rot_dims % 8 == 0 && fours <= 1024 && (((uintptr_t)proj | (uintptr_t)cache | (uintptr_t)bias | (uintptr_t)q_norm_w | (uintptr_t)k_norm_w | (uintptr_t)rope) & 15) == 0;
-    auto go = [&](auto kernel, auto value) {
-        using T = decltype(value);
-        hipLaunchKernelGGL(kernel, dim3(g.B * g.T), dim3(256), 0, s, g, (T*)proj, ldp, bias, q_norm_w, k_norm_w, eps, rope, rope_len, seqlens, (T*)cache);
-    };
-    if (dtype) go(!vec ? window_append_kernel<float> : fours <= 512 ? window_append_vec_kernel<float, 2> : window_append_vec_kernel<float, 4>, float{});
-    else go(!vec ? window_append_kernel<bf16_t> : fours <= 512 ? window_append_vec_kernel<bf16_t, 2> : window_append_vec_kernel<bf16_t, 4>, bf16_t{});
+    if (dtype)
+        hipLaunchKernelGGL((window_append_kernel<float>), dim3(g.B * g.T), dim3(256), 0, s, g, (float*)proj, ldp, bias, q_norm_w, k_norm_w, eps, rope, rope_len,
+                           seqlens, (float*)cache);
+    else
+        hipLaunchKernelGGL((window_append_kernel<bf16_t>), dim3(g.B * g.T), dim3(256), 0, s, g, (bf16_t*)proj, ldp, bias, q_norm_w, k_norm_w, eps, rope, rope_len,
+                           seqlens, (bf16_t*)cache);
     NC_CHECK_LAUNCH("window_append");
     return 0;
 }
