@@ -649,6 +649,31 @@ def test_quantize_with_transposed_copy_is_the_quantizer_plus_an_exact_transpose(
         ops.fp8_quantize_transposed(torch.zeros(24, 40, dtype=torch.bfloat16, device=DEV))        # not multiples of 16
 
 
+@pytest.mark.parametrize("T,splits", [(2, 0), (2, 16), (7, 4), (15, 2), (15, 0), (17, 0), (17, 8)])
+def test_append_of_several_tokens_clears_its_split_counters(ops, T, splits):
+    """Several new tokens per row: the launch that appends them clears the counters of the key splits, whatever the workspace holds; the same output and
+    cache as appending by hand and attending in one piece."""
+    say(f"append of {T} tokens, {splits} splits")
+    B, H, Hkv, Tmax = 3, 8, 4, 400
+    g = torch.Generator(device=DEV).manual_seed(T + splits)
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g, device=DEV).bfloat16()
+    q, k, v, kc, vc = normal(B, T, H, 128), normal(B, T, Hkv, 128), normal(B, T, Hkv, 128), normal(B, Tmax, Hkv, 128), normal(B, Tmax, Hkv, 128)
+    n = torch.tensor([0, 131, Tmax - T], dtype=torch.int32, device=DEV)
+    kw, vw = kc.clone(), vc.clone()
+    for b in range(B):
+        kw[b, n[b]:n[b] + T], vw[b, n[b]:n[b] + T] = k[b], v[b]
+    want = ops.decode_attention(q, kw, vw, n, splits=1)
+    for again in range(2):
+        for ws in ops._ATTN_WS.values():
+            ws.fill_(0xA5)
+        kd, vd = kc.clone(), vc.clone()
+        got = ops.decode_attention_append(q, k, v, kd, vd, n, splits=splits)
+        assert torch.equal(kd, kw) and torch.equal(vd, vw)
+        assert rel_l2(got, want) <= 2 * 2.0 ** -9            # one bf16 rounding each of the same fp32 sums
+
+
 @pytest.mark.parametrize("R,C", [(16, 16), (48, 400), (4096, 2048), (3456, 2432), (4096, 4096), (5248, 3200), (144, 16384)])
 @pytest.mark.parametrize("fmt", [torch.float8_e4m3fn, torch.float8_e5m2])
 def test_transposing_quantizer_in_one_launch(ops, R, C, fmt):
