@@ -2,7 +2,7 @@
 // Python loop at nanochat/gpt.py:459-524 (and of the module calls it makes into gpt.py:84-153 and
 // fp8.py:202-213).  One call enqueues every kernel of the step; no host synchronisation, no allocation.
 //
-// Per layer, decode (M = B*T <= 128 rows), 8 launches, each making a single dependent trip to memory:
+// Per layer, decode (M = B*T <= 128 rows), 7 or 8 launches, each making a single dependent trip to memory:
 //   mix_norm            x += mlp_out(prev) [read from split partials]; x = rl*x + xl*x0; xn = norm(x); amax(xn)
 //   linear q|k|v        quantize xn inside the GEMM; K split over workgroups           -> fp32 partials
 //   attention           each (row, kv head) workgroup first sums its heads' partials (three weight scales), applies
@@ -12,7 +12,7 @@
 //                       stand-alone qkv_rope_append kernel in front)
 //   linear c_proj       quantize y inside                                              -> partials
 //   mix_norm            x += o [from partials]; xn = norm(x); amax(xn)
-//   linear c_fc         quantize xn inside                                             -> partials
+//   linear c_fc         quantize xn inside; up to 64 rows of up to 2048 columns relu^2 and amax as well -> h2, otherwise -> partials and
 //   finish_partials     sum, scale, relu^2, amax                                       -> h2
 //   linear mlp c_proj   quantize h2 inside                                             -> partials (added by the next mix_norm)
 // Prefill (M > 128) uses the explicit convert kernel and the tiled GEMM instead of the fused small-M linear; the two narrow projections of a
