@@ -376,6 +376,12 @@ def test_gemm_relu2_epilogue_and_amax(ops, M, N, K, kernel):
     assert torch.equal(got, F.relu(plain).square())
 
 
+@pytest.mark.parametrize("M,N,K", [(130, 4096, 1024), (300, 320, 400), (700, 2244, 384), (129, 1024, 256), (1000, 1100, 144)])
+def test_gemm_relu2_of_few_tiles(ops, M, N, K):
+    """The relu^2 linear where its tiles leave compute units idle: lower tiles, straight into LDS where K is a multiple of 128."""
+    test_gemm_relu2_epilogue_and_amax(ops, M, N, K, 0)
+
+
 def test_gemm_softcap_epilogue(ops):
     say("gemm softcap")
     a, w = make_operands(64, 1024, 256, 11)
