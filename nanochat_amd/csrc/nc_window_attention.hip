@@ -191,9 +191,11 @@ __global__ __launch_bounds__(256) void window_step32_kernel(NcWindowGeom g, cons
     for (int v0 = v_begin; v0 < v_end; v0 += 4 * STEP32_KEYS) {
         v4f kf[STEP32_KEYS][QJ], vf[STEP32_KEYS][VJ];
         float s[STEP32_KEYS], m_new = m_run;
-        // (a place past the end of the run takes the run's last key, which this row sees, with weight 0)
+        // (a place past the end of the run takes the run's last key, which this row sees, with weight 0, and a value of zeros: an infinity in that
+        // key's value belongs to the sum once, and 0 times it is NaN)
 #pragma unroll
         for (int u = 0; u < STEP32_KEYS; u++) {
+            const bool there = v0 + 4 * u + grp < v_end;
             const float* const src = keys + (int64_t)list.key(min(v0 + 4 * u + grp, v_end - 1)) * rw;
 #pragma unroll
             for (int j = 0; j < QJ; j++) {
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(256) void window_step32_kernel(NcWindowGeom g, cons
 #pragma unroll
             for (int j = 0; j < VJ; j++) {
                 const int d = 64 * j + 4 * sub;
-                vf[u][j] = d < g.vdim_p ? *(const v4f*)(src + g.dim_p + d) : zero;
+                vf[u][j] = there && d < g.vdim_p ? *(const v4f*)(src + g.dim_p + d) : zero;
             }
         }
 #pragma unroll

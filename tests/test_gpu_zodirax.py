@@ -2,6 +2,7 @@
 sequences, slots that are used again, generation through the Engine; both storage types."""
 import functools
 import json
+import math
 
 import pytest
 import torch
@@ -240,6 +241,31 @@ def test_32_bit_steps_whose_keys_are_shared_out(heads, kv_heads, dim, vdim, wind
     for cuts in ([1] * 5, [62, 1, 1, 1, 1], [300, 1, 1]):
         toks = tokens(cfg, sum(cuts))
         check(run(model, toks, cuts), oracle(cfg, w, toks), torch.float32, f"portions {cuts}")
+
+
+@pytest.mark.parametrize("dim,vdim,n", [(64, 48, 20), (128, 128, 41), (160, 48, 100), (256, 250, 21)])
+def test_an_infinite_value_of_a_32_bit_step(dim, vdim, n):
+    """One cached token's value holds an infinity, whichever token it is: the step's sum is that infinity, not NaN.  (The norm behind the mixer makes NaN
+    of either, so the sums are looked at where they are left, in the workspace: the head's column and its product with the projection's weight.)"""
+    say(f"infinite value, {dim} and {vdim} dimensions, {n} tokens")
+    cfg = mechanism(pair(heads=2, kv_heads=2, dim=dim, vdim=vdim, rot_dims=16, window=500, keep_first=0, scale=0.02, left_scale=1.0, **OFF))
+    model, toks = build_model(Zodirax, cfg, weights(cfg, seed=3), torch.float32), tokens(cfg, n)
+    at = model.run_mixers()[0]
+    cache = model.new_cache(1, n)
+    model.forward(ids(toks[:-1]), kv_cache=cache)
+    model.forward(ids(toks[-1:]), kv_cache=cache)            # (its workspace stays)
+    cache.rewind(1)
+    value = cache.rows[0][0, :, at.row_width - at.vdim_p + vdim - 1]        # the second head's last column
+    for i in range(n - 1):
+        before = value[i].item()
+        value[i] = math.inf
+        for ws in model._workspaces.values():
+            ws.zero_()
+        model.forward(ids(toks[-1:]), kv_cache=cache)
+        infinite = sum(int(torch.isinf(ws[:ws.numel() // 4 * 4].view(torch.float32)).sum()) for ws in model._workspaces.values())
+        assert infinite > cfg["width"], f"token {i}: {infinite}"
+        cache.rewind(1)
+        value[i] = before
 
 
 def test_long_decoding():
