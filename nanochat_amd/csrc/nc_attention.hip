@@ -452,6 +452,29 @@ int nc_attn_splits(int B, int T, int Hkv, int window_left, int Tmax) {
     return pick_splits(B, T, Hkv, max_keys);
 }
 
+// What every launch here asks of its sizes; *nsplit: the key splits it takes, whose workspace is there.
+static int check_attention(int window_left, int B, int T, int H, int Hkv, int Tmax, const uint32_t* counters, const void* partials,
+                           size_t partial_bytes, int force_splits, int* nsplit) {
+    NC_CHECK_ARG(B > 0 && T > 0 && H > 0 && Hkv > 0 && Tmax > 0, "decode_attention: bad shape");
+    NC_CHECK_ARG(H % Hkv == 0, "decode_attention: n_head %d not a multiple of n_kv_head %d", H, Hkv);
+    const int G = H / Hkv;
+    NC_CHECK_ARG(G == 1 || G == 2 || G == 4 || G == 8, "decode_attention: query group size %d not in {1,2,4,8}", G);
+    NC_CHECK_ARG((long)B * T <= 65535 && Hkv <= 65535, "decode_attention: more than 65535 query rows in one launch");
+    *nsplit = force_splits > 0 ? force_splits : nc_attn_splits(B, T, Hkv, window_left, Tmax);
+    NC_CHECK_ARG(*nsplit >= 1 && *nsplit <= 16, "decode_attention: splits must be 1..16");
+    if (*nsplit > 1) {
+        const size_t need = (size_t)B * T * H * *nsplit * PART_STRIDE * sizeof(float);
+        NC_CHECK_ARG(counters && partials && partial_bytes >= need, "decode_attention: %zu bytes of split workspace needed, %zu given",
+                     need, partial_bytes);
+        NC_CHECK_ARG(((uintptr_t)partials & 15) == 0, "decode_attention: workspace must be 16-byte aligned");
+    }
+    return 0;
+}
+
+// many queries per row: the matrix-core kernel (a workgroup there covers 128 queries; below 16 queries per row
+// the per-query streaming kernel wastes less)
+static bool takes_prefill(int T, int force_splits) { return T >= 16 && force_splits <= 0; }
+
 // mode 0: q given, new tokens already in the cache.  mode 1: *rope names the raw q|k|v rows (rotary, QK-norm, value embedding and the
 // append are done here).  mode 2: q given, rope->k_new / rope->v_new hold the finished new key and value, appended here.
 static int launch_attention_impl(const bf16_t* q, const NcRopeSrc* rope, int mode, bf16_t* k_cache, bf16_t* v_cache,
@@ -460,21 +483,14 @@ static int launch_attention_impl(const bf16_t* q, const NcRopeSrc* rope, int mod
                                  int force_splits, int counters_are_zero, hipStream_t s, int k_min = 0, const float* extra = nullptr,
                                  int n_extra = 0) {
     NC_CHECK_ARG((q || mode == 1) && k_cache && v_cache && cache_seqlens && out, "decode_attention: null pointer");
-    // many queries per row: the matrix-core kernel (a workgroup there covers 128 queries; below 16 queries per row
-    // the per-query streaming kernel wastes less)
-    if (mode == 0 && T >= 16 && force_splits <= 0)
+    if (mode == 0 && takes_prefill(T, force_splits))
         return nc_launch_attention_prefill(q, k_cache, v_cache, cache_seqlens, window_left, out, B, T, H, Hkv, Tmax, seqlens_include_new,
                                            amax_ws, s);
-    NC_CHECK_ARG(B > 0 && T > 0 && H > 0 && Hkv > 0 && Tmax > 0, "decode_attention: bad shape");
-    NC_CHECK_ARG(H % Hkv == 0, "decode_attention: n_head %d not a multiple of n_kv_head %d", H, Hkv);
-    const int G = H / Hkv;
-    NC_CHECK_ARG(G == 1 || G == 2 || G == 4 || G == 8, "decode_attention: query group size %d not in {1,2,4,8}", G);
-    NC_CHECK_ARG((long)B * T <= 65535 && Hkv <= 65535, "decode_attention: more than 65535 query rows in one launch");
+    int nsplit;
+    if (const int rc = check_attention(window_left, B, T, H, Hkv, Tmax, counters, partials, partial_bytes, force_splits, &nsplit)) return rc;
+    const int G = H / Hkv, max_keys = (window_left >= 0 && window_left + 1 < Tmax) ? window_left + 1 : Tmax;
     NC_CHECK_ARG((!q || ((uintptr_t)q & 15) == 0) && ((uintptr_t)k_cache & 15) == 0 && ((uintptr_t)v_cache & 15) == 0,
                  "decode_attention: pointers must be 16-byte aligned");
-    int max_keys = (window_left >= 0 && window_left + 1 < Tmax) ? window_left + 1 : Tmax;
-    int nsplit = force_splits > 0 ? force_splits : pick_splits(B, T, Hkv, max_keys);
-    NC_CHECK_ARG(nsplit >= 1 && nsplit <= 16, "decode_attention: splits must be 1..16");
     if (mode != 0) {
         NC_CHECK_ARG(rope && T == 1 && !seqlens_include_new, "decode_attention: the in-kernel append needs one new token per row, not yet counted");
     }
@@ -484,15 +500,9 @@ static int launch_attention_impl(const bf16_t* q, const NcRopeSrc* rope, int mod
                      "decode_attention: value embedding needs gate weights, xn and idx");
     }
     if (mode == 2) NC_CHECK_ARG(rope->k_new && rope->v_new, "decode_attention: new key / value missing");
-    if (nsplit > 1) {
-        const size_t need = (size_t)B * T * H * nsplit * PART_STRIDE * sizeof(float);
-        NC_CHECK_ARG(counters && partials && partial_bytes >= need, "decode_attention: %zu bytes of split workspace needed, %zu given",
-                     need, partial_bytes);
-        NC_CHECK_ARG(((uintptr_t)partials & 15) == 0, "decode_attention: workspace must be 16-byte aligned");
-        if (!counters_are_zero) nc_clear_u32(counters, B * T * Hkv, s);
-    }
     NC_CHECK_ARG(!extra || (nsplit == 1 && mode == 0 && T == 1 && n_extra > 0 && k_min > 0),
                  "decode_attention: a shared first part goes with one split, one query per row and tokens already appended");
+    if (nsplit > 1 && !counters_are_zero) nc_clear_u32(counters, B * T * Hkv, s);
     // when the profiler is on, the launch carries its own event pair (kernel begin / end, no marker packets around it)
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     const bool timed = nc_prof_take(0, 0.0, 0, &ev0, &ev1);
@@ -619,11 +629,15 @@ int nc_launch_attention_append(const bf16_t* q, const bf16_t* k_new, const bf16_
         return launch_attention_impl(q, &src, 2, k_cache, v_cache, cache_seqlens, window_left, out, B, 1, H, Hkv, Tmax, 0, counters, partials,
                                      partial_bytes, amax_ws, force_splits, 0, s);
     }
+    // (nothing is written before the sizes and the workspace are known to be right: the counters are B T Hkv words of room for B T H)
+    int nsplit = 1;
+    if (takes_prefill(T, force_splits)) NC_CHECK_ARG(H % Hkv == 0, "attention_append: n_head %d not a multiple of n_kv_head %d", H, Hkv);
+    else if (const int rc = check_attention(window_left, B, T, H, Hkv, Tmax, counters, partials, partial_bytes, force_splits, &nsplit)) return rc;
     hipLaunchKernelGGL(kv_append_kernel, dim3(T, B), dim3(Hkv * 16 < 256 ? Hkv * 16 : 256), 0, s, k_new, v_new, k_cache, v_cache,
-                       cache_seqlens, T, Tmax, Hkv * 128, counters);
+                       cache_seqlens, T, Tmax, Hkv * 128, nsplit > 1 ? counters : nullptr);
     NC_CHECK_LAUNCH("kv_append");
     return launch_attention_impl(q, nullptr, 0, k_cache, v_cache, cache_seqlens, window_left, out, B, T, H, Hkv, Tmax, 0, counters, partials,
-                                 partial_bytes, amax_ws, force_splits, counters ? 1 : 0, s);
+                                 partial_bytes, amax_ws, force_splits, 1, s);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -680,6 +680,26 @@ def test_append_of_several_tokens_clears_its_split_counters(ops, T, splits):
         assert rel_l2(got, want) <= 2 * 2.0 ** -9            # one bf16 rounding each of the same fp32 sums
 
 
+@pytest.mark.parametrize("T,H,Hkv,splits", [(2, 2, 64, 0), (3, 3, 2, 4), (5, 6, 2, 1), (3, 4, 2, 17), (20, 2, 5, 0)])
+def test_append_refuses_sizes_before_it_writes(ops, T, H, Hkv, splits):
+    """Heads that do not go together, a group of three, too many splits: an error, and cache and workspace as they were.  (The split counters have room for
+    the query heads; the launch that appends would clear as many as there are key heads.)"""
+    from nanochat_amd import _lib
+    say(f"append refused: {T} tokens, {H} heads on {Hkv}, {splits} splits")
+    B, Tmax = 2, 600
+    q, out = (torch.zeros(B, T, H, 128, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    k, v = (torch.ones(B, T, Hkv, 128, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    kc, vc = (torch.zeros(B, Tmax, Hkv, 128, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    n = torch.zeros(B, dtype=torch.int32, device=DEV)
+    room = _lib.lib().nc_attention_workspace_bytes(B, T, max(H, Hkv), Tmax)
+    for given in (room, 256 + 16):
+        ws = torch.full((room,), 0xA5, dtype=torch.uint8, device=DEV)
+        rc = _lib.lib().nc_decode_attention_append(q.data_ptr(), k.data_ptr(), v.data_ptr(), kc.data_ptr(), vc.data_ptr(), n.data_ptr(), -1, out.data_ptr(), B, T,
+                                                   H, Hkv, Tmax, ws.data_ptr(), given, None, splits, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert rc == -1 and (ws == 0xA5).all() and not kc.any() and not vc.any()
+
+
 @pytest.mark.parametrize("R,C", [(16, 16), (48, 400), (4096, 2048), (3456, 2432), (4096, 4096), (5248, 3200), (144, 16384)])
 @pytest.mark.parametrize("fmt", [torch.float8_e4m3fn, torch.float8_e5m2])
 def test_transposing_quantizer_in_one_launch(ops, R, C, fmt):
