@@ -429,17 +429,27 @@ __global__ __launch_bounds__(256) void attn_partial_kernel(const bf16_t* __restr
 // than 256-byte ones only if enough workgroups remain).
 static int pick_heads_per_wg(int B, int T, int Hkv) { return (Hkv >= 2 && (long)B * T * ((Hkv + 1) / 2) * 4 >= 1536) ? 2 : 1; }
 
-static int pick_splits(int B, int T, int Hkv, int max_keys) {
+// Who clears the split counters of a launch: it, or whoever enqueued it (a pass clears those of all its launches at once).
+enum { COUNTERS_CLEAR = 0, COUNTERS_OF_PASS = 1, COUNTERS_CLEARED = 2 };
+
+static int pick_splits(int B, int T, int Hkv, int max_keys, int counters) {
     // One split whenever the (row, kv head or head pair) workgroups alone give every CU ~6-8 waves: measured at batch 64 x 13 heads,
     // one split streams 513 keys at 5.9 TB/s and 2048 keys at 5.6 TB/s, and every extra split only adds merge work.
     // Small batches need the splits to fill the machine; keep at least 64 keys per wave.
     const int hp = pick_heads_per_wg(B, T, Hkv);
     if (hp == 2) return 1;
-    // So do very few (row, head) pairs, down to one batch of 32 keys per wave (us a launch, 64 / 32 keys: 13 pairs, 513 keys 10.2 / 8.9, 1500 keys 11.6 / 11.7;
-    // 15 pairs of two query heads, 1000 keys 13.1 / 11.3; but 80 pairs, 640 keys 11.9 / 12.5).
+    // So do very few (row, head) pairs, which go on from two splits down to one batch of 32 keys per wave (us a launch, 64 / 32 keys: 13 pairs, 513 keys
+    // 10.2 / 8.9, 1500 keys 11.6 / 11.7; 15 pairs of two query heads, 1000 keys 13.1 / 11.3; but 80 pairs, 640 keys 11.9 / 12.5).  From one split to two
+    // a call by itself pays for the counters and the merge (13 pairs, 256 / 400 keys: 5.6 / 7.8 us in one, 7.8 / 8.8 in two) and needs a workspace, so it
+    // stays at 64 keys; in a pass the counters are zero anyway and the line lies at 48 (us a step of one row, one split / two: depth 20, 300 keys
+    // 710 / 721, 400 keys 737 / 721; depth 26, 300 keys 975 / 986, 500 keys 1010 / 992).
     const long base_waves = (long)B * T * Hkv * 4;
     int s = 1;
-    while (s < 16 && base_waves * s < 2048 && max_keys / (4 * s * 2) >= (base_waves * s < 256 ? 32 : 64)) s *= 2;
+    while (s < 16 && base_waves * s < 2048) {
+        const int least = base_waves * s >= 256 ? 64 : s > 1 ? 32 : counters == COUNTERS_OF_PASS ? 48 : 64;
+        if (max_keys / (4 * s * 2) < least) break;
+        s *= 2;
+    }
     return s;
 }
 
@@ -447,20 +457,22 @@ static int pick_splits(int B, int T, int Hkv, int max_keys) {
 size_t nc_attn_counter_bytes(int B, int T, int H) { return (((size_t)B * T * H * sizeof(uint32_t)) + 255) & ~(size_t)255; }
 size_t nc_attn_partial_bytes(int B, int T, int H) { return (size_t)B * T * H * 16 * PART_STRIDE * sizeof(float); }
 
+static int visible_keys(int window_left, int Tmax) { return (window_left >= 0 && window_left + 1 < Tmax) ? window_left + 1 : Tmax; }
+
+// of a launch inside a pass (no launch with the same sizes takes more)
 int nc_attn_splits(int B, int T, int Hkv, int window_left, int Tmax) {
-    const int max_keys = (window_left >= 0 && window_left + 1 < Tmax) ? window_left + 1 : Tmax;
-    return pick_splits(B, T, Hkv, max_keys);
+    return pick_splits(B, T, Hkv, visible_keys(window_left, Tmax), COUNTERS_OF_PASS);
 }
 
 // What every launch here asks of its sizes; *nsplit: the key splits it takes, whose workspace is there.
 static int check_attention(int window_left, int B, int T, int H, int Hkv, int Tmax, const uint32_t* counters, const void* partials,
-                           size_t partial_bytes, int force_splits, int* nsplit) {
+                           size_t partial_bytes, int force_splits, int who_clears, int* nsplit) {
     NC_CHECK_ARG(B > 0 && T > 0 && H > 0 && Hkv > 0 && Tmax > 0, "decode_attention: bad shape");
     NC_CHECK_ARG(H % Hkv == 0, "decode_attention: n_head %d not a multiple of n_kv_head %d", H, Hkv);
     const int G = H / Hkv;
     NC_CHECK_ARG(G == 1 || G == 2 || G == 4 || G == 8, "decode_attention: query group size %d not in {1,2,4,8}", G);
     NC_CHECK_ARG((long)B * T <= 65535 && Hkv <= 65535, "decode_attention: more than 65535 query rows in one launch");
-    *nsplit = force_splits > 0 ? force_splits : nc_attn_splits(B, T, Hkv, window_left, Tmax);
+    *nsplit = force_splits > 0 ? force_splits : pick_splits(B, T, Hkv, visible_keys(window_left, Tmax), who_clears);
     NC_CHECK_ARG(*nsplit >= 1 && *nsplit <= 16, "decode_attention: splits must be 1..16");
     if (*nsplit > 1) {
         const size_t need = (size_t)B * T * H * *nsplit * PART_STRIDE * sizeof(float);
@@ -480,15 +492,15 @@ static bool takes_prefill(int T, int force_splits) { return T >= 16 && force_spl
 static int launch_attention_impl(const bf16_t* q, const NcRopeSrc* rope, int mode, bf16_t* k_cache, bf16_t* v_cache,
                                  const int32_t* cache_seqlens, int window_left, bf16_t* out, int B, int T, int H, int Hkv, int Tmax,
                                  int seqlens_include_new, uint32_t* counters, void* partials, size_t partial_bytes, uint32_t* amax_ws,
-                                 int force_splits, int counters_are_zero, hipStream_t s, int k_min = 0, const float* extra = nullptr,
+                                 int force_splits, int who_clears, hipStream_t s, int k_min = 0, const float* extra = nullptr,
                                  int n_extra = 0) {
     NC_CHECK_ARG((q || mode == 1) && k_cache && v_cache && cache_seqlens && out, "decode_attention: null pointer");
     if (mode == 0 && takes_prefill(T, force_splits))
         return nc_launch_attention_prefill(q, k_cache, v_cache, cache_seqlens, window_left, out, B, T, H, Hkv, Tmax, seqlens_include_new,
                                            amax_ws, s);
     int nsplit;
-    if (const int rc = check_attention(window_left, B, T, H, Hkv, Tmax, counters, partials, partial_bytes, force_splits, &nsplit)) return rc;
-    const int G = H / Hkv, max_keys = (window_left >= 0 && window_left + 1 < Tmax) ? window_left + 1 : Tmax;
+    if (const int rc = check_attention(window_left, B, T, H, Hkv, Tmax, counters, partials, partial_bytes, force_splits, who_clears, &nsplit)) return rc;
+    const int G = H / Hkv, max_keys = visible_keys(window_left, Tmax);
     NC_CHECK_ARG((!q || ((uintptr_t)q & 15) == 0) && ((uintptr_t)k_cache & 15) == 0 && ((uintptr_t)v_cache & 15) == 0,
                  "decode_attention: pointers must be 16-byte aligned");
     if (mode != 0) {
@@ -502,7 +514,7 @@ static int launch_attention_impl(const bf16_t* q, const NcRopeSrc* rope, int mod
     if (mode == 2) NC_CHECK_ARG(rope->k_new && rope->v_new, "decode_attention: new key / value missing");
     NC_CHECK_ARG(!extra || (nsplit == 1 && mode == 0 && T == 1 && n_extra > 0 && k_min > 0),
                  "decode_attention: a shared first part goes with one split, one query per row and tokens already appended");
-    if (nsplit > 1 && !counters_are_zero) nc_clear_u32(counters, B * T * Hkv, s);
+    if (nsplit > 1 && who_clears == COUNTERS_CLEAR) nc_clear_u32(counters, B * T * Hkv, s);
     // when the profiler is on, the launch carries its own event pair (kernel begin / end, no marker packets around it)
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     const bool timed = nc_prof_take(0, 0.0, 0, &ev0, &ev1);
@@ -550,8 +562,7 @@ static int launch_attention_impl(const bf16_t* q, const NcRopeSrc* rope, int mod
 // What a launch with these shapes does: the number of key splits and the kv heads per workgroup (1 or 2).  `in_kernel_append`:
 // the decode forms that finish / append the new token themselves (they never take the many-queries kernel).
 void nc_attention_plan(int B, int T, int Hkv, int window_left, int Tmax, int force_splits, int* splits_out, int* heads_per_wg_out) {
-    const int max_keys = (window_left >= 0 && window_left + 1 < Tmax) ? window_left + 1 : Tmax;
-    const int nsplit = force_splits > 0 ? force_splits : pick_splits(B, T, Hkv, max_keys);
+    const int nsplit = force_splits > 0 ? force_splits : pick_splits(B, T, Hkv, visible_keys(window_left, Tmax), COUNTERS_CLEAR);
     if (splits_out) *splits_out = nsplit;
     if (heads_per_wg_out) *heads_per_wg_out = (force_splits > 0 || nsplit > 1) ? 1 : pick_heads_per_wg(B, T, Hkv);
 }
@@ -559,19 +570,19 @@ void nc_attention_plan(int B, int T, int Hkv, int window_left, int Tmax, int for
 int nc_launch_attention(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache, const int32_t* cache_seqlens,
                         int window_left, bf16_t* out, int B, int T, int H, int Hkv, int Tmax, int seqlens_include_new,
                         uint32_t* counters, void* partials, size_t partial_bytes, uint32_t* amax_ws, int force_splits,
-                        int counters_are_zero, hipStream_t s) {
+                        int counters_of_pass, hipStream_t s) {
     return launch_attention_impl(q, nullptr, 0, const_cast<bf16_t*>(k_cache), const_cast<bf16_t*>(v_cache), cache_seqlens, window_left, out,
                                  B, T, H, Hkv, Tmax, seqlens_include_new, counters, partials, partial_bytes, amax_ws, force_splits,
-                                 counters_are_zero, s);
+                                 counters_of_pass ? COUNTERS_OF_PASS : COUNTERS_CLEAR, s);
 }
 
 // Decode step, one new token per row, cache_seqlens not yet counting it: finish the q|k|v linear (rotary, QK-norm,
 // value embedding), append key and value at cache_seqlens[b], attend.  counters / partials as for nc_launch_attention.
 int nc_launch_attention_fused(NcRopeSrc rope, bf16_t* k_cache, bf16_t* v_cache, const int32_t* cache_seqlens, int window_left,
                               bf16_t* out, int B, int H, int Hkv, int Tmax, uint32_t* counters, void* partials, size_t partial_bytes,
-                              uint32_t* amax_ws, int force_splits, int counters_are_zero, hipStream_t s) {
+                              uint32_t* amax_ws, int force_splits, int counters_of_pass, hipStream_t s) {
     return launch_attention_impl(nullptr, &rope, 1, k_cache, v_cache, cache_seqlens, window_left, out, B, 1, H, Hkv, Tmax, 0, counters,
-                                 partials, partial_bytes, amax_ws, force_splits, counters_are_zero, s);
+                                 partials, partial_bytes, amax_ws, force_splits, counters_of_pass ? COUNTERS_OF_PASS : COUNTERS_CLEAR, s);
 }
 
 // Decode attention for rows that share their first `shared_len` cached tokens (one prompt replicated to every row,
@@ -591,7 +602,7 @@ int nc_launch_attention_shared(const bf16_t* q, const bf16_t* k_cache, const bf1
     if (rc) return rc;
     // (one split whatever the batch: a row's own tail is short, and the merge of the shared part belongs to the workgroup that has the row)
     return launch_attention_impl(q, nullptr, 0, const_cast<bf16_t*>(k_cache), const_cast<bf16_t*>(v_cache), cache_seqlens, window_left, out, B, 1,
-                                 H, Hkv, Tmax, seqlens_include_new, nullptr, nullptr, 0, amax_ws, 1, 1, s, shared_len, (const float*)shared_parts,
+                                 H, Hkv, Tmax, seqlens_include_new, nullptr, nullptr, 0, amax_ws, 1, COUNTERS_CLEARED, s, shared_len, (const float*)shared_parts,
                                  nchunks);
 }
 
@@ -627,17 +638,17 @@ int nc_launch_attention_append(const bf16_t* q, const bf16_t* k_new, const bf16_
         NcRopeSrc src{};
         src.k_new = k_new, src.v_new = v_new;
         return launch_attention_impl(q, &src, 2, k_cache, v_cache, cache_seqlens, window_left, out, B, 1, H, Hkv, Tmax, 0, counters, partials,
-                                     partial_bytes, amax_ws, force_splits, 0, s);
+                                     partial_bytes, amax_ws, force_splits, COUNTERS_CLEAR, s);
     }
     // (nothing is written before the sizes and the workspace are known to be right: the counters are B T Hkv words of room for B T H)
     int nsplit = 1;
     if (takes_prefill(T, force_splits)) NC_CHECK_ARG(H % Hkv == 0, "attention_append: n_head %d not a multiple of n_kv_head %d", H, Hkv);
-    else if (const int rc = check_attention(window_left, B, T, H, Hkv, Tmax, counters, partials, partial_bytes, force_splits, &nsplit)) return rc;
+    else if (const int rc = check_attention(window_left, B, T, H, Hkv, Tmax, counters, partials, partial_bytes, force_splits, COUNTERS_CLEARED, &nsplit)) return rc;
     hipLaunchKernelGGL(kv_append_kernel, dim3(T, B), dim3(Hkv * 16 < 256 ? Hkv * 16 : 256), 0, s, k_new, v_new, k_cache, v_cache,
                        cache_seqlens, T, Tmax, Hkv * 128, nsplit > 1 ? counters : nullptr);
     NC_CHECK_LAUNCH("kv_append");
     return launch_attention_impl(q, nullptr, 0, k_cache, v_cache, cache_seqlens, window_left, out, B, T, H, Hkv, Tmax, 0, counters, partials,
-                                 partial_bytes, amax_ws, force_splits, 1, s);
+                                 partial_bytes, amax_ws, force_splits, COUNTERS_CLEARED, s);
 }
 
 // ------------------------------------------------------------------------------------------------

@@ -117,7 +117,7 @@ size_t nc_attn_partial_bytes(int B, int T, int H);
 int nc_launch_attention(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache, const int32_t* cache_seqlens,
                         int window_left, bf16_t* out, int B, int T, int H, int Hkv, int Tmax, int seqlens_include_new,
                         uint32_t* counters, void* partials, size_t partial_bytes, uint32_t* amax_ws, int force_splits,
-                        int counters_are_zero, hipStream_t s);
+                        int counters_of_pass, hipStream_t s);
 
 // many query positions per row (nc_attention_prefill.hip): flash-attention forward on the bf16 matrix cores
 // compute units of the current device (looked up once per process and device)
@@ -147,7 +147,7 @@ int nc_launch_attention_static(const bf16_t* q, const bf16_t* k_cache, const bf1
 struct NcRopeSrc;
 int nc_launch_attention_fused(NcRopeSrc rope, bf16_t* k_cache, bf16_t* v_cache, const int32_t* cache_seqlens, int window_left,
                               bf16_t* out, int B, int H, int Hkv, int Tmax, uint32_t* counters, void* partials, size_t partial_bytes,
-                              uint32_t* amax_ws, int force_splits, int counters_are_zero, hipStream_t s);
+                              uint32_t* amax_ws, int force_splits, int counters_of_pass, hipStream_t s);
 
 // ---- sampling (nc_sample.hip)
 int nc_launch_softcap(const bf16_t* raw, float* out, int64_t n, float softcap, hipStream_t s);

@@ -680,6 +680,25 @@ def test_append_of_several_tokens_clears_its_split_counters(ops, T, splits):
         assert rel_l2(got, want) <= 2 * 2.0 ** -9            # one bf16 rounding each of the same fp32 sums
 
 
+@pytest.mark.parametrize("B,T,H,Hkv,Tmax", [(1, 1, 2, 2, 256), (1, 1, 26, 13, 300), (5, 1, 8, 4, 511), (2, 3, 4, 1, 400), (1, 15, 8, 2, 511)])
+def test_short_caches_need_no_workspace(ops, B, T, H, Hkv, Tmax):
+    """Below 512 keys a call by itself takes them in one piece, with and without a workspace, attending and appending."""
+    from nanochat_amd import _lib
+    say(f"no workspace: {B} rows of {T}, {H} heads on {Hkv}, {Tmax} keys")
+    assert ops.decode_attention_plan(B, T, Hkv, -1, Tmax)[0] == 1 and ops.decode_attention_plan(1, 1, Hkv, -1, 512)[0] > 1
+    g = torch.Generator(device=DEV).manual_seed(Tmax)
+    q, kc, vc = (torch.randn(*shape, generator=g, device=DEV).bfloat16() for shape in ((B, T, H, 128), (B, Tmax, Hkv, 128), (B, Tmax, Hkv, 128)))
+    n = torch.full((B,), Tmax - T, dtype=torch.int32, device=DEV)
+    want, got, appended = ops.decode_attention(q, kc, vc, n), torch.empty_like(q), torch.empty_like(q)
+    k, v = kc[:, Tmax - T:].contiguous(), vc[:, Tmax - T:].contiguous()
+    kd, vd = kc.clone(), vc.clone()
+    lib, s = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    _lib.check(lib.nc_decode_attention(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), n.data_ptr(), -1, got.data_ptr(), B, T, H, Hkv, Tmax, 0, None, 0, None, 0, s))
+    _lib.check(lib.nc_decode_attention_append(q.data_ptr(), k.data_ptr(), v.data_ptr(), kd.data_ptr(), vd.data_ptr(), n.data_ptr(), -1, appended.data_ptr(),
+                                              B, T, H, Hkv, Tmax, None, 0, None, 0, s))
+    assert torch.equal(got, want) and torch.equal(appended, want) and torch.equal(kd, kc) and torch.equal(vd, vc)
+
+
 @pytest.mark.parametrize("T,H,Hkv,splits", [(2, 2, 64, 0), (3, 3, 2, 4), (5, 6, 2, 1), (3, 4, 2, 17), (20, 2, 5, 0)])
 def test_append_refuses_sizes_before_it_writes(ops, T, H, Hkv, splits):
     """Heads that do not go together, a group of three, too many splits: an error, and cache and workspace as they were.  (The split counters have room for
