@@ -628,6 +628,10 @@ int nc_launch_embed_norm_smear(const int64_t* idx, const bf16_t* wte, const floa
     return 0;
 }
 
+// A wave to a row once that many workgroups would queue at the amax site; a wave takes a row's 512-column pieces one after the other, so the
+// line lies higher for wider rows (256 columns: 512 rows 4.5 -> 3.7 us; 1664: 1024 rows 6.7 against 7.2, 1792 rows 10.0 -> 8.5).
+bool nc_mix_norm_wave_rows(int rows, int cols) { return cols % 8 == 0 && cols <= 2048 && rows >= 512 + 256 * ((cols + 511) / 512); }
+
 static int launch_mix_norm_impl(bf16_t* x, const bf16_t* add, NcPartialSrc padd, const bf16_t* x0, const float* resid_lambda,
                                 const float* x0_lambda, const float* backout_lambda, const bf16_t* backout_src, bf16_t* backout_save,
                                 bf16_t* xn_out, int rows, int cols, uint32_t* amax_ws, hipStream_t s, int32_t* bump, int bump_by) {
@@ -648,10 +652,8 @@ static int launch_mix_norm_impl(bf16_t* x, const bf16_t* add, NcPartialSrc padd,
         if (padd.parts) hipLaunchKernelGGL((mix_norm_vec_kernel<NVV, true>), dim3(rows), dim3(256), 0, s, MIX_ARGS);      \
         else hipLaunchKernelGGL((mix_norm_vec_kernel<NVV, false>), dim3(rows), dim3(256), 0, s, MIX_ARGS);                \
     } while (0)
-    // a wave to a row once that many workgroups would queue at the amax site; a wave takes a row's 512-column pieces one after the other, so the
-    // line lies higher for wider rows (256 columns: 512 rows 4.5 -> 3.7 us; 1664: 1024 rows 6.7 against 7.2, 1792 rows 10.0 -> 8.5), and without a
-    // site a workgroup per row is the faster one at any count (1664 columns, 8192 rows: 22.5 against 25.5)
-    if (aligned && cols <= 2048 && !padd.parts && amax_ws && rows >= 512 + 256 * ((cols + 511) / 512))
+    // (without a site a workgroup per row is the faster one at any count: 1664 columns, 8192 rows 22.5 us against 25.5)
+    if (aligned && !padd.parts && amax_ws && nc_mix_norm_wave_rows(rows, cols))
         hipLaunchKernelGGL(mix_norm_rows_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, x, add, x0, resid_lambda, x0_lambda, backout_lambda,
                            backout_src, backout_save, xn_out, rows, cols, amax_ws, bump, bump_by);
     else if (aligned && cols <= 2048) MIX_LAUNCH(1);

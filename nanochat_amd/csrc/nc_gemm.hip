@@ -1420,9 +1420,13 @@ int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const
 // tokens leaves most CUs without a tile of a narrow weight otherwise, and K = 4 E is one chain of 32 to 52 steps of half a microsecond (170 rows,
 // 1024 x 4096: 24 tiles, 17 us).  us a prompt, in one piece / in shares: depth 16, 170 tokens 1208 / 1045, depth 20, 250 1776 / 1492, 500 1965 / 1756,
 // depth 26, 200 2257 / 1968, 400 2624 / 2418, depth 12, 1000 1096 / 1054.  From more than cus / 2 tiles on there is nothing to fill.  (The q|k|v linear
-// has three times the tiles and a consumer that reads fp32 sums more slowly than bf16: 1045 / 1087.)
+// has three times the tiles and a consumer that reads fp32 sums more slowly than bf16: 1045 / 1087.)  Nor do shares pay for up to 768 columns once the
+// row pass would take a wave to a row, which it does for bf16 rows only: the chain saved is 4 to 12 steps there (one piece / shares: depth 4, 800 rows
+// 296 / 320, 1792 334 / 357, depth 6, 1792 524 / 541, depth 8, 1100 648 / 676, depth 12, 1300 1122 / 1138; depth 14, 1100 1317 / 1317, depth 16, 1024
+// 1551 / 1533).
 int nc_gemm_prompt_splits(int M, int N, int K) {
     if (M <= 128 || K % 128 != 0 || N % 8 != 0 || N > 8192 || (long)M * K >= (1L << 31) || (long)N * K >= (1L << 31)) return 1;
+    if (N <= 768 && nc_mix_norm_wave_rows(M, N)) return 1;
     const long tiles = (long)((M + 63) / 64) * ((N + 127) / 128);
     long s = cu_count() / tiles;
     if (s > 8) s = 8;

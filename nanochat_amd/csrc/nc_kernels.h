@@ -95,6 +95,8 @@ int nc_launch_mix_norm(bf16_t* x, const bf16_t* add, const bf16_t* x0, const flo
                        int rows, int cols, uint32_t* amax_ws, hipStream_t s, int32_t* bump = nullptr, int bump_by = 0);
 // (bump: int32 [rows] or null; row r's workgroup adds bump_by to bump[r] when it is done -- the cache positions of a decode step)
 // same, with the added tensor given as split partials of the linear that produced it (decode path)
+// whether the launch above takes a wave to a row (with an amax site and bf16 rows to add; partial sums always take a workgroup to a row)
+bool nc_mix_norm_wave_rows(int rows, int cols);
 int nc_launch_mix_norm_p(bf16_t* x, NcPartialSrc add, const bf16_t* x0, const float* resid_lambda, const float* x0_lambda,
                          const float* backout_lambda, const bf16_t* backout_src, bf16_t* backout_save, bf16_t* xn_out,
                          int rows, int cols, uint32_t* amax_ws, hipStream_t s, int32_t* bump = nullptr, int bump_by = 0);

@@ -93,3 +93,17 @@ def test_hot_kernels_use_no_scratch_memory():
                         seen.add(k)
                         assert int(m.group(1)) <= kernels[k], f"{name} in {src} uses {m.group(1)} bytes of scratch per lane"
         assert seen == set(kernels), f"{src}: kernels not found in the compiler's report: {set(kernels) - seen}"
+
+
+def test_prompt_rows_that_go_a_wave_to_a_row_bring_no_partial_sums():
+    """The narrow projections of a prompt leave partial sums up to the row count at which the row pass of bf16 rows changes its form (models up to 768
+    wide; the sums are the only part of the workspace that a further row makes smaller)."""
+    def room(heads, rows):
+        m = _lib.ModelDesc(n_layer=2, n_head=heads, n_kv_head=heads, n_embd=128 * heads, vocab_size=512)
+        return _lib.lib().nc_gpt_workspace_bytes(ctypes.byref(m), 1, rows)
+    for heads, line in ((2, 768), (3, 768), (4, 768), (5, 1024), (6, 1024)):
+        shares = 4 * (line - 1) * 128 * heads * 2           # two shares at least
+        assert room(heads, line - 1) - room(heads, line - 2) < shares / 2
+        assert room(heads, line - 1) - room(heads, line) > shares / 2
+        assert room(heads, 2 * line) < 2 * room(heads, line) + 4096
+    assert room(7, 1024) > room(7, 1023)
