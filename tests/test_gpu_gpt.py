@@ -406,8 +406,32 @@ def test_long_prefill_matches_oracle(cfg_kwargs, B, P, trained_like):
 
 @pytest.mark.parametrize("heads,B,P", [(3, 1, 129), (5, 1, 193), (8, 1, 131), (5, 2, 320), (2, 3, 70)])
 def test_prompt_whose_narrow_projections_are_shared_out(heads, B, P):
-    """129 to some hundred rows: the projections leave partial sums that the row pass adds (2 to 5 shares of uneven length, ragged last tiles)."""
+    """129 to some hundred rows: the projections leave partial sums that the row pass adds (2 to 8 shares, even and uneven ones, ragged last tiles)."""
     test_long_prefill_matches_oracle(dict(sequence_len=512, vocab_size=512, n_layer=2, n_head=heads, n_kv_head=heads, n_embd=128 * heads, window_pattern="SL"), B, P, False)
+
+
+@pytest.mark.parametrize("heads,rows,of", [(8, 131, "mlp"), (8, 131, "attn"), (5, 193, "mlp"), (16, 500, "mlp"), (16, 500, "attn"), (13, 320, "mlp"), (4, 129, "mlp")])
+def test_shared_out_projection_is_the_one_in_one_piece(heads, rows, of):
+    """The same rows alone, whose projection is cut into 8, 2, 5, 2, 2, 3 and 4 shares, and ten to sixteen times over, where it is not cut.  The tensorwise
+    scales are the same, the other projection is zero, and a row that attends to itself alone has its value: so what differs is the order of fp32 sums,
+    which now and then turns the rounding of the projection's output and of the row it is added to (2^-8 of either at most)."""
+    say(f"shares and one piece, {heads} heads, {rows} rows, {of}")
+    from nanochat_amd.engine import KVCache
+    E = 128 * heads
+    _, model = build_pair(dict(sequence_len=128, vocab_size=1024, n_layer=2, n_head=heads, n_kv_head=heads, n_embd=E, window_pattern="L"), seed=heads)
+    with torch.no_grad():
+        for block in model.transformer.h:
+            (block.mlp if of == "attn" else block.attn).c_proj.weight.zero_()
+    idx = torch.randperm(1024, generator=torch.Generator().manual_seed(rows))[:rows, None]
+
+    def after_one_layer(times):
+        cache = KVCache(times * rows, heads, 4, 128, 2, DEV, torch.bfloat16)
+        return model.forward_tapped(idx.repeat(times, 1).to(DEV), kv_cache=cache)[1]["x"][:2, :rows, 0].float()
+    alone, many = after_one_layer(1), after_one_layer(16 if heads <= 8 else 10)
+    assert torch.equal(alone[0], many[0]) and not torch.equal(alone[0], alone[1])
+    off = (alone[1] - many[1]).abs()
+    assert (off > 0).float().mean() < 0.01
+    assert (off <= 2.0 ** -6 * many[1].abs().clamp(min=many[1].abs().mean())).all(), off.max().item()
 
 
 def test_ragged_rows():
