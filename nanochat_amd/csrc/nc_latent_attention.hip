@@ -836,15 +836,22 @@ int nc_launch_latent_attention(int dtype, const NcLatentGeom& g, const void* q_l
         else if (g.rank_p <= 256) GO32(2);
         else GO32(4);
 #undef GO32
-    } else if (dtype && step32_ok(g)) {
+        NC_CHECK_LAUNCH("latent32");
+        return 0;
+    }
+    if (dtype && step32_ok(g)) {
         const int splits = step32_splits(g);
         NC_CHECK_ARG(splits == 1 || (partials && partial_bytes >= nc_latent_partial_bytes(dtype, g)), "latent_attention: partial buffer too small");
 #define STEP32(J) hipLaunchKernelGGL((latent_step32_kernel<J>), dim3(rows, splits), dim3(256), 0, s, g, (const float*)q_lat, (const float*)cache, seqlens, (float*)out_lat, (float*)partials, splits)
         if (g.rank_p + g.rot_p <= 320) STEP32(5);
         else STEP32(9);
 #undef STEP32
+        NC_CHECK_LAUNCH("latent_step32");
         if (splits > 1) hipLaunchKernelGGL((latent_combine_kernel<float>), dim3(rows), dim3(128), 0, s, (const float*)partials, splits, g.rank_p, (float*)out_lat);
-    } else if (dtype)
+        NC_CHECK_LAUNCH("latent_combine");
+        return 0;
+    }
+    if (dtype)
         hipLaunchKernelGGL((latent_simple_kernel<float>), dim3(rows), dim3(256), bytes, s, g, (const float*)q_lat, (const float*)cache, seqlens, (float*)out_lat);
     else
         hipLaunchKernelGGL((latent_simple_kernel<bf16_t>), dim3(rows), dim3(256), bytes, s, g, (const bf16_t*)q_lat, (const bf16_t*)cache, seqlens,
