@@ -205,7 +205,7 @@ struct LinearRunner {
             return nc_launch_finish_partials((const float*)pbuf, used, w.site(site), nullptr, inv_w, segs, out, out_kind, softcap,
                                              out_amax, rows, N, ldc, s);
         }
-        // large M: explicit convert pass, tiled GEMM; relu^2 (out_kind 2) is a separate kernel there
+        // large M: explicit convert pass, tiled GEMM
         TRY(nc_launch_convert_only(in, (int64_t)rows * K, w.a8, w.inv + site, w.site(site), s));
         const int splits = src && out_kind == 0 && segs.nseg == 1 ? nc_gemm_prompt_splits(rows, N, K) : 1;
         if (splits > 1) {

@@ -1368,7 +1368,9 @@ int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const
                 // tile's K loop is one dependent step after the other: lower tiles put a workgroup on more CUs with less MFMA work per
                 // step, as long as they still fit one round of one workgroup per CU (512..1024 rows x 1664 columns with 64-row tiles:
                 // 8 us against 10.7 at K = 1664, 21 against 31 at K = 6656; 1792 rows with 96-row tiles: 10.0 / 11.5 and 27.9 / 30.5; the same for
-                // the relu^2 linear where it has that few: 170 x 4096 x 1024 12 us against 9, depth 26, 200 tokens 2356 -> 2257 us a prompt)
+                // the relu^2 linear where it has that few, us of 128-row / 64-row tiles with the clearing of its amax word: 170 x 4096 x 1024 11.6 / 9.3,
+                // 200 x 6656 x 1664 14.4 / 12.0, 1000 x 2048 x 512 10.9 / 10.2, 1000 x 1100 x 144 10.7 / 8.1; of 128-row / 96-row tiles: 500 x 5120 x 1280
+                // 13.9 / 13.0, 700 x 4096 x 1024 13.7 / 12.6, x 1008 13.9 / 12.8)
                 if (which == 5) {
                     const long tn = (N + 127) / 128;
                     if ((long)((M + 63) / 64) * tn <= cus) which = 10;

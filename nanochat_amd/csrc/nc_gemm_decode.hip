@@ -25,7 +25,7 @@
 //   gemm_decode_full_kernel     up to 64 rows, K <= 2048, relu^2 epilogue: unsplit, 32 columns per workgroup (few columns: 16),
 //                               the result leaves finished and the MLP activation needs no pass of its own
 //                               (64 rows 10.6 us against 8.3 + 4.4 us for the split linear and its finishing pass; 8 rows,
-//                               5120 x 1280, 6.6 against 3.8 + 3.9);
+//                               5120 x 1280, in a step 7.0 against 3.8 + 3.9);
 //   gemm_decode_kernel          everything else (longer K ranges walked in 512-wide chunks).
 //
 // Epilogues: 0 bf16;  1 fp32 softcap*tanh(bf16(v)/softcap) (lm_head, nanochat/gpt.py:512-515);
@@ -643,8 +643,10 @@ __global__ __launch_bounds__(256 * WR) __attribute__((amdgpu_waves_per_eu(WR, 2)
 // partial sums that cost more to write and to read back than the weights did, and the MLP activation needs no pass of its own.
 // The whole activation panel is converted into LDS once per workgroup ([K-step][16 MB rows][128 bytes] tiles) by 2 MB waves that do nothing
 // else; wave (cb, kq) then multiplies all rows with columns 16*cb .. +15 over a quarter of the K-steps, and the quarters meet through LDS.
-// MB = 4: 17 .. 64 rows, CB = 2.  MB = 1: up to 16 rows, 32 columns per workgroup (160 workgroups for 5120 columns: 7.2 us, 320 of 16 columns 7.7)
-// or, where that leaves half of the chip without one, 16.  (A step of 3 .. 16 GPT rows: 812 -> 798 us at depth 20, 8 rows, 267 -> 254 at depth 8, 16 rows.)
+// MB = 4: 17 .. 64 rows, CB = 2.  MB = 1: up to 16 rows, 32 columns per workgroup (5120 columns: 320 workgroups of 16 take 0.5 us more than 160 of 32)
+// or, where that leaves half of the chip without one, 16.  (us a step of 3 .. 16 GPT rows, split and finished / unsplit: depth 8, 16 rows 291 / 281,
+// depth 16, 12 rows 601 / 583, depth 20, 8 rows 804 / 799, 16 rows 898 / 882, depth 26, 16 rows 1259 / 1245; 3 rows 544 / 534 at depth 16 and within half a
+// per cent either way from depth 20 on.)
 // Still one trip to memory: activation rows first, then the weight rows, everything asked for before the first wait.
 #define NC_DGF_MAX_K 2048
 template <bool A_BF16, int NKS, int MB, int CB>

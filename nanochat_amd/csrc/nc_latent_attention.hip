@@ -787,8 +787,9 @@ int nc_launch_latent_append(int dtype, const NcLatentGeom& g, void* proj, int ld
 }
 
 namespace {
-// 32-bit rows for latent_step32_kernel, and the workgroups that share a row's keys: two per compute unit, 64 keys each at least.  (One token per
-// sequence: portions of several would gain as well, 30 tokens behind 400 599 -> 497 us, but a prompt's rows are to be about as exact in portions as
+// 32-bit rows for latent_step32_kernel, and the workgroups that share a row's keys: two per compute unit, 64 keys each at least.  (The shares, and with
+// them the order of a row's sums, go by the rows of the call: a sequence's last bits may depend on how many others step beside it.  One token per
+// sequence: portions of several would gain as well, 30 tokens behind 400 599 -> 497 us, but a prompt is held to be about as exact in portions as
 // in one piece, and the scores here, in 64 chains, are twice as exact as those of the kernels that take a whole prompt.)
 bool step32_ok(const NcLatentGeom& g) { return g.T == 1 && g.rank_p % 4 == 0 && g.rank_p + g.rot_p <= 576; }
 int step32_splits(const NcLatentGeom& g) {

@@ -5,8 +5,8 @@ convert_to_float8_training :243-266).  Differences that do not change results:
   * the weight is quantized once and kept (payload + inverse scale) until the parameter's storage or
     version counter changes; the reference re-quantizes it on every call (fp8.py:136), which for an
     unchanged weight produces the same bytes;
-  * without autograd (inference) no tensors are saved and the call is two launches (quantize, GEMM); with autograd the
-    three GEMMs of _Float8Matmul (fp8.py:123-192) run: e4m3 x e4m3 forward, e5m2 x e4m3 for both gradients,
+  * without autograd (inference) no tensors are saved and the call is two launches, quantize and GEMM (a third for up to 128 rows
+    whose sums are split; clear, amax and convert for a matrix past the one-launch quantizer); with autograd the three GEMMs of _Float8Matmul (fp8.py:123-192) run: e4m3 x e4m3 forward, e5m2 x e4m3 for both gradients,
     their transposed operands written by the quantization passes themselves instead of by separate copies.
 """
 import torch
