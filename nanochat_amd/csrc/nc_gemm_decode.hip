@@ -645,7 +645,7 @@ __global__ __launch_bounds__(256 * WR) __attribute__((amdgpu_waves_per_eu(WR, 2)
 // else; wave (cb, kq) then multiplies all rows with columns 16*cb .. +15 over a quarter of the K-steps, and the quarters meet through LDS.
 // MB = 4: 17 .. 64 rows, CB = 2.  MB = 1: up to 16 rows, 32 columns per workgroup (5120 columns: 320 workgroups of 16 take 0.5 us more than 160 of 32)
 // or, where that leaves half of the chip without one, 16.  (us a step of 3 .. 16 GPT rows, split and finished / unsplit: depth 8, 16 rows 291 / 281,
-// depth 16, 12 rows 601 / 583, depth 20, 8 rows 804 / 799, 16 rows 898 / 882, depth 26, 16 rows 1259 / 1245; 3 rows 544 / 534 at depth 16 and within half a
+// depth 16, 12 rows 601 / 583, depth 20, 8 rows 804 / 799, 16 rows 898 / 882, depth 26, 16 rows 1259 / 1245; 3 rows 544 / 534 at depth 16 and within one
 // per cent either way from depth 20 on.)
 // Still one trip to memory: activation rows first, then the weight rows, everything asked for before the first wait.
 #define NC_DGF_MAX_K 2048

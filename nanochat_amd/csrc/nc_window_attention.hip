@@ -628,7 +628,7 @@ int few_splits(const NcWindowGeom& g) {
     return splits < 1 ? 1 : splits > MAX_SPLITS ? MAX_SPLITS : splits;
 }
 // 32-bit rows for window_step32_kernel, and the workgroups that share a row's keys: two per compute unit, 64 keys each at least.  (So the order of a row's
-// sums goes by the rows of the call.  Portions of 2 to 31 tokens and wider heads have no such kernel yet: they take window_simple_kernel.)
+// sums goes by the rows of the call.  Portions of several tokens and heads past 256 dimensions have no such kernel yet: they take window_simple_kernel.)
 bool step32_ok(int dtype, const NcWindowGeom& g) { return dtype == 1 && g.T == 1 && g.dim_p <= 256 && g.vdim_p <= 256; }
 int step32_splits(const NcWindowGeom& g) {
     const int64_t most = (int64_t)g.window + g.keep_first;
