@@ -121,6 +121,15 @@ int nc_fp8_gemm_tn_grad(const uint8_t* a_e5m2, const uint8_t* b, const float* in
 int nc_fp8_gemm_tn_relu2(const uint8_t* a, const uint8_t* b, const float* inv_a, const float* inv_b, void* out,
                          uint32_t* out_amax, int M, int N, int K, int ldc, int kernel, nc_stream_t stream);
 
+/* The same with its result as the next linear reads it: out[M,N] = e4m3 of what nc_fp8_gemm_tn_relu2 gives, *inv_out its inverse scale, in one launch
+ * whose workgroups meet on the amax.  For shapes that are one round of tiles (.._fits).  left: bf16 [M,N] of room; meeting:
+ * nc_fp8_meeting_bytes(), all zero, cleared by the caller before every call; out and left 16-byte aligned.  spin_limit: polls (about half a
+ * microsecond each) before a workgroup stops waiting and leaves its tile to the others, below 0 the usual number. */
+size_t nc_fp8_meeting_bytes(void);
+int nc_fp8_gemm_relu2_e4m3_fits(int M, int N, int K);
+int nc_fp8_gemm_tn_relu2_e4m3(const uint8_t* a, const uint8_t* b, const float* inv_a, const float* inv_b, uint8_t* out, float* inv_out,
+                              uint16_t* left, void* meeting, int M, int N, int K, int64_t spin_limit, nc_stream_t stream);
+
 /* (1)+(2) fused for decode, M <= 128: Float8Linear.forward (nanochat/fp8.py:202-213) in one launch.
  * a_bf16 [M,K] is quantized inside the kernel with the tensorwise scale derived from *a_amax (fp32
  * bits of max|a|, e.g. produced by nc_rmsnorm / nc_mix_norm / nc_decode_attention), bit-identical to

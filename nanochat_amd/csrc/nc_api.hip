@@ -3,6 +3,7 @@
 #include "../../include/nanochat_amd.h"
 #include "nc_common.h"
 #include "nc_kernels.h"
+#include "nc_meeting.h"
 #include "nc_rope.h"
 
 extern "C" {
@@ -62,6 +63,10 @@ int nc_e4m3_encode_with_scale(const uint16_t* x, int64_t n, float scale, uint8_t
     return nc_launch_encode_with_scale(x, n, scale, 0, out, encoder, (hipStream_t)stream);
 }
 
+static NcMeeting meeting_of(void* words, int64_t spin_limit) {
+    return NcMeeting{(uint32_t*)words, spin_limit < 0 ? NC_MEETING_SPINS : spin_limit > 0xffffffffll ? 0xffffffffu : (uint32_t)spin_limit};
+}
+
 static int segs_from(const int32_t* seg_ends, int nseg, int N, NcGemmSegs* segs) {
     *segs = NcGemmSegs{1, {N, 0, 0, 0}};
     if (seg_ends) {
@@ -91,6 +96,15 @@ int nc_fp8_gemm_tn_relu2(const uint8_t* a, const uint8_t* b, const float* inv_a,
                          int N, int K, int ldc, int kernel, nc_stream_t stream) {
     NcGemmSegs segs{1, {N, 0, 0, 0}};
     return nc_launch_gemm(a, b, inv_a, inv_b, segs, out, 2, 0.f, M, N, K, ldc, kernel, nullptr, 0, (hipStream_t)stream, 0, out_amax);
+}
+
+size_t nc_fp8_meeting_bytes(void) { return NC_MEETING_WORDS * sizeof(uint32_t); }
+
+int nc_fp8_gemm_relu2_e4m3_fits(int M, int N, int K) { return nc_gemm_relu2_e4m3_kernel(M, N, K) != 0; }
+
+int nc_fp8_gemm_tn_relu2_e4m3(const uint8_t* a, const uint8_t* b, const float* inv_a, const float* inv_b, uint8_t* out, float* inv_out, uint16_t* left,
+                              void* meeting, int M, int N, int K, int64_t spin_limit, nc_stream_t stream) {
+    return nc_launch_gemm_relu2_e4m3(a, b, inv_a, inv_b, out, inv_out, nullptr, left, meeting_of(meeting, spin_limit), M, N, K, (hipStream_t)stream);
 }
 
 size_t nc_fp8_small_m_workspace_bytes(int M, int N, int K) {

@@ -22,17 +22,18 @@
 //   x, x0, xn, xb, o      bf16 [M,E]        residual stream, its initial value, normed rows, backout, GEMM out
 //   qkv                   bf16 [M,(H+2Hkv)*128]
 //   qh, y                 bf16 [M,H*128]    rotated queries, attention output
-//   h, h2                 bf16 [M,4E]       c_fc output (prefill only), relu^2
+//   h, h2                 bf16 [M,4E]       c_fc output (prefill only; or relu^2 of it as e4m3), relu^2
 //   a8                    u8   [M,4E]       quantized activations (prefill only)
 //   xl                    bf16 [B,E]        last-position rows (last_only lm_head at T > 1)
 //   inv                   fp32 [4L+1]       activation inverse scales (prefill only)
 //   zeroed                u32               amax sites [4L+1] x 8 slots on separate lines | attention split counters,
-//                                           cleared by the embedding kernel at the start of the call
+//                                           | meetings (prefill only), cleared by the embedding kernel at the start of the call
 //   gemm_parts, attn_parts                  split partials of the small-M linears and of attention
 #include <stdio.h>
 #include "../../include/nanochat_amd.h"
 #include "nc_common.h"
 #include "nc_kernels.h"
+#include "nc_meeting.h"
 #include "nc_rope.h"
 
 #define TRY(call)              \
@@ -72,6 +73,8 @@ struct Workspace {
     uint32_t *amax, *attn_counters;
     // handle of amax site i (tagged: NC_AMAX_SLOTS words on separate lines, see amax_read / amax_publish)
     uint32_t* site(int i) const { return nc_amax_slotted(amax + (size_t)i * NC_AMAX_SLOTS * NC_AMAX_STRIDE); }
+    uint32_t* meetings;        // prompts: one per amax site, for the launches that write their site's e4m3 rows themselves
+    NcMeeting meeting(int i) const { return NcMeeting{meetings + (size_t)i * NC_MEETING_WORDS, NC_MEETING_SPINS}; }
     int zero_words;
     uint8_t *gemm_parts, *gemm_parts2, *attn_parts, *shared_parts;
     size_t gemm_part_bytes, attn_part_bytes, shared_part_bytes;
@@ -121,10 +124,12 @@ Workspace carve(const nc_model_desc* m, int B, int T, void* base) {
             max_splits = sp > max_splits ? sp : max_splits;
         }
     const size_t attn_words = max_splits > 1 ? nc_attn_counter_bytes(B, T, m->n_head) / 4 : 0;
-    uint32_t* zero = c.take<uint32_t>(amax_words + attn_words);
+    const size_t meeting_words = small ? 0 : (4 * (size_t)m->n_layer + 1) * NC_MEETING_WORDS;
+    uint32_t* zero = c.take<uint32_t>(amax_words + attn_words + meeting_words);
     w.amax = zero;
     w.attn_counters = zero ? zero + amax_words : nullptr;
-    w.zero_words = (int)(amax_words + attn_words);
+    w.meetings = zero ? zero + amax_words + attn_words : nullptr;
+    w.zero_words = (int)(amax_words + attn_words + meeting_words);
     size_t gneed = 0;
     if (small) {
         const int shapes[5][2] = {{(int)qkv_w, (int)E}, {(int)E, m->n_head * 128}, {(int)(4 * E), (int)E}, {(int)E, (int)(4 * E)},
@@ -188,8 +193,18 @@ struct LinearRunner {
                             segs.nseg > 1 ? segs.end[0] : 0x7fffffff, segs.nseg > 2 ? segs.end[1] : 0x7fffffff};
         return 0;
     }
+    // relu^2 of a linear of many rows as e4m3 at w.h, its inverse scale in w.inv + out_site; false: not a shape of that launch
+    bool run_relu2_e4m3(const bf16_t* in, int rows, int site, const uint8_t* w8, const float* inv_w, int N, int K, int out_site, const uint8_t** out8, int* rc) const {
+        *out8 = nullptr;
+        if (rows <= 128 || !nc_gemm_relu2_e4m3_kernel(rows, N, K)) return false;
+        *rc = nc_launch_convert_only(in, (int64_t)rows * K, w.a8, w.inv + site, w.site(site), s);
+        if (!*rc) *rc = nc_launch_gemm_relu2_e4m3(w.a8, w8, w.inv + site, inv_w, (uint8_t*)w.h, w.inv + out_site, w.site(out_site), w.h2,
+                                                   w.meeting(out_site), rows, N, K, s);
+        *out8 = (const uint8_t*)w.h;
+        return true;
+    }
     int run(const bf16_t* in, int rows, int site, const uint8_t* w8, const float* inv_w, NcGemmSegs segs, void* out, int out_kind,
-            float softcap, uint32_t* out_amax, int N, int K, int ldc, NcPartialSrc* src, uint8_t* parts_buf = nullptr) const {
+            float softcap, uint32_t* out_amax, int N, int K, int ldc, NcPartialSrc* src, uint8_t* parts_buf = nullptr, const uint8_t* in8 = nullptr) const {
         if (src) *src = NO_PARTIALS;
         uint8_t* const pbuf = parts_buf ? parts_buf : w.gemm_parts;
         if (rows <= 128) {
@@ -205,22 +220,25 @@ struct LinearRunner {
             return nc_launch_finish_partials((const float*)pbuf, used, w.site(site), nullptr, inv_w, segs, out, out_kind, softcap,
                                              out_amax, rows, N, ldc, s);
         }
-        // large M: explicit convert pass, tiled GEMM
-        TRY(nc_launch_convert_only(in, (int64_t)rows * K, w.a8, w.inv + site, w.site(site), s));
+        // large M: explicit convert pass (unless the rows are e4m3 already: in8, their inverse scale in w.inv + site), tiled GEMM
+        if (!in8) {
+            TRY(nc_launch_convert_only(in, (int64_t)rows * K, w.a8, w.inv + site, w.site(site), s));
+            in8 = w.a8;
+        }
         const int splits = src && out_kind == 0 && segs.nseg == 1 ? nc_gemm_prompt_splits(rows, N, K) : 1;
         if (splits > 1) {
-            TRY(nc_launch_gemm_partials(w.a8, w8, (float*)pbuf, w.gemm_part_bytes, splits, rows, N, K, s));
+            TRY(nc_launch_gemm_partials(in8, w8, (float*)pbuf, w.gemm_part_bytes, splits, rows, N, K, s));
             *src = NcPartialSrc{(const float*)pbuf, splits, N, (size_t)rows * N, w.site(site), inv_w, 0x7fffffff, 0x7fffffff};
             return 0;
         }
         if (out_kind == 2) {
             // relu^2 and its amax in the GEMM's epilogue; past the 32-bit buffer offsets, the plain-load kernel and a separate pass
             if ((long)rows * K < (1L << 31) && (long)N * K < (1L << 31))
-                return nc_launch_gemm(w.a8, w8, w.inv + site, inv_w, segs, out, 2, 0.f, rows, N, K, ldc, 0, nullptr, 0, s, 0, out_amax);
-            TRY(nc_launch_gemm(w.a8, w8, w.inv + site, inv_w, segs, w.h, 0, 0.f, rows, N, K, N, 0, nullptr, 0, s));
+                return nc_launch_gemm(in8, w8, w.inv + site, inv_w, segs, out, 2, 0.f, rows, N, K, ldc, 0, nullptr, 0, s, 0, out_amax);
+            TRY(nc_launch_gemm(in8, w8, w.inv + site, inv_w, segs, w.h, 0, 0.f, rows, N, K, N, 0, nullptr, 0, s));
             return nc_launch_relu2(w.h, (bf16_t*)out, (int64_t)rows * N, out_amax, s);
         }
-        return nc_launch_gemm(w.a8, w8, w.inv + site, inv_w, segs, out, out_kind, softcap, rows, N, K, ldc, 0, nullptr, 0, s);
+        return nc_launch_gemm(in8, w8, w.inv + site, inv_w, segs, out, out_kind, softcap, rows, N, K, ldc, 0, nullptr, 0, s);
     }
 };
 }  // namespace
@@ -369,10 +387,14 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
         site++;
         // x += attn_out; xn = norm(x)
         TRY(mix(nullptr, nullptr, nullptr, nullptr, nullptr, w.site(site)));
-        // h2 = relu(c_fc(xn))^2 with its amax in the next slot
-        TRY(lin.run(w.xn, M, site, ly.w_fc, ly.inv_fc, one_seg(4 * E), w.h2, 2, 0.f, w.site(site + 1), 4 * E, E, 4 * E, nullptr));
+        // h2 = relu(c_fc(xn))^2 with its amax in the next slot, or as e4m3
+        const uint8_t* h8;
+        int rc = 0;
+        if (!lin.run_relu2_e4m3(w.xn, M, site, ly.w_fc, ly.inv_fc, 4 * E, E, site + 1, &h8, &rc))
+            rc = lin.run(w.xn, M, site, ly.w_fc, ly.inv_fc, one_seg(4 * E), w.h2, 2, 0.f, w.site(site + 1), 4 * E, E, 4 * E, nullptr);
+        if (rc) return rc;
         site++;
-        TRY(lin.run(w.h2, M, site, ly.w_mlp_proj, ly.inv_mlp_proj, one_seg(E), w.o, 0, 0.f, nullptr, E, 4 * E, E, &pending_parts));
+        TRY(lin.run(w.h2, M, site, ly.w_mlp_proj, ly.inv_mlp_proj, one_seg(E), w.o, 0, 0.f, nullptr, E, 4 * E, E, &pending_parts, nullptr, h8));
         pending_add = pending_parts.parts ? nullptr : w.o;
         site++;
     }

@@ -18,6 +18,7 @@
 #include <type_traits>
 #include "nc_common.h"
 #include "nc_kernels.h"
+#include "nc_meeting.h"
 
 // 16-byte chunk c of LDS row r (128-byte rows) is kept at chunk slot c ^ NC_SWZ(r) by the buffer-load kernels.  Measured on
 // gfx950: with this mapping a fragment read (16 rows per 16 lanes, ds_read_b128) runs at the rate of a lane-linear read
@@ -30,10 +31,14 @@ struct EpilogueArgs {
     const float* inv_b;
     NcGemmSegs segs;
     void* out;
-    int out_kind;            // 0 bf16, 1 fp32 softcap, 2 bf16 relu(v)^2 with the amax of the result published to out_amax
+    int out_kind;            // 0 bf16, 1 fp32 softcap, 2 bf16 relu(v)^2 with the amax of the result published to out_amax, 4 its e4m3 (q8_epilogue)
     float softcap;
     int ldc;
     uint32_t* out_amax;
+    // out_kind 4
+    NcMeeting meeting;
+    bf16_t* left;            // [M, N]: where a workgroup that leaves the meeting puts its tile
+    float* inv_out;
 };
 
 // relu(bf16(v))^2, to be rounded to bf16 by the caller's pack: the two eager ops of nanochat/gpt.py:139 on a bf16 tensor
@@ -293,6 +298,82 @@ __device__ __forceinline__ void bl_epilogue(v4f (&acc)[BM / WGM / 16][BN / WGN /
     }
     // no barrier and no wait here: the kernel ends, and a wave may retire with its stores still on their way, which frees the
     // CU for the next workgroup while the output drains
+}
+
+// ------------------------------------------------------------------------------------------------
+// relu^2 as the next linear reads it: every workgroup holds its tile until the launch knows the amax of the whole result (nc_meeting.h), and the tile
+// leaves as e4m3.  The launch of one round that writes bf16 ends in 24 MB of stores (1792 x 6656) that a conversion launch reads back: 26.7 + 8.4 us;
+// this way 29.3 us.  Same roundings (bf16, then e4m3 of that) and the same bits.  One tile per workgroup, all workgroups on the chip at once
+// (nc_gemm_relu2_e4m3_kernel).  N is a multiple of 16.
+template <int BM, int BN>
+__device__ __forceinline__ void q8_convert_left(const EpilogueArgs& ep, int wg, float amax, float scale, int M, int N, int tiles_m, int tiles_n) {
+    int tm, tn;
+    tile_coords(wg, tiles_m, tiles_n, tm, tn);
+    for (int id = threadIdx.x; id < BM * (BN / 16); id += blockDim.x) {
+        const int m = tm * BM + id / (BN / 16), n = tn * BN + id % (BN / 16) * 16;
+        if (m >= M || n >= N) continue;
+        const uint4* src = (const uint4*)(ep.left + (size_t)m * N + n);
+        *(uint4*)((uint8_t*)ep.out + (size_t)m * ep.ldc + n) = e4m3_of_bf16x16(src[0], src[1], scale);
+    }
+    if (wg == 0 && threadIdx.x == 0) meeting_result(amax, scale, ep.inv_out, ep.out_amax);
+}
+template <int BM, int BN, int WGM, int WGN>
+__device__ __forceinline__ void q8_epilogue(v4f (&acc)[BM / WGM / 16][BN / WGN / 16], uint8_t* lds, const EpilogueArgs& ep, float inv_a, const float (&sc)[4],
+                                            int m0, int n0, int M, int N, int tiles_m, int tiles_n) {
+    constexpr int WTM = BM / WGM / 16, WTN = BN / WGN / 16, WROWS = BM / WGM, WCOLS = BN / WGN, PITCH = WCOLS + 16, PIECES = WROWS * (WCOLS / 16);
+    static_assert(PIECES % 64 == 0 && WGM * WGN * WROWS * PITCH <= 2 * (BM + BN) * 128, "epilogue staging");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x / 64, wm = wave / WGN, wn = wave % WGN, frow = lane & 15, kb = lane >> 4;
+    uint2 held[WTM][WTN];                                      // the bf16 values, four neighbouring columns each
+    float am = 0.f;
+#pragma unroll
+    for (int j = 0; j < WTN; j++) {
+        const int n = n0 + wn * WCOLS + j * 16 + 4 * kb;
+        float inv_b = sc[0];
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            if (i + 1 < ep.segs.nseg && n >= ep.segs.end[i]) inv_b = sc[i + 1];
+#pragma unroll
+        for (int i = 0; i < WTM; i++) {
+            const v4f a4 = acc[i][j];
+            float o4[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) o4[r] = relu2_of((a4[r] * inv_a) * inv_b);
+            const uint2 pk = make_uint2(pack_bf16_hw(o4[0], o4[1]), pack_bf16_hw(o4[2], o4[3]));
+            held[i][j] = pk;
+            if (m0 + wm * WROWS + i * 16 + frow < M && n < N)
+                am = amax_fold(amax_fold(amax_fold(amax_fold(am, bf16_lo(pk.x)), bf16_hi(pk.x)), bf16_lo(pk.y)), bf16_hi(pk.y));
+        }
+    }
+    float amax;
+    bool left;
+    const bool here = meeting<WGM * WGN, 4>(ep.meeting, gridDim.x, blockIdx.x, am, amax, left, [&] {
+#pragma unroll
+        for (int j = 0; j < WTN; j++)
+#pragma unroll
+            for (int i = 0; i < WTM; i++) {
+                const int m = m0 + wm * WROWS + i * 16 + frow, n = n0 + wn * WCOLS + j * 16 + 4 * kb;
+                if (m < M && n < N) *(uint2*)(ep.left + (size_t)m * N + n) = held[i][j];
+            }
+    });
+    if (!here) return;
+    const float scale = scale_from_amax(amax);
+    if (blockIdx.x == 0 && threadIdx.x == 0) meeting_result(amax, scale, ep.inv_out, ep.out_amax);
+    // (every wave is done with the operand tiles: the meeting has barriers)
+    uint8_t* reg = lds + wave * WROWS * PITCH;
+#pragma unroll
+    for (int j = 0; j < WTN; j++)
+#pragma unroll
+        for (int i = 0; i < WTM; i++) *(uint32_t*)(reg + (i * 16 + frow) * PITCH + j * 16 + 4 * kb) = e4m3_of_bf16x4(held[i][j].x, held[i][j].y, scale);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_s_waitcnt(0xc07f);                        // lgkmcnt(0): the region is private to the wave
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int it = 0; it < PIECES / 64; it++) {
+        const int id = it * 64 + lane, row = id / (WCOLS / 16), c = id % (WCOLS / 16);
+        const int m = m0 + wm * WROWS + row, n = n0 + wn * WCOLS + c * 16;
+        if (m < M && n < N) *(uint4*)((uint8_t*)ep.out + (size_t)m * ep.ldc + n) = *(const uint4*)(reg + row * PITCH + c * 16);
+    }
+    if (left) meeting_take(ep.meeting, gridDim.x, [&](int w) { q8_convert_left<BM, BN>(ep, w, amax, scale, M, N, tiles_m, tiles_n); });
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -612,7 +693,7 @@ __device__ __forceinline__ void dl_step_barrier() {
 }
 
 // One tile per workgroup, launched tile by tile (any M, N).
-template <int A_FMT, bool RELU2>
+template <int A_FMT, int OUT_KIND>
 __global__ __launch_bounds__(512) void gemm_dl_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, EpilogueArgs ep, int M,
                                                       int N, int K, int tiles_m, int tiles_n) {
     constexpr int STAGE = 512 * 128;
@@ -671,7 +752,8 @@ __global__ __launch_bounds__(512) void gemm_dl_kernel(const uint8_t* __restrict_
     float sc[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) sc[i] = ep.inv_b[i < ep.segs.nseg ? i : 0];
-    bl_epilogue<256, 256, 4, 2, RELU2 ? 2 : 0>(acc, lds, ep, inv_a, sc, m0, n0, M, N);
+    if constexpr (OUT_KIND == 4) q8_epilogue<256, 256, 4, 2>(acc, lds, ep, inv_a, sc, m0, n0, M, N, tiles_m, tiles_n);
+    else bl_epilogue<256, 256, 4, 2, OUT_KIND>(acc, lds, ep, inv_a, sc, m0, n0, M, N);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -779,7 +861,7 @@ __device__ __forceinline__ void dln_fetch(const uint8_t* A, int a_bytes, const u
             __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_b, (lds_ptr_t)(st + 256 * 128 + i * 8192), 16, vo_b[i], k_off, 0, 0);
 }
 
-template <int NJ, bool RELU2, int A_FMT = 0>
+template <int NJ, int OUT_KIND, int A_FMT = 0>
 __global__ __launch_bounds__(512) void gemm_dln_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, EpilogueArgs ep, int M,
                                                        int N, int K, int tiles_m, int tiles_n) {
     constexpr int BN = 32 * NJ, STAGE = (256 + BN) * 128, B_PIECES = BN / 8, B_ROUNDS = (B_PIECES + 7) / 8;
@@ -833,7 +915,8 @@ __global__ __launch_bounds__(512) void gemm_dln_kernel(const uint8_t* __restrict
     float sc[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) sc[i] = ep.inv_b[i < ep.segs.nseg ? i : 0];
-    dln_epilogue<NJ, RELU2>(acc, lds, ep, inv_a, sc, g, m0, n0, M, N);
+    if constexpr (OUT_KIND == 4) q8_epilogue<256, BN, 4, 2>(acc, lds, ep, inv_a, sc, m0, n0, M, N, tiles_m, tiles_n);
+    else dln_epilogue<NJ, OUT_KIND == 2>(acc, lds, ep, inv_a, sc, g, m0, n0, M, N);
 }
 
 // the operand loads of one K-step of gemm_dr_kernel: `st` is the wave's first 1 KB piece of the stage, its pieces lie 4 KB apart
@@ -950,7 +1033,8 @@ __global__ __launch_bounds__(256) void gemm_dr_kernel(const uint8_t* __restrict_
         float sc[4];
 #pragma unroll
         for (int i = 0; i < 4; i++) sc[i] = ep.inv_b[i < ep.segs.nseg ? i : 0];
-        bl_epilogue<BM, 128, 2, 2, OUT_KIND>(acc, lds, ep, inv_a, sc, m0, n0, M, N);
+        if constexpr (OUT_KIND == 4) q8_epilogue<BM, 128, 2, 2>(acc, lds, ep, inv_a, sc, m0, n0, M, N, tiles_m, tiles_n);
+        else bl_epilogue<BM, 128, 2, 2, OUT_KIND>(acc, lds, ep, inv_a, sc, m0, n0, M, N);
     }
 }
 
@@ -1170,17 +1254,17 @@ static bool dlp_eligible(int M, int /*N*/, int K) {
     return rx >= 1 && rx <= 32 && (rx & (rx - 1)) == 0;
 }
 
-template <int A_FMT, bool RELU2>
+template <int A_FMT, int OUT_KIND>
 static int launch_dl_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, bool persistent, hipStream_t s) {
     const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
     const size_t lds_bytes = 2 * 512 * 128 + (persistent ? 8 * 4096 : 0);
-    const void* fn = persistent ? (const void*)gemm_dlp_kernel<A_FMT, RELU2> : (const void*)gemm_dl_kernel<A_FMT, RELU2>;
+    const void* fn = persistent ? (const void*)gemm_dlp_kernel<A_FMT, OUT_KIND == 2> : (const void*)gemm_dl_kernel<A_FMT, OUT_KIND>;
     hipError_t e = reserve_lds(fn, (int)lds_bytes);
     if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
     if (persistent)
-        hipLaunchKernelGGL((gemm_dlp_kernel<A_FMT, RELU2>), dim3(256), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m / 8, (N + 127) / 128);
+        hipLaunchKernelGGL((gemm_dlp_kernel<A_FMT, OUT_KIND == 2>), dim3(256), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m / 8, (N + 127) / 128);
     else
-        hipLaunchKernelGGL((gemm_dl_kernel<A_FMT, RELU2>), dim3(tiles_m * tiles_n), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
+        hipLaunchKernelGGL((gemm_dl_kernel<A_FMT, OUT_KIND>), dim3(tiles_m * tiles_n), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
     return 0;
 }
 
@@ -1218,20 +1302,21 @@ static bool dl_narrow_fills(int M, int N) {
     }
     return false;
 }
-template <int NJ, bool RELU2, int A_FMT>
+template <int NJ, int OUT_KIND, int A_FMT>
 static int launch_dln_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s) {
     const int tiles_m = (M + 255) / 256, tiles_n = (N + 32 * NJ - 1) / (32 * NJ);
     const size_t lds_bytes = 2 * (256 + 32 * NJ) * 128;
-    const void* fn = (const void*)gemm_dln_kernel<NJ, RELU2, A_FMT>;
+    const void* fn = (const void*)gemm_dln_kernel<NJ, OUT_KIND, A_FMT>;
     hipError_t e = reserve_lds(fn, (int)lds_bytes);
     if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
-    hipLaunchKernelGGL((gemm_dln_kernel<NJ, RELU2, A_FMT>), dim3(tiles_m * tiles_n), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
+    hipLaunchKernelGGL((gemm_dln_kernel<NJ, OUT_KIND, A_FMT>), dim3(tiles_m * tiles_n), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
     return 0;
 }
 template <int NJ>
 static int launch_dln_nj(int a_fmt, const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s) {
-    if (a_fmt == 1) return launch_dln_as<NJ, false, 1>(a, b, ep, M, N, K, s);
-    return ep.out_kind == 2 ? launch_dln_as<NJ, true, 0>(a, b, ep, M, N, K, s) : launch_dln_as<NJ, false, 0>(a, b, ep, M, N, K, s);
+    if (a_fmt == 1) return launch_dln_as<NJ, 0, 1>(a, b, ep, M, N, K, s);
+    if (ep.out_kind == 4) return launch_dln_as<NJ, 4, 0>(a, b, ep, M, N, K, s);
+    return ep.out_kind == 2 ? launch_dln_as<NJ, 2, 0>(a, b, ep, M, N, K, s) : launch_dln_as<NJ, 0, 0>(a, b, ep, M, N, K, s);
 }
 // bf16 or (e4m3 first operand only) relu^2 output, K a multiple of 128
 static int launch_dln(int nj, int a_fmt, const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s) {
@@ -1264,6 +1349,7 @@ static int launch_dr(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep,
     NC_CHECK_ARG((long)M * K < (1L << 31) && (long)N * K < (1L << 31), "fp8_gemm: buffer-load kernels need M*K and N*K below 2^31");
     NC_CHECK_ARG(K % 128 == 0, "fp8_gemm: the direct-to-LDS kernels need K %% 128 == 0, got %d", K);
     NC_CHECK_ARG(ep.out_kind != 1, "fp8_gemm: the direct-to-LDS kernels write bf16 only");
+    if (ep.out_kind == 4) return launch_dr_as<BM, 4>(a, b, ep, M, N, K, s);
     return ep.out_kind == 2 ? launch_dr_as<BM, 2>(a, b, ep, M, N, K, s) : launch_dr_as<BM, 0>(a, b, ep, M, N, K, s);
 }
 
@@ -1275,9 +1361,10 @@ static int launch_dl(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep,
     NC_CHECK_ARG(ep.out_kind != 1, "fp8_gemm: the direct-to-LDS kernels write bf16 only");
     if (persistent)
         NC_CHECK_ARG(dlp_eligible(M, N, K), "fp8_gemm: the persistent kernel needs M/256 (rounded up) to be 8, 16, ... 256 tile rows, got M=%d", M);
-    if (A_FMT == 0 && ep.out_kind == 2) return launch_dl_as<0, true>(a, b, ep, M, N, K, persistent, s);
+    if (A_FMT == 0 && ep.out_kind == 2) return launch_dl_as<0, 2>(a, b, ep, M, N, K, persistent, s);
+    if (A_FMT == 0 && ep.out_kind == 4 && !persistent) return launch_dl_as<0, 4>(a, b, ep, M, N, K, false, s);
     NC_CHECK_ARG(ep.out_kind == 0, "fp8_gemm: the relu^2 epilogue goes with an e4m3 first operand");
-    return launch_dl_as<A_FMT, false>(a, b, ep, M, N, K, persistent, s);
+    return launch_dl_as<A_FMT, 0>(a, b, ep, M, N, K, persistent, s);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1289,6 +1376,51 @@ static int launch_tile(const uint8_t* a, const uint8_t* b, const EpilogueArgs& e
     if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
     hipLaunchKernelGGL((gemm_tile_kernel<BM, BN>), dim3(tiles_m * tiles_n), dim3(256), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
     return 0;
+}
+
+// The kernel of a bf16, relu^2 or softcapped linear of e4m3 operands (the selectors of nc_launch_gemm).
+static int pick_kernel(int M, int N, int K, int out_kind) {
+    int which;
+    if (M <= 128) which = 1;
+    else if ((long)M * K >= (1L << 31) || (long)N * K >= (1L << 31)) which = 4;   // past the 32-bit buffer offsets
+    else {
+        const int cus = cu_count();
+        const long t256 = (long)((M + 255) / 256) * ((N + 255) / 256);
+        const long rounds = (t256 + cus - 1) / cus;
+        const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
+        if (out_kind != 1 && K % 128 == 0 && (8 * t256 >= 5 * cus || t128 > 2 * cus || dl_narrow_fills(M, N))) {
+            // 256x256 tiles fed straight into LDS whenever they occupy at least 5/8 of the CUs, or the 128x128 tiles, four times
+            // as many, would not fit the chip in one round of two workgroups per CU (below that the small tiles fill the chip
+            // better: 18 us against 22 for 1280 x 4992 x 1664, but 25 against 22.4 for 1792 rows); from two rounds of tiles on,
+            // the persistent form, which neither rounds the last round up nor pays a prologue per tile
+            which = (t256 >= 2 * cus && dlp_eligible(M, N, K)) ? 9 : 8;
+            if (which == 8) {
+                const int nj = dl_pick_nj(M, N);
+                if (nj < 8) which = 8 + nj;           // 12 .. 15
+            }
+        } else {
+            // 256x256 tiles move half the bytes per flop through L2 and LDS but run one workgroup per CU: take them
+            // when their count fills whole rounds of the CUs well, else the 128x128 tiles (two workgroups per CU)
+            which = (M >= 1024 && N >= 512 && 10 * t256 >= 8 * rounds * cus && rounds <= 2) ? 7 : 5;
+            // a prompt of a few hundred to two thousand rows against a narrow weight leaves CUs without a 128x128 tile, and each
+            // tile's K loop is one dependent step after the other: lower tiles put a workgroup on more CUs with less MFMA work per
+            // step, as long as they still fit one round of one workgroup per CU (512..1024 rows x 1664 columns with 64-row tiles:
+            // 8 us against 10.7 at K = 1664, 21 against 31 at K = 6656; 1792 rows with 96-row tiles: 10.0 / 11.5 and 27.9 / 30.5; the same for
+            // the relu^2 linear where it has that few, us of 128-row / 64-row tiles with the clearing of its amax word: 170 x 4096 x 1024 11.6 / 9.3,
+            // 200 x 6656 x 1664 14.4 / 12.0, 1000 x 2048 x 512 10.9 / 10.2, 1000 x 1100 x 144 10.7 / 8.1; of 128-row / 96-row tiles: 500 x 5120 x 1280
+            // 13.9 / 13.0, 700 x 4096 x 1024 13.7 / 12.6, x 1008 13.9 / 12.8)
+            if (which == 5) {
+                const long tn = (N + 127) / 128;
+                if ((long)((M + 63) / 64) * tn <= cus) which = 10;
+                else if ((long)((M + 95) / 96) * tn <= cus) which = 11;
+                // the same tiles fed straight into a ring of four LDS stages where K allows it: three K-steps of operands on their
+                // way instead of two and no ds_write phase (1792 x 1664 x 6656: 27.5 -> 25.6 us, 1024 rows: 21.9 -> 20.8 us; what is
+                // left is the L2's bandwidth: 28 KB per K-step and CU for tiles this small)
+                if (which >= 10 && K % 128 == 0 && out_kind != 1) which += 6;
+            }
+        }
+    }
+    return which;
 }
 
 int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const float* inv_b, NcGemmSegs segs,
@@ -1312,7 +1444,7 @@ int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const
         NC_CHECK_ARG(((uintptr_t)out & 7) == 0 && ldc % 4 == 0, "fp8_gemm: bf16 output needs 8-byte alignment and ldc %% 4 == 0");
     NC_CHECK_ARG(a_fmt == 0 || a_fmt == 1, "fp8_gemm: the format of a must be 0 (e4m3fn) or 1 (e5m2)");
     if (M == 0) return 0;
-    EpilogueArgs ep{inv_a, inv_b, segs, out, out_kind, softcap, ldc, out_amax};
+    EpilogueArgs ep{inv_a, inv_b, segs, out, out_kind, softcap, ldc, out_amax, NcMeeting{}, nullptr, nullptr};
     if (a_fmt == 1) {
         // gradient operand (the backward GEMMs): bf16 output through the 128x128 buffer-load tile or the 256x256 direct-to-LDS tiles
         NC_CHECK_ARG(out_kind == 0, "fp8_gemm: an e5m2 operand goes with bf16 output");
@@ -1341,48 +1473,7 @@ int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const
     // 8 direct-to-LDS 256x256 tile by tile, 9 the same persistent, 10 / 11 buffer-load tiles 64x128 / 96x128,
     // 12 .. 15 direct-to-LDS tiles of 256 x 128 / 160 / 192 / 224 tile by tile, 16 / 17 / 18 direct-to-LDS tiles of 64 / 96 / 128 x 128
     // with four stages
-    int which = force_kernel;
-    if (which == 0) {
-        if (M <= 128) which = 1;
-        else if ((long)M * K >= (1L << 31) || (long)N * K >= (1L << 31)) which = 4;   // past the 32-bit buffer offsets
-        else {
-            const int cus = cu_count();
-            const long t256 = (long)((M + 255) / 256) * ((N + 255) / 256);
-            const long rounds = (t256 + cus - 1) / cus;
-            const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128);
-            if (out_kind != 1 && K % 128 == 0 && (8 * t256 >= 5 * cus || t128 > 2 * cus || dl_narrow_fills(M, N))) {
-                // 256x256 tiles fed straight into LDS whenever they occupy at least 5/8 of the CUs, or the 128x128 tiles, four times
-                // as many, would not fit the chip in one round of two workgroups per CU (below that the small tiles fill the chip
-                // better: 18 us against 22 for 1280 x 4992 x 1664, but 25 against 22.4 for 1792 rows); from two rounds of tiles on,
-                // the persistent form, which neither rounds the last round up nor pays a prologue per tile
-                which = (t256 >= 2 * cus && dlp_eligible(M, N, K)) ? 9 : 8;
-                if (which == 8) {
-                    const int nj = dl_pick_nj(M, N);
-                    if (nj < 8) which = 8 + nj;           // 12 .. 15
-                }
-            } else {
-                // 256x256 tiles move half the bytes per flop through L2 and LDS but run one workgroup per CU: take them
-                // when their count fills whole rounds of the CUs well, else the 128x128 tiles (two workgroups per CU)
-                which = (M >= 1024 && N >= 512 && 10 * t256 >= 8 * rounds * cus && rounds <= 2) ? 7 : 5;
-                // a prompt of a few hundred to two thousand rows against a narrow weight leaves CUs without a 128x128 tile, and each
-                // tile's K loop is one dependent step after the other: lower tiles put a workgroup on more CUs with less MFMA work per
-                // step, as long as they still fit one round of one workgroup per CU (512..1024 rows x 1664 columns with 64-row tiles:
-                // 8 us against 10.7 at K = 1664, 21 against 31 at K = 6656; 1792 rows with 96-row tiles: 10.0 / 11.5 and 27.9 / 30.5; the same for
-                // the relu^2 linear where it has that few, us of 128-row / 64-row tiles with the clearing of its amax word: 170 x 4096 x 1024 11.6 / 9.3,
-                // 200 x 6656 x 1664 14.4 / 12.0, 1000 x 2048 x 512 10.9 / 10.2, 1000 x 1100 x 144 10.7 / 8.1; of 128-row / 96-row tiles: 500 x 5120 x 1280
-                // 13.9 / 13.0, 700 x 4096 x 1024 13.7 / 12.6, x 1008 13.9 / 12.8)
-                if (which == 5) {
-                    const long tn = (N + 127) / 128;
-                    if ((long)((M + 63) / 64) * tn <= cus) which = 10;
-                    else if ((long)((M + 95) / 96) * tn <= cus) which = 11;
-                    // the same tiles fed straight into a ring of four LDS stages where K allows it: three K-steps of operands on their
-                    // way instead of two and no ds_write phase (1792 x 1664 x 6656: 27.5 -> 25.6 us, 1024 rows: 21.9 -> 20.8 us; what is
-                    // left is the L2's bandwidth: 28 KB per K-step and CU for tiles this small)
-                    if (which >= 10 && K % 128 == 0 && out_kind != 1) which += 6;
-                }
-            }
-        }
-    }
+    const int which = force_kernel ? force_kernel : pick_kernel(M, N, K, out_kind);
     int rc = 0;
     if (which != 1) NC_CHECK_ARG(which >= 4 && which <= 18, "fp8_gemm: unknown kernel selector %d", force_kernel);
     NcProfScope prof(which == 1 ? -1 : 1, 2.0 * M * N * K, s, ((int64_t)N << 32) | (uint32_t)K);
@@ -1414,6 +1505,35 @@ int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const
     else NC_FAIL(-1, "fp8_gemm: unknown kernel selector %d", force_kernel);
     if (rc) return rc;
     NC_CHECK_LAUNCH("fp8_gemm");
+    return 0;
+}
+
+// The kernel that leaves relu^2 of a linear as e4m3 (out_kind 4), or 0: the tiles of pick_kernel where they are one round of one workgroup per CU (each
+// takes more than half of a CU's LDS), so that all of them can hold their tile until everybody's amax is known.
+int nc_gemm_relu2_e4m3_kernel(int M, int N, int K) {
+    if (M <= 128 || N % 16 != 0 || K % 128 != 0 || (long)M * K >= (1L << 31) || (long)N * K >= (1L << 31)) return 0;
+    const int which = pick_kernel(M, N, K, 2);
+    const int bm = which == 16 ? 64 : which == 17 ? 96 : which == 18 ? 128 : 256;
+    const int bn = which >= 16 && which <= 18 ? 128 : which >= 12 && which <= 15 ? 32 * (which - 8) : 256;
+    if (which != 8 && (which < 12 || which > 18)) return 0;
+    const long wgs = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
+    return wgs <= cu_count() && wgs <= 256 ? which : 0;
+}
+
+int nc_launch_gemm_relu2_e4m3(const uint8_t* a, const uint8_t* b, const float* inv_a, const float* inv_b, uint8_t* out, float* inv_out, uint32_t* out_amax,
+                              bf16_t* left, NcMeeting meeting, int M, int N, int K, hipStream_t s) {
+    NC_CHECK_ARG(a && b && inv_a && inv_b && out && inv_out && left && meeting.words, "fp8_gemm_relu2_e4m3: null pointer");
+    NC_CHECK_ARG((((uintptr_t)a | (uintptr_t)b | (uintptr_t)out | (uintptr_t)left) & 15) == 0, "fp8_gemm_relu2_e4m3: operands must be 16-byte aligned");
+    const int which = nc_gemm_relu2_e4m3_kernel(M, N, K);
+    NC_CHECK_ARG(which != 0, "fp8_gemm_relu2_e4m3: M=%d N=%d K=%d is not one round of tiles", M, N, K);
+    EpilogueArgs ep{inv_a, inv_b, NcGemmSegs{1, {N, 0, 0, 0}}, out, 4, 0.f, N, out_amax, meeting, left, inv_out};
+    NcProfScope prof(1, 2.0 * M * N * K, s, ((int64_t)N << 32) | (uint32_t)K);
+    const int rc = which == 8 ? launch_dl<0>(a, b, ep, M, N, K, false, s)
+                   : which == 16 ? launch_dr<64>(a, b, ep, M, N, K, s)
+                   : which == 17 ? launch_dr<96>(a, b, ep, M, N, K, s)
+                   : which == 18 ? launch_dr<128>(a, b, ep, M, N, K, s) : launch_dln(which - 8, 0, a, b, ep, M, N, K, s);
+    if (rc) return rc;
+    NC_CHECK_LAUNCH("fp8_gemm_relu2_e4m3");
     return 0;
 }
 

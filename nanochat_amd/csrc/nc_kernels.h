@@ -38,6 +38,13 @@ int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const
 int nc_gemm_prompt_splits(int M, int N, int K);
 int nc_launch_gemm_partials(const uint8_t* a, const uint8_t* b, float* parts, size_t part_bytes, int splits, int M, int N, int K, hipStream_t s);
 
+// relu^2 of a linear of more than 128 rows as e4m3 with its inverse scale and (out_amax, may be null) its amax, in one launch whose workgroups meet on the amax (nc_meeting.h); `left`:
+// bf16 [M, N] room.  nc_gemm_relu2_e4m3_kernel: whether the shape is one round of tiles (0: no).
+struct NcMeeting;
+int nc_gemm_relu2_e4m3_kernel(int M, int N, int K);
+int nc_launch_gemm_relu2_e4m3(const uint8_t* a, const uint8_t* b, const float* inv_a, const float* inv_b, uint8_t* out, float* inv_out, uint32_t* out_amax,
+                              bf16_t* left, NcMeeting meeting, int M, int N, int K, hipStream_t s);
+
 // small-M path (nc_gemm_decode.hip): A is e4m3 (+inv_a) or bf16 (+amax, quantized inside the kernel)
 // out_kind: 0 bf16, 1 softcapped fp32, 2 bf16 relu^2 with amax of the result into out_amax.
 // With K split over workgroups the raw fp32 sums land in `partials` [ksplits][M][N] and a consumer finishes them.

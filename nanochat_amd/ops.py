@@ -221,6 +221,27 @@ def fp8_gemm_relu2(a8, w8, inv_a, inv_w, kernel=0):
     return out, amax
 
 
+def _meeting(device):
+    return torch.zeros(_lib.lib().nc_fp8_meeting_bytes() // 4, dtype=torch.int32, device=device)
+
+
+def fp8_gemm_relu2_e4m3(a8, w8, inv_a, inv_w, spin_limit=-1):
+    """fp8_gemm_relu2 and fp8_quantize of its result in one launch, the same bits: (e4m3 [M,N], inverse scale fp32 0-dim).  For shapes that are one
+    round of tiles (ValueError otherwise).  spin_limit (tests): polls before a workgroup leaves its tile to the others."""
+    _need_cuda(a8, w8, inv_a, inv_w)
+    a8, w8 = a8.contiguous(), w8.contiguous()
+    M, K = a8.shape
+    N = w8.shape[0]
+    if not _lib.lib().nc_fp8_gemm_relu2_e4m3_fits(M, N, K):
+        raise ValueError(f"fp8_gemm_relu2_e4m3: {M} x {N} x {K} is not one round of tiles")
+    out = torch.empty(M, N, dtype=torch.float8_e4m3fn, device=a8.device)
+    left = torch.empty(M, N, dtype=torch.bfloat16, device=a8.device)
+    inv, meeting = torch.empty((), dtype=torch.float32, device=a8.device), _meeting(a8.device)
+    _lib.check(_lib.lib().nc_fp8_gemm_tn_relu2_e4m3(_ptr(a8), _ptr(w8), _ptr(inv_a.reshape(-1).float()), _ptr(inv_w.reshape(-1).float()), _ptr(out),
+                                                    _ptr(inv), _ptr(left), _ptr(meeting), M, N, K, spin_limit, _stream()))
+    return out, inv
+
+
 def fp8_linear_small_m(a_bf16, amax_bits, w8, inv_w, seg_ends=None, softcap=None, relu2=False, ksplits=0):
     """Float8Linear.forward for M <= 128 rows in one launch: a_bf16 [M,K] is quantized inside the GEMM with the
     tensorwise scale of amax_bits (int32 tensor holding the fp32 bits of max|a|).  Returns the output, and with

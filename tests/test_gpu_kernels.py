@@ -382,6 +382,24 @@ def test_gemm_relu2_of_few_tiles(ops, M, N, K):
     test_gemm_relu2_epilogue_and_amax(ops, M, N, K, 0)
 
 
+@pytest.mark.parametrize("spin_limit", [-1, 0])
+@pytest.mark.parametrize("M,N,K", [(1792, 6656, 1664), (1000, 5120, 1280), (1023, 4992, 128), (130, 4096, 1024), (300, 336, 256), (1000, 2256, 384), (2048, 8192, 512),
+                                   (1300, 4096, 1024), (129, 16, 128)])
+def test_gemm_relu2_written_as_e4m3(ops, M, N, K, spin_limit):
+    """relu^2 with its workgroups meeting on the amax: the bits of the bf16 result quantized by a launch of its own.  spin_limit 0: a workgroup that does not find
+    everybody at its first look leaves its tile to the others."""
+    say(f"gemm relu2 e4m3 M={M} N={N} K={K} spins={spin_limit}")
+    a, w = make_operands(M, N, K, seed=M + N + K)
+    a8, ia, _ = fp8_ref.to_fp8(a)
+    w8, iw, _ = fp8_ref.to_fp8(w)
+    args = a8.to(DEV), w8.to(DEV), ia.to(DEV), iw.to(DEV)
+    h, _ = ops.fp8_gemm_relu2(*args)
+    want, want_inv, _ = ops.fp8_quantize(h)
+    for _ in range(3):
+        got, inv = ops.fp8_gemm_relu2_e4m3(*args, spin_limit=spin_limit)
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)) and inv.item() == want_inv.item()
+
+
 def test_gemm_softcap_epilogue(ops):
     say("gemm softcap")
     a, w = make_operands(64, 1024, 256, 11)
