@@ -161,6 +161,14 @@ int nc_mix_norm(uint16_t* x, const uint16_t* add, const uint16_t* x0, const floa
                 uint16_t* backout_save, uint16_t* xn_out, int rows, int cols, uint32_t* amax_ws,
                 nc_stream_t stream);
 
+/* The same rows as the next linear reads them: out = e4m3 of rms_norm(x2), *inv_out its inverse scale, in one launch whose workgroups meet on the amax
+ * (meeting, spin_limit: as for nc_fp8_gemm_tn_relu2_e4m3); of xn_out [rows,cols] only the first 16 columns are written (all of them where a workgroup
+ * left).  The addend as bf16 (add) or as fp32 partial sums parts[nsplit][rows][cols] of an FP8 linear (1/scale(*parts_amax) and *parts_inv_b times
+ * their sum), or neither.  cols a multiple of 16 up to 2048; up to 2048 rows, 1024 with partial sums (as many as the chip holds). */
+int nc_mix_norm_e4m3(uint16_t* x, const uint16_t* add, const float* parts, int nsplit, const uint32_t* parts_amax, const float* parts_inv_b,
+                     const uint16_t* x0, const float* resid_lambda, const float* x0_lambda, uint16_t* xn_out, uint8_t* out, float* inv_out,
+                     void* meeting, int rows, int cols, int64_t spin_limit, nc_stream_t stream);
+
 /* relu(h)^2 elementwise in bf16 (+ amax): nanochat/gpt.py:139. */
 int nc_relu2(const uint16_t* h, uint16_t* out, int64_t n, uint32_t* amax_ws, nc_stream_t stream);
 

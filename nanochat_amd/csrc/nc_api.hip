@@ -153,6 +153,18 @@ int nc_mix_norm(uint16_t* x, const uint16_t* add, const uint16_t* x0, const floa
                               amax_ws, (hipStream_t)stream);
 }
 
+int nc_mix_norm_e4m3(uint16_t* x, const uint16_t* add, const float* parts, int nsplit, const uint32_t* parts_amax, const float* parts_inv_b, const uint16_t* x0,
+                     const float* resid_lambda, const float* x0_lambda, uint16_t* xn_out, uint8_t* out, float* inv_out, void* meeting, int rows, int cols,
+                     int64_t spin_limit, nc_stream_t stream) {
+    NC_CHECK_ARG(out && inv_out && meeting, "mix_norm_e4m3: null pointer");
+    NC_CHECK_ARG(!(add && parts), "mix_norm_e4m3: give the added tensor either as bf16 or as partials");
+    const NcQuantRows q8{out, inv_out, meeting_of(meeting, spin_limit), rows};
+    if (parts)
+        return nc_launch_mix_norm_p(x, NcPartialSrc{parts, nsplit, cols, (size_t)rows * cols, parts_amax, parts_inv_b, 0x7fffffff, 0x7fffffff}, x0, resid_lambda, x0_lambda,
+                                    nullptr, nullptr, nullptr, xn_out, rows, cols, nullptr, (hipStream_t)stream, nullptr, 0, &q8);
+    return nc_launch_mix_norm(x, add, x0, resid_lambda, x0_lambda, nullptr, nullptr, nullptr, xn_out, rows, cols, nullptr, (hipStream_t)stream, nullptr, 0, &q8);
+}
+
 int nc_relu2(const uint16_t* h, uint16_t* out, int64_t n, uint32_t* amax_ws, nc_stream_t stream) {
     return nc_launch_relu2(h, out, n, amax_ws, (hipStream_t)stream);
 }

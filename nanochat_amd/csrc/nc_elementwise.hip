@@ -11,6 +11,7 @@
 // follows (atomicMax on the fp32 bit pattern, valid because the values are non-negative).
 #include "nc_common.h"
 #include "nc_kernels.h"
+#include "nc_meeting.h"
 #include "nc_rope.h"
 
 __device__ __forceinline__ void block_amax_commit(float local_abs_max, uint32_t* amax_ws, float* red) {
@@ -181,22 +182,42 @@ __global__ __launch_bounds__(256) void mix_norm_kernel(bf16_t* __restrict__ x, c
     block_amax_commit(am, amax_ws, red);
 }
 
+// The row passes of a prompt write what the linear behind them reads (Q8): the workgroups hold their rows until the amax of all of them is known
+// (nc_meeting.h) and write them as e4m3; of the bf16 rows only the first 16 columns, which the value embedding's gate reads, go to memory.
+// 1792 rows of 1664 columns: 10.7 us, against 9.8 and 5.0 for the pass and a conversion launch; 500 rows of 1280 with two and three partial sums 7.4, against
+// 6.8 and 3.9.  The new residual stream is stored while the maxima travel.
+__device__ __forceinline__ void convert_left_rows(const NcQuantRows& q8, const bf16_t* __restrict__ xn, int wg, int rows_per_wg, int rows, int cols, float amax,
+                                                  float scale, uint32_t* amax_ws) {
+    const size_t first = (size_t)wg * rows_per_wg * cols, end = (size_t)min((wg + 1) * rows_per_wg, rows) * cols;
+    for (size_t at = first + threadIdx.x * 8; at < end; at += blockDim.x * 8) {
+        const uint4 w = *(const uint4*)(xn + at);
+        *(uint2*)(q8.out + at) = make_uint2(e4m3_of_bf16x4(w.x, w.y, scale), e4m3_of_bf16x4(w.z, w.w, scale));
+    }
+    if (wg == 0 && threadIdx.x == 0) meeting_result(amax, scale, q8.inv_out, amax_ws);
+}
+
 // Same contract as mix_norm_kernel for cols % 8 == 0 and cols <= 2048 * NV: the row stays in registers,
 // eight bf16 per 16-byte access, one reduction, one pass over memory.
 // PARTS: the addend arrives as split partial sums (decode).  Without them the kernel needs a third of the registers, and the
 // thousands of one-row workgroups of a prefill fit the chip in one round instead of two.
-template <int NV, bool PARTS>
-__global__ __launch_bounds__(256) void mix_norm_vec_kernel(bf16_t* __restrict__ x, const bf16_t* __restrict__ add, NcPartialSrc padd,
+// Q8_ROWS: rows to a workgroup of 256 threads each, as e4m3 (0: one row, as bf16).
+template <int NV, bool PARTS, int Q8_ROWS = 0>
+__global__ __launch_bounds__(256 * (Q8_ROWS > 1 ? Q8_ROWS : 1)) void mix_norm_vec_kernel(bf16_t* __restrict__ x, const bf16_t* __restrict__ add, NcPartialSrc padd,
                                                            const bf16_t* __restrict__ x0, const float* __restrict__ resid_lambda,
                                                            const float* __restrict__ x0_lambda, const float* __restrict__ backout_lambda,
                                                            const bf16_t* __restrict__ backout_src, bf16_t* __restrict__ backout_save,
                                                            bf16_t* __restrict__ xn_out, int cols, uint32_t* __restrict__ amax_ws,
-                                                           int32_t* __restrict__ bump, int bump_by) {
+                                                           int32_t* __restrict__ bump, int bump_by, NcQuantRows q8) {
     NC_ARG_NOW(x); NC_ARG_NOW(add); NC_ARG_NOW(padd.parts); NC_ARG_NOW(padd.nsplit); NC_ARG_NOW(padd.ld); NC_ARG_NOW(padd.split_stride);
     NC_ARG_NOW(padd.a_amax); NC_ARG_NOW(padd.inv_b); NC_ARG_NOW(x0); NC_ARG_NOW(resid_lambda); NC_ARG_NOW(x0_lambda);
     NC_ARG_NOW(backout_lambda); NC_ARG_NOW(backout_src); NC_ARG_NOW(backout_save); NC_ARG_NOW(xn_out); NC_ARG_NOW(cols); NC_ARG_NOW(amax_ws);
-    __shared__ float red[8];
-    const size_t base = (size_t)blockIdx.x * cols;
+    constexpr bool Q8 = Q8_ROWS > 0;
+    constexpr int ROWS = Q8 ? Q8_ROWS : 1;
+    __shared__ float red[4 * ROWS > 8 ? 4 * ROWS : 8];
+    const int tid = ROWS > 1 ? threadIdx.x & 255 : threadIdx.x, in_wg = ROWS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, row = blockIdx.x * ROWS + in_wg;
+    const int all_cols = cols;
+    if (ROWS > 1 && row >= q8.rows) cols = 0;                 // (past the last row: nothing is loaded or stored)
+    const size_t base = (size_t)row * all_cols;
     const bool has_parts = PARTS && padd.parts != nullptr;
     const bool writes_x = add || has_parts || resid_lambda || backout_lambda;
     const bf16_t* zsrc = resid_lambda ? x0 : (backout_lambda ? backout_src : nullptr);
@@ -212,13 +233,13 @@ __global__ __launch_bounds__(256) void mix_norm_vec_kernel(bf16_t* __restrict__ 
     float4 a0[PARTS ? NV : 1][8], a1[PARTS ? NV : 1][8];
 #pragma unroll
     for (int it = 0; it < NV; it++) {
-        const int c = (threadIdx.x + it * 256) * 8;
+        const int c = (tid + it * 256) * 8;
         if (c < cols) {
             xv[it] = *(const uint4*)(x + base + c);
             if (add) av[it] = *(const uint4*)(add + base + c);
             if (zsrc) zv[it] = *(const uint4*)(zsrc + base + c);
             if (has_parts) {
-                const float* pp = padd.parts + (size_t)blockIdx.x * padd.ld + c;
+                const float* pp = padd.parts + (size_t)row * padd.ld + c;
 #pragma unroll
                 for (int u = 0; u < 8; u++) {
                     const float* q = pp + (size_t)(u < padd.nsplit ? u : 0) * padd.split_stride;
@@ -237,7 +258,7 @@ __global__ __launch_bounds__(256) void mix_norm_vec_kernel(bf16_t* __restrict__ 
     float ss = 0.f;
 #pragma unroll
     for (int it = 0; it < NV; it++) {
-        const int c = (threadIdx.x + it * 256) * 8;
+        const int c = (tid + it * 256) * 8;
         if (c < cols) {
             const uint32_t xw[4] = {xv[it].x, xv[it].y, xv[it].z, xv[it].w};
 #pragma unroll
@@ -261,7 +282,7 @@ __global__ __launch_bounds__(256) void mix_norm_vec_kernel(bf16_t* __restrict__ 
                     }
                 }
                 // splits beyond the first eight: again eight at a time, loads first
-                const float* pp = padd.parts + (size_t)blockIdx.x * padd.ld + c;
+                const float* pp = padd.parts + (size_t)row * padd.ld + c;
                 for (int sp0 = 8; sp0 < padd.nsplit; sp0 += 8) {
                     float4 b0[8], b1[8];
 #pragma unroll
@@ -298,32 +319,73 @@ __global__ __launch_bounds__(256) void mix_norm_vec_kernel(bf16_t* __restrict__ 
                     v[it][2 * j + 1] = rbf(v[it][2 * j + 1] - rbf(bl * bf16_hi(zw[j])));
                 }
             }
-            if (writes_x)
+            if (writes_x && !Q8)
                 *(uint4*)(x + base + c) = make_uint4(pack_bf16(v[it][0], v[it][1]), pack_bf16(v[it][2], v[it][3]),
                                                      pack_bf16(v[it][4], v[it][5]), pack_bf16(v[it][6], v[it][7]));
 #pragma unroll
             for (int j = 0; j < 8; j++) ss += v[it][j] * v[it][j];
         }
     }
-    ss = block_sum<4>(ss, red);
-    const float rstd = 1.0f / sqrtf(ss / (float)cols + RMS_EPS);
+    if constexpr (ROWS > 1) {
+        ss = wave_sum(ss);
+        if ((tid & 63) == 0) red[4 * in_wg + (tid >> 6)] = ss;
+        __syncthreads();
+        ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) ss += red[4 * in_wg + i];
+    } else {
+        ss = block_sum<4>(ss, red);
+    }
+    const float rstd = 1.0f / sqrtf(ss / (float)all_cols + RMS_EPS);
     float am = 0.f;
+    uint4 o[NV];
 #pragma unroll
     for (int it = 0; it < NV; it++) {
-        const int c = (threadIdx.x + it * 256) * 8;
+        const int c = (tid + it * 256) * 8;
         if (c < cols) {
-            uint32_t o[4];
+            uint32_t w[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                o[j] = pack_bf16(v[it][2 * j] * rstd, v[it][2 * j + 1] * rstd);
-                am = amax_fold(amax_fold(am, bf16_lo(o[j])), bf16_hi(o[j]));
+                w[j] = pack_bf16(v[it][2 * j] * rstd, v[it][2 * j + 1] * rstd);
+                am = amax_fold(amax_fold(am, bf16_lo(w[j])), bf16_hi(w[j]));
             }
-            *(uint4*)(xn_out + base + c) = make_uint4(o[0], o[1], o[2], o[3]);
+            o[it] = make_uint4(w[0], w[1], w[2], w[3]);
+            if (!Q8) *(uint4*)(xn_out + base + c) = o[it];
         }
+    }
+    if constexpr (Q8) {
+        float amax;
+        bool left;
+        auto each = [&](auto f) {
+#pragma unroll
+            for (int it = 0; it < NV; it++) {
+                const int c = (tid + it * 256) * 8;
+                if (c < cols) f(base + c, o[it]);
+            }
+        };
+        auto meanwhile = [&] {
+#pragma unroll
+            for (int it = 0; it < NV; it++) {
+                const int c = (tid + it * 256) * 8;
+                if (c >= cols) continue;
+                if (writes_x)
+                    *(uint4*)(x + base + c) = make_uint4(pack_bf16(v[it][0], v[it][1]), pack_bf16(v[it][2], v[it][3]),
+                                                         pack_bf16(v[it][4], v[it][5]), pack_bf16(v[it][6], v[it][7]));
+                if (c < 16) *(uint4*)(xn_out + base + c) = o[it];
+            }
+        };
+        const bool here = meeting<4 * ROWS, 4>(q8.meeting, gridDim.x, blockIdx.x, am, amax, left, meanwhile,
+                                                          [&] { each([&](size_t at, const uint4& w) { *(uint4*)(xn_out + at) = w; }); });
+        if (!here) return;
+        const float scale = scale_from_amax(amax);
+        if (blockIdx.x == 0 && threadIdx.x == 0) meeting_result(amax, scale, q8.inv_out, amax_ws);
+        each([&](size_t at, const uint4& w) { *(uint2*)(q8.out + at) = make_uint2(e4m3_of_bf16x4(w.x, w.y, scale), e4m3_of_bf16x4(w.z, w.w, scale)); });
+        if (left) meeting_take(q8.meeting, gridDim.x, [&](int wg) { convert_left_rows(q8, xn_out, wg, ROWS, q8.rows, all_cols, amax, scale, amax_ws); });
+        return;
     }
     block_amax_commit(am, amax_ws, red);
     // the row's cache position, advanced here when this is the last kernel of a decode step that reads no positions any more
-    if (bump && threadIdx.x == 0) bump[blockIdx.x] += bump_by;
+    if (bump && threadIdx.x == 0) bump[row] += bump_by;
 }
 
 // The same rows for the many of a prompt, a wave to a row.  What bounds a thousand workgroups that each end with a maximum for the amax site is
@@ -331,17 +393,19 @@ __global__ __launch_bounds__(256) void mix_norm_vec_kernel(bf16_t* __restrict__ 
 // the rescale (1792 rows of 1664 columns with an amax site: 10.0 -> 8.5 us, and 12.2 -> 9.8 between a prompt's other kernels; 8 or 16 rows to a
 // workgroup: 9.3 and 10.9).  The lane holds the elements that threads lane, lane + 64, lane + 128 and lane + 192 of the kernel above hold and
 // sums them in that order: the same bits.
-__global__ __launch_bounds__(256) void mix_norm_rows_kernel(bf16_t* __restrict__ x, const bf16_t* __restrict__ add, const bf16_t* __restrict__ x0,
+template <bool Q8, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void mix_norm_rows_kernel(bf16_t* __restrict__ x, const bf16_t* __restrict__ add, const bf16_t* __restrict__ x0,
                                                             const float* __restrict__ resid_lambda, const float* __restrict__ x0_lambda,
                                                             const float* __restrict__ backout_lambda, const bf16_t* __restrict__ backout_src,
                                                             bf16_t* __restrict__ backout_save, bf16_t* __restrict__ xn_out, int rows, int cols,
-                                                            uint32_t* __restrict__ amax_ws, int32_t* __restrict__ bump, int bump_by) {
+                                                            uint32_t* __restrict__ amax_ws, int32_t* __restrict__ bump, int bump_by, NcQuantRows q8) {
     __shared__ float red[4];
-    const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    float am = 0.f;
+    const int row = blockIdx.x * WAVES + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const size_t base = (size_t)row * cols;
+    const bool writes_x = add || resid_lambda || backout_lambda;
+    float am = 0.f, v[4][8];
+    uint4 o[4];
     if (row < rows) {
-        const size_t base = (size_t)row * cols;
-        const bool writes_x = add || resid_lambda || backout_lambda;
         const bf16_t* zsrc = resid_lambda ? x0 : (backout_lambda ? backout_src : nullptr);
         const float rl = rbf(resid_lambda ? *resid_lambda : 0.f), xl = rbf(x0_lambda ? *x0_lambda : 0.f), bl = rbf(backout_lambda ? *backout_lambda : 0.f);
         uint4 xv[4], av[4], zv[4];
@@ -354,7 +418,7 @@ __global__ __launch_bounds__(256) void mix_norm_rows_kernel(bf16_t* __restrict__
                 if (zsrc) zv[w] = *(const uint4*)(zsrc + base + c);
             }
         }
-        float v[4][8], ss[4] = {0.f, 0.f, 0.f, 0.f};
+        float ss[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < 4; w++) {
             const int c = (w * 64 + lane) * 8;
@@ -387,7 +451,7 @@ __global__ __launch_bounds__(256) void mix_norm_rows_kernel(bf16_t* __restrict__
                         v[w][2 * j + 1] = rbf(v[w][2 * j + 1] - rbf(bl * bf16_hi(zw[j])));
                     }
                 }
-                if (writes_x)
+                if (writes_x && !Q8)
                     *(uint4*)(x + base + c) = make_uint4(pack_bf16(v[w][0], v[w][1]), pack_bf16(v[w][2], v[w][3]),
                                                          pack_bf16(v[w][4], v[w][5]), pack_bf16(v[w][6], v[w][7]));
 #pragma unroll
@@ -402,18 +466,49 @@ __global__ __launch_bounds__(256) void mix_norm_rows_kernel(bf16_t* __restrict__
         for (int w = 0; w < 4; w++) {
             const int c = (w * 64 + lane) * 8;
             if (c < cols) {
-                uint32_t o[4];
+                uint32_t ow[4];
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    o[j] = pack_bf16(v[w][2 * j] * rstd, v[w][2 * j + 1] * rstd);
-                    am = amax_fold(amax_fold(am, bf16_lo(o[j])), bf16_hi(o[j]));
+                    ow[j] = pack_bf16(v[w][2 * j] * rstd, v[w][2 * j + 1] * rstd);
+                    am = amax_fold(amax_fold(am, bf16_lo(ow[j])), bf16_hi(ow[j]));
                 }
-                *(uint4*)(xn_out + base + c) = make_uint4(o[0], o[1], o[2], o[3]);
+                o[w] = make_uint4(ow[0], ow[1], ow[2], ow[3]);
+                if (!Q8) *(uint4*)(xn_out + base + c) = o[w];
             }
         }
-        if (bump && lane == 0) bump[row] += bump_by;
+        if (!Q8 && bump && lane == 0) bump[row] += bump_by;
     }
-    block_amax_commit(am, amax_ws, red);
+    if constexpr (Q8) {
+        float amax;
+        bool left;
+        auto each = [&](auto f) {
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                const int c = (w * 64 + lane) * 8;
+                if (row < rows && c < cols) f(base + c, o[w]);
+            }
+        };
+        auto meanwhile = [&] {
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                const int c = (w * 64 + lane) * 8;
+                if (row >= rows || c >= cols) continue;
+                if (writes_x)
+                    *(uint4*)(x + base + c) = make_uint4(pack_bf16(v[w][0], v[w][1]), pack_bf16(v[w][2], v[w][3]),
+                                                         pack_bf16(v[w][4], v[w][5]), pack_bf16(v[w][6], v[w][7]));
+                if (c < 16) *(uint4*)(xn_out + base + c) = o[w];
+            }
+        };
+        const bool here = meeting<WAVES, 4>(q8.meeting, gridDim.x, blockIdx.x, am, amax, left, meanwhile,
+                                                              [&] { each([&](size_t at, const uint4& w) { *(uint4*)(xn_out + at) = w; }); });
+        if (!here) return;
+        const float scale = scale_from_amax(amax);
+        if (blockIdx.x == 0 && threadIdx.x == 0) meeting_result(amax, scale, q8.inv_out, amax_ws);
+        each([&](size_t at, const uint4& w) { *(uint2*)(q8.out + at) = make_uint2(e4m3_of_bf16x4(w.x, w.y, scale), e4m3_of_bf16x4(w.z, w.w, scale)); });
+        if (left) meeting_take(q8.meeting, gridDim.x, [&](int wg) { convert_left_rows(q8, xn_out, wg, WAVES, rows, cols, amax, scale, amax_ws); });
+    } else {
+        block_amax_commit(am, amax_ws, red);
+    }
 }
 
 // out = relu(h)^2, elementwise bf16, plus amax (gpt.py:139)
@@ -632,9 +727,16 @@ int nc_launch_embed_norm_smear(const int64_t* idx, const bf16_t* wte, const floa
 // line lies higher for wider rows (256 columns: 512 rows 4.5 -> 3.7 us; 1664: 1024 rows 6.7 against 7.2, 1792 rows 10.0 -> 8.5).
 bool nc_mix_norm_wave_rows(int rows, int cols) { return cols % 8 == 0 && cols <= 2048 && rows >= 512 + 256 * ((cols + 511) / 512); }
 
+// Rows as e4m3: a workgroup of 512 threads holds eight rows, a wave to a row, or, where the addend comes as partial sums, 256 threads to a row, one, two or
+// four rows.  At most one workgroup to a CU, and no more than 256 of them (nc_meeting.h).
+#define ROWS_Q8 8
+static int mix_norm_e4m3_wgs() { return nc_cu_count() < 256 ? nc_cu_count() : 256; }
+bool nc_mix_norm_e4m3_fits(int rows, int cols, bool parts) { return cols % 16 == 0 && cols <= 2048 && rows <= (parts ? 4 : ROWS_Q8) * mix_norm_e4m3_wgs(); }
+
 static int launch_mix_norm_impl(bf16_t* x, const bf16_t* add, NcPartialSrc padd, const bf16_t* x0, const float* resid_lambda,
                                 const float* x0_lambda, const float* backout_lambda, const bf16_t* backout_src, bf16_t* backout_save,
-                                bf16_t* xn_out, int rows, int cols, uint32_t* amax_ws, hipStream_t s, int32_t* bump, int bump_by) {
+                                bf16_t* xn_out, int rows, int cols, uint32_t* amax_ws, hipStream_t s, int32_t* bump, int bump_by,
+                                const NcQuantRows* q8 = nullptr) {
     NC_CHECK_ARG(x && xn_out, "mix_norm: null pointer");
     NC_CHECK_ARG(row_args_ok(rows, cols), "mix_norm: bad shape rows=%d cols=%d", rows, cols);
     NC_CHECK_ARG(!resid_lambda || (x0 && x0_lambda), "mix_norm: the residual mix needs x0 and x0_lambda");
@@ -646,16 +748,36 @@ static int launch_mix_norm_impl(bf16_t* x, const bf16_t* add, NcPartialSrc padd,
     const bool aligned = cols % 8 == 0 && (((uintptr_t)x | (uintptr_t)xn_out | (uintptr_t)add | (uintptr_t)x0 | (uintptr_t)backout_src |
                                             (uintptr_t)backout_save | (uintptr_t)padd.parts) & 15) == 0 && padd.ld % 4 == 0 &&
                          padd.split_stride % 4 == 0;
-#define MIX_ARGS x, add, padd, x0, resid_lambda, x0_lambda, backout_lambda, backout_src, backout_save, xn_out, cols, amax_ws, bump, bump_by
+#define MIX_ARGS x, add, padd, x0, resid_lambda, x0_lambda, backout_lambda, backout_src, backout_save, xn_out, cols, amax_ws, bump, bump_by, NcQuantRows{}
 #define MIX_LAUNCH(NVV)                                                                                                  \
     do {                                                                                                                 \
         if (padd.parts) hipLaunchKernelGGL((mix_norm_vec_kernel<NVV, true>), dim3(rows), dim3(256), 0, s, MIX_ARGS);      \
         else hipLaunchKernelGGL((mix_norm_vec_kernel<NVV, false>), dim3(rows), dim3(256), 0, s, MIX_ARGS);                \
     } while (0)
+    if (q8) {
+        const int wgs = mix_norm_e4m3_wgs();
+        NC_CHECK_ARG(aligned && !bump && ((uintptr_t)q8->out & 7) == 0 && q8->inv_out && q8->meeting.words && nc_mix_norm_e4m3_fits(rows, cols, padd.parts != nullptr),
+                     "mix_norm: rows=%d cols=%d cannot be written as e4m3", rows, cols);
+        NcQuantRows q = *q8;
+        q.rows = rows;
+#define MIX_Q8_PARTS(R)                                                                                                                                      \
+    hipLaunchKernelGGL((mix_norm_vec_kernel<1, true, R>), dim3((rows + R - 1) / R), dim3(256 * R), 0, s, x, add, padd, x0, resid_lambda, x0_lambda, backout_lambda, \
+                       backout_src, backout_save, xn_out, cols, amax_ws, bump, bump_by, q)
+        if (padd.parts) {
+            if (rows <= wgs) MIX_Q8_PARTS(1);
+            else if (rows <= 2 * wgs) MIX_Q8_PARTS(2);
+            else MIX_Q8_PARTS(4);
+        } else
+#undef MIX_Q8_PARTS
+            hipLaunchKernelGGL((mix_norm_rows_kernel<true, ROWS_Q8>), dim3((rows + ROWS_Q8 - 1) / ROWS_Q8), dim3(64 * ROWS_Q8), 0, s, x, add, x0, resid_lambda, x0_lambda, backout_lambda, backout_src,
+                               backout_save, xn_out, rows, cols, amax_ws, bump, bump_by, q);
+        NC_CHECK_LAUNCH("mix_norm_e4m3");
+        return 0;
+    }
     // (without a site a workgroup per row is the faster one at any count: 1664 columns, 8192 rows 22.5 us against 25.5)
     if (aligned && !padd.parts && amax_ws && nc_mix_norm_wave_rows(rows, cols))
-        hipLaunchKernelGGL(mix_norm_rows_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, x, add, x0, resid_lambda, x0_lambda, backout_lambda,
-                           backout_src, backout_save, xn_out, rows, cols, amax_ws, bump, bump_by);
+        hipLaunchKernelGGL((mix_norm_rows_kernel<false, 4>), dim3((rows + 3) / 4), dim3(256), 0, s, x, add, x0, resid_lambda, x0_lambda, backout_lambda,
+                           backout_src, backout_save, xn_out, rows, cols, amax_ws, bump, bump_by, NcQuantRows{});
     else if (aligned && cols <= 2048) MIX_LAUNCH(1);
     else if (aligned && cols <= 4096) MIX_LAUNCH(2);
     else if (aligned && cols <= 8192) MIX_LAUNCH(4);
@@ -672,18 +794,18 @@ static int launch_mix_norm_impl(bf16_t* x, const bf16_t* add, NcPartialSrc padd,
 
 int nc_launch_mix_norm(bf16_t* x, const bf16_t* add, const bf16_t* x0, const float* resid_lambda, const float* x0_lambda,
                        const float* backout_lambda, const bf16_t* backout_src, bf16_t* backout_save, bf16_t* xn_out,
-                       int rows, int cols, uint32_t* amax_ws, hipStream_t s, int32_t* bump, int bump_by) {
+                       int rows, int cols, uint32_t* amax_ws, hipStream_t s, int32_t* bump, int bump_by, const NcQuantRows* q8) {
     NcPartialSrc none{nullptr, 0, 0, 0, nullptr, nullptr, 0, 0};
     return launch_mix_norm_impl(x, add, none, x0, resid_lambda, x0_lambda, backout_lambda, backout_src, backout_save, xn_out, rows,
-                                cols, amax_ws, s, bump, bump_by);
+                                cols, amax_ws, s, bump, bump_by, q8);
 }
 
 int nc_launch_mix_norm_p(bf16_t* x, NcPartialSrc add, const bf16_t* x0, const float* resid_lambda, const float* x0_lambda,
                          const float* backout_lambda, const bf16_t* backout_src, bf16_t* backout_save, bf16_t* xn_out,
-                         int rows, int cols, uint32_t* amax_ws, hipStream_t s, int32_t* bump, int bump_by) {
+                         int rows, int cols, uint32_t* amax_ws, hipStream_t s, int32_t* bump, int bump_by, const NcQuantRows* q8) {
     NC_CHECK_ARG(!add.parts || (add.nsplit >= 1 && add.a_amax && add.inv_b && add.ld >= cols), "mix_norm: bad partial-sum source");
     return launch_mix_norm_impl(x, nullptr, add, x0, resid_lambda, x0_lambda, backout_lambda, backout_src, backout_save, xn_out, rows,
-                                cols, amax_ws, s, bump, bump_by);
+                                cols, amax_ws, s, bump, bump_by, q8);
 }
 
 int nc_launch_relu2(const bf16_t* h, bf16_t* out, int64_t n, uint32_t* amax_ws, hipStream_t s) {

@@ -194,10 +194,10 @@ struct LinearRunner {
         return 0;
     }
     // relu^2 of a linear of many rows as e4m3 at w.h, its inverse scale in w.inv + out_site; false: not a shape of that launch
-    bool run_relu2_e4m3(const bf16_t* in, int rows, int site, const uint8_t* w8, const float* inv_w, int N, int K, int out_site, const uint8_t** out8, int* rc) const {
+    bool run_relu2_e4m3(const bf16_t* in, const uint8_t* in8, int rows, int site, const uint8_t* w8, const float* inv_w, int N, int K, int out_site, const uint8_t** out8, int* rc) const {
         *out8 = nullptr;
         if (rows <= 128 || !nc_gemm_relu2_e4m3_kernel(rows, N, K)) return false;
-        *rc = nc_launch_convert_only(in, (int64_t)rows * K, w.a8, w.inv + site, w.site(site), s);
+        *rc = in8 ? 0 : nc_launch_convert_only(in, (int64_t)rows * K, w.a8, w.inv + site, w.site(site), s);
         if (!*rc) *rc = nc_launch_gemm_relu2_e4m3(w.a8, w8, w.inv + site, inv_w, (uint8_t*)w.h, w.inv + out_site, w.site(out_site), w.h2,
                                                    w.meeting(out_site), rows, N, K, s);
         *out8 = (const uint8_t*)w.h;
@@ -275,11 +275,16 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
     // output of the previous MLP projection, still to be added into the residual stream: bf16 rows or split partials
     const bf16_t* pending_add = nullptr;
     NcPartialSrc pending_parts = NO_PARTIALS;
+    // rows8: whether the pass left its rows as e4m3 in w.a8, their inverse scale in w.inv (a prompt's layers; the last rows are gathered first)
+    const uint8_t* rows8 = nullptr;
     auto mix = [&](const float* rl, const float* xl, const float* bl, const bf16_t* bsrc, bf16_t* save, uint32_t* amax,
-                   int32_t* bump = nullptr, int bump_by = 0) -> int {
+                   int32_t* bump = nullptr, int bump_by = 0, bool to_e4m3 = false) -> int {
+        const NcQuantRows q8{w.a8, w.inv + site, to_e4m3 ? w.meeting(site) : NcMeeting{}, M};
+        const NcQuantRows* const q = to_e4m3 && M > 128 && nc_mix_norm_e4m3_fits(M, E, pending_parts.parts != nullptr) ? &q8 : nullptr;
+        rows8 = q ? w.a8 : nullptr;
         if (pending_parts.parts)
-            return nc_launch_mix_norm_p(w.x, pending_parts, w.x0, rl, xl, bl, bsrc, save, w.xn, M, E, amax, s, bump, bump_by);
-        return nc_launch_mix_norm(w.x, pending_add, w.x0, rl, xl, bl, bsrc, save, w.xn, M, E, amax, s, bump, bump_by);
+            return nc_launch_mix_norm_p(w.x, pending_parts, w.x0, rl, xl, bl, bsrc, save, w.xn, M, E, amax, s, bump, bump_by, q);
+        return nc_launch_mix_norm(w.x, pending_add, w.x0, rl, xl, bl, bsrc, save, w.xn, M, E, amax, s, bump, bump_by, q);
     };
     // (measured at d26, steps without a synchronisation in between: one row 1.30 -> 1.13 ms, two rows 1.37 -> 1.27 ms)
     const bool fused = T == 1 && fused_rows(m, M);
@@ -337,12 +342,12 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
         NC_CHECK_ARG(ly.w_qkv && ly.inv_qkv && ly.w_attn_proj && ly.w_fc && ly.w_mlp_proj, "gpt_forward: layer %d has no FP8 weights", i);
         // x += mlp_out(prev layer); [save backout]; x = rl*x + xl*x0; xn = norm(x)
         bf16_t* save = (i > 0 && (i - 1) == L / 2) ? w.xb : nullptr;
-        TRY(mix(m->resid_lambdas + i, m->x0_lambdas + i, nullptr, nullptr, save, w.site(site)));
+        TRY(mix(m->resid_lambdas + i, m->x0_lambdas + i, nullptr, nullptr, save, w.site(site), nullptr, 0, true));
         if (tap_x) TRY(tap_copy(tap_x + (size_t)i * M * E, w.x, (size_t)M * E, s));
         // q|k|v = FP8 linear(xn): one activation quantization, three weight scales
         NcGemmSegs qkv_segs{3, {H * 128, (H + Hkv) * 128, qkv_w, 0}};
         NcPartialSrc qsrc;
-        TRY(lin.run(w.xn, M, site, ly.w_qkv, ly.inv_qkv, qkv_segs, w.qkv, 0, 0.f, nullptr, qkv_w, E, qkv_w, &qsrc));
+        TRY(lin.run(w.xn, M, site, ly.w_qkv, ly.inv_qkv, qkv_segs, w.qkv, 0, 0.f, nullptr, qkv_w, E, qkv_w, &qsrc, nullptr, rows8));
         site++;
         bf16_t* kc = kv->k_cache + (size_t)i * layer_elems;
         bf16_t* vc = kv->v_cache + (size_t)i * layer_elems;
@@ -386,12 +391,12 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
         pending_add = pending_parts.parts ? nullptr : w.o;
         site++;
         // x += attn_out; xn = norm(x)
-        TRY(mix(nullptr, nullptr, nullptr, nullptr, nullptr, w.site(site)));
+        TRY(mix(nullptr, nullptr, nullptr, nullptr, nullptr, w.site(site), nullptr, 0, true));
         // h2 = relu(c_fc(xn))^2 with its amax in the next slot, or as e4m3
         const uint8_t* h8;
         int rc = 0;
-        if (!lin.run_relu2_e4m3(w.xn, M, site, ly.w_fc, ly.inv_fc, 4 * E, E, site + 1, &h8, &rc))
-            rc = lin.run(w.xn, M, site, ly.w_fc, ly.inv_fc, one_seg(4 * E), w.h2, 2, 0.f, w.site(site + 1), 4 * E, E, 4 * E, nullptr);
+        if (!lin.run_relu2_e4m3(w.xn, rows8, M, site, ly.w_fc, ly.inv_fc, 4 * E, E, site + 1, &h8, &rc))
+            rc = lin.run(w.xn, M, site, ly.w_fc, ly.inv_fc, one_seg(4 * E), w.h2, 2, 0.f, w.site(site + 1), 4 * E, E, 4 * E, nullptr, nullptr, rows8);
         if (rc) return rc;
         site++;
         TRY(lin.run(w.h2, M, site, ly.w_mlp_proj, ly.inv_mlp_proj, one_seg(E), w.o, 0, 0.f, nullptr, E, 4 * E, E, &pending_parts, nullptr, h8));

@@ -346,7 +346,7 @@ __device__ __forceinline__ void q8_epilogue(v4f (&acc)[BM / WGM / 16][BN / WGN /
     }
     float amax;
     bool left;
-    const bool here = meeting<WGM * WGN, 4>(ep.meeting, gridDim.x, blockIdx.x, am, amax, left, [&] {
+    const bool here = meeting<WGM * WGN, 4>(ep.meeting, gridDim.x, blockIdx.x, am, amax, left, [] {}, [&] {
 #pragma unroll
         for (int j = 0; j < WTN; j++)
 #pragma unroll

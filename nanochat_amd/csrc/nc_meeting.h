@@ -3,7 +3,8 @@
 //
 // Memory (NC_MEETING_WORDS words, all zero before the launch): one word per workgroup, its maximum with the top bit set once it has arrived, and
 // behind them one bit per workgroup that left (below).  One trip to memory out, one back: every workgroup stores its word and polls everybody's, so
-// there is no counter for hundreds of atomics to queue up at (2.5 us between the last arrival and the maximum's being known everywhere).  Words and
+// there is no counter for hundreds of atomics to queue up at.  What the polls cost grows with the square of the workgroups, all of them reading the same
+// lines (row passes of 1792 rows: 112 workgroups 12.1 us, 224 10.7, 448 13.7), so few large workgroups meet best, and none beyond 256 but for attention's.  Words and
 // bits are read and written with device-scope atomics, at the device's point of coherence; no fence is needed on the way everybody takes.
 //
 // The launch is sized so that the chip holds all of it, but a workgroup may still not have started because another stream's kernel has its place.
@@ -15,13 +16,21 @@
 #pragma once
 #include "nc_common.h"
 
-#define NC_MEETING_WGS 1024
+#define NC_MEETING_WGS 512
 #define NC_MEETING_WORDS (NC_MEETING_WGS + NC_MEETING_WGS / 32)
 #define NC_MEETING_SPINS 400u             // polls of about half a microsecond before a workgroup leaves
 
 struct NcMeeting {
     uint32_t* words;          // nullptr: none
     uint32_t spins;
+};
+
+// rows that a kernel writes as e4m3 after a meeting
+struct NcQuantRows {
+    uint8_t* out;             // [rows][cols]
+    float* inv_out;
+    NcMeeting meeting;
+    int rows;
 };
 
 struct MeetingView {
@@ -50,11 +59,7 @@ __device__ __forceinline__ MeetingView meeting_look(const NcMeeting& m, int wgs)
     return MeetingView{__builtin_amdgcn_ballot_w64(all == 0u) == 0, mx, __builtin_amdgcn_ballot_w64(bits != 0u) != 0};
 }
 template <int POLLS>
-__device__ __forceinline__ MeetingView meeting_wait(const NcMeeting& m, int wgs, int self, uint32_t mine) {
-    if ((threadIdx.x & 63) == 0) __hip_atomic_store(m.words + self, mine | 0x80000000u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0);            // the word is there before anything is looked at
-    asm volatile("" ::: "memory");
+__device__ __forceinline__ MeetingView meeting_wait(const NcMeeting& m, int wgs) {
     for (uint32_t spin = 0;; spin++) {
         MeetingView view = meeting_look<POLLS>(m, wgs);
         if (view.complete || spin >= m.spins) {
@@ -65,21 +70,28 @@ __device__ __forceinline__ MeetingView meeting_wait(const NcMeeting& m, int wgs,
     }
 }
 
-// The whole meeting, for every thread of a workgroup of WAVES waves; am: each thread's maximum.  leave() stores the workgroup's values as bf16.
+// The whole meeting, for every thread of a workgroup of WAVES waves; am: each thread's maximum.  meanwhile(): what can be stored while the words travel;
+// leave() stores the workgroup's values as bf16.
 // Returns false when the workgroup left (its values are in memory and somebody else's business), else true with the tensor's amax and whether
 // meeting_take has to be called once the workgroup's own values are converted.
-template <int WAVES, int POLLS, typename Leave>
-__device__ __forceinline__ bool meeting(const NcMeeting& m, int wgs, int self, float am, float& amax, bool& left, Leave&& leave) {
+template <int WAVES, int POLLS, typename Meanwhile, typename Leave>
+__device__ __forceinline__ bool meeting(const NcMeeting& m, int wgs, int self, float am, float& amax, bool& left, Meanwhile&& meanwhile, Leave&& leave) {
     __shared__ uint32_t red[WAVES], out[3];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     am = wave_amax(am);
     if (lane == 0) red[wave] = __float_as_uint(am);
     __syncthreads();
-    if (wave == 0) {
+    uint32_t before = 0u;
+    if (threadIdx.x == 0) {
         uint32_t t = red[0];
 #pragma unroll
         for (int w = 1; w < WAVES; w++) t = red[w] > t ? red[w] : t;
-        const MeetingView view = meeting_wait<POLLS>(m, wgs, self, t);
+        before = __hip_atomic_exchange(m.words + self, t | 0x80000000u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    meanwhile();
+    if (wave == 0) {
+        asm volatile("" ::"v"(before) : "memory");       // the word is there (the exchange has returned) before anything is looked at
+        const MeetingView view = meeting_wait<POLLS>(m, wgs);
         if (lane == 0) out[0] = view.complete, out[1] = view.amax, out[2] = view.left;
     }
     __syncthreads();

@@ -322,6 +322,20 @@ def mix_norm(x, add=None, x0=None, resid_lambda=None, x0_lambda=None, backout_la
     return xn, saved
 
 
+def mix_norm_e4m3(x, add=None, parts=None, parts_amax=None, parts_inv=None, x0=None, resid_lambda=None, x0_lambda=None, spin_limit=-1):
+    """mix_norm (without backout) and fp8_quantize of its rows in one launch, the same bits: (e4m3 rows, inverse scale fp32 0-dim).  The addend as bf16
+    or as fp32 partial sums `parts` [splits, rows, cols] of an FP8 linear (parts_amax: its input's amax bits, parts_inv: its weight's inverse scale)."""
+    _need_cuda(x, add, parts)
+    assert x.is_contiguous() and x.dtype == torch.bfloat16
+    cols = x.shape[-1]
+    rows = x.numel() // cols
+    out, xn = torch.empty(x.shape, dtype=torch.float8_e4m3fn, device=x.device), torch.empty_like(x)
+    inv, meeting = torch.empty((), dtype=torch.float32, device=x.device), _meeting(x.device)
+    _lib.check(_lib.lib().nc_mix_norm_e4m3(_ptr(x), _ptr(add), _ptr(parts), parts.shape[0] if parts is not None else 0, _ptr(parts_amax), _ptr(parts_inv), _ptr(x0),
+                                           _ptr(resid_lambda), _ptr(x0_lambda), _ptr(xn), _ptr(out), _ptr(inv), _ptr(meeting), rows, cols, spin_limit, _stream()))
+    return out, inv
+
+
 def qkv_rope_append(qkv, xn, idx, ve_table, ve_gate_w, cos, sin, cache_seqlens, k_cache, v_cache, n_head, n_kv_head):
     """Rotary + QK-norm + gain on q,k; value-embedding gate on v; append k,v at cache_seqlens.. (in place).
     qkv [B,T,(H+2Hkv)*128] bf16.  Returns q [B,T,H,128]."""

@@ -861,6 +861,33 @@ def test_relu2(ops):
     assert torch.equal(ops.relu2(h.to(DEV)).cpu(), F.relu(h).square())
 
 
+@pytest.mark.parametrize("spin_limit", [-1, 0])
+@pytest.mark.parametrize("rows,cols,splits", [(1792, 1664, 0), (129, 256, 0), (333, 1040, 0), (1023, 512, 0), (2048, 2048, 0), (130, 1024, 8), (257, 1280, 2), (511, 2032, 4), (1023, 512, 2), (1024, 2048, 3), (257, 16, 9)])
+def test_mix_norm_written_as_e4m3(ops, rows, cols, splits, spin_limit):
+    """The row pass with its workgroups meeting on the amax: the bits of the bf16 pass quantized by a launch of its own, and the same residual stream."""
+    say(f"mix_norm e4m3 rows={rows} cols={cols} splits={splits} spins={spin_limit}")
+    g = torch.Generator(device=DEV).manual_seed(rows + cols)
+    x, x0, add = (torch.randn(rows, cols, generator=g, device=DEV).bfloat16() for _ in range(3))
+    rl, xl = torch.tensor([0.9], device=DEV), torch.tensor([0.3], device=DEV)
+    how = dict(add=add)
+    if splits:
+        parts = torch.randn(splits, rows, cols, generator=g, device=DEV)
+        amax, inv_b = torch.tensor([3.0], device=DEV), torch.tensor([0.01], device=DEV)
+        total = torch.zeros_like(parts[0])
+        for p in parts:
+            total = total + p
+        add = ((total * (1.0 / (448.0 / amax.double()).float())) * inv_b).bfloat16()
+        how = dict(parts=parts, parts_amax=amax.view(torch.int32), parts_inv=inv_b)
+    for mixed in (False, True):
+        mix = dict(x0=x0, resid_lambda=rl, x0_lambda=xl) if mixed else {}
+        want_x = x.clone()
+        xn, _ = ops.mix_norm(want_x, add, **mix)
+        want, want_inv, _ = ops.fp8_quantize(xn)
+        got_x = x.clone()
+        got, inv = ops.mix_norm_e4m3(got_x, **how, **mix, spin_limit=spin_limit)
+        assert torch.equal(got_x, want_x) and inv.item() == want_inv.item() and torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+
+
 def test_mix_norm_variants(ops):
     say("mix_norm")
     g = torch.Generator().manual_seed(0)
