@@ -919,16 +919,14 @@ __global__ __launch_bounds__(512) void gemm_dln_kernel(const uint8_t* __restrict
     else dln_epilogue<NJ, OUT_KIND == 2>(acc, lds, ep, inv_a, sc, g, m0, n0, M, N);
 }
 
-// the operand loads of one K-step of gemm_dr_kernel: `st` is the wave's first 1 KB piece of the stage, its pieces lie 4 KB apart
+// load r of the A_P + 4 operand loads of one K-step of gemm_dr_kernel: `st` is the wave's first 1 KB piece of the stage, its pieces lie 4 KB apart
 template <int A_P>
-__device__ __forceinline__ void dr_fetch(const uint8_t* A, int a_bytes, const uint8_t* B, int b_bytes, uint8_t* st, int b_part, const uint32_t* vo_a,
-                                         const uint32_t* vo_b, int k_off) {
+__device__ __forceinline__ void dr_load(const uint8_t* A, int a_bytes, const uint8_t* B, int b_bytes, uint8_t* st, int b_part, const uint32_t* vo_a,
+                                        const uint32_t* vo_b, int r, int k_off) {
     const __amdgpu_buffer_rsrc_t desc_a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, a_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t desc_b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, b_bytes, 0x00020000);
-#pragma unroll
-    for (int i = 0; i < A_P; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_a, (lds_ptr_t)(st + i * 4096), 16, vo_a[i], k_off, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 4; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_b, (lds_ptr_t)(st + b_part + i * 4096), 16, vo_b[i], k_off, 0, 0);
+    if (r < A_P) __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_a, (lds_ptr_t)(st + r * 4096), 16, vo_a[r], k_off, 0, 0);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_b, (lds_ptr_t)(st + b_part + (r - A_P) * 4096), 16, vo_b[r - A_P], k_off, 0, 0);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -946,8 +944,8 @@ template <int BM, int OUT_KIND>
 __global__ __launch_bounds__(256) void gemm_dr_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, EpilogueArgs ep, int M,
                                                       int N, int K, int tiles_m, int tiles_n) {
     constexpr int WTM = BM / 32, STAGE = (BM + 128) * 128, A_P = BM / 32, LOADS = A_P + 4;
-    // s_waitcnt vmcnt(2 * LOADS), other counters untouched: the loads of the two youngest steps may still be in flight
-    constexpr int WAIT2 = 0x0F70 | ((2 * LOADS) & 15) | (((2 * LOADS) >> 4) << 14);
+    // s_waitcnt vmcnt(n * LOADS) lgkmcnt(0): the loads of the n youngest steps may still be in flight, no LDS read
+    constexpr int WAIT2 = 0x0070 | ((2 * LOADS) & 15) | (((2 * LOADS) >> 4) << 14), WAIT3 = 0x0070 | ((3 * LOADS) & 15) | (((3 * LOADS) >> 4) << 14);
     extern __shared__ __align__(16) uint8_t lds[];
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
@@ -978,38 +976,65 @@ __global__ __launch_bounds__(256) void gemm_dr_kernel(const uint8_t* __restrict_
         for (int j = 0; j < 4; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
     auto fetch = [&](int t) {
-        dr_fetch<A_P>(A, M * K - k_first * 128, B, N * K - k_first * 128, lds + (t & 3) * STAGE + wave_s * 1024, BM * 128, vo_a, vo_b, t < ksteps ? t * 128 : 0);
+#pragma unroll
+        for (int r = 0; r < LOADS; r++)
+            dr_load<A_P>(A, M * K - k_first * 128, B, N * K - k_first * 128, lds + (t & 3) * STAGE + wave_s * 1024, BM * 128, vo_a, vo_b, r, t < ksteps ? t * 128 : 0);
     };
-    auto compute = [&](int t) {
-        const uint8_t* st = lds + (t & 3) * STAGE;
-        const uint8_t* a = st + g.wm * (BM / 2) * 128;
-        const uint8_t* b = st + BM * 128 + g.wn * 64 * 128;
-        v8i af[WTM], bf[2];
-        bf[0] = dl_frag(b, g);
+    // One step: its products, between them the reads of the next step's fragments (into other registers) and the loads of the step four ahead.  Neither
+    // the barrier nor an LDS read is waited for with the matrix cores idle: when the waves meet, every wave has read all of the stage of the step to be
+    // multiplied, so that stage is free for loads, and the next one has landed.
+    const int a_rd = g.wm * (BM / 2) * 128, b_rd = BM * 128 + g.wn * 64 * 128;
+    v8i fa[2][WTM], fb[2][4];
+    auto step = [&](int t, auto parity) __attribute__((always_inline)) {
+        constexpr int P = decltype(parity)::value, Q = 1 - P, READS = WTM + 4, PRODUCTS = 4 * WTM;
+        const uint8_t* const st = lds + ((t + 1) & 3) * STAGE;
+        const int k_off = t + 4 < ksteps ? (t + 4) * 128 : 0;
+        uint8_t* const to = lds + (t & 3) * STAGE + wave_s * 1024;
 #pragma unroll
-        for (int i = 0; i < WTM; i++) af[i] = dl_frag(a + i * 2048, g);
+        for (int j = 0; j < 4; j++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (j + 1 < 4) bf[(j + 1) & 1] = dl_frag(b + (j + 1) * 2048, g);
+            for (int i = 0; i < WTM; i++) {
+                const int n = j * WTM + i;
 #pragma unroll
-            for (int i = 0; i < WTM; i++) mfma_f8_acc_ordered<0>(acc[i][j], bf[j & 1], af[i]);
-        }
+                for (int r = 0; r < READS; r++)
+                    if (r * PRODUCTS / READS == n) {
+                        if (r == 0) fb[Q][0] = dl_frag(st + b_rd, g);
+                        else if (r <= WTM) fa[Q][r - 1] = dl_frag(st + a_rd + (r - 1) * 2048, g);
+                        else fb[Q][r - WTM] = dl_frag(st + b_rd + (r - WTM) * 2048, g);
+                    }
+#pragma unroll
+                for (int r = 0; r < LOADS; r++)
+                    if (r * PRODUCTS / LOADS == n) dr_load<A_P>(A, M * K - k_first * 128, B, N * K - k_first * 128, to, BM * 128, vo_a, vo_b, r, k_off);
+                mfma_f8_acc_ordered<0>(acc[i][j], fb[P][j], fa[P][i]);
+            }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(WAIT2);   // the operands of step t + 2 have landed, the fragments of step t + 1 are read (this wave's share; the barrier says everybody's)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
     };
     fetch(0);
     fetch(1);
     fetch(2);
+    fetch(3);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(WAIT3);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    fb[0][0] = dl_frag(lds + b_rd, g);
+#pragma unroll
+    for (int i = 0; i < WTM; i++) fa[0][i] = dl_frag(lds + a_rd + i * 2048, g);
+#pragma unroll
+    for (int j = 1; j < 4; j++) fb[0][j] = dl_frag(lds + b_rd + j * 2048, g);
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(WAIT2);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    for (int kt = 0; kt < ksteps; kt++) {
-        fetch(kt + 3);                       // into the stage that was read in step kt - 1: everyone is past the barrier that ended it
-        compute(kt);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(WAIT2);   // the operands of step kt + 1 have landed (this wave's share; the barrier says everybody's)
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+    int kt = 0;
+    for (; kt + 1 < ksteps; kt += 2) {
+        step(kt, std::integral_constant<int, 0>{});
+        step(kt + 1, std::integral_constant<int, 1>{});
     }
+    if (kt < ksteps) step(kt, std::integral_constant<int, 0>{});
     // the loads past the end of K are still landing in the stages: they must be done before the epilogue reuses the memory
     dl_step_barrier();
 
