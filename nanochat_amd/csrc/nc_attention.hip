@@ -493,11 +493,11 @@ static int launch_attention_impl(const bf16_t* q, const NcRopeSrc* rope, int mod
                                  const int32_t* cache_seqlens, int window_left, bf16_t* out, int B, int T, int H, int Hkv, int Tmax,
                                  int seqlens_include_new, uint32_t* counters, void* partials, size_t partial_bytes, uint32_t* amax_ws,
                                  int force_splits, int who_clears, hipStream_t s, int k_min = 0, const float* extra = nullptr,
-                                 int n_extra = 0) {
+                                 int n_extra = 0, const NcAhead* ahead = nullptr) {
     NC_CHECK_ARG((q || mode == 1) && k_cache && v_cache && cache_seqlens && out, "decode_attention: null pointer");
     if (mode == 0 && takes_prefill(T, force_splits))
         return nc_launch_attention_prefill(q, k_cache, v_cache, cache_seqlens, window_left, out, B, T, H, Hkv, Tmax, seqlens_include_new,
-                                           amax_ws, s);
+                                           amax_ws, s, ahead);
     int nsplit;
     if (const int rc = check_attention(window_left, B, T, H, Hkv, Tmax, counters, partials, partial_bytes, force_splits, who_clears, &nsplit)) return rc;
     const int G = H / Hkv, max_keys = visible_keys(window_left, Tmax);
@@ -570,10 +570,10 @@ void nc_attention_plan(int B, int T, int Hkv, int window_left, int Tmax, int for
 int nc_launch_attention(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache, const int32_t* cache_seqlens,
                         int window_left, bf16_t* out, int B, int T, int H, int Hkv, int Tmax, int seqlens_include_new,
                         uint32_t* counters, void* partials, size_t partial_bytes, uint32_t* amax_ws, int force_splits,
-                        int counters_of_pass, hipStream_t s) {
+                        int counters_of_pass, hipStream_t s, const NcAhead* ahead) {
     return launch_attention_impl(q, nullptr, 0, const_cast<bf16_t*>(k_cache), const_cast<bf16_t*>(v_cache), cache_seqlens, window_left, out,
                                  B, T, H, Hkv, Tmax, seqlens_include_new, counters, partials, partial_bytes, amax_ws, force_splits,
-                                 counters_of_pass ? COUNTERS_OF_PASS : COUNTERS_CLEAR, s);
+                                 counters_of_pass ? COUNTERS_OF_PASS : COUNTERS_CLEAR, s, 0, nullptr, 0, ahead);
 }
 
 // Decode step, one new token per row, cache_seqlens not yet counting it: finish the q|k|v linear (rotary, QK-norm,

@@ -16,6 +16,7 @@
 // next block are in flight while the current one is multiplied.
 #include "nc_common.h"
 #include "nc_kernels.h"
+#include "nc_prefetch.h"
 
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v16f __attribute__((ext_vector_type(16)));
@@ -69,8 +70,13 @@ template <int GS, int KS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
                                                            const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ cache_seqlens,
                                                            int window_left, int seqlens_include_new, bf16_t* __restrict__ out,
-                                                           uint32_t* __restrict__ amax_ws, int T, int H, int Hkv, int Tmax, PfUnitMap map) {
+                                                           uint32_t* __restrict__ amax_ws, int T, int H, int Hkv, int Tmax, PfUnitMap map, NcAhead ahead, int B) {
     constexpr int QT = 128 / (GS * KS);                        // queries per workgroup
+    if ((int)blockIdx.z >= B) {                                // (workgroups of no row: they come last)
+        const int wg = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * (blockIdx.z - B));
+        if (wg < NC_AHEAD_WGS) read_ahead<256>(ahead, wg, NC_AHEAD_WGS);
+        return;
+    }
     __shared__ __align__(16) uint8_t lds[2 * PF_KBYTES + 2 * PF_VBYTES];
     __shared__ float red[4];
     uint8_t* const lds_k = lds;
@@ -594,7 +600,7 @@ static void pf_balance_units(PfUnitMap& map, int nx, int ny, int cus) {
 
 int nc_launch_attention_prefill(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache, const int32_t* cache_seqlens,
                                 int window_left, bf16_t* out, int B, int T, int H, int Hkv, int Tmax, int seqlens_include_new,
-                                uint32_t* amax_ws, hipStream_t s) {
+                                uint32_t* amax_ws, hipStream_t s, const NcAhead* ahead) {
     NC_CHECK_ARG(q && k_cache && v_cache && cache_seqlens && out, "prefill_attention: null pointer");
     NC_CHECK_ARG(B > 0 && T > 0 && H > 0 && Hkv > 0 && Tmax > 0 && H % Hkv == 0, "prefill_attention: bad shape");
     NC_CHECK_ARG(B <= 65535 && H <= 65535, "prefill_attention: more than 65535 rows or heads in one launch");
@@ -608,7 +614,10 @@ int nc_launch_attention_prefill(const bf16_t* q, const bf16_t* k_cache, const bf
     const long long wgs1 = (long long)B * Hkv * (G / GS) * ((T + 128 / GS - 1) / (128 / GS));
     const int KS = (GS <= 2 && wgs1 < 2LL * nc_cu_count()) ? 2 : 1;
     const int QT = 128 / (GS * KS);
-    const dim3 grid((T + QT - 1) / QT, Hkv * (G / GS), B);
+    dim3 grid((T + QT - 1) / QT, Hkv * (G / GS), B);
+    const int slices = (NC_AHEAD_WGS + (int)(grid.x * grid.y) - 1) / (int)(grid.x * grid.y);
+    const bool reads_ahead = ahead && ahead->n > 0 && B + slices <= 65535;
+    if (reads_ahead) grid.z += slices;
     NC_CHECK_ARG(grid.y <= 65535, "prefill_attention: too many heads in one launch");
     PfUnitMap map;                         // passed by value
     map.on = 0;
@@ -616,7 +625,7 @@ int nc_launch_attention_prefill(const bf16_t* q, const bf16_t* k_cache, const bf
     if (B == 1 && (window_left < 0 || window_left >= Tmax)) pf_balance_units(map, (int)grid.x, (int)grid.y, nc_cu_count());
 #define PF_LAUNCH(GG, KK)                                                                                                              \
     hipLaunchKernelGGL((attn_prefill_kernel<GG, KK>), grid, dim3(256), 0, s, q, k_cache, v_cache, cache_seqlens, window_left,          \
-                       seqlens_include_new, out, amax_ws, T, H, Hkv, Tmax, map)
+                       seqlens_include_new, out, amax_ws, T, H, Hkv, Tmax, map, reads_ahead ? *ahead : NcAhead{}, B)
     if (GS == 4) PF_LAUNCH(4, 1);
     else if (GS == 2 && KS == 2) PF_LAUNCH(2, 2);
     else if (GS == 2) PF_LAUNCH(2, 1);

@@ -34,6 +34,7 @@
 #include "nc_common.h"
 #include "nc_kernels.h"
 #include "nc_meeting.h"
+#include "nc_prefetch.h"
 #include "nc_rope.h"
 
 #define TRY(call)              \
@@ -383,8 +384,15 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
             else
                 TRY(nc_launch_qkv_rope_append(w.qkv, qkv_w, w.xn, E, idx, ly.ve_table, ly.ve_gate_w, m->cos, m->sin, m->rope_len,
                                               kv->cache_seqlens, kc, vc, w.qh, B, T, H, Hkv, kv->max_seq_len, m->padded_vocab, s));
+            // meanwhile the weights of the linears up to the next attention come out of HBM
+            NcAhead ahead{};
+            ahead.add(ly.w_attn_proj, (size_t)E * H * 128);
+            ahead.add(ly.w_fc, (size_t)4 * E * E);
+            ahead.add(ly.w_mlp_proj, (size_t)4 * E * E);
+            if (i + 1 < L) ahead.add(m->layers[i + 1].w_qkv, (size_t)qkv_w * E);
+            else ahead.add(m->w_lm_head, (size_t)m->vocab_size * E);
             TRY(nc_launch_attention(w.qh, kc, vc, kv->cache_seqlens, ly.window_left, w.y, B, T, H, Hkv, kv->max_seq_len, 0,
-                                    w.attn_counters, w.attn_parts, w.attn_part_bytes, w.site(site), 0, 1, s));
+                                    w.attn_counters, w.attn_parts, w.attn_part_bytes, w.site(site), 0, 1, s, &ahead));
         }
         if (tap_y) TRY(tap_copy(tap_y + (size_t)i * M * H * 128, w.y, (size_t)M * H * 128, s));
         TRY(lin.run(w.y, M, site, ly.w_attn_proj, ly.inv_attn_proj, one_seg(E), w.o, 0, 0.f, nullptr, E, H * 128, E, &pending_parts));

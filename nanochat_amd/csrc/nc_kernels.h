@@ -123,19 +123,20 @@ int nc_launch_kv_prefill_copy(const void* src, void* dst, int layers, int src_ro
                               int n_tokens, int token_bytes, hipStream_t s);
 
 // ---- attention (nc_attention.hip)
+struct NcAhead;               // (nc_prefetch.h) weights that the many-queries kernel reads ahead for the linears behind it, or null
 size_t nc_attn_counter_bytes(int B, int T, int H);
 size_t nc_attn_partial_bytes(int B, int T, int H);
 int nc_launch_attention(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache, const int32_t* cache_seqlens,
                         int window_left, bf16_t* out, int B, int T, int H, int Hkv, int Tmax, int seqlens_include_new,
                         uint32_t* counters, void* partials, size_t partial_bytes, uint32_t* amax_ws, int force_splits,
-                        int counters_of_pass, hipStream_t s);
+                        int counters_of_pass, hipStream_t s, const NcAhead* ahead = nullptr);
 
 // many query positions per row (nc_attention_prefill.hip): flash-attention forward on the bf16 matrix cores
 // compute units of the current device (looked up once per process and device)
 int nc_cu_count();
 int nc_launch_attention_prefill(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache, const int32_t* cache_seqlens,
                                 int window_left, bf16_t* out, int B, int T, int H, int Hkv, int Tmax, int seqlens_include_new,
-                                uint32_t* amax_ws, hipStream_t s);
+                                uint32_t* amax_ws, hipStream_t s, const NcAhead* ahead = nullptr);
 int nc_attn_splits(int B, int T, int Hkv, int window_left, int Tmax);
 // rows that share their first cached tokens (nc_attention_prefill.hip, nc_attention.hip)
 void nc_attn_shared_plan(int rows, int H, int Hkv, int shared_len, int* chunk_keys_out, int* nchunks_out);

@@ -1,0 +1,41 @@
+// Weights on their way while the memory is idle.  A forward pass reads each weight once, and the weights of a model of more than 256 MB have left the
+// last-level cache by the next pass: the linears of a prompt, whose tiles wait for one K-step of their operands after the other, then run at the
+// latency of HBM (us, weights in HBM / in that cache: 1792 x 1664 x 6656 33.7 / 24.3, 1792 x 4992 x 1664 27.2 / 22.7, 1792 x 6656 x 1664 29.5 / 25.2).
+// A launch that computes while the memory has nothing to do (attention of a prompt) carries some workgroups more that read the weights of the
+// linears behind it, 32 KB at a time, one run of addresses after the other, and throw away what they read.
+#pragma once
+#include "nc_common.h"
+
+#define NC_AHEAD_RANGES 4
+#define NC_AHEAD_WGS 128                      // workgroups of 256 threads: 33 MB in some 8 us
+struct NcAhead {
+    const void* p[NC_AHEAD_RANGES];
+    uint32_t bytes[NC_AHEAD_RANGES];
+    int n;
+    void add(const void* ptr, size_t size) {
+        if (n == NC_AHEAD_RANGES || !ptr || ((uintptr_t)ptr & 15) || size >= 1u << 31) return;
+        p[n] = ptr, bytes[n] = (uint32_t)size, n++;
+    }
+};
+
+// for the `wg`th of `wgs` workgroups of THREADS threads; a load past the end of a range returns zeros.  (Not with the non-temporal hint: such loads leave
+// nothing in the last-level cache.)
+template <int THREADS>
+__device__ __forceinline__ void read_ahead(const NcAhead& a, int wg, int wgs) {
+    constexpr uint32_t CHUNK = 32768, UNROLL = CHUNK / (16 * THREADS);
+#pragma unroll
+    for (int r = 0; r < NC_AHEAD_RANGES; r++) {
+        if (r >= a.n) return;
+        const uint32_t n = a.bytes[r];
+        const __amdgpu_buffer_rsrc_t desc = __builtin_amdgcn_make_buffer_rsrc((void*)a.p[r], 0, n, 0x00020000);
+        for (uint32_t c = (uint32_t)wg * CHUNK; c < n; c += (uint32_t)wgs * CHUNK) {
+            v4i v[UNROLL];
+#pragma unroll
+            for (uint32_t i = 0; i < UNROLL; i++) v[i] = __builtin_amdgcn_raw_buffer_load_b128(desc, c + (i * THREADS + threadIdx.x) * 16, 0, 0);
+            v4i x = v[0];
+#pragma unroll
+            for (uint32_t i = 1; i < UNROLL; i++) x ^= v[i];
+            asm volatile("" ::"v"(x));            // (the loads are not dead code)
+        }
+    }
+}
