@@ -70,11 +70,10 @@ template <int GS, int KS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
                                                            const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ cache_seqlens,
                                                            int window_left, int seqlens_include_new, bf16_t* __restrict__ out,
-                                                           uint32_t* __restrict__ amax_ws, int T, int H, int Hkv, int Tmax, PfUnitMap map, NcAhead ahead, int B) {
+                                                           uint32_t* __restrict__ amax_ws, int T, int H, int Hkv, int Tmax, PfUnitMap map, NcAhead ahead, int nx, int units, int B) {
     constexpr int QT = 128 / (GS * KS);                        // queries per workgroup
-    if ((int)blockIdx.z >= B) {                                // (workgroups of no row: they come last)
-        const int wg = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * (blockIdx.z - B));
-        if (wg < NC_AHEAD_WGS) read_ahead<256>(ahead, wg, NC_AHEAD_WGS);
+    if ((int)blockIdx.x >= units * B) {                        // (workgroups of no row: they come last)
+        read_ahead<256>(ahead, blockIdx.x - units * B, gridDim.x - units * B);
         return;
     }
     __shared__ __align__(16) uint8_t lds[2 * PF_KBYTES + 2 * PF_VBYTES];
@@ -86,10 +85,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // Workgroups go to the eight XCDs in turn by their linear index, and each XCD has an L2 of its own: the (tile, head) pairs of a
     // row are numbered so that one XCD gets a contiguous run of them, i.e. all tiles of a few heads, and the keys and values of a head
     // are then read into one L2 instead of all eight.  Within a head the tiles come from the end of the sequence, longest first.
-    const int b = blockIdx.z;
+    const int b = B == 1 ? 0 : (int)blockIdx.x / units;
     int qb0, hy;
     {
-        const int nx = gridDim.x, total = nx * (int)gridDim.y, lid = (int)blockIdx.x + nx * (int)blockIdx.y;
+        const int total = units, lid = (int)blockIdx.x - b * units;
         const int xcd = lid & 7, slot = lid >> 3;
         const int unit = map.on ? (int)map.unit[lid] : xcd * (total >> 3) + min(xcd, total & 7) + slot;
         hy = unit / nx;
@@ -614,18 +613,16 @@ int nc_launch_attention_prefill(const bf16_t* q, const bf16_t* k_cache, const bf
     const long long wgs1 = (long long)B * Hkv * (G / GS) * ((T + 128 / GS - 1) / (128 / GS));
     const int KS = (GS <= 2 && wgs1 < 2LL * nc_cu_count()) ? 2 : 1;
     const int QT = 128 / (GS * KS);
-    dim3 grid((T + QT - 1) / QT, Hkv * (G / GS), B);
-    const int slices = (NC_AHEAD_WGS + (int)(grid.x * grid.y) - 1) / (int)(grid.x * grid.y);
-    const bool reads_ahead = ahead && ahead->n > 0 && B + slices <= 65535;
-    if (reads_ahead) grid.z += slices;
-    NC_CHECK_ARG(grid.y <= 65535, "prefill_attention: too many heads in one launch");
+    const int nx = (T + QT - 1) / QT, ny = Hkv * (G / GS), extra = ahead && ahead->n > 0 ? NC_AHEAD_WGS : 0;
+    NC_CHECK_ARG((long long)nx * ny * B + extra < (1LL << 31), "prefill_attention: too many workgroups in one launch");
+    const dim3 grid(nx * ny * B + extra);
     PfUnitMap map;                         // passed by value
     map.on = 0;
     // one row whose queries see every key before them (a window of at least the cache length is none): the long prompt of a prefill
-    if (B == 1 && (window_left < 0 || window_left >= Tmax)) pf_balance_units(map, (int)grid.x, (int)grid.y, nc_cu_count());
+    if (B == 1 && (window_left < 0 || window_left >= Tmax)) pf_balance_units(map, nx, ny, nc_cu_count());
 #define PF_LAUNCH(GG, KK)                                                                                                              \
     hipLaunchKernelGGL((attn_prefill_kernel<GG, KK>), grid, dim3(256), 0, s, q, k_cache, v_cache, cache_seqlens, window_left,          \
-                       seqlens_include_new, out, amax_ws, T, H, Hkv, Tmax, map, reads_ahead ? *ahead : NcAhead{}, B)
+                       seqlens_include_new, out, amax_ws, T, H, Hkv, Tmax, map, extra ? *ahead : NcAhead{}, nx, nx * ny, B)
     if (GS == 4) PF_LAUNCH(4, 1);
     else if (GS == 2 && KS == 2) PF_LAUNCH(2, 2);
     else if (GS == 2) PF_LAUNCH(2, 1);
