@@ -184,6 +184,14 @@ int nc_qkv_rope_append(const uint16_t* qkv, int ld_qkv, const uint16_t* xn, int 
                        int rope_len, const int32_t* cache_seqlens, uint16_t* k_cache, uint16_t* v_cache,
                        uint16_t* q_out, int B, int T, int H, int Hkv, int Tmax, int vocab_rows, nc_stream_t stream);
 
+/* nc_fp8_gemm_tn of the stacked q|k|v weight (inv_w: three scales) and nc_qkv_rope_append of its rows in one launch, the same bits: a [B*T,K] e4m3, w
+ * [(H+2Hkv)*128,K].  For more than 128 rows, K a multiple of 128, operands below 2 GiB, ld_xn a multiple of 8 and 16-byte aligned tensors; 1 is
+ * returned, and nothing done, for anything else.  kernel: 0 auto, 16 / 17 tiles of 64 / 96 x 128 with four LDS stages, 102..106 of 128..384 x 128. */
+int nc_qkv_linear_rope_append(const uint8_t* a, const uint8_t* w, const float* inv_a, const float* inv_w, const uint16_t* xn, int ld_xn,
+                              const int64_t* idx, const uint16_t* ve_table, const float* ve_gate_w, const uint16_t* cos, const uint16_t* sin,
+                              int rope_len, const int32_t* cache_seqlens, uint16_t* k_cache, uint16_t* v_cache, uint16_t* q_out, int B, int T,
+                              int K, int H, int Hkv, int Tmax, int vocab_rows, int kernel, nc_stream_t stream);
+
 /* (3) Attention of T new tokens per row over the KV cache (decode: T = 1): flash_attn_with_kvcache
  * as called at nanochat/gpt.py:113-120 (nanochat/flash_attention.py:139-185), after the append.
  * q bf16 [B*T,H,128]; caches bf16 [B,Tmax,Hkv,128]; out bf16 [B*T,H,128].

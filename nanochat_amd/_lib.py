@@ -14,7 +14,7 @@ EXPORTS = [
     "nc_fp8_quantize_tensorwise_as", "nc_fp8_encode_with_scale", "nc_fp8_transpose", "nc_fp8_gemm_tn_grad", "nc_fp8_gemm_tn_relu2", "nc_fp8_meeting_bytes",
     "nc_fp8_gemm_relu2_e4m3_fits", "nc_fp8_gemm_tn_relu2_e4m3",
     "nc_fp8_small_m_workspace_bytes", "nc_fp8_linear_small_m",
-    "nc_rmsnorm", "nc_embed_norm_smear", "nc_mix_norm", "nc_mix_norm_e4m3", "nc_relu2", "nc_qkv_rope_append",
+    "nc_rmsnorm", "nc_embed_norm_smear", "nc_mix_norm", "nc_mix_norm_e4m3", "nc_relu2", "nc_qkv_rope_append", "nc_qkv_linear_rope_append",
     "nc_attention_workspace_bytes", "nc_decode_attention", "nc_kv_cache_prefill", "nc_softcap", "nc_sample",
     "nc_gpt_workspace_bytes", "nc_gpt_forward", "nc_profile_enable", "nc_profile_read", "nc_profile_read_gemm",
     "nc_decode_attention_append", "nc_qkv_rope_append_attention", "nc_decode_attention_plan", "nc_gpt_forward_tapped",
@@ -138,6 +138,7 @@ def _bind(lib):
         "nc_mix_norm_e4m3": (i, [p, p, p, i, p, p, p, p, p, p, p, p, p, i, i, i64, p]),
         "nc_relu2": (i, [p, p, i64, p, p]),
         "nc_qkv_rope_append": (i, [p, i, p, i, p, p, p, p, p, i, p, p, p, p, i, i, i, i, i, i, p]),
+        "nc_qkv_linear_rope_append": (i, [p, p, p, p, p, i, p, p, p, p, p, i, p, p, p, p, i, i, i, i, i, i, i, i, p]),
         "nc_attention_workspace_bytes": (sz, [i, i, i, i]),
         "nc_decode_attention": (i, [p, p, p, p, i, p, i, i, i, i, i, i, p, sz, p, i, p]),
         "nc_decode_attention_append": (i, [p, p, p, p, p, p, i, p, i, i, i, i, i, p, sz, p, i, p]),

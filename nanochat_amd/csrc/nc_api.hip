@@ -177,6 +177,17 @@ int nc_qkv_rope_append(const uint16_t* qkv, int ld_qkv, const uint16_t* xn, int 
                                      v_cache, q_out, B, T, H, Hkv, Tmax, vocab_rows, (hipStream_t)stream);
 }
 
+int nc_qkv_linear_rope_append(const uint8_t* a, const uint8_t* w, const float* inv_a, const float* inv_w, const uint16_t* xn, int ld_xn, const int64_t* idx,
+                              const uint16_t* ve_table, const float* ve_gate_w, const uint16_t* cos, const uint16_t* sin, int rope_len,
+                              const int32_t* cache_seqlens, uint16_t* k_cache, uint16_t* v_cache, uint16_t* q_out, int B, int T, int K, int H, int Hkv, int Tmax,
+                              int vocab_rows, int kernel, nc_stream_t stream) {
+    NC_CHECK_ARG(B > 0 && T > 0 && H > 0 && Hkv > 0 && K > 0, "qkv_rope: bad shape");
+    const NcGemmSegs segs{3, {H * 128, (H + Hkv) * 128, (H + 2 * Hkv) * 128, 0}};
+    const NcRopeSrc src{nullptr, 0, NcPartialSrc{nullptr, 0, 0, 0, nullptr, nullptr, 0, 0}, xn, ld_xn, idx, ve_table, ve_gate_w, cos, sin, rope_len, vocab_rows, nullptr, nullptr};
+    const NcRopeDst dst{cache_seqlens, k_cache, v_cache, q_out, T, H, Hkv, Tmax};
+    return nc_launch_gemm_qkv_rope(a, w, inv_a, inv_w, segs, src, dst, B * T, K, (hipStream_t)stream, kernel);
+}
+
 size_t nc_attention_workspace_bytes(int B, int T, int H, int Tmax) {
     (void)Tmax;
     if (B <= 0 || T <= 0 || H <= 0) return 0;

@@ -347,11 +347,24 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
         if (tap_x) TRY(tap_copy(tap_x + (size_t)i * M * E, w.x, (size_t)M * E, s));
         // q|k|v = FP8 linear(xn): one activation quantization, three weight scales
         NcGemmSegs qkv_segs{3, {H * 128, (H + Hkv) * 128, qkv_w, 0}};
-        NcPartialSrc qsrc;
-        TRY(lin.run(w.xn, M, site, ly.w_qkv, ly.inv_qkv, qkv_segs, w.qkv, 0, 0.f, nullptr, qkv_w, E, qkv_w, &qsrc, nullptr, rows8));
-        site++;
         bf16_t* kc = kv->k_cache + (size_t)i * layer_elems;
         bf16_t* vc = kv->v_cache + (size_t)i * layer_elems;
+        NcPartialSrc qsrc = NO_PARTIALS;
+        bool heads_done = false;
+        if (T > 1 && M > 128) {
+            // a prompt: the linear finishes its heads itself
+            if (!rows8) {
+                TRY(nc_launch_convert_only(w.xn, (int64_t)M * E, w.a8, w.inv + site, w.site(site), s));
+                rows8 = w.a8;
+            }
+            const NcRopeSrc rope{nullptr, qkv_w, NO_PARTIALS, w.xn, E, idx, ly.ve_table, ly.ve_gate_w, m->cos, m->sin, m->rope_len, m->padded_vocab, nullptr, nullptr};
+            const int rc = nc_launch_gemm_qkv_rope(rows8, ly.w_qkv, w.inv + site, ly.inv_qkv, qkv_segs, rope,
+                                                   NcRopeDst{kv->cache_seqlens, kc, vc, w.qh, T, H, Hkv, kv->max_seq_len}, M, E, s);
+            if (rc < 0) return rc;
+            heads_done = rc == 0;
+        }
+        if (!heads_done) TRY(lin.run(w.xn, M, site, ly.w_qkv, ly.inv_qkv, qkv_segs, w.qkv, 0, 0.f, nullptr, qkv_w, E, qkv_w, &qsrc, nullptr, rows8));
+        site++;
         // rows that begin with one replicated prompt: a layer that sees a long stretch of it reads that stretch once for all rows
         bool shared_done = false;
         if (T == 1 && (long)B * Hkv >= NC_SHARED_MIN_ROW_HEADS && kv->shared_prefix > 0 && kv->uniform_pos >= kv->shared_prefix && w.shared_parts) {
@@ -378,7 +391,8 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
             TRY(nc_launch_attention_fused(rope, kc, vc, kv->cache_seqlens, ly.window_left, w.y, B, H, Hkv, kv->max_seq_len,
                                           w.attn_counters, w.attn_parts, w.attn_part_bytes, w.site(site), 0, 1, s));
         } else {
-            if (qsrc.parts)
+            if (heads_done) {
+            } else if (qsrc.parts)
                 TRY(nc_launch_qkv_rope_append_p(qsrc, w.xn, E, idx, ly.ve_table, ly.ve_gate_w, m->cos, m->sin, m->rope_len,
                                                 kv->cache_seqlens, kc, vc, w.qh, B, T, H, Hkv, kv->max_seq_len, m->padded_vocab, s));
             else

@@ -19,6 +19,7 @@
 #include "nc_common.h"
 #include "nc_kernels.h"
 #include "nc_meeting.h"
+#include "nc_rope.h"
 
 // 16-byte chunk c of LDS row r (128-byte rows) is kept at chunk slot c ^ NC_SWZ(r) by the buffer-load kernels.  Measured on
 // gfx950: with this mapping a fragment read (16 rows per 16 lanes, ds_read_b128) runs at the rate of a lane-linear read
@@ -40,6 +41,12 @@ struct EpilogueArgs {
     bf16_t* left;            // [M, N]: where a workgroup that leaves the meeting puts its tile
     float* inv_out;
 };
+// out_kind 5: the q|k|v linear of a prompt, whose rows go on to rotary, norm and cache (rope_epilogue)
+struct RopeArgs {
+    NcRopeSrc src;
+    NcRopeDst dst;
+};
+struct NoRope {};
 
 // relu(bf16(v))^2, to be rounded to bf16 by the caller's pack: the two eager ops of nanochat/gpt.py:139 on a bf16 tensor
 __device__ __forceinline__ float relu2_of(float v) {
@@ -374,6 +381,44 @@ __device__ __forceinline__ void q8_epilogue(v4f (&acc)[BM / WGM / 16][BN / WGN /
         if (m < M && n < N) *(uint4*)((uint8_t*)ep.out + (size_t)m * ep.ldc + n) = *(const uint4*)(reg + row * PITCH + c * 16);
     }
     if (left) meeting_take(ep.meeting, gridDim.x, [&](int w) { q8_convert_left<BM, BN>(ep, w, amax, scale, M, N, tiles_m, tiles_n); });
+}
+
+// ------------------------------------------------------------------------------------------------
+// The q|k|v linear of a prompt with what comes behind it: a tile is 128 columns wide, which is one head, so rotary, QK-norm, gain, value embedding and the
+// append to the cache are done on the tile as it leaves through LDS, and the 18 MB of bf16 rows (1792 x 4992) that a launch of its own read back are
+// never written.  Same roundings as the two launches, same bits.  1792 x 4992 x 1664 in a d26 prompt: 26.6 us against 20.0 and 14.2.
+template <int BM, int WGM, int WGN>
+__device__ __forceinline__ void rope_epilogue(v4f (&acc)[BM / WGM / 16][128 / WGN / 16], uint8_t* lds, const EpilogueArgs& ep, const RopeArgs& rope, float inv_a,
+                                              const float (&sc)[4], int m0, int n0, int M) {
+    constexpr int WTM = BM / WGM / 16, WTN = 128 / WGN / 16, WROWS = BM / WGM, WCOLS = 128 / WGN, PITCH = 272, NT = 64 * WGM * WGN, ROUNDS = BM / (NT / 8);
+    static_assert(BM % (NT / 8) == 0 && BM * PITCH <= 2 * (BM + 128) * 128, "epilogue staging");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x / 64, wm = wave / WGN, wn = wave % WGN, frow = lane & 15, kb = lane >> 4;
+    const int hh = n0 / 128, part = threadIdx.x & 7;
+    // (every segment is whole heads: one scale for the tile)
+    float inv_b = sc[0];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+        if (i + 1 < ep.segs.nseg && n0 >= ep.segs.end[i]) inv_b = sc[i + 1];
+    __syncthreads();                                       // every wave is done with the operand tiles
+#pragma unroll
+    for (int j = 0; j < WTN; j++)
+#pragma unroll
+        for (int i = 0; i < WTM; i++) {
+            const v4f a4 = acc[i][j];
+            *(uint2*)(lds + (wm * WROWS + i * 16 + frow) * PITCH + (wn * WCOLS + j * 16 + 4 * kb) * 2) =
+                make_uint2(pack_bf16_hw((a4[0] * inv_a) * inv_b, (a4[1] * inv_a) * inv_b), pack_bf16_hw((a4[2] * inv_a) * inv_b, (a4[3] * inv_a) * inv_b));
+        }
+    // (asked for here, where the accumulators' registers are free)
+    RopeVecRaw raw[ROUNDS];
+#pragma unroll
+    for (int it = 0; it < ROUNDS; it++) rope_vec_load(rope.src, rope.dst, min(m0 + it * (NT / 8) + (int)(threadIdx.x >> 3), M - 1), hh, part, raw[it]);
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < ROUNDS; it++) {
+        const int row = it * (NT / 8) + (threadIdx.x >> 3), token = m0 + row;
+        const uint8_t* src = lds + row * PITCH + part * 16;
+        rope_vec_finish(rope.src, rope.dst, raw[it], *(const uint4*)src, *(const uint4*)(src + 128), min(token, M - 1), hh, part, token < M);
+    }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -919,6 +964,86 @@ __global__ __launch_bounds__(512) void gemm_dln_kernel(const uint8_t* __restrict
     else dln_epilogue<NJ, OUT_KIND == 2>(acc, lds, ep, inv_a, sc, g, m0, n0, M, N);
 }
 
+// The same once more with tiles of 64 WTM rows x 128 columns (WTM = 2 .. 6 blocks of 16 rows per wave): whole heads of the q|k|v linear, for rope_epilogue.  The
+// 320-row tile has the area of the 256 x 160 one.
+template <int WTM>
+__device__ __forceinline__ void rope_fetch(const uint8_t* A, int a_bytes, const uint8_t* B, int b_bytes, uint8_t* st, const uint32_t* vo_a, const uint32_t* vo_b, int k_off) {
+    const __amdgpu_buffer_rsrc_t desc_a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, a_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t desc_b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, b_bytes, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < WTM; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_a, (lds_ptr_t)(st + i * 8192), 16, vo_a[i], k_off, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_b, (lds_ptr_t)(st + WTM * 8192 + i * 8192), 16, vo_b[i], k_off, 0, 0);
+}
+template <int WTM>
+__global__ __launch_bounds__(512) void gemm_rope_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, EpilogueArgs ep, RopeArgs rope, int M, int N,
+                                                        int K, int tiles_m, int tiles_n) {
+    constexpr int BM = 64 * WTM, STAGE = (BM + 128) * 128;
+    extern __shared__ __align__(16) uint8_t lds[];
+    int tm, tn;
+    tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+    const int m0 = tm * BM, n0 = tn * 128;
+    const DlGeom g = dl_geom();
+    const int wave_s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // piece i of this wave is the 1 KB block (wave + 8 i) of its operand's part of the stage: tile rows 8 wave + 64 i + sub
+    uint32_t vo_a[WTM], vo_b[2];
+#pragma unroll
+    for (int i = 0; i < WTM; i++) {
+        const int ra = m0 + 8 * g.wave + 64 * i + g.sub;
+        vo_a[i] = ra < M ? (uint32_t)ra * (uint32_t)K + g.gch * 16 : NC_BUF_OOB;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int rb = n0 + 8 * g.wave + 64 * i + g.sub;
+        vo_b[i] = rb < N ? (uint32_t)rb * (uint32_t)K + g.gch * 16 : NC_BUF_OOB;
+    }
+    const int ksteps = K / 128;
+    v4f acc[WTM][4];
+#pragma unroll
+    for (int i = 0; i < WTM; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    auto fetch = [&](int t, int buf) {
+        if (t < ksteps) rope_fetch<WTM>(A, M * K, B, N * K, lds + buf * STAGE + wave_s * 1024, vo_a, vo_b, t * 128);
+    };
+    auto compute = [&](const uint8_t* st, int t, int buf) {
+        const uint8_t* a = st + g.wm * (16 * WTM) * 128;
+        const uint8_t* b = st + BM * 128 + g.wn * 64 * 128;
+        v8i bf[4], af[2];
+        af[0] = dl_frag(a, g);
+#pragma unroll
+        for (int j = 0; j < 4; j++) bf[j] = dl_frag(b + j * 2048, g);
+        fetch(t, buf);
+#pragma unroll
+        for (int i = 0; i < WTM; i++) {
+            if (i + 1 < WTM) af[(i + 1) & 1] = dl_frag(a + (i + 1) * 2048, g);    // one group ahead of its use
+#pragma unroll
+            for (int j = 0; j < 4; j++) mfma_f8_acc_ordered<0>(acc[i][j], bf[j], af[i & 1]);
+        }
+    };
+    fetch(0, 0);
+    dl_step_barrier();
+    int kt = 0;
+    for (; kt + 1 < ksteps; kt += 2) {
+        compute(lds, kt + 1, 1);
+        dl_step_barrier();
+        compute(lds + STAGE, kt + 2, 0);
+        dl_step_barrier();
+    }
+    if (kt < ksteps) compute(lds, ksteps, 0);
+
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < WTM; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) asm volatile("" : "+a"(acc[i][j]));
+    const float inv_a = *ep.inv_a;
+    float sc[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) sc[i] = ep.inv_b[i < ep.segs.nseg ? i : 0];
+    rope_epilogue<BM, 4, 2>(acc, lds, ep, rope, inv_a, sc, m0, n0, M);
+}
+
 // load r of the A_P + 4 operand loads of one K-step of gemm_dr_kernel: `st` is the wave's first 1 KB piece of the stage, its pieces lie 4 KB apart
 template <int A_P>
 __device__ __forceinline__ void dr_load(const uint8_t* A, int a_bytes, const uint8_t* B, int b_bytes, uint8_t* st, int b_part, const uint32_t* vo_a,
@@ -940,9 +1065,9 @@ __device__ __forceinline__ void dr_load(const uint8_t* A, int a_bytes, const uin
 //
 // OUT_KIND 3: the K-steps are dealt to gridDim.y workgroups per tile, which leave raw fp32 sums ([share][M][N] at ep.out) for the row pass
 // that adds the linear's output to the residual stream anyway (nc_gemm_prompt_splits).
-template <int BM, int OUT_KIND>
+template <int BM, int OUT_KIND, typename Rope = NoRope>
 __global__ __launch_bounds__(256) void gemm_dr_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, EpilogueArgs ep, int M,
-                                                      int N, int K, int tiles_m, int tiles_n) {
+                                                      int N, int K, int tiles_m, int tiles_n, Rope rope) {
     constexpr int WTM = BM / 32, STAGE = (BM + 128) * 128, A_P = BM / 32, LOADS = A_P + 4;
     // s_waitcnt vmcnt(n * LOADS) lgkmcnt(0): the loads of the n youngest steps may still be in flight, no LDS read
     constexpr int WAIT2 = 0x0070 | ((2 * LOADS) & 15) | (((2 * LOADS) >> 4) << 14), WAIT3 = 0x0070 | ((3 * LOADS) & 15) | (((3 * LOADS) >> 4) << 14);
@@ -1059,6 +1184,7 @@ __global__ __launch_bounds__(256) void gemm_dr_kernel(const uint8_t* __restrict_
 #pragma unroll
         for (int i = 0; i < 4; i++) sc[i] = ep.inv_b[i < ep.segs.nseg ? i : 0];
         if constexpr (OUT_KIND == 4) q8_epilogue<BM, 128, 2, 2>(acc, lds, ep, inv_a, sc, m0, n0, M, N, tiles_m, tiles_n);
+        else if constexpr (OUT_KIND == 5) rope_epilogue<BM, 2, 2>(acc, lds, ep, rope, inv_a, sc, m0, n0, M);
         else bl_epilogue<BM, 128, 2, 2, OUT_KIND>(acc, lds, ep, inv_a, sc, m0, n0, M, N);
     }
 }
@@ -1358,14 +1484,14 @@ static int launch_dln(int nj, int a_fmt, const uint8_t* a, const uint8_t* b, con
     NC_FAIL(-1, "fp8_gemm: tile widths of 128, 160, 192 and 224 columns only, not %d", 32 * nj);
 }
 
-template <int BM, int OUT_KIND>
-static int launch_dr_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s, int splits = 1) {
+template <int BM, int OUT_KIND, typename Rope = NoRope>
+static int launch_dr_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s, int splits = 1, Rope rope = Rope{}) {
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + 127) / 128;
     const size_t lds_bytes = 4 * (size_t)(BM + 128) * 128;
-    const void* fn = (const void*)gemm_dr_kernel<BM, OUT_KIND>;
+    const void* fn = (const void*)gemm_dr_kernel<BM, OUT_KIND, Rope>;
     hipError_t e = reserve_lds(fn, (int)lds_bytes);
     if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
-    hipLaunchKernelGGL((gemm_dr_kernel<BM, OUT_KIND>), dim3(tiles_m * tiles_n, splits), dim3(256), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
+    hipLaunchKernelGGL((gemm_dr_kernel<BM, OUT_KIND, Rope>), dim3(tiles_m * tiles_n, splits), dim3(256), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n, rope);
     return 0;
 }
 // e4m3 operands, bf16 or relu^2 output, K a multiple of 128
@@ -1530,6 +1656,60 @@ int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const
     else NC_FAIL(-1, "fp8_gemm: unknown kernel selector %d", force_kernel);
     if (rc) return rc;
     NC_CHECK_LAUNCH("fp8_gemm");
+    return 0;
+}
+
+// The tiles of the q|k|v linear that finish its heads: those of 64 or 96 x 128 where pick_kernel takes them (16, 17), otherwise 64 WTM x 128 (returned as
+// 100 + WTM) with the least cost by the count of dl_cost, a tile of 64 x 128 being its unit of area; 0: none.
+static int rope_tiles(int M, int N, int K) {
+    if (M <= 128 || N % 128 != 0 || K % 128 != 0 || (long)M * K >= (1L << 31) || (long)N * K >= (1L << 31)) return 0;
+    const int which = pick_kernel(M, N, K, 0);
+    if (which == 16 || which == 17) return which;
+    const int cus = cu_count();
+    int best = 0;
+    double best_cost = 0.0;
+    for (int w = 2; w <= 6; w++) {
+        const long tiles = (long)((M + 64 * w - 1) / (64 * w)) * (N / 128);
+        double cost = 0.0;
+        for (long left = tiles; left > 0; left -= cus) cost += (6.0 + w) * (1.0 + 0.2 * (double)(left < cus ? left : cus) / cus);
+        if (!best || cost < best_cost) best = w, best_cost = cost;
+    }
+    return 100 + best;
+}
+template <int WTM>
+static int launch_gemm_rope(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, const RopeArgs& rope, int M, int N, int K, hipStream_t s) {
+    const int tiles_m = (M + 64 * WTM - 1) / (64 * WTM), tiles_n = N / 128;
+    const size_t lds_bytes = 2 * (64 * WTM + 128) * 128;
+    const hipError_t e = reserve_lds((const void*)gemm_rope_kernel<WTM>, (int)lds_bytes);
+    if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
+    hipLaunchKernelGGL(gemm_rope_kernel<WTM>, dim3(tiles_m * tiles_n), dim3(512), lds_bytes, s, a, b, ep, rope, M, N, K, tiles_m, tiles_n);
+    return 0;
+}
+// 1: not a shape or an alignment of this launch
+int nc_launch_gemm_qkv_rope(const uint8_t* a, const uint8_t* b, const float* inv_a, const float* inv_b, NcGemmSegs segs, const NcRopeSrc& src, const NcRopeDst& dst,
+                            int M, int K, hipStream_t s, int force_kernel) {
+    NC_CHECK_ARG(a && b && inv_a && inv_b, "qkv_rope: null pointer");
+    NC_CHECK_ARG(dst.T > 0 && dst.H > 0 && dst.Hkv > 0 && dst.H % dst.Hkv == 0 && dst.Tmax > 0, "qkv_rope: bad shape");
+    const int N = (dst.H + 2 * dst.Hkv) * 128, fits = rope_tiles(M, N, K), which = fits && force_kernel ? force_kernel : fits;
+    NC_CHECK_ARG(!which || which == 16 || which == 17 || (which >= 102 && which <= 106), "qkv_rope: unknown kernel selector %d", force_kernel);
+    if (!which || M % dst.T != 0 || !rope_vec_aligned(src, dst)) return 1;
+    NC_CHECK_ARG((((uintptr_t)a | (uintptr_t)b) & 15) == 0, "qkv_rope: operands must be 16-byte aligned");
+    NC_CHECK_ARG(src.cos_t && src.sin_t && src.rope_len > 0 && dst.cache_seqlens && dst.k_cache && dst.v_cache && dst.q_out && (!src.ve_table || (src.ve_gate_w && src.xn && src.idx && src.ld_xn >= 12)),
+                 "qkv_rope: null pointer");
+    NC_CHECK_ARG(segs.nseg >= 1 && segs.nseg <= 4 && segs.end[segs.nseg - 1] == N, "qkv_rope: segments must end at %d columns", N);
+    for (int i = 0; i < segs.nseg; i++) NC_CHECK_ARG(segs.end[i] % 128 == 0, "qkv_rope: segments must be whole heads");
+    EpilogueArgs ep{};
+    ep.inv_a = inv_a, ep.inv_b = inv_b, ep.segs = segs;
+    const RopeArgs rope{src, dst};
+    NcProfScope prof(1, 2.0 * M * N * K, s, ((int64_t)N << 32) | (uint32_t)K);
+    const int rc = which == 16 ? launch_dr_as<64, 5, RopeArgs>(a, b, ep, M, N, K, s, 1, rope)
+                   : which == 17 ? launch_dr_as<96, 5, RopeArgs>(a, b, ep, M, N, K, s, 1, rope)
+                   : which == 102 ? launch_gemm_rope<2>(a, b, ep, rope, M, N, K, s)
+                   : which == 103 ? launch_gemm_rope<3>(a, b, ep, rope, M, N, K, s)
+                   : which == 104 ? launch_gemm_rope<4>(a, b, ep, rope, M, N, K, s)
+                   : which == 105 ? launch_gemm_rope<5>(a, b, ep, rope, M, N, K, s) : launch_gemm_rope<6>(a, b, ep, rope, M, N, K, s);
+    if (rc) return rc;
+    NC_CHECK_LAUNCH("qkv_rope");
     return 0;
 }
 

@@ -45,6 +45,12 @@ int nc_gemm_relu2_e4m3_kernel(int M, int N, int K);
 int nc_launch_gemm_relu2_e4m3(const uint8_t* a, const uint8_t* b, const float* inv_a, const float* inv_b, uint8_t* out, float* inv_out, uint32_t* out_amax,
                               bf16_t* left, NcMeeting meeting, int M, int N, int K, hipStream_t s);
 
+// the q|k|v linear of a prompt with rotary, QK-norm, value embedding and the append to the cache in its epilogue (nc_rope.h); 1: not a shape or an alignment of it
+struct NcRopeSrc;
+struct NcRopeDst;
+int nc_launch_gemm_qkv_rope(const uint8_t* a, const uint8_t* b, const float* inv_a, const float* inv_b, NcGemmSegs segs, const NcRopeSrc& src, const NcRopeDst& dst,
+                            int M, int K, hipStream_t s, int force_kernel = 0);
+
 // small-M path (nc_gemm_decode.hip): A is e4m3 (+inv_a) or bf16 (+amax, quantized inside the kernel)
 // out_kind: 0 bf16, 1 softcapped fp32, 2 bf16 relu^2 with amax of the result into out_amax.
 // With K split over workgroups the raw fp32 sums land in `partials` [ksplits][M][N] and a consumer finishes them.

@@ -143,3 +143,110 @@ __device__ __forceinline__ void rope_head(const NcRopeSrc& r, int token, int pos
     rope_head_load(r, token, pos, hh, H, Hkv, lane, w);
     rope_head_finish(r, token, hh, H, Hkv, lane, w, amax_from_lanes(amax_lane), o1, o2);
 }
+
+// ------------------------------------------------------------------------------------------------
+// The same for many tokens whose q|k|v rows are finished bf16 values: eight lanes share a head, each holding eight consecutive elements of its first half
+// and the eight they pair with in the second half (element j rotates with j + 64), all accesses 16 bytes wide; the mean of squares of the QK-norm is a
+// sum over the 8 lanes.  Same rounding points as rope_head_finish.  Used by the stand-alone kernel and by the epilogue of the q|k|v linear.
+struct NcRopeDst {
+    const int32_t* cache_seqlens;
+    bf16_t *k_cache, *v_cache, *q_out;
+    int T, H, Hkv, Tmax;
+};
+struct RopeVecRaw {           // what one head of one token needs beside its values, as loaded
+    uint4 e1, e2;             // q, k heads: cos, sin;  v heads with a value embedding: its two halves
+    uint4 xg0;
+    uint2 xg1;                // v heads: xn[0 .. 11]
+    int b, pos;
+};
+__device__ __forceinline__ void rope_vec_load(const NcRopeSrc& r, const NcRopeDst& d, int token, int hh, int part, RopeVecRaw& w) {
+    w.b = token / d.T;
+    w.pos = d.cache_seqlens[w.b] + token % d.T;
+    w.e1 = w.e2 = w.xg0 = make_uint4(0, 0, 0, 0);
+    w.xg1 = make_uint2(0, 0);
+    if (hh < d.H + d.Hkv) {
+        const int rp = w.pos < r.rope_len ? (w.pos < 0 ? 0 : w.pos) : r.rope_len - 1;
+        w.e1 = *(const uint4*)(r.cos_t + (size_t)rp * 64 + part * 8), w.e2 = *(const uint4*)(r.sin_t + (size_t)rp * 64 + part * 8);
+    } else if (r.ve_table) {
+        int64_t tok = r.idx[token];
+        if (tok < 0 || tok >= r.vocab_rows) tok = 0;
+        const bf16_t* ve = r.ve_table + ((size_t)tok * d.Hkv + (hh - d.H - d.Hkv)) * 128 + part * 8;
+        w.e1 = *(const uint4*)ve, w.e2 = *(const uint4*)(ve + 64);
+        const bf16_t* xg = r.xn + (size_t)token * r.ld_xn;
+        w.xg0 = *(const uint4*)xg, w.xg1 = *(const uint2*)(xg + 8);
+    }
+}
+// The arithmetic is what bounds it (1792 tokens of 39 heads: 6 us of instructions over the whole chip): two roundings to a conversion.
+__device__ __forceinline__ void rbf2(float& a, float& b) {
+    const uint32_t u = pack_bf16(a, b);
+    a = bf16_lo(u), b = bf16_hi(u);
+}
+// xa, xb: the lane's elements of the head; every lane of the eight takes part, `live` ones store
+__device__ __forceinline__ void rope_vec_finish(const NcRopeSrc& r, const NcRopeDst& d, const RopeVecRaw& w, uint4 xa, uint4 xb, int token, int hh, int part, bool live) {
+    const uint32_t wa[4] = {xa.x, xa.y, xa.z, xa.w}, wb[4] = {xb.x, xb.y, xb.z, xb.w};
+    const uint32_t ea[4] = {w.e1.x, w.e1.y, w.e1.z, w.e1.w}, eb[4] = {w.e2.x, w.e2.y, w.e2.z, w.e2.w};
+    float x1[8], x2[8], o1[8], o2[8];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        x1[2 * j] = bf16_lo(wa[j]), x1[2 * j + 1] = bf16_hi(wa[j]);
+        x2[2 * j] = bf16_lo(wb[j]), x2[2 * j + 1] = bf16_hi(wb[j]);
+    }
+    if (hh < d.H + d.Hkv) {
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float c = (e & 1) ? bf16_hi(ea[e >> 1]) : bf16_lo(ea[e >> 1]);
+            const float sn = (e & 1) ? bf16_hi(eb[e >> 1]) : bf16_lo(eb[e >> 1]);
+            float a = x1[e] * c, b = x2[e] * sn, f = x1[e] * (-sn), g = x2[e] * c;
+            rbf2(a, b), rbf2(f, g);
+            a += b, f += g;
+            rbf2(a, f);
+            o1[e] = a, o2[e] = f;
+            ss += o1[e] * o1[e] + o2[e] * o2[e];
+        }
+        ss += __shfl_xor(ss, 1);
+        ss += __shfl_xor(ss, 2);
+        ss += __shfl_xor(ss, 4);
+        const float rstd = 1.0f / sqrtf(ss / 128.0f + RMS_EPS);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            float a = o1[e] * rstd, b = o2[e] * rstd;
+            rbf2(a, b);
+            o1[e] = a * 1.2f, o2[e] = b * 1.2f;               // (rounded where they are packed)
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) o1[e] = x1[e], o2[e] = x2[e];
+        if (r.ve_table) {
+            const int hv = hh - d.H - d.Hkv;
+            const uint32_t xg[6] = {w.xg0.x, w.xg0.y, w.xg0.z, w.xg0.w, w.xg1.x, w.xg1.y};
+            float dot = 0.f;
+#pragma unroll
+            for (int c = 0; c < 12; c++) dot += ((c & 1) ? bf16_hi(xg[c >> 1]) : bf16_lo(xg[c >> 1])) * rbf(r.ve_gate_w[hv * 12 + c]);
+            const float gate = rbf(3.0f * rbf(sigmoidf_(rbf(dot))));
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const float v1 = (e & 1) ? bf16_hi(ea[e >> 1]) : bf16_lo(ea[e >> 1]);
+                const float v2 = (e & 1) ? bf16_hi(eb[e >> 1]) : bf16_lo(eb[e >> 1]);
+                float a = gate * v1, b = gate * v2;
+                rbf2(a, b);
+                o1[e] += a, o2[e] += b;                       // (rounded where they are packed)
+            }
+        }
+    }
+    if (!live) return;
+    bf16_t* dst;
+    if (hh < d.H) dst = d.q_out + ((size_t)token * d.H + hh) * 128;
+    else {
+        if (w.pos < 0 || w.pos >= d.Tmax) return;
+        const bool is_k = hh < d.H + d.Hkv;
+        dst = (is_k ? d.k_cache : d.v_cache) + (((size_t)w.b * d.Tmax + w.pos) * d.Hkv + (is_k ? hh - d.H : hh - d.H - d.Hkv)) * 128;
+    }
+    dst += part * 8;
+    *(uint4*)dst = make_uint4(pack_bf16(o1[0], o1[1]), pack_bf16(o1[2], o1[3]), pack_bf16(o1[4], o1[5]), pack_bf16(o1[6], o1[7]));
+    *(uint4*)(dst + 64) = make_uint4(pack_bf16(o2[0], o2[1]), pack_bf16(o2[2], o2[3]), pack_bf16(o2[4], o2[5]), pack_bf16(o2[6], o2[7]));
+}
+// what the eight lanes ask of their pointers
+static inline bool rope_vec_aligned(const NcRopeSrc& r, const NcRopeDst& d) {
+    return r.ld_xn % 8 == 0 && (((uintptr_t)d.k_cache | (uintptr_t)d.v_cache | (uintptr_t)d.q_out | (uintptr_t)r.cos_t | (uintptr_t)r.sin_t | (uintptr_t)r.ve_table | (uintptr_t)r.xn) & 15) == 0;
+}

@@ -356,6 +356,28 @@ def qkv_rope_append(qkv, xn, idx, ve_table, ve_gate_w, cos, sin, cache_seqlens, 
     return q
 
 
+def qkv_linear_rope_append(a8, w8, inv_a, inv_w, xn, idx, ve_table, ve_gate_w, cos, sin, cache_seqlens, k_cache, v_cache, n_head, n_kv_head, kernel=0):
+    """fp8_gemm of the stacked q|k|v weight (three scales) on a8 [B,T,K] and qkv_rope_append in one launch, the same bits.  Returns q [B,T,H,128]; ValueError
+    where that launch does not take the shape (see nc_qkv_linear_rope_append)."""
+    _need_cuda(a8, w8, k_cache, v_cache, cache_seqlens)
+    B, T, K = a8.shape
+    a8, w8 = a8.contiguous(), w8.contiguous()
+    if w8.shape != ((n_head + 2 * n_kv_head) * 128, K) or inv_w.numel() != 3:
+        raise ValueError(f"qkv_linear_rope_append: weight {tuple(w8.shape)} with {inv_w.numel()} scales for {n_head} + 2 x {n_kv_head} heads of {K} inputs")
+    q = torch.empty(B, T, n_head, 128, dtype=torch.bfloat16, device=a8.device)
+    assert k_cache.is_contiguous() and v_cache.is_contiguous()
+    xn = xn.contiguous() if xn is not None else None
+    gate = ve_gate_w.float().contiguous() if ve_gate_w is not None else None
+    idx = idx.contiguous() if idx is not None else None
+    rc = _lib.lib().nc_qkv_linear_rope_append(_ptr(a8), _ptr(w8), _ptr(inv_a.reshape(-1).float()), _ptr(inv_w.reshape(-1).float()), _ptr(xn), xn.shape[-1] if xn is not None else 0,
+                                              _ptr(idx), _ptr(ve_table), _ptr(gate), _ptr(cos), _ptr(sin), cos.shape[0], _ptr(cache_seqlens), _ptr(k_cache), _ptr(v_cache), _ptr(q),
+                                              B, T, K, n_head, n_kv_head, k_cache.shape[1], ve_table.shape[0] if ve_table is not None else 0, kernel, _stream())
+    if rc > 0:
+        raise ValueError(f"qkv_linear_rope_append: {B} x {T} tokens, K={K}")
+    _lib.check(rc)
+    return q
+
+
 # ----------------------------------------------------------------------------- (3) attention
 def decode_attention(q, k_cache, v_cache, cache_seqlens, window_left=-1, seqlens_include_new=False, splits=0):
     """Attention of q [B,T,H,128] over caches [B,Tmax,Hkv,128] whose new tokens are already appended."""

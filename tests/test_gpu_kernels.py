@@ -861,6 +861,32 @@ def test_relu2(ops):
     assert torch.equal(ops.relu2(h.to(DEV)).cpu(), F.relu(h).square())
 
 
+@pytest.mark.parametrize("B,T,K,H,Hkv,ve,kernel", [(1, 1792, 1664, 13, 13, True, 0), (1, 130, 256, 2, 1, True, 0), (2, 333, 384, 6, 6, False, 0), (4, 448, 256, 13, 13, True, 0),
+                                                   (1, 129, 128, 1, 1, True, 16), (3, 65, 256, 4, 2, True, 17), (1, 255, 128, 2, 2, False, 102), (5, 77, 256, 2, 1, True, 103),
+                                                   (1, 1025, 256, 8, 4, True, 104), (1, 321, 384, 3, 3, True, 105), (2, 383, 128, 4, 1, False, 106)])
+def test_qkv_linear_finishes_its_heads(ops, B, T, K, H, Hkv, ve, kernel):
+    """The q|k|v linear with rotary, norm, value embedding and append in its epilogue: the bits of the two launches, and nothing written beside the new rows."""
+    say(f"qkv linear rope B={B} T={T} K={K} H={H} Hkv={Hkv} ve={ve} kernel={kernel}")
+    g = torch.Generator(device=DEV).manual_seed(T + K)
+    heads = H + 2 * Hkv
+    a8, inv_a, _ = ops.fp8_quantize(torch.randn(B, T, K, generator=g, device=DEV).bfloat16())
+    w8, _, _ = ops.fp8_quantize(torch.randn(heads * 128, K, generator=g, device=DEV).bfloat16())
+    inv_w = torch.tensor([0.01, 0.02, 0.03], device=DEV)
+    xn, idx = torch.randn(B, T, 16, generator=g, device=DEV).bfloat16(), torch.randint(-1, 51, (B, T), generator=g, device=DEV)
+    table = torch.randn(50, Hkv * 128, generator=g, device=DEV).bfloat16() if ve else None
+    gate = torch.randn(Hkv, 12, generator=g, device=DEV) if ve else None
+    lengths = torch.arange(B, device=DEV, dtype=torch.int32) * 3
+    Tmax = T + 3 * B - 5 if B > 2 else T + 3 * B                        # (the last row of many does not fit whole)
+    angles = torch.rand(Tmax + 20, 64, generator=g, device=DEV) * 6
+    cos, sin = angles.cos().bfloat16(), angles.sin().bfloat16()
+    caches = [torch.randn(B, Tmax, Hkv, 128, generator=g, device=DEV).bfloat16() for _ in range(2)]
+    want_k, want_v, got_k, got_v = caches[0].clone(), caches[1].clone(), caches[0].clone(), caches[1].clone()
+    qkv = ops.fp8_gemm(a8.view(B * T, K), w8, inv_a, inv_w, seg_ends=[H * 128, (H + Hkv) * 128, heads * 128])
+    want = ops.qkv_rope_append(qkv.view(B, T, -1), xn, idx, table, gate, cos, sin, lengths, want_k, want_v, H, Hkv)
+    got = ops.qkv_linear_rope_append(a8, w8, inv_a, inv_w, xn, idx, table, gate, cos, sin, lengths, got_k, got_v, H, Hkv, kernel=kernel)
+    assert torch.equal(got, want) and torch.equal(got_k, want_k) and torch.equal(got_v, want_v)
+
+
 @pytest.mark.parametrize("spin_limit", [-1, 0])
 @pytest.mark.parametrize("rows,cols,splits", [(1792, 1664, 0), (129, 256, 0), (333, 1040, 0), (1023, 512, 0), (2048, 2048, 0), (130, 1024, 8), (257, 1280, 2), (511, 2032, 4), (1023, 512, 2), (1024, 2048, 3), (257, 16, 9)])
 def test_mix_norm_written_as_e4m3(ops, rows, cols, splits, spin_limit):
