@@ -548,10 +548,11 @@ __global__ __launch_bounds__(128) void latent_combine_kernel(const float* __rest
 template <int DN, int DR, int DV, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void latent_expanded_kernel(
     NcLatentGeom g, const bf16_t* __restrict__ q, int ldq, const bf16_t* __restrict__ kv, int keys_alloc, const bf16_t* __restrict__ cache,
-    const int32_t* __restrict__ seqlens, bf16_t* __restrict__ out, int ldo) {
+    const int32_t* __restrict__ seqlens, bf16_t* __restrict__ out, int ldo, NcAhead ahead) {
     constexpr int DQK = DN + DR, KPITCH = DQK * 2 + 16, VPITCH = DV * 2 + 64, NTHR = 64 * NW, KB = 16 * NW, QT = 32 * NW;
     constexpr int NCH = DN / 8, RCH = DR / 8, VCH = DV / 8, NL = KB * NCH / NTHR, RL = KB * RCH / NTHR, VL = KB * VCH / NTHR;
     __shared__ __align__(16) uint8_t lds[KB * KPITCH + KB * VPITCH];
+    if (reads_ahead<NTHR>(ahead, g.B)) return;
     uint8_t* const lds_v = lds + KB * KPITCH;
     const lds_u8_t lds_v3 = (lds_u8_t)lds + KB * KPITCH;
     const int b = blockIdx.z;
@@ -759,13 +760,13 @@ int launch_mfma(const NcLatentGeom& g, const bf16_t* q, const bf16_t* cache, con
 }
 template <int DN, int DR, int DV>
 int launch_expanded(const NcLatentGeom& g, const bf16_t* q, int ldq, const bf16_t* kv, int keys, const bf16_t* cache, const int32_t* seqlens, bf16_t* out,
-                    int ldo, hipStream_t s) {
+                    int ldo, const NcAhead* ahead, hipStream_t s) {
     if ((int64_t)((g.T + 127) / 128) * g.heads * g.B >= 200)
-        hipLaunchKernelGGL((latent_expanded_kernel<DN, DR, DV, 4>), dim3((g.T + 127) / 128, g.heads, g.B), dim3(256), 0, s, g, q, ldq, kv, keys, cache,
-                           seqlens, out, ldo);
+        hipLaunchKernelGGL((latent_expanded_kernel<DN, DR, DV, 4>), nc_ahead_grid(dim3((g.T + 127) / 128, g.heads, g.B), ahead), dim3(256), 0, s, g, q, ldq, kv, keys, cache,
+                           seqlens, out, ldo, ahead ? *ahead : NcAhead{});
     else
-        hipLaunchKernelGGL((latent_expanded_kernel<DN, DR, DV, 2>), dim3((g.T + 63) / 64, g.heads, g.B), dim3(128), 0, s, g, q, ldq, kv, keys, cache, seqlens,
-                           out, ldo);
+        hipLaunchKernelGGL((latent_expanded_kernel<DN, DR, DV, 2>), nc_ahead_grid(dim3((g.T + 63) / 64, g.heads, g.B), ahead), dim3(128), 0, s, g, q, ldq, kv, keys, cache, seqlens,
+                           out, ldo, ahead ? *ahead : NcAhead{});
     NC_CHECK_LAUNCH("latent_expanded");
     return 0;
 }
@@ -864,13 +865,13 @@ int nc_launch_latent_attention(int dtype, const NcLatentGeom& g, const void* q_l
 bool nc_latent_expanded_ok(int dtype, const NcLatentGeom& g) { return dtype == 0 && g.dim_p <= 128 && g.rot_p <= 64 && g.vdim_p <= 128; }
 
 int nc_launch_latent_expanded(const NcLatentGeom& g, const bf16_t* q, int ldq, const bf16_t* kv, int keys, const bf16_t* cache, const int32_t* seqlens,
-                              bf16_t* out, int ldo, hipStream_t s) {
+                              bf16_t* out, int ldo, const NcAhead* ahead, hipStream_t s) {
     NC_CHECK_ARG(nc_latent_expanded_ok(0, g) && keys >= g.pos_max + g.T && keys <= g.Tmax, "latent_expanded: sizes not supported");
     const int dqk = g.dim_p + g.rot_p;
     // causal pairs: all earlier keys and half of the new ones
     NcProfScope prof(NC_CLS_LATENT, 2.0 * g.B * g.heads * g.T * (g.pos_max + 0.5 * (g.T + 1)) * (dqk + g.vdim_p), s, g.T);
     NC_CHECK_ARG((int64_t)keys * g.heads * (g.dim_p + g.vdim_p) * 2 < (1ll << 31), "latent_expanded: %d keys past 2 GiB", keys);
-#define GO(N, R, V) launch_expanded<N, R, V>(g, q, ldq, kv, keys, cache, seqlens, out, ldo, s)
+#define GO(N, R, V) launch_expanded<N, R, V>(g, q, ldq, kv, keys, cache, seqlens, out, ldo, ahead, s)
 #define GO_V(N, R) (g.vdim_p <= 64 ? GO(N, R, 64) : GO(N, R, 128))
     if (g.dim_p <= 64) return g.rot_p <= 32 ? GO_V(64, 32) : GO_V(64, 64);
     return g.rot_p <= 32 ? GO_V(128, 32) : GO_V(128, 64);

@@ -17,6 +17,12 @@ struct NcAhead {
         p[n] = ptr, bytes[n] = (uint32_t)size, n++;
     }
 };
+// Launches whose grid counts rows in z carry the workgroups that read ahead in the slices behind them.
+static inline dim3 nc_ahead_grid(dim3 grid, const NcAhead* a) {
+    const unsigned per = grid.x * grid.y, slices = (NC_AHEAD_WGS + per - 1) / per;
+    if (a && a->n > 0 && grid.z + slices <= 65535) grid.z += slices;
+    return grid;
+}
 
 // for the `wg`th of `wgs` workgroups of THREADS threads; a load past the end of a range returns zeros.  (Not with the non-temporal hint: such loads leave
 // nothing in the last-level cache.)
@@ -38,4 +44,12 @@ __device__ __forceinline__ void read_ahead(const NcAhead& a, int wg, int wgs) {
             asm volatile("" ::"v"(x));            // (the loads are not dead code)
         }
     }
+}
+// whether this workgroup is one of those (it has read its share then and has nothing else to do)
+template <int THREADS>
+__device__ __forceinline__ bool reads_ahead(const NcAhead& a, int rows) {
+    if ((int)blockIdx.z < rows) return false;
+    const int wg = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * ((int)blockIdx.z - rows));
+    if (wg < NC_AHEAD_WGS) read_ahead<THREADS>(a, wg, NC_AHEAD_WGS);
+    return true;
 }

@@ -279,11 +279,12 @@ __global__ __launch_bounds__(256) void retention_scan_kernel(NcRetentionGeom g, 
 template <int DK, int DV, int C>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void retention_chunk_out_kernel(NcRetentionGeom g, const bf16_t* __restrict__ proj, int ldp, const float* __restrict__ decay,
                                                                   const float* __restrict__ rope, int rope_len, const int32_t* __restrict__ seqlens,
-                                                                  const bf16_t* __restrict__ prefix, int chunks, float eps, bf16_t* __restrict__ out, int ldo) {
+                                                                  const bf16_t* __restrict__ prefix, int chunks, float eps, bf16_t* __restrict__ out, int ldo, NcAhead ahead) {
     constexpr int QB = C / 32, VS = 4 / QB, NT = DV / 32 / VS, KP = DK * 2 + 16, VP = DV * 2 + 64;
     static_assert(NT >= 1, "value columns per wave");
     __shared__ __align__(16) uint8_t lds[C * (2 * KP + VP)];
     __shared__ float red[VS][C];
+    if (reads_ahead<256>(ahead, g.B)) return;
     uint8_t *const lk_hi = lds, *const lk_lo = lds + C * KP, *const lv = lds + 2 * C * KP;
     const int chunk = blockIdx.x, h = blockIdx.y, b = blockIdx.z, tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), qb = wave % QB, vs = wave / QB;
@@ -594,7 +595,7 @@ int chunk_size(int dtype, const NcRetentionGeom& g) {
 }
 template <int DK, int DV, int C>
 int launch_chunked(const NcRetentionGeom& g, const bf16_t* proj, int ldp, const float* decay, const float* rope, int rope_len, const int32_t* seqlens,
-                   const float* state_in, float* state_out, float eps, bf16_t* out, int ldo, void* workspace, hipStream_t s) {
+                   const float* state_in, float* state_out, float eps, bf16_t* out, int ldo, void* workspace, const NcAhead* ahead, hipStream_t s) {
     const int chunks = (g.T + C - 1) / C;
     float* kv = (float*)workspace;
     bf16_t* prefix = (bf16_t*)(kv + (int64_t)g.B * chunks * g.heads * DK * DV);
@@ -602,8 +603,8 @@ int launch_chunked(const NcRetentionGeom& g, const bf16_t* proj, int ldp, const 
                        chunks);
     hipLaunchKernelGGL(retention_scan_kernel, dim3((DK * DV + 1023) / 1024, g.heads, g.B), dim3(256), 0, s, g, decay, seqlens, kv, prefix, state_in, state_out,
                        chunks, C);
-    hipLaunchKernelGGL((retention_chunk_out_kernel<DK, DV, C>), dim3(chunks, g.heads, g.B), dim3(256), 0, s, g, proj, ldp, decay, rope, rope_len, seqlens,
-                       prefix, chunks, eps, out, ldo);
+    hipLaunchKernelGGL((retention_chunk_out_kernel<DK, DV, C>), nc_ahead_grid(dim3(chunks, g.heads, g.B), ahead), dim3(256), 0, s, g, proj, ldp, decay, rope, rope_len, seqlens,
+                       prefix, chunks, eps, out, ldo, ahead ? *ahead : NcAhead{});
     NC_CHECK_LAUNCH("retention_chunked");
     return 0;
 }
@@ -634,7 +635,7 @@ size_t nc_retention_workspace_bytes(int dtype, const NcRetentionGeom& g) {
 
 int nc_launch_retention(int dtype, const NcRetentionGeom& g, const void* proj, int ldp, const float* decay, const float* rope, int rope_len,
                         const int32_t* seqlens, const float* state_in, float* state_out, float eps, void* out, int ldo, void* workspace,
-                        hipStream_t s) {
+                        const NcAhead* ahead, hipStream_t s) {
     NC_CHECK_ARG(g.rot_dims % 2 == 0 && g.rot_dims <= g.dim && g.dim <= g.dim_p && g.vdim <= g.vdim_p && g.dim_p % 8 == 0 && g.vdim_p % 8 == 0,
                  "retention: dim=%d/%d vdim=%d/%d rot=%d", g.dim, g.dim_p, g.vdim, g.vdim_p, g.rot_dims);
     NC_CHECK_ARG(state_in != state_out, "retention: the state is not updated in place");
@@ -663,7 +664,7 @@ int nc_launch_retention(int dtype, const NcRetentionGeom& g, const void* proj, i
     const bf16_t* p = (const bf16_t*)proj;
     bf16_t* o = (bf16_t*)out;
 #define CHUNKED(K, V, CC) \
-    if (g.dim_p == K && g.vdim_p == V) return launch_chunked<K, V, CC>(g, p, ldp, decay, rope, rope_len, seqlens, state_in, state_out, eps, o, ldo, workspace, s);
+    if (g.dim_p == K && g.vdim_p == V) return launch_chunked<K, V, CC>(g, p, ldp, decay, rope, rope_len, seqlens, state_in, state_out, eps, o, ldo, workspace, ahead, s);
     CHUNKED(64, 64, 64) CHUNKED(64, 128, 64) CHUNKED(64, 256, 64) CHUNKED(128, 64, 64) CHUNKED(128, 128, 64) CHUNKED(128, 256, 64)
     CHUNKED(256, 128, 32) CHUNKED(256, 256, 32)
 #undef CHUNKED

@@ -198,7 +198,8 @@ template <typename T, int SP, int MODE>
 __global__ __launch_bounds__(256) void scan_kernel(NcScanGeom g, int lg, const T* __restrict__ u, const float* __restrict__ dt, const float* __restrict__ bc,
                                                    const float* __restrict__ a_log2, const float* __restrict__ skip, const T* __restrict__ z, int ldz,
                                                    const int32_t* __restrict__ seqlens, const float* __restrict__ state_in, float* __restrict__ state_out,
-                                                   T* __restrict__ out, int ldo, float* __restrict__ ends, float* __restrict__ sum_dt, int chunks, int chunk_len) {
+                                                   T* __restrict__ out, int ldo, float* __restrict__ ends, float* __restrict__ sum_dt, int chunks, int chunk_len, NcAhead ahead) {
+    if (MODE != SCAN_SUMS && reads_ahead<256>(ahead, g.B)) return;
     extern __shared__ __align__(16) float lds[];            // [TB][2][state_p]: B, C
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cw = 64 / lg, part = lane / cw;
     const int c_at = ((int)blockIdx.x * 4 + wave) * cw + lane % cw, c = min(c_at, g.inner_p - 1);
@@ -330,21 +331,21 @@ int chunk_count(const NcScanGeom& g) {
 
 template <typename T, int SP>
 int launch_scan(const NcScanGeom& g, int lg, const T* u, const float* dt, const float* bc, const float* a_log2, const float* skip, const T* z, int ldz,
-                const int32_t* seqlens, const float* state_in, float* state_out, T* out, int ldo, void* workspace, hipStream_t s) {
+                const int32_t* seqlens, const float* state_in, float* state_out, T* out, int ldo, void* workspace, const NcAhead* ahead, hipStream_t s) {
     const int chunks = chunk_count(g), len = chunk_len(g), xs = channel_groups(g, lg), bytes = TB * 2 * g.state_p * 4;
     if (chunks == 1) {
-        hipLaunchKernelGGL((scan_kernel<T, SP, SCAN_WHOLE>), dim3(xs, 1, g.B), dim3(256), bytes, s, g, lg, u, dt, bc, a_log2, skip, z, ldz, seqlens, state_in, state_out,
-                           out, ldo, nullptr, nullptr, 1, 0);
+        hipLaunchKernelGGL((scan_kernel<T, SP, SCAN_WHOLE>), nc_ahead_grid(dim3(xs, 1, g.B), ahead), dim3(256), bytes, s, g, lg, u, dt, bc, a_log2, skip, z, ldz, seqlens, state_in, state_out,
+                           out, ldo, nullptr, nullptr, 1, 0, ahead ? *ahead : NcAhead{});
         NC_CHECK_LAUNCH("scan");
         return 0;
     }
     float* ends = (float*)workspace;
     float* sum_dt = ends + (int64_t)g.B * (chunks - 1) * g.state_p * g.inner_p;
     hipLaunchKernelGGL((scan_kernel<T, SP, SCAN_SUMS>), dim3(xs, chunks - 1, g.B), dim3(256), bytes, s, g, lg, u, dt, bc, a_log2, skip, z, ldz, seqlens, state_in,
-                       state_out, out, ldo, ends, sum_dt, chunks, len);
+                       state_out, out, ldo, ends, sum_dt, chunks, len, NcAhead{});
     hipLaunchKernelGGL(scan_chunks_kernel, dim3((g.inner_p + 255) / 256, g.state_p, g.B), dim3(256), 0, s, g, a_log2, seqlens, state_in, ends, sum_dt, chunks);
-    hipLaunchKernelGGL((scan_kernel<T, SP, SCAN_OUT>), dim3(xs, chunks, g.B), dim3(256), bytes, s, g, lg, u, dt, bc, a_log2, skip, z, ldz, seqlens, state_in, state_out,
-                       out, ldo, ends, sum_dt, chunks, len);
+    hipLaunchKernelGGL((scan_kernel<T, SP, SCAN_OUT>), nc_ahead_grid(dim3(xs, chunks, g.B), ahead), dim3(256), bytes, s, g, lg, u, dt, bc, a_log2, skip, z, ldz, seqlens, state_in, state_out,
+                       out, ldo, ends, sum_dt, chunks, len, ahead ? *ahead : NcAhead{});
     NC_CHECK_LAUNCH("scan_chunked");
     return 0;
 }
@@ -414,7 +415,7 @@ size_t nc_scan_workspace_bytes(const NcScanGeom& g) {
 }
 
 int nc_launch_scan(int dtype, const NcScanGeom& g, const void* u, const float* dt, const float* bc, const float* a_log2, const float* skip, const void* z, int ldz,
-                   const int32_t* seqlens, const float* state_in, float* state_out, void* out, int ldo, void* workspace, hipStream_t s) {
+                   const int32_t* seqlens, const float* state_in, float* state_out, void* out, int ldo, void* workspace, const NcAhead* ahead, hipStream_t s) {
     int sp = 0, lg = 0;
     NC_CHECK_ARG(lanes_of(g.state_p, sp, lg) && g.state <= g.state_p, "scan: %d states per channel in %d", g.state, g.state_p);
     NC_CHECK_ARG(u && dt && bc && a_log2 && skip && z && out && state_in != state_out, "scan: null operand");
@@ -423,9 +424,9 @@ int nc_launch_scan(int dtype, const NcScanGeom& g, const void* u, const float* d
     NcProfScope prof(NC_CLS_SCAN, (double)g.B * (8.0 * g.state * g.inner_p + (double)g.T * g.inner_p * (4 + (dtype ? 12 : 6))), s, g.T);
 #define GO(SP)                                                                                                                                           \
     (dtype ? launch_scan<float, SP>(g, lg, (const float*)u, dt, bc, a_log2, skip, (const float*)z, ldz, seqlens, state_in, state_out, (float*)out, ldo,   \
-                                    workspace, s)                                                                                                         \
+                                    workspace, ahead, s)                                                                                                         \
            : launch_scan<bf16_t, SP>(g, lg, (const bf16_t*)u, dt, bc, a_log2, skip, (const bf16_t*)z, ldz, seqlens, state_in, state_out, (bf16_t*)out, ldo, \
-                                     workspace, s))
+                                     workspace, ahead, s))
     switch (sp) {
         case 16: return GO(16);
         case 12: return GO(12);

@@ -175,7 +175,7 @@ void* at(void* p, int64_t elems, int dtype) { return (uint8_t*)p + elems * (dtyp
 // A mixer reads its columns of the projected rows (`proj`, leading dimension ldp) and writes its columns of what the output matrix multiplies
 // (`cat`, leading dimension ld_cat).
 int run_latent_attention(int dt, const nc_stack_mixer& l, const NcLatentGeom& g, const Workspace& w, void* proj, int ldp, float eps, int rope_len,
-                         const int32_t* seqlens, void* cache, void* cat, int ld_cat, hipStream_t s) {
+                         const int32_t* seqlens, void* cache, void* cat, int ld_cat, const NcAhead* ahead, hipStream_t s) {
     const int M = g.B * g.T, qd = l.dim_p + l.rot_p, rw = l.rank_p + l.rot_p, head_w = l.dim_p + l.vdim_p;
     const bool ex = expand(dt, l, g);
     TRY(nc_launch_latent_append(dt, g, proj, ldp, l.kv_norm_w, eps, l.rope, rope_len, seqlens, cache, ex ? nullptr : w.q_lat, s));
@@ -185,7 +185,7 @@ int run_latent_attention(int dt, const nc_stack_mixer& l, const NcLatentGeom& g,
         e.batch = g.B, e.a_stride = (int64_t)g.Tmax * rw, e.w_stride = 0, e.out_stride = (int64_t)keys * l.heads * head_w;
         nc_linear_seg(e, e.N, NC_SEG_PLAIN, w.kv, l.heads * head_w);
         TRY(nc_launch_linear_tiled(dt, e, s));
-        return nc_launch_latent_expanded(g, (const bf16_t*)proj, ldp, (const bf16_t*)w.kv, keys, (const bf16_t*)cache, seqlens, (bf16_t*)cat, ld_cat, s);
+        return nc_launch_latent_expanded(g, (const bf16_t*)proj, ldp, (const bf16_t*)w.kv, keys, (const bf16_t*)cache, seqlens, (bf16_t*)cat, ld_cat, ahead, s);
     }
     // unrotated queries into latent space, one product per head
     NcLinear q = nc_linear(proj, ldp, l.w_uk_t, M, l.rank_p, l.dim_p);
@@ -201,21 +201,21 @@ int run_latent_attention(int dt, const nc_stack_mixer& l, const NcLatentGeom& g,
 }
 
 int run_window_attention(int dt, const nc_stack_mixer& l, const NcWindowGeom& g, const Workspace& w, void* proj, int ldp, float eps, int rope_len,
-                         const int32_t* seqlens, void* cache, void* cat, int ld_cat, hipStream_t s) {
+                         const int32_t* seqlens, void* cache, void* cat, int ld_cat, const NcAhead* ahead, hipStream_t s) {
     TRY(nc_launch_window_append(dt, g, proj, ldp, l.qkv_bias, l.q_norm_w, l.k_norm_w, eps, l.rope, rope_len, seqlens, cache, s));
-    return nc_launch_window_attention(dt, g, proj, ldp, cache, l.sink, seqlens, cat, ld_cat, w.att_parts, w.att_part_bytes, s);
+    return nc_launch_window_attention(dt, g, proj, ldp, cache, l.sink, seqlens, cat, ld_cat, w.att_parts, w.att_part_bytes, ahead, s);
 }
 
 int run_retention(int dt, const nc_stack_mixer& l, const NcRetentionGeom& g, const Workspace& w, const void* proj, int ldp, float eps, int rope_len,
-                  const int32_t* seqlens, const float* state_in, float* state_out, void* cat, int ld_cat, hipStream_t s) {
-    TRY(nc_launch_retention(dt, g, proj, ldp, l.decay, l.rope, rope_len, seqlens, state_in, state_out, eps, cat, ld_cat, w.ret, s));
+                  const int32_t* seqlens, const float* state_in, float* state_out, void* cat, int ld_cat, const NcAhead* ahead, hipStream_t s) {
+    TRY(nc_launch_retention(dt, g, proj, ldp, l.decay, l.rope, rope_len, seqlens, state_in, state_out, eps, cat, ld_cat, w.ret, ahead, s));
     if (!g.raw) return 0;
     const void* gate = at(proj, (int64_t)l.heads * (2 * l.dim_p + l.vdim_p), dt);
     return nc_launch_joint_gate(dt, g.raw, l.heads * l.vdim_p, l.heads * l.vdim, gate, ldp, l.out_norm_w, eps, l.out_scale, cat, ld_cat, g.B * g.T, s);
 }
 
 int run_selective_scan(int dt, const nc_stack_mixer& l, const NcScanGeom& g, const Workspace& w, const void* proj, int ldp, const int32_t* seqlens,
-                       const float* state_in, float* state_out, void* cat, int ld_cat, hipStream_t s) {
+                       const float* state_in, float* state_out, void* cat, int ld_cat, const NcAhead* ahead, hipStream_t s) {
     const int M = g.B * g.T, N = scan_x_cols(l), splits = scan_x_splits(dt, l, M);
     TRY(nc_launch_scan_conv(dt, g, proj, ldp, l.conv_w, l.conv_b, seqlens, state_in, state_out, w.u, s));
     NcLinear x = nc_linear(w.u, l.inner_p, l.w_x, M, N, l.inner_p);
@@ -230,37 +230,62 @@ int run_selective_scan(int dt, const nc_stack_mixer& l, const NcScanGeom& g, con
     NcLinear d = nc_linear(w.dtr, l.dt_rank_p, l.w_dt, M, l.inner_p, l.dt_rank_p);
     nc_linear_seg(d, d.N, NC_SEG_SOFTPLUS, w.dt, l.inner_p, 0.f, 0.f, l.dt_b);
     TRY(nc_launch_linear(dt, d, s));
-    return nc_launch_scan(dt, g, w.u, w.dt, w.bc, l.a_log2, l.skip, z, ldp, seqlens, state_in, state_out, cat, ld_cat, w.ret, s);
+    return nc_launch_scan(dt, g, w.u, w.dt, w.bc, l.a_log2, l.skip, z, ldp, seqlens, state_in, state_out, cat, ld_cat, w.ret, ahead, s);
 }
 
 // The mixers of one layer run, on the projected rows w.proj, into w.cat.
-int run_mixers(const nc_stack_model* m, const nc_stack_cache* kv, const nc_stack_run& run, const Workspace& w, int B, int T, hipStream_t s) {
+int run_mixers(const nc_stack_model* m, const nc_stack_cache* kv, const nc_stack_run& run, const Workspace& w, int B, int T, const NcAhead& weights, hipStream_t s) {
     const nc_stack_layer& l = m->layers[run.layer];
     const int dt = m->dtype;
     int col = 0, to = 0;
     for (int j = 0; j < l.n_mixers; j++) {
         const nc_stack_mixer& x = l.mix[j];
         const int slot = run.slot[j];
+        const NcAhead* const ahead = j + 1 == l.n_mixers ? &weights : nullptr;
         void *proj = at(w.proj, col, dt), *cat = at(w.cat, to, dt);
         switch (x.kind) {
             case NC_MIXER_LATENT_ATTENTION:
                 TRY(run_latent_attention(dt, x, latent_geom(x, B, T, kv->max_seq_len, kv->pos_max), w, proj, l.mix_cols, m->eps, m->rope_len, kv->cache_seqlens,
-                                         kv->rows[slot], cat, l.k_out, s));
+                                         kv->rows[slot], cat, l.k_out, ahead, s));
                 break;
             case NC_MIXER_RETENTION:
                 TRY(run_retention(dt, x, retention_geom(x, B, T, x.gate == NC_GATE_JOINT_NORM_SIGMOID ? w.raw : nullptr), w, proj, l.mix_cols, m->eps, m->rope_len,
-                                  kv->cache_seqlens, kv->state_in[slot], kv->state_out[slot], cat, l.k_out, s));
+                                  kv->cache_seqlens, kv->state_in[slot], kv->state_out[slot], cat, l.k_out, ahead, s));
                 break;
             case NC_MIXER_WINDOW_ATTENTION:
                 TRY(run_window_attention(dt, x, window_geom(x, B, T, kv->max_seq_len, kv->pos_max), w, proj, l.mix_cols, m->eps, m->rope_len, kv->cache_seqlens,
-                                         kv->rows[slot], cat, l.k_out, s));
+                                         kv->rows[slot], cat, l.k_out, ahead, s));
                 break;
             default:
-                TRY(run_selective_scan(dt, x, scan_geom(x, B, T), w, proj, l.mix_cols, kv->cache_seqlens, kv->state_in[slot], kv->state_out[slot], cat, l.k_out, s));
+                TRY(run_selective_scan(dt, x, scan_geom(x, B, T), w, proj, l.mix_cols, kv->cache_seqlens, kv->state_in[slot], kv->state_out[slot], cat, l.k_out, ahead, s));
         }
         col += x.cols, to += x.out;
     }
     return 0;
+}
+// What a prompt's last mixer reads ahead (nc_prefetch.h): the output matrix, and a dense layer's next input matrix, as far as the memory brings them while the
+// mixer of M rows runs.  us a linear, weights in HBM / in the last-level cache: 1792 rows, 12544 x 2048 107 / 95, 2048 x 4096 45 / 34, 2048 x 8192 81 / 60, 300
+// rows, 6144 x 2048 25 / 16; 32-bit products gain nothing.  us a prompt, without / with: Palilix of width 2048, 1792 tokens, 3648 / 3547, of dense layers, 500
+// tokens, 1175 / 1066 (32 or 64 KB a row, which leaves the input matrix out: 1175), Zodirax of width 2048, 800 tokens, 2285 / 2248.
+// Beginnings of what does not fit (experts, Zodirax's feed-forward) cost the mixers more than they gave: 3648 -> 3770.
+constexpr size_t AHEAD_BYTES_PER_ROW = 98304;
+NcAhead weights_behind(const nc_stack_model* m, int i, int M) {
+    NcAhead a{};
+    if (m->dtype || M <= NC_FEW_ROWS) return a;
+    const nc_stack_layer& l = m->layers[m->runs[i].layer];
+    const size_t W = m->width_p;
+    // whole matrices only: the tiles of a launch start all over its matrix
+    size_t left = (size_t)M * AHEAD_BYTES_PER_ROW;
+    auto add = [&](const void* p, size_t elems) {
+        if (2 * elems <= left) a.add(p, 2 * elems), left -= 2 * elems;
+    };
+    // (the scans and recurrences of a wide post-norm layer keep the memory busy themselves: width 4096 4280 with its 34 and 67 MB, 4275 without)
+    if (l.block != NC_BLOCK_POST_NORM || 2 * W * l.k_out <= 24u << 20) add(l.w_out, W * l.k_out);
+    if (l.block != NC_BLOCK_POST_NORM && l.ff != NC_FF_EXPERTS && i + 1 < m->n_runs) {
+        const nc_stack_layer& next = m->layers[m->runs[i + 1].layer];
+        add(next.w_in, (size_t)next.n_in * W);
+    }
+    return a;
 }
 // The columns of the input matrix that are the mixers' own.
 void mixer_segs(const nc_stack_layer& l, NcLinear& in, const Workspace& w, int dt) {
@@ -417,7 +442,7 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
         if (l.router_cols) nc_linear_seg(in, l.mix_cols + l.router_cols, NC_SEG_F32, w.router, l.router_cols);
         if (!post && l.ff_cols) nc_linear_seg(in, l.n_in, ff_seg_kind(l.ff), at(w.cat, l.mix_out, dt), l.k_out, l.ff_limit);
         TRY(nc_launch_linear(dt, in, s));
-        TRY(run_mixers(m, kv, run, w, B, T, s));
+        TRY(run_mixers(m, kv, run, w, B, T, weights_behind(m, i, M), s));
 
         NcRowAdd add{};
         add.x = w.x, add.tokens_per_row = T;
@@ -434,7 +459,9 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
                 add.post_norm_w = l.norm2_w, add.h = nullptr;
             }
         } else {
-            if (l.ff == NC_FF_EXPERTS) TRY(run_experts(dt, l, M, Wp, w, s));
+            // a prompt's output matrix before the experts, whose weights would push it out of the last-level cache again
+            const bool few = M <= NC_FEW_ROWS;
+            if (l.ff == NC_FF_EXPERTS && few) TRY(run_experts(dt, l, M, Wp, w, s));
             if (nc_linear_splits(dt, M, Wp, l.k_out) > 1) {
                 TRY(run_sums(dt, w.cat, l.w_out, M, Wp, l.k_out, w.parts, add, s));
             } else {
@@ -442,6 +469,7 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
                 nc_linear_seg(out, Wp, NC_SEG_RESIDUAL, w.x, Wp);
                 TRY(nc_launch_linear(dt, out, s));
             }
+            if (l.ff == NC_FF_EXPERTS && !few) TRY(run_experts(dt, l, M, Wp, w, s));
             if (l.ff == NC_FF_EXPERTS) add.expert_out = w.e_out, add.slot_of = w.slot_of, add.slot_w = w.slot_w, add.top = l.top;
         }
         if (taps) add.tap = taps + (int64_t)i * M * Wp;

@@ -445,12 +445,13 @@ __global__ __launch_bounds__(64) void window_combine_kernel(const float* __restr
 template <int DQ, int DV, int NQ, int KS>
 __global__ __launch_bounds__(64 * NQ * KS) __attribute__((amdgpu_waves_per_eu(2, 2))) void window_prefill_kernel(
     NcWindowGeom g, const bf16_t* __restrict__ q, int ldq, const bf16_t* __restrict__ cache, const float* __restrict__ sink,
-    const int32_t* __restrict__ seqlens, bf16_t* __restrict__ out, int ldo) {
+    const int32_t* __restrict__ seqlens, bf16_t* __restrict__ out, int ldo, NcAhead ahead) {
     constexpr int KPITCH = DQ * 2 + 16, VPITCH = DV * 2 + 64, NW = NQ * KS, NTHR = 64 * NW, KB = 16 * NW, QT = 32 * NQ;
     constexpr int KCH = DQ / 8, VCH = DV / 8, KL = KB * KCH / NTHR, VL = KB * VCH / NTHR;
     constexpr int STAGE = KB * KPITCH + KB * VPITCH, O_PITCH = DV + 4, SUM = KS > 1 ? NQ * 32 * (O_PITCH + 2) * 4 : 0;
     static_assert(KS == 1 || (KS == 2 && KB >= 64), "every wave has a block of a stage");
     __shared__ __align__(16) uint8_t lds[STAGE > SUM ? STAGE : SUM];
+    if (reads_ahead<NTHR>(ahead, g.B)) return;
     uint8_t* const lds_v = lds + KB * KPITCH;
     const lds_u8_t lds_v3 = (lds_u8_t)lds + KB * KPITCH;
     const int b = blockIdx.z;
@@ -654,11 +655,11 @@ int launch_few(const NcWindowGeom& g, const bf16_t* q, int ldq, const bf16_t* ca
 }
 template <int DQ, int DV>
 int launch_prefill(const NcWindowGeom& g, const bf16_t* q, int ldq, const bf16_t* cache, const float* sink, const int32_t* seqlens, bf16_t* out, int ldo,
-                   hipStream_t s) {
+                   const NcAhead* ahead, hipStream_t s) {
     if ((int64_t)((g.T + 127) / 128) * g.heads * g.B >= 2 * nc_cu_count())
-        hipLaunchKernelGGL((window_prefill_kernel<DQ, DV, 4, 1>), dim3((g.T + 127) / 128, g.heads, g.B), dim3(256), 0, s, g, q, ldq, cache, sink, seqlens, out, ldo);
+        hipLaunchKernelGGL((window_prefill_kernel<DQ, DV, 4, 1>), nc_ahead_grid(dim3((g.T + 127) / 128, g.heads, g.B), ahead), dim3(256), 0, s, g, q, ldq, cache, sink, seqlens, out, ldo, ahead ? *ahead : NcAhead{});
     else
-        hipLaunchKernelGGL((window_prefill_kernel<DQ, DV, 2, 2>), dim3((g.T + 63) / 64, g.heads, g.B), dim3(256), 0, s, g, q, ldq, cache, sink, seqlens, out, ldo);
+        hipLaunchKernelGGL((window_prefill_kernel<DQ, DV, 2, 2>), nc_ahead_grid(dim3((g.T + 63) / 64, g.heads, g.B), ahead), dim3(256), 0, s, g, q, ldq, cache, sink, seqlens, out, ldo, ahead ? *ahead : NcAhead{});
     NC_CHECK_LAUNCH("window_prefill");
     return 0;
 }
@@ -687,7 +688,7 @@ size_t nc_window_partial_bytes(int dtype, const NcWindowGeom& g) {
 }
 
 int nc_launch_window_attention(int dtype, const NcWindowGeom& g, const void* q, int ldq, const void* cache, const float* sink, const int32_t* seqlens, void* out,
-                               int ldo, void* partials, size_t partial_bytes, hipStream_t s) {
+                               int ldo, void* partials, size_t partial_bytes, const NcAhead* ahead, hipStream_t s) {
     NC_CHECK_ARG(g.kv_heads >= 1 && g.heads % g.kv_heads == 0 && g.window >= 1 && g.keep_first >= 0, "window_attention: %d of %d heads, window %d, first %d",
                  g.kv_heads, g.heads, g.window, g.keep_first);
     NC_CHECK_ARG(g.dim_p % 32 == 0 && g.vdim_p % 16 == 0 && ldq % 8 == 0 && ldo % 4 == 0 && sink && g.pos_max + g.T <= g.Tmax, "window_attention: sizes");
@@ -703,7 +704,7 @@ int nc_launch_window_attention(int dtype, const NcWindowGeom& g, const void* q, 
         bf16_t* o = (bf16_t*)out;
         const int splits = few ? few_splits(g) : 1;
         NC_CHECK_ARG(splits == 1 || (partials && partial_bytes >= nc_window_partial_bytes(dtype, g)), "window_attention: partial buffer too small");
-#define GO(Q, V) (few ? launch_few<Q, V>(g, qq, ldq, c, sink, seqlens, o, ldo, (float*)partials, splits, s) : launch_prefill<Q, V>(g, qq, ldq, c, sink, seqlens, o, ldo, s))
+#define GO(Q, V) (few ? launch_few<Q, V>(g, qq, ldq, c, sink, seqlens, o, ldo, (float*)partials, splits, s) : launch_prefill<Q, V>(g, qq, ldq, c, sink, seqlens, o, ldo, ahead, s))
 #define GO_V(Q) (g.vdim_p <= 64 ? GO(Q, 64) : GO(Q, 128))
         if (g.dim_p <= 64) return GO_V(64);
         if (g.dim_p <= 128) return GO_V(128);
