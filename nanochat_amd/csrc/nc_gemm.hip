@@ -737,6 +737,90 @@ __device__ __forceinline__ void dl_step_barrier() {
     asm volatile("" ::: "memory");
 }
 
+// The K loop of the tiles that are launched one by one: eight waves in a 4 x 2 grid.  One operand is HELD, four blocks of 16 rows per wave whose fragments are
+// read a step ahead into registers of their own, through a ring of three stages; the other is STREAMED, NS blocks per wave, each read one group of
+// products ahead of its use, through two stages.  With both operands read behind the barrier a step began with ten LDS reads per wave (80 KB a workgroup,
+// 640 clocks) that nothing overlapped; now with two, the held operand's loads have two steps to arrive, and the loads go out between the products.  us, before /
+// after: 8192 x 1664 x 6656 112.7 / 107.5 in 256 x 192 tiles, 85.5 / 82 in 256 x 256 ones; of thirteen steps 1792 x 4992 x 1664 19.9 / 20.0, 1792 x 6656 x 1664
+// 22.0 / 21.9: what is left there is the launch, the first loads and the write.  Same products in the same order.
+//   A_HELD: rows of A in the grid's first direction (acc[held][streamed]), else rows of B in the second (acc[streamed][held]).
+//   HP: held pieces of 1 KB per wave and step: what may still be in flight when a step ends, while there is a step three ahead to load.
+__device__ __forceinline__ void dl_piece(const uint8_t* p, int bytes, uint8_t* st, uint32_t vo, int k_off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00020000), (lds_ptr_t)st, 16, vo, k_off, 0, 0);
+}
+template <bool A_HELD, int NS> constexpr int dl_stream_stage() { return (A_HELD ? 32 : 64) * NS * 128; }
+template <bool A_HELD, int NS, int HP> constexpr int dl_ring_lds() { return 3 * HP * 8192 + 2 * dl_stream_stage<A_HELD, NS>(); }
+template <bool A_HELD, int NS, int HP, int A_FMT, typename Acc>
+__device__ __forceinline__ void dl_ring(Acc& acc, const uint8_t* A, int a_bytes, const uint8_t* B, int b_bytes, uint8_t* lds, const DlGeom& g, int wave_s,
+                                        const uint32_t* vo_h, const uint32_t* vo_s, int ksteps) {
+    constexpr int H_ST = HP * 8192, S_ST = dl_stream_stage<A_HELD, NS>(), S_PIECES = S_ST / 1024, S_ROUNDS = (S_PIECES + 7) / 8, WAIT = 0x0070 | HP;
+    uint8_t* const ring_s = lds + 3 * H_ST;
+    const int rd_h = (A_HELD ? g.wm : g.wn) * 64 * 128, rd_s = (A_HELD ? g.wn : g.wm) * 16 * NS * 128;
+    // piece r of a step's loads: S_ROUNDS of the streamed operand first, then HP of the held one
+    auto load_h = [&](int r, int t, int at) {
+        if (t < ksteps) dl_piece(A_HELD ? A : B, A_HELD ? a_bytes : b_bytes, lds + at + wave_s * 1024 + r * 8192, vo_h[r], t * 128);
+    };
+    auto load_s = [&](int r, int t, int buf) {
+        if (t < ksteps && (S_PIECES % 8 == 0 || wave_s + 8 * r < S_PIECES))       // uniform per wave
+            dl_piece(A_HELD ? B : A, A_HELD ? b_bytes : a_bytes, ring_s + buf * S_ST + wave_s * 1024 + r * 8192, vo_s[r], t * 128);
+    };
+    auto meet = [&](bool in_flight) {
+        asm volatile("" ::: "memory");
+        if (in_flight) __builtin_amdgcn_s_waitcnt(WAIT);
+        else __builtin_amdgcn_s_waitcnt(0x0070); // the next step's streamed operand and the held one behind it have landed, every fragment is read (this wave's share)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    v8i held[2][4];
+    int at0 = 0, at1 = H_ST, at2 = 2 * H_ST;     // stages of the held operand of this step, the next and the one after
+    auto step = [&](int t, auto parity) __attribute__((always_inline)) {
+        constexpr int P = decltype(parity)::value, Q = 1 - P;
+        const uint8_t* const ss = ring_s + P * S_ST + rd_s;
+        const uint8_t* const hs = lds + at1 + rd_h;
+        v8i sf[2];
+        sf[0] = dl_frag(ss, g);
+#pragma unroll
+        for (int j = 0; j < NS; j++) {
+            if (j + 1 < NS) sf[(j + 1) & 1] = dl_frag(ss + (j + 1) * 2048, g);    // one group ahead of its use
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (i * NS / 4 == j) held[Q][i] = dl_frag(hs + i * 2048, g);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+#pragma unroll
+                for (int r = 0; r < S_ROUNDS + HP; r++)
+                    if (r * 4 * NS / (S_ROUNDS + HP) == 4 * j + i) {
+                        if (r < S_ROUNDS) load_s(r, t + 1, Q);
+                        else load_h(r - S_ROUNDS, t + 3, at0);
+                    }
+                if constexpr (A_HELD) mfma_f8_acc_ordered<A_FMT>(acc[i][j], sf[j & 1], held[P][i]);
+                else mfma_f8_acc_ordered<A_FMT>(acc[j][i], held[P][i], sf[j & 1]);
+            }
+        }
+        meet(t + 3 < ksteps);
+        const int first = at0;
+        at0 = at1, at1 = at2, at2 = first;
+    };
+#pragma unroll
+    for (int r = 0; r < S_ROUNDS; r++) load_s(r, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 3 * HP; r++) load_h(r % HP, r / HP, r / HP * H_ST);
+    asm volatile("" ::: "memory");
+    if (ksteps > 2) __builtin_amdgcn_s_waitcnt(0x0070 | (2 * HP));       // the first step's operands
+    else __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 4; i++) held[0][i] = dl_frag(lds + at0 + rd_h + i * 2048, g);
+    meet(ksteps > 2);
+    int kt = 0;
+    for (; kt + 1 < ksteps; kt += 2) {
+        step(kt, std::integral_constant<int, 0>{});
+        step(kt + 1, std::integral_constant<int, 1>{});
+    }
+    if (kt < ksteps) step(kt, std::integral_constant<int, 0>{});
+}
+
 // One tile per workgroup, launched tile by tile (any M, N).
 template <int A_FMT, int OUT_KIND>
 __global__ __launch_bounds__(512) void gemm_dl_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, EpilogueArgs ep, int M,
@@ -775,18 +859,23 @@ __global__ __launch_bounds__(512) void gemm_dl_kernel(const uint8_t* __restrict_
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(i < 4 ? desc_a : desc_b, (lds_ptr_t)(st + i * 8192), 16, vo[i], t * 128, 0, 0);
         }
     };
-    // step kt computes from buffer kt & 1 while the loads of step kt + 1 land in the other one; the barrier at its end
-    // says both that those loads are complete for every wave and that nobody reads buffer kt & 1 any more
-    fetch(0, 0);
-    dl_step_barrier();
-    int kt = 0;
-    for (; kt + 1 < ksteps; kt += 2) {
-        dl_compute<false, false, A_FMT>(acc, lds, g, [&] { fetch(kt + 1, 1); });
+    if constexpr (OUT_KIND == 0) {
+        dl_ring<true, 8, 4, A_FMT>(acc, A, M * K, B, N * K, lds, g, wave_s, vo, vo + 4, ksteps);
+    } else {
+        // (no room for the third stage beside the words of the other epilogues)
+        // step kt computes from buffer kt & 1 while the loads of step kt + 1 land in the other one; the barrier at its end
+        // says both that those loads are complete for every wave and that nobody reads buffer kt & 1 any more
+        fetch(0, 0);
         dl_step_barrier();
-        dl_compute<false, false, A_FMT>(acc, lds + STAGE, g, [&] { fetch(kt + 2, 0); });
-        dl_step_barrier();
+        int kt = 0;
+        for (; kt + 1 < ksteps; kt += 2) {
+            dl_compute<false, false, A_FMT>(acc, lds, g, [&] { fetch(kt + 1, 1); });
+            dl_step_barrier();
+            dl_compute<false, false, A_FMT>(acc, lds + STAGE, g, [&] { fetch(kt + 2, 0); });
+            dl_step_barrier();
+        }
+        if (kt < ksteps) dl_compute<false, false, A_FMT>(acc, lds, g);
     }
-    if (kt < ksteps) dl_compute<false, false, A_FMT>(acc, lds, g);
 
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
@@ -805,24 +894,6 @@ __global__ __launch_bounds__(512) void gemm_dl_kernel(const uint8_t* __restrict_
 // The same tile-by-tile kernel with a narrower tile: 256 rows x 32 NJ columns (NJ = 4 .. 7 blocks of 16 columns per wave).  A launch of
 // one round -- a prompt of one to two thousand rows -- lasts as long as one tile, whatever the number of CUs that got one: 1792 x 4992
 // is 140 tiles of 256 x 256 on 256 CUs, but 224 tiles of 256 x 160, each 5/8 of the matrix work.  The launch picks NJ (dl_pick_nj).
-// A wave's B pieces beyond the tile's 32 NJ rows are not loaded (the test is uniform per wave), the stage is 256 + 32 NJ rows.
-template <int NJ, int A_FMT = 0, typename F = DlNothing>
-__device__ __forceinline__ void dln_compute(v4f (&acc)[4][NJ], const uint8_t* st, const DlGeom& g, F&& behind_first_reads = F()) {
-    const uint8_t* a = st + g.wm * 64 * 128;
-    const uint8_t* b = st + 256 * 128 + g.wn * (16 * NJ) * 128;
-    v8i af[4], bf[2];
-    bf[0] = dl_frag(b, g);
-#pragma unroll
-    for (int i = 0; i < 4; i++) af[i] = dl_frag(a + i * 2048, g);
-    behind_first_reads();
-#pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        if (j + 1 < NJ) bf[(j + 1) & 1] = dl_frag(b + (j + 1) * 2048, g);    // one group ahead of its use
-#pragma unroll
-        for (int i = 0; i < 4; i++) mfma_f8_acc_ordered<A_FMT>(acc[i][j], bf[j & 1], af[i]);
-    }
-}
-
 // Epilogue for a wave block of 64 x 16 NJ outputs, bf16 (RELU2: relu(v)^2 and its maximum): the block is parked in the wave's own
 // LDS region (rows of 32 NJ + 16 bytes) and leaves as a linear sequence of 16-byte pieces, so a store instruction writes runs of
 // 32 NJ contiguous bytes per row.
@@ -892,24 +963,10 @@ __device__ __forceinline__ void dln_epilogue(v4f (&acc)[4][NJ], uint8_t* lds, co
     }
 }
 
-// the operand loads of one K-step: `st` is the wave's first 1 KB piece of the stage (uniform: the LDS address of a load goes through M0)
-template <int NJ>
-__device__ __forceinline__ void dln_fetch(const uint8_t* A, int a_bytes, const uint8_t* B, int b_bytes, uint8_t* st, const uint32_t* vo_a,
-                                          const uint32_t* vo_b, int wave_s, int k_off) {
-    const __amdgpu_buffer_rsrc_t desc_a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, a_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t desc_b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, b_bytes, 0x00020000);
-#pragma unroll
-    for (int i = 0; i < 4; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_a, (lds_ptr_t)(st + i * 8192), 16, vo_a[i], k_off, 0, 0);
-#pragma unroll
-    for (int i = 0; i < (4 * NJ + 7) / 8; i++)
-        if (wave_s + 8 * i < 4 * NJ)                      // uniform per wave
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_b, (lds_ptr_t)(st + 256 * 128 + i * 8192), 16, vo_b[i], k_off, 0, 0);
-}
-
 template <int NJ, int OUT_KIND, int A_FMT = 0>
 __global__ __launch_bounds__(512) void gemm_dln_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, EpilogueArgs ep, int M,
                                                        int N, int K, int tiles_m, int tiles_n) {
-    constexpr int BN = 32 * NJ, STAGE = (256 + BN) * 128, B_PIECES = BN / 8, B_ROUNDS = (B_PIECES + 7) / 8;
+    constexpr int BN = 32 * NJ, B_ROUNDS = (BN / 8 + 7) / 8;
     extern __shared__ __align__(16) uint8_t lds[];
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
@@ -937,19 +994,7 @@ __global__ __launch_bounds__(512) void gemm_dln_kernel(const uint8_t* __restrict
 #pragma unroll
         for (int j = 0; j < NJ; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-    auto fetch = [&](int t, int buf) {
-        if (t < ksteps) dln_fetch<NJ>(A, M * K, B, N * K, lds + buf * STAGE + wave_s * 1024, vo_a, vo_b, wave_s, t * 128);
-    };
-    fetch(0, 0);
-    dl_step_barrier();
-    int kt = 0;
-    for (; kt + 1 < ksteps; kt += 2) {
-        dln_compute<NJ, A_FMT>(acc, lds, g, [&] { fetch(kt + 1, 1); });
-        dl_step_barrier();
-        dln_compute<NJ, A_FMT>(acc, lds + STAGE, g, [&] { fetch(kt + 2, 0); });
-        dl_step_barrier();
-    }
-    if (kt < ksteps) dln_compute<NJ, A_FMT>(acc, lds, g);
+    dl_ring<true, NJ, 4, A_FMT>(acc, A, M * K, B, N * K, lds, g, wave_s, vo_a, vo_b, ksteps);
 
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
@@ -967,18 +1012,9 @@ __global__ __launch_bounds__(512) void gemm_dln_kernel(const uint8_t* __restrict
 // The same once more with tiles of 64 WTM rows x 128 columns (WTM = 2 .. 6 blocks of 16 rows per wave): whole heads of the q|k|v linear, for rope_epilogue.  The
 // 320-row tile has the area of the 256 x 160 one.
 template <int WTM>
-__device__ __forceinline__ void rope_fetch(const uint8_t* A, int a_bytes, const uint8_t* B, int b_bytes, uint8_t* st, const uint32_t* vo_a, const uint32_t* vo_b, int k_off) {
-    const __amdgpu_buffer_rsrc_t desc_a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, a_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t desc_b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, b_bytes, 0x00020000);
-#pragma unroll
-    for (int i = 0; i < WTM; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_a, (lds_ptr_t)(st + i * 8192), 16, vo_a[i], k_off, 0, 0);
-#pragma unroll
-    for (int i = 0; i < 2; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_b, (lds_ptr_t)(st + WTM * 8192 + i * 8192), 16, vo_b[i], k_off, 0, 0);
-}
-template <int WTM>
 __global__ __launch_bounds__(512) void gemm_rope_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, EpilogueArgs ep, RopeArgs rope, int M, int N,
                                                         int K, int tiles_m, int tiles_n) {
-    constexpr int BM = 64 * WTM, STAGE = (BM + 128) * 128;
+    constexpr int BM = 64 * WTM;
     extern __shared__ __align__(16) uint8_t lds[];
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
@@ -1003,34 +1039,7 @@ __global__ __launch_bounds__(512) void gemm_rope_kernel(const uint8_t* __restric
     for (int i = 0; i < WTM; i++)
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    auto fetch = [&](int t, int buf) {
-        if (t < ksteps) rope_fetch<WTM>(A, M * K, B, N * K, lds + buf * STAGE + wave_s * 1024, vo_a, vo_b, t * 128);
-    };
-    auto compute = [&](const uint8_t* st, int t, int buf) {
-        const uint8_t* a = st + g.wm * (16 * WTM) * 128;
-        const uint8_t* b = st + BM * 128 + g.wn * 64 * 128;
-        v8i bf[4], af[2];
-        af[0] = dl_frag(a, g);
-#pragma unroll
-        for (int j = 0; j < 4; j++) bf[j] = dl_frag(b + j * 2048, g);
-        fetch(t, buf);
-#pragma unroll
-        for (int i = 0; i < WTM; i++) {
-            if (i + 1 < WTM) af[(i + 1) & 1] = dl_frag(a + (i + 1) * 2048, g);    // one group ahead of its use
-#pragma unroll
-            for (int j = 0; j < 4; j++) mfma_f8_acc_ordered<0>(acc[i][j], bf[j], af[i & 1]);
-        }
-    };
-    fetch(0, 0);
-    dl_step_barrier();
-    int kt = 0;
-    for (; kt + 1 < ksteps; kt += 2) {
-        compute(lds, kt + 1, 1);
-        dl_step_barrier();
-        compute(lds + STAGE, kt + 2, 0);
-        dl_step_barrier();
-    }
-    if (kt < ksteps) compute(lds, ksteps, 0);
+    dl_ring<false, WTM, 2, 0>(acc, A, M * K, B, N * K, lds, g, wave_s, vo_b, vo_a, ksteps);
 
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
@@ -1059,8 +1068,9 @@ __device__ __forceinline__ void dr_load(const uint8_t* A, int a_bytes, const uin
 // ring of FOUR operand stages.  Where the 256-row tiles would leave most CUs without one (1792 x 1664: 49 or 91 tiles), the launch is
 // one round of small tiles, one workgroup of one wave per SIMD on each CU: nothing hides the latency of a K-step's operands then but
 // the depth of the prefetch.  The register-staged tiles have two K-steps in flight and pay a ds_write phase per step; here the operands
-// of three steps ahead are on their way into LDS while one is multiplied, and a step costs its MFMAs or the L2's bandwidth, whichever
-// is longer.  Past the end of K the loads are issued all the same (the first step's operands again, into stages nobody reads), so that
+// of four steps ahead are on their way into LDS while one is multiplied from registers that were filled during the step before, and a step costs its
+// loads (28 KB at some 35 bytes a clock for 96 x 128) or its products, whichever is longer: 0.40 -> 0.33 us a step by the second set of registers.  Past
+// the end of K the loads are issued all the same (the first step's operands again, into stages nobody reads), so that
 // the count the barrier waits for is the same in every step.
 //
 // OUT_KIND 3: the K-steps are dealt to gridDim.y workgroups per tile, which leave raw fp32 sums ([share][M][N] at ep.out) for the row pass
@@ -1408,7 +1418,7 @@ static bool dlp_eligible(int M, int /*N*/, int K) {
 template <int A_FMT, int OUT_KIND>
 static int launch_dl_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, bool persistent, hipStream_t s) {
     const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
-    const size_t lds_bytes = 2 * 512 * 128 + (persistent ? 8 * 4096 : 0);
+    const size_t lds_bytes = persistent ? 2 * 512 * 128 + 8 * 4096 : OUT_KIND == 0 ? dl_ring_lds<true, 8, 4>() : 2 * 512 * 128;
     const void* fn = persistent ? (const void*)gemm_dlp_kernel<A_FMT, OUT_KIND == 2> : (const void*)gemm_dl_kernel<A_FMT, OUT_KIND>;
     hipError_t e = reserve_lds(fn, (int)lds_bytes);
     if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
@@ -1456,7 +1466,7 @@ static bool dl_narrow_fills(int M, int N) {
 template <int NJ, int OUT_KIND, int A_FMT>
 static int launch_dln_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s) {
     const int tiles_m = (M + 255) / 256, tiles_n = (N + 32 * NJ - 1) / (32 * NJ);
-    const size_t lds_bytes = 2 * (256 + 32 * NJ) * 128;
+    const size_t lds_bytes = dl_ring_lds<true, NJ, 4>();
     const void* fn = (const void*)gemm_dln_kernel<NJ, OUT_KIND, A_FMT>;
     hipError_t e = reserve_lds(fn, (int)lds_bytes);
     if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
@@ -1565,8 +1575,7 @@ static int pick_kernel(int M, int N, int K, int out_kind) {
                 if ((long)((M + 63) / 64) * tn <= cus) which = 10;
                 else if ((long)((M + 95) / 96) * tn <= cus) which = 11;
                 // the same tiles fed straight into a ring of four LDS stages where K allows it: three K-steps of operands on their
-                // way instead of two and no ds_write phase (1792 x 1664 x 6656: 27.5 -> 25.6 us, 1024 rows: 21.9 -> 20.8 us; what is
-                // left is the L2's bandwidth: 28 KB per K-step and CU for tiles this small)
+                // way instead of two and no ds_write phase (1792 x 1664 x 6656: 27.5 -> 21.3 us, 1000 rows: 21.9 -> 17.1 us)
                 if (which >= 10 && K % 128 == 0 && out_kind != 1) which += 6;
             }
         }
@@ -1679,7 +1688,7 @@ static int rope_tiles(int M, int N, int K) {
 template <int WTM>
 static int launch_gemm_rope(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, const RopeArgs& rope, int M, int N, int K, hipStream_t s) {
     const int tiles_m = (M + 64 * WTM - 1) / (64 * WTM), tiles_n = N / 128;
-    const size_t lds_bytes = 2 * (64 * WTM + 128) * 128;
+    const size_t lds_bytes = dl_ring_lds<false, WTM, 2>();
     const hipError_t e = reserve_lds((const void*)gemm_rope_kernel<WTM>, (int)lds_bytes);
     if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
     hipLaunchKernelGGL(gemm_rope_kernel<WTM>, dim3(tiles_m * tiles_n), dim3(512), lds_bytes, s, a, b, ep, rope, M, N, K, tiles_m, tiles_n);
