@@ -462,6 +462,148 @@ __global__ __launch_bounds__(64 * WM * WN) void linear_tiled_kernel(NcLinear g, 
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// 256 x 256 outputs of many bf16 rows, eight waves of 64 x 128 (4 x 2): a K-step of 128 bytes asks the LDS for 196 KB of fragments and 64 KB of operands beside
+// 2048 clocks of products, where the 128 x 256 tiles ask for 131 + 48 KB beside 1024: those run at the rate of the LDS, these at that of the products.
+// The rows go through a ring of three stages and are read a step ahead into registers of their own, the weight through two stages, read one group of
+// products ahead (160 KB in all; three stages of both do not fit).  What is left of the tiles behind whole rounds over the compute units is cut into halves
+// of 256 x 128 where those fit one round: 1792 rows are 7 tiles of 256, and rounds of whole tiles alone would lose what they gain.  Same products in the same
+// order as in linear_tiled_kernel.  us, 128 x 256 tiles / these: 1792 x 21760 x 4096 291 / 258, x 22528 290 / 260, x 8192 106 / 92, 1792 x 12544 x 2048 91 / 81, x
+// 7936 58 / 51, 4096^3 112 / 99.5 (1.38 PFLOP/s; a large product of the library's 1.23).
+struct BigFrag {
+    v4i lo, hi;
+};
+template <int NS>
+__device__ __forceinline__ void big_tile(const NcLinear& g, int m0, int n0, uint32_t a_bytes, uint8_t* lds) {
+    constexpr int A_ST = 256 * 128, W_ST = 32 * NS * 128, W_P = NS / 2, HP = 4, WCOLS = 16 * NS;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wm = wave >> 1, wn = wave & 1, frow = lane & 15, piece = lane >> 4;
+    const int sub = lane >> 3, gch = (lane & 7) ^ sub ^ (wave & 1);
+    const int rd_lo = frow * 128 + ((2 * piece ^ TILE_SWZ(frow)) << 4), rd_hi = frow * 128 + (((2 * piece + 1) ^ TILE_SWZ(frow)) << 4);
+    const uint32_t row_a = (uint32_t)g.lda * 2, row_w = (uint32_t)g.ldw * 2;
+    const int ksteps = g.K / 64;
+    const uint8_t* const A = (const uint8_t*)g.a;
+    const uint8_t* const W = (const uint8_t*)((const bf16_t*)g.w + (int64_t)n0 * g.ldw);
+    const uint32_t w_bytes = (uint32_t)(min(g.N - n0, 32 * NS) - 1) * row_w + (uint32_t)g.K * 2;
+    // piece i of this wave is the 1 KB block (wave + 8 i) of its operand's stage
+    uint32_t vo_a[HP], vo_w[W_P];
+#pragma unroll
+    for (int i = 0; i < HP; i++) {
+        const int r = m0 + 8 * wave + 64 * i + sub;
+        vo_a[i] = r < g.M ? (uint32_t)r * row_a + gch * 16 : TILE_OOB;
+    }
+#pragma unroll
+    for (int i = 0; i < W_P; i++) {
+        const int r = 8 * wave + 64 * i + sub;
+        vo_w[i] = n0 + r < g.N ? (uint32_t)r * row_w + gch * 16 : TILE_OOB;
+    }
+    v4f acc[4][NS];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < NS; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    uint8_t* const ring_w = lds + 3 * A_ST;
+    auto load_a = [&](int r, int t, int at) {
+        if (t < ksteps) tile_load<false>(A, a_bytes, lds + at + wave * 1024 + r * 8192, vo_a[r], t * 128);
+    };
+    auto load_w = [&](int r, int t, int buf) {
+        if (t < ksteps) tile_load<false>(W, w_bytes, ring_w + buf * W_ST + wave * 1024 + r * 8192, vo_w[r], t * 128);
+    };
+    auto frag = [&](const uint8_t* p) { return BigFrag{*(const v4i*)(p + rd_lo), *(const v4i*)(p + rd_hi)}; };
+    auto meet = [&](bool in_flight) {
+        asm volatile("" ::: "memory");
+        if (in_flight) __builtin_amdgcn_s_waitcnt(0x0070 | HP);      // (the rows of the step three ahead may still be on their way)
+        else __builtin_amdgcn_s_waitcnt(0x0070);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    BigFrag held[2][4];
+    int at0 = 0, at1 = A_ST, at2 = 2 * A_ST;        // stages of the rows of this step, the next and the one after
+    auto step = [&](int t, auto parity) __attribute__((always_inline)) {
+        constexpr int P = decltype(parity)::value, Q = 1 - P, LOADS = W_P + HP, PRODUCTS = 8 * NS;
+        const uint8_t* const ws = ring_w + P * W_ST + wn * WCOLS * 128;
+        const uint8_t* const as = lds + at1 + wm * 64 * 128;
+        BigFrag wf[2];
+        wf[0] = frag(ws);
+#pragma unroll
+        for (int j = 0; j < NS; j++) {
+            if (j + 1 < NS) wf[(j + 1) & 1] = frag(ws + (j + 1) * 2048);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (i * NS / 4 == j) held[Q][i] = frag(as + i * 2048);
+#pragma unroll
+            for (int n = 0; n < 8; n++) {
+                const int i = n & 3;
+#pragma unroll
+                for (int r = 0; r < LOADS; r++)
+                    if (r * PRODUCTS / LOADS == 8 * j + n) {
+                        if (r < W_P) load_w(r, t + 1, Q);
+                        else load_a(r - W_P, t + 3, at0);
+                    }
+                mma_part<bf16_t>(acc[i][j], n < 4 ? wf[j & 1].lo : wf[j & 1].hi, n < 4 ? held[P][i].lo : held[P][i].hi, 0);
+            }
+        }
+        meet(t + 3 < ksteps);
+        const int first = at0;
+        at0 = at1, at1 = at2, at2 = first;
+    };
+#pragma unroll
+    for (int r = 0; r < W_P; r++) load_w(r, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 3 * HP; r++) load_a(r % HP, r / HP, r / HP * A_ST);
+    asm volatile("" ::: "memory");
+    if (ksteps > 2) __builtin_amdgcn_s_waitcnt(0x0070 | (2 * HP));   // the first step's operands
+    else __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 4; i++) held[0][i] = frag(lds + wm * 64 * 128 + i * 2048);
+    meet(ksteps > 2);
+    int kt = 0;
+    for (; kt + 1 < ksteps; kt += 2) {
+        step(kt, std::integral_constant<int, 0>{});
+        step(kt + 1, std::integral_constant<int, 1>{});
+    }
+    if (kt < ksteps) step(kt, std::integral_constant<int, 0>{});
+    // out through LDS, each wave its own part (see linear_tiled_kernel)
+    constexpr int ROW = WCOLS + 4, SUBS = 2, CHUNKS = WCOLS / 8, ROWS_AT_ONCE = 64 / CHUNKS;
+    static_assert(8 * 16 * SUBS * ROW * 4 <= 3 * A_ST + 2 * W_ST, "output staging");
+    float* const own = (float*)lds + wave * 16 * SUBS * ROW;
+    const int c = 8 * (lane % CHUNKS), n = n0 + wn * WCOLS + c;
+    NcSeg sg = g.seg[0];
+    int base = 0;
+#pragma unroll
+    for (int i = 1; i < 4; i++)
+        if (i < g.nseg && n >= g.seg[i - 1].end) sg = g.seg[i], base = g.seg[i - 1].end;
+    if (g.partials) sg = NcSeg{g.N, NC_SEG_F32, g.partials, g.N, 0.f, 0.f, nullptr}, base = 0;
+#pragma unroll
+    for (int i0 = 0; i0 < 4; i0 += SUBS) {
+#pragma unroll
+        for (int i = 0; i < SUBS; i++)
+#pragma unroll
+            for (int j = 0; j < NS; j++) *(v4f*)(own + (16 * i + frow) * ROW + 16 * j + 4 * piece) = acc[i0 + i][j];
+#pragma unroll 1
+        for (int r = lane / CHUNKS; r < 16 * SUBS; r += ROWS_AT_ONCE) {
+            const int m = m0 + wm * 64 + 16 * i0 + r;
+            if (m >= g.M || n >= g.N) break;
+            const float* v = own + r * ROW + c;
+            store_cols8<bf16_t>(sg, g.N, 0, m, n, n - base, *(const v4f*)v, *(const v4f*)(v + 4));
+        }
+    }
+}
+// `full` workgroups with a whole tile, the rest with half a one
+__global__ __launch_bounds__(512) void linear_big_kernel(NcLinear g, int tiles_m, int full, uint32_t a_bytes) {
+    extern __shared__ __align__(16) uint8_t lds[];
+    // every XCD gets a contiguous run of the tiles, and of the halves behind them; a band of TILE_GROUP_M tile rows column by column
+    const bool half = (int)blockIdx.x >= full;
+    const int id = half ? (int)blockIdx.x - full : (int)blockIdx.x, total = half ? (int)gridDim.x - full : full;
+    const int lin = (id & 7) * (total >> 3) + min(id & 7, total & 7) + (id >> 3), tile = half ? full + lin / 2 : lin;
+    const int tiles_n = (g.N + 255) / 256, band = TILE_GROUP_M * tiles_n, first = tile / band * TILE_GROUP_M, rows = min(TILE_GROUP_M, tiles_m - first);
+    const int m0 = (first + tile % band % rows) * 256, n0 = tile % band / rows * 256 + (half ? lin % 2 * 128 : 0);
+    if (n0 >= g.N) return;
+    if (half) big_tile<4>(g, m0, n0, a_bytes, lds);
+    else big_tile<8>(g, m0, n0, a_bytes, lds);
+}
+
 int reserve_dynamic_lds(const void* fn, int bytes, std::atomic<uint64_t>& done) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev > 63) dev = 0;
@@ -518,8 +660,26 @@ int launch_tiled(const NcLinear& l, hipStream_t s) {
     NC_CHECK_LAUNCH("linear_tiled");
     return 0;
 }
+// whole tiles of 256 x 256 of a launch; the others are cut in two where the halves fit half a round
+int big_full_tiles(int64_t tiles) {
+    const int cus = nc_cu_count(), rest = (int)(tiles % cus);
+    return (int)(2 * rest <= cus ? tiles - rest : tiles);
+}
+int launch_big(const NcLinear& l, hipStream_t s) {
+    static std::atomic<uint64_t> done{0};
+    constexpr int LDS = 5 * 256 * 128;
+    if (int rc = reserve_dynamic_lds((const void*)linear_big_kernel, LDS, done)) return rc;
+    const int64_t a_bytes = linear_a_bytes(l, 2);
+    NC_CHECK_ARG(!l.tiles && !l.a_rows && l.batch == 1 && l.splits == 1 && l.K % 64 == 0, "linear: not a product of the 256 x 256 tiles");
+    NC_CHECK_ARG(a_bytes < TILE_BYTES && 256 * l.ldw * 2 < TILE_BYTES, "linear: operand past 2 GiB");
+    const int tm = (l.M + 255) / 256, tn = (l.N + 255) / 256, tiles = tm * tn, full = big_full_tiles(tiles);
+    hipLaunchKernelGGL(linear_big_kernel, dim3(full + 2 * (tiles - full)), dim3(512), LDS, s, l, tm, full, (uint32_t)a_bytes);
+    NC_CHECK_LAUNCH("linear_big");
+    return 0;
+}
 // tile shapes: 1 = 64 x 128 (two workgroups per compute unit), 2 = 128 x 256, 3 = 128 x 128, 4 = 64 x 64 (two), 5 = 32 x 64 (two),
 // 6 = 32 x 32 (two)
+constexpr int BIG_SHAPE = 7;                  // bf16: 256 x 256 and halves of it
 constexpr int SHAPES = 6, SHAPE_ROWS[SHAPES + 1] = {0, 64, 128, 128, 64, 32, 32}, SHAPE_COLS[SHAPES + 1] = {0, 128, 256, 128, 64, 64, 32};
 template <typename T>
 int launch_tiled_shape(const NcLinear& l, int shape, hipStream_t s) {
@@ -541,6 +701,7 @@ int launch_tiled_shape(const NcLinear& l, int shape, hipStream_t s) {
 // us at K = 2048 (bf16) or 1024 (fp32), tenths: what a launch takes per round of tiles over the compute units, and beside the rounds.  A tile of
 // bf16 costs its loads, one of fp32 its products, where narrow tiles lose less.
 constexpr int ROUND_COST[2][SHAPES + 1] = {{0, 125, 270, 185, 90, 60, 50}, {0, 320, 1200, 620, 175, 100, 70}}, BASE_COST[2][SHAPES + 1] = {{0, 10, 0, 0, 10, 25, 25}, {0, 30, 0, 0, 30, 40, 40}};
+constexpr int BIG_COST = 500, BIG_HALF_COST = 295;       // ... of a round of 256 x 256 tiles, and of one of halves of them
 int64_t shape_tiles(const NcLinear& l, int shape) {
     return (int64_t)((l.M + SHAPE_ROWS[shape] - 1) / SHAPE_ROWS[shape]) * ((l.N + SHAPE_COLS[shape] - 1) / SHAPE_COLS[shape]) * l.batch * l.splits;
 }
@@ -558,6 +719,10 @@ int choose_shape(const NcLinear& l, int dtype) {
     for (int i = SHAPES; i >= (l.M <= NC_FEW_ROWS ? 4 : 1); i--) {
         const int64_t cost = (shape_tiles(l, i) + cus - 1) / cus * ROUND_COST[dtype][i] + BASE_COST[dtype][i];
         if (!shape || cost < best) best = cost, shape = i;
+    }
+    if (!dtype && !l.tiles && !l.a_rows && l.batch == 1 && l.splits == 1 && l.M > NC_FEW_ROWS) {
+        const int64_t tiles = (int64_t)((l.M + 255) / 256) * ((l.N + 255) / 256), full = big_full_tiles(tiles);
+        if ((full + cus - 1) / cus * BIG_COST + (full < tiles ? BIG_HALF_COST : 0) < best) shape = BIG_SHAPE;
     }
     return shape;
 }
@@ -592,9 +757,10 @@ int nc_launch_linear_few(int dtype, const NcLinear& l, hipStream_t s, int cls) {
 
 int nc_launch_linear_tiled(int dtype, const NcLinear& l, hipStream_t s, int cls, int shape) {
     if (int rc = check_linear(l, dtype)) return rc;
-    NC_CHECK_ARG(l.K % 64 == 0 && l.splits <= l.K / 64 && shape >= 0 && shape <= SHAPES, "linear: the tiled kernel takes whole K-steps");
+    NC_CHECK_ARG(l.K % 64 == 0 && l.splits <= l.K / 64 && shape >= 0 && (shape <= SHAPES || (shape == BIG_SHAPE && !dtype)), "linear: the tiled kernel takes whole K-steps");
     NcProfScope prof(cls, linear_units(l, dtype, !l.tiles ? l.M <= NC_FEW_ROWS : l.tile_rows <= 32), s, linear_tag(l));
     if (!shape) shape = !l.tiles ? choose_shape(l, dtype) : l.tile_rows <= 32 ? 5 : l.tile_rows <= 64 ? (l.few ? 4 : 1) : 2;
+    if (shape == BIG_SHAPE) return launch_big(l, s);
     // (the wider shapes have one chain: they are no place for a group whose sums are those of few rows)
     if (l.tiles) NC_CHECK_ARG(l.tile_rows <= SHAPE_ROWS[shape] && (!l.few || shape >= 4), "linear: group tiles of %d rows", l.tile_rows);
     return dtype ? launch_tiled_shape<float>(l, shape, s) : launch_tiled_shape<bf16_t>(l, shape, s);

@@ -77,6 +77,17 @@ def test_tiles_at_their_edges(kernel, dtype):
         assert torch.allclose(got.double(), a.double() @ w.double().T, rtol=tol, atol=tol), (M, N, K)
 
 
+@pytest.mark.parametrize("kind", [0, 1, 2, 3, 6, 7])
+def test_wide_tiles_have_the_sums_of_the_others(kind):
+    """Tiles of 256 x 256 and halves of them (the last but one: 256 whole and 90 half ones, the last row of halves ending behind the last column), to the bit."""
+    say(f"256 x 256 tiles, kind {kind}")
+    g = torch.Generator(device=DEV).manual_seed(9)
+    for M, N, K in [(1, 16, 64), (255, 144, 128), (256, 256, 192), (257, 528, 320), (300, 1072, 448), (1700, 10912, 192), (1792, 4096, 64)]:
+        a, w = torch.randn(M, K, generator=g, device=DEV).bfloat16(), (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).bfloat16()
+        want = ops.stack_linear(a, w, kind=kind, limit=0.6, kernel=4)
+        assert torch.equal(ops.stack_linear(a, w, kind=kind, limit=0.6, kernel=9), want), (M, N, K)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_few_rows_have_the_same_sums_in_every_kernel(dtype):
     """Up to 64 rows a result does not depend on the kernel or the tile: the same additions in the same order, to the bit (sums of one K-step, of
