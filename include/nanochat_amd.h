@@ -56,13 +56,13 @@ int nc_fp8_encode_with_scale(const uint16_t* x, int64_t n, float scale, int fp8_
  * elements: what the registers of the workgroups resident on the chip hold): every element is read from memory once, the
  * workgroups meet on the tensor's amax, the payload is converted from registers.  Other tensors take the two passes of
  * nc_fp8_quantize_tensorwise_as; results are bit-identical either way.  state: nc_fp8_quantize_state_bytes() bytes, 128-byte
- * aligned, ALL ZERO before the first call with it; every call leaves it all zero (words 257 and 320 excepted, see below),
+ * aligned, ALL ZERO before the first call with it; every call leaves words 0 to 319 all zero (word 257 excepted, see below),
  * so one allocation serves all calls that do not overlap in time; calls that overlap need a state each.  The one-launch grid
  * is sized to half of what the GPU holds of it, so that two such grids at once (of this or any other process on the GPU) are
  * both resident; with more of them at once a workgroup can wait for peers that have no slot yet.  That wait is bounded: a
  * workgroup whose wait runs out works the amax out by itself from the whole tensor (slow, same bits) and is counted in word
  * 257 of the state, which no kernel reads or clears -- a host that wants to know reads it; the results are correct either way.
- * Word 320 is scratch of the two-pass path. */
+ * The words from 320 on are scratch of the two-pass path. */
 size_t nc_fp8_quantize_state_bytes(void);
 int nc_fp8_quantize_tensorwise_fused(const void* x, int x_dtype, int64_t n, int fp8_format, uint8_t* out, float* scale_out,
                                      float* inv_scale_out, void* state, int encoder, nc_stream_t stream);

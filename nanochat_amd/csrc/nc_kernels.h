@@ -11,7 +11,7 @@ typedef uint16_t bf16_t;
 void nc_clear_u32(uint32_t* p, int n, hipStream_t s);
 int nc_launch_quantize(const void* x, int x_dtype, int64_t n, int fmt, uint8_t* out, float* scale_out, float* inv_out,
                        uint32_t* amax_ws, int encoder, hipStream_t s);
-#define NC_QUANTIZE_STATE_BYTES 1536
+#define NC_QUANTIZE_STATE_BYTES (1536 + 1024)
 #define NC_QUANTIZE_DEFAULT_SPINS (1u << 22)      // ~4 M polls of a few hundred ns each before a workgroup stops waiting
 int nc_launch_quantize_fused(const void* x, int x_dtype, int64_t n, int fmt, uint8_t* out, float* scale_out, float* inv_out,
                              uint32_t* state, int encoder, hipStream_t s, uint32_t spin_limit = NC_QUANTIZE_DEFAULT_SPINS);

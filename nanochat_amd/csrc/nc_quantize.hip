@@ -11,9 +11,12 @@
 
 // ---------------------------------------------------------------- pass 1: amax
 // bf16: |x| ordering equals integer ordering of the low 15 bits; fp32 likewise on 31 bits.
-// Each thread takes 16-byte vectors grid-stride; one atomicMax per block on the fp32 bit pattern.
-template <bool IS_BF16>
-__global__ __launch_bounds__(256) void amax_kernel(const void* __restrict__ x, int64_t n, uint32_t* __restrict__ amax_bits) {
+// Each thread takes 16-byte vectors grid-stride; one atomicMax per block on the fp32 bit pattern.  WORDS: blocks of
+// 1024, each of which stores its maximum in a word of its own instead; the convert pass joins them (amax_of_words): nothing to clear beforehand, a launch
+// of 4 us less (8192 x 6656 with its transposed copy: 60 us in three launches, 56 in two; words of 1024 blocks of 256 cost the convert pass 1.2 us).
+#define QZ_WORDS 256
+template <bool IS_BF16, bool WORDS = false>
+__global__ __launch_bounds__(WORDS ? 1024 : 256) void amax_kernel(const void* __restrict__ x, int64_t n, uint32_t* __restrict__ amax_bits) {
     constexpr int PER_VEC = IS_BF16 ? 8 : 4;
     const int64_t nvec = n / PER_VEC;
     const uint4* xv = (const uint4*)x;
@@ -49,24 +52,42 @@ __global__ __launch_bounds__(256) void amax_kernel(const void* __restrict__ x, i
         }
     }
     m = wave_max_u32(m);
-    __shared__ uint32_t red[4];
+    constexpr int WAVES = WORDS ? 16 : 4;
+    __shared__ uint32_t red[WAVES];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     if (lane == 0) red[w] = m;
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t t = red[0];
-        for (int i = 1; i < 4; i++) t = t > red[i] ? t : red[i];
+        for (int i = 1; i < WAVES; i++) t = t > red[i] ? t : red[i];
         // atomics on one word serialize: skip the ones that cannot change it
-        if (t > __hip_atomic_load(amax_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(amax_bits, t);
+        if (WORDS) amax_bits[blockIdx.x] = t;
+        else if (t > __hip_atomic_load(amax_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(amax_bits, t);
     }
 }
 
+// The maximum of the first pass's words, for every thread of a workgroup of 256: each thread's word, read before the workgroup's part of the tensor (loads
+// come back in order: it is joined while those are still under way), then the whole.
+static_assert(QZ_WORDS == 256, "a word for every thread of the convert passes");
+__device__ __forceinline__ uint32_t amax_word(const uint32_t* __restrict__ words, int n) { return (int)threadIdx.x < n ? words[threadIdx.x] : 0u; }
+__device__ __forceinline__ float amax_of_words(uint32_t m) {
+    __shared__ uint32_t red[4];
+    m = wave_max_u32(m);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    m = red[0];
+#pragma unroll
+    for (int i = 1; i < 4; i++) m = red[i] > m ? red[i] : m;
+    return __uint_as_float(m);
+}
+
 // ---------------------------------------------------------------- pass 2: convert
-template <bool IS_BF16, bool HW_CVT, int FMT = 0>
+// (words: how many words the first pass left, 0: an amax site)
+template <bool IS_BF16, bool HW_CVT, int FMT = 0, bool WORDS = false>
 __global__ __launch_bounds__(256) void convert_kernel(const void* __restrict__ x, int64_t n, const uint32_t* __restrict__ amax_bits,
                                                       uint8_t* __restrict__ out, float* __restrict__ scale_out,
-                                                      float* __restrict__ inv_out) {
-    const float amax = amax_read(amax_bits);
+                                                      float* __restrict__ inv_out, int words) {
+    const float amax = WORDS ? amax_of_words(amax_word(amax_bits, words)) : amax_read(amax_bits);
     const float scale = scale_from_amax(amax, fp8_max<FMT>());
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         if (scale_out) *scale_out = scale;
@@ -137,41 +158,48 @@ void nc_clear_u32(uint32_t* p, int n, hipStream_t s) {
     hipLaunchKernelGGL(clear_u32_kernel, dim3((n + 63) / 64), dim3(64), 0, s, p, n);
 }
 
-template <int FMT>
+template <int FMT, bool WORDS>
 static void launch_quantize_fmt(const void* x, int x_dtype, int64_t n, uint8_t* out, float* scale_out, float* inv_out, uint32_t* amax_ws,
                                 int encoder, int g1, int g2, hipStream_t s) {
     if (x_dtype == 0) {
-        hipLaunchKernelGGL(amax_kernel<true>, dim3(g1), dim3(256), 0, s, x, n, amax_ws);
+        hipLaunchKernelGGL((amax_kernel<true, WORDS>), dim3(g1), dim3(WORDS ? 1024 : 256), 0, s, x, n, amax_ws);
         if (encoder == 0)
-            hipLaunchKernelGGL((convert_kernel<true, true, FMT>), dim3(g2), dim3(256), 0, s, x, n, amax_ws, out, scale_out, inv_out);
+            hipLaunchKernelGGL((convert_kernel<true, true, FMT, WORDS>), dim3(g2), dim3(256), 0, s, x, n, amax_ws, out, scale_out, inv_out, g1);
         else
-            hipLaunchKernelGGL((convert_kernel<true, false, FMT>), dim3(g2), dim3(256), 0, s, x, n, amax_ws, out, scale_out, inv_out);
+            hipLaunchKernelGGL((convert_kernel<true, false, FMT, WORDS>), dim3(g2), dim3(256), 0, s, x, n, amax_ws, out, scale_out, inv_out, g1);
     } else {
-        hipLaunchKernelGGL(amax_kernel<false>, dim3(g1), dim3(256), 0, s, x, n, amax_ws);
+        hipLaunchKernelGGL((amax_kernel<false, WORDS>), dim3(g1), dim3(WORDS ? 1024 : 256), 0, s, x, n, amax_ws);
         if (encoder == 0)
-            hipLaunchKernelGGL((convert_kernel<false, true, FMT>), dim3(g2), dim3(256), 0, s, x, n, amax_ws, out, scale_out, inv_out);
+            hipLaunchKernelGGL((convert_kernel<false, true, FMT, WORDS>), dim3(g2), dim3(256), 0, s, x, n, amax_ws, out, scale_out, inv_out, g1);
         else
-            hipLaunchKernelGGL((convert_kernel<false, false, FMT>), dim3(g2), dim3(256), 0, s, x, n, amax_ws, out, scale_out, inv_out);
+            hipLaunchKernelGGL((convert_kernel<false, false, FMT, WORDS>), dim3(g2), dim3(256), 0, s, x, n, amax_ws, out, scale_out, inv_out, g1);
     }
 }
 
-int nc_launch_quantize(const void* x, int x_dtype, int64_t n, int fmt, uint8_t* out, float* scale_out, float* inv_out,
-                       uint32_t* amax_ws, int encoder, hipStream_t s) {
+// words: room for QZ_WORDS words at amax_ws, otherwise one
+static int launch_two_passes(const void* x, int x_dtype, int64_t n, int fmt, uint8_t* out, float* scale_out, float* inv_out, uint32_t* amax_ws, bool words,
+                             int encoder, hipStream_t s) {
     NC_CHECK_ARG(n >= 0, "fp8_quantize: negative element count");
     NC_CHECK_ARG(inv_out && amax_ws && (n == 0 || (x && out)), "fp8_quantize: null pointer");
     NC_CHECK_ARG(x_dtype == 0 || x_dtype == 1, "fp8_quantize: dtype must be 0 (bf16) or 1 (fp32)");
     NC_CHECK_ARG(fmt == 0 || fmt == 1, "fp8_quantize: format must be 0 (e4m3fn) or 1 (e5m2)");
     NC_CHECK_ARG(((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0, "fp8_quantize: pointers must be 16-byte aligned");
-    nc_clear_u32(amax_ws, 1, s);
+    if (!words) nc_clear_u32(amax_ws, 1, s);
     NcProfScope prof(2, 3.0 * n, s);
     const int per_vec = x_dtype == 0 ? 8 : 4;
-    // at most 1024 blocks x 256 threads, four loads per thread and trip; every block ends with one atomic on the same word
-    int g1 = grid_for(n / per_vec, 1024, 1024);
+    // at most 1024 blocks x 256 threads (or as many threads in blocks of 1024), four loads per thread and trip
+    int g1 = words ? grid_for(n / per_vec, 4096, QZ_WORDS) : grid_for(n / per_vec, 1024, 1024);
     int g2 = grid_for(n / 16, 256, 4096);
-    if (fmt == 0) launch_quantize_fmt<0>(x, x_dtype, n, out, scale_out, inv_out, amax_ws, encoder, g1, g2, s);
-    else launch_quantize_fmt<1>(x, x_dtype, n, out, scale_out, inv_out, amax_ws, encoder, g1, g2, s);
+    if (words && fmt == 0) launch_quantize_fmt<0, true>(x, x_dtype, n, out, scale_out, inv_out, amax_ws, encoder, g1, g2, s);
+    else if (words) launch_quantize_fmt<1, true>(x, x_dtype, n, out, scale_out, inv_out, amax_ws, encoder, g1, g2, s);
+    else if (fmt == 0) launch_quantize_fmt<0, false>(x, x_dtype, n, out, scale_out, inv_out, amax_ws, encoder, g1, g2, s);
+    else launch_quantize_fmt<1, false>(x, x_dtype, n, out, scale_out, inv_out, amax_ws, encoder, g1, g2, s);
     NC_CHECK_LAUNCH("fp8_quantize");
     return 0;
+}
+int nc_launch_quantize(const void* x, int x_dtype, int64_t n, int fmt, uint8_t* out, float* scale_out, float* inv_out,
+                       uint32_t* amax_ws, int encoder, hipStream_t s) {
+    return launch_two_passes(x, x_dtype, n, fmt, out, scale_out, inv_out, amax_ws, false, encoder, s);
 }
 
 // ---------------------------------------------------------------- one launch: amax, grid-wide meeting, convert
@@ -198,14 +226,15 @@ int nc_launch_quantize(const void* x, int x_dtype, int64_t n, int fmt, uint8_t* 
 // leave clears it; every workgroup leaves exactly once, after it has arrived).  Slot k (k = blockIdx.x % 8) lives on its own
 // 128-byte line: word 0 the running maximum, word 1 the arrivals (one address would serialize the grid's atomics at ~6 ns each).
 // Line 8: departures, the count of workgroups that ever took the slow way (sticky), slots reported.  Line 9: the flag that the
-// last reported slot raises and one lane per workgroup watches.  Line 10, word 0: scratch of the two-pass path.
+// last reported slot raises and one lane per workgroup watches.  From line 12 on: the words of the two-pass path (QZ_WORDS).
 #define QF_SLOTS 8
 #define QF_STRIDE 32
 #define QF_DEPART (QF_SLOTS * QF_STRIDE)
 #define QF_ERROR (QF_SLOTS * QF_STRIDE + 1)
 #define QF_SLOTS_DONE (QF_SLOTS * QF_STRIDE + 2)
 #define QF_FLAG ((QF_SLOTS + 1) * QF_STRIDE)
-#define QF_SCRATCH ((QF_SLOTS + 2) * QF_STRIDE)
+#define QF_SCRATCH ((QF_SLOTS + 4) * QF_STRIDE)
+static_assert((QF_SCRATCH + QZ_WORDS) * 4 <= NC_QUANTIZE_STATE_BYTES, "the quantizer's state");
 // What a workgroup does between its share of the tensor's maximum (m: each thread's) and the whole of it: `block` of `blocks` workgroups
 // of 256 threads of a launch on x[16 n16].
 __device__ __forceinline__ float qf_tensor_amax(uint32_t m, uint32_t* __restrict__ state, uint32_t spin_limit, uint32_t blocks, uint32_t block,
@@ -381,8 +410,8 @@ static bool try_fused_any(const bf16_t* x, int64_t n16, uint8_t* out, float* sca
            try_fused<FMT, HW_CVT, 4>(x, n16, out, scale_out, inv_out, state, lim, s) || try_fused<FMT, HW_CVT, 8>(x, n16, out, scale_out, inv_out, state, lim, s);
 }
 
-// state: NC_QUANTIZE_STATE_BYTES (1 KB + 16).  Tensors the one-launch kernel does not take (fp32 input, an element count that is
-// not a multiple of 16, more elements than fit on the chip) go through the two passes, with the state's last word as their scratch.
+// state: NC_QUANTIZE_STATE_BYTES.  Tensors the one-launch kernel does not take (fp32 input, an element count that is
+// not a multiple of 16, more elements than fit on the chip) go through the two passes, with the rest of the state as their scratch.
 // spin_limit: polls of the meeting's flag (a few hundred ns each) before a workgroup stops waiting and takes the slow way;
 // NC_QUANTIZE_DEFAULT_SPINS in ordinary use, a tiny value from the test that drives the slow way.
 int nc_launch_quantize_fused(const void* x, int x_dtype, int64_t n, int fmt, uint8_t* out, float* scale_out, float* inv_out,
@@ -406,14 +435,14 @@ int nc_launch_quantize_fused(const void* x, int x_dtype, int64_t n, int fmt, uin
             return 0;
         }
     }
-    return nc_launch_quantize(x, x_dtype, n, fmt, out, scale_out, inv_out, state + QF_SCRATCH, encoder, s);
+    return launch_two_passes(x, x_dtype, n, fmt, out, scale_out, inv_out, state + QF_SCRATCH, true, encoder, s);
 }
 
 // Convert only, with amax already reduced into amax_ws by a producer kernel.
 int nc_launch_convert_only(const void* x, int64_t n, uint8_t* out, float* inv_out, const uint32_t* amax_ws, hipStream_t s) {
     NcProfScope prof(2, 3.0 * n, s);
     int g2 = grid_for(n / 16, 256, 4096);
-    hipLaunchKernelGGL((convert_kernel<true, true>), dim3(g2), dim3(256), 0, s, x, n, amax_ws, out, (float*)nullptr, inv_out);
+    hipLaunchKernelGGL((convert_kernel<true, true>), dim3(g2), dim3(256), 0, s, x, n, amax_ws, out, (float*)nullptr, inv_out, 0);
     NC_CHECK_LAUNCH("fp8_convert");
     return 0;
 }
@@ -530,15 +559,16 @@ __device__ __forceinline__ void convert_tile(const TileRows& tile, float scale, 
             *(uint4*)(out_t + (size_t)(c0 + row) * R + r0 + lc16) = *(const uint4*)(tb + row * TP_PITCH + lc16);
     }
 }
-template <int FMT>
+template <int FMT, bool WORDS>
 __global__ __launch_bounds__(256) void convert_transpose_kernel(const bf16_t* __restrict__ x, int R, int C, const uint32_t* __restrict__ amax_bits,
                                                                 uint8_t* __restrict__ out, uint8_t* __restrict__ out_t,
-                                                                float* __restrict__ scale_out, float* __restrict__ inv_out) {
+                                                                float* __restrict__ scale_out, float* __restrict__ inv_out, int words) {
     __shared__ __align__(16) uint8_t ta[128 * TP_PITCH], tb[128 * TP_PITCH];
     const int r0 = blockIdx.y * 128, c0 = blockIdx.x * 128, t = threadIdx.x;
+    const uint32_t share = WORDS ? amax_word(amax_bits, words) : 0u;
     TileRows tile;
     load_tile(tile, x, R, C, r0, c0, t);
-    const float scale = scale_from_amax(amax_read(amax_bits), fp8_max<FMT>());
+    const float scale = scale_from_amax(WORDS ? amax_of_words(share) : amax_read(amax_bits), fp8_max<FMT>());
     if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) {
         if (scale_out) *scale_out = scale;
         *inv_out = 1.0f / scale;
@@ -607,6 +637,28 @@ static bool try_transposed(const bf16_t* x, int R, int C, uint8_t* out, uint8_t*
     return true;
 }
 
+template <int FMT, bool WORDS>
+static void launch_transposed_fmt(const bf16_t* x, int R, int C, uint8_t* out, uint8_t* out_t, float* scale_out, float* inv_out, uint32_t* amax_ws, hipStream_t s) {
+    const int64_t n = (int64_t)R * C;
+    const int g1 = WORDS ? grid_for(n / 8, 4096, QZ_WORDS) : grid_for(n / 8, 1024, 1024);
+    hipLaunchKernelGGL((amax_kernel<true, WORDS>), dim3(g1), dim3(WORDS ? 1024 : 256), 0, s, (const void*)x, n, amax_ws);
+    hipLaunchKernelGGL((convert_transpose_kernel<FMT, WORDS>), dim3((C + 127) / 128, (R + 127) / 128), dim3(256), 0, s, x, R, C, amax_ws, out, out_t, scale_out, inv_out, g1);
+}
+// words: as for launch_two_passes
+static int launch_transposed_passes(const bf16_t* x, int R, int C, int fmt, uint8_t* out, uint8_t* out_t, float* scale_out, float* inv_out, uint32_t* amax_ws, bool words,
+                                    hipStream_t s) {
+    if (const int rc = check_transposed(x, R, C, fmt, out, out_t, inv_out, amax_ws)) return rc;
+    if (R == 0 || C == 0) return 0;
+    if (!words) nc_clear_u32(amax_ws, 1, s);
+    NcProfScope prof(2, 4.0 * R * C, s);             // 2 bytes read + 2 x 1 byte written per element
+    if (words && fmt == 0) launch_transposed_fmt<0, true>(x, R, C, out, out_t, scale_out, inv_out, amax_ws, s);
+    else if (words) launch_transposed_fmt<1, true>(x, R, C, out, out_t, scale_out, inv_out, amax_ws, s);
+    else if (fmt == 0) launch_transposed_fmt<0, false>(x, R, C, out, out_t, scale_out, inv_out, amax_ws, s);
+    else launch_transposed_fmt<1, false>(x, R, C, out, out_t, scale_out, inv_out, amax_ws, s);
+    NC_CHECK_LAUNCH("fp8_quantize_transposed");
+    return 0;
+}
+
 int nc_launch_quantize_transposed_fused(const bf16_t* x, int R, int C, int fmt, uint8_t* out, uint8_t* out_t, float* scale_out, float* inv_out,
                                         uint32_t* state, uint32_t spin_limit, hipStream_t s) {
     if (const int rc = check_transposed(x, R, C, fmt, out, out_t, inv_out, state)) return rc;
@@ -623,22 +675,12 @@ int nc_launch_quantize_transposed_fused(const bf16_t* x, int R, int C, int fmt, 
             return 0;
         }
     }
-    return nc_launch_quantize_transposed(x, R, C, fmt, out, out_t, scale_out, inv_out, state + QF_SCRATCH, s);
+    return launch_transposed_passes(x, R, C, fmt, out, out_t, scale_out, inv_out, state + QF_SCRATCH, true, s);
 }
 
 int nc_launch_quantize_transposed(const bf16_t* x, int R, int C, int fmt, uint8_t* out, uint8_t* out_t, float* scale_out, float* inv_out,
                                   uint32_t* amax_ws, hipStream_t s) {
-    if (const int rc = check_transposed(x, R, C, fmt, out, out_t, inv_out, amax_ws)) return rc;
-    if (R == 0 || C == 0) return 0;
-    const int64_t n = (int64_t)R * C;
-    nc_clear_u32(amax_ws, 1, s);
-    NcProfScope prof(2, 4.0 * n, s);             // 2 bytes read + 2 x 1 byte written per element
-    hipLaunchKernelGGL(amax_kernel<true>, dim3(grid_for(n / 8, 1024, 1024)), dim3(256), 0, s, (const void*)x, n, amax_ws);
-    const dim3 grid((C + 127) / 128, (R + 127) / 128);
-    if (fmt == 0) hipLaunchKernelGGL(convert_transpose_kernel<0>, grid, dim3(256), 0, s, x, R, C, amax_ws, out, out_t, scale_out, inv_out);
-    else hipLaunchKernelGGL(convert_transpose_kernel<1>, grid, dim3(256), 0, s, x, R, C, amax_ws, out, out_t, scale_out, inv_out);
-    NC_CHECK_LAUNCH("fp8_quantize_transposed");
-    return 0;
+    return launch_transposed_passes(x, R, C, fmt, out, out_t, scale_out, inv_out, amax_ws, false, s);
 }
 
 int nc_launch_transpose_u8(const uint8_t* src, int R, int C, uint8_t* dst, hipStream_t s) {

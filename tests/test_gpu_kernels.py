@@ -1370,3 +1370,39 @@ def test_mix_norm_of_many_rows_has_the_bits_of_a_row_alone(ops, cols, over):
                 assert torch.equal(amax.view(torch.float32), xn.abs().max().float().reshape(1))
         for name, many, alone in zip(("x", "xn", "saved"), *res):
             assert torch.equal(many, alone), (kind, name)
+
+
+@pytest.mark.parametrize("R,C", [(4096, 12288), (16, 8192 * 512)])
+@pytest.mark.parametrize("fmt", [torch.float8_e4m3fn, torch.float8_e5m2])
+def test_quantize_of_tensors_beyond_the_one_launch_form(ops, R, C, fmt):
+    """50 and 67 million elements: the workgroups of the amax pass leave a word each in the quantizer's state and the convert pass joins them.  The largest
+    element goes to the first, an inner and the last workgroup's share in turn; a call after one with larger elements, and a small one that leaves fewer
+    words (fp32: never one launch), do not read what the larger left.  Payloads and scale against the entry that keeps one word, bit for bit."""
+    say(f"quantize, two passes {R}x{C} {fmt}")
+    import ctypes as C_
+    from nanochat_amd import _lib
+    g = torch.Generator(device=DEV).manual_seed(R + C)
+    x = torch.randn(R, C, device=DEV, generator=g).bfloat16()
+    stream = C_.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def one_word(t):
+        out = torch.empty(t.shape, dtype=torch.uint8, device=DEV)
+        sc = torch.zeros(2, dtype=torch.float32, device=DEV)
+        ws = torch.zeros(1, dtype=torch.int32, device=DEV)
+        _lib.check(_lib.lib().nc_fp8_quantize_tensorwise_as(t.data_ptr(), 0 if t.dtype == torch.bfloat16 else 1, t.numel(), ops._FP8_FORMATS[fmt], out.data_ptr(),
+                                                            sc.data_ptr(), sc.data_ptr() + 4, ws.data_ptr(), 0, stream))
+        return out, sc
+
+    for at, big in ((0, 128.0), (R * C // 2 + 12345, 64.0), (R * C - 1, 32.0)):
+        x.view(-1)[at] = big
+        want, sc = one_word(x)
+        assert sc[0].item() == torch.finfo(fmt).max / big
+        for p, inv, scale in (ops.fp8_quantize(x, fp8_dtype=fmt), ops.fp8_quantize_transposed(x, fp8_dtype=fmt)[::2] + (sc[0],)):
+            assert torch.equal(p.view(torch.uint8), want) and torch.equal(inv, sc[1]) and torch.equal(scale, sc[0])
+        p, pt, inv, scale = ops.fp8_quantize_transposed(x, fp8_dtype=fmt)
+        assert torch.equal(pt.view(torch.uint8), want.T) and torch.equal(scale, sc[0])
+        small = x[:7, :77].float().contiguous() / 128
+        want, sc = one_word(small)
+        p, inv, scale = ops.fp8_quantize(small, fp8_dtype=fmt)
+        assert torch.equal(p.view(torch.uint8), want) and torch.equal(scale, sc[0])
+        x.view(-1)[at] = 0.5
