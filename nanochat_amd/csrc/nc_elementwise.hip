@@ -200,14 +200,15 @@ __device__ __forceinline__ void convert_left_rows(const NcQuantRows& q8, const b
 // eight bf16 per 16-byte access, one reduction, one pass over memory.
 // PARTS: the addend arrives as split partial sums (decode).  Without them the kernel needs a third of the registers, and the
 // thousands of one-row workgroups of a prefill fit the chip in one round instead of two.
-// Q8_ROWS: rows to a workgroup of 256 threads each, as e4m3 (0: one row, as bf16).
+// Q8_ROWS: rows to a workgroup of 256 threads each, as e4m3 (0: one row, as bf16; a decode step's 52 launches carry no arguments that they do not read).
+struct NoQuantRows {};
 template <int NV, bool PARTS, int Q8_ROWS = 0>
 __global__ __launch_bounds__(256 * (Q8_ROWS > 1 ? Q8_ROWS : 1)) void mix_norm_vec_kernel(bf16_t* __restrict__ x, const bf16_t* __restrict__ add, NcPartialSrc padd,
                                                            const bf16_t* __restrict__ x0, const float* __restrict__ resid_lambda,
                                                            const float* __restrict__ x0_lambda, const float* __restrict__ backout_lambda,
                                                            const bf16_t* __restrict__ backout_src, bf16_t* __restrict__ backout_save,
                                                            bf16_t* __restrict__ xn_out, int cols, uint32_t* __restrict__ amax_ws,
-                                                           int32_t* __restrict__ bump, int bump_by, NcQuantRows q8) {
+                                                           int32_t* __restrict__ bump, int bump_by, std::conditional_t<(Q8_ROWS > 0), NcQuantRows, NoQuantRows> q8) {
     NC_ARG_NOW(x); NC_ARG_NOW(add); NC_ARG_NOW(padd.parts); NC_ARG_NOW(padd.nsplit); NC_ARG_NOW(padd.ld); NC_ARG_NOW(padd.split_stride);
     NC_ARG_NOW(padd.a_amax); NC_ARG_NOW(padd.inv_b); NC_ARG_NOW(x0); NC_ARG_NOW(resid_lambda); NC_ARG_NOW(x0_lambda);
     NC_ARG_NOW(backout_lambda); NC_ARG_NOW(backout_src); NC_ARG_NOW(backout_save); NC_ARG_NOW(xn_out); NC_ARG_NOW(cols); NC_ARG_NOW(amax_ws);
@@ -216,7 +217,8 @@ __global__ __launch_bounds__(256 * (Q8_ROWS > 1 ? Q8_ROWS : 1)) void mix_norm_ve
     __shared__ float red[4 * ROWS > 8 ? 4 * ROWS : 8];
     const int tid = ROWS > 1 ? threadIdx.x & 255 : threadIdx.x, in_wg = ROWS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, row = blockIdx.x * ROWS + in_wg;
     const int all_cols = cols;
-    if (ROWS > 1 && row >= q8.rows) cols = 0;                 // (past the last row: nothing is loaded or stored)
+    if constexpr (ROWS > 1)
+        if (row >= q8.rows) cols = 0;                         // (past the last row: nothing is loaded or stored)
     const size_t base = (size_t)row * all_cols;
     const bool has_parts = PARTS && padd.parts != nullptr;
     const bool writes_x = add || has_parts || resid_lambda || backout_lambda;
@@ -681,7 +683,7 @@ static int launch_mix_norm_impl(bf16_t* x, const bf16_t* add, NcPartialSrc padd,
     const bool aligned = cols % 8 == 0 && (((uintptr_t)x | (uintptr_t)xn_out | (uintptr_t)add | (uintptr_t)x0 | (uintptr_t)backout_src |
                                             (uintptr_t)backout_save | (uintptr_t)padd.parts) & 15) == 0 && padd.ld % 4 == 0 &&
                          padd.split_stride % 4 == 0;
-#define MIX_ARGS x, add, padd, x0, resid_lambda, x0_lambda, backout_lambda, backout_src, backout_save, xn_out, cols, amax_ws, bump, bump_by, NcQuantRows{}
+#define MIX_ARGS x, add, padd, x0, resid_lambda, x0_lambda, backout_lambda, backout_src, backout_save, xn_out, cols, amax_ws, bump, bump_by, NoQuantRows{}
 #define MIX_LAUNCH(NVV)                                                                                                  \
     do {                                                                                                                 \
         if (padd.parts) hipLaunchKernelGGL((mix_norm_vec_kernel<NVV, true>), dim3(rows), dim3(256), 0, s, MIX_ARGS);      \
