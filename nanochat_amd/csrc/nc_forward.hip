@@ -15,8 +15,13 @@
 //   linear c_fc         quantize xn inside; up to 64 rows of up to 2048 columns relu^2 and amax as well -> h2, otherwise -> partials and
 //   finish_partials     sum, scale, relu^2, amax                                       -> h2
 //   linear mlp c_proj   quantize h2 inside                                             -> partials (added by the next mix_norm)
-// Prefill (M > 128) uses the explicit convert kernel and the tiled GEMM instead of the fused small-M linear; the two narrow projections of a
-// few hundred rows leave partial sums to mix_norm as well.
+// Prefill (M > 128) uses the tiled GEMM instead of the fused small-M linear.  Where its workgroups are all resident at once (and the call has more than one
+// token per row for the third), a producer writes what the next launch reads, 8 launches a layer instead of 12:
+//   mix_norm            the workgroups meet on the amax of the rows and write them as e4m3
+//   linear c_fc         relu^2, the meeting, e4m3
+//   linear q|k|v        rotary, QK-norm, gain, VE gate and append in its epilogue
+// otherwise the convert kernel and the rotary kernel follow as launches of their own.  Attention's launch also reads the weights of the next linears ahead
+// (nc_prefetch.h); its output goes through the convert kernel.  The two narrow projections of a few hundred rows leave partial sums to mix_norm as well.
 //
 // Workspace (carved from the caller's buffer, 256-byte aligned pieces), M = B*T rows:
 //   x, x0, xn, xb, o      bf16 [M,E]        residual stream, its initial value, normed rows, backout, GEMM out

@@ -6,6 +6,7 @@
 //
 //   linear_tiled_kernel  tiles of 32 x 64 to 128 x 256 outputs, operands straight into a ring of LDS stages; the summed index may be dealt to
 //                        several workgroups, whose consumer adds their sums.
+//   linear_big_kernel    bf16 tiles of 256 x 256 (and halves of 256 x 128 behind whole rounds of them), unsplit, for many rows.
 //   linear_few_kernel    few rows of a small weight, or a summed index that is no multiple of 64: operands straight into registers, no LDS in
 //                        the loop.
 //
