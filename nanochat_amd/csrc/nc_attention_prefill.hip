@@ -14,6 +14,7 @@
 // Keys and values go through LDS in blocks of 32, both as [key][d] (K rows padded to 272 B, V rows to 320 B); the V^T operand
 // comes out of LDS through the transposing read (ds_read_b64_tr_b16), so nothing is shuffled while staging.  The loads of the
 // next block are in flight while the current one is multiplied.
+#include <type_traits>
 #include "nc_common.h"
 #include "nc_kernels.h"
 #include "nc_prefetch.h"
@@ -66,15 +67,32 @@ struct PfUnitMap {
     int on;
     uint16_t unit[512];
 };
-template <int GS, int KS>
+// Launches that read weights ahead for the linears behind them (nc_prefetch.h) are one line of workgroups, units to a row, the ones that read behind all rows.
+// The others have a dimension for each of (tile, head, row) and no argument that they do not use: with the line's check in front of everything else a
+// launch of two tiles per head took 7.4 us instead of 7.0 (65 tokens of 6 heads).  A line holds fewer than 2^32 threads, that is 2^24 workgroups: of a longer
+// one only what is left of a division by that is launched, without an error.
+struct PfLine {
+    NcAhead ahead;
+    int nx, units, B;
+};
+struct PfGrid {};
+template <int GS, int KS, typename Place>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_prefill_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache,
                                                            const bf16_t* __restrict__ v_cache, const int32_t* __restrict__ cache_seqlens,
                                                            int window_left, int seqlens_include_new, bf16_t* __restrict__ out,
-                                                           uint32_t* __restrict__ amax_ws, int T, int H, int Hkv, int Tmax, PfUnitMap map, NcAhead ahead, int nx, int units, int B) {
+                                                           uint32_t* __restrict__ amax_ws, int T, int H, int Hkv, int Tmax, PfUnitMap map, Place place) {
     constexpr int QT = 128 / (GS * KS);                        // queries per workgroup
-    if ((int)blockIdx.x >= units * B) {                        // (workgroups of no row: they come last)
-        read_ahead<256>(ahead, blockIdx.x - units * B, gridDim.x - units * B);
-        return;
+    constexpr bool LINE = std::is_same_v<Place, PfLine>;
+    int b, nx, total, lid;                                     // the row, its tiles, its (tile, head) pairs and which of them this is
+    if constexpr (LINE) {
+        const int behind = (int)blockIdx.x - place.units * place.B;
+        if (behind >= 0) {
+            read_ahead<256>(place.ahead, behind, gridDim.x - place.units * place.B);
+            return;
+        }
+        nx = place.nx, total = place.units, b = place.B == 1 ? 0 : (int)blockIdx.x / total, lid = (int)blockIdx.x - b * total;
+    } else {
+        nx = gridDim.x, total = nx * (int)gridDim.y, b = blockIdx.z, lid = (int)blockIdx.x + nx * (int)blockIdx.y;
     }
     __shared__ __align__(16) uint8_t lds[2 * PF_KBYTES + 2 * PF_VBYTES];
     __shared__ float red[4];
@@ -85,10 +103,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // Workgroups go to the eight XCDs in turn by their linear index, and each XCD has an L2 of its own: the (tile, head) pairs of a
     // row are numbered so that one XCD gets a contiguous run of them, i.e. all tiles of a few heads, and the keys and values of a head
     // are then read into one L2 instead of all eight.  Within a head the tiles come from the end of the sequence, longest first.
-    const int b = B == 1 ? 0 : (int)blockIdx.x / units;
     int qb0, hy;
     {
-        const int total = units, lid = (int)blockIdx.x - b * units;
         const int xcd = lid & 7, slot = lid >> 3;
         const int unit = map.on ? (int)map.unit[lid] : xcd * (total >> 3) + min(xcd, total & 7) + slot;
         hy = unit / nx;
@@ -613,22 +629,27 @@ int nc_launch_attention_prefill(const bf16_t* q, const bf16_t* k_cache, const bf
     const long long wgs1 = (long long)B * Hkv * (G / GS) * ((T + 128 / GS - 1) / (128 / GS));
     const int KS = (GS <= 2 && wgs1 < 2LL * nc_cu_count()) ? 2 : 1;
     const int QT = 128 / (GS * KS);
-    const int nx = (T + QT - 1) / QT, ny = Hkv * (G / GS), extra = ahead && ahead->n > 0 ? NC_AHEAD_WGS : 0;
-    NC_CHECK_ARG((long long)nx * ny * B + extra < (1LL << 31), "prefill_attention: too many workgroups in one launch");
-    const dim3 grid(nx * ny * B + extra);
+    const int nx = (T + QT - 1) / QT, ny = Hkv * (G / GS);
+    const bool line = ahead && ahead->n > 0 && (long long)nx * ny * B + NC_AHEAD_WGS < (1LL << 24);
     PfUnitMap map;                         // passed by value
     map.on = 0;
     // one row whose queries see every key before them (a window of at least the cache length is none): the long prompt of a prefill
     if (B == 1 && (window_left < 0 || window_left >= Tmax)) pf_balance_units(map, nx, ny, nc_cu_count());
+#define PF_LAUNCH_AT(GG, KK, Place, grid, place)                                                                                       \
+    hipLaunchKernelGGL((attn_prefill_kernel<GG, KK, Place>), grid, dim3(256), 0, s, q, k_cache, v_cache, cache_seqlens, window_left,   \
+                       seqlens_include_new, out, amax_ws, T, H, Hkv, Tmax, map, place)
 #define PF_LAUNCH(GG, KK)                                                                                                              \
-    hipLaunchKernelGGL((attn_prefill_kernel<GG, KK>), grid, dim3(256), 0, s, q, k_cache, v_cache, cache_seqlens, window_left,          \
-                       seqlens_include_new, out, amax_ws, T, H, Hkv, Tmax, map, extra ? *ahead : NcAhead{}, nx, nx * ny, B)
+    do {                                                                                                                               \
+        if (line) PF_LAUNCH_AT(GG, KK, PfLine, dim3(nx * ny * B + NC_AHEAD_WGS), (PfLine{*ahead, nx, nx * ny, B}));                    \
+        else PF_LAUNCH_AT(GG, KK, PfGrid, dim3(nx, ny, B), PfGrid{});                                                                  \
+    } while (0)
     if (GS == 4) PF_LAUNCH(4, 1);
     else if (GS == 2 && KS == 2) PF_LAUNCH(2, 2);
     else if (GS == 2) PF_LAUNCH(2, 1);
     else if (KS == 2) PF_LAUNCH(1, 2);
     else PF_LAUNCH(1, 1);
 #undef PF_LAUNCH
+#undef PF_LAUNCH_AT
     NC_CHECK_LAUNCH("prefill_attention");
     return 0;
 }

@@ -1119,6 +1119,32 @@ def test_attention_many_rows_of_many_queries(ops, B, T, H, Hkv, window):
     attn_case(ops, B, T, H, Hkv, 128, seqlens, window, 0, seed=B * T)
 
 
+def test_attention_of_more_workgroups_than_a_line_holds(ops):
+    """65535 rows of 257 heads on one key head, 16 queries each: 16.8 million workgroups, 2^32 threads and more, which a grid takes in three dimensions but
+    not in one.  Every row has the same queries, keys and values, so the first row's output against the oracle and all others against that."""
+    from nanochat_amd import _lib
+    B, T, H = 65535, 16, 257
+    need = 2 * B * T * H * 256 + 2 * B * T * 256 + (4 << 30)
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < need:
+        pytest.skip(f"{need >> 30} GiB of GPU memory needed")
+    say(f"attention, {B} rows of {H} heads")
+    g = torch.Generator().manual_seed(11)
+    q1, k1, v1 = (torch.randn(1, T, h, 128, generator=g).bfloat16() for h in (H, 1, 1))
+    n = torch.zeros(B, dtype=torch.int32, device=DEV)
+    q, kc, vc = (t.to(DEV).expand(B, -1, -1, -1).contiguous() for t in (q1, k1, v1))
+    out = torch.zeros_like(q)
+    rc = _lib.lib().nc_decode_attention(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), n.data_ptr(), -1, out.data_ptr(), B, T, H, 1, T, 0, None, 0, None, 0,
+                                        torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc)
+    want = attention_with_kvcache(q1.float(), k1.float(), v1.float(), cache_seqlens=torch.zeros(1, dtype=torch.int32), window_size=(-1, 0))
+    assert torch.allclose(out[:1].float().cpu(), want, atol=1e-2, rtol=1e-2)
+    first = out[:1].view(torch.int16)
+    assert all(bool((part.view(torch.int16) == first).all()) for part in out.split(2048))
+    del q, out, kc, vc, first
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("T,gain", [(300, 0.02), (300, 0.2), (130, 1.0)])
 def test_attention_prefill_scores_that_keep_growing(ops, T, gain):
     """Every key scores higher than the one before it (by `gain` per key on average, in units of the softmax exponent), so the running
