@@ -331,6 +331,8 @@ typedef struct nc_cache_desc {
 } nc_cache_desc;
 
 size_t nc_gpt_workspace_bytes(const nc_model_desc* model /*host*/, int B, int T);
+/* 1: the attention launches of such a forward read the weights of the linears behind them ahead (host only; the results do not depend on it). */
+int nc_gpt_reads_ahead(const nc_model_desc* model /*host*/, int B, int T);
 
 /* idx int64 [B,T]; logits_out fp32 [B*T, vocab_size] (all positions) or, with last_only = 1,
  * [B, vocab_size] (the last position of every row, which is all Engine.generate reads).

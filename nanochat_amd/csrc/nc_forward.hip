@@ -165,6 +165,18 @@ Workspace carve(const nc_model_desc* m, int B, int T, void* base) {
     return w;
 }
 
+// Whether the attention launches of a prompt read the weights of the linears behind them ahead (nc_prefetch.h), E (qkv_w + H 128 + 8 E) bytes a layer.
+// The tiles of more than 128 rows wait for their weights.  Up to 64 rows the linears are streams of the weight themselves and gain nothing, while attention
+// (6.6 us for 40 tokens of 13 heads) ends with the reading (9.8 us for 33 MB): us without / with, depth 26, 16 tokens 1229 / 1281, 32 1377 / 1415, 64 1565 / 1604.  Between
+// the two it depends on whether the reading ends with attention: 20 MB (depth 20) 65 tokens 1274 / 1246, 128 1446 / 1390, 4 x 17 1255 / 1265, 24 MB (depth 22) 65
+// tokens 1476 / 1463, 128 1663 / 1633, but 28 MB (depth 24) 65 tokens 1592 / 1607, 4 x 24 1698 / 1711, 33 MB (depth 26) 65 tokens 1851 / 1867, 128 2113 / 2098, 4 x 20
+// 1906 / 1922.  Beyond 128 rows, depth 26: 8 x 32 1854 / 1761, 64 x 16 3001 / 2733.
+constexpr size_t AHEAD_LAYER_BYTES_FEW = 24u << 20;
+bool reads_ahead(const nc_model_desc* m, int M) {
+    const size_t E = m->n_embd, layer = E * ((size_t)(2 * m->n_head + 2 * m->n_kv_head) * 128 + 8 * E);
+    return M > 128 || (M > 64 && layer <= AHEAD_LAYER_BYTES_FEW);
+}
+
 NcGemmSegs one_seg(int n) { return NcGemmSegs{1, {n, 0, 0, 0}}; }
 
 __global__ void gather_last_rows_kernel(const bf16_t* __restrict__ x, bf16_t* __restrict__ out, int T, int E) {
@@ -253,6 +265,8 @@ extern "C" size_t nc_gpt_workspace_bytes(const nc_model_desc* model, int B, int 
     if (!model || B <= 0 || T <= 0) return 0;
     return carve(model, B, T, nullptr).total;
 }
+
+extern "C" int nc_gpt_reads_ahead(const nc_model_desc* model, int B, int T) { return model && B > 0 && T >= 16 && reads_ahead(model, B * T); }
 
 // tap_x (or nullptr): bf16 [L+1, M, E], slot i = the residual stream as layer i reads it (after the lambda mix, gpt.py:500), slot L = the
 // final normalised rows (gpt.py:508).  tap_y (or nullptr): bf16 [L, M, H*128], the attention outputs before c_proj (gpt.py:113-124).
@@ -405,11 +419,13 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
                                               kv->cache_seqlens, kc, vc, w.qh, B, T, H, Hkv, kv->max_seq_len, m->padded_vocab, s));
             // meanwhile the weights of the linears up to the next attention come out of HBM
             NcAhead ahead{};
-            ahead.add(ly.w_attn_proj, (size_t)E * H * 128);
-            ahead.add(ly.w_fc, (size_t)4 * E * E);
-            ahead.add(ly.w_mlp_proj, (size_t)4 * E * E);
-            if (i + 1 < L) ahead.add(m->layers[i + 1].w_qkv, (size_t)qkv_w * E);
-            else ahead.add(m->w_lm_head, (size_t)m->vocab_size * E);
+            if (reads_ahead(m, M)) {
+                ahead.add(ly.w_attn_proj, (size_t)E * H * 128);
+                ahead.add(ly.w_fc, (size_t)4 * E * E);
+                ahead.add(ly.w_mlp_proj, (size_t)4 * E * E);
+                if (i + 1 < L) ahead.add(m->layers[i + 1].w_qkv, (size_t)qkv_w * E);
+                else ahead.add(m->w_lm_head, (size_t)m->vocab_size * E);
+            }
             TRY(nc_launch_attention(w.qh, kc, vc, kv->cache_seqlens, ly.window_left, w.y, B, T, H, Hkv, kv->max_seq_len, 0,
                                     w.attn_counters, w.attn_parts, w.attn_part_bytes, w.site(site), 0, 1, s, &ahead));
         }

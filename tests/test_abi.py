@@ -107,3 +107,14 @@ def test_prompt_rows_that_go_a_wave_to_a_row_bring_no_partial_sums():
         assert room(heads, line - 1) - room(heads, line) > shares / 2
         assert room(heads, 2 * line) < 2 * room(heads, line) + 4096
     assert room(7, 1024) > room(7, 1023)
+
+
+def test_which_prompts_read_weights_ahead():
+    """Calls whose linears are streams of the weight themselves (up to 64 rows, a step of any batch) read nothing ahead; from 65 to 128 rows those do whose
+    layer comes while its attention runs."""
+    def ahead(heads, B, T):
+        m = _lib.ModelDesc(n_layer=2 * heads, n_head=heads, n_kv_head=heads, n_embd=128 * heads, vocab_size=32768)
+        return _lib.lib().nc_gpt_reads_ahead(ctypes.byref(m), B, T)
+    assert not any(ahead(13, B, T) for B, T in [(1, 16), (1, 64), (4, 16), (1, 65), (4, 20), (1, 128), (500, 1), (200, 2), (10, 15)])
+    assert all(ahead(13, B, T) for B, T in [(1, 129), (9, 16), (1, 1792), (8, 1024)])
+    assert [ahead(10, 1, T) for T in (16, 64, 65, 128, 129)] == [0, 0, 1, 1, 1]
