@@ -545,10 +545,10 @@ __global__ __launch_bounds__(128) void latent_combine_kernel(const float* __rest
 // DR); keys and values come through buffer descriptors that end behind the workgroup's last key, pieces past a head's own sizes through
 // an offset no descriptor reaches: both read zeros.
 #define LA_OOB 0x80000000u
-template <int DN, int DR, int DV, int NW>
+template <int DN, int DR, int DV, int NW, typename Ahead>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void latent_expanded_kernel(
     NcLatentGeom g, const bf16_t* __restrict__ q, int ldq, const bf16_t* __restrict__ kv, int keys_alloc, const bf16_t* __restrict__ cache,
-    const int32_t* __restrict__ seqlens, bf16_t* __restrict__ out, int ldo, NcAhead ahead) {
+    const int32_t* __restrict__ seqlens, bf16_t* __restrict__ out, int ldo, Ahead ahead) {
     constexpr int DQK = DN + DR, KPITCH = DQK * 2 + 16, VPITCH = DV * 2 + 64, NTHR = 64 * NW, KB = 16 * NW, QT = 32 * NW;
     constexpr int NCH = DN / 8, RCH = DR / 8, VCH = DV / 8, NL = KB * NCH / NTHR, RL = KB * RCH / NTHR, VL = KB * VCH / NTHR;
     __shared__ __align__(16) uint8_t lds[KB * KPITCH + KB * VPITCH];
@@ -762,11 +762,13 @@ template <int DN, int DR, int DV>
 int launch_expanded(const NcLatentGeom& g, const bf16_t* q, int ldq, const bf16_t* kv, int keys, const bf16_t* cache, const int32_t* seqlens, bf16_t* out,
                     int ldo, const NcAhead* ahead, hipStream_t s) {
     if ((int64_t)((g.T + 127) / 128) * g.heads * g.B >= 200)
-        hipLaunchKernelGGL((latent_expanded_kernel<DN, DR, DV, 4>), nc_ahead_grid(dim3((g.T + 127) / 128, g.heads, g.B), ahead), dim3(256), 0, s, g, q, ldq, kv, keys, cache,
-                           seqlens, out, ldo, ahead ? *ahead : NcAhead{});
+        nc_launch_ahead(dim3((g.T + 127) / 128, g.heads, g.B), ahead, [&](dim3 grid, auto a) {
+            hipLaunchKernelGGL((latent_expanded_kernel<DN, DR, DV, 4, decltype(a)>), grid, dim3(256), 0, s, g, q, ldq, kv, keys, cache, seqlens, out, ldo, a);
+        });
     else
-        hipLaunchKernelGGL((latent_expanded_kernel<DN, DR, DV, 2>), nc_ahead_grid(dim3((g.T + 63) / 64, g.heads, g.B), ahead), dim3(128), 0, s, g, q, ldq, kv, keys, cache, seqlens,
-                           out, ldo, ahead ? *ahead : NcAhead{});
+        nc_launch_ahead(dim3((g.T + 63) / 64, g.heads, g.B), ahead, [&](dim3 grid, auto a) {
+            hipLaunchKernelGGL((latent_expanded_kernel<DN, DR, DV, 2, decltype(a)>), grid, dim3(128), 0, s, g, q, ldq, kv, keys, cache, seqlens, out, ldo, a);
+        });
     NC_CHECK_LAUNCH("latent_expanded");
     return 0;
 }

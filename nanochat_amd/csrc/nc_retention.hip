@@ -276,10 +276,10 @@ __global__ __launch_bounds__(256) void retention_scan_kernel(NcRetentionGeom g, 
 
 // The outputs of one chunk and head.  Four waves: C / 32 blocks of 32 queries x the value columns dealt to 4 / (C / 32) waves, each of which
 // computes the scores of its queries for itself.  Transposed like the attention kernels (a lane owns one query): S^T = K Q^T, O^T = V^T P^T.
-template <int DK, int DV, int C>
+template <int DK, int DV, int C, typename Ahead>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void retention_chunk_out_kernel(NcRetentionGeom g, const bf16_t* __restrict__ proj, int ldp, const float* __restrict__ decay,
                                                                   const float* __restrict__ rope, int rope_len, const int32_t* __restrict__ seqlens,
-                                                                  const bf16_t* __restrict__ prefix, int chunks, float eps, bf16_t* __restrict__ out, int ldo, NcAhead ahead) {
+                                                                  const bf16_t* __restrict__ prefix, int chunks, float eps, bf16_t* __restrict__ out, int ldo, Ahead ahead) {
     constexpr int QB = C / 32, VS = 4 / QB, NT = DV / 32 / VS, KP = DK * 2 + 16, VP = DV * 2 + 64;
     static_assert(NT >= 1, "value columns per wave");
     __shared__ __align__(16) uint8_t lds[C * (2 * KP + VP)];
@@ -603,8 +603,10 @@ int launch_chunked(const NcRetentionGeom& g, const bf16_t* proj, int ldp, const 
                        chunks);
     hipLaunchKernelGGL(retention_scan_kernel, dim3((DK * DV + 1023) / 1024, g.heads, g.B), dim3(256), 0, s, g, decay, seqlens, kv, prefix, state_in, state_out,
                        chunks, C);
-    hipLaunchKernelGGL((retention_chunk_out_kernel<DK, DV, C>), nc_ahead_grid(dim3(chunks, g.heads, g.B), ahead), dim3(256), 0, s, g, proj, ldp, decay, rope, rope_len, seqlens,
-                       prefix, chunks, eps, out, ldo, ahead ? *ahead : NcAhead{});
+    nc_launch_ahead(dim3(chunks, g.heads, g.B), ahead, [&](dim3 grid, auto a) {
+        hipLaunchKernelGGL((retention_chunk_out_kernel<DK, DV, C, decltype(a)>), grid, dim3(256), 0, s, g, proj, ldp, decay, rope, rope_len, seqlens, prefix, chunks, eps, out,
+                           ldo, a);
+    });
     NC_CHECK_LAUNCH("retention_chunked");
     return 0;
 }

@@ -194,12 +194,12 @@ __global__ __launch_bounds__(256) void scan_step_kernel(NcScanGeom g, NcScanStep
 
 // MODE WHOLE: all tokens from the stored state, outputs, state out.  SUMS: one chunk from zero, its end and its sum of dt into `ends` /
 // `sum_dt`.  OUT: one chunk from its start in `ends`, outputs; the last chunk stores the state.
-template <typename T, int SP, int MODE>
+template <typename T, int SP, int MODE, typename Ahead>
 __global__ __launch_bounds__(256) void scan_kernel(NcScanGeom g, int lg, const T* __restrict__ u, const float* __restrict__ dt, const float* __restrict__ bc,
                                                    const float* __restrict__ a_log2, const float* __restrict__ skip, const T* __restrict__ z, int ldz,
                                                    const int32_t* __restrict__ seqlens, const float* __restrict__ state_in, float* __restrict__ state_out,
-                                                   T* __restrict__ out, int ldo, float* __restrict__ ends, float* __restrict__ sum_dt, int chunks, int chunk_len, NcAhead ahead) {
-    if (MODE != SCAN_SUMS && reads_ahead<256>(ahead, g.B)) return;
+                                                   T* __restrict__ out, int ldo, float* __restrict__ ends, float* __restrict__ sum_dt, int chunks, int chunk_len, Ahead ahead) {
+    if (reads_ahead<256>(ahead, g.B)) return;
     extern __shared__ __align__(16) float lds[];            // [TB][2][state_p]: B, C
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cw = 64 / lg, part = lane / cw;
     const int c_at = ((int)blockIdx.x * 4 + wave) * cw + lane % cw, c = min(c_at, g.inner_p - 1);
@@ -334,18 +334,22 @@ int launch_scan(const NcScanGeom& g, int lg, const T* u, const float* dt, const 
                 const int32_t* seqlens, const float* state_in, float* state_out, T* out, int ldo, void* workspace, const NcAhead* ahead, hipStream_t s) {
     const int chunks = chunk_count(g), len = chunk_len(g), xs = channel_groups(g, lg), bytes = TB * 2 * g.state_p * 4;
     if (chunks == 1) {
-        hipLaunchKernelGGL((scan_kernel<T, SP, SCAN_WHOLE>), nc_ahead_grid(dim3(xs, 1, g.B), ahead), dim3(256), bytes, s, g, lg, u, dt, bc, a_log2, skip, z, ldz, seqlens, state_in, state_out,
-                           out, ldo, nullptr, nullptr, 1, 0, ahead ? *ahead : NcAhead{});
+        nc_launch_ahead<sizeof(T) == 2>(dim3(xs, 1, g.B), ahead, [&](dim3 grid, auto a) {
+            hipLaunchKernelGGL((scan_kernel<T, SP, SCAN_WHOLE, decltype(a)>), grid, dim3(256), bytes, s, g, lg, u, dt, bc, a_log2, skip, z, ldz, seqlens, state_in, state_out, out,
+                               ldo, nullptr, nullptr, 1, 0, a);
+        });
         NC_CHECK_LAUNCH("scan");
         return 0;
     }
     float* ends = (float*)workspace;
     float* sum_dt = ends + (int64_t)g.B * (chunks - 1) * g.state_p * g.inner_p;
-    hipLaunchKernelGGL((scan_kernel<T, SP, SCAN_SUMS>), dim3(xs, chunks - 1, g.B), dim3(256), bytes, s, g, lg, u, dt, bc, a_log2, skip, z, ldz, seqlens, state_in,
-                       state_out, out, ldo, ends, sum_dt, chunks, len, NcAhead{});
+    hipLaunchKernelGGL((scan_kernel<T, SP, SCAN_SUMS, NcNoAhead>), dim3(xs, chunks - 1, g.B), dim3(256), bytes, s, g, lg, u, dt, bc, a_log2, skip, z, ldz, seqlens, state_in,
+                       state_out, out, ldo, ends, sum_dt, chunks, len, NcNoAhead{});
     hipLaunchKernelGGL(scan_chunks_kernel, dim3((g.inner_p + 255) / 256, g.state_p, g.B), dim3(256), 0, s, g, a_log2, seqlens, state_in, ends, sum_dt, chunks);
-    hipLaunchKernelGGL((scan_kernel<T, SP, SCAN_OUT>), nc_ahead_grid(dim3(xs, chunks, g.B), ahead), dim3(256), bytes, s, g, lg, u, dt, bc, a_log2, skip, z, ldz, seqlens, state_in, state_out,
-                       out, ldo, ends, sum_dt, chunks, len, ahead ? *ahead : NcAhead{});
+    nc_launch_ahead<sizeof(T) == 2>(dim3(xs, chunks, g.B), ahead, [&](dim3 grid, auto a) {
+        hipLaunchKernelGGL((scan_kernel<T, SP, SCAN_OUT, decltype(a)>), grid, dim3(256), bytes, s, g, lg, u, dt, bc, a_log2, skip, z, ldz, seqlens, state_in, state_out, out, ldo,
+                           ends, sum_dt, chunks, len, a);
+    });
     NC_CHECK_LAUNCH("scan_chunked");
     return 0;
 }

@@ -442,10 +442,10 @@ __global__ __launch_bounds__(64) void window_combine_kernel(const float* __restr
 // Flash attention written transposed (S^T = K Q^T, O^T = V^T P^T with v_mfma_f32_32x32x16_bf16; a lane owns one query's column of both):
 // NQ groups of 32 queries, one head per workgroup, KB entries of the workgroup's key list at a time through LDS; the blocks of 32 keys are
 // dealt to KS waves per group, whose sums meet in LDS at the end.
-template <int DQ, int DV, int NQ, int KS>
+template <int DQ, int DV, int NQ, int KS, typename Ahead>
 __global__ __launch_bounds__(64 * NQ * KS) __attribute__((amdgpu_waves_per_eu(2, 2))) void window_prefill_kernel(
     NcWindowGeom g, const bf16_t* __restrict__ q, int ldq, const bf16_t* __restrict__ cache, const float* __restrict__ sink,
-    const int32_t* __restrict__ seqlens, bf16_t* __restrict__ out, int ldo, NcAhead ahead) {
+    const int32_t* __restrict__ seqlens, bf16_t* __restrict__ out, int ldo, Ahead ahead) {
     constexpr int KPITCH = DQ * 2 + 16, VPITCH = DV * 2 + 64, NW = NQ * KS, NTHR = 64 * NW, KB = 16 * NW, QT = 32 * NQ;
     constexpr int KCH = DQ / 8, VCH = DV / 8, KL = KB * KCH / NTHR, VL = KB * VCH / NTHR;
     constexpr int STAGE = KB * KPITCH + KB * VPITCH, O_PITCH = DV + 4, SUM = KS > 1 ? NQ * 32 * (O_PITCH + 2) * 4 : 0;
@@ -657,9 +657,13 @@ template <int DQ, int DV>
 int launch_prefill(const NcWindowGeom& g, const bf16_t* q, int ldq, const bf16_t* cache, const float* sink, const int32_t* seqlens, bf16_t* out, int ldo,
                    const NcAhead* ahead, hipStream_t s) {
     if ((int64_t)((g.T + 127) / 128) * g.heads * g.B >= 2 * nc_cu_count())
-        hipLaunchKernelGGL((window_prefill_kernel<DQ, DV, 4, 1>), nc_ahead_grid(dim3((g.T + 127) / 128, g.heads, g.B), ahead), dim3(256), 0, s, g, q, ldq, cache, sink, seqlens, out, ldo, ahead ? *ahead : NcAhead{});
+        nc_launch_ahead(dim3((g.T + 127) / 128, g.heads, g.B), ahead, [&](dim3 grid, auto a) {
+            hipLaunchKernelGGL((window_prefill_kernel<DQ, DV, 4, 1, decltype(a)>), grid, dim3(256), 0, s, g, q, ldq, cache, sink, seqlens, out, ldo, a);
+        });
     else
-        hipLaunchKernelGGL((window_prefill_kernel<DQ, DV, 2, 2>), nc_ahead_grid(dim3((g.T + 63) / 64, g.heads, g.B), ahead), dim3(256), 0, s, g, q, ldq, cache, sink, seqlens, out, ldo, ahead ? *ahead : NcAhead{});
+        nc_launch_ahead(dim3((g.T + 63) / 64, g.heads, g.B), ahead, [&](dim3 grid, auto a) {
+            hipLaunchKernelGGL((window_prefill_kernel<DQ, DV, 2, 2, decltype(a)>), grid, dim3(256), 0, s, g, q, ldq, cache, sink, seqlens, out, ldo, a);
+        });
     NC_CHECK_LAUNCH("window_prefill");
     return 0;
 }
