@@ -118,3 +118,12 @@ def test_which_prompts_read_weights_ahead():
     assert not any(ahead(13, B, T) for B, T in [(1, 16), (1, 64), (4, 16), (1, 65), (4, 20), (1, 128), (500, 1), (200, 2), (10, 15)])
     assert all(ahead(13, B, T) for B, T in [(1, 129), (9, 16), (1, 1792), (8, 1024)])
     assert [ahead(10, 1, T) for T in (16, 64, 65, 128, 129)] == [0, 0, 1, 1, 1]
+
+
+def test_models_that_stay_in_the_last_level_cache_read_nothing_ahead():
+    """Weights and the prompt's keys and values together: depth 12 with any prompt, depth 14 (164 MB) up to some 700 tokens, depth 16 (234 MB) never."""
+    def ahead(heads, T, kv_heads=None):
+        m = _lib.ModelDesc(n_layer=2 * heads, n_head=heads, n_kv_head=kv_heads or heads, n_embd=128 * heads, vocab_size=32768)
+        return _lib.lib().nc_gpt_reads_ahead(ctypes.byref(m), 1, T)
+    assert not any(ahead(heads, T) for heads in (2, 4, 6) for T in (129, 500, 1792))
+    assert [ahead(7, T) for T in (200, 400, 1000, 1792)] == [0, 0, 1, 1] and ahead(8, 130) == 1 and ahead(7, 1000, kv_heads=1) == 0
