@@ -607,37 +607,21 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_bl_kernel(const uint8_t* 
 }
 
 
-// Per-process cache of what never changes while the process lives: which kernels have had their dynamic LDS limit raised on which device (hipFuncSetAttribute costs microseconds per call, a launch-bound caller notices).
 #include <atomic>
 namespace {
-constexpr int NC_GEMM_MAX_DEVICES = 64;
-int current_device() {
-    int dev = 0;
-    return hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < NC_GEMM_MAX_DEVICES ? dev : 0;
-}
 int cu_count() { return nc_cu_count(); }
-// slot: one per kernel family that asks for dynamic LDS (the attribute is set for the instantiation actually launched, so the
-// cache is keyed by the function pointer as well)
-hipError_t reserve_lds(const void* fn, int bytes) {
-    struct Entry {
-        std::atomic<const void*> fn;
-        std::atomic<int> bytes;
-    };
-    static Entry done[NC_GEMM_MAX_DEVICES][32];
-    const int dev = current_device();
-    for (auto& e : done[dev]) {
-        const void* f = e.fn.load(std::memory_order_acquire);
-        if (f == fn && e.bytes.load(std::memory_order_relaxed) >= bytes) return hipSuccess;
-        if (f == nullptr || f == fn) {
-            const hipError_t rc = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-            if (rc == hipSuccess) {
-                e.bytes.store(bytes, std::memory_order_relaxed);
-                e.fn.store(fn, std::memory_order_release);
-            }
-            return rc;
-        }
-    }
-    return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);      // table full: just set it
+// Raises a kernel's limit of dynamic LDS (always to the same value), once per device.  The flags belong to the kernel: over
+// fifty of them ask here, and a table that they shared had room for 32, behind which every launch searched it and set the limit again (0.1 us of 5.7).
+template <auto KERNEL>
+int reserve_lds(size_t bytes) {
+    static std::atomic<uint64_t> done{0};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev > 63) dev = 0;
+    if (done.load(std::memory_order_acquire) >> dev & 1) return 0;
+    const hipError_t e = hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", bytes, hipGetErrorString(e));
+    done.fetch_or(1ull << dev, std::memory_order_release);
+    return 0;
 }
 }  // namespace
 
@@ -645,9 +629,7 @@ template <int BM, int BN, int WGM, int WGN, bool INTERLEAVE, int A_FMT, int OUT_
 static int launch_bl_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s) {
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     const size_t lds_bytes = 2 * (size_t)(BM + BN) * 128;
-    const void* fn = (const void*)gemm_bl_kernel<BM, BN, WGM, WGN, OUT_KIND, INTERLEAVE, A_FMT>;
-    hipError_t e = reserve_lds(fn, (int)lds_bytes);
-    if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
+    if (int rc = reserve_lds<gemm_bl_kernel<BM, BN, WGM, WGN, OUT_KIND, INTERLEAVE, A_FMT>>(lds_bytes)) return rc;
     hipLaunchKernelGGL((gemm_bl_kernel<BM, BN, WGM, WGN, OUT_KIND, INTERLEAVE, A_FMT>), dim3(tiles_m * tiles_n), dim3(64 * WGM * WGN), lds_bytes, s, a, b,
                        ep, M, N, K, tiles_m, tiles_n);
     return 0;
@@ -1419,9 +1401,7 @@ template <int A_FMT, int OUT_KIND>
 static int launch_dl_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, bool persistent, hipStream_t s) {
     const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
     const size_t lds_bytes = persistent ? 2 * 512 * 128 + 8 * 4096 : OUT_KIND == 0 ? dl_ring_lds<true, 8, 4>() : 2 * 512 * 128;
-    const void* fn = persistent ? (const void*)gemm_dlp_kernel<A_FMT, OUT_KIND == 2> : (const void*)gemm_dl_kernel<A_FMT, OUT_KIND>;
-    hipError_t e = reserve_lds(fn, (int)lds_bytes);
-    if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
+    if (int rc = persistent ? reserve_lds<gemm_dlp_kernel<A_FMT, OUT_KIND == 2>>(lds_bytes) : reserve_lds<gemm_dl_kernel<A_FMT, OUT_KIND>>(lds_bytes)) return rc;
     if (persistent)
         hipLaunchKernelGGL((gemm_dlp_kernel<A_FMT, OUT_KIND == 2>), dim3(256), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m / 8, (N + 127) / 128);
     else
@@ -1467,9 +1447,7 @@ template <int NJ, int OUT_KIND, int A_FMT>
 static int launch_dln_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s) {
     const int tiles_m = (M + 255) / 256, tiles_n = (N + 32 * NJ - 1) / (32 * NJ);
     const size_t lds_bytes = dl_ring_lds<true, NJ, 4>();
-    const void* fn = (const void*)gemm_dln_kernel<NJ, OUT_KIND, A_FMT>;
-    hipError_t e = reserve_lds(fn, (int)lds_bytes);
-    if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
+    if (int rc = reserve_lds<gemm_dln_kernel<NJ, OUT_KIND, A_FMT>>(lds_bytes)) return rc;
     hipLaunchKernelGGL((gemm_dln_kernel<NJ, OUT_KIND, A_FMT>), dim3(tiles_m * tiles_n), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
     return 0;
 }
@@ -1498,9 +1476,7 @@ template <int BM, int OUT_KIND, typename Rope = NoRope>
 static int launch_dr_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s, int splits = 1, Rope rope = Rope{}) {
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + 127) / 128;
     const size_t lds_bytes = 4 * (size_t)(BM + 128) * 128;
-    const void* fn = (const void*)gemm_dr_kernel<BM, OUT_KIND, Rope>;
-    hipError_t e = reserve_lds(fn, (int)lds_bytes);
-    if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
+    if (int rc = reserve_lds<gemm_dr_kernel<BM, OUT_KIND, Rope>>(lds_bytes)) return rc;
     hipLaunchKernelGGL((gemm_dr_kernel<BM, OUT_KIND, Rope>), dim3(tiles_m * tiles_n, splits), dim3(256), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n, rope);
     return 0;
 }
@@ -1533,8 +1509,7 @@ template <int BM, int BN>
 static int launch_tile(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s) {
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     const size_t lds_bytes = 2 * (size_t)(BM + BN) * 128;
-    hipError_t e = reserve_lds((const void*)gemm_tile_kernel<BM, BN>, (int)lds_bytes);
-    if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
+    if (int rc = reserve_lds<gemm_tile_kernel<BM, BN>>(lds_bytes)) return rc;
     hipLaunchKernelGGL((gemm_tile_kernel<BM, BN>), dim3(tiles_m * tiles_n), dim3(256), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
     return 0;
 }
@@ -1689,8 +1664,7 @@ template <int WTM>
 static int launch_gemm_rope(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, const RopeArgs& rope, int M, int N, int K, hipStream_t s) {
     const int tiles_m = (M + 64 * WTM - 1) / (64 * WTM), tiles_n = N / 128;
     const size_t lds_bytes = dl_ring_lds<false, WTM, 2>();
-    const hipError_t e = reserve_lds((const void*)gemm_rope_kernel<WTM>, (int)lds_bytes);
-    if (e != hipSuccess) NC_FAIL(-2, "fp8_gemm: cannot reserve %zu bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
+    if (int rc = reserve_lds<gemm_rope_kernel<WTM>>(lds_bytes)) return rc;
     hipLaunchKernelGGL(gemm_rope_kernel<WTM>, dim3(tiles_m * tiles_n), dim3(512), lds_bytes, s, a, b, ep, rope, M, N, K, tiles_m, tiles_n);
     return 0;
 }
