@@ -376,7 +376,7 @@ __global__ __launch_bounds__(256 * (Q8_ROWS > 1 ? Q8_ROWS : 1)) void mix_norm_ve
                 if (c < 16) *(uint4*)(xn_out + base + c) = o[it];
             }
         };
-        const bool here = meeting<4 * ROWS, 4>(q8.meeting, gridDim.x, blockIdx.x, am, amax, left, meanwhile,
+        const bool here = meeting<4 * ROWS>(q8.meeting, gridDim.x, blockIdx.x, am, amax, left, meanwhile,
                                                           [&] { each([&](size_t at, const uint4& w) { *(uint4*)(xn_out + at) = w; }); });
         if (!here) return;
         const float scale = scale_from_amax(amax);
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(64 * WAVES) void mix_norm_rows_kernel(bf16_t* __res
                 if (c < 16) *(uint4*)(xn_out + base + c) = o[w];
             }
         };
-        const bool here = meeting<WAVES, 4>(q8.meeting, gridDim.x, blockIdx.x, am, amax, left, meanwhile,
+        const bool here = meeting<WAVES>(q8.meeting, gridDim.x, blockIdx.x, am, amax, left, meanwhile,
                                                               [&] { each([&](size_t at, const uint4& w) { *(uint4*)(xn_out + at) = w; }); });
         if (!here) return;
         const float scale = scale_from_amax(amax);
@@ -663,10 +663,9 @@ int nc_launch_embed_norm_smear(const int64_t* idx, const bf16_t* wte, const floa
 bool nc_mix_norm_wave_rows(int rows, int cols) { return cols % 8 == 0 && cols <= 2048 && rows >= 512 + 256 * ((cols + 511) / 512); }
 
 // Rows as e4m3: a workgroup of 512 threads holds eight rows, a wave to a row, or, where the addend comes as partial sums, 256 threads to a row, one, two or
-// four rows.  At most one workgroup to a CU, and no more than 256 of them (nc_meeting.h).
+// four rows.  One workgroup to a CU at most (nc_meeting_wgs).
 #define ROWS_Q8 8
-static int mix_norm_e4m3_wgs() { return nc_cu_count() < 256 ? nc_cu_count() : 256; }
-bool nc_mix_norm_e4m3_fits(int rows, int cols, bool parts) { return cols % 16 == 0 && cols <= 2048 && rows <= (parts ? 4 : ROWS_Q8) * mix_norm_e4m3_wgs(); }
+bool nc_mix_norm_e4m3_fits(int rows, int cols, bool parts) { return cols % 16 == 0 && cols <= 2048 && rows <= (parts ? 4 : ROWS_Q8) * nc_meeting_wgs(); }
 
 static int launch_mix_norm_impl(bf16_t* x, const bf16_t* add, NcPartialSrc padd, const bf16_t* x0, const float* resid_lambda,
                                 const float* x0_lambda, const float* backout_lambda, const bf16_t* backout_src, bf16_t* backout_save,
@@ -690,7 +689,7 @@ static int launch_mix_norm_impl(bf16_t* x, const bf16_t* add, NcPartialSrc padd,
         else hipLaunchKernelGGL((mix_norm_vec_kernel<NVV, false>), dim3(rows), dim3(256), 0, s, MIX_ARGS);                \
     } while (0)
     if (q8) {
-        const int wgs = mix_norm_e4m3_wgs();
+        const int wgs = nc_meeting_wgs();
         NC_CHECK_ARG(aligned && !bump && ((uintptr_t)q8->out & 7) == 0 && q8->inv_out && q8->meeting.words && nc_mix_norm_e4m3_fits(rows, cols, padd.parts != nullptr),
                      "mix_norm: rows=%d cols=%d cannot be written as e4m3", rows, cols);
         NcQuantRows q = *q8;

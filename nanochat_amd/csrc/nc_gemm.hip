@@ -353,7 +353,7 @@ __device__ __forceinline__ void q8_epilogue(v4f (&acc)[BM / WGM / 16][BN / WGN /
     }
     float amax;
     bool left;
-    const bool here = meeting<WGM * WGN, 4>(ep.meeting, gridDim.x, blockIdx.x, am, amax, left, [] {}, [&] {
+    const bool here = meeting<WGM * WGN>(ep.meeting, gridDim.x, blockIdx.x, am, amax, left, [] {}, [&] {
 #pragma unroll
         for (int j = 0; j < WTN; j++)
 #pragma unroll
@@ -1705,7 +1705,7 @@ int nc_gemm_relu2_e4m3_kernel(int M, int N, int K) {
     const int bn = which >= 16 && which <= 18 ? 128 : which >= 12 && which <= 15 ? 32 * (which - 8) : 256;
     if (which != 8 && (which < 12 || which > 18)) return 0;
     const long wgs = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
-    return wgs <= cu_count() && wgs <= 256 ? which : 0;
+    return wgs <= nc_meeting_wgs() ? which : 0;
 }
 
 int nc_launch_gemm_relu2_e4m3(const uint8_t* a, const uint8_t* b, const float* inv_a, const float* inv_b, uint8_t* out, float* inv_out, uint32_t* out_amax,

@@ -4,8 +4,8 @@
 // Memory (NC_MEETING_WORDS words, all zero before the launch): one word per workgroup, its maximum with the top bit set once it has arrived, and
 // behind them one bit per workgroup that left (below).  One trip to memory out, one back: every workgroup stores its word and polls everybody's, so
 // there is no counter for hundreds of atomics to queue up at.  What the polls cost grows with the square of the workgroups, all of them reading the same
-// lines (row passes of 1792 rows: 112 workgroups 12.1 us, 224 10.7, 448 13.7), so few large workgroups meet best, and none beyond 256 but for attention's.  Words and
-// bits are read and written with device-scope atomics, at the device's point of coherence; no fence is needed on the way everybody takes.
+// lines (row passes of 1792 rows: 112 workgroups 12.1 us, 224 10.7, 448 13.7), so few large workgroups meet best; a launch that meets has at most
+// NC_MEETING_WGS (nc_meeting_wgs).  Words and bits are read and written with device-scope atomics, at the device's point of coherence; no fence is needed on the way everybody takes.
 //
 // The launch is sized so that the chip holds all of it, but a workgroup may still not have started because another stream's kernel has its place.
 // The wait is therefore bounded: a workgroup whose polls run out LEAVES.  It stores its values as bf16 in memory, makes them visible, sets its bit and
@@ -15,10 +15,16 @@
 // goes on like everybody), or its bit was set before Z's word was and Z sees it.
 #pragma once
 #include "nc_common.h"
+#include "nc_kernels.h"
 
-#define NC_MEETING_WGS 512
+#define NC_MEETING_WGS 256               // a word and a bit each, and every poll looks at all of them
 #define NC_MEETING_WORDS (NC_MEETING_WGS + NC_MEETING_WGS / 32)
 #define NC_MEETING_SPINS 400u             // polls of about half a microsecond before a workgroup leaves
+
+static_assert(NC_MEETING_WGS % 64 == 0 && NC_MEETING_WGS / 32 <= 64, "a wave looks at 64 words at a time and at all bits at once");
+
+// how many workgroups of one to a compute unit can meet
+static inline int nc_meeting_wgs() { return nc_cu_count() < NC_MEETING_WGS ? nc_cu_count() : NC_MEETING_WGS; }
 
 struct NcMeeting {
     uint32_t* words;          // nullptr: none
@@ -39,10 +45,10 @@ struct MeetingView {
     bool left;                //   somebody has left values behind
 };
 
-// For one whole wave of the workgroup; `mine` is the workgroup's maximum (a non-negative float's bits, NaN included), POLLS * 64 >= workgroups.
-template <int POLLS>
+// For one whole wave of the workgroup (a maximum is a non-negative float's bits, NaN included).
 __device__ __forceinline__ MeetingView meeting_look(const NcMeeting& m, int wgs) {
     const int lane = threadIdx.x & 63;
+    constexpr int POLLS = NC_MEETING_WGS / 64;
     uint32_t v[POLLS];
 #pragma unroll
     for (int i = 0; i < POLLS; i++) {
@@ -58,10 +64,9 @@ __device__ __forceinline__ MeetingView meeting_look(const NcMeeting& m, int wgs)
     }
     return MeetingView{__builtin_amdgcn_ballot_w64(all == 0u) == 0, mx, __builtin_amdgcn_ballot_w64(bits != 0u) != 0};
 }
-template <int POLLS>
 __device__ __forceinline__ MeetingView meeting_wait(const NcMeeting& m, int wgs) {
     for (uint32_t spin = 0;; spin++) {
-        MeetingView view = meeting_look<POLLS>(m, wgs);
+        MeetingView view = meeting_look(m, wgs);
         if (view.complete || spin >= m.spins) {
             view.amax = wave_max_u32(view.amax);
             return view;
@@ -74,7 +79,7 @@ __device__ __forceinline__ MeetingView meeting_wait(const NcMeeting& m, int wgs)
 // leave() stores the workgroup's values as bf16.
 // Returns false when the workgroup left (its values are in memory and somebody else's business), else true with the tensor's amax and whether
 // meeting_take has to be called once the workgroup's own values are converted.
-template <int WAVES, int POLLS, typename Meanwhile, typename Leave>
+template <int WAVES, typename Meanwhile, typename Leave>
 __device__ __forceinline__ bool meeting(const NcMeeting& m, int wgs, int self, float am, float& amax, bool& left, Meanwhile&& meanwhile, Leave&& leave) {
     __shared__ uint32_t red[WAVES], out[3];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -91,7 +96,7 @@ __device__ __forceinline__ bool meeting(const NcMeeting& m, int wgs, int self, f
     meanwhile();
     if (wave == 0) {
         asm volatile("" ::"v"(before) : "memory");       // the word is there (the exchange has returned) before anything is looked at
-        const MeetingView view = meeting_wait<POLLS>(m, wgs);
+        const MeetingView view = meeting_wait(m, wgs);
         if (lane == 0) out[0] = view.complete, out[1] = view.amax, out[2] = view.left;
     }
     __syncthreads();
@@ -107,7 +112,7 @@ __device__ __forceinline__ bool meeting(const NcMeeting& m, int wgs, int self, f
             asm volatile("" ::: "memory");
             __builtin_amdgcn_s_waitcnt(0);
             asm volatile("" ::: "memory");
-            MeetingView view = meeting_look<POLLS>(m, wgs);
+            MeetingView view = meeting_look(m, wgs);
             view.amax = wave_max_u32(view.amax);
             if (lane == 0) out[0] = view.complete, out[1] = view.amax, out[2] = view.left;
         }
@@ -137,7 +142,7 @@ __device__ __forceinline__ void meeting_take(const NcMeeting& m, int wgs, Conver
     }
 }
 
-// sixteen bf16 values, two 16-byte vectors, as e4m3
+// four bf16 values, and sixteen (two 16-byte vectors), as e4m3
 __device__ __forceinline__ uint32_t e4m3_of_bf16x4(uint32_t lo, uint32_t hi, float scale) {
     return fp8_pack4<0, true>(clamp448(bf16_lo(lo) * scale), clamp448(bf16_hi(lo) * scale), clamp448(bf16_lo(hi) * scale), clamp448(bf16_hi(hi) * scale));
 }

@@ -127,3 +127,10 @@ def test_models_that_stay_in_the_last_level_cache_read_nothing_ahead():
         return _lib.lib().nc_gpt_reads_ahead(ctypes.byref(m), 1, T)
     assert not any(ahead(heads, T) for heads in (2, 4, 6) for T in (129, 500, 1792))
     assert [ahead(7, T) for T in (200, 400, 1000, 1792)] == [0, 0, 1, 1] and ahead(8, 130) == 1 and ahead(7, 1000, kv_heads=1) == 0
+
+
+def test_a_launch_that_meets_has_a_word_for_every_workgroup():
+    """The words' size follows from the most workgroups that may meet, and no shape is let in that has one more (257 tiles of 256 x 256)."""
+    lib = _lib.lib()
+    assert lib.nc_fp8_meeting_bytes() == 4 * (256 + 256 // 32)
+    assert [lib.nc_fp8_gemm_relu2_e4m3_fits(M, 4096, 512) for M in (4096, 4097)] == [1, 0]
