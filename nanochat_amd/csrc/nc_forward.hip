@@ -217,7 +217,7 @@ struct LinearRunner {
         *out8 = nullptr;
         if (rows <= 128 || !nc_gemm_relu2_e4m3_kernel(rows, N, K)) return false;
         *rc = in8 ? 0 : nc_launch_convert_only(in, (int64_t)rows * K, w.a8, w.inv + site, w.site(site), s);
-        if (!*rc) *rc = nc_launch_gemm_relu2_e4m3(w.a8, w8, w.inv + site, inv_w, (uint8_t*)w.h, w.inv + out_site, w.site(out_site), w.h2,
+        if (!*rc) *rc = nc_launch_gemm_relu2_e4m3(in8 ? in8 : w.a8, w8, w.inv + site, inv_w, (uint8_t*)w.h, w.inv + out_site, w.site(out_site), w.h2,
                                                    w.meeting(out_site), rows, N, K, s);
         *out8 = (const uint8_t*)w.h;
         return true;
