@@ -1486,7 +1486,8 @@ static int launch_dr(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep,
     NC_CHECK_ARG((long)M * K < (1L << 31) && (long)N * K < (1L << 31), "fp8_gemm: buffer-load kernels need M*K and N*K below 2^31");
     NC_CHECK_ARG(K % 128 == 0, "fp8_gemm: the direct-to-LDS kernels need K %% 128 == 0, got %d", K);
     NC_CHECK_ARG(ep.out_kind != 1, "fp8_gemm: the direct-to-LDS kernels write bf16 only");
-    if (ep.out_kind == 4) return launch_dr_as<BM, 4>(a, b, ep, M, N, K, s);
+    if constexpr (BM < 128)
+        if (ep.out_kind == 4) return launch_dr_as<BM, 4>(a, b, ep, M, N, K, s);      // (what pick_kernel takes)
     return ep.out_kind == 2 ? launch_dr_as<BM, 2>(a, b, ep, M, N, K, s) : launch_dr_as<BM, 0>(a, b, ep, M, N, K, s);
 }
 
@@ -1701,9 +1702,8 @@ int nc_launch_gemm_qkv_rope(const uint8_t* a, const uint8_t* b, const float* inv
 int nc_gemm_relu2_e4m3_kernel(int M, int N, int K) {
     if (M <= 128 || N % 16 != 0 || K % 128 != 0 || (long)M * K >= (1L << 31) || (long)N * K >= (1L << 31)) return 0;
     const int which = pick_kernel(M, N, K, 2);
-    const int bm = which == 16 ? 64 : which == 17 ? 96 : which == 18 ? 128 : 256;
-    const int bn = which >= 16 && which <= 18 ? 128 : which >= 12 && which <= 15 ? 32 * (which - 8) : 256;
-    if (which != 8 && (which < 12 || which > 18)) return 0;
+    const int bm = which == 16 ? 64 : which == 17 ? 96 : 256, bn = which >= 16 ? 128 : which >= 12 ? 32 * (which - 8) : 256;
+    if (which != 8 && (which < 12 || which > 17)) return 0;
     const long wgs = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
     return wgs <= nc_meeting_wgs() ? which : 0;
 }
@@ -1718,8 +1718,7 @@ int nc_launch_gemm_relu2_e4m3(const uint8_t* a, const uint8_t* b, const float* i
     NcProfScope prof(1, 2.0 * M * N * K, s, ((int64_t)N << 32) | (uint32_t)K);
     const int rc = which == 8 ? launch_dl<0>(a, b, ep, M, N, K, false, s)
                    : which == 16 ? launch_dr<64>(a, b, ep, M, N, K, s)
-                   : which == 17 ? launch_dr<96>(a, b, ep, M, N, K, s)
-                   : which == 18 ? launch_dr<128>(a, b, ep, M, N, K, s) : launch_dln(which - 8, 0, a, b, ep, M, N, K, s);
+                   : which == 17 ? launch_dr<96>(a, b, ep, M, N, K, s) : launch_dln(which - 8, 0, a, b, ep, M, N, K, s);
     if (rc) return rc;
     NC_CHECK_LAUNCH("fp8_gemm_relu2_e4m3");
     return 0;
