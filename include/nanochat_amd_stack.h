@@ -155,6 +155,12 @@ int nc_stack_forward(const nc_stack_model* model /*host*/, const nc_stack_cache*
 int nc_stack_linear(int dtype, const void* a, int64_t lda, const void* w, void* out, int ldc, int M, int N, int K, int kind, float limit,
                     int kernel, nc_stream_t stream);
 
+/* The same with its columns in up to four runs that each go their own way, as the forward's stacked weights do: run i ends behind column ends[i] (a multiple
+ * of 16), has a kind and an output of its own; HOST arrays.  Kinds as above and 4 (float, added to what is there) and, for the last run, which may end
+ * anywhere, 5 (float logits, soft-capped at limit if it is above 0). */
+int nc_stack_linear_runs(int dtype, const void* a, int64_t lda, const void* w, int M, int N, int K, int n_runs, const int32_t* ends, const int32_t* kinds,
+                         void* const* outs, const int32_t* lds, float limit, int kernel, nc_stream_t stream);
+
 /* KVCache.prefill for one slot of either kind of cache: rows [0, n_bytes) of every batch row, src_rows 1 (broadcast) or dst_rows. */
 int nc_stack_cache_copy(const void* src, void* dst, int src_rows, int dst_rows, int64_t src_row_bytes, int64_t dst_row_bytes,
                         int64_t n_bytes, nc_stream_t stream);

@@ -522,6 +522,21 @@ extern "C" int nc_stack_linear(int dtype, const void* a, int64_t lda, const void
     return nc_launch_linear_tiled(dtype, l, (hipStream_t)stream, NC_CLS_LINEAR, kernel - 2);
 }
 
+extern "C" int nc_stack_linear_runs(int dtype, const void* a, int64_t lda, const void* w, int M, int N, int K, int n_runs, const int32_t* ends, const int32_t* kinds,
+                                    void* const* outs, const int32_t* lds, float limit, int kernel, nc_stream_t stream) {
+    NC_CHECK_ARG(ends && kinds && outs && lds && n_runs >= 1 && n_runs <= 4 && ends[n_runs - 1] == N && kernel >= 0 && kernel <= 9, "stack_linear_runs: %d runs of %d columns", n_runs, N);
+    NcLinear l = nc_linear(a, lda, w, M, N, K);
+    for (int i = 0; i < n_runs; i++) {
+        const bool logits = kinds[i] == NC_SEG_LOGITS;
+        NC_CHECK_ARG(outs[i] && kinds[i] >= NC_SEG_PLAIN && kinds[i] <= NC_SEG_SWIGLU && ends[i] > (i ? ends[i - 1] : 0) && (logits ? i + 1 == n_runs : ends[i] % 16 == 0),
+                     "stack_linear_runs: run %d of kind %d ends at %d", i, kinds[i], ends[i]);
+        nc_linear_seg(l, ends[i], kinds[i], outs[i], lds[i], logits ? 1.f : limit, logits ? limit : 0.f);
+    }
+    if (kernel == 0) return nc_launch_linear(dtype, l, (hipStream_t)stream);
+    if (kernel == 1) return nc_launch_linear_few(dtype, l, (hipStream_t)stream);
+    return nc_launch_linear_tiled(dtype, l, (hipStream_t)stream, NC_CLS_LINEAR, kernel - 2);
+}
+
 extern "C" int nc_stack_cache_copy(const void* src, void* dst, int src_rows, int dst_rows, int64_t src_row_bytes, int64_t dst_row_bytes, int64_t n_bytes,
                                    nc_stream_t stream) {
     return nc_launch_stack_cache_copy(src, dst, src_rows, dst_rows, src_row_bytes, dst_row_bytes, n_bytes, (hipStream_t)stream);

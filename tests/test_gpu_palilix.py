@@ -90,6 +90,38 @@ def test_wide_tiles_have_the_sums_of_the_others(kind):
         assert torch.equal(ops.stack_linear(a, w, kind=kind, limit=0.6, kernel=9), want), (M, N, K)
 
 
+# columns and kind of each run; the ends lie inside tiles of 256, inside halves of them, on a tile's border, and the last one inside a group of eight columns
+WIDE_RUNS = {"mixers, router, GLU": [(208, 0), (64, 3), (432, 2)], "residual": [(560, 4)], "residual behind a border": [(256, 0), (304, 4)], "logits": [(1003, 5)],
+             "four": [(16, 6), (240, 7), (144, 1), (201, 5)]}
+
+
+@pytest.mark.parametrize("M", [130, 257, 1700])
+@pytest.mark.parametrize("runs", WIDE_RUNS)
+def test_wide_tiles_of_stacked_weights(runs, M):
+    """What a forward sends through the 256 x 256 tiles: several runs of columns, sums added to the residual stream, logits; whole tiles and, for 1700 rows, halves
+    behind 256 of them.  To the bit those of the 64 x 64 tiles, also where the kernel is chosen; nothing else is written."""
+    say(f"256 x 256 tiles, {runs}, {M} rows")
+    g = torch.Generator(device=DEV).manual_seed(M)
+    parts = WIDE_RUNS[runs]
+    if M == 1700 and len(parts) < 4:
+        parts = [(9472, 0)] + parts                  # (280 tiles and more; those behind the 256th are cut into halves)
+    N, K = sum(cols for cols, _ in parts), 192
+    a, w = torch.randn(M, K, generator=g, device=DEV).bfloat16(), (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).bfloat16()
+    stream = torch.randn(M, 1024, generator=g, device=DEV)
+    got = []
+    for kernel in (4, 9, 0):
+        # (rows longer than their columns, and a row behind the last)
+        room = [torch.full((M + 1, (cols // 2 if kind in (2, 7) else cols) + 8), 7.0, dtype=torch.float32 if kind in (3, 4, 5) else torch.bfloat16, device=DEV) for cols, kind in parts]
+        views = [t[:M, :-8] for t in room]
+        for (cols, kind), v in zip(parts, views):
+            if kind == 4:
+                v.copy_(stream[:, :cols])
+        ops.stack_linear_runs(a, w, [(cols, kind, v) for (cols, kind), v in zip(parts, views)], limit=0.6, kernel=kernel)
+        assert all((t[M] == 7).all() and (t[:, -8:] == 7).all() for t in room)
+        got.append([v.clone() for v in views])
+    assert all(torch.equal(x, y) for other in got[1:] for x, y in zip(got[0], other))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_few_rows_have_the_same_sums_in_every_kernel(dtype):
     """Up to 64 rows a result does not depend on the kernel or the tile: the same additions in the same order, to the bit (sums of one K-step, of
