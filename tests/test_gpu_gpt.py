@@ -434,6 +434,35 @@ def test_shared_out_projection_is_the_one_in_one_piece(heads, rows, of):
     assert (off <= 2.0 ** -6 * many[1].abs().clamp(min=many[1].abs().mean())).all(), off.max().item()
 
 
+@pytest.mark.parametrize("depth,T", [(4, 1792), (6, 300), (12, 1000)])
+def test_prompts_on_two_streams(depth, T):
+    """Two prompts at once, each with a model, a cache and a stream of its own: the launches whose workgroups wait for each other share the chip with another
+    stream's.  Logits and caches as of one prompt after the other, to the bit."""
+    from nanochat_amd.engine import KVCache
+    from nanochat_amd.synthetic import config_for_depth, random_init_model
+    say(f"two streams, depth {depth}, {T} tokens")
+    cfg = config_for_depth(depth, vocab_size=1024)
+    models = [random_init_model(cfg, DEV, seed=i) for i in range(2)]
+    prompts = [torch.randint(0, 1024, (1, T), generator=torch.Generator().manual_seed(i)).to(DEV) for i in range(2)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+
+    def caches():
+        return [KVCache(1, cfg.n_kv_head, T, 128, cfg.n_layer, DEV, torch.bfloat16) for _ in range(2)]
+    alone = caches()
+    want = [m.forward_last(p, kv_cache=c).clone() for m, p, c in zip(models, prompts, alone)]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        together = caches()
+        torch.cuda.synchronize()
+        got = [None, None]
+        for i in range(2):
+            with torch.cuda.stream(streams[i]):
+                got[i] = models[i].forward_last(prompts[i], kv_cache=together[i])
+        torch.cuda.synchronize()
+        for i in range(2):
+            assert torch.equal(got[i], want[i]) and torch.equal(together[i].k_cache, alone[i].k_cache) and torch.equal(together[i].v_cache, alone[i].v_cache)
+
+
 @pytest.mark.parametrize("heads,kv_heads,B,T", [(2, 2, 1, 130), (2, 1, 3, 100), (4, 1, 1, 700), (3, 3, 40, 20)])
 def test_prompts_that_read_weights_ahead(heads, kv_heads, B, T):
     """A model that is large by its vocabulary, so that attention's launch reads the next weights ahead, and the same model without most of the vocabulary,

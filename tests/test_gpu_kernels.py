@@ -400,6 +400,29 @@ def test_gemm_relu2_written_as_e4m3(ops, M, N, K, spin_limit):
         assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)) and inv.item() == want_inv.item()
 
 
+@pytest.mark.parametrize("spin_limit", [-1, 0])
+@pytest.mark.parametrize("what", ["zeros", "not a number", "overflow"])
+@pytest.mark.parametrize("M,N,K", [(1792, 6656, 1664), (300, 336, 256), (1000, 2256, 384)])
+def test_gemm_relu2_written_as_e4m3_at_the_ends_of_the_numbers(ops, M, N, K, what, spin_limit):
+    """A result of zeros, one row of NaN, squares beyond bfloat16: payload and inverse scale are those of the two launches, bit for bit."""
+    say(f"gemm relu2 e4m3 of {what} M={M} N={N} K={K} spins={spin_limit}")
+    a, w = make_operands(M, N, K, seed=M)
+    a8, ia, _ = fp8_ref.to_fp8(a)
+    w8, iw, _ = fp8_ref.to_fp8(w)
+    a8, w8, ia, iw = (t.to(DEV) for t in (a8, w8, ia, iw))
+    if what == "zeros":
+        a8.view(torch.uint8).zero_()
+    elif what == "not a number":
+        a8.view(torch.uint8)[M // 2, 3] = 0x7F
+    else:
+        ia = ia * 1e30
+    h, _ = ops.fp8_gemm_relu2(a8, w8, ia, iw)
+    assert {"zeros": not h.any(), "not a number": h.isnan().any(), "overflow": h.isinf().any()}[what]
+    want, want_inv, _ = ops.fp8_quantize(h)
+    got, inv = ops.fp8_gemm_relu2_e4m3(a8, w8, ia, iw, spin_limit=spin_limit)
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)) and torch.equal(inv.view(torch.int32), want_inv.view(torch.int32))
+
+
 def test_gemm_softcap_epilogue(ops):
     say("gemm softcap")
     a, w = make_operands(64, 1024, 256, 11)
@@ -912,6 +935,31 @@ def test_mix_norm_written_as_e4m3(ops, rows, cols, splits, spin_limit):
         got_x = x.clone()
         got, inv = ops.mix_norm_e4m3(got_x, **how, **mix, spin_limit=spin_limit)
         assert torch.equal(got_x, want_x) and inv.item() == want_inv.item() and torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+
+
+@pytest.mark.parametrize("spin_limit", [-1, 0])
+@pytest.mark.parametrize("value", [0.0, float("nan"), float("inf")])
+@pytest.mark.parametrize("rows,cols,splits", [(1792, 1664, 0), (333, 1040, 0), (257, 1280, 2), (130, 1024, 8)])
+def test_mix_norm_written_as_e4m3_at_the_ends_of_the_numbers(ops, rows, cols, splits, value, spin_limit):
+    """Rows of zeros alone, a NaN or an infinity in one of them: rows, payload and inverse scale are those of the two launches, bit for bit."""
+    say(f"mix_norm e4m3 of {value} rows={rows} cols={cols} splits={splits} spins={spin_limit}")
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, cols, generator=g).bfloat16().to(DEV)
+    if value == 0.0:
+        x.zero_()
+    else:
+        x[rows // 3, 7] = value
+    how = {}
+    if splits:
+        # (partial sums of zeros: what is added leaves the rows as they are)
+        how = dict(parts=torch.zeros(splits, rows, cols, device=DEV), parts_amax=torch.tensor([f32_bits(3.0)], dtype=torch.int32, device=DEV), parts_inv=torch.ones(1, device=DEV))
+    want_x = x.clone()
+    xn, _ = ops.mix_norm(want_x, torch.zeros_like(x))
+    want, want_inv, _ = ops.fp8_quantize(xn)
+    got_x = x.clone()
+    got, inv = ops.mix_norm_e4m3(got_x, **(how or dict(add=torch.zeros_like(x))), spin_limit=spin_limit)
+    assert torch.equal(got_x.view(torch.int16), want_x.view(torch.int16))
+    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8)) and torch.equal(inv.view(torch.int32), want_inv.view(torch.int32))
 
 
 def test_mix_norm_variants(ops):
