@@ -21,7 +21,7 @@
 //   linear c_fc         relu^2, the meeting, e4m3
 //   linear q|k|v        rotary, QK-norm, gain, VE gate and append in its epilogue
 // otherwise the convert kernel and the rotary kernel follow as launches of their own.  Attention's launch also reads the weights of the next linears ahead
-// (nc_prefetch.h); its output goes through the convert kernel.  The two narrow projections of a few hundred rows leave partial sums to mix_norm as well.
+// where that pays (reads_ahead, nc_prefetch.h); its output goes through the convert kernel.  The two narrow projections of a few hundred rows leave partial sums to mix_norm as well.
 //
 // Workspace (carved from the caller's buffer, 256-byte aligned pieces), M = B*T rows:
 //   x, x0, xn, xb, o      bf16 [M,E]        residual stream, its initial value, normed rows, backout, GEMM out

@@ -1645,7 +1645,9 @@ int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const
 }
 
 // The tiles of the q|k|v linear that finish its heads: those of 64 or 96 x 128 where pick_kernel takes them (16, 17), otherwise 64 WTM x 128 (returned as
-// 100 + WTM) with the least cost by the count of dl_cost, a tile of 64 x 128 being its unit of area; 0: none.
+// 100 + WTM) with the least cost by the count of dl_cost, a tile of 64 x 128 being its unit of area; 0: none.  Also where pick_kernel has the persistent kernel: us a
+// prompt with it and a rotary launch / this way, depth 26, 2 x 1792 tokens 6701 / 6561, 8 x 1024 12652 / 12355, 4096 7649 / 7382, depth 12, 8 x 1024 2643 / 2513, depth 8,
+// 32 x 1024 3418 / 3324; of few key heads (depth 24, 6 of 12, 4 x 1024) 5528 / 5617.
 static int rope_tiles(int M, int N, int K) {
     if (M <= 128 || N % 128 != 0 || K % 128 != 0 || (long)M * K >= (1L << 31) || (long)N * K >= (1L << 31)) return 0;
     const int which = pick_kernel(M, N, K, 0);

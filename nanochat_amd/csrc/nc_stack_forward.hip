@@ -266,8 +266,11 @@ int run_mixers(const nc_stack_model* m, const nc_stack_cache* kv, const nc_stack
 // What a prompt's last mixer reads ahead (nc_prefetch.h): the output matrix, and a dense layer's next input matrix, as far as the memory brings them while the
 // mixer of M rows runs.  us a linear, weights in HBM / in the last-level cache: 1792 rows, 12544 x 2048 107 / 95, 2048 x 4096 45 / 34, 2048 x 8192 81 / 60, 300
 // rows, 6144 x 2048 25 / 16; 32-bit products gain nothing.  us a prompt, without / with: Palilix of width 2048, 1792 tokens, 3648 / 3547, of dense layers, 500
-// tokens, 1175 / 1066 (32 or 64 KB a row, which leaves the input matrix out: 1175), Zodirax of width 2048, 800 tokens, 2285 / 2248.
+// tokens, 1175 / 1066, Zodirax of width 2048, 800 tokens, 2285 / 2248.
 // Beginnings of what does not fit (experts, Zodirax's feed-forward) cost the mixers more than they gave: 3648 -> 3770.
+// The bytes a row are a compromise (us a prompt, 32 / 64 / 96 / 160 KB a row, which takes the input matrix in from ever fewer rows on): one dense Palilix group of width
+// 2048, 300 tokens 572 / 572 / 572 / 518, 500 621 / 622 / 573 / 573, 800 850 / 783 / 784 / 838, 1400 1053 / 1063 / 1114 / 1118, of width 3072, 800 tokens 1294 / 1293 / 1295 / 1224,
+// with experts, width 2048, 500 tokens 889 / 885 / 874 / 871, 1000 1127 / 1109 / 1104 / 1103.  No prompt of these is slower than without reading.
 constexpr size_t AHEAD_BYTES_PER_ROW = 98304;
 bool reads_ahead(const nc_stack_model* m, int M) {
     if (m->dtype || M <= NC_FEW_ROWS) return false;
@@ -290,7 +293,8 @@ NcAhead weights_behind(const nc_stack_model* m, int i, int M) {
     auto add = [&](const void* p, size_t elems) {
         if (2 * elems <= left) a.add(p, 2 * elems), left -= 2 * elems;
     };
-    // (the scans and recurrences of a wide post-norm layer keep the memory busy themselves: width 4096 4280 with its 34 and 67 MB, 4275 without)
+    // (the scans and recurrences of a wide post-norm layer keep the memory busy themselves: Zodirax group of width 4096 (34 and 67 MB), 1792 tokens 4151 with it, 4123
+    // without, 500 tokens 1895 / 1891; of width 2048 500 tokens 862 / 876, 1000 1222 / 1245.  Between them it would pay: width 3072 1367 / 1412)
     if (l.block != NC_BLOCK_POST_NORM || 2 * W * l.k_out <= 24u << 20) add(l.w_out, W * l.k_out);
     if (l.block != NC_BLOCK_POST_NORM && l.ff != NC_FF_EXPERTS && i + 1 < m->n_runs) {
         const nc_stack_layer& next = m->layers[m->runs[i + 1].layer];
