@@ -803,8 +803,14 @@ __device__ __forceinline__ void dl_ring(Acc& acc, const uint8_t* A, int a_bytes,
     if (kt < ksteps) step(kt, std::integral_constant<int, 0>{});
 }
 
+// Short sums take a K loop of two stages: the ring asks for two steps of its held operand before the first products, and what it saves a step is little beside few
+// columns.  us, two stages / ring: 256 x 128 tiles, 2048 x 4096 x 256 8.1 / 8.4, x 1024 12.7 / 12.8, x 1536 16.3 / 16.2, x 4096 34.6 / 32.0; 256 x 160 tiles, 1792 x 4992 x
+// 256 9.5 / 9.7, x 1024 14.7 / 14.9, x 1536 18.4 / 18.3, x 4096 37.0 / 36.4; 256 x 192 tiles, 1792 x 6656 x 128 8.3 / 8.5, x 256 10.0 / 10.1, x 512 12.2 / 12.1; 256 x 256
+// tiles, 8192 x 2048 x 128 10.1 / 10.4, x 256 11.95 / 12.0, x 768 17.2 / 17.3, x 1536 25.5 / 25.3.  NJ: columns of a tile / 32.
+constexpr bool dl_two_stages(int NJ, int K) { return K <= (NJ <= 5 ? 1024 : 128); }
+
 // One tile per workgroup, launched tile by tile (any M, N).
-template <int A_FMT, int OUT_KIND>
+template <int A_FMT, int OUT_KIND, bool RING = OUT_KIND == 0>
 __global__ __launch_bounds__(512) void gemm_dl_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, EpilogueArgs ep, int M,
                                                       int N, int K, int tiles_m, int tiles_n) {
     constexpr int STAGE = 512 * 128;
@@ -841,10 +847,10 @@ __global__ __launch_bounds__(512) void gemm_dl_kernel(const uint8_t* __restrict_
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(i < 4 ? desc_a : desc_b, (lds_ptr_t)(st + i * 8192), 16, vo[i], t * 128, 0, 0);
         }
     };
-    if constexpr (OUT_KIND == 0) {
+    if constexpr (RING) {
         dl_ring<true, 8, 4, A_FMT>(acc, A, M * K, B, N * K, lds, g, wave_s, vo, vo + 4, ksteps);
     } else {
-        // (no room for the third stage beside the words of the other epilogues)
+        // (and where there is no room for the third stage beside the words of the other epilogues)
         // step kt computes from buffer kt & 1 while the loads of step kt + 1 land in the other one; the barrier at its end
         // says both that those loads are complete for every wave and that nobody reads buffer kt & 1 any more
         fetch(0, 0);
@@ -945,10 +951,41 @@ __device__ __forceinline__ void dln_epilogue(v4f (&acc)[4][NJ], uint8_t* lds, co
     }
 }
 
-template <int NJ, int OUT_KIND, int A_FMT = 0>
+template <int NJ, int A_FMT = 0, typename F = DlNothing>
+__device__ __forceinline__ void dln_compute(v4f (&acc)[4][NJ], const uint8_t* st, const DlGeom& g, F&& behind_first_reads = F()) {
+    const uint8_t* a = st + g.wm * 64 * 128;
+    const uint8_t* b = st + 256 * 128 + g.wn * (16 * NJ) * 128;
+    v8i af[4], bf[2];
+    bf[0] = dl_frag(b, g);
+#pragma unroll
+    for (int i = 0; i < 4; i++) af[i] = dl_frag(a + i * 2048, g);
+    behind_first_reads();
+#pragma unroll
+    for (int j = 0; j < NJ; j++) {
+        if (j + 1 < NJ) bf[(j + 1) & 1] = dl_frag(b + (j + 1) * 2048, g);    // one group ahead of its use
+#pragma unroll
+        for (int i = 0; i < 4; i++) mfma_f8_acc_ordered<A_FMT>(acc[i][j], bf[j & 1], af[i]);
+    }
+}
+
+// the operand loads of one K-step: `st` is the wave's first 1 KB piece of the stage (uniform: the LDS address of a load goes through M0)
+template <int NJ>
+__device__ __forceinline__ void dln_fetch(const uint8_t* A, int a_bytes, const uint8_t* B, int b_bytes, uint8_t* st, const uint32_t* vo_a,
+                                          const uint32_t* vo_b, int wave_s, int k_off) {
+    const __amdgpu_buffer_rsrc_t desc_a = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, a_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t desc_b = __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, b_bytes, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < 4; i++) __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_a, (lds_ptr_t)(st + i * 8192), 16, vo_a[i], k_off, 0, 0);
+#pragma unroll
+    for (int i = 0; i < (4 * NJ + 7) / 8; i++)
+        if (wave_s + 8 * i < 4 * NJ)                      // uniform per wave
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(desc_b, (lds_ptr_t)(st + 256 * 128 + i * 8192), 16, vo_b[i], k_off, 0, 0);
+}
+
+template <int NJ, int OUT_KIND, int A_FMT = 0, bool RING = true>
 __global__ __launch_bounds__(512) void gemm_dln_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, EpilogueArgs ep, int M,
                                                        int N, int K, int tiles_m, int tiles_n) {
-    constexpr int BN = 32 * NJ, B_ROUNDS = (BN / 8 + 7) / 8;
+    constexpr int BN = 32 * NJ, STAGE = (256 + BN) * 128, B_ROUNDS = (BN / 8 + 7) / 8;
     extern __shared__ __align__(16) uint8_t lds[];
     int tm, tn;
     tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
@@ -976,7 +1013,23 @@ __global__ __launch_bounds__(512) void gemm_dln_kernel(const uint8_t* __restrict
 #pragma unroll
         for (int j = 0; j < NJ; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
 
-    dl_ring<true, NJ, 4, A_FMT>(acc, A, M * K, B, N * K, lds, g, wave_s, vo_a, vo_b, ksteps);
+    if constexpr (RING) {
+        dl_ring<true, NJ, 4, A_FMT>(acc, A, M * K, B, N * K, lds, g, wave_s, vo_a, vo_b, ksteps);
+    } else {
+        auto fetch = [&](int t, int buf) {
+            if (t < ksteps) dln_fetch<NJ>(A, M * K, B, N * K, lds + buf * STAGE + wave_s * 1024, vo_a, vo_b, wave_s, t * 128);
+        };
+        fetch(0, 0);
+        dl_step_barrier();
+        int kt = 0;
+        for (; kt + 1 < ksteps; kt += 2) {
+            dln_compute<NJ, A_FMT>(acc, lds, g, [&] { fetch(kt + 1, 1); });
+            dl_step_barrier();
+            dln_compute<NJ, A_FMT>(acc, lds + STAGE, g, [&] { fetch(kt + 2, 0); });
+            dl_step_barrier();
+        }
+        if (kt < ksteps) dln_compute<NJ, A_FMT>(acc, lds, g);
+    }
 
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 #pragma unroll
@@ -1400,13 +1453,20 @@ static bool dlp_eligible(int M, int /*N*/, int K) {
 template <int A_FMT, int OUT_KIND>
 static int launch_dl_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, bool persistent, hipStream_t s) {
     const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
-    const size_t lds_bytes = persistent ? 2 * 512 * 128 + 8 * 4096 : OUT_KIND == 0 ? dl_ring_lds<true, 8, 4>() : 2 * 512 * 128;
-    if (int rc = persistent ? reserve_lds<gemm_dlp_kernel<A_FMT, OUT_KIND == 2>>(lds_bytes) : reserve_lds<gemm_dl_kernel<A_FMT, OUT_KIND>>(lds_bytes)) return rc;
-    if (persistent)
-        hipLaunchKernelGGL((gemm_dlp_kernel<A_FMT, OUT_KIND == 2>), dim3(256), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m / 8, (N + 127) / 128);
-    else
-        hipLaunchKernelGGL((gemm_dl_kernel<A_FMT, OUT_KIND>), dim3(tiles_m * tiles_n), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
-    return 0;
+    constexpr size_t STAGES = 2 * 512 * 128;
+    if (persistent) {
+        if (int rc = reserve_lds<gemm_dlp_kernel<A_FMT, OUT_KIND == 2>>(STAGES + 8 * 4096)) return rc;
+        hipLaunchKernelGGL((gemm_dlp_kernel<A_FMT, OUT_KIND == 2>), dim3(256), dim3(512), STAGES + 8 * 4096, s, a, b, ep, M, N, K, tiles_m / 8, (N + 127) / 128);
+        return 0;
+    }
+    auto launch = [&](auto ring, size_t lds_bytes) -> int {
+        if (int rc = reserve_lds<gemm_dl_kernel<A_FMT, OUT_KIND, ring>>(lds_bytes)) return rc;
+        hipLaunchKernelGGL((gemm_dl_kernel<A_FMT, OUT_KIND, ring>), dim3(tiles_m * tiles_n), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
+        return 0;
+    };
+    if constexpr (OUT_KIND == 0)
+        if (!dl_two_stages(8, K)) return launch(std::true_type{}, dl_ring_lds<true, 8, 4>());
+    return launch(std::false_type{}, STAGES);
 }
 
 // Blocks of 16 columns per wave (tile width 32 NJ, NJ = 4 .. 8) for a launch of 256-row tiles that is not persistent.  Measured at
@@ -1446,10 +1506,12 @@ static bool dl_narrow_fills(int M, int N) {
 template <int NJ, int OUT_KIND, int A_FMT>
 static int launch_dln_as(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s) {
     const int tiles_m = (M + 255) / 256, tiles_n = (N + 32 * NJ - 1) / (32 * NJ);
-    const size_t lds_bytes = dl_ring_lds<true, NJ, 4>();
-    if (int rc = reserve_lds<gemm_dln_kernel<NJ, OUT_KIND, A_FMT>>(lds_bytes)) return rc;
-    hipLaunchKernelGGL((gemm_dln_kernel<NJ, OUT_KIND, A_FMT>), dim3(tiles_m * tiles_n), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
-    return 0;
+    auto launch = [&](auto ring, size_t lds_bytes) -> int {
+        if (int rc = reserve_lds<gemm_dln_kernel<NJ, OUT_KIND, A_FMT, ring>>(lds_bytes)) return rc;
+        hipLaunchKernelGGL((gemm_dln_kernel<NJ, OUT_KIND, A_FMT, ring>), dim3(tiles_m * tiles_n), dim3(512), lds_bytes, s, a, b, ep, M, N, K, tiles_m, tiles_n);
+        return 0;
+    };
+    return dl_two_stages(NJ, K) ? launch(std::false_type{}, 2 * (256 + 32 * NJ) * 128) : launch(std::true_type{}, dl_ring_lds<true, NJ, 4>());
 }
 template <int NJ>
 static int launch_dln_nj(int a_fmt, const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, int M, int N, int K, hipStream_t s) {

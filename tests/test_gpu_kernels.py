@@ -311,6 +311,22 @@ def test_gemm_direct_to_lds_kernels_agree_bit_for_bit_on_seeded_shapes(ops):
             assert torch.equal(got, want), (M, N, K, kernel)
 
 
+@pytest.mark.parametrize("K", [128, 256, 384, 1024, 1152, 1280])
+def test_gemm_narrow_tiles_on_both_sides_of_their_loops(ops, K):
+    """Tiles of 256 x 128 and 256 x 160 take a K loop of two stages up to K = 1024, wider ones up to 128, and the ring of three beyond: plain, relu^2 and e5m2 outputs
+    have the bits of the 128 x 128 tiles (of one, two, three, eight, nine and ten steps; ragged rows and columns)."""
+    M, N = 300, 1004
+    say(f"gemm, narrow tiles, K={K}")
+    a, w = make_operands(M, N, K, seed=K)
+    a8, ia, _ = fp8_ref.to_fp8(a)
+    w8, iw, _ = fp8_ref.to_fp8(w)
+    a8, w8, ia, iw = (t.to(DEV) for t in (a8, w8, ia, iw))
+    e5 = ops.fp8_quantize(a.to(DEV).bfloat16(), fp8_dtype=torch.float8_e5m2)[0]
+    for run in (lambda k: ops.fp8_gemm(a8, w8, ia, iw, kernel=k), lambda k: ops.fp8_gemm_relu2(a8, w8, ia, iw, kernel=k)[0], lambda k: ops.fp8_gemm_grad(e5, w8, ia, iw, kernel=k)):
+        want = run(5)
+        assert all(torch.equal(run(k), want) for k in (8, 12, 13, 14, 15))
+
+
 def test_gemm_one_hot_weight_is_a_gather(ops):
     say("gemm one-hot")
     M, N, K = 64, 128, 256
