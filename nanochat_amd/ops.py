@@ -576,11 +576,11 @@ def stack_linear_runs(a, w, runs, limit=0.0, kernel=0):
     stack_linear and 4 (float, added to what is there), 5 (float logits, soft-capped at limit)."""
     _need_cuda(a, w, *(out for _, _, out in runs))
     (M, K), N, n = a.shape, w.shape[0], len(runs)
-    assert w.shape[1] == K and a.dtype == w.dtype and a.is_contiguous() and w.is_contiguous() and sum(cols for cols, _, _ in runs) == N
+    assert w.shape[1] == K and a.dtype == w.dtype and a.stride(1) == 1 and w.is_contiguous() and sum(cols for cols, _, _ in runs) == N
     for cols, kind, out in runs:
         assert tuple(out.shape) == (M, cols // 2 if kind in (2, 7) else cols) and out.stride(1) == 1 and out.dtype == (torch.float32 if kind in (3, 4, 5) else a.dtype)
     ends = (C.c_int32 * n)(*(sum(cols for cols, _, _ in runs[:i + 1]) for i in range(n)))
     kinds, lds = (C.c_int32 * n)(*(kind for _, kind, _ in runs)), (C.c_int32 * n)(*(out.stride(0) for _, _, out in runs))
-    rc = _lib.stack_lib().nc_stack_linear_runs(STACK_DTYPES[a.dtype], _ptr(a), K, _ptr(w), M, N, K, n, ends, kinds, (C.c_void_p * n)(*(_ptr(out) for _, _, out in runs)), lds,
+    rc = _lib.stack_lib().nc_stack_linear_runs(STACK_DTYPES[a.dtype], _ptr(a), a.stride(0), _ptr(w), M, N, K, n, ends, kinds, (C.c_void_p * n)(*(_ptr(out) for _, _, out in runs)), lds,
                                                limit, kernel, _stream())
     _lib.check(rc, _lib.stack_lib())

@@ -937,3 +937,41 @@ def test_decode_step_captured_in_a_graph_replays_like_the_eager_step(B):
     assert torch.equal(graphed.k_cache[:, :, :P + steps], eager.k_cache[:, :, :P + steps])
     assert torch.equal(graphed.v_cache[:, :, :P + steps], eager.v_cache[:, :, :P + steps])
 
+
+@pytest.mark.parametrize("heads,kv_heads,B,T", [(4, 2, 1, 300), (3, 3, 2, 700), (2, 1, 9, 16)])
+def test_prompt_captured_in_a_graph_replays_like_the_eager_pass(heads, kv_heads, B, T):
+    """nc_gpt_forward of a prompt makes no allocation, copy or fill of its own, and the words that its workgroups meet on are cleared by a kernel of every pass:
+    captured once and replayed with other tokens, with eager passes and synchronisations in between, it has the logits and the cache of the eager pass."""
+    import ctypes
+    from nanochat_amd import _lib
+    from nanochat_amd.engine import KVCache
+    from nanochat_amd.gpt import GPTConfig
+    from nanochat_amd.synthetic import random_init_model
+    say(f"prompt under graph capture: {heads} heads on {kv_heads}, {B} x {T} tokens")
+    cfg = GPTConfig(sequence_len=1024, vocab_size=1024, n_layer=3, n_head=heads, n_kv_head=kv_heads, n_embd=128 * heads, window_pattern="SL")
+    model = random_init_model(cfg, DEV, seed=5)
+    md, lib = model._ensure_plan(), _lib.lib()
+    g = torch.Generator().manual_seed(6)
+    ws = torch.empty(lib.nc_gpt_workspace_bytes(ctypes.byref(md), B, T) + 256, dtype=torch.uint8, device=DEV)
+    ids = torch.zeros(B, T, dtype=torch.long, device=DEV)
+
+    def a_pass(cache, logits, prev, stream):
+        cd = _lib.CacheDesc()
+        cd.k_cache, cd.v_cache, cd.cache_seqlens, cd.prev_out = cache.k_cache.data_ptr(), cache.v_cache.data_ptr(), cache.cache_seqlens.data_ptr(), prev.data_ptr()
+        cd.batch, cd.max_seq_len = B, T
+        _lib.check(lib.nc_gpt_forward(ctypes.byref(md), ctypes.byref(cd), ids.data_ptr(), B, T, logits.data_ptr(), 0, ws.data_ptr() + (-ws.data_ptr()) % 256, ws.numel() - 256, stream))
+    eager, graphed = ([KVCache(B, kv_heads, T, 128, 3, DEV, torch.bfloat16), torch.zeros(B * T, 1024, device=DEV), torch.zeros(B, 1, 128 * heads, dtype=torch.bfloat16, device=DEV)]
+                      for _ in range(2))
+    a_pass(*eager, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        a_pass(*graphed, torch.cuda.current_stream().cuda_stream)
+    for replay in range(4):
+        ids.copy_(torch.randint(0, 1024, (B, T), generator=g))
+        graph.replay()
+        torch.cuda.synchronize()
+        a_pass(*eager, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert eager[1].any() and torch.equal(graphed[1], eager[1]) and torch.equal(graphed[2], eager[2]), replay
+        assert torch.equal(graphed[0].k_cache, eager[0].k_cache) and torch.equal(graphed[0].v_cache, eager[0].v_cache)
