@@ -171,13 +171,10 @@ Workspace carve(const nc_model_desc* m, int B, int T, void* base) {
 // the two it depends on whether the reading ends with attention: 20 MB (depth 20) 65 tokens 1274 / 1246, 128 1446 / 1390, 4 x 17 1255 / 1265, 24 MB (depth 22) 65
 // tokens 1476 / 1463, 128 1663 / 1633, but 28 MB (depth 24) 65 tokens 1592 / 1607, 4 x 24 1698 / 1711, 33 MB (depth 26) 65 tokens 1851 / 1867, 128 2113 / 2098, 4 x 20
 // 1906 / 1922.  Beyond 128 rows, depth 26: 8 x 32 1854 / 1761, 64 x 16 3001 / 2733.
-// Weights and cached rows of less than two thirds of the last-level cache stay there: us without / with, depth 8 (50 MB) 400 tokens 481 / 488, depth 10 (70 MB) 200
-// 562 / 573, depth 12 (110 MB) 200 tokens 675 / 687, 500 794 / 783, 900 876 / 886, 1792 1023 / 1023, depth 14 (164 MB) 200 tokens 822 / 822, 300 877 / 861, 500 943 / 922, 1792
-// 1385 / 1289, depth 16 (234 MB) 130 tokens 897 / 876.
-constexpr size_t AHEAD_LAYER_BYTES_FEW = 24u << 20, AHEAD_MODEL_BYTES = 170u << 20;
+constexpr size_t AHEAD_LAYER_BYTES_FEW = 24u << 20;
 bool reads_ahead(const nc_model_desc* m, int M) {
     const size_t E = m->n_embd, layer = E * ((size_t)(2 * m->n_head + 2 * m->n_kv_head) * 128 + 8 * E), rows = (size_t)M * m->n_kv_head * 512;
-    if (m->n_layer * (layer + rows) + m->vocab_size * E <= AHEAD_MODEL_BYTES) return false;
+    if (m->n_layer * (layer + rows) + m->vocab_size * E <= NC_AHEAD_MODEL_BYTES) return false;
     return M > 128 || (M > 64 && layer <= AHEAD_LAYER_BYTES_FEW);
 }
 

@@ -7,7 +7,12 @@
 #include "nc_common.h"
 
 // A model whose weights and cached rows stay in that cache (256 MB, with a pass's activations) gains nothing, and its launches last longer by the workgroups
-// that read: each caller has a size from which on it asks for the reading.
+// that read.  us without / with: GPT of depth 8 (50 MB with the head), 200 tokens 437 / 442, depth 10 (70 MB) 562 / 573, depth 12 (110 MB) 679 / 693, 1792 1023 / 1023,
+// depth 14 (164 MB) 130 tokens 784 / 793, 1792 (254 with the keys) 1385 / 1289, depth 16 (234 MB) 130 tokens 897 / 876; stacks: dense Palilix of width 1024 (172
+// MB) 500 tokens 352 / 354.5, 1792 646 / 654, Zodirax of width 1024 (193 MB) 200 tokens 458 / 465, Palilix of width 512 (361 MB) 500 tokens 449 / 451, of width 1024
+// (746 MB) 578 / 571.
+constexpr size_t NC_AHEAD_MODEL_BYTES = 200u << 20;
+
 #define NC_AHEAD_RANGES 4
 #define NC_AHEAD_WGS 128                      // workgroups of 256 threads: 33 MB in some 8 us
 struct NcAhead {

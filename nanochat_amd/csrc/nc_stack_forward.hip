@@ -272,9 +272,6 @@ int run_mixers(const nc_stack_model* m, const nc_stack_cache* kv, const nc_stack
 // 2048, 300 tokens 572 / 572 / 572 / 518, 500 621 / 622 / 573 / 573, 800 850 / 783 / 784 / 838, 1400 1053 / 1063 / 1114 / 1118, of width 3072, 800 tokens 1294 / 1293 / 1295 / 1224,
 // with experts, width 2048, 500 tokens 889 / 885 / 874 / 871, 1000 1127 / 1109 / 1104 / 1103.  No prompt of these is slower than without reading.
 constexpr size_t AHEAD_BYTES_PER_ROW = 98304;
-// Weights of less than 200 MB stay in the last-level cache: us without / with, dense Palilix of width 1024 (172 MB) 500 tokens 352 / 354.5, 1792 646 / 654, Zodirax of width
-// 1024 (193 MB) 200 tokens 458 / 465, 500 514 / 520; Palilix of width 512 (361 MB) 500 tokens 449 / 451, of width 1024 (746 MB) 578 / 571.
-constexpr size_t AHEAD_MODEL_BYTES = 200u << 20;
 bool reads_ahead(const nc_stack_model* m, int M) {
     if (m->dtype || M <= NC_FEW_ROWS) return false;
     const size_t W = m->width_p;
@@ -285,7 +282,7 @@ bool reads_ahead(const nc_stack_model* m, int M) {
         if (l.block == NC_BLOCK_POST_NORM) elems += W * ((size_t)l.ff_cols + l.ff_p);
         if (l.ff == NC_FF_EXPERTS) elems += 3 * W * l.experts * l.expert_ff_p;
     }
-    return 2 * elems > AHEAD_MODEL_BYTES;
+    return 2 * elems > NC_AHEAD_MODEL_BYTES;
 }
 NcAhead weights_behind(const nc_stack_model* m, int i, int M) {
     NcAhead a{};
