@@ -138,9 +138,6 @@ typedef struct nc_stack_cache {
 /* Workspace for one forward of T tokens per row, n_logits rows of logits, at most max_keys keys per row. */
 size_t nc_stack_workspace_bytes(const nc_stack_model* model /*host*/, int B, int T, int n_logits, int max_keys);
 
-/* 1: the last mixers of such a forward read weights of the linears behind them ahead (host only; the results do not depend on it). */
-int nc_stack_reads_ahead(const nc_stack_model* model /*host*/, int B, int T);
-
 /* idx int64 [B,T]; logit_rows int32 [n_logits]: flat indices (row * T + token) whose logits are wanted (device); logits_out fp32
  * [n_logits, vocab].  n_logits may be 0.  taps (or NULL): fp32 [n_runs, B*T, width_p], the residual stream after every run. */
 int nc_stack_forward(const nc_stack_model* model /*host*/, const nc_stack_cache* cache /*host*/, const int64_t* idx, int B, int T,

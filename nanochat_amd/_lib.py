@@ -24,7 +24,7 @@ EXPORTS = [
 ]
 
 
-STACK_EXPORTS = ["nc_stack_abi_version", "nc_last_error", "nc_stack_workspace_bytes", "nc_stack_reads_ahead", "nc_stack_forward", "nc_stack_linear", "nc_stack_linear_runs", "nc_stack_cache_copy",
+STACK_EXPORTS = ["nc_stack_abi_version", "nc_last_error", "nc_stack_workspace_bytes", "nc_stack_forward", "nc_stack_linear", "nc_stack_linear_runs", "nc_stack_cache_copy",
                  "nc_profile_enable", "nc_profile_read", "nc_profile_read_gemm"]
 
 
@@ -95,7 +95,6 @@ def _bind_stack(lib):
         "nc_stack_abi_version": (i, []),
         "nc_last_error": (C.c_char_p, []),
         "nc_stack_workspace_bytes": (sz, [C.POINTER(StackModel), i, i, i, i]),
-        "nc_stack_reads_ahead": (i, [C.POINTER(StackModel), i, i]),
         "nc_stack_forward": (i, [C.POINTER(StackModel), C.POINTER(StackCacheDesc), p, i, i, p, i, p, p, sz, p, p]),
         "nc_stack_linear": (i, [i, p, i64, p, p, i, i, i, i, i, f, i, p]),
         "nc_stack_linear_runs": (i, [i, p, i64, p, i, i, i, i, p, p, p, p, f, i, p]),

@@ -173,8 +173,7 @@ Workspace carve(const nc_model_desc* m, int B, int T, void* base) {
 // 1906 / 1922.  Beyond 128 rows, depth 26: 8 x 32 1854 / 1761, 64 x 16 3001 / 2733.
 constexpr size_t AHEAD_LAYER_BYTES_FEW = 24u << 20;
 bool reads_ahead(const nc_model_desc* m, int M) {
-    const size_t E = m->n_embd, layer = E * ((size_t)(2 * m->n_head + 2 * m->n_kv_head) * 128 + 8 * E), rows = (size_t)M * m->n_kv_head * 512;
-    if (m->n_layer * (layer + rows) + m->vocab_size * E <= NC_AHEAD_MODEL_BYTES) return false;
+    const size_t E = m->n_embd, layer = E * ((size_t)(2 * m->n_head + 2 * m->n_kv_head) * 128 + 8 * E);
     return M > 128 || (M > 64 && layer <= AHEAD_LAYER_BYTES_FEW);
 }
 

@@ -1,17 +1,13 @@
 // Weights on their way while the memory is idle.  A forward pass reads each weight once, and the weights of a model of more than 256 MB have left the
 // last-level cache by the next pass: the linears of a prompt, whose tiles wait for one K-step of their operands after the other, then run at the
 // latency of HBM (us, weights in HBM / in that cache: 1792 x 1664 x 6656 33.7 / 24.3, 1792 x 4992 x 1664 27.2 / 22.7, 1792 x 6656 x 1664 29.5 / 25.2).
+// (Smaller models too have their weights pushed out by what runs between two passes: us without / with, other models' passes in between, and in brackets with the card to
+// itself: GPT of depth 12 (110 MB) 500 tokens 822 / 790 (794 / 783), depth 10, 200 tokens 573 / 566 (562 / 573), dense Palilix of width 1024 (172 MB) 500 tokens 380 / 369 (352 /
+// 354.5), Zodirax of width 1024, 200 tokens 484 / 478 (458 / 465).  So no rule looks at the size of the model.)
 // A launch that computes while the memory has nothing to do (attention of a prompt) carries some workgroups more that read the weights of the
 // linears behind it, 32 KB at a time, one run of addresses after the other, and throw away what they read.
 #pragma once
 #include "nc_common.h"
-
-// A model whose weights and cached rows stay in that cache (256 MB, with a pass's activations) gains nothing, and its launches last longer by the workgroups
-// that read.  us without / with: GPT of depth 8 (50 MB with the head), 200 tokens 437 / 442, depth 10 (70 MB) 562 / 573, depth 12 (110 MB) 679 / 693, 1792 1023 / 1023,
-// depth 14 (164 MB) 130 tokens 784 / 793, 1792 (254 with the keys) 1385 / 1289, depth 16 (234 MB) 130 tokens 897 / 876; stacks: dense Palilix of width 1024 (172
-// MB) 500 tokens 352 / 354.5, 1792 646 / 654, Zodirax of width 1024 (193 MB) 200 tokens 458 / 465, Palilix of width 512 (361 MB) 500 tokens 449 / 451, of width 1024
-// (746 MB) 578 / 571.
-constexpr size_t NC_AHEAD_MODEL_BYTES = 200u << 20;
 
 #define NC_AHEAD_RANGES 4
 #define NC_AHEAD_WGS 128                      // workgroups of 256 threads: 33 MB in some 8 us

@@ -272,20 +272,9 @@ int run_mixers(const nc_stack_model* m, const nc_stack_cache* kv, const nc_stack
 // 2048, 300 tokens 572 / 572 / 572 / 518, 500 621 / 622 / 573 / 573, 800 850 / 783 / 784 / 838, 1400 1053 / 1063 / 1114 / 1118, of width 3072, 800 tokens 1294 / 1293 / 1295 / 1224,
 // with experts, width 2048, 500 tokens 889 / 885 / 874 / 871, 1000 1127 / 1109 / 1104 / 1103.  No prompt of these is slower than without reading.
 constexpr size_t AHEAD_BYTES_PER_ROW = 98304;
-bool reads_ahead(const nc_stack_model* m, int M) {
-    if (m->dtype || M <= NC_FEW_ROWS) return false;
-    const size_t W = m->width_p;
-    size_t elems = W * m->vocab;
-    for (int i = 0; i < m->n_layers; i++) {
-        const nc_stack_layer& l = m->layers[i];
-        elems += W * ((size_t)l.n_in + l.k_out);
-        if (l.block == NC_BLOCK_POST_NORM) elems += W * ((size_t)l.ff_cols + l.ff_p);
-        if (l.ff == NC_FF_EXPERTS) elems += 3 * W * l.experts * l.expert_ff_p;
-    }
-    return 2 * elems > NC_AHEAD_MODEL_BYTES;
-}
 NcAhead weights_behind(const nc_stack_model* m, int i, int M) {
     NcAhead a{};
+    if (m->dtype || M <= NC_FEW_ROWS) return a;
     const nc_stack_layer& l = m->layers[m->runs[i].layer];
     const size_t W = m->width_p;
     // whole matrices only: the tiles of a launch start all over its matrix
@@ -419,8 +408,6 @@ extern "C" size_t nc_stack_workspace_bytes(const nc_stack_model* m, int B, int T
     return carve(m, B, T, n_logits, max_keys, nullptr).total;
 }
 
-extern "C" int nc_stack_reads_ahead(const nc_stack_model* m, int B, int T) { return m && B > 0 && T > 0 && reads_ahead(m, B * T); }
-
 extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* kv, const int64_t* idx, int B, int T, const int32_t* logit_rows,
                                 int n_logits, float* logits_out, void* workspace, size_t workspace_bytes, float* taps, nc_stream_t stream) {
     hipStream_t s = (hipStream_t)stream;
@@ -450,7 +437,6 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
     entry_norm(m, m->runs[0], norm, norm_w);
     TRY(nc_launch_stack_embed(dt, idx, m->embed, m->embed_scale, m->runs[0].step >= 0 ? m->steps + (int64_t)m->runs[0].step * Wp : nullptr, m->vocab, w.x,
                               again ? w.x0 : nullptr, norm, norm_w, m->eps, w.h, M, m->width, Wp, s));
-    const bool ahead = reads_ahead(m, M);
     for (int i = 0; i < m->n_runs; i++) {
         const nc_stack_run& run = m->runs[i];
         const nc_stack_layer& l = m->layers[run.layer];
@@ -460,7 +446,7 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
         if (l.router_cols) nc_linear_seg(in, l.mix_cols + l.router_cols, NC_SEG_F32, w.router, l.router_cols);
         if (!post && l.ff_cols) nc_linear_seg(in, l.n_in, ff_seg_kind(l.ff), at(w.cat, l.mix_out, dt), l.k_out, l.ff_limit);
         TRY(nc_launch_linear(dt, in, s));
-        TRY(run_mixers(m, kv, run, w, B, T, ahead ? weights_behind(m, i, M) : NcAhead{}, s));
+        TRY(run_mixers(m, kv, run, w, B, T, weights_behind(m, i, M), s));
 
         NcRowAdd add{};
         add.x = w.x, add.tokens_per_row = T;

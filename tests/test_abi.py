@@ -120,15 +120,6 @@ def test_which_prompts_read_weights_ahead():
     assert [ahead(10, 1, T) for T in (16, 64, 65, 128, 129)] == [0, 0, 1, 1, 1]
 
 
-def test_models_that_stay_in_the_last_level_cache_read_nothing_ahead():
-    """Weights and the prompt's keys and values together: depth 12 with any prompt, depth 14 (164 MB) up to some 700 tokens, depth 16 (234 MB) never."""
-    def ahead(heads, T, kv_heads=None):
-        m = _lib.ModelDesc(n_layer=2 * heads, n_head=heads, n_kv_head=kv_heads or heads, n_embd=128 * heads, vocab_size=32768)
-        return _lib.lib().nc_gpt_reads_ahead(ctypes.byref(m), 1, T)
-    assert not any(ahead(heads, T) for heads in (2, 4, 6) for T in (129, 500, 1792))
-    assert [ahead(7, T) for T in (200, 400, 1000, 1792)] == [0, 0, 1, 1] and ahead(8, 130) == 1 and ahead(7, 1000, kv_heads=1) == 0
-
-
 def test_a_launch_that_meets_has_a_word_for_every_workgroup():
     """The words' size follows from the most workgroups that may meet, and no shape is let in that has one more (257 tiles of 256 x 256)."""
     lib = _lib.lib()

@@ -463,33 +463,6 @@ def test_prompts_on_two_streams(depth, T):
             assert torch.equal(got[i], want[i]) and torch.equal(together[i].k_cache, alone[i].k_cache) and torch.equal(together[i].v_cache, alone[i].v_cache)
 
 
-@pytest.mark.parametrize("heads,kv_heads,B,T", [(2, 2, 1, 130), (2, 1, 3, 100), (4, 1, 1, 700), (3, 3, 40, 20)])
-def test_prompts_that_read_weights_ahead(heads, kv_heads, B, T):
-    """A model that is large by its vocabulary, so that attention's launch reads the next weights ahead, and the same model without most of the vocabulary,
-    where it does not: logits of the common tokens and the cache, to the bit.  (The head's largest weight is a common token's.)"""
-    import ctypes
-    from nanochat_amd import _lib
-    from nanochat_amd.engine import KVCache
-    from nanochat_amd.gpt import GPT, GPTConfig
-    from nanochat_amd.synthetic import random_init_model
-    say(f"reading ahead: {heads} heads on {kv_heads}, {B} x {T} tokens")
-    few, E = 512, 128 * heads
-    def cfg(vocab):
-        return GPTConfig(sequence_len=1024, vocab_size=vocab, n_layer=2, n_head=heads, n_kv_head=kv_heads, n_embd=E)
-    big, small = (random_init_model(cfg(v), DEV, seed=3) for v in (-(-(200 << 20) // E // 64) * 64, few))
-    with torch.no_grad():
-        big.lm_head.weight[0, 0] = 1.0
-        for a, b in zip(small.parameters(), big.parameters()):
-            a.copy_(b[:a.shape[0]])
-    idx = torch.randint(0, few, (B, T), generator=torch.Generator().manual_seed(T)).to(DEV)
-    out = []
-    for model, reads in ((big, 1), (small, 0)):
-        assert _lib.lib().nc_gpt_reads_ahead(ctypes.byref(model._ensure_plan()), B, T) == reads
-        cache = KVCache(B, kv_heads, T, 128, 2, DEV, torch.bfloat16)
-        out.append((model.forward_last(idx, kv_cache=cache)[..., :few].clone(), cache.k_cache, cache.v_cache))
-    assert all(torch.equal(a, b) for a, b in zip(*out))
-
-
 def test_ragged_rows():
     """Per-row cache lengths (outside the reference's GPT.forward, inside FA3's signature): every row
     must equal the same row run alone."""

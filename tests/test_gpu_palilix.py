@@ -1,6 +1,5 @@
 """Palilix on the GPU against the plain restatement in oracle/palilix_ref.py (float64): whole prompts, decoding, portions, batches of
 unequal sequences, slots that are used again, generation through the Engine; both storage types."""
-import ctypes
 import functools
 import json
 import math
@@ -8,12 +7,11 @@ import math
 import pytest
 import torch
 
-from nanochat_amd import _lib, ops
+from nanochat_amd import ops
 from nanochat_amd.engine import Engine
 from nanochat_amd.palilix import Palilix
 from nanochat_amd.registry import load_model
-from nanochat_amd.synthetic import SyntheticTokenizer, palilix_config, random_stack_model, zodirax_config
-from nanochat_amd.zodirax import Zodirax
+from nanochat_amd.synthetic import SyntheticTokenizer
 from oracle import palilix_ref as ref
 from palilix_cases import CASES, config, dense, latent, moe, retention, variant, weights
 from stack_helpers import BAR, DEV, DTYPES, build_model, check, ids, judge, rel_rms, run, say, tokens, trace_runner, write_model
@@ -747,26 +745,3 @@ def test_trace_replay(tmp_path):
     grown = mod.Replay(model, 10)                      # more tokens than were announced
     grown.step([{"id": "c", "tokens": toks[:10], "want": []}], [])
     check(grown.step([{"id": "c", "tokens": toks[10:45], "want": [34]}], ["c"]), want[44:], torch.float32, "grown")
-
-
-# ------------------------------------------------------------------------------------------------ weights read ahead
-@pytest.mark.parametrize("B,T", [(1, 70), (3, 40), (1, 700)])
-@pytest.mark.parametrize("make,cls", [(lambda v: palilix_config(256, 2, rank=128, experts=8, expert_ff=64, vocab=v), Palilix), (lambda v: palilix_config(256, 2, vocab=v, dense=True), Palilix),
-                                      (lambda v: zodirax_config(256, 4, window=50, vocab=v), Zodirax)], ids=["experts", "dense", "zodirax"])
-def test_prompts_that_read_weights_ahead(make, cls, B, T):
-    """A model that is large by its vocabulary, so that the last mixers read the next weights ahead, and the same model without most of the vocabulary, where
-    they do not: logits of the common tokens, cached rows and states, to the bit."""
-    say(f"reading ahead: {cls.__name__}, {B} x {T} tokens")
-    few, many = 512, (201 << 20) // 512
-    big, small = (random_stack_model(cls, make(v), DEV) for v in (many, few))
-    with torch.no_grad():
-        for name, t in small.held_tensors().items():
-            t.copy_(big.held_tensors()[name][:t.shape[0]])
-    idx = torch.randint(0, few, (B, T), generator=torch.Generator().manual_seed(T)).to(DEV)
-    out = []
-    for model, reads in ((big, 1), (small, 0)):
-        cache = model.new_cache(B, T)
-        logits = model.forward_last(idx, kv_cache=cache)[..., :few].clone()
-        assert _lib.stack_lib().nc_stack_reads_ahead(ctypes.byref(model._ensure_plan(T)), B, T) == reads
-        out.append([logits, *cache.rows, *cache.state_buffers()[0]])
-    assert len(out[0]) == len(out[1]) > 2 and all(torch.equal(a, b) for a, b in zip(*out))
