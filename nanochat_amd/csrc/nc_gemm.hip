@@ -1709,24 +1709,21 @@ int nc_launch_gemm(const uint8_t* a, const uint8_t* b, const float* inv_a, const
     return 0;
 }
 
-// The tiles of the q|k|v linear that finish its heads: those of 64 or 96 x 128 where pick_kernel takes them (16, 17), otherwise 64 WTM x 128 (returned as
-// 100 + WTM) with the least cost by the count of dl_cost, a tile of 64 x 128 being its unit of area; 0: none.  Also where pick_kernel has the persistent kernel: us a
-// prompt with it and a rotary launch / this way, depth 26, 2 x 1792 tokens 6701 / 6561, 8 x 1024 12652 / 12355, 4096 7649 / 7382, depth 12, 8 x 1024 2643 / 2513, depth 8,
-// 32 x 1024 3418 / 3324; of few key heads (depth 24, 6 of 12, 4 x 1024) 5528 / 5617.
+// The tiles of the q|k|v linear that finish its heads: those of 64 or 96 x 128 where pick_kernel takes them (16, 17), otherwise 64 w x 128 (returned as
+// 100 + w); 0: none.  Two workgroups of the 128-row tile fit a CU (80 KB of LDS each), one of the higher ones, whose epilogue nothing overlaps.  So the low tile
+// is taken in one round of one or two to a CU and wherever the others need a second round; a single round of higher tiles beats it (i) at 192 rows, (ii) where the
+// low ones would go into a second round.  us, 128-row tiles / the best of the others (w) / a linear and a rotary launch: 1300 x 4992 x 1664 19.5 / 21.4 (4) / 25.8,
+// 1792 x 29.4 / 25.3 (5) / 31.8, 2048 x 29.5 / 28.8 (6) / 33.9, 3072 x 35.6 / 41.3 (4) / 44.3, 4096 x 46.9 / 50.1 (5) / 61.4, 6144 x 67.0 / 80.6 (4) / 81.6; few key heads,
+// 1300 x 3072 x 1536 17.0 / 16.8 (3) / 24.7, 2048 x 18.1 / 20.5 (4) / 23.7, 3072 x 28.6 / 25.2 (5) / 32.0, 4096 x 29.6 / 38.5 (4) / 37.6, 8192 x 1536 x 768 22.1 / 28.8 (4) / 33.4.
 static int rope_tiles(int M, int N, int K) {
     if (M <= 128 || N % 128 != 0 || K % 128 != 0 || (long)M * K >= (1L << 31) || (long)N * K >= (1L << 31)) return 0;
     const int which = pick_kernel(M, N, K, 0);
     if (which == 16 || which == 17) return which;
-    const int cus = cu_count();
-    int best = 0;
-    double best_cost = 0.0;
-    for (int w = 2; w <= 6; w++) {
-        const long tiles = (long)((M + 64 * w - 1) / (64 * w)) * (N / 128);
-        double cost = 0.0;
-        for (long left = tiles; left > 0; left -= cus) cost += (6.0 + w) * (1.0 + 0.2 * (double)(left < cus ? left : cus) / cus);
-        if (!best || cost < best_cost) best = w, best_cost = cost;
-    }
-    return 100 + best;
+    const long cus = cu_count(), columns = N / 128, low = (M + 127) / 128 * columns;
+    if (low <= cus) return 102;
+    for (int w = 3; w <= 6; w++)
+        if ((M + 64 * w - 1) / (64 * w) * columns <= cus) return w == 3 || low > 2 * cus ? 100 + w : 102;
+    return 102;
 }
 template <int WTM>
 static int launch_gemm_rope(const uint8_t* a, const uint8_t* b, const EpilogueArgs& ep, const RopeArgs& rope, int M, int N, int K, hipStream_t s) {

@@ -902,7 +902,8 @@ def test_relu2(ops):
 
 @pytest.mark.parametrize("B,T,K,H,Hkv,ve,kernel", [(1, 1792, 1664, 13, 13, True, 0), (1, 130, 256, 2, 1, True, 0), (2, 333, 384, 6, 6, False, 0), (4, 448, 256, 13, 13, True, 0),
                                                    (1, 129, 128, 1, 1, True, 16), (3, 65, 256, 4, 2, True, 17), (1, 255, 128, 2, 2, False, 102), (5, 77, 256, 2, 1, True, 103),
-                                                   (1, 1025, 256, 8, 4, True, 104), (1, 321, 384, 3, 3, True, 105), (2, 383, 128, 4, 1, False, 106)])
+                                                   (1, 1025, 256, 8, 4, True, 104), (1, 321, 384, 3, 3, True, 105), (2, 383, 128, 4, 1, False, 106),
+                                                   (1, 1299, 128, 13, 13, True, 0), (4, 1024, 128, 12, 6, True, 0), (3, 683, 256, 13, 13, False, 0), (5, 1229, 256, 13, 13, True, 0)])
 def test_qkv_linear_finishes_its_heads(ops, B, T, K, H, Hkv, ve, kernel):
     """The q|k|v linear with rotary, norm, value embedding and append in its epilogue: the bits of the two launches, and nothing written beside the new rows."""
     say(f"qkv linear rope B={B} T={T} K={K} H={H} Hkv={Hkv} ve={ve} kernel={kernel}")
