@@ -342,6 +342,11 @@ int nc_gpt_forward(const nc_model_desc* model /*host*/, const nc_cache_desc* cac
                    int B, int T, float* logits_out, int last_only, void* workspace, size_t workspace_bytes,
                    nc_stream_t stream);
 
+/* A one-token forward of up to 8 rows whose layers run in one launch (nc_gpt_forward takes it where it can), of which only `present` workgroups are started: as if
+ * the others had found no place on the chip beside other streams' kernels.  The results do not depend on it.  For tests; fails where the forward is not one of those. */
+int nc_gpt_forward_present(const nc_model_desc* model /*host*/, const nc_cache_desc* cache /*host*/, const int64_t* idx, int B,
+                           float* logits_out, void* workspace, size_t workspace_bytes, int present, nc_stream_t stream);
+
 /* The same forward with its intermediate activations copied out, for layer-by-layer comparison with another implementation
  * (no counterpart in the reference; tests only).  tap_x (or NULL): bf16 [n_layer+1, B*T, E]; slot i is the residual stream as
  * layer i reads it, i.e. after `x = resid_lambdas[i]*x + x0_lambdas[i]*x0` (nanochat/gpt.py:500), slot n_layer the final

@@ -89,9 +89,16 @@ __global__ __launch_bounds__(256) void embed_norm_smear_decode_kernel(const int6
                                                                       const float* __restrict__ smear_lambda,
                                                                       const bf16_t* __restrict__ prev_in, bf16_t* __restrict__ prev_out,
                                                                       bf16_t* __restrict__ x_out, bf16_t* __restrict__ x0_out, int E,
-                                                                      int vocab_rows, uint32_t* __restrict__ clear_words, int n_clear) {
+                                                                      int vocab_rows, uint32_t* __restrict__ clear_words, int n_clear, int rows,
+                                                                      uint4* __restrict__ fill, uint32_t n_fill) {
     __shared__ float red[8];
     __shared__ float head[24];
+    if ((int)blockIdx.x >= rows) {
+        // workgroups behind the rows' set the exchange of a step in one launch to "unwritten" (nc_step.hip)
+        const uint4 ones = make_uint4(~0u, ~0u, ~0u, ~0u);
+        for (uint32_t i = (blockIdx.x - rows) * 256 + threadIdx.x; i < n_fill; i += (gridDim.x - rows) * 256) fill[i] = ones;
+        return;
+    }
     const int b = blockIdx.x, c0 = threadIdx.x * 8;
     const bool mine = c0 < E;
     int64_t tok = idx[b];
@@ -105,7 +112,7 @@ __global__ __launch_bounds__(256) void embed_norm_smear_decode_kernel(const int6
     const float sw = (threadIdx.x & 63) < 24 ? smear_w[threadIdx.x & 63] : 0.f;      // lane c of every wave holds gate weight c
     const float lam = *smear_lambda;
     // first kernel of a forward pass: it also zeroes the pass's amax slots and arrival counters
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n_clear; i += gridDim.x * 256) clear_words[i] = 0u;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n_clear; i += rows * 256) clear_words[i] = 0u;
 
     const uint32_t ew[4] = {ev.x, ev.y, ev.z, ev.w};
     float v[8], ss = 0.f;
@@ -642,15 +649,17 @@ int nc_launch_rmsnorm(const bf16_t* x, bf16_t* out, int rows, int cols, uint32_t
 
 int nc_launch_embed_norm_smear(const int64_t* idx, const bf16_t* wte, const float* smear_w, const float* smear_lambda,
                                const bf16_t* prev_in, bf16_t* prev_out, bf16_t* x_out, bf16_t* x0_out, int B, int T, int E,
-                               int vocab_rows, uint32_t* clear_words, int n_clear, hipStream_t s) {
+                               int vocab_rows, uint32_t* clear_words, int n_clear, hipStream_t s, void* fill, size_t fill_bytes) {
     NC_CHECK_ARG(idx && wte && smear_w && smear_lambda && prev_out && x_out, "embed_norm_smear: null pointer");
     NC_CHECK_ARG(B > 0 && T > 0 && E >= 24 && E <= 8192, "embed_norm_smear: bad shape B=%d T=%d E=%d", B, T, E);
     NcProfScope prof(3, 4.0 * B * T * E, s);
     const bool vec = T == 1 && E % 8 == 0 && E <= 2048 &&
                      (((uintptr_t)wte | (uintptr_t)prev_in | (uintptr_t)prev_out | (uintptr_t)x_out | (uintptr_t)x0_out) & 15) == 0;
+    NC_CHECK_ARG(fill_bytes == 0 || (vec && fill_bytes % 16 == 0 && ((uintptr_t)fill & 15) == 0), "embed_norm_smear: cannot fill %zu bytes", fill_bytes);
+    const int fill_wgs = (int)((fill_bytes + 32767) / 32768 < 128 ? (fill_bytes + 32767) / 32768 : 128);
     if (vec)
-        hipLaunchKernelGGL(embed_norm_smear_decode_kernel, dim3(B), dim3(256), 0, s, idx, wte, smear_w, smear_lambda, prev_in, prev_out,
-                           x_out, x0_out, E, vocab_rows, clear_words, clear_words ? n_clear : 0);
+        hipLaunchKernelGGL(embed_norm_smear_decode_kernel, dim3(B + fill_wgs), dim3(256), 0, s, idx, wte, smear_w, smear_lambda, prev_in, prev_out,
+                           x_out, x0_out, E, vocab_rows, clear_words, clear_words ? n_clear : 0, B, (uint4*)fill, (uint32_t)(fill_bytes / 16));
     else
         hipLaunchKernelGGL(embed_norm_smear_kernel, dim3(B * T), dim3(256), 2 * E * sizeof(float), s, idx, wte, smear_w, smear_lambda,
                            prev_in, prev_out, x_out, x0_out, T, E, vocab_rows, clear_words, clear_words ? n_clear : 0);

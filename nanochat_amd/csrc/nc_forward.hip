@@ -2,7 +2,8 @@
 // Python loop at nanochat/gpt.py:459-524 (and of the module calls it makes into gpt.py:84-153 and
 // fp8.py:202-213).  One call enqueues every kernel of the step; no host synchronisation, no allocation.
 //
-// Per layer, decode (M = B*T <= 128 rows), 7 or 8 launches, each making a single dependent trip to memory:
+// A decode step of up to 8 rows (where nc_step_fits): three launches, embedding, all layers, lm_head.
+// Per layer, decode otherwise (M = B*T <= 128 rows), 7 or 8 launches, each making a single dependent trip to memory:
 //   mix_norm            x += mlp_out(prev) [read from split partials]; x = rl*x + xl*x0; xn = norm(x); amax(xn)
 //   linear q|k|v        quantize xn inside the GEMM; K split over workgroups           -> fp32 partials
 //   attention           each (row, kv head) workgroup first sums its heads' partials (three weight scales), applies
@@ -34,6 +35,7 @@
 //   zeroed                u32               amax sites [4L+1] x 8 slots on separate lines | attention split counters,
 //                                           | meetings (prefill only), cleared by the embedding kernel at the start of the call
 //   gemm_parts, attn_parts                  split partials of the small-M linears and of attention
+//   step_words, step_exchange               the one launch of a step of few rows (nc_step.hip): registration, and what its workgroups hand each other
 #include <stdio.h>
 #include "../../include/nanochat_amd.h"
 #include "nc_common.h"
@@ -83,6 +85,10 @@ struct Workspace {
     NcMeeting meeting(int i) const { return NcMeeting{meetings + (size_t)i * NC_MEETING_WORDS, NC_MEETING_SPINS}; }
     int zero_words;
     uint8_t *gemm_parts, *gemm_parts2, *attn_parts, *shared_parts;
+    uint32_t* step_words;      // steps of few rows (nc_step.hip): NC_STEP_WORDS, and the amax site of the rows they leave
+    uint8_t* step_exchange;
+    size_t step_exchange_bytes;
+    uint32_t* step_site() const { return nc_amax_slotted(step_words + NC_STEP_WORDS); }
     size_t gemm_part_bytes, attn_part_bytes, shared_part_bytes;
     size_t total;
 };
@@ -98,6 +104,8 @@ bool fused_rows(const nc_model_desc* m, int M) {
     return nc_gemm_decode_splits(qkv_w, E) > 1 && nc_gemm_decode_splits(E, m->n_head * 128) > 1 && nc_gemm_decode_splits(4 * E, E) > 1 &&
            nc_gemm_decode_splits(E, 4 * E) > 1;
 }
+
+constexpr int STEP_CLEARED = NC_STEP_WORDS + NC_AMAX_SLOTS * NC_AMAX_STRIDE;
 
 Workspace carve(const nc_model_desc* m, int B, int T, void* base) {
     const size_t M = (size_t)B * T, E = m->n_embd;
@@ -161,6 +169,12 @@ Workspace carve(const nc_model_desc* m, int B, int T, void* base) {
     // turns out to be, the launch cuts it into at most as many chunks as a whole cache row would get
     w.shared_part_bytes = (T == 1 && (long)B * m->n_kv_head >= NC_SHARED_MIN_ROW_HEADS) ? nc_attn_shared_partial_bytes(B, m->n_head, m->n_kv_head, 1 << 20) : 0;
     w.shared_parts = c.take<uint8_t>(w.shared_part_bytes);
+    const bool step = T == 1 && nc_step_fits(B, m->n_layer, m->n_embd, m->n_head, m->n_kv_head);
+    w.step_words = c.take<uint32_t>(step ? STEP_CLEARED : 0);
+    NcStepArgs sizes{};
+    sizes.B = B, sizes.L = m->n_layer, sizes.E = m->n_embd, sizes.H = m->n_head, sizes.Hkv = m->n_kv_head;
+    w.step_exchange_bytes = step ? nc_step_exchange(sizes, NC_STEP_MAX_KEYS) : 0;      // (the most it takes: the cache's length is not known here)
+    w.step_exchange = c.take<uint8_t>(w.step_exchange_bytes);
     w.total = (c.off + 255) & ~(size_t)255;
     return w;
 }
@@ -175,6 +189,23 @@ constexpr size_t AHEAD_LAYER_BYTES_FEW = 24u << 20;
 bool reads_ahead(const nc_model_desc* m, int M) {
     const size_t E = m->n_embd, layer = E * ((size_t)(2 * m->n_head + 2 * m->n_kv_head) * 128 + 8 * E);
     return M > 128 || (M > 64 && layer <= AHEAD_LAYER_BYTES_FEW);
+}
+
+int most_visible_keys(const nc_model_desc* m, int Tmax) {
+    int most = 0;
+    for (int i = 0; i < m->n_layer; i++) {
+        const int w = m->layers[i].window_left, n = w >= 0 && w < Tmax ? w : Tmax;
+        most = n > most ? n : most;
+    }
+    return most;
+}
+
+// Whether a step goes through nc_step.hip.  Launches of their own have what one has not: times of each kernel (the profiler), rows of any alignment, and a
+// prompt that is read once for all rows.
+bool takes_step(const nc_model_desc* m, const nc_cache_desc* kv, int B) {
+    const uintptr_t pointers = (uintptr_t)m->wte | (uintptr_t)kv->prev_in | (uintptr_t)kv->prev_out | (uintptr_t)kv->k_cache | (uintptr_t)kv->v_cache;
+    return nc_step_fits(B, m->n_layer, m->n_embd, m->n_head, m->n_kv_head) && !nc_prof_on() && (pointers & 15) == 0 && kv->max_seq_len < NC_STEP_MAX_KEYS &&
+           !(kv->shared_prefix > 0 && B * m->n_kv_head >= NC_SHARED_MIN_ROW_HEADS);
 }
 
 NcGemmSegs one_seg(int n) { return NcGemmSegs{1, {n, 0, 0, 0}}; }
@@ -271,7 +302,7 @@ extern "C" int nc_gpt_reads_ahead(const nc_model_desc* model, int B, int T) { re
 // tap_x (or nullptr): bf16 [L+1, M, E], slot i = the residual stream as layer i reads it (after the lambda mix, gpt.py:500), slot L = the
 // final normalised rows (gpt.py:508).  tap_y (or nullptr): bf16 [L, M, H*128], the attention outputs before c_proj (gpt.py:113-124).
 static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, const int64_t* idx, int B, int T, float* logits_out,
-                            int last_only, void* workspace, size_t workspace_bytes, bf16_t* tap_x, bf16_t* tap_y, hipStream_t s) {
+                            int last_only, void* workspace, size_t workspace_bytes, bf16_t* tap_x, bf16_t* tap_y, hipStream_t s, int present = 0) {
     NC_CHECK_ARG(m && kv && idx && logits_out && workspace, "gpt_forward: null pointer");
     NC_CHECK_ARG(B > 0 && T > 0, "gpt_forward: bad batch/time B=%d T=%d", B, T);
     NC_CHECK_ARG(m->n_embd == m->n_head * 128, "gpt_forward: head_dim must be 128 (n_embd=%d n_head=%d)", m->n_embd, m->n_head);
@@ -287,6 +318,31 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
     const size_t layer_elems = (size_t)B * kv->max_seq_len * Hkv * 128;
     const LinearRunner lin{w, s};
     int site = 0;   // amax / inv slot of the next FP8 linear input
+
+    // a step of few rows: embedding, one launch for all layers, lm_head
+    if (T == 1 && !tap_x && !tap_y && takes_step(m, kv, B)) {
+        NcStepArgs a{};
+        a.x0 = w.x0, a.xb = w.xb, a.xn = w.xn, a.exchange = w.step_exchange, a.words = w.step_words, a.head_site = w.step_site();
+        a.k_cache = kv->k_cache, a.v_cache = kv->v_cache, a.cache_seqlens = (int32_t*)kv->cache_seqlens, a.idx = idx, a.cos_t = m->cos, a.sin_t = m->sin;
+        a.resid_lambdas = m->resid_lambdas, a.x0_lambdas = m->x0_lambdas, a.backout_lambda = m->backout_lambda;
+        a.layer_elems = layer_elems;
+        a.B = B, a.L = L, a.E = E, a.H = H, a.Hkv = Hkv, a.Tmax = kv->max_seq_len, a.rope_len = m->rope_len, a.vocab_rows = m->padded_vocab, a.advance = kv->advance;
+        NcStepLayers layers{};
+        for (int i = 0; i < L; i++) {
+            const nc_layer_desc& ly = m->layers[i];
+            NC_CHECK_ARG(ly.w_qkv && ly.inv_qkv && ly.w_attn_proj && ly.w_fc && ly.w_mlp_proj, "gpt_forward: layer %d has no FP8 weights", i);
+            layers.layer[i] = NcStepLayer{ly.w_qkv, ly.inv_qkv, ly.w_attn_proj, ly.inv_attn_proj, ly.w_fc, ly.inv_fc, ly.w_mlp_proj, ly.inv_mlp_proj,
+                                          ly.ve_table, ly.ve_gate_w, ly.window_left, 0};
+        }
+        const size_t fill = nc_step_exchange(a, most_visible_keys(m, kv->max_seq_len));
+        NC_CHECK_ARG(fill <= w.step_exchange_bytes, "gpt_forward: exchange of %zu bytes, %zu in the workspace", fill, w.step_exchange_bytes);
+        TRY(nc_launch_embed_norm_smear(idx, m->wte, m->smear_w, m->smear_lambda, kv->prev_in, kv->prev_out, w.x, w.x0, B, T, E, m->padded_vocab, w.step_words,
+                                       STEP_CLEARED, s, w.step_exchange, fill));
+        TRY(nc_launch_step(a, layers, present, s));
+        return nc_launch_gemm_decode(w.xn, 1, w.step_site(), nullptr, m->w_lm_head, m->inv_lm_head, one_seg(m->vocab_size), logits_out, 1, m->softcap, nullptr, M,
+                                     m->vocab_size, E, m->vocab_size, (float*)w.gemm_parts, w.gemm_part_bytes, 1, nullptr, s);
+    }
+    NC_CHECK_ARG(present == 0, "gpt_forward: not a step that one launch takes");
 
     // x0 is the post-smear embedding; layer 0 reads it through both x and x0 (gpt.py:495,500)
     TRY(nc_launch_embed_norm_smear(idx, m->wte, m->smear_w, m->smear_lambda, kv->prev_in, kv->prev_out, w.x, w.x0, B, T, E,
@@ -479,6 +535,12 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
 extern "C" int nc_gpt_forward(const nc_model_desc* m, const nc_cache_desc* kv, const int64_t* idx, int B, int T, float* logits_out,
                               int last_only, void* workspace, size_t workspace_bytes, nc_stream_t stream) {
     return gpt_forward_impl(m, kv, idx, B, T, logits_out, last_only, workspace, workspace_bytes, nullptr, nullptr, (hipStream_t)stream);
+}
+
+extern "C" int nc_gpt_forward_present(const nc_model_desc* m, const nc_cache_desc* kv, const int64_t* idx, int B, float* logits_out, void* workspace,
+                                      size_t workspace_bytes, int present, nc_stream_t stream) {
+    NC_CHECK_ARG(present > 0, "gpt_forward_present: no workgroups");
+    return gpt_forward_impl(m, kv, idx, B, 1, logits_out, 1, workspace, workspace_bytes, nullptr, nullptr, (hipStream_t)stream, present);
 }
 
 extern "C" int nc_gpt_forward_tapped(const nc_model_desc* m, const nc_cache_desc* kv, const int64_t* idx, int B, int T, float* logits_out,

@@ -102,7 +102,8 @@ struct NcRowRecipe {
 int nc_launch_rmsnorm(const bf16_t* x, bf16_t* out, int rows, int cols, uint32_t* amax_ws, hipStream_t s);
 int nc_launch_embed_norm_smear(const int64_t* idx, const bf16_t* wte, const float* smear_w, const float* smear_lambda,
                                const bf16_t* prev_in, bf16_t* prev_out, bf16_t* x_out, bf16_t* x0_out, int B, int T, int E,
-                               int vocab_rows, uint32_t* clear_words, int n_clear, hipStream_t s);
+                               int vocab_rows, uint32_t* clear_words, int n_clear, hipStream_t s, void* fill = nullptr, size_t fill_bytes = 0);
+// (fill: 16-byte aligned; set to ones by the same launch, one token per row only)
 struct NcQuantRows;           // (nc_meeting.h) the normalised rows as e4m3 with their inverse scale; of the bf16 rows the first 16 columns
 bool nc_mix_norm_e4m3_fits(int rows, int cols, bool parts);
 int nc_launch_mix_norm(bf16_t* x, const bf16_t* add, const bf16_t* x0, const float* resid_lambda, const float* x0_lambda,
@@ -167,6 +168,53 @@ int nc_launch_attention_fused(NcRopeSrc rope, bf16_t* k_cache, bf16_t* v_cache, 
                               bf16_t* out, int B, int H, int Hkv, int Tmax, uint32_t* counters, void* partials, size_t partial_bytes,
                               uint32_t* amax_ws, int force_splits, int counters_of_pass, hipStream_t s);
 
+// ---- the layers of a decode step of few rows in one launch (nc_step.hip)
+#define NC_STEP_ROWS 8
+#define NC_STEP_MAX_LAYERS 40
+#define NC_STEP_MAX_E 1792
+#define NC_STEP_MAX_KEYS (1 << 24)        // of a cache row
+#define NC_STEP_SPLIT_KEYS 128            // of a row's kv head to a workgroup, while there are workgroups
+#define NC_STEP_MAX_SPLITS 12
+#define NC_STEP_WORDS (3 * 32)           // zero before the launch
+struct NcStepLayer {
+    const uint8_t* w_qkv;
+    const float* inv_qkv;
+    const uint8_t* w_attn_proj;
+    const float* inv_attn_proj;
+    const uint8_t* w_fc;
+    const float* inv_fc;
+    const uint8_t* w_mlp_proj;
+    const float* inv_mlp_proj;
+    const bf16_t* ve_table;
+    const float* ve_gate_w;
+    int window_left, reserved;
+};
+struct NcStepArgs {                       // (by value, with the layers behind it: under 4 KB)
+    const bf16_t* x0;                     // [B,E] embedded rows
+    bf16_t *xb, *xn;                      // [B,E] the backout rows (scratch), the final normalised rows
+    uint8_t* exchange;                    // what the workgroups hand each other (nc_step_exchange), every byte 0xff before the launch
+    uint32_t* words;                      // NC_STEP_WORDS
+    uint32_t* head_site;                  // amax of xn
+    bf16_t *k_cache, *v_cache;
+    int32_t* cache_seqlens;
+    const int64_t* idx;
+    const bf16_t *cos_t, *sin_t;
+    const float *resid_lambdas, *x0_lambdas, *backout_lambda;
+    size_t layer_elems;                   // of the caches
+    int B, L, E, H, Hkv, Tmax, rope_len, vocab_rows, advance;
+    // set by nc_step_exchange: workgroups, a layer's part of `exchange` and what lies where in it (q|k|v at its start), and behind the layers the parts of rows whose keys several workgroups share
+    int wgs, layer_bytes, off_y, off_proj, off_h, off_mlp, parts_bytes;
+    uint8_t* parts;
+};
+struct NcStepLayers {
+    NcStepLayer layer[NC_STEP_MAX_LAYERS];
+};
+static_assert(sizeof(NcStepArgs) % 8 == 0 && sizeof(NcStepArgs) + sizeof(NcStepLayers) <= 4096, "kernel arguments");
+size_t nc_step_exchange(NcStepArgs& a, int most_keys);   // B, L, E, H, Hkv and exchange are given, and how many keys a row may have; returns the bytes that `exchange` takes
+bool nc_step_fits(int B, int L, int E, int H, int Hkv);
+// present: workgroups that are started (tests: as if the others had found no place), 0: all
+int nc_launch_step(const NcStepArgs& a, const NcStepLayers& layers, int present, hipStream_t s);
+
 // ---- sampling (nc_sample.hip)
 int nc_launch_softcap(const bf16_t* raw, float* out, int64_t n, float softcap, hipStream_t s);
 int nc_launch_sample(const float* logits, int B, int V, int ld, float temperature, int top_k, const float* noise,
@@ -175,6 +223,7 @@ int nc_launch_sample(const float* logits, int B, int V, int ld, float temperatur
 // ---- optional event timing (nc_profile.hip)
 int nc_prof_begin(int cls, double units, hipStream_t s, int64_t tag = 0);
 void nc_prof_end(int slot, hipStream_t s);
+bool nc_prof_on();
 bool nc_prof_take(int cls, double units, int64_t tag, hipEvent_t* start, hipEvent_t* stop);
 struct NcProfScope {
     int slot;

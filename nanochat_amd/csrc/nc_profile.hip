@@ -20,6 +20,8 @@ int g_created = 0, g_used = 0;
 bool g_on = false;
 }  // namespace
 
+bool nc_prof_on() { return g_on; }
+
 int nc_prof_begin(int cls, double units, hipStream_t s, int64_t tag) {
     if (!g_on || cls < 0 || g_used >= POOL) return -1;
     if (g_used >= g_created) {

@@ -463,6 +463,120 @@ def test_prompts_on_two_streams(depth, T):
             assert torch.equal(got[i], want[i]) and torch.equal(together[i].k_cache, alone[i].k_cache) and torch.equal(together[i].v_cache, alone[i].v_cache)
 
 
+def _step_model(layers, heads, kv_heads, pattern="SSL", sequence_len=512, seed=5):
+    """A model whose sublayers write a part of the residual stream (as in perf/cases.py): a last bit in one layer is then no more than a few thousandths of the logits."""
+    from nanochat_amd.gpt import GPTConfig
+    from nanochat_amd.synthetic import random_init_model
+    cfg = GPTConfig(sequence_len=sequence_len, vocab_size=1024, n_layer=layers, n_head=heads, n_kv_head=kv_heads, n_embd=128 * heads, window_pattern=pattern)
+    model = random_init_model(cfg, DEV, seed=seed)
+    with torch.no_grad():
+        for block in model.transformer.h:
+            block.attn.c_proj.weight.mul_(0.1)
+            block.mlp.c_proj.weight.mul_(0.1)
+    return model
+
+
+def _step_cache(model, lengths, room, seed=6):
+    """Rows that hold `lengths` tokens each, and the embedding of the last one."""
+    from nanochat_amd.engine import KVCache
+    cfg = model.config
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    cache = KVCache(len(lengths), cfg.n_kv_head, max(lengths) + room, 128, cfg.n_layer, DEV, torch.bfloat16)
+    cache.k_cache.normal_(0.0, 1.2, generator=g)
+    cache.v_cache.normal_(0.0, 1.0, generator=g)
+    cache.set_seqlens(torch.tensor(lengths, dtype=torch.int32))
+    cache.prev_embedding = torch.nn.functional.rms_norm(torch.randn(len(lengths), 1, cfg.n_embd, generator=g, device=DEV), (cfg.n_embd,)).bfloat16()
+    return cache
+
+
+class _Present:
+    """The library with forwards of which only so many workgroups are started."""
+
+    def __init__(self, lib, present):
+        self._lib, self._present = lib, present
+
+    def __getattr__(self, name):
+        return getattr(self._lib, name)
+
+    def nc_gpt_forward(self, md, cd, idx, B, T, logits, last_only, ws, ws_bytes, stream):
+        return self._lib.nc_gpt_forward_present(md, cd, idx, B, logits, ws, ws_bytes, self._present, stream)
+
+
+# the edges of the launch's forms: 512, 1024, 1536 and 1792 columns, one and two query heads to a key head, one row and eight, rows that are empty, of one batch of keys
+# and one more, at the border of a workgroup's share of keys (128), past a window, and of unequal length
+STEP_CASES = [(3, 2, 2, [0]), (4, 2, 2, [63, 1]), (3, 4, 4, [127, 128, 129]), (5, 4, 2, [300]), (3, 5, 5, [5] * 8), (4, 8, 4, [0, 31, 32, 33, 256, 257, 500, 511]), (3, 9, 9, [700, 2]),
+              (3, 12, 6, [40] * 7), (4, 13, 13, [1000]), (3, 13, 13, [600] * 8), (3, 14, 7, [513, 512, 511]), (3, 14, 14, [130] * 4)]
+
+
+@pytest.mark.parametrize("layers, heads, kv_heads, lengths", STEP_CASES)
+def test_step_of_few_rows_in_one_launch_against_the_separate_launches(layers, heads, kv_heads, lengths, monkeypatch):
+    """Up to eight rows: all layers of a step in one launch, whose workgroups share the work out among those that have a place.  Against the separate launches
+    (what a tapped forward takes), which round in the same places and sum in another order: most results have the same bits.  Where a sum rounds the other
+    way, a bf16 value moves by 2^-8 of itself and an e4m3 value by 2^-3, and the layers behind carry it on; 2e-2 of the logits is half of what the oracle's own two
+    attention forms differ by.  With any number of workgroups the bits are the same."""
+    say(f"step in one launch: {layers} layers, {heads} heads on {kv_heads}, rows of {lengths}")
+    from nanochat_amd import gpt as gpt_module
+    B = len(lengths)
+    model = _step_model(layers, heads, kv_heads, sequence_len=512)
+    g = torch.Generator(device=DEV).manual_seed(7)
+    toks = [torch.randint(0, 1024, (B, 1), generator=g, device=DEV) for _ in range(2)]
+    real = gpt_module._lib.lib()
+
+    def steps(run, present=0):
+        cache = _step_cache(model, lengths, 2)
+        before = cache.k_cache.clone()
+        with monkeypatch.context() as m:
+            if present:
+                m.setattr(gpt_module._lib, "lib", lambda: _Present(real, present))
+            logits = [run(t, cache) for t in toks]
+            torch.cuda.synchronize()
+        for b, n in enumerate(lengths):
+            assert torch.equal(cache.k_cache[:, b, :n], before[:, b, :n])
+        assert cache.cache_seqlens.tolist() == [n + 2 for n in lengths]
+        return torch.stack(logits), cache.k_cache, cache.v_cache
+    one = steps(lambda t, c: model.forward_last(t, kv_cache=c))
+    apart = steps(lambda t, c: model.forward_tapped(t, kv_cache=c)[0][:, -1])
+    for got, want in zip(one, apart):
+        assert torch.isfinite(got).all()
+        assert rel_l2(got, want) <= 2e-2
+    for present in (1, 7, 100):
+        for got, want in zip(steps(lambda t, c: model.forward_last(t, kv_cache=c), present), one):
+            assert torch.equal(got, want), present
+
+
+def test_steps_and_prompts_on_three_streams():
+    """Steps of two models and the prompts of a third at once: no launch may wait for workgroups that the others keep from starting."""
+    say("steps on two streams beside prompts on a third")
+    from nanochat_amd.engine import KVCache
+    models = [_step_model(6, 13, 13, seed=1), _step_model(4, 4, 4, seed=2), _step_model(6, 10, 10, seed=3)]
+    g = torch.Generator(device=DEV).manual_seed(8)
+    toks = [torch.randint(0, 1024, (b, 1), generator=g, device=DEV) for b in (3, 8)] + [torch.randint(0, 1024, (1, 600), generator=g, device=DEV)]
+    reps = 12
+
+    def run(i):
+        if i == 2:
+            out = []
+            for _ in range(reps):
+                cache = KVCache(1, 10, 600, 128, 6, DEV, torch.bfloat16)
+                out.append(models[2].forward_last(toks[2], kv_cache=cache))
+            return out
+        cache = _step_cache(models[i], [200 + 3 * b for b in range(toks[i].shape[0])], reps)
+        return [models[i].forward_last(toks[i], kv_cache=cache) for _ in range(reps)]
+    alone = [torch.stack(run(i)) for i in range(3)]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    for s in streams:
+        s.wait_stream(torch.cuda.current_stream())
+    for _ in range(3):
+        together = [None] * 3
+        for i, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                together[i] = run(i)
+        torch.cuda.synchronize()
+        for i in range(3):
+            assert torch.equal(torch.stack(together[i]), alone[i]), i
+
+
 def test_ragged_rows():
     """Per-row cache lengths (outside the reference's GPT.forward, inside FA3's signature): every row
     must equal the same row run alone."""
