@@ -153,6 +153,14 @@ struct NcRoute {
     int tile_rows, max_tiles;
 };
 int nc_launch_stack_route(const NcRoute& r, int M, hipStream_t s);
+// Rows rows[0 .. n-1] of four arrays, one behind the other; pitches and bytes in multiples of 16.
+struct NcSelect {
+    const void* from;
+    void* to;
+    int64_t pitch;                 // bytes from row to row, on both sides
+    int bytes;                     // of a row that are copied (0: none)
+};
+int nc_launch_stack_select(const NcSelect (&parts)[4], const int32_t* rows, int n, hipStream_t s);
 int nc_launch_stack_cache_copy(const void* src, void* dst, int src_rows, int dst_rows, int64_t src_stride, int64_t dst_stride, int64_t bytes,
                                hipStream_t s);
 

@@ -11,6 +11,7 @@
 //   linear   projections . h;  mixers, side by side if there are two  -> `cat`
 //   linear   w_out . cat -> sums in fp32 (few rows; 32-bit: partial ones);  row add  x += norm1(sums) -> h
 //   linear   gate and up . h, activation in the epilogue;  linear  down -> sums;  row add  x += norm2(sums) -> h
+// The last run's mixers are followed by a gather of the rows whose logits are wanted, and by nothing if there are none.
 #include "../../include/nanochat_amd_stack.h"
 #include "nc_stack.h"
 
@@ -38,6 +39,8 @@ struct Workspace {
     void *h, *proj, *cat, *h_last, *q_lat, *o_lat, *kv, *att_parts, *ret, *act, *e_out, *u, *dtr;
     float* slot_w;
     int32_t *chosen, *slot_of, *perm, *tiles, *n_tiles;
+    float *sel_x, *sel_router;        // the rows that go on behind the last run's mixers (goes_on_alone)
+    void *sel_h, *sel_cat;
     size_t att_part_bytes, part_bytes, total;
 };
 
@@ -76,6 +79,17 @@ int expert_tile_rows(const nc_stack_layer& l, int M) {
 int expert_max_tiles(const nc_stack_layer& l, int M, int tile_rows) {
     const int pairs = M * l.top;
     return pairs / tile_rows + (pairs < l.experts ? pairs : l.experts);
+}
+// Behind the mixers of the last run every row is by itself, and of a prompt one row a sequence has logits: only the chosen rows take part in the rest of that run, gathered by a
+// launch of their own (3 to 4 us).  Of experts that pays from two rows less on, of other layers from 64 (with `in_two_products`; us, all rows / the chosen one: Palilix with experts,
+// width 2048, 1792 tokens 3514 / 3238, 100 828 / 709, width 512, 3 tokens 247 / 244, 32-bit, width 1024, 333 tokens 1018 / 910; dense, width 2048, 1000 tokens 831 / 760, width 512, 40 tokens
+// 226 / 229, 65 242 / 242, 256 261 / 259; Zodirax, width 4096, 1792 tokens 4034 / 3603, 2048, 65 tokens 595 / 578, 512, 128 tokens 386 / 384).
+bool goes_on_alone(const nc_stack_layer& l, int M, int n_logits) { return n_logits > 0 && M - n_logits >= (l.ff == NC_FF_EXPERTS ? 2 : 64); }
+// ... and the columns of its input matrix that the mixers do not read become a product of the chosen rows alone, where the products of the others are worth a launch and a second
+// trip for the weight (us, one product / two: dense, width 512, 1000 tokens 353 / 352, 1024, 256 tokens 306 / 306, 1000 462 / 453, 2048, 256 tokens 471 / 463; experts with
+// a shared one of 2048, width 2048, 400 tokens 894 / 900; 32-bit, width 768, 200 tokens 481 / 476, 896, 70 380 / 383).
+bool in_two_products(int dtype, const nc_stack_layer& l, int Wp, int M, int n_logits) {
+    return (double)(M - n_logits) * (l.n_in - l.mix_cols) * Wp >= (dtype ? 4e8 : 4e9);
 }
 size_t max_of(size_t a, size_t b) { return a > b ? a : b; }
 
@@ -134,6 +148,16 @@ Workspace carve(const nc_stack_model* m, int B, int T, int n_logits, int max_key
             eout = max_of(eout, p * Wp * es);
         }
     }
+    // (a run of a layer that is not there is refused by the forward, which asks here first)
+    const int end_of = m->n_runs > 0 ? m->runs[m->n_runs - 1].layer : -1;
+    size_t sel = 0, sel_router = 0;
+    if (end_of >= 0 && end_of < m->n_layers && goes_on_alone(m->layers[end_of], (int)M, n_logits)) {
+        const nc_stack_layer& l = m->layers[end_of];
+        sel = n_logits, sel_router = sel * l.router_cols * 4;
+        parts = max_of(parts, nc_linear_splits(m->dtype, n_logits, (int)Wp, l.k_out) * sel * Wp * 4);
+        if (l.block == NC_BLOCK_POST_NORM && l.ff) parts = max_of(parts, nc_linear_splits(m->dtype, n_logits, (int)Wp, l.ff_p) * sel * Wp * 4);
+        if (l.ff == NC_FF_EXPERTS) tiles = max_of(tiles, expert_max_tiles(l, n_logits, expert_tile_rows(l, n_logits)));
+    }
     Carver c(base);
     Workspace w;
     w.x = (float*)c.take(M * Wp * 4);
@@ -165,6 +189,10 @@ Workspace carve(const nc_stack_model* m, int B, int T, int n_logits, int max_key
     w.bc = (float*)c.take(bc);
     w.dt = (float*)c.take(dt);
     w.x_parts = (float*)c.take(x_parts);
+    w.sel_x = (float*)c.take(sel * Wp * 4);
+    w.sel_h = c.take(sel * Wp * es);
+    w.sel_cat = c.take(sel * m->max_k_out * es);
+    w.sel_router = (float*)c.take(sel_router);
     w.total = (c.off + 255) & ~(size_t)255;
     return w;
 }
@@ -441,39 +469,62 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
         const nc_stack_run& run = m->runs[i];
         const nc_stack_layer& l = m->layers[run.layer];
         const bool post = l.block == NC_BLOCK_POST_NORM;
-        NcLinear in = nc_linear(w.h, Wp, l.w_in, M, l.n_in, Wp);
+        // the last run may end early for all rows but the chosen ones (goes_on_alone), or for all
+        const bool last = i + 1 == m->n_runs && !taps, alone = last && logit_rows && goes_on_alone(l, M, n_logits), ends = last && n_logits == 0;
+        // columns of the input matrix behind the mixers' own: router logits, and the feed-forward's first matrix, which goes to `cat`
+        auto rest_segs = [&](NcLinear& g, int col, const Workspace& to) {
+            if (l.router_cols) nc_linear_seg(g, col + l.router_cols, NC_SEG_F32, to.router, l.router_cols);
+            if (l.ff_cols) nc_linear_seg(g, col + l.router_cols + l.ff_cols, ff_seg_kind(l.ff), at(to.cat, l.mix_out, dt), l.k_out, l.ff_limit);
+        };
+        const bool mixers_only = !post && (ends || (alone && in_two_products(dt, l, Wp, M, n_logits)));
+        NcLinear in = nc_linear(w.h, Wp, l.w_in, M, mixers_only ? l.mix_cols : l.n_in, Wp);
         mixer_segs(l, in, w, dt);
-        if (l.router_cols) nc_linear_seg(in, l.mix_cols + l.router_cols, NC_SEG_F32, w.router, l.router_cols);
-        if (!post && l.ff_cols) nc_linear_seg(in, l.n_in, ff_seg_kind(l.ff), at(w.cat, l.mix_out, dt), l.k_out, l.ff_limit);
+        if (!post && !mixers_only) rest_segs(in, l.mix_cols, w);
         TRY(nc_launch_linear(dt, in, s));
-        TRY(run_mixers(m, kv, run, w, B, T, weights_behind(m, i, M), s));
+        TRY(run_mixers(m, kv, run, w, B, T, ends ? NcAhead{} : weights_behind(m, i, M), s));
+        if (ends) return 0;
+        Workspace r = w;
+        const int R = alone ? n_logits : M;
+        if (alone) {
+            r.x = w.sel_x, r.h = w.sel_h, r.cat = w.sel_cat, r.router = w.sel_router;
+            const int es = dt ? 4 : 2;
+            const NcSelect x{w.x, r.x, (int64_t)Wp * 4, Wp * 4}, cat{w.cat, r.cat, (int64_t)l.k_out * es, (mixers_only ? l.mix_out : l.k_out) * es};
+            const NcSelect h{w.h, r.h, (int64_t)Wp * es, mixers_only || l.ff == NC_FF_EXPERTS ? Wp * es : 0};
+            const NcSelect router{w.router, r.router, (int64_t)l.router_cols * 4, mixers_only ? 0 : l.router_cols * 4}, parts[4] = {x, cat, h, router};
+            TRY(nc_launch_stack_select(parts, logit_rows, R, s));
+            if (mixers_only && l.n_in > l.mix_cols) {
+                NcLinear rest = nc_linear(r.h, Wp, at(l.w_in, (int64_t)l.mix_cols * Wp, dt), R, l.n_in - l.mix_cols, Wp);
+                rest_segs(rest, 0, r);
+                TRY(nc_launch_linear(dt, rest, s));
+            }
+        }
 
         NcRowAdd add{};
-        add.x = w.x, add.tokens_per_row = T;
+        add.x = r.x, add.tokens_per_row = T;
         if (post) {
-            TRY(run_sums(dt, w.cat, l.w_out, M, Wp, l.k_out, w.parts, add, s));
+            TRY(run_sums(dt, r.cat, l.w_out, R, Wp, l.k_out, w.parts, add, s));
             add.post_norm_w = l.norm_w;
             if (l.ff) {
-                add.norm = NC_ROW_COPY, add.h = w.h;
-                TRY(nc_launch_stack_row_add(dt, add, m->eps, M, M, m->width, Wp, s));
-                NcLinear up = nc_linear(w.h, Wp, l.w_ff_in, M, l.ff_cols, Wp);
+                add.norm = NC_ROW_COPY, add.h = r.h;
+                TRY(nc_launch_stack_row_add(dt, add, m->eps, R, R, m->width, Wp, s));
+                NcLinear up = nc_linear(r.h, Wp, l.w_ff_in, R, l.ff_cols, Wp);
                 nc_linear_seg(up, l.ff_cols, ff_seg_kind(l.ff), w.act, l.ff_p);
                 TRY(nc_launch_linear(dt, up, s));
-                TRY(run_sums(dt, w.act, l.w_ff_out, M, Wp, l.ff_p, w.parts, add, s));
+                TRY(run_sums(dt, w.act, l.w_ff_out, R, Wp, l.ff_p, w.parts, add, s));
                 add.post_norm_w = l.norm2_w, add.h = nullptr;
             }
         } else {
             // a prompt's output matrix before the experts, whose weights would push it out of the last-level cache again
-            const bool few = M <= NC_FEW_ROWS;
-            if (l.ff == NC_FF_EXPERTS && few) TRY(run_experts(dt, l, M, Wp, w, s));
-            if (nc_linear_splits(dt, M, Wp, l.k_out) > 1) {
-                TRY(run_sums(dt, w.cat, l.w_out, M, Wp, l.k_out, w.parts, add, s));
+            const bool few = R <= NC_FEW_ROWS;
+            if (l.ff == NC_FF_EXPERTS && few) TRY(run_experts(dt, l, R, Wp, r, s));
+            if (nc_linear_splits(dt, R, Wp, l.k_out) > 1) {
+                TRY(run_sums(dt, r.cat, l.w_out, R, Wp, l.k_out, w.parts, add, s));
             } else {
-                NcLinear out = nc_linear(w.cat, l.k_out, l.w_out, M, Wp, l.k_out);
-                nc_linear_seg(out, Wp, NC_SEG_RESIDUAL, w.x, Wp);
+                NcLinear out = nc_linear(r.cat, l.k_out, l.w_out, R, Wp, l.k_out);
+                nc_linear_seg(out, Wp, NC_SEG_RESIDUAL, r.x, Wp);
                 TRY(nc_launch_linear(dt, out, s));
             }
-            if (l.ff == NC_FF_EXPERTS && !few) TRY(run_experts(dt, l, M, Wp, w, s));
+            if (l.ff == NC_FF_EXPERTS && !few) TRY(run_experts(dt, l, R, Wp, r, s));
             if (l.ff == NC_FF_EXPERTS) add.expert_out = w.e_out, add.slot_of = w.slot_of, add.slot_w = w.slot_w, add.top = l.top;
         }
         if (taps) add.tap = taps + (int64_t)i * M * Wp;
@@ -492,9 +543,9 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
             add.x = w.x, add.tokens_per_row = T;
         }
         if (n_logits == 0) return 0;
-        add.norm = final_norm, add.norm_w = m->final_norm_w, add.h = w.h_last, add.rows = logit_rows;
+        add.norm = final_norm, add.norm_w = m->final_norm_w, add.h = w.h_last, add.rows = alone ? nullptr : logit_rows;
         if (kv->advance) add.bump = kv->cache_seqlens, add.bump_by = kv->advance;
-        TRY(nc_launch_stack_row_add(dt, add, m->eps, M, n_logits, m->width, Wp, s));
+        TRY(nc_launch_stack_row_add(dt, add, m->eps, R, n_logits, m->width, Wp, s));
         NcLinear head = nc_linear(w.h_last, Wp, m->head, n_logits, m->vocab, Wp);
         nc_linear_seg(head, m->vocab, NC_SEG_LOGITS, logits_out, m->vocab, m->logit_scale, m->logit_softcap);
         TRY(nc_launch_linear(dt, head, s));

@@ -329,6 +329,17 @@ __global__ __launch_bounds__(256) void stack_cache_copy_kernel(const uint8_t* __
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < pieces; i += (int64_t)gridDim.x * 256) d[i] = s[i];
 }
 
+struct Select4 {
+    NcSelect part[4];
+};
+__global__ __launch_bounds__(256) void stack_select_kernel(Select4 all, const int32_t* __restrict__ rows) {
+    const int64_t i = blockIdx.x, m = rows[i];
+    const NcSelect p = all.part[blockIdx.y];
+    const uint4* const src = (const uint4*)((const uint8_t*)p.from + m * p.pitch);
+    uint4* const dst = (uint4*)((uint8_t*)p.to + i * p.pitch);
+    for (int k = threadIdx.x; k < p.bytes / 16; k += 256) dst[k] = src[k];
+}
+
 // columns per thread: 4 per step of 1024 columns
 #define STEPS_SWITCH(width_p, CALL)                      \
     do {                                                 \
@@ -393,6 +404,19 @@ int nc_launch_stack_cache_copy(const void* src, void* dst, int src_rows, int dst
     hipLaunchKernelGGL(stack_cache_copy_kernel, dim3(gx, dst_rows), dim3(256), 0, s, (const uint8_t*)src, (uint8_t*)dst, src_rows, src_stride, dst_stride,
                        pieces);
     NC_CHECK_LAUNCH("stack_cache_copy");
+    return 0;
+}
+
+int nc_launch_stack_select(const NcSelect (&parts)[4], const int32_t* rows, int n, hipStream_t s) {
+    double bytes = 0;
+    for (const NcSelect& p : parts) {
+        NC_CHECK_ARG((p.bytes == 0 || (p.from && p.to)) && p.pitch % 16 == 0 && p.bytes % 16 == 0 && p.bytes <= p.pitch, "stack_select: rows of %d bytes", p.bytes);
+        bytes += 2.0 * p.bytes * n;
+    }
+    NC_CHECK_ARG(rows && n > 0, "stack_select: no rows");
+    NcProfScope prof(NC_CLS_ROWS, bytes, s);
+    hipLaunchKernelGGL(stack_select_kernel, dim3(n, 4), dim3(256), 0, s, Select4{{parts[0], parts[1], parts[2], parts[3]}}, rows);
+    NC_CHECK_LAUNCH("stack_select");
     return 0;
 }
 

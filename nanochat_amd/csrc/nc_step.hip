@@ -491,6 +491,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
                     if (v >= LIST_CLOSED)                          // whoever closed the list is about to say how long it was
                         for (spin = 0; spin < WAIT_POLLS; spin++)
                             if ((v = __hip_atomic_load(ARG(words) + W_TEAM, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0) break;
+                    if (v - 1u >= (uint32_t)wgs) v = (uint32_t)wgs, lost = 1;       // (not one of a team: somebody else writes here.  Every wait below still ends)
                     if (lane == 0) said[1] = v;
                 }
                 __syncthreads();
