@@ -81,10 +81,14 @@ int expert_max_tiles(const nc_stack_layer& l, int M, int tile_rows) {
     return pairs / tile_rows + (pairs < l.experts ? pairs : l.experts);
 }
 // Behind the mixers of the last run every row is by itself, and of a prompt one row a sequence has logits: only the chosen rows take part in the rest of that run, gathered by a
-// launch of their own (3 to 4 us).  Of experts that pays from two rows less on, of other layers from 64 (with `in_two_products`; us, all rows / the chosen one: Palilix with experts,
+// launch of their own (3 to 4 us).  Of experts that pays from two rows less on, of other layers by their width (with `in_two_products`; us, all rows / the chosen one: Palilix with experts,
 // width 2048, 1792 tokens 3514 / 3238, 100 828 / 709, width 512, 3 tokens 247 / 244, 32-bit, width 1024, 333 tokens 1018 / 910; dense, width 2048, 1000 tokens 831 / 760, width 512, 40 tokens
-// 226 / 229, 65 242 / 242, 256 261 / 259; Zodirax, width 4096, 1792 tokens 4034 / 3603, 2048, 65 tokens 595 / 578, 512, 128 tokens 386 / 384).
-bool goes_on_alone(const nc_stack_layer& l, int M, int n_logits) { return n_logits > 0 && M - n_logits >= (l.ff == NC_FF_EXPERTS ? 2 : 64); }
+// 226 / 229, 65 242 / 242, 256 261 / 259; Zodirax, width 4096, 1792 tokens 4034 / 3603, 2048, 40 tokens 489 / 483, 1024, 40 373 / 369, 512, 128 386 / 384; 32-bit, width 384, 65 tokens
+// 504 / 510).
+bool goes_on_alone(const nc_stack_layer& l, int Wp, int M, int n_logits) {
+    const int64_t others = (int64_t)M - n_logits;
+    return n_logits > 0 && (l.ff == NC_FF_EXPERTS ? others >= 2 : others * Wp >= 48 * 1024);
+}
 // ... and the columns of its input matrix that the mixers do not read become a product of the chosen rows alone, where the products of the others are worth a launch and a second
 // trip for the weight (us, one product / two: dense, width 512, 1000 tokens 353 / 352, 1024, 256 tokens 306 / 306, 1000 462 / 453, 2048, 256 tokens 471 / 463; experts with
 // a shared one of 2048, width 2048, 400 tokens 894 / 900; 32-bit, width 768, 200 tokens 481 / 476, 896, 70 380 / 383).
@@ -151,7 +155,7 @@ Workspace carve(const nc_stack_model* m, int B, int T, int n_logits, int max_key
     // (a run of a layer that is not there is refused by the forward, which asks here first)
     const int end_of = m->n_runs > 0 ? m->runs[m->n_runs - 1].layer : -1;
     size_t sel = 0, sel_router = 0;
-    if (end_of >= 0 && end_of < m->n_layers && goes_on_alone(m->layers[end_of], (int)M, n_logits)) {
+    if (end_of >= 0 && end_of < m->n_layers && goes_on_alone(m->layers[end_of], (int)Wp, (int)M, n_logits)) {
         const nc_stack_layer& l = m->layers[end_of];
         sel = n_logits, sel_router = sel * l.router_cols * 4;
         parts = max_of(parts, nc_linear_splits(m->dtype, n_logits, (int)Wp, l.k_out) * sel * Wp * 4);
@@ -470,7 +474,7 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
         const nc_stack_layer& l = m->layers[run.layer];
         const bool post = l.block == NC_BLOCK_POST_NORM;
         // the last run may end early for all rows but the chosen ones (goes_on_alone), or for all
-        const bool last = i + 1 == m->n_runs && !taps, alone = last && logit_rows && goes_on_alone(l, M, n_logits), ends = last && n_logits == 0;
+        const bool last = i + 1 == m->n_runs && !taps, alone = last && logit_rows && goes_on_alone(l, Wp, M, n_logits), ends = last && n_logits == 0;
         // columns of the input matrix behind the mixers' own: router logits, and the feed-forward's first matrix, which goes to `cat`
         auto rest_segs = [&](NcLinear& g, int col, const Workspace& to) {
             if (l.router_cols) nc_linear_seg(g, col + l.router_cols, NC_SEG_F32, to.router, l.router_cols);
