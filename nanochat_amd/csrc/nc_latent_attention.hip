@@ -760,7 +760,7 @@ int launch_mfma(const NcLatentGeom& g, const bf16_t* q, const bf16_t* cache, con
 }
 template <int DN, int DR, int DV>
 int launch_expanded(const NcLatentGeom& g, const bf16_t* q, int ldq, const bf16_t* kv, int keys, const bf16_t* cache, const int32_t* seqlens, bf16_t* out,
-                    int ldo, const NcAhead* ahead, hipStream_t s) {
+                    int ldo, const NcBehind* ahead, hipStream_t s) {
     if ((int64_t)((g.T + 127) / 128) * g.heads * g.B >= 200)
         nc_launch_ahead(dim3((g.T + 127) / 128, g.heads, g.B), ahead, [&](dim3 grid, auto a) {
             hipLaunchKernelGGL((latent_expanded_kernel<DN, DR, DV, 4, decltype(a)>), grid, dim3(256), 0, s, g, q, ldq, kv, keys, cache, seqlens, out, ldo, a);
@@ -867,7 +867,7 @@ int nc_launch_latent_attention(int dtype, const NcLatentGeom& g, const void* q_l
 bool nc_latent_expanded_ok(int dtype, const NcLatentGeom& g) { return dtype == 0 && g.dim_p <= 128 && g.rot_p <= 64 && g.vdim_p <= 128; }
 
 int nc_launch_latent_expanded(const NcLatentGeom& g, const bf16_t* q, int ldq, const bf16_t* kv, int keys, const bf16_t* cache, const int32_t* seqlens,
-                              bf16_t* out, int ldo, const NcAhead* ahead, hipStream_t s) {
+                              bf16_t* out, int ldo, const NcBehind* ahead, hipStream_t s) {
     NC_CHECK_ARG(nc_latent_expanded_ok(0, g) && keys >= g.pos_max + g.T && keys <= g.Tmax, "latent_expanded: sizes not supported");
     const int dqk = g.dim_p + g.rot_p;
     // causal pairs: all earlier keys and half of the new ones

@@ -37,6 +37,22 @@ static inline void nc_launch_ahead(dim3 grid, const NcAhead* a, Launch&& launch)
     launch(grid, NcNoAhead{});
 }
 
+// What a mixer's launch is told beside its own work: what to read ahead, or (the last mixers of a prompt) the rows whose results are wanted, flat indices row * T + token.
+struct NcBehind : NcAhead {
+    const int32_t* chosen;
+    int n_chosen;                 // 0: all rows
+};
+// Launches of tiles of tokens take a form that leaves out the tiles without a chosen one; it reads nothing ahead.
+struct NcChosen {
+    const int32_t* rows;
+    int n;
+};
+template <typename Launch>
+static inline void nc_launch_behind(dim3 grid, const NcBehind* a, Launch&& launch) {
+    if (a && a->n_chosen > 0) launch(grid, NcChosen{a->chosen, a->n_chosen});
+    else nc_launch_ahead(grid, a, launch);
+}
+
 // for the `wg`th of `wgs` workgroups of THREADS threads; a load past the end of a range returns zeros.  (Not with the non-temporal hint: such loads leave
 // nothing in the last-level cache.)
 template <int THREADS>
@@ -68,3 +84,13 @@ __device__ __forceinline__ bool reads_ahead(const NcAhead& a, int rows) {
 }
 template <int THREADS>
 __device__ __forceinline__ bool reads_ahead(NcNoAhead, int) { return false; }
+template <int THREADS>
+__device__ __forceinline__ bool reads_ahead(const NcChosen&, int) { return false; }
+// whether none of the rows first .. end - 1 is chosen; the same in every wave
+template <typename A>
+__device__ __forceinline__ bool none_chosen(const A&, int64_t, int64_t) { return false; }
+__device__ __forceinline__ bool none_chosen(const NcChosen& c, int64_t first, int64_t end) {
+    bool hit = false;
+    for (int i = threadIdx.x & 63; i < c.n; i += 64) hit |= c.rows[i] >= first && c.rows[i] < end;
+    return __builtin_amdgcn_ballot_w64(hit) == 0;
+}

@@ -290,6 +290,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void r
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), qb = wave % QB, vs = wave / QB;
     const int col = lane & 31, hl = lane >> 5;
     const int half = g.rot_dims / 2, pos0 = seqlens[b], t0 = chunk * C, n = min(C, g.T - t0);
+    if (none_chosen(ahead, (int64_t)b * g.T + t0, (int64_t)b * g.T + t0 + n)) return;
     const float l2 = decay[2 * h + 1];
     const bf16_t* base = proj + ((int64_t)b * g.T + t0) * ldp;
     const float2* turns = (const float2*)rope;
@@ -595,7 +596,7 @@ int chunk_size(int dtype, const NcRetentionGeom& g) {
 }
 template <int DK, int DV, int C>
 int launch_chunked(const NcRetentionGeom& g, const bf16_t* proj, int ldp, const float* decay, const float* rope, int rope_len, const int32_t* seqlens,
-                   const float* state_in, float* state_out, float eps, bf16_t* out, int ldo, void* workspace, const NcAhead* ahead, hipStream_t s) {
+                   const float* state_in, float* state_out, float eps, bf16_t* out, int ldo, void* workspace, const NcBehind* ahead, hipStream_t s) {
     const int chunks = (g.T + C - 1) / C;
     float* kv = (float*)workspace;
     bf16_t* prefix = (bf16_t*)(kv + (int64_t)g.B * chunks * g.heads * DK * DV);
@@ -603,7 +604,7 @@ int launch_chunked(const NcRetentionGeom& g, const bf16_t* proj, int ldp, const 
                        chunks);
     hipLaunchKernelGGL(retention_scan_kernel, dim3((DK * DV + 1023) / 1024, g.heads, g.B), dim3(256), 0, s, g, decay, seqlens, kv, prefix, state_in, state_out,
                        chunks, C);
-    nc_launch_ahead(dim3(chunks, g.heads, g.B), ahead, [&](dim3 grid, auto a) {
+    nc_launch_behind(dim3(chunks, g.heads, g.B), ahead, [&](dim3 grid, auto a) {
         hipLaunchKernelGGL((retention_chunk_out_kernel<DK, DV, C, decltype(a)>), grid, dim3(256), 0, s, g, proj, ldp, decay, rope, rope_len, seqlens, prefix, chunks, eps, out,
                            ldo, a);
     });
@@ -637,7 +638,7 @@ size_t nc_retention_workspace_bytes(int dtype, const NcRetentionGeom& g) {
 
 int nc_launch_retention(int dtype, const NcRetentionGeom& g, const void* proj, int ldp, const float* decay, const float* rope, int rope_len,
                         const int32_t* seqlens, const float* state_in, float* state_out, float eps, void* out, int ldo, void* workspace,
-                        const NcAhead* ahead, hipStream_t s) {
+                        const NcBehind* ahead, hipStream_t s) {
     NC_CHECK_ARG(g.rot_dims % 2 == 0 && g.rot_dims <= g.dim && g.dim <= g.dim_p && g.vdim <= g.vdim_p && g.dim_p % 8 == 0 && g.vdim_p % 8 == 0,
                  "retention: dim=%d/%d vdim=%d/%d rot=%d", g.dim, g.dim_p, g.vdim, g.vdim_p, g.rot_dims);
     NC_CHECK_ARG(state_in != state_out, "retention: the state is not updated in place");

@@ -331,7 +331,7 @@ int chunk_count(const NcScanGeom& g) {
 
 template <typename T, int SP>
 int launch_scan(const NcScanGeom& g, int lg, const T* u, const float* dt, const float* bc, const float* a_log2, const float* skip, const T* z, int ldz,
-                const int32_t* seqlens, const float* state_in, float* state_out, T* out, int ldo, void* workspace, const NcAhead* ahead, hipStream_t s) {
+                const int32_t* seqlens, const float* state_in, float* state_out, T* out, int ldo, void* workspace, const NcBehind* ahead, hipStream_t s) {
     const int chunks = chunk_count(g), len = chunk_len(g), xs = channel_groups(g, lg), bytes = TB * 2 * g.state_p * 4;
     if (chunks == 1) {
         nc_launch_ahead<sizeof(T) == 2>(dim3(xs, 1, g.B), ahead, [&](dim3 grid, auto a) {
@@ -419,7 +419,7 @@ size_t nc_scan_workspace_bytes(const NcScanGeom& g) {
 }
 
 int nc_launch_scan(int dtype, const NcScanGeom& g, const void* u, const float* dt, const float* bc, const float* a_log2, const float* skip, const void* z, int ldz,
-                   const int32_t* seqlens, const float* state_in, float* state_out, void* out, int ldo, void* workspace, const NcAhead* ahead, hipStream_t s) {
+                   const int32_t* seqlens, const float* state_in, float* state_out, void* out, int ldo, void* workspace, const NcBehind* ahead, hipStream_t s) {
     int sp = 0, lg = 0;
     NC_CHECK_ARG(lanes_of(g.state_p, sp, lg) && g.state <= g.state_p, "scan: %d states per channel in %d", g.state, g.state_p);
     NC_CHECK_ARG(u && dt && bc && a_log2 && skip && z && out && state_in != state_out, "scan: null operand");

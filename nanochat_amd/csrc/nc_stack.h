@@ -182,7 +182,7 @@ int nc_launch_latent_attention(int dtype, const NcLatentGeom& g, const void* q_l
 // Attention over keys and values expanded per head: kv T [B][keys][heads * (dim_p + vdim_p)], rotated key parts from the cache.
 bool nc_latent_expanded_ok(int dtype, const NcLatentGeom& g);
 int nc_launch_latent_expanded(const NcLatentGeom& g, const bf16_t* q, int ldq, const bf16_t* kv, int keys, const bf16_t* cache,
-                              const int32_t* seqlens, bf16_t* out, int ldo, const NcAhead* ahead, hipStream_t s);
+                              const int32_t* seqlens, bf16_t* out, int ldo, const NcBehind* ahead, hipStream_t s);
 
 // ---------------------------------------------------------------- retention (nc_retention.hip)
 struct NcRetentionGeom {
@@ -195,10 +195,10 @@ struct NcRetentionGeom {
 size_t nc_retention_workspace_bytes(int dtype, const NcRetentionGeom& g);
 int nc_launch_retention(int dtype, const NcRetentionGeom& g, const void* proj, int ldp, const float* decay, const float* rope, int rope_len,
                         const int32_t* seqlens, const float* state_in, float* state_out, float eps, void* out, int ldo, void* workspace,
-                        const NcAhead* ahead, hipStream_t s);
+                        const NcBehind* ahead, hipStream_t s);
 // out = rms_norm(raw row, over `count` values of its `cols`) * w * sigmoid(gate) * scale
 int nc_launch_joint_gate(int dtype, const float* raw, int cols, int count, const void* gate, int ldg, const float* w, float eps, float scale, void* out,
-                         int ldo, int M, hipStream_t s);
+                         int ldo, int M, hipStream_t s, const int32_t* rows = nullptr);
 
 // ---------------------------------------------------------------- window attention (nc_window_attention.hip)
 struct NcWindowGeom {
@@ -212,7 +212,7 @@ int nc_launch_window_append(int dtype, const NcWindowGeom& g, void* proj, int ld
                             const float* rope, int rope_len, const int32_t* seqlens, void* cache, hipStream_t s);
 size_t nc_window_partial_bytes(int dtype, const NcWindowGeom& g);
 int nc_launch_window_attention(int dtype, const NcWindowGeom& g, const void* q, int ldq, const void* cache, const float* sink, const int32_t* seqlens, void* out,
-                               int ldo, void* partials, size_t partial_bytes, const NcAhead* ahead, hipStream_t s);
+                               int ldo, void* partials, size_t partial_bytes, const NcBehind* ahead, hipStream_t s);
 
 // ---------------------------------------------------------------- selective scan (nc_selective_scan.hip)
 struct NcScanGeom {
@@ -247,4 +247,4 @@ int nc_launch_scan_step(int dtype, const NcScanGeom& g, const NcScanStep& p, hip
 size_t nc_scan_workspace_bytes(const NcScanGeom& g);
 int nc_launch_scan(int dtype, const NcScanGeom& g, const void* u, const float* dt, const float* bc, const float* a_log2, const float* skip,
                    const void* z, int ldz, const int32_t* seqlens, const float* state_in, float* state_out, void* out, int ldo, void* workspace,
-                   const NcAhead* ahead, hipStream_t s);
+                   const NcBehind* ahead, hipStream_t s);

@@ -95,6 +95,9 @@ bool goes_on_alone(const nc_stack_layer& l, int Wp, int M, int n_logits) {
 bool in_two_products(int dtype, const nc_stack_layer& l, int Wp, int M, int n_logits) {
     return (double)(M - n_logits) * (l.n_in - l.mix_cols) * Wp >= (dtype ? 4e8 : 4e9);
 }
+// Up to so many chosen rows the last mixers leave out tiles of tokens without one (us, all tiles / the chosen one, 1792 tokens of 32 heads: window attention 77 / 42, read-out of the
+// chunked recurrence 37 / 17).  Attention over expanded keys does not: it lasts as long as its last tile (70 / 67), beside which the weights behind it are read.
+constexpr int CHOSEN_TILES = 64;
 size_t max_of(size_t a, size_t b) { return a > b ? a : b; }
 
 Workspace carve(const nc_stack_model* m, int B, int T, int n_logits, int max_keys, void* base) {
@@ -207,7 +210,7 @@ void* at(void* p, int64_t elems, int dtype) { return (uint8_t*)p + elems * (dtyp
 // A mixer reads its columns of the projected rows (`proj`, leading dimension ldp) and writes its columns of what the output matrix multiplies
 // (`cat`, leading dimension ld_cat).
 int run_latent_attention(int dt, const nc_stack_mixer& l, const NcLatentGeom& g, const Workspace& w, void* proj, int ldp, float eps, int rope_len,
-                         const int32_t* seqlens, void* cache, void* cat, int ld_cat, const NcAhead* ahead, hipStream_t s) {
+                         const int32_t* seqlens, void* cache, void* cat, int ld_cat, const NcBehind* ahead, hipStream_t s) {
     const int M = g.B * g.T, qd = l.dim_p + l.rot_p, rw = l.rank_p + l.rot_p, head_w = l.dim_p + l.vdim_p;
     const bool ex = expand(dt, l, g);
     TRY(nc_launch_latent_append(dt, g, proj, ldp, l.kv_norm_w, eps, l.rope, rope_len, seqlens, cache, ex ? nullptr : w.q_lat, s));
@@ -233,21 +236,23 @@ int run_latent_attention(int dt, const nc_stack_mixer& l, const NcLatentGeom& g,
 }
 
 int run_window_attention(int dt, const nc_stack_mixer& l, const NcWindowGeom& g, const Workspace& w, void* proj, int ldp, float eps, int rope_len,
-                         const int32_t* seqlens, void* cache, void* cat, int ld_cat, const NcAhead* ahead, hipStream_t s) {
+                         const int32_t* seqlens, void* cache, void* cat, int ld_cat, const NcBehind* ahead, hipStream_t s) {
     TRY(nc_launch_window_append(dt, g, proj, ldp, l.qkv_bias, l.q_norm_w, l.k_norm_w, eps, l.rope, rope_len, seqlens, cache, s));
     return nc_launch_window_attention(dt, g, proj, ldp, cache, l.sink, seqlens, cat, ld_cat, w.att_parts, w.att_part_bytes, ahead, s);
 }
 
 int run_retention(int dt, const nc_stack_mixer& l, const NcRetentionGeom& g, const Workspace& w, const void* proj, int ldp, float eps, int rope_len,
-                  const int32_t* seqlens, const float* state_in, float* state_out, void* cat, int ld_cat, const NcAhead* ahead, hipStream_t s) {
+                  const int32_t* seqlens, const float* state_in, float* state_out, void* cat, int ld_cat, const NcBehind* ahead, hipStream_t s) {
     TRY(nc_launch_retention(dt, g, proj, ldp, l.decay, l.rope, rope_len, seqlens, state_in, state_out, eps, cat, ld_cat, w.ret, ahead, s));
     if (!g.raw) return 0;
     const void* gate = at(proj, (int64_t)l.heads * (2 * l.dim_p + l.vdim_p), dt);
-    return nc_launch_joint_gate(dt, g.raw, l.heads * l.vdim_p, l.heads * l.vdim, gate, ldp, l.out_norm_w, eps, l.out_scale, cat, ld_cat, g.B * g.T, s);
+    const bool some = ahead && ahead->n_chosen > 0;
+    return nc_launch_joint_gate(dt, g.raw, l.heads * l.vdim_p, l.heads * l.vdim, gate, ldp, l.out_norm_w, eps, l.out_scale, cat, ld_cat, some ? ahead->n_chosen : g.B * g.T, s,
+                                some ? ahead->chosen : nullptr);
 }
 
 int run_selective_scan(int dt, const nc_stack_mixer& l, const NcScanGeom& g, const Workspace& w, const void* proj, int ldp, const int32_t* seqlens,
-                       const float* state_in, float* state_out, void* cat, int ld_cat, const NcAhead* ahead, hipStream_t s) {
+                       const float* state_in, float* state_out, void* cat, int ld_cat, const NcBehind* ahead, hipStream_t s) {
     const int M = g.B * g.T, N = scan_x_cols(l), splits = scan_x_splits(dt, l, M);
     TRY(nc_launch_scan_conv(dt, g, proj, ldp, l.conv_w, l.conv_b, seqlens, state_in, state_out, w.u, s));
     NcLinear x = nc_linear(w.u, l.inner_p, l.w_x, M, N, l.inner_p);
@@ -266,14 +271,16 @@ int run_selective_scan(int dt, const nc_stack_mixer& l, const NcScanGeom& g, con
 }
 
 // The mixers of one layer run, on the projected rows w.proj, into w.cat.
-int run_mixers(const nc_stack_model* m, const nc_stack_cache* kv, const nc_stack_run& run, const Workspace& w, int B, int T, const NcAhead& weights, hipStream_t s) {
+int run_mixers(const nc_stack_model* m, const nc_stack_cache* kv, const nc_stack_run& run, const Workspace& w, int B, int T, const NcBehind& weights, hipStream_t s) {
     const nc_stack_layer& l = m->layers[run.layer];
     const int dt = m->dtype;
     int col = 0, to = 0;
     for (int j = 0; j < l.n_mixers; j++) {
         const nc_stack_mixer& x = l.mix[j];
         const int slot = run.slot[j];
-        const NcAhead* const ahead = j + 1 == l.n_mixers ? &weights : nullptr;
+        NcBehind own = weights;
+        if (j + 1 < l.n_mixers) own.n = 0;              // (nothing to read ahead)
+        const NcBehind* const ahead = &own;
         void *proj = at(w.proj, col, dt), *cat = at(w.cat, to, dt);
         switch (x.kind) {
             case NC_MIXER_LATENT_ATTENTION:
@@ -304,8 +311,8 @@ int run_mixers(const nc_stack_model* m, const nc_stack_cache* kv, const nc_stack
 // 2048, 300 tokens 572 / 572 / 572 / 518, 500 621 / 622 / 573 / 573, 800 850 / 783 / 784 / 838, 1400 1053 / 1063 / 1114 / 1118, of width 3072, 800 tokens 1294 / 1293 / 1295 / 1224,
 // with experts, width 2048, 500 tokens 889 / 885 / 874 / 871, 1000 1127 / 1109 / 1104 / 1103.  No prompt of these is slower than without reading.
 constexpr size_t AHEAD_BYTES_PER_ROW = 98304;
-NcAhead weights_behind(const nc_stack_model* m, int i, int M) {
-    NcAhead a{};
+NcBehind weights_behind(const nc_stack_model* m, int i, int M) {
+    NcBehind a{};
     if (m->dtype || M <= NC_FEW_ROWS) return a;
     const nc_stack_layer& l = m->layers[m->runs[i].layer];
     const size_t W = m->width_p;
@@ -485,7 +492,9 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
         mixer_segs(l, in, w, dt);
         if (!post && !mixers_only) rest_segs(in, l.mix_cols, w);
         TRY(nc_launch_linear(dt, in, s));
-        TRY(run_mixers(m, kv, run, w, B, T, ends ? NcAhead{} : weights_behind(m, i, M), s));
+        NcBehind behind = ends ? NcBehind{} : weights_behind(m, i, M);
+        if (alone && n_logits <= CHOSEN_TILES) behind.chosen = logit_rows, behind.n_chosen = n_logits;
+        TRY(run_mixers(m, kv, run, w, B, T, behind, s));
         if (ends) return 0;
         Workspace r = w;
         const int R = alone ? n_logits : M;

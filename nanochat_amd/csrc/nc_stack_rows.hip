@@ -301,12 +301,12 @@ __global__ __launch_bounds__(1024) void route_sort_kernel(NcRoute r, int M) {
 }
 
 // ------------------------------------------------------------------------------------------------ joint norm and gate
-// One workgroup per row; the row passes twice, the second time out of the cache.
+// One workgroup per row (per chosen one, if there are any); the row passes twice, the second time out of the cache.
 template <typename T>
 __global__ __launch_bounds__(256) void joint_gate_kernel(const float* __restrict__ raw, int cols, int count, const T* __restrict__ gate, int ldg,
-                                                         const float* __restrict__ w, float eps, float scale, T* __restrict__ out, int ldo) {
+                                                         const float* __restrict__ w, float eps, float scale, T* __restrict__ out, int ldo, const int32_t* __restrict__ rows) {
     __shared__ float red[4];
-    const int64_t m = blockIdx.x;
+    const int64_t m = rows ? rows[blockIdx.x] : (int)blockIdx.x;
     const float* o = raw + m * cols;
     float sq = 0.f;
     for (int c = 4 * threadIdx.x; c < cols; c += 1024) {
@@ -421,13 +421,13 @@ int nc_launch_stack_select(const NcSelect (&parts)[4], const int32_t* rows, int 
 }
 
 int nc_launch_joint_gate(int dtype, const float* raw, int cols, int count, const void* gate, int ldg, const float* w, float eps, float scale, void* out,
-                         int ldo, int M, hipStream_t s) {
+                         int ldo, int M, hipStream_t s, const int32_t* rows) {
     NC_CHECK_ARG(raw && gate && w && out && cols % 4 == 0 && count > 0 && count <= cols && ldg % 4 == 0 && ldo % 4 == 0, "joint_gate: %d of %d columns", count, cols);
     NcProfScope prof(NC_CLS_ROWS, (double)M * cols * (dtype ? 12 : 8), s);
     if (dtype)
-        hipLaunchKernelGGL((joint_gate_kernel<float>), dim3(M), dim3(256), 0, s, raw, cols, count, (const float*)gate, ldg, w, eps, scale, (float*)out, ldo);
+        hipLaunchKernelGGL((joint_gate_kernel<float>), dim3(M), dim3(256), 0, s, raw, cols, count, (const float*)gate, ldg, w, eps, scale, (float*)out, ldo, rows);
     else
-        hipLaunchKernelGGL((joint_gate_kernel<bf16_t>), dim3(M), dim3(256), 0, s, raw, cols, count, (const bf16_t*)gate, ldg, w, eps, scale, (bf16_t*)out, ldo);
+        hipLaunchKernelGGL((joint_gate_kernel<bf16_t>), dim3(M), dim3(256), 0, s, raw, cols, count, (const bf16_t*)gate, ldg, w, eps, scale, (bf16_t*)out, ldo, rows);
     NC_CHECK_LAUNCH("joint_gate");
     return 0;
 }

@@ -462,6 +462,7 @@ __global__ __launch_bounds__(64 * NQ * KS) __attribute__((amdgpu_waves_per_eu(2,
         h = unit / nx;
         qb0 = unit % nx * QT;
     }
+    if (none_chosen(ahead, (int64_t)b * g.T + qb0, (int64_t)b * g.T + min(qb0 + QT, g.T))) return;
     const int kvh = h / (g.heads / g.kv_heads), head_w = g.dim_p + g.vdim_p, rw = g.kv_heads * head_w;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, hl = lane >> 5;
@@ -655,13 +656,13 @@ int launch_few(const NcWindowGeom& g, const bf16_t* q, int ldq, const bf16_t* ca
 }
 template <int DQ, int DV>
 int launch_prefill(const NcWindowGeom& g, const bf16_t* q, int ldq, const bf16_t* cache, const float* sink, const int32_t* seqlens, bf16_t* out, int ldo,
-                   const NcAhead* ahead, hipStream_t s) {
+                   const NcBehind* ahead, hipStream_t s) {
     if ((int64_t)((g.T + 127) / 128) * g.heads * g.B >= 2 * nc_cu_count())
-        nc_launch_ahead(dim3((g.T + 127) / 128, g.heads, g.B), ahead, [&](dim3 grid, auto a) {
+        nc_launch_behind(dim3((g.T + 127) / 128, g.heads, g.B), ahead, [&](dim3 grid, auto a) {
             hipLaunchKernelGGL((window_prefill_kernel<DQ, DV, 4, 1, decltype(a)>), grid, dim3(256), 0, s, g, q, ldq, cache, sink, seqlens, out, ldo, a);
         });
     else
-        nc_launch_ahead(dim3((g.T + 63) / 64, g.heads, g.B), ahead, [&](dim3 grid, auto a) {
+        nc_launch_behind(dim3((g.T + 63) / 64, g.heads, g.B), ahead, [&](dim3 grid, auto a) {
             hipLaunchKernelGGL((window_prefill_kernel<DQ, DV, 2, 2, decltype(a)>), grid, dim3(256), 0, s, g, q, ldq, cache, sink, seqlens, out, ldo, a);
         });
     NC_CHECK_LAUNCH("window_prefill");
@@ -692,7 +693,7 @@ size_t nc_window_partial_bytes(int dtype, const NcWindowGeom& g) {
 }
 
 int nc_launch_window_attention(int dtype, const NcWindowGeom& g, const void* q, int ldq, const void* cache, const float* sink, const int32_t* seqlens, void* out,
-                               int ldo, void* partials, size_t partial_bytes, const NcAhead* ahead, hipStream_t s) {
+                               int ldo, void* partials, size_t partial_bytes, const NcBehind* ahead, hipStream_t s) {
     NC_CHECK_ARG(g.kv_heads >= 1 && g.heads % g.kv_heads == 0 && g.window >= 1 && g.keep_first >= 0, "window_attention: %d of %d heads, window %d, first %d",
                  g.kv_heads, g.heads, g.window, g.keep_first);
     NC_CHECK_ARG(g.dim_p % 32 == 0 && g.vdim_p % 16 == 0 && ldq % 8 == 0 && ldo % 4 == 0 && sink && g.pos_max + g.T <= g.Tmax, "window_attention: sizes");

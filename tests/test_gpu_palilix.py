@@ -652,13 +652,16 @@ def test_chosen_places_and_errors():
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("end", ["experts", "experts and shared", "dense", "wide"])
+@pytest.mark.parametrize("end", ["experts", "experts and shared", "dense", "recurrence", "wide"])
 def test_rows_that_go_on_alone(end, dtype):
     """Behind the last mixers only the rows with logits go on, from two other rows (experts) or 256 (dense, width 192) on, and of many columns times rows the input matrix is two products
-    then: the same logits as where all rows go on, cache and states as well, for places in any order, more than once, and for none.  (Other kernels: a rounding of one layer.)"""
+    then; the recurrence's read-out leaves out chunks without one.  The same logits as where all rows go on, cache and states as well, for places in any order, more than
+    once, and for none.  (Other kernels: a rounding of one layer.)"""
     say(f"chosen rows, {end}, {dtype}")
-    last = {"experts": moe(experts=20, top=3, ff=64), "experts and shared": moe(experts=20, top=3, ff=64, shared=(192, 0.5)), "dense": dense(ff=320), "wide": dense(ff=4096)}[end]
-    cfg = config([(retention(heads=1, dim=64, vdim=64, rot_dims=32), dense(ff=64)), (latent(), last)], width=1024 if end == "wide" else 192, vocab=70)
+    last = {"experts": moe(experts=20, top=3, ff=64), "experts and shared": moe(experts=20, top=3, ff=64, shared=(192, 0.5)), "dense": dense(ff=320), "recurrence": dense(ff=320),
+            "wide": dense(ff=4096)}[end]
+    first, mixer = retention(heads=1, dim=64, vdim=64, rot_dims=32), retention(heads=2, dim=64, vdim=64, rot_dims=32) if end == "recurrence" else latent()
+    cfg = config([(first, dense(ff=64)), (mixer, last)], width=1024 if end == "wide" else 192, vocab=70)
     model = build(cfg, weights(cfg, seed=5), dtype)
     for B, T in ((1, 2), (1, 3), (1, 18), (1, 65), (3, 70), (1, 256), (1, 257), (2, 200)) if end != "wide" else ((1, 120), (2, 540)):
         toks = torch.tensor([tokens(cfg, T, seed=b + 1) for b in range(B)], device=DEV)
