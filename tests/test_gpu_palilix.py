@@ -663,7 +663,7 @@ def test_rows_that_go_on_alone(end, dtype):
     first, mixer = retention(heads=1, dim=64, vdim=64, rot_dims=32), retention(heads=2, dim=64, vdim=64, rot_dims=32) if end == "recurrence" else latent()
     cfg = config([(first, dense(ff=64)), (mixer, last)], width=1024 if end == "wide" else 192, vocab=70)
     model = build(cfg, weights(cfg, seed=5), dtype)
-    for B, T in ((1, 2), (1, 3), (1, 18), (1, 65), (3, 70), (1, 256), (1, 257), (2, 200)) if end != "wide" else ((1, 120), (2, 540)):
+    for B, T in ((1, 2), (1, 3), (20, 1), (1, 18), (1, 65), (3, 70), (1, 256), (1, 257), (2, 200)) if end != "wide" else ((1, 120), (2, 540)):
         toks = torch.tensor([tokens(cfg, T, seed=b + 1) for b in range(B)], device=DEV)
         full, some, none = (model.new_cache(B, T + 1) for _ in range(3))
         every = model.forward(toks, kv_cache=full).view(B * T, -1)

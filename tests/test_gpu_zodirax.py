@@ -173,7 +173,7 @@ def test_rows_that_go_on_alone(end, dtype):
     say(f"chosen rows, {end}, {dtype}")
     cfg = config([(mamba(), dense()), {"pair": (pair(), dense(ff=320)), "pair alone": (pair(), None), "scan": (mamba(inner=200), dense(ff=80))}[end]], vocab=70)
     model = build_model(Zodirax, cfg, weights(cfg, seed=5), dtype)
-    for B, T in ((3, 70), (1, 384), (1, 385), (2, 300)):
+    for B, T in ((400, 1), (3, 70), (1, 384), (1, 385), (2, 300)):
         toks = torch.tensor([tokens(cfg, T, seed=b + 1) for b in range(B)], device=DEV)
         full, some, none = (model.new_cache(B, T + 1) for _ in range(3))
         every = model.forward(toks, kv_cache=full).view(B * T, -1)
