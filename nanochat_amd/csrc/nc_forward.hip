@@ -200,12 +200,28 @@ int most_visible_keys(const nc_model_desc* m, int Tmax) {
     return most;
 }
 
-// Whether a step goes through nc_step.hip.  Launches of their own have what one has not: times of each kernel (the profiler), rows of any alignment, and a
-// prompt that is read once for all rows.
+// Whether a step goes through nc_step.hip.  Launches of their own have what one has not: times of each kernel (the profiler), rows of any alignment, a
+// prompt that is read once for all rows, and a model without the subtraction at its end.
 bool takes_step(const nc_model_desc* m, const nc_cache_desc* kv, int B) {
     const uintptr_t pointers = (uintptr_t)m->wte | (uintptr_t)kv->prev_in | (uintptr_t)kv->prev_out | (uintptr_t)kv->k_cache | (uintptr_t)kv->v_cache;
-    return nc_step_fits(B, m->n_layer, m->n_embd, m->n_head, m->n_kv_head) && !nc_prof_on() && (pointers & 15) == 0 && kv->max_seq_len < NC_STEP_MAX_KEYS &&
-           !(kv->shared_prefix > 0 && B * m->n_kv_head >= NC_SHARED_MIN_ROW_HEADS);
+    return nc_step_fits(B, m->n_layer, m->n_embd, m->n_head, m->n_kv_head) && !nc_prof_on() && (pointers & 15) == 0 && m->backout_lambda &&
+           kv->max_seq_len < NC_STEP_MAX_KEYS && !(kv->shared_prefix > 0 && B * m->n_kv_head >= NC_SHARED_MIN_ROW_HEADS);
+}
+
+// One launch reads what all layers point at: what the separate launches refuse, each where it comes to it, is refused in front of it.
+int check_step(const nc_model_desc* m, const nc_cache_desc* kv) {
+    NC_CHECK_ARG(m->layers && m->resid_lambdas && m->x0_lambdas, "gpt_forward: layers or their lambdas missing");
+    NC_CHECK_ARG(m->cos && m->sin && m->rope_len > 0, "gpt_forward: rotary source missing");
+    NC_CHECK_ARG(kv->max_seq_len > 0, "gpt_forward: a cache of %d tokens", kv->max_seq_len);
+    for (int i = 0; i < m->n_layer; i++) {
+        const nc_layer_desc& ly = m->layers[i];
+        NC_CHECK_ARG(ly.w_qkv && ly.inv_qkv && ly.w_attn_proj && ly.w_fc && ly.w_mlp_proj, "gpt_forward: layer %d has no FP8 weights", i);
+        NC_CHECK_ARG(ly.inv_attn_proj && ly.inv_fc && ly.inv_mlp_proj, "gpt_forward: layer %d has no weight scales", i);
+        NC_CHECK_ARG((((uintptr_t)ly.w_qkv | (uintptr_t)ly.w_attn_proj | (uintptr_t)ly.w_fc | (uintptr_t)ly.w_mlp_proj) & 15) == 0,
+                     "gpt_forward: layer %d: weights must be 16-byte aligned", i);
+        NC_CHECK_ARG(!ly.ve_table || ly.ve_gate_w, "gpt_forward: layer %d: value embedding needs gate weights", i);
+    }
+    return 0;
 }
 
 NcGemmSegs one_seg(int n) { return NcGemmSegs{1, {n, 0, 0, 0}}; }
@@ -321,6 +337,7 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
 
     // a step of few rows: embedding, one launch for all layers, lm_head
     if (T == 1 && !tap_x && !tap_y && takes_step(m, kv, B)) {
+        TRY(check_step(m, kv));
         NcStepArgs a{};
         a.x0 = w.x0, a.xb = w.xb, a.xn = w.xn, a.exchange = w.step_exchange, a.words = w.step_words, a.head_site = w.step_site();
         a.k_cache = kv->k_cache, a.v_cache = kv->v_cache, a.cache_seqlens = (int32_t*)kv->cache_seqlens, a.idx = idx, a.cos_t = m->cos, a.sin_t = m->sin;
@@ -330,7 +347,6 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
         NcStepLayers layers{};
         for (int i = 0; i < L; i++) {
             const nc_layer_desc& ly = m->layers[i];
-            NC_CHECK_ARG(ly.w_qkv && ly.inv_qkv && ly.w_attn_proj && ly.w_fc && ly.w_mlp_proj, "gpt_forward: layer %d has no FP8 weights", i);
             layers.layer[i] = NcStepLayer{ly.w_qkv, ly.inv_qkv, ly.w_attn_proj, ly.inv_attn_proj, ly.w_fc, ly.inv_fc, ly.w_mlp_proj, ly.inv_mlp_proj,
                                           ly.ve_table, ly.ve_gate_w, ly.window_left, 0};
         }

@@ -4,6 +4,9 @@ import os
 import re
 from concurrent.futures import ThreadPoolExecutor
 
+import pytest
+import torch
+
 from nanochat_amd import _lib
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -125,3 +128,47 @@ def test_a_launch_that_meets_has_a_word_for_every_workgroup():
     lib = _lib.lib()
     assert lib.nc_fp8_meeting_bytes() == 4 * (256 + 256 // 32)
     assert [lib.nc_fp8_gemm_relu2_e4m3_fits(M, 4096, 512) for M in (4096, 4097)] == [1, 0]
+
+
+def _step_descriptors():
+    """A step of one row, three layers of width 256, complete and nowhere in memory: its host checks look at no device."""
+    at = 1 << 20
+    layers = (_lib.LayerDesc * 3)()
+    for ly in layers:
+        for name, kind in _lib.LayerDesc._fields_:
+            setattr(ly, name, -1 if name == "window_left" else 0 if name == "reserved" else at)
+    model = _lib.ModelDesc(n_layer=3, n_head=2, n_kv_head=2, n_embd=256, vocab_size=512, padded_vocab=512, rope_len=64, softcap=15.0)
+    for name, kind in _lib.ModelDesc._fields_:
+        if kind is ctypes.c_void_p:
+            setattr(model, name, at)
+    model.layers = ctypes.cast(layers, type(model.layers))
+    cache = _lib.CacheDesc(k_cache=at, v_cache=at, cache_seqlens=at, prev_out=at, batch=1, max_seq_len=64)
+    return model, layers, cache
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="descriptors of no memory: a check that is missing would reach a launch")
+@pytest.mark.parametrize("what, field, value, message", [
+    ("layer", "w_qkv", None, b"no FP8 weights"), ("layer", "inv_attn_proj", None, b"no weight scales"), ("layer", "inv_fc", None, b"no weight scales"),
+    ("layer", "inv_mlp_proj", None, b"no weight scales"), ("layer", "ve_gate_w", None, b"gate weights"),
+    *[("layer", w, (1 << 20) + 8, b"16-byte aligned") for w in ("w_qkv", "w_attn_proj", "w_fc", "w_mlp_proj")],
+    ("model", "cos", None, b"rotary"), ("model", "sin", None, b"rotary"), ("model", "rope_len", 0, b"rotary"), ("model", "resid_lambdas", None, b"lambdas"),
+    ("model", "x0_lambdas", None, b"lambdas"), ("cache", "max_seq_len", 0, b"cache of 0 tokens")])
+def test_a_step_in_one_launch_refuses_what_the_separate_launches_refuse(what, field, value, message):
+    """The last layer's pointers, the tables and the cache's length are looked at before anything is launched."""
+    lib = _lib.lib()
+    model, layers, cache = _step_descriptors()
+    room = lib.nc_gpt_workspace_bytes(ctypes.byref(model), 1, 1)
+    setattr({"layer": layers[2], "model": model, "cache": cache}[what], field, value)
+    assert lib.nc_gpt_forward(ctypes.byref(model), ctypes.byref(cache), 1 << 20, 1, 1, 1 << 20, 1, 1 << 20, room, None) == -1
+    assert message in lib.nc_last_error()
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="descriptors of no memory")
+def test_a_model_without_backout_takes_the_separate_launches():
+    """They leave the subtraction out; the one launch reads its factor."""
+    lib = _lib.lib()
+    model, _, cache = _step_descriptors()
+    model.backout_lambda = None
+    room = lib.nc_gpt_workspace_bytes(ctypes.byref(model), 1, 1)
+    assert lib.nc_gpt_forward_present(ctypes.byref(model), ctypes.byref(cache), 1 << 20, 1, 1 << 20, 1 << 20, room, 1, None) == -1
+    assert b"not a step that one launch takes" in lib.nc_last_error()
