@@ -347,6 +347,9 @@ int nc_gpt_forward(const nc_model_desc* model /*host*/, const nc_cache_desc* cac
 int nc_gpt_forward_present(const nc_model_desc* model /*host*/, const nc_cache_desc* cache /*host*/, const int64_t* idx, int B,
                            float* logits_out, void* workspace, size_t workspace_bytes, int present, nc_stream_t stream);
 
+/* After how many looks (half a microsecond or more each) such a forward begins with `registered` workgroups, where the others find no place; 0: not one of those (host only). */
+int nc_gpt_step_list_polls(const nc_model_desc* model /*host*/, int B, int registered);
+
 /* The same forward with its intermediate activations copied out, for layer-by-layer comparison with another implementation
  * (no counterpart in the reference; tests only).  tap_x (or NULL): bf16 [n_layer+1, B*T, E]; slot i is the residual stream as
  * layer i reads it, i.e. after `x = resid_lambdas[i]*x + x0_lambdas[i]*x0` (nanochat/gpt.py:500), slot n_layer the final

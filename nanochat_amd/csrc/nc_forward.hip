@@ -553,6 +553,14 @@ extern "C" int nc_gpt_forward(const nc_model_desc* m, const nc_cache_desc* kv, c
     return gpt_forward_impl(m, kv, idx, B, T, logits_out, last_only, workspace, workspace_bytes, nullptr, nullptr, (hipStream_t)stream);
 }
 
+extern "C" int nc_gpt_step_list_polls(const nc_model_desc* m, int B, int registered) {
+    if (!m || !nc_step_fits(B, m->n_layer, m->n_embd, m->n_head, m->n_kv_head)) return 0;
+    NcStepArgs a{};
+    a.B = B, a.L = m->n_layer, a.E = m->n_embd, a.H = m->n_head, a.Hkv = m->n_kv_head;
+    (void)nc_step_exchange(a, 1);
+    return (int)nc_step_list_polls(a, registered);
+}
+
 extern "C" int nc_gpt_forward_present(const nc_model_desc* m, const nc_cache_desc* kv, const int64_t* idx, int B, float* logits_out, void* workspace,
                                       size_t workspace_bytes, int present, nc_stream_t stream) {
     NC_CHECK_ARG(present > 0, "gpt_forward_present: no workgroups");

@@ -202,8 +202,9 @@ struct NcStepArgs {                       // (by value, with the layers behind i
     const float *resid_lambdas, *x0_lambdas, *backout_lambda;
     size_t layer_elems;                   // of the caches
     int B, L, E, H, Hkv, Tmax, rope_len, vocab_rows, advance;
-    // set by nc_step_exchange: workgroups, a layer's part of `exchange` and what lies where in it (q|k|v at its start), and behind the layers the parts of rows whose keys several workgroups share
+    // set by nc_step_exchange: workgroups, how long one waits for them (nc_step_list_polls), a layer's part of `exchange` and what lies where in it (q|k|v at its start), and behind the layers the parts of rows whose keys several workgroups share
     int wgs, layer_bytes, off_y, off_proj, off_h, off_mlp, parts_bytes;
+    uint32_t round_polls;
     uint8_t* parts;
 };
 struct NcStepLayers {
@@ -212,6 +213,8 @@ struct NcStepLayers {
 static_assert(sizeof(NcStepArgs) % 8 == 0 && sizeof(NcStepArgs) + sizeof(NcStepLayers) <= 4096, "kernel arguments");
 size_t nc_step_exchange(NcStepArgs& a, int most_keys);   // B, L, E, H, Hkv and exchange are given, and how many keys a row may have; returns the bytes that `exchange` takes
 bool nc_step_fits(int B, int L, int E, int H, int Hkv);
+// polls (half a microsecond or more) after which `registered` of the launch's workgroups begin without the others; behind nc_step_exchange
+uint32_t nc_step_list_polls(const NcStepArgs& a, int registered);
 // present: workgroups that are started (tests: as if the others had found no place), 0: all
 int nc_launch_step(const NcStepArgs& a, const NcStepLayers& layers, int present, hipStream_t s);
 

@@ -23,8 +23,13 @@
 // step with the weights first, 620 with the rows first; bringing them into the L2 by workgroups that do nothing else gained nothing more).
 //
 // Who takes part.  Nothing promises that the chip holds all workgroups at once: another stream's kernels may have their places.  So the workgroups
-// register, and whoever has waited LIST_POLLS for the others closes the list: those on it share the work out among themselves (`team`), the others leave when they start.
+// register, and whoever has waited long enough for the others closes the list: those on it share the work out among themselves (`team`), the others leave when they start.
 // A team of any size gives the same bits, and everything that is waited for behind the registration comes from workgroups that are running.
+// How long: a team of n takes wgs / n rounds of tiles for every product, so what is missed by beginning with few grows as 1 / n, while other streams' kernels end
+// in some 20 to 800 us and leave their places (list_polls).  us a step, 30 us whatever the team / so, beside prompts of 1792 tokens on another stream: depth 20, 8 rows
+// 800 .. 1360 / 605 .. 650 (a quarter of the teams had 32 to 60 workgroups, now none less than 96), depth 26, 8 rows 930 .. 1670 / 930 .. 1060; beside steps of 64 rows
+// 673 .. 735 / 618 .. 644 and 1006 .. 1176 / 965 .. 987; two such steps beside each other 1108 / 1084.  (Teams of so many, us a step of depth 20, 8 rows: 1 44900,
+// 8 6310, 32 1955, 64 1085, 128 730, 256 575.)
 //
 // us a step, separate launches / this: depth 4, one row 107 / 68; depth 10, 3 rows 300 / 171; depth 16, 4 rows of 1000 keys 590 / 344; depth 20, 640 keys, one row
 // 702 / 451, 8 rows 787 / 555; depth 26, 2000 keys, one row 965 / 648, 8 rows 1172 / 885.
@@ -52,9 +57,16 @@ constexpr uint32_t UNWRITTEN = 0xffffffffu;
 constexpr int LINE = 32;
 enum { W_LIST = 0, W_TEAM = LINE, W_LOST = 2 * LINE };
 constexpr uint32_t LIST_CLOSED = 1u << 30;
-// Polls of half a microsecond or more before the list is closed, and before a wait for registered workgroups is given up (they are running: only a workspace
-// that somebody else writes to gets there; the rows become NaN).
-constexpr uint32_t LIST_POLLS = 64, WAIT_POLLS = 1u << 18;
+// Polls of half a microsecond or more before a wait for registered workgroups is given up (they are running: only a workspace that somebody else writes to
+// gets there; the rows become NaN).
+constexpr uint32_t WAIT_POLLS = 1u << 18;
+// ... and before a list of `registered` workgroups of `wgs` is closed: some 30 us, and for every round of tiles behind the second as long as such a round takes
+// (`round_polls`), at most some 8 ms (a bound for kernels that wait for each other's places).
+constexpr uint32_t LIST_POLLS = 64, LIST_POLLS_MOST = 1u << 14;
+__host__ __device__ inline uint32_t list_polls(uint32_t registered, uint32_t wgs, uint32_t round_polls) {
+    const uint32_t n = registered < 1 ? 1 : registered, more = 2 * n >= wgs ? 0 : (wgs - 2 * n + n - 1) / n;      // rounds behind the second
+    return LIST_POLLS + (more * round_polls < LIST_POLLS_MOST ? more * round_polls : LIST_POLLS_MOST);
+}
 
 // Registers that a condition may leave alone are "written" here without an instruction: the compiler would otherwise carry what an earlier layer left in them
 // through the whole loop.
@@ -481,7 +493,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
                     for (;; spin++) {
                         v = __hip_atomic_load(ARG(words) + W_LIST, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                         if (v >= LIST_CLOSED || v == (uint32_t)wgs) break;
-                        if (spin >= LIST_POLLS) {
+                        if (spin >= LIST_POLLS && spin >= list_polls((uint32_t)__builtin_amdgcn_readfirstlane((int)v), (uint32_t)wgs, ARG(round_polls))) {
                             if (lane == 0) v = __hip_atomic_fetch_or(ARG(words) + W_LIST, LIST_CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                             v = (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
                             if (v < LIST_CLOSED && lane == 0) __hip_atomic_store(ARG(words) + W_TEAM, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -959,6 +971,14 @@ bool nc_step_fits(int B, int L, int E, int H, int Hkv) {
     return nc_cu_count() >= step_wgs(E);
 }
 
+// A round of tiles of all of a step's products, in polls: a workgroup takes in some 4 KB of weights between two of them (us for one more round, measured with so many workgroups started:
+// depth 4, one row 4, depth 10, 3 rows 47, depth 20, 8 rows 170, depth 26, 8 rows 270).
+static uint32_t round_polls(const NcStepArgs& a) {
+    return (uint32_t)((int64_t)a.L * a.E * (a.E * 10 + a.Hkv * 256) / a.wgs / 4096);
+}
+
+uint32_t nc_step_list_polls(const NcStepArgs& a, int registered) { return list_polls((uint32_t)registered, (uint32_t)a.wgs, a.round_polls); }
+
 size_t nc_step_exchange(NcStepArgs& a, int most_keys) {
     int at = 0;
     auto take = [&](int bytes) {
@@ -966,7 +986,7 @@ size_t nc_step_exchange(NcStepArgs& a, int most_keys) {
         at += (bytes + 255) & ~255;
         return here;
     };
-    a.wgs = step_wgs(a.E);
+    a.wgs = step_wgs(a.E), a.round_polls = round_polls(a);
     take(a.B * (a.H + 2 * a.Hkv) * 256);
     a.off_y = take(a.B * a.E * 2);
     a.off_proj = take(a.B * a.E * 2);

@@ -172,3 +172,17 @@ def test_a_model_without_backout_takes_the_separate_launches():
     room = lib.nc_gpt_workspace_bytes(ctypes.byref(model), 1, 1)
     assert lib.nc_gpt_forward_present(ctypes.byref(model), ctypes.byref(cache), 1 << 20, 1, 1 << 20, 1 << 20, room, 1, None) == -1
     assert b"not a step that one launch takes" in lib.nc_last_error()
+
+
+def test_how_long_a_step_in_one_launch_waits_for_its_workgroups():
+    """The smaller the team it would begin with, the longer, as a round of tiles more costs by the model's weights; a bound of some 8 ms; not longer for half of them."""
+    def polls(heads, layers, registered, B=1):
+        m = _lib.ModelDesc(n_layer=layers, n_head=heads, n_kv_head=heads, n_embd=128 * heads, vocab_size=512)
+        return _lib.lib().nc_gpt_step_list_polls(ctypes.byref(m), B, registered)
+    for heads, layers, wgs in ((2, 4, 128), (5, 10, 128), (8, 16, 128), (10, 20, 256), (13, 26, 256)):
+        waits = [polls(heads, layers, n) for n in range(1, wgs + 1)]
+        assert waits == sorted(waits, reverse=True) and set(waits[wgs // 2 - 1:]) == {64} and waits[0] <= 64 + (1 << 14)
+        assert waits[wgs // 4 - 1] - 64 == 2 * (waits[wgs // 3] - 64) > 0           # four rounds and three
+    assert polls(13, 26, 32) > 2 * polls(5, 10, 32) > 2 * polls(2, 4, 32)
+    assert polls(13, 26, 8) > 1 << 13 and polls(2, 4, 8) < 256
+    assert polls(13, 26, 8, B=9) == 0
