@@ -347,6 +347,11 @@ int nc_gpt_forward(const nc_model_desc* model /*host*/, const nc_cache_desc* cac
 int nc_gpt_forward_present(const nc_model_desc* model /*host*/, const nc_cache_desc* cache /*host*/, const int64_t* idx, int B,
                            float* logits_out, void* workspace, size_t workspace_bytes, int present, nc_stream_t stream);
 
+/* The same, in which a wait of one workgroup for another is given up after wait_polls looks: what an overwritten workspace would lead to.  Such a forward ends
+ * with logits of NaN; its token's keys and values, and with `advance` the positions, are not to be relied on.  For tests. */
+int nc_gpt_forward_giving_up(const nc_model_desc* model /*host*/, const nc_cache_desc* cache /*host*/, const int64_t* idx, int B,
+                             float* logits_out, void* workspace, size_t workspace_bytes, int present, int wait_polls, nc_stream_t stream);
+
 /* After how many looks (half a microsecond or more each) such a forward begins with `registered` workgroups, where the others find no place; 0: not one of those (host only). */
 int nc_gpt_step_list_polls(const nc_model_desc* model /*host*/, int B, int registered);
 

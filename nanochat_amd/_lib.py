@@ -17,7 +17,7 @@ EXPORTS = [
     "nc_rmsnorm", "nc_embed_norm_smear", "nc_mix_norm", "nc_mix_norm_e4m3", "nc_relu2", "nc_qkv_rope_append", "nc_qkv_linear_rope_append",
     "nc_attention_workspace_bytes", "nc_decode_attention", "nc_kv_cache_prefill", "nc_softcap", "nc_sample",
     "nc_gpt_workspace_bytes", "nc_gpt_reads_ahead", "nc_gpt_forward", "nc_profile_enable", "nc_profile_read", "nc_profile_read_gemm",
-    "nc_decode_attention_append", "nc_qkv_rope_append_attention", "nc_decode_attention_plan", "nc_gpt_forward_tapped", "nc_gpt_forward_present", "nc_gpt_step_list_polls",
+    "nc_decode_attention_append", "nc_qkv_rope_append_attention", "nc_decode_attention_plan", "nc_gpt_forward_tapped", "nc_gpt_forward_present", "nc_gpt_step_list_polls", "nc_gpt_forward_giving_up",
     "nc_decode_attention_static", "nc_decode_attention_static_max_row_heads",
     "nc_fp8_quantize_state_bytes", "nc_fp8_quantize_tensorwise_fused", "nc_fp8_quantize_tensorwise_fused_bounded", "nc_probe_fp8_mfma_ceiling", "nc_probe_hbm_read", "nc_fp8_quantize_tensorwise_transposed", "nc_fp8_quantize_tensorwise_transposed_fused",
     "nc_decode_attention_shared", "nc_decode_attention_shared_workspace_bytes",
@@ -156,6 +156,7 @@ def _bind(lib):
         "nc_gpt_reads_ahead": (i, [C.POINTER(ModelDesc), i, i]),
         "nc_gpt_forward": (i, [C.POINTER(ModelDesc), C.POINTER(CacheDesc), p, i, i, p, i, p, sz, p]),
         "nc_gpt_forward_present": (i, [C.POINTER(ModelDesc), C.POINTER(CacheDesc), p, i, p, p, sz, i, p]),
+        "nc_gpt_forward_giving_up": (i, [C.POINTER(ModelDesc), C.POINTER(CacheDesc), p, i, p, p, sz, i, i, p]),
         "nc_gpt_step_list_polls": (i, [C.POINTER(ModelDesc), i, i]),
         "nc_gpt_forward_tapped": (i, [C.POINTER(ModelDesc), C.POINTER(CacheDesc), p, i, i, p, i, p, sz, p, p, p]),
         "nc_profile_enable": (i, [i]),

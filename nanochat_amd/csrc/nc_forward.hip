@@ -318,7 +318,8 @@ extern "C" int nc_gpt_reads_ahead(const nc_model_desc* model, int B, int T) { re
 // tap_x (or nullptr): bf16 [L+1, M, E], slot i = the residual stream as layer i reads it (after the lambda mix, gpt.py:500), slot L = the
 // final normalised rows (gpt.py:508).  tap_y (or nullptr): bf16 [L, M, H*128], the attention outputs before c_proj (gpt.py:113-124).
 static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, const int64_t* idx, int B, int T, float* logits_out,
-                            int last_only, void* workspace, size_t workspace_bytes, bf16_t* tap_x, bf16_t* tap_y, hipStream_t s, int present = 0) {
+                            int last_only, void* workspace, size_t workspace_bytes, bf16_t* tap_x, bf16_t* tap_y, hipStream_t s, int present = 0,
+                            uint32_t wait_polls = NC_STEP_WAIT_POLLS) {
     NC_CHECK_ARG(m && kv && idx && logits_out && workspace, "gpt_forward: null pointer");
     NC_CHECK_ARG(B > 0 && T > 0, "gpt_forward: bad batch/time B=%d T=%d", B, T);
     NC_CHECK_ARG(m->n_embd == m->n_head * 128, "gpt_forward: head_dim must be 128 (n_embd=%d n_head=%d)", m->n_embd, m->n_head);
@@ -344,6 +345,7 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
         a.resid_lambdas = m->resid_lambdas, a.x0_lambdas = m->x0_lambdas, a.backout_lambda = m->backout_lambda;
         a.layer_elems = layer_elems;
         a.B = B, a.L = L, a.E = E, a.H = H, a.Hkv = Hkv, a.Tmax = kv->max_seq_len, a.rope_len = m->rope_len, a.vocab_rows = m->padded_vocab, a.advance = kv->advance;
+        a.wait_polls = wait_polls;
         NcStepLayers layers{};
         for (int i = 0; i < L; i++) {
             const nc_layer_desc& ly = m->layers[i];
@@ -565,6 +567,12 @@ extern "C" int nc_gpt_forward_present(const nc_model_desc* m, const nc_cache_des
                                       size_t workspace_bytes, int present, nc_stream_t stream) {
     NC_CHECK_ARG(present > 0, "gpt_forward_present: no workgroups");
     return gpt_forward_impl(m, kv, idx, B, 1, logits_out, 1, workspace, workspace_bytes, nullptr, nullptr, (hipStream_t)stream, present);
+}
+
+extern "C" int nc_gpt_forward_giving_up(const nc_model_desc* m, const nc_cache_desc* kv, const int64_t* idx, int B, float* logits_out, void* workspace,
+                                        size_t workspace_bytes, int present, int wait_polls, nc_stream_t stream) {
+    NC_CHECK_ARG(present > 0 && wait_polls > 0, "gpt_forward_giving_up: %d workgroups, %d polls", present, wait_polls);
+    return gpt_forward_impl(m, kv, idx, B, 1, logits_out, 1, workspace, workspace_bytes, nullptr, nullptr, (hipStream_t)stream, present, (uint32_t)wait_polls);
 }
 
 extern "C" int nc_gpt_forward_tapped(const nc_model_desc* m, const nc_cache_desc* kv, const int64_t* idx, int B, int T, float* logits_out,

@@ -175,7 +175,8 @@ int nc_launch_attention_fused(NcRopeSrc rope, bf16_t* k_cache, bf16_t* v_cache, 
 #define NC_STEP_MAX_KEYS (1 << 24)        // of a cache row
 #define NC_STEP_SPLIT_KEYS 128            // of a row's kv head to a workgroup, while there are workgroups
 #define NC_STEP_MAX_SPLITS 12
-#define NC_STEP_WORDS (3 * 32)           // zero before the launch
+#define NC_STEP_WORDS (2 * 32)           // zero before the launch
+#define NC_STEP_WAIT_POLLS (1u << 22)    // two seconds or more
 struct NcStepLayer {
     const uint8_t* w_qkv;
     const float* inv_qkv;
@@ -202,6 +203,7 @@ struct NcStepArgs {                       // (by value, with the layers behind i
     const float *resid_lambdas, *x0_lambdas, *backout_lambda;
     size_t layer_elems;                   // of the caches
     int B, L, E, H, Hkv, Tmax, rope_len, vocab_rows, advance;
+    uint32_t wait_polls;                  // after which a wait for workgroups that are running is given up (NC_STEP_WAIT_POLLS)
     // set by nc_step_exchange: workgroups, how long one waits for them (nc_step_list_polls), a layer's part of `exchange` and what lies where in it (q|k|v at its start), and behind the layers the parts of rows whose keys several workgroups share
     int wgs, layer_bytes, off_y, off_proj, off_h, off_mlp, parts_bytes;
     uint32_t round_polls;

@@ -25,6 +25,8 @@
 // Who takes part.  Nothing promises that the chip holds all workgroups at once: another stream's kernels may have their places.  So the workgroups
 // register, and whoever has waited long enough for the others closes the list: those on it share the work out among themselves (`team`), the others leave when they start.
 // A team of any size gives the same bits, and everything that is waited for behind the registration comes from workgroups that are running.
+// Only a workspace that somebody else writes to could keep one waiting: a wait ends after seconds (NC_STEP_WAIT_POLLS; the longest of a running team, a share of a million keys
+// beside an idle one, is some 50 ms).  Whoever gives up says so in the amax of the last rows, with a NaN that no later one takes away: the logits are NaN.
 // How long: a team of n takes wgs / n rounds of tiles for every product, so what is missed by beginning with few grows as 1 / n, while other streams' kernels end
 // in some 20 to 800 us and leave their places (list_polls).  us a step, 30 us whatever the team / so, beside prompts of 1792 tokens on another stream: depth 20, 8 rows
 // 800 .. 1360 / 605 .. 650 (a quarter of the teams had 32 to 60 workgroups, now none less than 96), depth 26, 8 rows 930 .. 1670 / 930 .. 1060; beside steps of 64 rows
@@ -55,12 +57,9 @@ constexpr uint32_t UNWRITTEN = 0xffffffffu;
 
 // words (NC_STEP_WORDS, zero before the launch), each on a line of its own
 constexpr int LINE = 32;
-enum { W_LIST = 0, W_TEAM = LINE, W_LOST = 2 * LINE };
+enum { W_LIST = 0, W_TEAM = LINE };
 constexpr uint32_t LIST_CLOSED = 1u << 30;
-// Polls of half a microsecond or more before a wait for registered workgroups is given up (they are running: only a workspace that somebody else writes to
-// gets there; the rows become NaN).
-constexpr uint32_t WAIT_POLLS = 1u << 18;
-// ... and before a list of `registered` workgroups of `wgs` is closed: some 30 us, and for every round of tiles behind the second as long as such a round takes
+// Polls of half a microsecond or more before a list of `registered` workgroups of `wgs` is closed: some 30 us, and for every round of tiles behind the second as long as such a round takes
 // (`round_polls`), at most some 8 ms (a bound for kernels that wait for each other's places).
 constexpr uint32_t LIST_POLLS = 64, LIST_POLLS_MOST = 1u << 14;
 __host__ __device__ inline uint32_t list_polls(uint32_t registered, uint32_t wgs, uint32_t round_polls) {
@@ -278,7 +277,6 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
     __shared__ float last_amax[ROW_WAVES];
     __shared__ int pos_of[NC_STEP_ROWS], splits_of[NC_STEP_MAX_LAYERS];
     __shared__ uint32_t said[2];
-    __shared__ int lost;
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kw = wave - ROW_WAVES;
     int tid = threadIdx.x, lane = tid & 63, idx = blockIdx.x;
@@ -291,7 +289,6 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
         const uint32_t* src = device_pointer<const uint32_t>((uint64_t)__builtin_amdgcn_kernarg_segment_ptr());
         const int words = (int)(sizeof(NcStepArgs) / 4) + (int)(sizeof(NcStepLayer) / 4) * ((const NcStepArgs*)(const void*)src)->L;
         for (int i = tid; i < words; i += THREADS) table[i] = src[i];
-        if (tid == 0) lost = 0;
         if (tid < ROW_WAVES) red[tid] = 0;
     }
     __syncthreads();
@@ -325,14 +322,14 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
     __syncthreads();
     if (said[0] >= LIST_CLOSED) return;                            // the others have shared the work out already
 
-    // ---- the others: loads until all of a wave's pieces have been written
+    // ---- the others: loads until all of a wave's pieces have been written, or the wait is given up, and every later one of this workgroup with it
+    auto give_up = [&]() INLINE { table[offsetof(NcStepArgs, wait_polls) / 4] = 0; };
     auto hear = [&](auto&& load_all) INLINE {
         for (uint32_t spin = 0;; spin++) {
             asm volatile("" ::: "memory");                         // (a load of the next round is another load)
             if (__builtin_amdgcn_ballot_w64(load_all()) == 0) break;
-            if (spin >= (lost ? 0u : WAIT_POLLS)) {
-                lost = 1;
-                if (lane == 0) __hip_atomic_store(ARG(words) + W_LOST, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (spin >= ARG(wait_polls)) {
+                give_up();
                 break;
             }
         }
@@ -501,9 +498,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
                         }
                     }
                     if (v >= LIST_CLOSED)                          // whoever closed the list is about to say how long it was
-                        for (spin = 0; spin < WAIT_POLLS; spin++)
+                        for (spin = 0; spin < ARG(wait_polls); spin++)
                             if ((v = __hip_atomic_load(ARG(words) + W_TEAM, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0) break;
-                    if (v - 1u >= (uint32_t)wgs) v = (uint32_t)wgs, lost = 1;       // (not one of a team: somebody else writes here.  Every wait below still ends)
+                    if (v - 1u >= (uint32_t)wgs) v = (uint32_t)wgs, give_up();       // (not one of a team: somebody else writes here.  Every wait below still ends)
                     if (lane == 0) said[1] = v;
                 }
                 __syncthreads();
@@ -928,7 +925,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
         }
     }
     // ---------------------------------------------------------------- the last rows: x += mlp, less the saved rows, norm
-    if (idx != 0) return;
+    const float GAVE_UP = __uint_as_float(0x7fc00000u);
+    if (idx != 0) {
+        if (tid == 0 && ARG(wait_polls) == 0) amax_publish(ARG(head_site), GAVE_UP);
+        return;
+    }
     phase();
     const int B = ARG(B), E = ARG(E);
     const float bl = rbf(*ARG(backout_lambda));
@@ -954,8 +955,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
         float all = last_amax[0];
 #pragma unroll
         for (int w = 1; w < ROW_WAVES; w++) all = amax_join(all, last_amax[w]);
-        if (lost || __hip_atomic_load(ARG(words) + W_LOST, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) all = __uint_as_float(0x7fc00000u);
-        amax_publish(ARG(head_site), all);
+        amax_publish(ARG(head_site), ARG(wait_polls) == 0 ? GAVE_UP : all);
     }
     if (ARG(advance) && tid < B) ARG(cache_seqlens)[tid] = pos_of[tid] + ARG(advance);
 }

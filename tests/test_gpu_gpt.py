@@ -490,15 +490,17 @@ def _step_cache(model, lengths, room, seed=6):
 
 
 class _Present:
-    """The library with forwards of which only so many workgroups are started."""
+    """The library with forwards of which only so many workgroups are started, or whose waits are given up after so many looks."""
 
-    def __init__(self, lib, present):
-        self._lib, self._present = lib, present
+    def __init__(self, lib, present, wait_polls=None):
+        self._lib, self._present, self._wait_polls = lib, present, wait_polls
 
     def __getattr__(self, name):
         return getattr(self._lib, name)
 
     def nc_gpt_forward(self, md, cd, idx, B, T, logits, last_only, ws, ws_bytes, stream):
+        if self._wait_polls is not None:
+            return self._lib.nc_gpt_forward_giving_up(md, cd, idx, B, logits, ws, ws_bytes, self._present, self._wait_polls, stream)
         return self._lib.nc_gpt_forward_present(md, cd, idx, B, logits, ws, ws_bytes, self._present, stream)
 
 
@@ -542,6 +544,28 @@ def test_step_of_few_rows_in_one_launch_against_the_separate_launches(layers, he
     for present in (1, 7, 100):
         for got, want in zip(steps(lambda t, c: model.forward_last(t, kv_cache=c), present), one):
             assert torch.equal(got, want), present
+
+
+@pytest.mark.parametrize("layers, heads, kv_heads, lengths, present", [(3, 2, 2, [70], 128), (3, 4, 2, [300, 5, 0], 100), (4, 13, 13, [600] * 8, 256), (3, 14, 7, [513], 7)])
+def test_a_step_whose_waits_are_given_up_ends_with_nan(layers, heads, kv_heads, lengths, present, monkeypatch):
+    """A workgroup that stops waiting, here after two looks (and, in a team that is not complete, without having heard how large it is), goes on with words that nobody has
+    written.  No logit looks like a number then, every workgroup comes to its end, other tokens' keys stay as they were, and the next step is a step like any other."""
+    say(f"step given up: {layers} layers, {heads} heads on {kv_heads}, rows of {lengths}, {present} workgroups")
+    from nanochat_amd import gpt as gpt_module
+    model = _step_model(layers, heads, kv_heads, sequence_len=512)
+    toks = torch.randint(0, 1024, (len(lengths), 1), generator=torch.Generator(device=DEV).manual_seed(7), device=DEV)
+    want = model.forward_last(toks, kv_cache=_step_cache(model, lengths, 2))
+    real = gpt_module._lib.lib()
+    cache = _step_cache(model, lengths, 2)
+    before = cache.k_cache.clone()
+    with monkeypatch.context() as m:
+        m.setattr(gpt_module._lib, "lib", lambda: _Present(real, present, 1))
+        logits = model.forward_last(toks, kv_cache=cache)
+        torch.cuda.synchronize()
+    assert torch.isnan(logits).all()
+    for b, n in enumerate(lengths):
+        assert torch.equal(cache.k_cache[:, b, :n], before[:, b, :n]) and torch.equal(cache.k_cache[:, b, n + 1:], before[:, b, n + 1:])
+    assert torch.equal(model.forward_last(toks, kv_cache=_step_cache(model, lengths, 2)), want)
 
 
 def test_steps_and_prompts_on_three_streams():
