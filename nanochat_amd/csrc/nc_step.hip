@@ -485,7 +485,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
             const float rl = scales[layer][6], xl = scales[layer][7], i0 = scales[layer][0], i1 = scales[layer][1], i2 = scales[layer][2];
             if (layer == 0) {
                 // who is here
-                if (wave == 0) {
+                int asks = wave;                                   // (its own copy: the comparison would be kept, in memory, through the loop)
+                asm volatile("" : "+s"(asks));
+                if (asks == 0) {
                     uint32_t v = 0, spin = 0;
                     for (;; spin++) {
                         v = __hip_atomic_load(ARG(words) + W_LIST, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -571,7 +573,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
                         if (tok < 0 || tok >= ARG(vocab_rows)) tok = 0;
                         const bf16_t* ve = r.ve_table + ((size_t)tok * Hkv + hk) * 128;
                         raw.e1 = ve[lane], raw.e2 = ve[lane + 64];
-                        raw.xg = gate_in[b][lane < 12 ? lane : 0];
+                        int at_lane = lane;                                            // (its own copy: the address would be kept, in memory, through the loop)
+                        asm volatile("" : "+v"(at_lane));
+                        raw.xg = gate_in[b][at_lane < 12 ? at_lane : 0];
                     }
                     const int qkv_w = (H + 2 * Hkv) * 128;
                     const __amdgpu_buffer_rsrc_t desc_qkv = rows_desc(from_others(layer, 0), B * qkv_w * 2);

@@ -65,6 +65,7 @@ def test_hot_kernels_use_no_scratch_memory():
     # touch them with no instruction
     hot = {"nc_attention.hip": {"attn_partial_kernel": 32},
            "nc_gemm_decode.hip": {"gemm_decode_kernel": 0, "finish_partials_kernel": 0},
+           "nc_step.hip": {"step_kernel": 0},
            "nc_elementwise.hip": {"mix_norm_vec_kernel": 0, "kv_prefill_copy_kernel": 0, "qkv_rope_append_kernel": 0},
            "nc_gemm.hip": {"gemm_dl_kernel": 0, "gemm_dlp_kernel": 64},
            "nc_attention_prefill.hip": {"attn_prefill_kernel": 0},
