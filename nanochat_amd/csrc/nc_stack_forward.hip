@@ -81,13 +81,15 @@ int expert_max_tiles(const nc_stack_layer& l, int M, int tile_rows) {
     return pairs / tile_rows + (pairs < l.experts ? pairs : l.experts);
 }
 // Behind the mixers of the last run every row is by itself, and of a prompt one row a sequence has logits: only the chosen rows take part in the rest of that run, gathered by a
-// launch of their own (3 to 4 us).  Of experts that pays from two rows less on, of other layers by their width (with `in_two_products`; us, all rows / the chosen one: Palilix with experts,
+// launch of their own (3 to 4 us for one).  Of experts that pays from two rows less on, of other layers by their width (with `in_two_products`; us, all rows / the chosen one: Palilix with experts,
 // width 2048, 1792 tokens 3514 / 3238, 100 828 / 709, width 512, 3 tokens 247 / 244, 32-bit, width 1024, 333 tokens 1018 / 910; dense, width 2048, 1000 tokens 831 / 760, width 512, 40 tokens
 // 226 / 229, 65 242 / 242, 256 261 / 259; Zodirax, width 4096, 1792 tokens 4034 / 3603, 2048, 40 tokens 489 / 483, 1024, 40 373 / 369, 512, 128 386 / 384; 32-bit, width 384, 65 tokens
-// 504 / 510).
+// 504 / 510).  Up to half of the rows: more of them cost more to copy than the others would have (us, all rows / the chosen ones, a half, three quarters and nine tenths of them: experts, width 2048,
+// 1792 tokens 1956 / 1919, 2035 / 2035, 2071 / 2093, 400 tokens 1117 / 1098, 1147 / 1144, 1152 / 1164; dense, width 2048, 400 tokens 619 / 619, 645 / 654, 649 / 658; Zodirax, width
+// 2048, 1792 tokens 1820 / 1773, 1895 / 1878, 1929 / 1945; 32-bit, width 512, 333 tokens 652 / 649, 661 / 666, 685 / 687).
 bool goes_on_alone(const nc_stack_layer& l, int Wp, int M, int n_logits) {
     const int64_t others = (int64_t)M - n_logits;
-    return n_logits > 0 && (l.ff == NC_FF_EXPERTS ? others >= 2 : others * Wp >= 48 * 1024);
+    return n_logits > 0 && n_logits <= others && (l.ff == NC_FF_EXPERTS ? others >= 2 : others * Wp >= 48 * 1024);
 }
 // ... and the columns of its input matrix that the mixers do not read become a product of the chosen rows alone, where the products of the others are worth a launch and a second
 // trip for the weight (us, one product / two: dense, width 512, 1000 tokens 353 / 352, 1024, 256 tokens 306 / 306, 1000 462 / 453, 2048, 256 tokens 471 / 463; experts with

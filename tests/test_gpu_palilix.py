@@ -654,7 +654,7 @@ def test_chosen_places_and_errors():
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("end", ["experts", "experts and shared", "dense", "recurrence", "wide"])
 def test_rows_that_go_on_alone(end, dtype):
-    """Behind the last mixers only the rows with logits go on, from two other rows (experts) or 256 (dense, width 192) on, and of many columns times rows the input matrix is two products
+    """Behind the last mixers only the rows with logits go on, up to half of all and from two other rows (experts) or 256 (dense, width 192) on, and of many columns times rows the input matrix is two products
     then; the recurrence's read-out leaves out chunks without one.  The same logits as where all rows go on, cache and states as well, for places in any order, more than
     once, and for none.  (Other kernels: a rounding of one layer.)"""
     say(f"chosen rows, {end}, {dtype}")
@@ -668,7 +668,7 @@ def test_rows_that_go_on_alone(end, dtype):
         full, some, none = (model.new_cache(B, T + 1) for _ in range(3))
         every = model.forward(toks, kv_cache=full).view(B * T, -1)
         places = [(7 * k) % (B * T) for k in range(max(1, B * T - 257))]
-        for chosen in (None, places, [B * T - 1, 0, B * T - 1], list(range(B * T - 1))):
+        for chosen in (None, places, [B * T - 1, 0, B * T - 1], list(range(B * T - 1)), list(range(1, B * T, 2))):
             some.reset()
             got = model.forward_last(toks, kv_cache=some) if chosen is None else model.forward_at(toks, chosen, kv_cache=some)
             check(got, every[[b * T + T - 1 for b in range(B)] if chosen is None else chosen].cpu(), dtype, f"{B} x {T}, {'last' if chosen is None else len(chosen)}")

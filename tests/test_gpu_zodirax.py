@@ -168,7 +168,7 @@ def test_bars_would_show_a_mistake(mistake, monkeypatch):
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("end", ["pair", "pair alone", "scan"])
 def test_rows_that_go_on_alone(end, dtype):
-    """Behind the last mixers only the rows with logits go on, from 384 other rows of 128 columns on: the same logits as where all rows go on, caches and states as well, for places in any
+    """Behind the last mixers only the rows with logits go on, up to half of all and from 384 other rows of 128 columns on: the same logits as where all rows go on, caches and states as well, for places in any
     order, more than once, and for none.  (Other kernels: a rounding of one layer.)"""
     say(f"chosen rows, {end}, {dtype}")
     cfg = config([(mamba(), dense()), {"pair": (pair(), dense(ff=320)), "pair alone": (pair(), None), "scan": (mamba(inner=200), dense(ff=80))}[end]], vocab=70)
@@ -177,7 +177,7 @@ def test_rows_that_go_on_alone(end, dtype):
         toks = torch.tensor([tokens(cfg, T, seed=b + 1) for b in range(B)], device=DEV)
         full, some, none = (model.new_cache(B, T + 1) for _ in range(3))
         every = model.forward(toks, kv_cache=full).view(B * T, -1)
-        for chosen in (None, [(7 * k) % (B * T) for k in range(max(1, B * T - 385))], [B * T - 1, 0, B * T - 1]):
+        for chosen in (None, [(7 * k) % (B * T) for k in range(max(1, B * T - 385))], [B * T - 1, 0, B * T - 1], list(range(1, B * T, 2))):
             some.reset()
             got = model.forward_last(toks, kv_cache=some) if chosen is None else model.forward_at(toks, chosen, kv_cache=some)
             check(got, every[[b * T + T - 1 for b in range(B)] if chosen is None else chosen].cpu(), dtype, f"{B} x {T}, {'last' if chosen is None else len(chosen)}")

@@ -3,6 +3,7 @@ import ctypes
 import json
 import re
 import struct
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -14,7 +15,7 @@ from nanochat_amd.engine import Engine, StackCache
 from nanochat_amd.palilix import Palilix, stack_config
 from nanochat_amd.stack import Experts, LatentAttention, LayerStack, Retention
 from oracle import palilix_ref as ref
-from palilix_cases import CASES, config, latent, moe, retention, tensor_shapes, variant, weights
+from palilix_cases import CASES, config, dense, latent, moe, retention, tensor_shapes, variant, weights
 from stack_helpers import rel_rms, tokens
 
 
@@ -59,6 +60,29 @@ def test_errors_come_before_any_gpu_call():
     lib = _lib.stack_lib()
     assert lib.nc_stack_linear(0, None, 64, None, None, 16, 1, 16, 64, 0, 0.0, 0, None) == -1
     assert lib.nc_stack_cache_copy(None, None, 1, 1, 16, 16, 16, None) == -1 and b"rows" in lib.nc_last_error()
+
+
+def plan(cfg, dtype=torch.float32):
+    """The model's descriptor over weights in host memory, for what the library works out on the host; with it what keeps that memory."""
+    model = meta_model(cfg, dtype).load_tensors(weights(cfg), torch.device("cpu"))
+    model.get_device = lambda: SimpleNamespace(type="cuda")
+    model._build_plan()
+    md, layers = model._plan[:2]
+    md.rope_len = 1024
+    for layer in layers:
+        for mix in layer.mix:
+            mix.rope = md.embed
+    return md, model
+
+
+@pytest.mark.parametrize("last", [moe(experts=20, top=3, ff=64), dense(ff=320)], ids=["experts", "dense"])
+def test_most_rows_chosen_take_no_gather(last):
+    """Rows that go on alone behind the last mixers have memory of their own.  Where more than half of the rows are chosen all go on, and the logits' rows are all that is asked for."""
+    md, _ = plan(config([(latent(), last)], width=192, vocab=70))
+    room = [_lib.stack_lib().nc_stack_workspace_bytes(ctypes.byref(md), 1, 1000, n, 1000) for n in range(1001)]
+    row = 192 * 4
+    assert all(room[n] - room[n - 1] <= row + 256 for n in range(502, 1001)) and room[1000] > room[501]
+    assert room[500] - room[499] > 2 * row and room[500] > room[501]
 
 
 # ------------------------------------------------------------------------------------------------ configuration
