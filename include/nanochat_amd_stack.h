@@ -135,7 +135,8 @@ typedef struct nc_stack_cache {
     int advance;                    /* != 0: the last row kernel adds it to every cache_seqlens entry */
 } nc_stack_cache;
 
-/* Workspace for one forward of T tokens per row, n_logits rows of logits, at most max_keys keys per row. */
+/* Workspace for one forward of T tokens per row, n_logits rows of logits, at most max_keys keys per row.  Up to half of the rows' logits: with room for those rows to go on alone
+ * behind the last mixers, which can be more than the logits of all rows ask for.  A workspace for the logits of more rows is taken all the same; all rows go on then. */
 size_t nc_stack_workspace_bytes(const nc_stack_model* model /*host*/, int B, int T, int n_logits, int max_keys);
 
 /* idx int64 [B,T]; logit_rows int32 [n_logits]: flat indices (row * T + token) whose logits are wanted (device); logits_out fp32

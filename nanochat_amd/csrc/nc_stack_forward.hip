@@ -39,8 +39,9 @@ struct Workspace {
     void *h, *proj, *cat, *h_last, *q_lat, *o_lat, *kv, *att_parts, *ret, *act, *e_out, *u, *dtr;
     float* slot_w;
     int32_t *chosen, *slot_of, *perm, *tiles, *n_tiles;
-    float *sel_x, *sel_router;        // the rows that go on behind the last run's mixers (goes_on_alone)
+    float *sel_x, *sel_router;        // the rows that go on behind the last run's mixers (goes_on_alone), if there is room for them
     void *sel_h, *sel_cat;
+    bool gathers;
     size_t att_part_bytes, part_bytes, total;
 };
 
@@ -102,7 +103,8 @@ bool in_two_products(int dtype, const nc_stack_layer& l, int Wp, int M, int n_lo
 constexpr int CHOSEN_TILES = 64;
 size_t max_of(size_t a, size_t b) { return a > b ? a : b; }
 
-Workspace carve(const nc_stack_model* m, int B, int T, int n_logits, int max_keys, void* base) {
+// gather: with room for the rows that go on alone
+Workspace carve(const nc_stack_model* m, int B, int T, int n_logits, int max_keys, void* base, bool gather = true) {
     const size_t M = (size_t)B * T, Wp = m->width_p, es = m->dtype ? 4 : 2;
     size_t proj = 0, router = 0, parts = 0, qlat = 0, olat = 0, kv = 0, att = 0, ret = 0, act = 0, eout = 0, pairs = 0, tiles = 0, raw = 0, bc = 0, dt = 0, u = 0,
            dtr = 0, x_parts = 0;
@@ -160,7 +162,8 @@ Workspace carve(const nc_stack_model* m, int B, int T, int n_logits, int max_key
     // (a run of a layer that is not there is refused by the forward, which asks here first)
     const int end_of = m->n_runs > 0 ? m->runs[m->n_runs - 1].layer : -1;
     size_t sel = 0, sel_router = 0;
-    if (end_of >= 0 && end_of < m->n_layers && goes_on_alone(m->layers[end_of], (int)Wp, (int)M, n_logits)) {
+    gather = gather && end_of >= 0 && end_of < m->n_layers && goes_on_alone(m->layers[end_of], (int)Wp, (int)M, n_logits);
+    if (gather) {
         const nc_stack_layer& l = m->layers[end_of];
         sel = n_logits, sel_router = sel * l.router_cols * 4;
         parts = max_of(parts, nc_linear_splits(m->dtype, n_logits, (int)Wp, l.k_out) * sel * Wp * 4);
@@ -169,6 +172,7 @@ Workspace carve(const nc_stack_model* m, int B, int T, int n_logits, int max_key
     }
     Carver c(base);
     Workspace w;
+    w.gathers = gather;
     w.x = (float*)c.take(M * Wp * 4);
     w.x0 = (float*)c.take(again ? M * Wp * 4 : 0);
     w.h = c.take(M * Wp * es);
@@ -463,8 +467,10 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
     for (int i = 0; i < m->n_layers; i++) TRY(check_layer(m->layers[i], i));
     const int M = B * T, Wp = m->width_p, dt = m->dtype;
     const int keys = kv->pos_max + T;
-    // the caller sized the workspace for its own bound on the keys; what this call needs is never more than that
-    const Workspace w = carve(m, B, T, n_logits, keys, workspace);
+    // the caller sized the workspace for its own bound on the keys; what this call needs is never more than that.  One that was sized for the logits of more rows, or of all, has room
+    // for these, but not always for their gather: all rows go on then
+    Workspace w = carve(m, B, T, n_logits, keys, workspace, logit_rows && !taps);
+    if (workspace_bytes < w.total) w = carve(m, B, T, n_logits, keys, workspace, false);
     NC_CHECK_ARG(workspace_bytes >= w.total, "stack_forward: workspace of %zu bytes needed, %zu given", w.total, workspace_bytes);
     bool again = false;
     for (int i = 0; i < m->n_runs; i++) {
@@ -483,7 +489,7 @@ extern "C" int nc_stack_forward(const nc_stack_model* m, const nc_stack_cache* k
         const nc_stack_layer& l = m->layers[run.layer];
         const bool post = l.block == NC_BLOCK_POST_NORM;
         // the last run may end early for all rows but the chosen ones (goes_on_alone), or for all
-        const bool last = i + 1 == m->n_runs && !taps, alone = last && logit_rows && goes_on_alone(l, Wp, M, n_logits), ends = last && n_logits == 0;
+        const bool last = i + 1 == m->n_runs && !taps, alone = last && w.gathers, ends = last && n_logits == 0;
         // columns of the input matrix behind the mixers' own: router logits, and the feed-forward's first matrix, which goes to `cat`
         auto rest_segs = [&](NcLinear& g, int col, const Workspace& to) {
             if (l.router_cols) nc_linear_seg(g, col + l.router_cols, NC_SEG_F32, to.router, l.router_cols);

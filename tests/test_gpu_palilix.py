@@ -1,5 +1,6 @@
 """Palilix on the GPU against the plain restatement in oracle/palilix_ref.py (float64): whole prompts, decoding, portions, batches of
 unequal sequences, slots that are used again, generation through the Engine; both storage types."""
+import ctypes
 import functools
 import json
 import math
@@ -677,6 +678,28 @@ def test_rows_that_go_on_alone(end, dtype):
         want = model.forward(step, kv_cache=full)
         for cache in (some, none):
             assert torch.equal(model.forward(step, kv_cache=cache), want), (B, T)
+
+
+def test_chosen_rows_in_a_workspace_for_all_rows(monkeypatch):
+    """Room for the logits of all rows is not always room for a gather of half of them: all rows go on then, and nothing is written behind the workspace."""
+    say("chosen rows, workspace for all rows")
+    cfg = config([(retention(heads=1, dim=64, vdim=64, rot_dims=32), dense(ff=64)), (latent(), moe(experts=20, top=3, ff=64))], width=192, vocab=70)
+    model = build(cfg, weights(cfg, seed=5), torch.bfloat16)
+    toks = torch.tensor([tokens(cfg, 300)], device=DEV)
+    every = model.forward(toks).view(300, -1)
+    guard, lib = [], ops._lib.stack_lib()
+
+    def for_all(md, B, T, n_logits, keys):
+        room = lib.nc_stack_workspace_bytes(ctypes.byref(md), B, T, B * T, keys)
+        assert room < lib.nc_stack_workspace_bytes(ctypes.byref(md), B, T, n_logits, keys)
+        t = torch.full((room + 4096,), 77, dtype=torch.uint8, device=DEV)
+        off = -t.data_ptr() % 256
+        guard.append(t[off + room:])
+        return t.data_ptr() + off, room
+    monkeypatch.setattr(model, "_workspace", for_all)
+    chosen = list(range(1, 300, 2))
+    check(model.forward_at(toks, chosen), every[chosen].cpu(), torch.bfloat16, "half of 300")
+    assert len(guard) == 1 and bool((guard[0] == 77).all())
 
 
 # ------------------------------------------------------------------------------------------------ generation

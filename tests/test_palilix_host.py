@@ -85,6 +85,23 @@ def test_most_rows_chosen_take_no_gather(last):
     assert room[500] - room[499] > 2 * row and room[500] > room[501]
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="weights in host memory: the call is to end where the launches begin")
+@pytest.mark.parametrize("last", [moe(experts=20, top=3, ff=64), dense(ff=320)], ids=["experts", "dense"])
+def test_a_workspace_for_all_rows_takes_any_selection(last):
+    """One for the logits of all 1000 rows is not refused for those of one, of half or of nearly all of them, and no less than for no logits is ever taken."""
+    lib = _lib.stack_lib()
+    md, _ = plan(config([(latent(), last)], width=192, vocab=70))
+    at = md.embed
+    rows = (ctypes.c_void_p * 1)(at)
+    cache = _lib.StackCacheDesc(rows=rows, state_in=rows, state_out=rows, cache_seqlens=at, batch=1, max_seq_len=1000)
+    room = {n: lib.nc_stack_workspace_bytes(ctypes.byref(md), 1, 1000, n, 1000) for n in (0, 1, 500, 999, 1000)}
+    assert room[500] > room[1000]
+    for n in (0, 1, 500, 999):
+        for given, refused in ((room[1000], False), (room[0] - 256, True)):
+            rc = lib.nc_stack_forward(ctypes.byref(md), ctypes.byref(cache), at, 1, 1000, at, n, at, 1 << 20, given, None, None)
+            assert rc != 0 and (b"workspace of" in lib.nc_last_error()) == refused, (n, given, lib.nc_last_error())
+
+
 # ------------------------------------------------------------------------------------------------ configuration
 @pytest.mark.parametrize("name", list(CASES))
 def test_tensor_table_and_sizes(name):
