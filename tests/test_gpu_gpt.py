@@ -23,6 +23,7 @@ import pytest
 import torch
 
 from oracle import gpt_ref, decode_ref
+from step_cases import KV_BAR, LOGIT_BAR, STEP_CASES, appended, apart, fill, step_model
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -476,15 +477,21 @@ def _step_model(layers, heads, kv_heads, pattern="SSL", sequence_len=512, seed=5
     return model
 
 
-def _step_cache(model, lengths, room, seed=6):
-    """Rows that hold `lengths` tokens each, and the embedding of the last one."""
+def _empty_cache(model, lengths, room):
     from nanochat_amd.engine import KVCache
     cfg = model.config
-    g = torch.Generator(device=DEV).manual_seed(seed)
     cache = KVCache(len(lengths), cfg.n_kv_head, max(lengths) + room, 128, cfg.n_layer, DEV, torch.bfloat16)
+    cache.set_seqlens(torch.tensor(lengths, dtype=torch.int32))
+    return cache
+
+
+def _step_cache(model, lengths, room, seed=6):
+    """Rows that hold `lengths` tokens each, and the embedding of the last one."""
+    cfg = model.config
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    cache = _empty_cache(model, lengths, room)
     cache.k_cache.normal_(0.0, 1.2, generator=g)
     cache.v_cache.normal_(0.0, 1.0, generator=g)
-    cache.set_seqlens(torch.tensor(lengths, dtype=torch.int32))
     cache.prev_embedding = torch.nn.functional.rms_norm(torch.randn(len(lengths), 1, cfg.n_embd, generator=g, device=DEV), (cfg.n_embd,)).bfloat16()
     return cache
 
@@ -504,46 +511,42 @@ class _Present:
         return self._lib.nc_gpt_forward_present(md, cd, idx, B, logits, ws, ws_bytes, self._present, stream)
 
 
-# the edges of the launch's forms: 512, 1024, 1536 and 1792 columns, one and two query heads to a key head, one row and eight, rows that are empty, of one batch of keys
-# and one more, at the border of a workgroup's share of keys (128), past a window, and of unequal length
-STEP_CASES = [(3, 2, 2, [0]), (4, 2, 2, [63, 1]), (3, 4, 4, [127, 128, 129]), (5, 4, 2, [300]), (3, 5, 5, [5] * 8), (4, 8, 4, [0, 31, 32, 33, 256, 257, 500, 511]), (3, 9, 9, [700, 2]),
-              (3, 12, 6, [40] * 7), (4, 13, 13, [1000]), (3, 13, 13, [600] * 8), (3, 14, 7, [513, 512, 511]), (3, 14, 14, [130] * 4)]
-
-
-@pytest.mark.parametrize("layers, heads, kv_heads, lengths", STEP_CASES)
-def test_step_of_few_rows_in_one_launch_against_the_separate_launches(layers, heads, kv_heads, lengths, monkeypatch):
-    """Up to eight rows: all layers of a step in one launch, whose workgroups share the work out among those that have a place.  Against the separate launches
-    (what a tapped forward takes), which round in the same places and sum in another order: most results have the same bits.  Where a sum rounds the other
-    way, a bf16 value moves by 2^-8 of itself and an e4m3 value by 2^-3, and the layers behind carry it on; 2e-2 of the logits is half of what the oracle's own two
-    attention forms differ by.  With any number of workgroups the bits are the same."""
+@pytest.mark.parametrize("layers, heads, kv_heads, lengths, pattern", STEP_CASES)
+def test_step_of_few_rows_in_one_launch_against_the_separate_launches(layers, heads, kv_heads, lengths, pattern, monkeypatch):
+    """Up to eight rows: all layers of a step in one launch, whose workgroups share the work out among those that have a place.  Against the separate launches (what a tapped forward takes):
+    the keys and values that either appends, layer by layer and row by row, and each row's logits, with keys that stand out in each stretch of them (step_cases.py; what a lost one moves:
+    test_step_cases.py).  With any number of workgroups the bits are the same."""
     say(f"step in one launch: {layers} layers, {heads} heads on {kv_heads}, rows of {lengths}")
     from nanochat_amd import gpt as gpt_module
     B = len(lengths)
-    model = _step_model(layers, heads, kv_heads, sequence_len=512)
+    model = step_model(layers, heads, kv_heads, pattern, DEV)
     g = torch.Generator(device=DEV).manual_seed(7)
     toks = [torch.randint(0, 1024, (B, 1), generator=g, device=DEV) for _ in range(2)]
     real = gpt_module._lib.lib()
 
     def steps(run, present=0):
-        cache = _step_cache(model, lengths, 2)
-        before = cache.k_cache.clone()
+        cache = fill(_empty_cache(model, lengths, 2), model.config, lengths)
+        before = cache.k_cache.clone(), cache.v_cache.clone()
         with monkeypatch.context() as m:
             if present:
                 m.setattr(gpt_module._lib, "lib", lambda: _Present(real, present))
             logits = [run(t, cache) for t in toks]
             torch.cuda.synchronize()
         for b, n in enumerate(lengths):
-            assert torch.equal(cache.k_cache[:, b, :n], before[:, b, :n])
+            for now, then in zip((cache.k_cache, cache.v_cache), before):
+                assert torch.equal(now[:, b, :n], then[:, b, :n]) and torch.equal(now[:, b, n + 2:], then[:, b, n + 2:])
         assert cache.cache_seqlens.tolist() == [n + 2 for n in lengths]
-        return torch.stack(logits), cache.k_cache, cache.v_cache
+        return torch.stack(logits), appended(cache, lengths, 0), appended(cache, lengths, 1)
     one = steps(lambda t, c: model.forward_last(t, kv_cache=c))
-    apart = steps(lambda t, c: model.forward_tapped(t, kv_cache=c)[0][:, -1])
-    for got, want in zip(one, apart):
+    want = steps(lambda t, c: model.forward_tapped(t, kv_cache=c)[0][:, -1])
+    for got, ref, limit in zip(one, want, (LOGIT_BAR, KV_BAR, KV_BAR)):
         assert torch.isfinite(got).all()
-        assert rel_l2(got, want) <= 2e-2
+        off = apart(got, ref)
+        print(f"[bar] largest difference of a row {off.max().item():.5f} of {limit}")
+        assert (off <= limit).all(), off
     for present in (1, 7, 100):
-        for got, want in zip(steps(lambda t, c: model.forward_last(t, kv_cache=c), present), one):
-            assert torch.equal(got, want), present
+        for got, ref in zip(steps(lambda t, c: model.forward_last(t, kv_cache=c), present), one):
+            assert torch.equal(got, ref), present
 
 
 @pytest.mark.parametrize("layers, heads, kv_heads, lengths, present", [(3, 2, 2, [70], 128), (3, 4, 2, [300, 5, 0], 100), (4, 13, 13, [600] * 8, 256), (3, 14, 7, [513], 7)])
