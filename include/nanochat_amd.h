@@ -368,7 +368,9 @@ int nc_gpt_forward_tapped(const nc_model_desc* model /*host*/, const nc_cache_de
  * While enabled, every launch made by this library is bracketed by a HIP event pair on its stream.
  * Classes: 0 attention (partial + combine), 1 FP8 GEMM, 2 quantize/convert, 3 row kernels, 4 sampler, 5 nc_probe_hbm_read.
  * `units` are the algorithmic bytes (classes 0,2,3,4) or flops (class 1) of the launches.  Not thread
- * safe; at most 16384 launches are recorded per enable. */
+ * safe; at most 16384 launches are recorded per enable.  A step of up to 8 rows whose layers run in one launch has no
+ * classes: while enabled it is taken apart into the launches that other steps are made of, so its classes' times say what
+ * those cost and not what a step costs otherwise. */
 int nc_profile_enable(int on);
 int nc_profile_read(int cls, double* total_ms /*host*/, double* total_units /*host*/, int64_t* count /*host*/);
 /* The FP8 GEMM launches (class 1) of one weight shape [N,K] only: the decode step's four linears and lm_head apart. */

@@ -741,7 +741,8 @@ int nc_linear_splits(int dtype, int M, int N, int K) {
         const int nb = M <= 16 ? 16 : 32, wgs = (N + nb - 1) / nb;
         while (splits < 8 && wgs * splits < 384 && K / (splits * 2) >= 256) splits *= 2;
     } else if (dtype && K % 64 == 0 && K >= 512) {
-        // fp32: four shares, whatever the number of rows, so that a row's sums do not depend on how many came with it.  Few tiles fill the chip with
+        // fp32: four shares, whatever the number of rows above NC_FEW_ROWS, so that a row's sums do not depend on how many of them came with it.  (The chosen rows of a prompt
+        // go through the last output matrix by themselves: their number counts there, not the prompt's length.)  Few tiles fill the chip with
         // them (333 x 1024 x 5120: 152 us in one piece, 45 in four), many lose nothing (a prompt of 1792 tokens, in one piece / two / four: width
         // 2048 6675 / 6637 / 6414 us, 1024 3307 / 3319 / 3349, 640 1425 / 1376 / 1363).  bf16 sums of many rows stay one chain.
         splits = 4;

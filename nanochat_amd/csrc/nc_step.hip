@@ -33,8 +33,8 @@
 // 673 .. 735 / 618 .. 644 and 1006 .. 1176 / 965 .. 987; two such steps beside each other 1108 / 1084.  (Teams of so many, us a step of depth 20, 8 rows: 1 44900,
 // 8 6310, 32 1955, 64 1085, 128 730, 256 575.)
 //
-// us a step, separate launches / this: depth 4, one row 107 / 68; depth 10, 3 rows 300 / 171; depth 16, 4 rows of 1000 keys 590 / 344; depth 20, 640 keys, one row
-// 702 / 451, 8 rows 787 / 555; depth 26, 2000 keys, one row 965 / 648, 8 rows 1172 / 885.
+// us a step, separate launches / this, one card: depth 4, one row of 63 keys 119 / 64; depth 10, 3 rows of 500 345 / 205; depth 16, 4 rows of 1000 563 / 344; depth 18, 5 rows of 400 670 / 462;
+// depth 20, 640 keys, one row 702 / 446, 8 rows 798 / 551; depth 24 with 6 key heads, 8 rows of 1500 1017 / 686; depth 26, 2000 keys, one row 969 / 644, 8 rows 1176 / 881.
 #include <atomic>
 #include <stddef.h>
 #include <type_traits>
@@ -258,11 +258,11 @@ __device__ __forceinline__ T argument(const uint32_t* at) {
 }
 
 // NV: 512-column pieces of a residual row, so E <= 512 NV (and <= NC_STEP_MAX_E).  G: query heads per kv head.
-// Wave 0 is the one that deals with the other workgroups: it sums what the others have multiplied, stores it, counts the workgroup's arrival and polls, while
-// the others have the next weights or keys on their way.  It also finishes the heads of attention.
+// The first ROW_WAVES waves hear the other workgroups and make the rows, a wave to a row; then they sum what the last GW waves have multiplied, and send it.  In attention the first G + 2
+// finish the row's own heads, and the first G of them join what the others have read.
 template <int NV, int G>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3))) void step_kernel(NcStepArgs, NcStepLayers) {
-    constexpr int TMAX = NV == 1 ? 1 : 2;                          // tiles of a workgroup: c_fc has E / 4 of them (nc_step_wgs)
+    constexpr int TMAX = NV == 1 ? 1 : 2;                          // tiles of a workgroup: c_fc has E / 4 of them (step_wgs)
     constexpr int E_MAX = NV < 4 ? 512 * NV : NC_STEP_MAX_E;
     constexpr int RA = (E_MAX / 128 + GW - 1) / GW;                // K-steps of a wave: E / 128 over GW waves
     constexpr int RF = (4 * E_MAX / 128 + GW - 1) / GW;            //            and 4 E / 128
@@ -966,8 +966,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
 }  // namespace
 
 // ------------------------------------------------------------------------------------------------
-// Workgroups, one to a compute unit.  Half of the units where a product has no more than two tiles for each of them then (us a step, 128 / 256: depth 4, one row 68 / 70,
-// depth 10, 3 rows 171 / 175, depth 16, 4 rows 344 / 354), all of them for wider models (depth 20, 8 rows 578 / 556, depth 26, 8 rows of 2000 keys 948 / 885).
+// Workgroups, one to a compute unit.  Half of the units where a product has no more than two tiles for each of them then (us a step, 128 / 256: depth 4, one row 63.5 / 65.7,
+// depth 8 with 2 key heads, 8 rows 154 / 165, depth 10, 3 rows 205 / 210, depth 16 with 4 key heads, 5 rows 352 / 360), all of them for wider models (depth 20, 8 rows 730 with 128 of
+// 256 started / 551, depth 26, 8 rows of 2000 keys 1178 / 881).
 static int step_wgs(int E) { return E <= 1024 ? 128 : 256; }
 
 bool nc_step_fits(int B, int L, int E, int H, int Hkv) {
