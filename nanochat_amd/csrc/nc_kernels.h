@@ -174,7 +174,9 @@ int nc_launch_attention_fused(NcRopeSrc rope, bf16_t* k_cache, bf16_t* v_cache, 
 #define NC_STEP_MAX_E 1792
 #define NC_STEP_MAX_KEYS (1 << 24)        // of a cache row
 #define NC_STEP_SPLIT_KEYS 128            // of a row's kv head to a workgroup, while there are workgroups
-#define NC_STEP_MAX_SPLITS 12
+#define NC_STEP_FEW_SPLITS 12
+#define NC_STEP_LONG_SPLIT_KEYS 1024      // ... to each of more than 12
+#define NC_STEP_MAX_SPLITS 24
 #define NC_STEP_WORDS (2 * 32)           // zero before the launch
 #define NC_STEP_WAIT_POLLS (1u << 22)    // two seconds or more
 struct NcStepLayer {

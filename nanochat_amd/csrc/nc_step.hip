@@ -238,10 +238,12 @@ __device__ __forceinline__ int small_quotient(int a, int b) {
 template <typename P>
 __device__ __forceinline__ P* device_pointer(uint64_t bits) { return (P*)(__attribute__((address_space(1))) P*)bits; }
 
-// how many workgroups share the keys of a row's kv head when there are `most` of them
+// How many workgroups share the keys of a row's kv head when there are `most` of them: 128 keys or more for each of up to 12, 1024 for each of up to 24 (their parts are joined 12 at a time).
+// us a step of one row, up to 12 / so, and the separate launches' 16: 60000 keys, depth 4 288 / 189, 264, depth 12 927 / 648, 937, depth 26 2514 / 2122, 2547; 120000 keys, depth 4 350 / 227, 307.
 __host__ __device__ inline int step_splits(int most, int wgs, int pairs) {
-    const int by_wgs = wgs / pairs, room = by_wgs < NC_STEP_MAX_SPLITS ? by_wgs : NC_STEP_MAX_SPLITS, wanted = (most + NC_STEP_SPLIT_KEYS - 1) / NC_STEP_SPLIT_KEYS;
-    const int splits = wanted < room ? wanted : room;
+    const int few = (most + NC_STEP_SPLIT_KEYS - 1) / NC_STEP_SPLIT_KEYS, many = most / NC_STEP_LONG_SPLIT_KEYS;
+    const int wanted = few < NC_STEP_FEW_SPLITS ? few : many < NC_STEP_FEW_SPLITS ? NC_STEP_FEW_SPLITS : many < NC_STEP_MAX_SPLITS ? many : NC_STEP_MAX_SPLITS;
+    const int room = wgs / pairs, splits = wanted < room ? wanted : room;
     return splits < 1 ? 1 : splits;
 }
 
@@ -761,9 +763,10 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
                         if (half == 0) coherent_store_f4(mine + 4 + d, sendable(s[0]), sendable(s[1]), sendable(s[2]), sendable(s[3]));
                         if (lane == 0) store8_sc1(mine, __float_as_uint(sendable(mm)), __float_as_uint(sendable(ls)));
                     } else {
-                        if (splits > 1) {
-                            constexpr int OTHERS = NC_STEP_MAX_SPLITS / 2;
-                            const __amdgpu_buffer_rsrc_t desc = rows_desc(parts, ((splits - 1) * G - h) * MERGE_STRIDE * 4);
+                        const __amdgpu_buffer_rsrc_t desc = rows_desc(parts, ((splits - 1) * G - h) * MERGE_STRIDE * 4);
+                        for (int from_split = 0; from_split < splits - 1; from_split += NC_STEP_FEW_SPLITS) {
+                            constexpr int OTHERS = NC_STEP_FEW_SPLITS / 2;
+                            const int others = splits - 1 - from_split;
                             Pieces<OTHERS> o;
                             v2i oml[OTHERS];
 #pragma unroll
@@ -773,28 +776,28 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
                                 bool wait = false;
 #pragma unroll
                                 for (int i = 0; i < OTHERS; i++)
-                                    if (2 * i < splits - 1) {
-                                        const uint32_t from = 2 * i + half < splits - 1 ? (uint32_t)((2 * i + half) * G * MERGE_STRIDE) * 4u : OOB;
+                                    if (2 * i < others) {
+                                        const uint32_t from = 2 * i + half < others ? (uint32_t)((from_split + 2 * i + half) * G * MERGE_STRIDE) * 4u : OOB;
                                         oml[i] = __builtin_amdgcn_raw_buffer_load_b64(desc, from, 0, SC1);
                                         o[i] = load16_sc1(desc, from == OOB ? OOB : from + 16 + d * 4);
                                     }
 #pragma unroll
                                 for (int i = 0; i < OTHERS; i++)
-                                    if (2 * i < splits - 1) wait |= unwritten(o[i]) || (uint32_t)oml[i][0] == UNWRITTEN || (uint32_t)oml[i][1] == UNWRITTEN;
+                                    if (2 * i < others) wait |= unwritten(o[i]) || (uint32_t)oml[i][0] == UNWRITTEN || (uint32_t)oml[i][1] == UNWRITTEN;
                                 return wait;
                             });
                             float all = mm;
 #pragma unroll
                             for (int i = 0; i < OTHERS; i++)
-                                if (2 * i < splits - 1) all = fmaxf(all, 2 * i + half < splits - 1 ? __int_as_float(oml[i][0]) : mm);
+                                if (2 * i < others) all = fmaxf(all, 2 * i + half < others ? __int_as_float(oml[i][0]) : mm);
                             r = swap32(all);
                             all = fmaxf(__int_as_float(r[0]), __int_as_float(r[1]));
                             const float own = half == 0 ? exp2f(mm - all) : 0.f;
-                            ls *= own, s *= own;
+                            ls *= own, s *= own, mm = all;
 #pragma unroll
                             for (int i = 0; i < OTHERS; i++)
-                                if (2 * i < splits - 1) {
-                                    const float sc = 2 * i + half < splits - 1 ? exp2f(__int_as_float(oml[i][0]) - all) : 0.f;
+                                if (2 * i < others) {
+                                    const float sc = 2 * i + half < others ? exp2f(__int_as_float(oml[i][0]) - all) : 0.f;
                                     ls += __int_as_float(oml[i][1]) * sc;
 #pragma unroll
                                     for (int e = 0; e < 4; e++) s[e] += __int_as_float(o[i][e]) * sc;

@@ -511,21 +511,21 @@ class _Present:
         return self._lib.nc_gpt_forward_present(md, cd, idx, B, logits, ws, ws_bytes, self._present, stream)
 
 
-@pytest.mark.parametrize("layers, heads, kv_heads, lengths, pattern", STEP_CASES)
-def test_step_of_few_rows_in_one_launch_against_the_separate_launches(layers, heads, kv_heads, lengths, pattern, monkeypatch):
+@pytest.mark.parametrize("case", STEP_CASES, ids=str)
+def test_step_of_few_rows_in_one_launch_against_the_separate_launches(case, monkeypatch):
     """Up to eight rows: all layers of a step in one launch, whose workgroups share the work out among those that have a place.  Against the separate launches (what a tapped forward takes):
     the keys and values that either appends, layer by layer and row by row, and each row's logits, with keys that stand out in each stretch of them (step_cases.py; what a lost one moves:
     test_step_cases.py).  With any number of workgroups the bits are the same."""
-    say(f"step in one launch: {layers} layers, {heads} heads on {kv_heads}, rows of {lengths}")
+    say(f"step in one launch: {case}")
     from nanochat_amd import gpt as gpt_module
-    B = len(lengths)
-    model = step_model(layers, heads, kv_heads, pattern, DEV)
+    lengths, B = case.lengths, len(case.lengths)
+    model = step_model(case, DEV)
     g = torch.Generator(device=DEV).manual_seed(7)
     toks = [torch.randint(0, 1024, (B, 1), generator=g, device=DEV) for _ in range(2)]
     real = gpt_module._lib.lib()
 
     def steps(run, present=0):
-        cache = fill(_empty_cache(model, lengths, 2), model.config, lengths)
+        cache = fill(_empty_cache(model, lengths, 2), model.config, case)
         before = cache.k_cache.clone(), cache.v_cache.clone()
         with monkeypatch.context() as m:
             if present:
