@@ -352,8 +352,9 @@ int nc_gpt_forward_present(const nc_model_desc* model /*host*/, const nc_cache_d
 int nc_gpt_forward_giving_up(const nc_model_desc* model /*host*/, const nc_cache_desc* cache /*host*/, const int64_t* idx, int B,
                              float* logits_out, void* workspace, size_t workspace_bytes, int present, int wait_polls, nc_stream_t stream);
 
-/* After how many looks (half a microsecond or more each) such a forward begins with `registered` workgroups, where the others find no place; 0: not one of those (host only). */
-int nc_gpt_step_list_polls(const nc_model_desc* model /*host*/, int B, int registered);
+/* After how many looks (half a microsecond or more each) such a forward, over a cache of max_seq_len tokens, begins with `registered` workgroups, where the others find no place;
+ * 0: not one of those (host only). */
+int nc_gpt_step_list_polls(const nc_model_desc* model /*host*/, int B, int max_seq_len, int registered);
 
 /* The same forward with its intermediate activations copied out, for layer-by-layer comparison with another implementation
  * (no counterpart in the reference; tests only).  tap_x (or NULL): bf16 [n_layer+1, B*T, E]; slot i is the residual stream as

@@ -157,7 +157,7 @@ def _bind(lib):
         "nc_gpt_forward": (i, [C.POINTER(ModelDesc), C.POINTER(CacheDesc), p, i, i, p, i, p, sz, p]),
         "nc_gpt_forward_present": (i, [C.POINTER(ModelDesc), C.POINTER(CacheDesc), p, i, p, p, sz, i, p]),
         "nc_gpt_forward_giving_up": (i, [C.POINTER(ModelDesc), C.POINTER(CacheDesc), p, i, p, p, sz, i, i, p]),
-        "nc_gpt_step_list_polls": (i, [C.POINTER(ModelDesc), i, i]),
+        "nc_gpt_step_list_polls": (i, [C.POINTER(ModelDesc), i, i, i]),
         "nc_gpt_forward_tapped": (i, [C.POINTER(ModelDesc), C.POINTER(CacheDesc), p, i, i, p, i, p, sz, p, p, p]),
         "nc_profile_enable": (i, [i]),
         "nc_profile_read": (i, [i, C.POINTER(C.c_double), C.POINTER(C.c_double), C.POINTER(C.c_int64)]),

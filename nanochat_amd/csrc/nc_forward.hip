@@ -173,7 +173,7 @@ Workspace carve(const nc_model_desc* m, int B, int T, void* base) {
     w.step_words = c.take<uint32_t>(step ? STEP_CLEARED : 0);
     NcStepArgs sizes{};
     sizes.B = B, sizes.L = m->n_layer, sizes.E = m->n_embd, sizes.H = m->n_head, sizes.Hkv = m->n_kv_head;
-    w.step_exchange_bytes = step ? nc_step_exchange(sizes, NC_STEP_MAX_KEYS) : 0;      // (the most it takes: the cache's length is not known here)
+    w.step_exchange_bytes = step ? nc_step_exchange(sizes, NC_STEP_MAX_KEYS, NC_STEP_MAX_KEYS) : 0;      // (the most it takes: the cache's length is not known here)
     w.step_exchange = c.take<uint8_t>(w.step_exchange_bytes);
     w.total = (c.off + 255) & ~(size_t)255;
     return w;
@@ -191,13 +191,18 @@ bool reads_ahead(const nc_model_desc* m, int M) {
     return M > 128 || (M > 64 && layer <= AHEAD_LAYER_BYTES_FEW);
 }
 
-int most_visible_keys(const nc_model_desc* m, int Tmax) {
+// cached keys that a row sees in a layer when its cache is full: at most, and in the mean of the layers
+struct VisibleKeys {
+    int most, mean;
+};
+VisibleKeys visible_keys(const nc_model_desc* m, int Tmax) {
     int most = 0;
+    int64_t sum = 0;
     for (int i = 0; i < m->n_layer; i++) {
         const int w = m->layers[i].window_left, n = w >= 0 && w < Tmax ? w : Tmax;
-        most = n > most ? n : most;
+        most = n > most ? n : most, sum += n;
     }
-    return most;
+    return VisibleKeys{most, (int)(sum / m->n_layer)};
 }
 
 // Whether a step goes through nc_step.hip.  Launches of their own have what one has not: times of each kernel (the profiler), rows of any alignment, a
@@ -352,7 +357,8 @@ static int gpt_forward_impl(const nc_model_desc* m, const nc_cache_desc* kv, con
             layers.layer[i] = NcStepLayer{ly.w_qkv, ly.inv_qkv, ly.w_attn_proj, ly.inv_attn_proj, ly.w_fc, ly.inv_fc, ly.w_mlp_proj, ly.inv_mlp_proj,
                                           ly.ve_table, ly.ve_gate_w, ly.window_left, 0};
         }
-        const size_t fill = nc_step_exchange(a, most_visible_keys(m, kv->max_seq_len));
+        const VisibleKeys keys = visible_keys(m, kv->max_seq_len);
+        const size_t fill = nc_step_exchange(a, keys.most, keys.mean);
         NC_CHECK_ARG(fill <= w.step_exchange_bytes, "gpt_forward: exchange of %zu bytes, %zu in the workspace", fill, w.step_exchange_bytes);
         TRY(nc_launch_embed_norm_smear(idx, m->wte, m->smear_w, m->smear_lambda, kv->prev_in, kv->prev_out, w.x, w.x0, B, T, E, m->padded_vocab, w.step_words,
                                        STEP_CLEARED, s, w.step_exchange, fill));
@@ -555,11 +561,12 @@ extern "C" int nc_gpt_forward(const nc_model_desc* m, const nc_cache_desc* kv, c
     return gpt_forward_impl(m, kv, idx, B, T, logits_out, last_only, workspace, workspace_bytes, nullptr, nullptr, (hipStream_t)stream);
 }
 
-extern "C" int nc_gpt_step_list_polls(const nc_model_desc* m, int B, int registered) {
-    if (!m || !nc_step_fits(B, m->n_layer, m->n_embd, m->n_head, m->n_kv_head)) return 0;
+extern "C" int nc_gpt_step_list_polls(const nc_model_desc* m, int B, int max_seq_len, int registered) {
+    if (!m || !m->layers || !nc_step_fits(B, m->n_layer, m->n_embd, m->n_head, m->n_kv_head)) return 0;
     NcStepArgs a{};
     a.B = B, a.L = m->n_layer, a.E = m->n_embd, a.H = m->n_head, a.Hkv = m->n_kv_head;
-    (void)nc_step_exchange(a, 1);
+    const VisibleKeys keys = visible_keys(m, max_seq_len);
+    (void)nc_step_exchange(a, keys.most, keys.mean);
     return (int)nc_step_list_polls(a, registered);
 }
 

@@ -177,6 +177,7 @@ int nc_launch_attention_fused(NcRopeSrc rope, bf16_t* k_cache, bf16_t* v_cache, 
 #define NC_STEP_FEW_SPLITS 12
 #define NC_STEP_LONG_SPLIT_KEYS 1024      // ... to each of more than 12
 #define NC_STEP_MAX_SPLITS 24
+#define NC_STEP_MANY_KEYS 98304           // of all rows' kv heads in a layer
 #define NC_STEP_WORDS (2 * 32)           // zero before the launch
 #define NC_STEP_WAIT_POLLS (1u << 22)    // two seconds or more
 struct NcStepLayer {
@@ -215,7 +216,8 @@ struct NcStepLayers {
     NcStepLayer layer[NC_STEP_MAX_LAYERS];
 };
 static_assert(sizeof(NcStepArgs) % 8 == 0 && sizeof(NcStepArgs) + sizeof(NcStepLayers) <= 4096, "kernel arguments");
-size_t nc_step_exchange(NcStepArgs& a, int most_keys);   // B, L, E, H, Hkv and exchange are given, and how many keys a row may have; returns the bytes that `exchange` takes
+// B, L, E, H, Hkv and exchange are given, and how many keys a row may have in a layer, at most and in the mean of the layers; returns the bytes that `exchange` takes
+size_t nc_step_exchange(NcStepArgs& a, int most_keys, int mean_keys);
 bool nc_step_fits(int B, int L, int E, int H, int Hkv);
 // polls (half a microsecond or more) after which `registered` of the launch's workgroups begin without the others; behind nc_step_exchange
 uint32_t nc_step_list_polls(const NcStepArgs& a, int registered);

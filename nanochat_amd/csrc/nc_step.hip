@@ -971,12 +971,14 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
 // ------------------------------------------------------------------------------------------------
 // Workgroups, one to a compute unit.  Half of the units where a product has no more than two tiles for each of them then (us a step, 128 / 256: depth 4, one row 63.5 / 65.7,
 // depth 8 with 2 key heads, 8 rows 154 / 165, depth 10, 3 rows 205 / 210, depth 16 with 4 key heads, 5 rows 352 / 360), all of them for wider models (depth 20, 8 rows 730 with 128 of
-// 256 started / 551, depth 26, 8 rows of 2000 keys 1178 / 881).
-static int step_wgs(int E) { return E <= 1024 ? 128 : 256; }
+// 256 started / 551, depth 26, 8 rows of 2000 keys 1178 / 881), and where there are many keys: those are read as fast as there are units (128 / 256 / the separate launches, depth 10, 8 rows of 2000
+// keys in every layer 305 / 289 / 388, 8000 570 / 460 / 576, depth 12, 8 rows of 8000 882 / 620 / 743, of 60000 5043 / 3020 / 3104, depth 16, 6 rows of 8000 1220 / 855 / 1066; from some 40 to 100 thousand keys
+// of all heads on, which models of 2048 positions do not have: 82 thousand, depth 16, 8 rows 419 / 420).  By the room in the cache: where the rows are is not known here.
+static int step_wgs(int E, int64_t keys) { return E <= 1024 && (keys < NC_STEP_MANY_KEYS || nc_cu_count() < 256) ? 128 : 256; }
 
 bool nc_step_fits(int B, int L, int E, int H, int Hkv) {
     if (B < 1 || B > NC_STEP_ROWS || L < 3 || L > NC_STEP_MAX_LAYERS || E > NC_STEP_MAX_E || E != H * 128 || Hkv < 1 || (H != Hkv && H != 2 * Hkv)) return false;
-    return nc_cu_count() >= step_wgs(E);
+    return nc_cu_count() >= step_wgs(E, 0);
 }
 
 // A round of tiles of all of a step's products, in polls: a workgroup takes in some 4 KB of weights between two of them (us for one more round, measured with so many workgroups started:
@@ -987,14 +989,14 @@ static uint32_t round_polls(const NcStepArgs& a) {
 
 uint32_t nc_step_list_polls(const NcStepArgs& a, int registered) { return list_polls((uint32_t)registered, (uint32_t)a.wgs, a.round_polls); }
 
-size_t nc_step_exchange(NcStepArgs& a, int most_keys) {
+size_t nc_step_exchange(NcStepArgs& a, int most_keys, int mean_keys) {
     int at = 0;
     auto take = [&](int bytes) {
         const int here = at;
         at += (bytes + 255) & ~255;
         return here;
     };
-    a.wgs = step_wgs(a.E), a.round_polls = round_polls(a);
+    a.wgs = step_wgs(a.E, (int64_t)a.B * a.Hkv * mean_keys), a.round_polls = round_polls(a);
     take(a.B * (a.H + 2 * a.Hkv) * 256);
     a.off_y = take(a.B * a.E * 2);
     a.off_proj = take(a.B * a.E * 2);
@@ -1024,7 +1026,7 @@ static int launch(const NcStepArgs& a, const NcStepLayers& layers, int present, 
 }
 
 int nc_launch_step(const NcStepArgs& a, const NcStepLayers& layers, int present, hipStream_t s) {
-    NC_CHECK_ARG(nc_step_fits(a.B, a.L, a.E, a.H, a.Hkv) && a.wgs == step_wgs(a.E) && present >= 0 && present <= a.wgs, "step: not a shape of this kernel");
+    NC_CHECK_ARG(nc_step_fits(a.B, a.L, a.E, a.H, a.Hkv) && (a.wgs == 256 || (a.wgs == 128 && a.E <= 1024)) && present >= 0 && present <= a.wgs, "step: not a shape of this kernel");
     if (present == 0) present = a.wgs;
 #define STEP(NVV) (a.H == a.Hkv ? launch<NVV, 1>(a, layers, present, s) : launch<NVV, 2>(a, layers, present, s))
     return a.E <= 512 ? STEP(1) : a.E <= 1024 ? STEP(2) : a.E <= 1536 ? STEP(3) : STEP(4);

@@ -177,9 +177,10 @@ def test_a_model_without_backout_takes_the_separate_launches():
 
 def test_how_long_a_step_in_one_launch_waits_for_its_workgroups():
     """The smaller the team it would begin with, the longer, as a round of tiles more costs by the model's weights; a bound of some 8 ms; not longer for half of them."""
-    def polls(heads, layers, registered, B=1):
-        m = _lib.ModelDesc(n_layer=layers, n_head=heads, n_kv_head=heads, n_embd=128 * heads, vocab_size=512)
-        return _lib.lib().nc_gpt_step_list_polls(ctypes.byref(m), B, registered)
+    def polls(heads, layers, registered, B=1, keys=64, windows=(-1,)):
+        each = (_lib.LayerDesc * layers)(*[_lib.LayerDesc(window_left=windows[i % len(windows)]) for i in range(layers)])
+        m = _lib.ModelDesc(n_layer=layers, n_head=heads, n_kv_head=heads, n_embd=128 * heads, vocab_size=512, layers=each)
+        return _lib.lib().nc_gpt_step_list_polls(ctypes.byref(m), B, keys, registered)
     for heads, layers, wgs in ((2, 4, 128), (5, 10, 128), (8, 16, 128), (10, 20, 256), (13, 26, 256)):
         waits = [polls(heads, layers, n) for n in range(1, wgs + 1)]
         assert waits == sorted(waits, reverse=True) and set(waits[wgs // 2 - 1:]) == {64} and waits[0] <= 64 + (1 << 14)
@@ -187,3 +188,7 @@ def test_how_long_a_step_in_one_launch_waits_for_its_workgroups():
     assert polls(13, 26, 32) > 2 * polls(5, 10, 32) > 2 * polls(2, 4, 32)
     assert polls(13, 26, 8) > 1 << 13 and polls(2, 4, 8) < 256
     assert polls(13, 26, 8, B=9) == 0
+    # 100 are most of 128, and few of 256: as many are wanted of narrow models with many keys, in the mean of their layers
+    for heads, layers, B, line in ((2, 4, 8, 6144), (6, 12, 8, 2048), (8, 16, 1, 12288)):
+        assert [polls(heads, layers, 100, B, keys) > 64 for keys in (1, line - 1, line, 4 * line)] == [False, False, True, True]
+        assert [polls(heads, layers, 100, B, 4 * line, (0, w)) > 64 for w in (line, 2 * line - 1, 2 * line, -1)] == [False, False, True, True]
